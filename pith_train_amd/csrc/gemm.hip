@@ -263,8 +263,9 @@ static int launch_gemm(const GemmArgs& a, hipStream_t stream) {
 
 // PT_GEMM_IMPL overrides the choice of kernel for measurements: "t" = one 128x128 tile per
 // workgroup, "p0" = persistent two-phase kernel, "q0" / "q1" = persistent software-pipelined kernel
-// (8 / 4 waves), "r0" = persistent kernel with the row-split loop.  Unset: chosen per call from the shape (below).
-enum { IMPL_UNSET = -3, IMPL_AUTO = -2, IMPL_TILE = -1, IMPL_PIPELINED = 100, IMPL_ROWSPLIT = 200 };
+// (8 / 4 waves), "r0" = persistent kernel with the row-split loop, "s64" / "s128" = one 64 / 128 x 128
+// tile per workgroup with a deep load ring.  Unset: chosen per call from the shape (below).
+enum { IMPL_UNSET = -3, IMPL_AUTO = -2, IMPL_TILE = -1, IMPL_PIPELINED = 100, IMPL_ROWSPLIT = 200, IMPL_SMALL = 1000 };
 static int g_impl = IMPL_UNSET;
 static bool parse_impl(const char* e, int& impl) {
   if (!e || !*e || !strcmp(e, "auto")) impl = IMPL_AUTO;
@@ -272,6 +273,8 @@ static bool parse_impl(const char* e, int& impl) {
   else if (!strcmp(e, "p0")) impl = 0;
   else if (!strcmp(e, "q0") || !strcmp(e, "q1")) impl = IMPL_PIPELINED + (e[1] - '0');
   else if (!strcmp(e, "r0")) impl = IMPL_ROWSPLIT;
+  else if (!strcmp(e, "s64")) impl = IMPL_SMALL + 64;
+  else if (!strcmp(e, "s128")) impl = IMPL_SMALL + 128;
   else return false;
   return true;
 }
@@ -297,6 +300,20 @@ static int preferred_kernel(const GemmArgs& g) {
   return g.red >= 512 ? KERNEL_PIPELINED : KERNEL_TWO_PHASE;
 }
 
+// Problems too small for 256 x 256 tiles to fill 256 compute units go to the kernel with one 64 x 128 or
+// 128 x 128 tile per workgroup (gemm_small.hip): tile rows, or 0 when the persistent kernels are the
+// better choice.  While all 64-row tiles run at once the smaller tile wins (1001 x 512 x 2048: 10.5 us
+// against 13.1 with 128 rows and 25.0 for the pipelined kernel; 4096 x 512 x 4096: 18.5, 23.4, 46.0);
+// with more of them, 128-row tiles do up to two rounds of workgroups (2048 x 2048 x 2816, 256 tiles: 19.0
+// against 35.4; 4096 x 2048 x 2048, 512 tiles: 27.8 against 28.8; 4352 x 2048 x 1536 in 16 groups, 544
+// tiles: 31.9 against 27.5), past which the persistent kernels' overlap of one tile's stores with the
+// next tile's loads counts for more.
+static int small_tile_rows(const GemmArgs& g) {
+  const int64_t cols = cdiv(g.rows_b, 128) * (g.mode == GEMM_K_GROUPED ? g.G : 1);
+  if (cdiv(g.rows_a, 64) * cols <= 256) return 64;
+  return cdiv(g.rows_a, 128) * cols <= 512 ? 128 : 0;
+}
+
 // The persistent kernels address operands through 32-bit buffer offsets (signed range for the
 // loads, whose out-of-range marker is bit 31) and the result through an unsigned 32-bit byte
 // offset from the start of the output (of one group's block in the k-grouped mode, of the
@@ -314,11 +331,12 @@ static bool fits_persistent(const GemmArgs& g) {
 static int dispatch_gemm(const GemmArgs& g, hipStream_t stream) {
   const int impl = gemm_impl();
   const bool fits = fits_persistent(g);
-  if (g.b_kmajor) {  // one kernel reads this layout, whatever kernel was selected for the others
+  if (g.b_kmajor) {  // two kernels read this layout, whatever kernel was selected for the others
     PT_REQUIRE(fits, "gemm: the reduction-major b operand needs the row-split kernel, which addresses operands below 2 GiB "
                      "and an output below 4 GiB through 32-bit byte offsets; larger problems take the NT entry point on the "
                      "transposed operand");
-    return launch_gemm_rowsplit(g, 0, stream);
+    const int rows = impl >= IMPL_SMALL ? impl - IMPL_SMALL : impl == IMPL_AUTO ? small_tile_rows(g) : 0;
+    return rows ? launch_gemm_small(g, rows, stream) : launch_gemm_rowsplit(g, 0, stream);
   }
   PT_REQUIRE((!g.out_row_index && !g.bias) || (impl != IMPL_TILE && fits),
              "gemm: scattered output rows and the fused bias need the persistent kernels, which address every operand and "
@@ -326,12 +344,14 @@ static int dispatch_gemm(const GemmArgs& g, hipStream_t stream) {
              "output below 4 GiB");
   if (impl == IMPL_TILE || !fits) return launch_gemm<128, 128, 2, 2>(g, stream);
   if (impl == IMPL_AUTO) {
+    if (const int rows = small_tile_rows(g)) return launch_gemm_small(g, rows, stream);
     switch (preferred_kernel(g)) {
       case KERNEL_ROWSPLIT: return launch_gemm_rowsplit(g, 0, stream);
       case KERNEL_PIPELINED: return launch_gemm_pipelined(g, 0, stream);
       default: return launch_gemm_persistent(g, 0, stream);
     }
   }
+  if (impl >= IMPL_SMALL) return launch_gemm_small(g, impl - IMPL_SMALL, stream);
   if (impl >= IMPL_ROWSPLIT) return launch_gemm_rowsplit(g, impl - IMPL_ROWSPLIT, stream);
   if (impl >= IMPL_PIPELINED) return launch_gemm_pipelined(g, impl - IMPL_PIPELINED, stream);
   return launch_gemm_persistent(g, impl, stream);
@@ -343,7 +363,7 @@ using namespace pt;
 
 extern "C" int pt_gemm_select_kernel(const char* name) {
   int impl;
-  PT_REQUIRE(parse_impl(name, impl), "gemm_select_kernel: unknown kernel '%s' (auto, p0, q0, q1, r0, t)", name);
+  PT_REQUIRE(parse_impl(name, impl), "gemm_select_kernel: unknown kernel '%s' (auto, p0, q0, q1, r0, s64, s128, t)", name);
   g_impl = impl;
   return PT_OK;
 }

@@ -41,5 +41,7 @@ int launch_gemm_persistent(const GemmArgs& a, int variant, hipStream_t stream);
 int launch_gemm_pipelined(const GemmArgs& a, int variant, hipStream_t stream);
 // persistent kernel whose two steps per 128-block split the tile by rows (gemm_rowsplit.hip)
 int launch_gemm_rowsplit(const GemmArgs& a, int variant, hipStream_t stream);
+// one tile of 64 or 128 rows x 128 columns per workgroup, for small problems (gemm_small.hip)
+int launch_gemm_small(const GemmArgs& a, int rows, hipStream_t stream);
 
 }  // namespace pt

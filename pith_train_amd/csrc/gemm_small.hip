@@ -1,0 +1,233 @@
+// FP8 GEMM for problems that do not fill the GPU with 256 x 256 tiles (gfx950).
+//
+// A layer with few tokens has a handful of large tiles: most compute units stay idle, and the ones
+// that work spend their time waiting for one operand stage after the other.  Here a workgroup of
+// four waves owns one BM x 128 tile (BM = 64 or 128), so there are four to eight times as many
+// workgroups, and the LDS holds a ring of four or five 128-deep stages, all of them requested
+// ahead: a step waits only for the stage requested three or four steps earlier.  There is no
+// persistent loop, no tile table and no scan over the groups (a tile finds its group with one
+// ballot over the group ends), which keeps the time before the first load and the code that has to
+// be fetched short.
+//
+// Operand layouts in LDS, direct-to-LDS loads, scale handling and result stores are those of the
+// persistent kernels (gemm_persistent_parts.h); the MFMAs run in the same order, so the results have
+// the same bits.
+#include "gemm_persistent_parts.h"
+
+namespace pt {
+
+template <int MODE, int BM, bool ACC, bool BT>
+__global__ __launch_bounds__(256, 1) void fp8_gemm_small_kernel(GemmArgs p) {
+  constexpr int BN = 128, BK = 128;
+  constexpr int NS = BM == 64 ? 5 : 4;  // stages in the LDS ring: 120 or 128 KiB
+  constexpr int TM = BM / 64, TN = 2;   // waves 2 x 2, each TM x 2 blocks of 32 x 32
+  constexpr int STAGE = (BM + BN) * BK;
+  constexpr int LA = BM / 32, LB = BN / 32;  // 1 KiB loads of a and of b per wave and stage
+  constexpr int NP = LA + LB + 1;            // and one of scales
+  constexpr int kWait = (NS - 2) * NP;       // loads of the stages after the one a step needs
+  static_assert(kWait < 64, "vmcnt is a 6-bit counter");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // [NS][STAGE] | [NS][BM + BN] scales | 256 B sink | staging
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm0 = (wave >> 1) * (BM / 2), wn0 = (wave & 1) * 64;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  const uint32_t sc_base = lds_base + NS * STAGE;
+
+  // ---- which tile: an XCD takes an eighth of the list (its tiles share operand panels in that L2).
+  // The m-grouped row count is known on the device only; workgroups past the real list end here. ----
+  const int total = MODE == GEMM_M_GROUPED ? p.offs[p.G - 1] / BM * p.tiles_b : (int)p.total_tiles;
+  const int per_xcd = (total + 7) >> 3;
+  const int idx = blockIdx.x >> 3;
+  const int t = (blockIdx.x & 7) * per_xcd + idx;
+  if (idx >= per_xcd || t >= total) return;
+  Tile T;
+  if (MODE == GEMM_M_GROUPED) {
+    const int tr = t / p.tiles_b;
+    T.a_row0 = tr * BM;
+    T.b_row0 = (t - tr * p.tiles_b) * BN;
+    int g = 0;  // groups that end at or before the tile's first row; groups are multiples of 128 rows
+    for (int g0 = 0; g0 < p.G; g0 += 64) {
+      const int q = g0 + lane;
+      g += __popcll(__ballot(q < p.G && p.offs[q < p.G ? q : 0] <= T.a_row0));
+    }
+    T.g = __builtin_amdgcn_readfirstlane(g);
+    T.a_lim = T.a_row0 + BM; T.b_lim = (int)p.rows_b;
+    T.k_begin = 0; T.k_len = (int)p.red; T.kb0 = 0;
+  } else {
+    const int per_g = p.tiles_a * p.tiles_b;
+    const int g = t / per_g, r = t - g * per_g;
+    const int ta = r / p.tiles_b;
+    T.g = g;
+    T.a_row0 = ta * BM; T.b_row0 = (r - ta * p.tiles_b) * BN;
+    T.a_lim = (int)p.rows_a; T.b_lim = (int)p.rows_b;
+    T.k_begin = 0; T.k_len = (int)p.red; T.kb0 = 0;
+    if (MODE == GEMM_K_GROUPED) {
+      T.k_begin = __builtin_amdgcn_readfirstlane(g ? k_group_end(p, g - 1) : 0);
+      T.k_len = __builtin_amdgcn_readfirstlane(k_group_end(p, g)) - T.k_begin;
+      T.kb0 = T.k_begin >> 7;
+    }
+  }
+  const int nk = (T.k_len + 127) >> 7;
+
+  // ---- loads (layout and swizzle as in gemm_rowsplit.hip) ----
+  const int chunk = (lane & 7) ^ (lane >> 3) ^ (wave & 1);
+  const uint32_t va = (uint32_t)(lane >> 3) * (uint32_t)p.lda + chunk * 16;
+  // Row-major b as a.  Reduction-major b: a stage holds 128 reduction rows of 128 bytes, logical
+  // 16-byte chunk c of row k at position c ^ 2 ((k >> 1) & 3): the eight rows a transposing read
+  // touches lie two to a 256-byte bank line, and the four row pairs put a chunk at four positions.
+  const int bt_chunk = (lane & 7) ^ (2 * ((lane >> 4) & 3));
+  const uint32_t vb = (uint32_t)(lane >> 3) * (uint32_t)p.ldb + (BT ? bt_chunk : chunk) * 16;
+  const v4i rs_a = make_rsrc(p.a, (uint32_t)p.a_bytes);
+  const v4i rs_b = make_rsrc(p.b + (MODE == GEMM_M_GROUPED ? (int64_t)T.g * p.b_stride_g : 0), (uint32_t)p.b_bytes);
+  const v4i rs_sa = make_rsrc(p.sa, (uint32_t)p.sa_bytes);
+  const v4i rs_sb = make_rsrc(p.sb + (MODE == GEMM_M_GROUPED ? (int64_t)T.g * p.sb_stride_g : 0), (uint32_t)p.sb_bytes);
+  constexpr int SLA = BM / 64;  // scale loads of a (the next two are b's, the fourth of BM = 64 goes to the sink)
+  const bool sc_a = wave < SLA, sc_real = wave < SLA + 2;
+  uint32_t vs;
+  if (sc_a) vs = (uint32_t)(((int64_t)((T.a_row0 + 64 * wave + lane) >> p.sa_shift) * p.sa_rs + (int64_t)T.kb0 * p.sa_ks) * 4);
+  else      vs = (uint32_t)(((int64_t)((T.b_row0 + 64 * (wave - SLA) + lane) >> p.sb_shift) * p.sb_rs + (int64_t)T.kb0 * p.sb_ks) * 4);
+  const int a_rows = T.a_lim - T.a_row0;
+  const uint32_t soA0 = (uint32_t)T.a_row0 * (uint32_t)p.lda + T.k_begin;
+  const uint32_t soB0 = BT ? (uint32_t)T.b_row0 : (uint32_t)T.b_row0 * (uint32_t)p.ldb + T.k_begin;
+  const bool bt_in = T.b_row0 + bt_chunk * 16 < T.b_lim;
+
+  auto issue_stage = [&](int it) {
+    // past the end of the reduction the same loads run out of range, so that every step counts alike
+    const int slot = it % NS;
+    const uint32_t sA = lds_base + slot * STAGE, sB = sA + BM * BK;
+    const bool ok = it < nk;
+    const uint32_t koff = (uint32_t)it * BK;
+    const bool in = ok && (int)(koff + chunk * 16) < T.k_len;
+#pragma unroll
+    for (int k = 0; k < LA; ++k) {
+      const int q = 4 * k + wave;
+      dma16(rs_a, in && 8 * q < a_rows ? va : kOob, soA0 + koff + (uint32_t)(8 * q) * (uint32_t)p.lda, sA + q * 1024);
+    }
+#pragma unroll
+    for (int k = 0; k < LB; ++k) {
+      const int q = 4 * k + wave;
+      if constexpr (BT) dma16(rs_b, ok && bt_in ? vb : kOob, soB0 + (koff + 8 * q) * (uint32_t)p.ldb, sB + q * 1024);
+      else              dma16(rs_b, in ? vb : kOob, soB0 + koff + (uint32_t)(8 * q) * (uint32_t)p.ldb, sB + q * 1024);
+    }
+    const uint32_t dst = sc_real ? sc_base + slot * (BM + BN) * 4 + wave * 256 : sc_base + NS * (BM + BN) * 4;
+    if (sc_a) dma4(rs_sa, ok ? vs : kOob, (uint32_t)(it * p.sa_ks * 4), dst);
+    else      dma4(rs_sb, ok && sc_real ? vs : kOob, (uint32_t)(it * p.sb_ks * 4), dst);
+  };
+
+  // ---- fragment reads ----
+  const int fs_rd = (lane & 7) ^ ((lane >> 3) & 1);
+  int coff[2][2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) coff[ks][h] = (lane & 31) * 128 + (((ks * 4 + (lane >> 5) * 2 + h) ^ fs_rd) << 4);
+  auto read_frag = [&](const uint8_t* base, int ks) -> v8i {
+    const uint4 lo = *(const uint4*)(base + coff[ks][0]);
+    const uint4 hi = *(const uint4*)(base + coff[ks][1]);
+    return v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+  };
+  uint32_t bt_rd[2];  // the lane's byte offset for b block j, reduction rows 0-7 of a 64-deep half
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int s16 = lane & 15, g16 = lane >> 4, k = s16 >> 1;
+    const int c = (wn0 >> 4) + 2 * j + (g16 & 1);
+    bt_rd[j] = (uint32_t)((32 * (g16 >> 1) + k) * 128 + ((c ^ (2 * ((k >> 1) & 3))) << 4) + 8 * (s16 & 1));
+  }
+  auto read_b = [&](const uint8_t* sB, int j, int ks) -> v8i {
+    if constexpr (BT) {
+      typedef int v2i_t __attribute__((ext_vector_type(2)));
+      v8i r;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const v2i_t w = __builtin_amdgcn_ds_read_tr8_b64_v2i32((v2i_t __attribute__((address_space(3)))*)(sB + bt_rd[j] + ks * (64 * 128) + q * 8 * 128));
+        r[2 * q] = w[0];
+        r[2 * q + 1] = w[1];
+      }
+      return r;
+    } else {
+      return read_frag(sB + (wn0 + 32 * j) * BK, ks);
+    }
+  };
+
+  v16f acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+#pragma unroll 1
+  for (int s = 0; s < NS - 1; ++s) issue_stage(s);
+#pragma unroll 1
+  for (int it = 0; it < nk; ++it) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kWait) : "memory");
+    __syncthreads();  // stage `it` is complete, and every wave has read the stage whose slot is refilled next
+    issue_stage(it + NS - 1);
+    const uint8_t* sA = lds + (it % NS) * STAGE;
+    const uint8_t* sB = sA + BM * BK;
+    const float* sc = (const float*)(lds + NS * STAGE) + (it % NS) * (BM + BN);
+    int sca[TM], scb[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) sca[i] = (int)(__float_as_uint(sc[wm0 + 32 * i + (lane & 31)]) >> 23);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) scb[j] = (int)(__float_as_uint(sc[BM + wn0 + 32 * j + (lane & 31)]) >> 23);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      v8i fa[TM], fb[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fa[i] = read_frag(sA + (wm0 + 32 * i) * BK, ks);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fb[j] = read_b(sB, j, ks);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[i], fb[j], acc[i][j], 0, 0, 0, sca[i], 0, scb[j]);
+    }
+  }
+  wait_all_vmem();  // nothing may still be writing into this workgroup's LDS when it retires
+  if (MODE == GEMM_K_GROUPED && nk == 0 && ACC) return;
+  store_tile<MODE, TM, TN, ACC, 0>(acc, p, T, wm0, wn0, lane, lds + NS * STAGE + NS * (BM + BN) * 4 + 256 + wave * 2048);
+}
+
+template <int MODE, int BM, bool ACC, bool BT>
+static int launch_small(GemmArgs a, hipStream_t stream) {
+  constexpr int NS = BM == 64 ? 5 : 4;
+  constexpr size_t lds = (size_t)NS * (BM + 128) * 128 + NS * (BM + 128) * 4 + 256 + 4 * 2048;
+  static bool attr_set = false;
+  auto kernel = fp8_gemm_small_kernel<MODE, BM, ACC, BT>;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) { set_error("gemm: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e)); return PT_ERR_LAUNCH; }
+    attr_set = true;
+  }
+  a.tiles_a = (int)cdiv(a.rows_a, BM);
+  a.tiles_b = (int)cdiv(a.rows_b, 128);
+  a.total_tiles = (int64_t)a.tiles_a * a.tiles_b * (MODE == GEMM_K_GROUPED ? a.G : 1);
+  if (a.total_tiles == 0) return PT_OK;
+  PT_REQUIRE(a.total_tiles < (1ll << 28), "gemm: too many tiles");
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(cdiv(a.total_tiles, 8) * 8)), dim3(256), lds, stream, a);
+  return check_launch("fp8_gemm_small_kernel");
+}
+
+template <int BM>
+static int launch_small_mode(const GemmArgs& a, hipStream_t stream) {
+  switch (a.mode) {
+    case GEMM_DENSE: return launch_small<GEMM_DENSE, BM, false, false>(a, stream);
+    case GEMM_M_GROUPED:
+      return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true>(a, stream)
+                        : launch_small<GEMM_M_GROUPED, BM, false, false>(a, stream);
+    default:
+      return a.accumulate ? launch_small<GEMM_K_GROUPED, BM, true, false>(a, stream)
+                          : launch_small<GEMM_K_GROUPED, BM, false, false>(a, stream);
+  }
+}
+
+int launch_gemm_small(const GemmArgs& a, int rows, hipStream_t stream) {
+  PT_REQUIRE(rows == 64 || rows == 128, "gemm: the small-problem kernel has tiles of 64 or 128 rows");
+  return rows == 64 ? launch_small_mode<64>(a, stream) : launch_small_mode<128>(a, stream);
+}
+
+}  // namespace pt

@@ -1,0 +1,79 @@
+"""The small-problem GEMM kernel (64- and 128-row tiles) against the persistent kernels: same MFMAs in
+the same order, so the same bits, at the edges of its tiles and of its reduction stages."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _fp8(g, *shape):
+    return (torch.randn(shape, generator=g) * 60).to(torch.float8_e4m3fn).cuda()
+
+
+def _scale(g, *shape):
+    return torch.exp2(torch.randint(-8, 2, shape, generator=g).float()).cuda()
+
+
+def _cdiv(a, b):
+    return -(-a // b)
+
+
+def _same_bits(run, out, reference):
+    from pith_train_amd import _lib
+
+    results = {}
+    for name in (reference, "s64", "s128"):
+        _lib.call("pt_gemm_select_kernel", name.encode())
+        try:
+            out.fill_(0.5)
+            run()
+            torch.cuda.synchronize()
+            results[name] = out.clone()
+        finally:
+            _lib.call("pt_gemm_select_kernel", None)
+    for name in ("s64", "s128"):
+        assert torch.equal(results[name], results[reference]), f"{name} differs from {reference}"
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 8, 16), (64, 128, 128), (65, 129, 144), (1001, 512, 2048), (130, 1003, 656), (128, 264, 5 * 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_dense(m, n, k, dtype):
+    from pith_train_amd import _lib
+
+    g = torch.Generator().manual_seed(m + n + k)
+    a, sa, b, sb = _fp8(g, m, k), _scale(g, m, _cdiv(k, 128)), _fp8(g, n, k), _scale(g, _cdiv(n, 128), _cdiv(k, 128))
+    out = torch.empty((m, n), device="cuda", dtype=dtype)
+    _same_bits(lambda: _lib.call("pt_gemm_nt_dense", a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), out.data_ptr(),
+                                 _lib.dtype_code(dtype), m, n, k, _lib.stream_ptr()), out, "q0")
+
+
+@pytest.mark.parametrize("rows,n,k", [([128, 0, 384, 128], 264, 400), ([256] * 3, 128, 128), ([128] * 70, 72, 1040)])
+@pytest.mark.parametrize("form", ["nt", "nn", "nn_scatter", "wgrad", "wgrad_add"])
+def test_grouped(rows, n, k, form):
+    from pith_train_amd.operators.grouped_linear import k_grouped_fp8_wgrad, m_grouped_fp8_gemm_nn, m_grouped_fp8_gemm_nt
+
+    g = torch.Generator().manual_seed(n + k)
+    if form != "nt":
+        n = _cdiv(n, 16) * 16
+    G, M = len(rows), sum(rows)
+    offs = torch.tensor(rows).cumsum(0).to(torch.int32).cuda()
+    if form.startswith("wgrad"):
+        dy, dys, x, xs = _fp8(g, n, M), _scale(g, M // 128, n), _fp8(g, k, M), _scale(g, M // 128, k)
+        out = torch.empty((G, n, k), device="cuda", dtype=torch.bfloat16)
+        _same_bits(lambda: k_grouped_fp8_wgrad((dy, dys), (x, xs), out, offs, form == "wgrad_add"), out, "r0")
+        return
+    cap = M + 256  # a buffer sized for more rows than the routing produced
+    a, sa = _fp8(g, cap, k), _scale(g, cap, _cdiv(k, 128))
+    out = torch.empty((cap, n), device="cuda", dtype=torch.bfloat16)
+    if form == "nt":
+        b, sb = _fp8(g, G, n, k), _scale(g, G, _cdiv(n, 128), _cdiv(k, 128))
+        _same_bits(lambda: m_grouped_fp8_gemm_nt((a, sa), (b, sb), out, offs), out, "r0")
+        return
+    b, sb = _fp8(g, G, k, n), _scale(g, G, _cdiv(k, 128), _cdiv(n, 128))
+    index = None
+    if form == "nn_scatter":
+        index = torch.randperm(cap, generator=g).to(torch.int32)
+        index[::7] = -1
+        index = index.cuda()
+    _same_bits(lambda: m_grouped_fp8_gemm_nn((a, sa), (b, sb), out, offs, index), out, "r0")
