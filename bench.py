@@ -15,8 +15,10 @@ same layer (the reference's pure-PyTorch BF16 grouped-linear semantics) on a bou
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
+import struct
 import sys
 import time
 
@@ -151,8 +153,10 @@ class GemmTimer:
     NAMES = ("pt_gemm_m_grouped_nt", "pt_gemm_m_grouped_nt_scatter", "pt_gemm_m_grouped_nt_bias",
              "pt_gemm_m_grouped_nn", "pt_gemm_m_grouped_nn_scatter",
              "pt_gemm_m_grouped_nt_scatter_bias", "pt_gemm_k_grouped_wgrad",
-             "pt_gemm_k_grouped_wgrad_ld",
+             "pt_gemm_k_grouped_wgrad_ld", "pt_gemm_k_grouped_wgrad_pair",
              "pt_gemm_nt_dense", "pt_gemm_nt_dense_splitk", "pt_gemm_nt_dense_ld", "pt_gemm_nt_dense_splitk_ld")
+
+    WHOLE_STEPS = ("pt_experts_forward", "pt_experts_backward", "pt_experts_weight_gradient", "pt_linear_forward", "pt_linear_backward")
 
     def __init__(self):
         self.records = []
@@ -177,20 +181,40 @@ class GemmTimer:
                 sizes = {"pt_gemm_nt_dense": args[6:9], "pt_gemm_nt_dense_splitk": args[7:10],
                          "pt_gemm_nt_dense_ld": args[8:11], "pt_gemm_nt_dense_splitk_ld": args[9:12],
                          "pt_gemm_k_grouped_wgrad": args[9:12],
-                         "pt_gemm_k_grouped_wgrad_ld": args[11:14]}.get(name, args[8:11])
+                         "pt_gemm_k_grouped_wgrad_ld": args[11:14],
+                         "pt_gemm_k_grouped_wgrad_pair": args[11:14]}.get(name, args[8:11])
                 timer.records.append((name, a, b, "x".join(str(int(v)) for v in sizes)))
             else:
                 orig(name, *args)
 
         _lib.call = call
-        # modules imported `_lib` (the module), so they see the patched attribute
+        # modules imported `_lib` (the module), so they see the patched attribute; the entry points that
+        # a whole-step call runs report themselves through the library's observer
+        self.other = []
+        self.all_enabled = False
+        pending = []
+
+        def observe(name, begin, a, b, c):
+            name = name.decode()
+            gemm = name in GemmTimer.NAMES
+            if not (timer.enabled if gemm else timer.all_enabled):
+                return
+            event = torch.cuda.Event(enable_timing=True)
+            event.record()
+            if begin:
+                pending.append(event)
+            elif gemm:
+                timer.records.append((name, pending.pop(), event, f"{a}x{b}x{c}"))
+            else:
+                timer.other.append((name, pending.pop(), event, None, (a, b, c)))
+
+        self._observer = ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64)(observe)
+        _lib.load().pt_set_observer(ctypes.cast(self._observer, ctypes.c_void_p))
         return self
 
     def install_all(self):
         """Second mode, used after the timed region only: events around every other entry point too,
-        collected in ``other`` as (name, start, end, args)."""
-        self.other = []
-        self.all_enabled = False
+        collected in ``other`` as (name, start, end, args, sizes)."""
         import torch
 
         from pith_train_amd import _lib
@@ -199,13 +223,13 @@ class GemmTimer:
         timer = self
 
         def call(name, *args):
-            if timer.all_enabled and name not in GemmTimer.NAMES:
+            if timer.all_enabled and name not in GemmTimer.NAMES and name not in GemmTimer.WHOLE_STEPS:
                 a = torch.cuda.Event(enable_timing=True)
                 b = torch.cuda.Event(enable_timing=True)
                 a.record()
                 inner(name, *args)
                 b.record()
-                timer.other.append((name, a, b, args))
+                timer.other.append((name, a, b, args, None))
             else:
                 inner(name, *args)
 
@@ -220,8 +244,28 @@ class GemmTimer:
         buffer capacities; the kernels stop at the real count, which is what is priced."""
         sc = 4.0 / 128
 
+        rows = lambda m: min(int(m), padded_rows)  # noqa: E731
+
+        def nbytes_of_step(name, sizes):  # an entry point inside a whole-step call: (rows, columns, source rows)
+            r, cols, src = sizes
+            if name == "pt_quant_rowwise_colwise":
+                return rows(r) * cols * (4 + 2 * sc)
+            if name == "pt_quant_rowwise_colwise_rows":
+                return (min(rows(r), routed_rows) * 2 + rows(r) * (2 + 2 * sc)) * cols + 4 * rows(r)
+            if name in ("pt_silu_mul_quant_rowwise_colwise", "pt_clamped_swiglu_quant_rowwise_colwise"):
+                return rows(r) * cols * (4 + 2 + 2 * sc)
+            if name in ("pt_silu_mul_bwd_quant_rowwise_colwise", "pt_clamped_swiglu_bwd_quant_rowwise_colwise"):
+                return rows(r) * cols * (2 + 4 + 2 * (2 + 2 * sc))
+            if name == "pt_quant_rowwise_transpose_ld":
+                return r * cols * (4 + 2 * sc)
+            if name == "pt_quant_rowwise_blockwise_transpose_ld":
+                return r * cols * (4 + sc)
+            return None
+
         def nbytes(name, a):
-            rows = lambda m: min(int(m), padded_rows)  # noqa: E731
+            if name == "pt_quant_weights":
+                parts = struct.unpack(f"={10 * a[1]}q", a[0])
+                return sum(3 * parts[i + 1] * parts[i + 2] * parts[i + 3] for i in range(0, len(parts), 10))
             if name == "pt_quant_rowwise_colwise":
                 return rows(a[2]) * a[3] * (4 + 2 * sc)
             if name == "pt_quant_rowwise_colwise_rows":
@@ -241,11 +285,11 @@ class GemmTimer:
             return None
 
         agg = {}
-        for name, a, b, args in self.other:
+        for name, a, b, args, sizes in self.other:
             d = agg.setdefault(name, [0.0, 0, 0.0])
             d[0] += a.elapsed_time(b) * 1e3
             d[1] += 1
-            nb = nbytes(name, args)
+            nb = nbytes(name, args) if args is not None else nbytes_of_step(name, sizes)
             d[2] += nb if nb else 0.0
         out = []
         for name, (us, n, nb) in sorted(agg.items(), key=lambda kv: -kv[1][0]):

@@ -112,7 +112,9 @@ int pt_quant_rowwise_transpose(const void* x, int dtype, int64_t M, int64_t N, i
                                pt_stream_t stream);
 /* The same with a row pitch ld_t >= M (bytes) for t_fp8: a reduction over all tokens reads the
  * transposed operand along rows, and a power-of-two pitch (M = 8192, 32768 tokens) puts those rows
- * on few memory channels.  No counterpart in the reference (its transposed outputs are packed). */
+ * on few memory channels.  A pitch that is a multiple of 16 and at least M rounded up to 16 also gets
+ * the columns from M to there filled with zeros (a reduction in 16-byte chunks reads them).  No
+ * counterpart in the reference (its transposed outputs are packed). */
 int pt_quant_rowwise_transpose_ld(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx,
                                   void* tok_fp8, float* tok_scale, void* t_fp8, int64_t ld_t,
                                   float* t_scale, pt_stream_t stream);
@@ -138,6 +140,19 @@ int pt_quant_blockwise_transpose_batched(const void* x, int dtype, int64_t G, in
                                          int64_t stride_g, int64_t stride_row, void* fp8,
                                          float* scale, void* fp8_t, float* scale_t,
                                          pt_stream_t stream);
+/* Several weights (up to PT_QUANT_WEIGHTS_MAX, one dtype) quantised in their forward layout by one launch:
+ * the projections of an expert block after an optimizer step.  x [G, N, K] with strides in elements;
+ * fp8 [G, N, K] and scale [G, ceil(N/128), ceil(K/128)] may be slices of larger tensors (group strides
+ * in bytes and in floats).  All fields are 8 bytes wide. */
+#define PT_QUANT_WEIGHTS_MAX 4
+typedef struct {
+  const void* x;
+  int64_t G, N, K, stride_g, stride_row;
+  void* fp8; int64_t fp8_stride_g;
+  float* scale; int64_t scale_stride_g;
+} pt_quant_weight;
+int pt_quant_weights(const pt_quant_weight* parts /* host */, int32_t n, int dtype, pt_stream_t stream);
+
 /* The same into slices of larger outputs: group strides for fp8 / scale, and for the transposed
  * twin its row pitch t_ld (>= N), group stride, and the row length scale_t_ld of its scale grid.
  * Separate gate and up weights are quantised into one fused [G, 2I, K] operand this way (the up
@@ -253,6 +268,13 @@ int pt_gemm_k_grouped_wgrad_ld(const void* dy_t_fp8, const float* dy_scale, int6
                                void* out, int out_dtype, int accumulate, const int32_t* offs,
                                int32_t num_groups, int64_t M, int64_t N, int64_t K,
                                pt_stream_t stream);
+/* The same for two parameters whose gradients are the first `split` (a multiple of 128) and the remaining
+ * rows of every group's [N, K] result: one launch instead of two on halves of dy_t.  out0 [G, split, K],
+ * out1 [G, N - split, K]. */
+int pt_gemm_k_grouped_wgrad_pair(const void* dy_t_fp8, const float* dy_scale, const void* x_t_fp8,
+                                 const float* x_scale, void* out0, void* out1, int64_t split,
+                                 int out_dtype, int accumulate, const int32_t* offs, int32_t G,
+                                 int64_t M, int64_t N, int64_t K, pt_stream_t stream);
 
 /* Which GEMM kernel the three entry points above launch: "auto" (or NULL: per call from the
  * shape; the default unless the environment variable PT_GEMM_IMPL names one of the others),
@@ -411,6 +433,10 @@ int pt_segment_sum(const void* x, const int32_t* offs, int32_t num_groups, void*
 int pt_segment_sum_rows(const void* x, int64_t x_rows, const int32_t* row_index, const int32_t* offs,
                         int32_t num_groups, void* out, int64_t M, int64_t H, int dtype,
                         int out_dtype, pt_stream_t stream);
+/* pt_segment_sum of fp32 rows that each stand for `unit` grouped rows (per-tile column sums): group g owns
+ * rows offs[g-1] / unit .. offs[g] / unit - 1. */
+int pt_segment_sum_tiles(const float* x, const int32_t* offs, int32_t unit, int32_t num_groups,
+                         void* out, int64_t M, int64_t H, int out_dtype, pt_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------
  * Top-k weighted combine with the residual: the memory-bound step that follows the expert path.
@@ -482,6 +508,112 @@ int pt_router_topk_bwd(const void* logits, int64_t ld_logits, int dtype, int64_t
                        int32_t topk_group, const int64_t* topk_idx, const float* d_weight,
                        const float* d_scores, void* d_logits, int64_t ld_dlogits,
                        pt_stream_t stream);
+
+/* ------------------------------------------------------------------------------------------
+ * Whole steps as one call: the launches of a forward or a backward are prepared and queued here
+ * instead of one by one by the caller.  The argument blocks are read on the host during the call;
+ * every field is 8 bytes wide.
+ * ------------------------------------------------------------------------------------------ */
+
+/* Forward of an expert block (gate_up projection, SwiGLU, down projection; FP8 operands).
+ * x bf16 [x_rows, K] (row stride ldx).  With row_map (int32 [M], the scatter's source map, negative =
+ * padding) grouped row r is x[row_map[r]], or x[expand_idx[row_map[r]]] with expand_idx (int64
+ * [n_expand]); the row count is then read from offs[G-1].  Without it x has M grouped rows.
+ * gate_up bf16 [M, 2*half] is an output that the backward reads.  out bf16: row_map'd to
+ * [out_rows, H] when scatter != 0, else [M, H].  clamped != 0: the clamped SwiGLU on interleaved pairs
+ * (alpha, limit) with the biases gu_bias [G, 2*half] and dn_bias [G, H] (may be NULL) added by the
+ * GEMMs' stores; otherwise silu(gate) * up on concatenated halves.  x_t [K, M] and h_t [half, M] bytes with
+ * scales [M/128, K] and [M/128, half]: the transposed activations that the weight gradients read.  Not
+ * needed afterwards: composed_map int32 [M] (with expand_idx), x_fp8 [M, K] and h_fp8 [M, half] with
+ * their 1x128 scales. */
+typedef struct {
+  const void* x; int64_t x_rows, ldx;
+  int64_t M, K, half, H, G;
+  const int32_t* offs;
+  const int32_t* row_map;
+  const int64_t* expand_idx; int64_t n_expand;
+  const void* gu_fp8; const float* gu_scale; const void* gu_bias;
+  const void* dn_fp8; const float* dn_scale; const void* dn_bias;
+  void* gate_up;
+  void* out; int64_t out_rows, scatter;
+  int64_t clamped; double alpha, limit;
+  void* x_t; float* x_t_scale; void* h_t; float* h_t_scale;
+  int32_t* composed_map; void* x_fp8; float* x_scale; void* h_fp8; float* h_scale;
+  pt_stream_t stream;
+} pt_experts_forward_args;
+int pt_experts_forward(const pt_experts_forward_args* args /* host */);
+
+/* Backward of the same block, up to the quantised gradient of gate_up: dgu_fp8 [M, 2*half] and dgu_scale
+ * [M, ceil(2*half/128)], from which the input gradient follows with one pt_gemm_m_grouped_nn(_scatter) on
+ * the gate_up weight.  grad_out bf16 [grad_rows, H]; out_map: row_map when the forward scattered its
+ * result (the gradient arrives un-permuted), else NULL; limit_rows != 0: the row count is offs[G-1] (the
+ * forward had a row_map).  dn_dg: the down weight, dn_forward_layout != 0 for the forward-layout tensor, 0
+ * for the transposed twin.  dy_t [H, M] and dgu_t [2*half, M] bytes with scales [M/128, .]: the transposed
+ * gradients of the weight-gradient GEMMs (kept by the caller when it runs those later).  Not needed
+ * afterwards: dy_fp8 [M, H] with 1x128 scales, grad_h bf16 [M, half], col_sum fp32 [M/128, 2*half].
+ * dw_down [G, H, half] bf16 (NULL = not computed here), dw_gate_up [G, 2*half, K] or, when dw_up is given,
+ * [G, half, K] each (pt_experts_weight_gradient only); *_add != 0: added to what is there.  d_gu_bias / d_dn_bias [G, 2*half] /
+ * [G, H] in the types given: NULL = none. */
+typedef struct {
+  const void* grad_out; int64_t grad_rows;
+  int64_t M, K, half, H, G;
+  const int32_t* offs;
+  const int32_t* out_map; int64_t limit_rows;
+  const void* dn_dg; const float* dn_dg_scale; int64_t dn_forward_layout;
+  const void* gate_up;
+  const void* x_t; const float* x_t_scale; const void* h_t; const float* h_t_scale;
+  void* dgu_fp8; float* dgu_scale;
+  void* dy_t; float* dy_t_scale; void* dgu_t; float* dgu_t_scale;
+  void* dy_fp8; float* dy_scale; void* grad_h; float* col_sum;
+  void* dw_down; int64_t dw_down_add;
+  void* dw_gate_up; int64_t dw_gate_up_add;
+  void* dw_up; int64_t dw_up_add;
+  int64_t clamped; double alpha, limit;
+  void* d_gu_bias; int64_t d_gu_bias_dtype;
+  void* d_dn_bias; int64_t d_dn_bias_dtype;
+  pt_stream_t stream;
+} pt_experts_backward_args;
+int pt_experts_backward(const pt_experts_backward_args* args /* host */);
+/* The gate_up weight gradient of the same block from the same arguments (dw_gate_up, dw_up): the last
+ * launch of a backward, after the caller has queued the input gradient. */
+int pt_experts_weight_gradient(const pt_experts_backward_args* args /* host */);
+/* Forward of a dense FP8 linear (fp8_act_weight_gemm, operators/linear.py:44-60): x [M, K] in dtype,
+ * y [M, N] in y_dtype (PT_BF16 or PT_F32); x_t (row pitch ld_t >= M bytes) and x_t_scale are the transposed
+ * operand the weight gradient reads.  K % 16 == 0. */
+typedef struct {
+  const void* x; int64_t dtype, M, K, ldx;
+  const void* w_fp8; const float* w_scale; int64_t N;
+  void* y; int64_t y_dtype;
+  void* x_t; int64_t ld_t; float* x_t_scale;
+  int64_t splits, split_len;
+  void* workspace;
+  pt_stream_t stream;
+} pt_linear_forward_args;
+int64_t pt_linear_forward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t splits);
+int pt_linear_forward(const pt_linear_forward_args* args /* host */);
+
+/* Backward (fp8_dgrad_wgrad, operators/linear.py:63-83): grad [M, N] in dtype -> grad_x [M, K] through
+ * the transposed weight w_t [K, N], grad_w [N, K] through x_t [K, M]; both in out_dtype.  N % 16 == 0;
+ * M % 16 == 0 unless x_t was written by pt_linear_forward with a pitch of at least M rounded up to 16
+ * (its columns past M are zero).  splits / split_len per GEMM: the reduction ranges of
+ * pt_gemm_nt_dense_splitk (1 = not split). */
+typedef struct {
+  const void* grad; int64_t dtype, M, N, ldg;
+  const void* w_t_fp8; const float* w_t_scale; int64_t K;
+  const void* x_t; int64_t ld_xt; const float* x_t_scale;
+  void* grad_x; void* grad_w; int64_t out_dtype;
+  int64_t x_splits, x_split_len, w_splits, w_split_len;
+  void* workspace;
+  pt_stream_t stream;
+} pt_linear_backward_args;
+int64_t pt_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t x_splits, int64_t w_splits);
+int pt_linear_backward(const pt_linear_backward_args* args /* host */);
+
+/* Measurement: `fn`, when not NULL, is called on the host before (begin = 1) and after (begin = 0) every
+ * entry point that the whole-step functions above run, with its name and {M, N, K} of a GEMM or
+ * {rows, columns, source rows} of a quantisation. */
+typedef void (*pt_observer_t)(const char* name, int begin, int64_t a, int64_t b, int64_t c);
+void pt_set_observer(pt_observer_t fn);
 
 /* In-place fused cross-entropy with mean reduction (CrossEntropy.forward and its Triton kernel
  * cross_entropy_fwd, operators/cross_entropy.py:16-78,86-118): logits [N,V] in dtype are

@@ -17,6 +17,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("PITHTRAIN_HIP_LIB") or os.path.join(_HERE, "libpithtrain_hip.so")
 
 PT_BF16, PT_F32, PT_F16 = 0, 1, 2
+PT_QUANT_WEIGHTS_MAX = 4
 PT_CH_ROWMAJOR, PT_CH_TRANSPOSED, PT_CH_KMAJOR = 0, 1, 2
 
 _DTYPE_CODE = {torch.bfloat16: PT_BF16, torch.float32: PT_F32, torch.float16: PT_F16}
@@ -40,6 +41,7 @@ SIGNATURES = {
     "pt_quant_blockwise_transpose_batched": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, P, P, P, P]),
     "pt_quant_blockwise_transpose_batched_into": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, I64, P, I64, P, I64, I64, P, I64,
                                                           I64, P]),
+    "pt_quant_weights": (c_int, [c_char_p, I32, c_int, P]),
     "pt_gemm_nt_dense": (c_int, [P, P, P, P, P, c_int, I64, I64, I64, P]),
     "pt_gemm_nt_dense_splitk": (c_int, [P, P, P, P, P, I32, I64, I64, I64, I64, P]),
     "pt_gemm_nt_dense_ld": (c_int, [P, I64, P, P, I64, P, P, c_int, I64, I64, I64, P]),
@@ -53,6 +55,7 @@ SIGNATURES = {
     "pt_gemm_m_grouped_nt_scatter": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P]),
     "pt_gemm_k_grouped_wgrad": (c_int, [P, P, P, P, P, c_int, c_int, P, I32, I64, I64, I64, P]),
     "pt_gemm_k_grouped_wgrad_ld": (c_int, [P, P, I64, P, P, I64, P, c_int, c_int, P, I32, I64, I64, I64, P]),
+    "pt_gemm_k_grouped_wgrad_pair": (c_int, [P, P, P, P, P, P, I64, c_int, c_int, P, I32, I64, I64, I64, P]),
     "pt_gemm_select_kernel": (c_int, [ctypes.c_char_p]),
     "pt_moe_combine_fwd": (c_int, [P, I64, P, P, I64, P, I64, I64, I32, I64, c_int, P]),
     "pt_moe_combine_bwd": (c_int, [P, I64, P, I64, P, P, I64, P, I64, I32, I64, c_int, P]),
@@ -85,6 +88,16 @@ SIGNATURES = {
     "pt_indexed_bias_add_fwd": (c_int, [P, P, P, P, I64, I64, c_int, P]),
     "pt_segment_sum": (c_int, [P, P, I32, P, I64, I64, c_int, c_int, P]),
     "pt_segment_sum_rows": (c_int, [P, I64, P, P, I32, P, I64, I64, c_int, c_int, P]),
+    "pt_segment_sum_tiles": (c_int, [P, P, I32, I32, P, I64, I64, c_int, P]),
+    # whole steps: one host block of 8-byte fields (struct.pack) instead of an argument each
+    "pt_experts_forward": (c_int, [c_char_p]),
+    "pt_experts_backward": (c_int, [c_char_p]),
+    "pt_experts_weight_gradient": (c_int, [c_char_p]),
+    "pt_linear_forward_workspace_bytes": (I64, [I64, I64, I64, I64]),
+    "pt_linear_forward": (c_int, [c_char_p]),
+    "pt_linear_backward_workspace_bytes": (I64, [I64, I64, I64, I64, I64]),
+    "pt_linear_backward": (c_int, [c_char_p]),
+    "pt_set_observer": (None, [P]),
 }
 
 _lib = None
@@ -126,7 +139,13 @@ def ptr(t: torch.Tensor | None):
 
 
 def stream_ptr(device=None):
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle on ``device``, without building a ``torch.cuda.Stream`` for it."""
+    index = device.index if isinstance(device, torch.device) else None
+    if index is None:
+        if device is not None and not isinstance(device, torch.device):
+            return torch.cuda.current_stream(device).cuda_stream
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def require_cuda(*tensors: torch.Tensor):

@@ -197,12 +197,13 @@ __global__ __launch_bounds__(256) void bias_add_kernel(const char* x, const char
 // i.e. the sum runs over the grouped order while x stays un-permuted.
 template <typename S, typename O>
 __global__ __launch_bounds__(256) void segment_sum_kernel(const char* x, const int32_t* offs, char* out, int64_t M,
-                                                          int64_t H, int vec, const int32_t* row_index, int64_t x_rows) {
+                                                          int64_t H, int vec, const int32_t* row_index, int64_t x_rows,
+                                                          int32_t unit) {
   __shared__ float s[16][129];
   const int g = blockIdx.y;
   const int cc = threadIdx.x & 15, rl = threadIdx.x >> 4;
-  int64_t start = g == 0 ? 0 : (int64_t)offs[g - 1];
-  int64_t end = offs[g];
+  int64_t start = g == 0 ? 0 : (int64_t)offs[g - 1] / unit;
+  int64_t end = offs[g] / unit;
   if (end > M) end = M;
   if (start > M) start = M;
   const int64_t h0 = (int64_t)blockIdx.x * 128 + cc * 8;
@@ -391,13 +392,13 @@ extern "C" int pt_indexed_bias_add_fwd(const void* x, const void* bias, const in
 }
 
 static int segment_sum_impl(const void* x, int64_t x_rows, const int32_t* row_index, const int32_t* offs, int32_t num_groups,
-                            void* out, int64_t M, int64_t H, int dtype, int out_dtype, pt_stream_t stream) {
+                            void* out, int64_t M, int64_t H, int dtype, int out_dtype, pt_stream_t stream, int32_t unit = 1) {
   if (num_groups == 0 || H == 0) return PT_OK;
   PT_REQUIRE(num_groups > 0 && num_groups <= 65535 && H > 0 && M >= 0 && x_rows >= 0 && x && offs && out, "segment_sum: bad arguments");
   const int vec = (H % 8 == 0) && aligned16(x);
   dim3 grid((unsigned)cdiv(H, 128), (unsigned)num_groups);
   hipStream_t s = (hipStream_t)stream;
-#define PT_SEG(SI, SO) segment_sum_kernel<SI, SO><<<grid, 256, 0, s>>>((const char*)x, offs, (char*)out, M, H, vec, row_index, x_rows)
+#define PT_SEG(SI, SO) segment_sum_kernel<SI, SO><<<grid, 256, 0, s>>>((const char*)x, offs, (char*)out, M, H, vec, row_index, x_rows, unit)
   if (dtype == PT_BF16 && out_dtype == PT_BF16) PT_SEG(st_bf16, st_bf16);
   else if (dtype == PT_BF16 && out_dtype == PT_F32) PT_SEG(st_bf16, st_f32);
   else if (dtype == PT_F16 && out_dtype == PT_F16) PT_SEG(st_f16, st_f16);
@@ -419,4 +420,10 @@ extern "C" int pt_segment_sum_rows(const void* x, int64_t x_rows, const int32_t*
                                    pt_stream_t stream) {
   PT_REQUIRE(row_index, "segment_sum_rows: null row_index");
   return segment_sum_impl(x, x_rows, row_index, offs, num_groups, out, M, H, dtype, out_dtype, stream);
+}
+
+extern "C" int pt_segment_sum_tiles(const float* x, const int32_t* offs, int32_t unit, int32_t num_groups, void* out, int64_t M,
+                                    int64_t H, int out_dtype, pt_stream_t stream) {
+  PT_REQUIRE(unit > 0, "segment_sum_tiles: unit must be positive");
+  return segment_sum_impl(x, M, nullptr, offs, num_groups, out, M, H, PT_F32, out_dtype, stream, unit);
 }

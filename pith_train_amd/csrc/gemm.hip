@@ -565,7 +565,8 @@ extern "C" int pt_gemm_m_grouped_nt_bias(const void* a_fp8, const float* a_scale
 
 static int gemm_k_grouped_wgrad_impl(const void* dy_t_fp8, const float* dy_scale, int64_t ld_dy_scale, const void* x_t_fp8,
                                      const float* x_scale, int64_t ld_x_scale, void* out, int out_dtype, int accumulate,
-                                     const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, pt_stream_t stream) {
+                                     const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, pt_stream_t stream,
+                                     void* out2 = nullptr, int64_t split = 0) {
   PT_REQUIRE(M >= 0 && N >= 0 && K >= 0 && G > 0, "gemm_k_grouped_wgrad: bad sizes");
   if (N == 0 || K == 0) return PT_OK;
   PT_REQUIRE(M % 128 == 0, "gemm_k_grouped_wgrad: M=%lld must be a multiple of 128", (long long)M);
@@ -581,11 +582,27 @@ static int gemm_k_grouped_wgrad_impl(const void* dy_t_fp8, const float* dy_scale
   g.out = out; g.ldo = K; g.out_dtype = out_dtype; g.accumulate = accumulate;
   g.rows_a = N; g.rows_b = K; g.red = M; g.mode = GEMM_K_GROUPED; g.offs = offs; g.G = G;
   g.out_stride_g = N * K;
+  if (split) { g.out2 = out2; g.split_row = split; g.out_stride_g = split * K; g.out2_stride_g = (N - split) * K; }
   g.a_bytes = N * M; g.b_bytes = K * M;
   g.sa_bytes = ((M / 128 - 1) * ld_dy_scale + N) * 4; g.sb_bytes = ((M / 128 - 1) * ld_x_scale + K) * 4;
   g.tiles_a = (int)cdiv(N, 128); g.tiles_b = (int)cdiv(K, 128);
   g.total_tiles = (int64_t)g.tiles_a * g.tiles_b * G;
   return dispatch_gemm(g, (hipStream_t)stream);
+}
+
+extern "C" int pt_gemm_k_grouped_wgrad_pair(const void* dy_t_fp8, const float* dy_scale, const void* x_t_fp8, const float* x_scale,
+                                            void* out0, void* out1, int64_t split, int out_dtype, int accumulate,
+                                            const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, pt_stream_t stream) {
+  PT_REQUIRE(split > 0 && split < N && split % 128 == 0 && out1, "gemm_k_grouped_wgrad_pair: split=%lld of N=%lld rows", (long long)split, (long long)N);
+  const int64_t lim = (1ll << 31) - 1;
+  // the tile-per-workgroup kernel (extents past 31 bits) has one output; the wide stores want both aligned alike
+  const bool one = gemm_impl() != IMPL_TILE && N * M < lim && K * M < lim && M < lim && N * K * 4 < (1ll << 32) &&
+                   (M / 128) * N * 4 < lim && (M / 128) * K * 4 < lim && al16(out0) == al16(out1) &&
+                   (split * K) % 8 == ((N - split) * K) % 8;
+  if (one) return gemm_k_grouped_wgrad_impl(dy_t_fp8, dy_scale, N, x_t_fp8, x_scale, K, out0, out_dtype, accumulate, offs, G, M, N, K, stream, out1, split);
+  if (int rc = gemm_k_grouped_wgrad_impl(dy_t_fp8, dy_scale, N, x_t_fp8, x_scale, K, out0, out_dtype, accumulate, offs, G, M, split, K, stream)) return rc;
+  return gemm_k_grouped_wgrad_impl((const uint8_t*)dy_t_fp8 + split * M, dy_scale + split, N, x_t_fp8, x_scale, K, out1, out_dtype,
+                                   accumulate, offs, G, M, N - split, K, stream);
 }
 
 extern "C" int pt_gemm_k_grouped_wgrad(const void* dy_t_fp8, const float* dy_scale, const void* x_t_fp8, const float* x_scale,

@@ -24,6 +24,9 @@ struct GemmArgs {
   int64_t out_rows;                       // rows of the output when out_row_index is given
   const void* bias;                       // m-grouped only: [G, rows_b] in the output's type, row g added to the rows of group g
   int64_t split_len;                      // k-grouped with offs == null: group g reduces over [g, g + 1) * split_len (split-K)
+  void* out2; int64_t split_row;          // k-grouped: result rows from split_row on (a multiple of 128; 0 = none) go to out2, a second
+                                          // parameter's gradient (group stride out2_stride_g) whose row 0 is row split_row
+  int64_t out2_stride_g;
   int b_kmajor;                           // m-grouped, row-split kernel: b is [red, rows_b] per group (row pitch ldb) instead of [rows_b, red]
 };
 

@@ -421,7 +421,7 @@ __device__ __forceinline__ void pin_acc(v16f& a) {
 // tile).  `stg` is the wave's 2 KiB LDS staging area.  PIN != 0: the accumulators were produced by
 // inline-assembly MFMAs; each block is handed to the compiler only right before its store, so
 // that it is converted and copied out one block at a time.
-template <int MODE, int TM, int TN, bool ACC, int PIN>
+template <int MODE, int TM, int TN, bool ACC, int PIN, bool PAIR = false>
 __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& p, const Tile& T, int wm0, int wn0, int lane,
                                            uint8_t* stg) {
   const uint32_t esz = p.out_dtype == PT_F32 ? 4 : 2;
@@ -433,8 +433,17 @@ __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& 
   // (PT_GEMM_ABLATE_STORES, measurement builds only: it ends before the first, so every store
   // instruction runs and nothing is written.)
   char* outp = (char*)p.out + (MODE == GEMM_K_GROUPED ? (int64_t)T.g * p.out_stride_g * esz : 0);
-  const __amdgpu_buffer_rsrc_t rs_out = __builtin_amdgcn_make_buffer_rsrc(outp, 0, kAblateStores ? 0 : (int)((uint32_t)T.a_lim * pitch), kRsrcFlags);
-  const uint32_t s_tile = (uint32_t)(T.a_row0 + wm0) * pitch + (uint32_t)(T.b_row0 + wn0) * esz;
+  int row0 = T.a_row0 + wm0, row_lim = T.a_lim;
+  if (MODE == GEMM_K_GROUPED && PAIR && p.split_row) {  // a wave's rows lie on one side of the split
+    if (row0 >= (int)p.split_row) {
+      outp = (char*)p.out2 + (int64_t)T.g * p.out2_stride_g * esz;
+      row0 -= (int)p.split_row; row_lim -= (int)p.split_row;
+    } else {
+      row_lim = row_lim < (int)p.split_row ? row_lim : (int)p.split_row;
+    }
+  }
+  const __amdgpu_buffer_rsrc_t rs_out = __builtin_amdgcn_make_buffer_rsrc(outp, 0, kAblateStores ? 0 : (int)((uint32_t)row_lim * pitch), kRsrcFlags);
+  const uint32_t s_tile = (uint32_t)row0 * pitch + (uint32_t)(T.b_row0 + wn0) * esz;
   const int colw = T.b_row0 + wn0 + (lane & 31);
   static_assert(TN % 2 == 0, "the wide stores take column blocks in pairs");
   if (MODE == GEMM_M_GROUPED && p.out_row_index) {

@@ -42,7 +42,8 @@ namespace pt {
 
 // BT: the b operand is given reduction-major, [red][rows_b] with row pitch ldb (the forward layout of
 // a weight, read by its input-gradient GEMM), instead of [rows_b][red].
-template <int MODE, int BM, int BN, int WGM, int WGN, bool ACC, bool BT = false>
+// PAIR (k-grouped): the result rows from split_row on go to a second output.
+template <int MODE, int BM, int BN, int WGM, int WGN, bool ACC, bool BT = false, bool PAIR = false>
 __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel(GemmArgs p) {
   constexpr int NW = WGM * WGN;
   constexpr int WM = BM / WGM, WN = BN / WGN;
@@ -396,18 +397,18 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
     // ---- epilogue ----
     if (!wave_active) continue;
     if (MODE == GEMM_K_GROUPED && nk == 0 && ACC) continue;
-    store_tile<MODE, TM, TN, ACC, 2>(acc, p, C, wm0, wn0, lane, lds + NS * STAGE + SC_RING * (BM + BN) * 4 + 512 + wave * 2048);
+    store_tile<MODE, TM, TN, ACC, 2, PAIR>(acc, p, C, wm0, wn0, lane, lds + NS * STAGE + SC_RING * (BM + BN) * 4 + 512 + wave * 2048);
   }
   wait_all_vmem();  // nothing may still be writing into this workgroup's LDS when it retires
 }
 
-template <int MODE, int BM, int BN, int WGM, int WGN, bool ACC, bool BT = false>
+template <int MODE, int BM, int BN, int WGM, int WGN, bool ACC, bool BT = false, bool PAIR = false>
 static int launch_one(GemmArgs a, hipStream_t stream) {
   // LDS: two operand stages, two stages of scales, a sink line, 2 KiB of result staging per wave
   constexpr size_t lds = (size_t)2 * (BM + BN) * 128 + 2 * (BM + BN) * 4 + 512 + (size_t)WGM * WGN * 2048;
   static bool attr_set = false;
   const int64_t upper = plan_tiles(a, BM, BN);
-  return launch_persistent_grid(fp8_gemm_nt_rowsplit_kernel<MODE, BM, BN, WGM, WGN, ACC, BT>, "fp8_gemm_nt_rowsplit_kernel", a, upper, WGM * WGN * 64, lds, attr_set, stream);
+  return launch_persistent_grid(fp8_gemm_nt_rowsplit_kernel<MODE, BM, BN, WGM, WGN, ACC, BT, PAIR>, "fp8_gemm_nt_rowsplit_kernel", a, upper, WGM * WGN * 64, lds, attr_set, stream);
 }
 
 template <int BM, int BN, int WGM, int WGN>
@@ -418,6 +419,9 @@ static int launch_mode(const GemmArgs& a, hipStream_t stream) {
       return a.b_kmajor ? launch_one<GEMM_M_GROUPED, BM, BN, WGM, WGN, false, true>(a, stream)
                         : launch_one<GEMM_M_GROUPED, BM, BN, WGM, WGN, false>(a, stream);
     default:
+      if (a.split_row)
+        return a.accumulate ? launch_one<GEMM_K_GROUPED, BM, BN, WGM, WGN, true, false, true>(a, stream)
+                            : launch_one<GEMM_K_GROUPED, BM, BN, WGM, WGN, false, false, true>(a, stream);
       return a.accumulate ? launch_one<GEMM_K_GROUPED, BM, BN, WGM, WGN, true>(a, stream)
                           : launch_one<GEMM_K_GROUPED, BM, BN, WGM, WGN, false>(a, stream);
   }

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_small_kernel(GemmArgs p) {
   }
   wait_all_vmem();  // nothing may still be writing into this workgroup's LDS when it retires
   if (MODE == GEMM_K_GROUPED && nk == 0 && ACC) return;
-  store_tile<MODE, TM, TN, ACC, 0>(acc, p, T, wm0, wn0, lane, lds + NS * STAGE + NS * (BM + BN) * 4 + 256 + wave * 2048);
+  store_tile<MODE, TM, TN, ACC, 0, MODE == GEMM_K_GROUPED>(acc, p, T, wm0, wn0, lane, lds + NS * STAGE + NS * (BM + BN) * 4 + 256 + wave * 2048);
 }
 
 template <int MODE, int BM, bool ACC, bool BT>

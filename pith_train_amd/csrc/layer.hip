@@ -1,0 +1,205 @@
+// Whole steps as one host call (no kernels here): the forward and the backward of an expert block and
+// of a dense linear queue their launches from this file.
+//
+// A layer with few tokens is bound by the host: a launch costs about 3.5 us of host time, and every
+// separate call from Python added 6-10 us of argument conversion, allocation and stream lookup to it
+// (toy layer, 22 calls: 400 us a step against 170 us of kernels).  Here a step is one call with one
+// block of arguments.
+#include "common.h"
+
+namespace pt {
+
+static int64_t up(int64_t x) { return (x + 255) & ~(int64_t)255; }
+
+static pt_observer_t g_observer = nullptr;
+
+// runs one entry point, with the observer around it, and returns from the caller on failure
+#define PT_STEP(NAME, A, B, C, ...)                         \
+  do {                                                      \
+    if (g_observer) g_observer(#NAME, 1, (A), (B), (C));    \
+    if (int rc_ = NAME(__VA_ARGS__)) return rc_;            \
+    if (g_observer) g_observer(#NAME, 0, (A), (B), (C));    \
+  } while (0)
+
+// Carves consecutive 256-byte aligned pieces out of a buffer (a null buffer gives offsets).
+struct Carve {
+  uintptr_t p;
+  explicit Carve(const void* base) : p((uintptr_t)base) {}
+  void* bytes(int64_t n) { void* r = (void*)p; p += (uintptr_t)up(n); return r; }
+  float* floats(int64_t n) { return (float*)bytes(4 * n); }
+};
+
+}  // namespace pt
+
+using namespace pt;
+
+extern "C" void pt_set_observer(pt_observer_t fn) { g_observer = fn; }
+
+extern "C" int pt_experts_forward(const pt_experts_forward_args* args) {
+  PT_REQUIRE(args, "experts_forward: null arguments");
+  const pt_experts_forward_args& a = *args;
+  PT_REQUIRE(a.M >= 0 && a.M % 128 == 0 && a.K > 0 && a.half > 0 && a.H > 0 && a.G > 0 && a.G < (1ll << 31), "experts_forward: bad sizes");
+  PT_REQUIRE(a.offs && a.gate_up && a.out && a.x_fp8 && a.x_scale && a.x_t && a.x_t_scale && a.h_fp8 && a.h_scale && a.h_t && a.h_t_scale,
+             "experts_forward: null pointer");
+  PT_REQUIRE(!a.expand_idx || a.composed_map, "experts_forward: expand_idx needs composed_map");
+  PT_REQUIRE(a.row_map || (!a.expand_idx && !a.scatter), "experts_forward: expand_idx and scatter need row_map");
+  if (a.M == 0) return PT_OK;
+  const int32_t G = (int32_t)a.G;
+  const int32_t* limit = a.row_map ? a.offs + G - 1 : nullptr;  // rows past it hold nothing
+  const int32_t* in_map = a.row_map;
+  if (a.expand_idx) {
+    PT_STEP(pt_compose_row_map, a.M, 0, 0, a.row_map, a.M, a.expand_idx, a.n_expand, a.x_rows, a.composed_map, a.stream);
+    in_map = a.composed_map;
+  }
+  if (in_map)
+    PT_STEP(pt_quant_rowwise_colwise_rows, a.M, a.K, a.x_rows, a.x, PT_BF16, a.M, a.K, a.ldx, in_map, a.x_fp8, a.x_scale, a.x_t, a.x_t_scale,
+            PT_CH_TRANSPOSED, a.offs, G, a.stream);
+  else
+    PT_STEP(pt_quant_rowwise_colwise, a.M, a.K, a.x_rows, a.x, PT_BF16, a.M, a.K, a.ldx, a.x_fp8, a.x_scale, a.x_t, a.x_t_scale, PT_CH_TRANSPOSED,
+            nullptr, 0, a.stream);
+  if (a.gu_bias)
+    PT_STEP(pt_gemm_m_grouped_nt_bias, a.M, 2 * a.half, a.K, a.x_fp8, a.x_scale, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M,
+            2 * a.half, a.K, a.gu_bias, a.stream);
+  else
+    PT_STEP(pt_gemm_m_grouped_nt, a.M, 2 * a.half, a.K, a.x_fp8, a.x_scale, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M,
+            2 * a.half, a.K, a.stream);
+  if (a.clamped)
+    PT_STEP(pt_clamped_swiglu_quant_rowwise_colwise, a.M, a.half, 0, a.gate_up, a.M, a.half, 2 * a.half, (float)a.alpha,
+            (float)a.limit, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit, a.stream);
+  else
+    PT_STEP(pt_silu_mul_quant_rowwise_colwise, a.M, a.half, 0, a.gate_up, a.M, a.half, 2 * a.half, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit,
+            a.stream);
+  if (a.scatter && a.dn_bias)
+    PT_STEP(pt_gemm_m_grouped_nt_scatter_bias, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M,
+            a.H, a.half, a.row_map, a.out_rows, a.dn_bias, a.stream);
+  else if (a.scatter)
+    PT_STEP(pt_gemm_m_grouped_nt_scatter, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H,
+            a.half, a.row_map, a.out_rows, a.stream);
+  else if (a.dn_bias)
+    PT_STEP(pt_gemm_m_grouped_nt_bias, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H,
+            a.half, a.dn_bias, a.stream);
+  else
+    PT_STEP(pt_gemm_m_grouped_nt, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H, a.half,
+            a.stream);
+  return PT_OK;
+}
+
+extern "C" int pt_experts_backward(const pt_experts_backward_args* args) {
+  PT_REQUIRE(args, "experts_backward: null arguments");
+  const pt_experts_backward_args& a = *args;
+  PT_REQUIRE(a.M >= 0 && a.M % 128 == 0 && a.K > 0 && a.half > 0 && a.H > 0 && a.G > 0 && a.G < (1ll << 31), "experts_backward: bad sizes");
+  PT_REQUIRE(a.grad_out && a.offs && a.gate_up && a.h_t && a.h_t_scale && a.dy_fp8 && a.dy_scale && a.dy_t && a.dy_t_scale && a.grad_h && a.dgu_fp8 &&
+                 a.dgu_scale && a.dgu_t && a.dgu_t_scale, "experts_backward: null pointer");
+  if (a.M == 0) return PT_OK;
+  const int32_t G = (int32_t)a.G;
+  const int32_t* limit = a.limit_rows ? a.offs + G - 1 : nullptr;
+  if (a.out_map)
+    PT_STEP(pt_quant_rowwise_colwise_rows, a.M, a.H, a.grad_rows, a.grad_out, PT_BF16, a.M, a.H, a.H, a.out_map, a.dy_fp8, a.dy_scale, a.dy_t,
+            a.dy_t_scale, PT_CH_TRANSPOSED, a.offs, G, a.stream);
+  else
+    PT_STEP(pt_quant_rowwise_colwise, a.M, a.H, a.grad_rows, a.grad_out, PT_BF16, a.M, a.H, a.H, a.dy_fp8, a.dy_scale, a.dy_t, a.dy_t_scale,
+            PT_CH_TRANSPOSED, nullptr, 0, a.stream);
+  if (a.d_dn_bias) {
+    if (a.out_map)
+      PT_STEP(pt_segment_sum_rows, a.M, a.H, 0, a.grad_out, a.grad_rows, a.out_map, a.offs, G, a.d_dn_bias, a.M, a.H, PT_BF16,
+              (int)a.d_dn_bias_dtype, a.stream);
+    else
+      PT_STEP(pt_segment_sum, a.M, a.H, 0, a.grad_out, a.offs, G, a.d_dn_bias, a.M, a.H, PT_BF16, (int)a.d_dn_bias_dtype, a.stream);
+  }
+  if (a.dn_forward_layout)
+    PT_STEP(pt_gemm_m_grouped_nn, a.M, a.half, a.H, a.dy_fp8, a.dy_scale, a.dn_dg, a.dn_dg_scale, a.grad_h, PT_BF16, a.offs, G, a.M, a.half, a.H,
+            a.stream);
+  else
+    PT_STEP(pt_gemm_m_grouped_nt, a.M, a.half, a.H, a.dy_fp8, a.dy_scale, a.dn_dg, a.dn_dg_scale, a.grad_h, PT_BF16, a.offs, G, a.M, a.half, a.H,
+            a.stream);
+  if (a.dw_down)
+    PT_STEP(pt_gemm_k_grouped_wgrad, a.M, a.H, a.half, a.dy_t, a.dy_t_scale, a.h_t, a.h_t_scale, a.dw_down, PT_BF16, (int)a.dw_down_add, a.offs, G,
+            a.M, a.H, a.half, a.stream);
+  if (a.clamped)
+    PT_STEP(pt_clamped_swiglu_bwd_quant_rowwise_colwise, a.M, a.half, 0, a.grad_h, a.half, a.gate_up, 2 * a.half, a.M, a.half,
+            (float)a.alpha, (float)a.limit, a.dgu_fp8, a.dgu_scale, a.dgu_t, a.dgu_t_scale, a.col_sum, limit, a.stream);
+  else
+    PT_STEP(pt_silu_mul_bwd_quant_rowwise_colwise, a.M, a.half, 0, a.grad_h, a.half, a.gate_up, 2 * a.half, a.M, a.half, a.dgu_fp8, a.dgu_scale,
+            a.dgu_t, a.dgu_t_scale, limit, a.stream);
+  if (a.d_gu_bias)  // groups are whole 128-row tiles: their ends in tiles index the per-tile column sums
+    PT_STEP(pt_segment_sum_tiles, a.M / 128, 2 * a.half, 0, a.col_sum, a.offs, 128, G, a.d_gu_bias, a.M / 128, 2 * a.half,
+            (int)a.d_gu_bias_dtype, a.stream);
+  return PT_OK;
+}
+
+extern "C" int pt_experts_weight_gradient(const pt_experts_backward_args* args) {
+  PT_REQUIRE(args, "experts_weight_gradient: null arguments");
+  const pt_experts_backward_args& a = *args;
+  PT_REQUIRE(a.M >= 0 && a.M % 128 == 0 && a.offs && a.x_t && a.x_t_scale && a.dgu_t && a.dgu_t_scale && a.dw_gate_up, "experts_weight_gradient: bad arguments");
+  const int32_t G = (int32_t)a.G;
+  if (!a.dw_up)
+    PT_STEP(pt_gemm_k_grouped_wgrad, a.M, 2 * a.half, a.K, a.dgu_t, a.dgu_t_scale, a.x_t, a.x_t_scale, a.dw_gate_up, PT_BF16, (int)a.dw_gate_up_add,
+            a.offs, G, a.M, 2 * a.half, a.K, a.stream);
+  else if ((a.dw_gate_up_add != 0) == (a.dw_up_add != 0) && a.half % 128 == 0)
+    PT_STEP(pt_gemm_k_grouped_wgrad_pair, a.M, 2 * a.half, a.K, a.dgu_t, a.dgu_t_scale, a.x_t, a.x_t_scale, a.dw_gate_up, a.dw_up, a.half, PT_BF16,
+            (int)a.dw_up_add, a.offs, G, a.M, 2 * a.half, a.K, a.stream);
+  else {
+    PT_STEP(pt_gemm_k_grouped_wgrad_ld, a.M, a.half, a.K, a.dgu_t, a.dgu_t_scale, 2 * a.half, a.x_t, a.x_t_scale, a.K, a.dw_gate_up, PT_BF16,
+            (int)a.dw_gate_up_add, a.offs, G, a.M, a.half, a.K, a.stream);
+    PT_STEP(pt_gemm_k_grouped_wgrad_ld, a.M, a.half, a.K, (const uint8_t*)a.dgu_t + a.half * a.M, a.dgu_t_scale + a.half, 2 * a.half, a.x_t,
+            a.x_t_scale, a.K, a.dw_up, PT_BF16, (int)a.dw_up_add, a.offs, G, a.M, a.half, a.K, a.stream);
+  }
+  return PT_OK;
+}
+
+// out[m, n] = a b^T, its reduction cut into ranges when splits > 1 (fp32 slabs in `slabs`)
+static int dense_gemm(const void* a, int64_t lda, const float* as, const void* b, int64_t ldb, const float* bs, void* out, int out_dtype,
+                      int64_t M, int64_t N, int64_t K, int64_t splits, int64_t split_len, float* slabs, pt_stream_t stream) {
+  if (splits > 1) {
+    PT_STEP(pt_gemm_nt_dense_splitk_ld, M, N, K, a, lda, as, b, ldb, bs, slabs, (int32_t)splits, split_len, M, N, K, stream);
+    PT_STEP(pt_sum_partials, M, N, splits, slabs, (int32_t)splits, M * N, out, out_dtype, stream);
+  } else {
+    PT_STEP(pt_gemm_nt_dense_ld, M, N, K, a, lda, as, b, ldb, bs, out, out_dtype, M, N, K, stream);
+  }
+  return PT_OK;
+}
+
+extern "C" int64_t pt_linear_forward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t splits) {
+  return up(M * K) + up(4 * M * cdiv(K, 128)) + (splits > 1 ? up(4 * splits * M * N) : 0);
+}
+
+extern "C" int pt_linear_forward(const pt_linear_forward_args* args) {
+  PT_REQUIRE(args, "linear_forward: null arguments");
+  const pt_linear_forward_args& a = *args;
+  PT_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0 && a.x && a.workspace, "linear_forward: bad arguments");
+  Carve ws(a.workspace);
+  void* x_fp8 = ws.bytes(a.M * a.K);
+  float* x_s = ws.floats(a.M * cdiv(a.K, 128));
+  PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, x_fp8, x_s, a.x_t, a.ld_t,
+          a.x_t_scale, a.stream);
+  return dense_gemm(x_fp8, a.K, x_s, a.w_fp8, a.K, a.w_scale, a.y, (int)a.y_dtype, a.M, a.N, a.K, a.splits, a.split_len,
+                    (float*)(void*)ws.p, a.stream);
+}
+
+// workspace: gradient bytes and scales | its transposed form and scales | slabs of whichever GEMM is split
+extern "C" int64_t pt_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t x_splits, int64_t w_splits) {
+  const int64_t sx = x_splits > 1 ? 4 * x_splits * M * K : 0, sw = w_splits > 1 ? 4 * w_splits * N * K : 0;
+  return up(M * N) + up(4 * M * cdiv(N, 128)) + up(N * (M + 256)) + up(4 * N * cdiv(M, 128)) + up(sx > sw ? sx : sw);
+}
+
+extern "C" int pt_linear_backward(const pt_linear_backward_args* args) {
+  PT_REQUIRE(args, "linear_backward: null arguments");
+  const pt_linear_backward_args& a = *args;
+  PT_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0 && a.grad && a.workspace, "linear_backward: bad arguments");
+  const int64_t red = (a.M + 15) & ~(int64_t)15;  // the weight gradient's reduction, zero-filled to whole 16-byte chunks
+  PT_REQUIRE(a.ld_xt >= red && a.ld_xt % 16 == 0, "linear_backward: the transposed input needs a row pitch of %lld or more, a multiple of 16",
+             (long long)red);
+  // a pitch that is no multiple of 256 bytes spreads the rows of a reduction step over the memory channels
+  const int64_t ld_t = red >= 2048 && red % 256 == 0 ? red + 128 : red;
+  Carve ws(a.workspace);
+  void* g_fp8 = ws.bytes(a.M * a.N);
+  float* g_s = ws.floats(a.M * cdiv(a.N, 128));
+  void* g_t = ws.bytes(a.N * (a.M + 256));
+  float* g_ts = ws.floats(a.N * cdiv(a.M, 128));
+  float* slabs = (float*)(void*)ws.p;
+  PT_STEP(pt_quant_rowwise_transpose_ld, a.M, a.N, a.M, a.grad, (int)a.dtype, a.M, a.N, a.ldg, g_fp8, g_s, g_t, ld_t, g_ts, a.stream);
+  if (int rc = dense_gemm(g_fp8, a.N, g_s, a.w_t_fp8, a.N, a.w_t_scale, a.grad_x, (int)a.out_dtype, a.M, a.K, a.N, a.x_splits,
+                          a.x_split_len, slabs, a.stream)) return rc;
+  return dense_gemm(g_t, ld_t, g_ts, a.x_t, a.ld_xt, a.x_t_scale, a.grad_w, (int)a.out_dtype, a.N, a.K, red, a.w_splits, a.w_split_len,
+                    slabs, a.stream);
+}

@@ -729,6 +729,43 @@ void quant_tile_kernel(QuantArgs p) {
   else      quant_tile_body<T, AM, BMODE, BL, BS, PRO, false>(p, s_colmax, s_blk, s_t, s_colsum, tc, tr, g);
 }
 
+// Several small weights quantised without their twins in one launch (gate, up and down of an expert
+// block): the parts' tiles are numbered one after the other (toy layer: 5.9 us for three weights against
+// 3 x 4.8).  A workgroup finds its part before it can load anything, which costs large weights 2.5 %
+// (128 experts: 316.6 us against 308.9 in two launches); they keep launches of their own.
+struct QuantWeightsArgs {
+  QuantArgs part[PT_QUANT_WEIGHTS_MAX];
+  int64_t end[PT_QUANT_WEIGHTS_MAX];  // number of tiles of the parts up to and including this one
+  int n;
+};
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void quant_weights_kernel(QuantWeightsArgs w) {
+  __shared__ float s_colmax[4][128];
+  __shared__ float s_blk[4];
+  int64_t bid = blockIdx.x;
+  int i = 0;
+  while (i + 1 < w.n && bid >= w.end[i]) ++i;
+  if (i) bid -= w.end[i - 1];
+  const QuantArgs& p = w.part[i];
+  const int tc = (int)(bid % p.tiles_n); bid /= p.tiles_n;
+  const int tr = (int)(bid % p.tiles_m);
+  const int64_t g = bid / p.tiles_m;
+  const bool full = (int64_t)tr * 128 + 128 <= p.M && (int64_t)tc * 128 + 128 <= p.N && p.vec_in && p.vec_out;
+  if (full) quant_tile_body<T, A_BLOCK, B_BLOCK, BL_NONE, BS_MB_N, PRO_NONE, true>(p, s_colmax, s_blk, nullptr, nullptr, tc, tr, g);
+  else      quant_tile_body<T, A_BLOCK, B_BLOCK, BL_NONE, BS_MB_N, PRO_NONE, false>(p, s_colmax, s_blk, nullptr, nullptr, tc, tr, g);
+}
+
+static int launch_quant_weights(const QuantWeightsArgs& w, int dtype, hipStream_t stream) {
+  const int64_t blocks = w.n ? w.end[w.n - 1] : 0;
+  if (blocks == 0) return PT_OK;
+  PT_REQUIRE(blocks < (1ll << 31), "quant: grid too large (%lld tiles)", (long long)blocks);
+  if (dtype == PT_BF16) hipLaunchKernelGGL((quant_weights_kernel<bf16_tag>), dim3((unsigned)blocks), dim3(256), 0, stream, w);
+  else if (dtype == PT_F32) hipLaunchKernelGGL((quant_weights_kernel<float>), dim3((unsigned)blocks), dim3(256), 0, stream, w);
+  else if (dtype == PT_F16) hipLaunchKernelGGL((quant_weights_kernel<f16_tag>), dim3((unsigned)blocks), dim3(256), 0, stream, w);
+  else PT_REQUIRE(false, "quant: unsupported dtype %d (bf16, fp16 and fp32 only)", dtype);
+  return check_launch("quant_weights_kernel");
+}
+
 template <int AM, int BMODE, int BL, int BS>
 static int launch_quant(const QuantArgs& a, int dtype, int64_t G, hipStream_t stream) {
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n * G;
@@ -807,6 +844,13 @@ static int quant_rowwise_colwise_impl(const void* x, int dtype, int64_t M, int64
   PT_REQUIRE(false, "quant_rowwise_colwise: bad ch_layout %d", ch_layout);
 }
 
+// The transposed twin of a dense linear's operand may be written in whole 16-byte chunks when its pitch has
+// room for the last one: the columns past M are then zeros (rows outside the tensor are zero in the
+// tile), which is what a reduction over a ragged token count wants to read.
+static bool whole_chunks(int64_t M, int64_t ld_t, const void* t_fp8) {
+  return ld_t % 16 == 0 && ld_t >= ((M + 15) & ~(int64_t)15) && ((uintptr_t)t_fp8) % 16 == 0;
+}
+
 static int quant_rowwise_transpose_impl(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx, void* tok_fp8,
                                         float* tok_scale, void* t_fp8, int64_t ld_t, float* t_scale, pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && N >= 0 && ldx >= N && ld_t >= M, "quant_rowwise_transpose: bad shape");
@@ -816,7 +860,7 @@ static int quant_rowwise_transpose_impl(const void* x, int dtype, int64_t M, int
   fill_common(a, x, dtype, M, N, ldx);
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)t_fp8; a.b_scale = t_scale;
   a.ld_t = ld_t;
-  a.vec_out_t = a.vec_out_t && ld_t % 16 == 0 && ((uintptr_t)t_fp8) % 16 == 0;
+  a.vec_out_t = whole_chunks(M, ld_t, t_fp8);
   return launch_quant<A_ROW, B_COL, BL_TRANSPOSED, BS_N_MB>(a, dtype, 1, (hipStream_t)stream);
 }
 
@@ -842,7 +886,7 @@ static int quant_rowwise_blockwise_transpose_impl(const void* x, int dtype, int6
   fill_common(a, x, dtype, M, K, ldx);
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)blk_t_fp8; a.b_scale = blk_t_scale;
   a.ld_t = ld_t;
-  a.vec_out_t = a.vec_out_t && ld_t % 16 == 0 && ((uintptr_t)blk_t_fp8) % 16 == 0;
+  a.vec_out_t = whole_chunks(M, ld_t, blk_t_fp8);
   return launch_quant<A_ROW, B_BLOCK, BL_TRANSPOSED, BS_MB_N>(a, dtype, 1, (hipStream_t)stream);
 }
 
@@ -860,6 +904,43 @@ extern "C" int pt_quant_rowwise_blockwise_transpose_ld(const void* x, int dtype,
   return quant_rowwise_blockwise_transpose_impl(x, dtype, M, K, ldx, tok_fp8, tok_scale, blk_t_fp8, ld_t, blk_t_scale, stream);
 }
 
+static int fill_blockwise(QuantArgs& a, const void* x, int dtype, int64_t G, int64_t N, int64_t K, int64_t stride_g,
+                          int64_t stride_row, void* fp8, int64_t fp8_stride_g, float* scale, int64_t scale_stride_g) {
+  PT_REQUIRE(x && fp8 && scale, "quant_blockwise: null pointer");
+  PT_REQUIRE(fp8_stride_g >= N * K, "quant_blockwise: output stride smaller than the tensor");
+  fill_common(a, x, dtype, N, K, stride_row);
+  const int eb = dtype == PT_F32 ? 4 : 2;
+  a.vec_in = a.vec_in && ((stride_g * eb) % 16 == 0);
+  a.x_stride_g = stride_g;
+  a.a_out = (uint8_t*)fp8; a.a_stride_g = fp8_stride_g; a.a_scale = scale; a.a_scale_stride_g = scale_stride_g;
+  a.vec_out = a.vec_out && (fp8_stride_g % 8 == 0) && (((uintptr_t)fp8) % 8 == 0);
+  return PT_OK;
+}
+
+extern "C" int pt_quant_weights(const pt_quant_weight* parts, int32_t n, int dtype, pt_stream_t stream) {
+  PT_REQUIRE(parts && n >= 0 && n <= PT_QUANT_WEIGHTS_MAX, "quant_weights: %d parts (at most %d)", n, PT_QUANT_WEIGHTS_MAX);
+  QuantWeightsArgs w;
+  w.n = 0;
+  int64_t tiles = 0;
+  for (int i = 0; i < n; ++i) {
+    const pt_quant_weight& q = parts[i];
+    PT_REQUIRE(q.G >= 0 && q.N >= 0 && q.K >= 0 && q.stride_row >= q.K, "quant_weights: bad shape");
+    if (q.G == 0 || q.N == 0 || q.K == 0) continue;
+    QuantArgs& a = w.part[w.n];
+    if (int rc = fill_blockwise(a, q.x, dtype, q.G, q.N, q.K, q.stride_g, q.stride_row, q.fp8, q.fp8_stride_g, q.scale, q.scale_stride_g)) return rc;
+    tiles += (int64_t)a.tiles_m * a.tiles_n * q.G;
+    w.end[w.n++] = tiles;
+  }
+  if (tiles > 8192) {  // more than a handful of rounds of workgroups
+    for (int i = 0, j = 0; i < n; ++i) {
+      if (parts[i].G == 0 || parts[i].N == 0 || parts[i].K == 0) continue;
+      if (int rc = launch_quant<A_BLOCK, B_BLOCK, BL_NONE, BS_MB_N>(w.part[j++], dtype, parts[i].G, (hipStream_t)stream)) return rc;
+    }
+    return PT_OK;
+  }
+  return launch_quant_weights(w, dtype, (hipStream_t)stream);
+}
+
 static int quant_blockwise_transpose_batched_impl(const void* x, int dtype, int64_t G, int64_t N, int64_t K, int64_t stride_g,
                                                   int64_t stride_row, void* fp8, int64_t fp8_stride_g, float* scale,
                                                   int64_t scale_stride_g, void* fp8_t, int64_t t_ld, int64_t t_stride_g,
@@ -867,21 +948,19 @@ static int quant_blockwise_transpose_batched_impl(const void* x, int dtype, int6
                                                   pt_stream_t stream) {
   PT_REQUIRE(G >= 0 && N >= 0 && K >= 0 && stride_row >= K, "quant_blockwise_transpose_batched: bad shape");
   if (G == 0 || N == 0 || K == 0) return PT_OK;
-  PT_REQUIRE(x && fp8 && scale && (fp8_t != nullptr) == (scale_t != nullptr), "quant_blockwise_transpose_batched: null pointer");
+  PT_REQUIRE((fp8_t != nullptr) == (scale_t != nullptr), "quant_blockwise_transpose_batched: null pointer");
+  if (!fp8_t) {
+    const pt_quant_weight one = {x, G, N, K, stride_g, stride_row, fp8, fp8_stride_g, scale, scale_stride_g};
+    return pt_quant_weights(&one, 1, dtype, stream);
+  }
   QuantArgs a;
-  fill_common(a, x, dtype, N, K, stride_row);
-  PT_REQUIRE(fp8_stride_g >= N * K && (!fp8_t || (t_ld >= N && t_stride_g >= K * t_ld - (t_ld - N) && scale_t_ld >= a.tiles_m)),
+  if (int rc = fill_blockwise(a, x, dtype, G, N, K, stride_g, stride_row, fp8, fp8_stride_g, scale, scale_stride_g)) return rc;
+  PT_REQUIRE(t_ld >= N && t_stride_g >= K * t_ld - (t_ld - N) && scale_t_ld >= a.tiles_m,
              "quant_blockwise_transpose_batched: output strides smaller than the tensors");
-  const int eb = dtype == PT_F32 ? 4 : 2;
-  a.vec_in = a.vec_in && ((stride_g * eb) % 16 == 0);
-  a.x_stride_g = stride_g;
-  a.a_out = (uint8_t*)fp8; a.a_stride_g = fp8_stride_g; a.a_scale = scale; a.a_scale_stride_g = scale_stride_g;
   a.b_out = (uint8_t*)fp8_t; a.b_stride_g = t_stride_g; a.b_scale = scale_t; a.b_scale_stride_g = scale_t_stride_g;
   a.ld_t = t_ld; a.bs_ld = scale_t_ld;
   // 16-byte transposed stores need every row start aligned: the pitch, the group stride and the base
   a.vec_out_t = a.vec_out_t && (t_ld % 16 == 0) && (t_stride_g % 16 == 0) && (((uintptr_t)fp8_t) % 16 == 0);
-  a.vec_out = a.vec_out && (fp8_stride_g % 8 == 0) && (((uintptr_t)fp8) % 8 == 0);
-  if (!fp8_t) return launch_quant<A_BLOCK, B_BLOCK, BL_NONE, BS_MB_N>(a, dtype, G, (hipStream_t)stream);
   return launch_quant<A_BLOCK, B_BLOCK, BL_TRANSPOSED, BS_MB_N>(a, dtype, G, (hipStream_t)stream);
 }
 

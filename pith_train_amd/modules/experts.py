@@ -22,7 +22,7 @@ import torch.nn as nn
 from ..dualpipe_utils import FP8WeightCacheControl
 from ..operators import fused_experts
 from ..operators.clamped_swiglu import clamped_swiglu
-from ..operators.deepgemm_quantize import fp8cast_grouped_weight, fp8cast_grouped_weight_cat, weight_twin_enabled
+from ..operators.deepgemm_quantize import fp8cast_grouped_weight, fp8cast_grouped_weight_cat, fp8cast_grouped_weights, weight_twin_enabled
 from ..operators.grouped_linear import FP8GroupedLinear, FP8GroupedLinearFunc, GroupedLinearFunc
 from ..operators.indexed_bias_add import indexed_bias_add
 from ..operators.silu_mul import silu_mul, silu_mul_halves
@@ -34,6 +34,18 @@ from ..operators.token_scatter import (
     scatter_for_grouped_gemm,
 )
 from . import training
+
+
+def _weight(linear: nn.Module) -> torch.Tensor:
+    """``linear.weight`` without the module's attribute search (a microsecond each, and a step of a small
+    layer makes twenty of them)."""
+    w = linear._parameters.get("weight")
+    return w if w is not None else linear.weight
+
+
+def _cached(cache, version: int, now: int, twin: bool) -> bool:
+    """Whether a module's cached quantised weight is of this version and has the twin that is asked for."""
+    return cache is not None and version == now and (cache[2] is not None) == twin
 
 
 class Qwen3MoeExperts(nn.Module):
@@ -57,6 +69,33 @@ class Qwen3MoeExperts(nn.Module):
             self._gu_version = ver
         return self._gu_cache
 
+    def _projections(self):
+        m = self._modules
+        return m["gate_proj"], m["up_proj"], m["down_proj"]
+
+    def one_node(self, x) -> bool:
+        """Whether the block runs as one autograd node on ``x``."""
+        if not training.fp8 or x.dtype != torch.bfloat16:
+            return False
+        gate, up, down = self._projections()
+        return (isinstance(gate, FP8GroupedLinear) and isinstance(up, FP8GroupedLinear) and isinstance(down, FP8GroupedLinear)
+                and fused_experts.supported_split(x, _weight(gate), _weight(up), _weight(down)))
+
+    def _quantized_weights(self):
+        """The fused gate/up operand and the down operand, quantised by one launch when both are stale."""
+        ver, twin = FP8WeightCacheControl.version, weight_twin_enabled()
+        gate, up, down = self._projections()
+        if torch.compiler.is_compiling():
+            return self._fused_gate_up_quant(), down._get_quantized_weight()
+        gu_ok = _cached(self._gu_cache, self._gu_version, ver, twin)
+        down_ok = _cached(down._wq_cache, down._wq_version, ver, twin)
+        if not (gu_ok or down_ok):
+            self._gu_cache, down._wq_cache = fp8cast_grouped_weights([[_weight(gate), _weight(up)], [_weight(down)]])
+            self._gu_version = down._wq_version = ver
+        elif not (gu_ok and down_ok):
+            return self._fused_gate_up_quant(), down._get_quantized_weight()
+        return self._gu_cache, down._wq_cache
+
     def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, fuse_activation: bool = True,
                 expand_idx=None):
         """``row_map`` (extension, FP8 layers only): the scatter's int32 source-row map.  ``x`` is
@@ -68,12 +107,10 @@ class Qwen3MoeExperts(nn.Module):
         autograd node on a fused gate_up operand: the tokens are quantised once instead of once
         per projection, one GEMM serves both, and the SwiGLU and its gradient are computed inside
         the kernels that quantise them (same bits as the three-operator composition)."""
-        if (fuse_activation and training.fp8 and x.shape[0] > 0 and isinstance(self.gate_proj, FP8GroupedLinear)
-                and isinstance(self.up_proj, FP8GroupedLinear) and isinstance(self.down_proj, FP8GroupedLinear)
-                and fused_experts.supported_split(x, self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight)):
+        if fuse_activation and x.shape[0] > 0 and self.one_node(x):
+            gate, up, down = self._projections()
             return fused_experts.FP8SwiGLUSplitExpertsFunc.apply(
-                x, self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, grouped_mm_offs,
-                self._fused_gate_up_quant(), self.down_proj._get_quantized_weight(), row_map, expand_idx,
+                x, _weight(gate), _weight(up), _weight(down), grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
             )  # fmt: skip
         assert expand_idx is None, "expand_idx needs the one-node FP8 path"
         gi = precompute_group_indices(grouped_mm_offs, x.shape[0])
@@ -113,17 +150,38 @@ class Qwen35MoeExperts(nn.Module):
         self.gate_up_proj = training.GroupedLinear(num_experts, hidden_size, 2 * moe_intermediate_size)
         self.down_proj = training.GroupedLinear(num_experts, moe_intermediate_size, hidden_size)
 
+    def one_node(self, x) -> bool:
+        """Whether the block runs as one autograd node on ``x``."""
+        if not training.fp8 or x.dtype != torch.bfloat16:
+            return False
+        gate_up, down = self._modules["gate_up_proj"], self._modules["down_proj"]
+        return (isinstance(gate_up, FP8GroupedLinear) and isinstance(down, FP8GroupedLinear)
+                and fused_experts.supported(x, _weight(gate_up), _weight(down)))
+
+    def _quantized_weights(self):
+        """Both operands, quantised by one launch when both are stale."""
+        ver, twin = FP8WeightCacheControl.version, weight_twin_enabled()
+        gu, down = self._modules["gate_up_proj"], self._modules["down_proj"]
+        if not torch.compiler.is_compiling():
+            gu_ok = _cached(gu._wq_cache, gu._wq_version, ver, twin)
+            down_ok = _cached(down._wq_cache, down._wq_version, ver, twin)
+            if not (gu_ok or down_ok):
+                gu._wq_cache, down._wq_cache = fp8cast_grouped_weights([[_weight(gu)], [_weight(down)]])
+                gu._wq_version = down._wq_version = ver
+                gu_ok = down_ok = True
+            if gu_ok and down_ok:
+                return gu._wq_cache, down._wq_cache
+        return gu._get_quantized_weight(), down._get_quantized_weight()
+
     def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, fuse_activation: bool = True,
                 expand_idx=None):
         """``row_map`` / ``expand_idx``: see :meth:`Qwen3MoeExperts.forward`.  With ``fuse_activation`` (FP8 layers)
         the block runs as one autograd node whose SwiGLU output and SwiGLU gradient are computed
         inside the kernels that quantise them (same bits as the three-operator composition)."""
-        if (fuse_activation and training.fp8 and x.shape[0] > 0 and isinstance(self.gate_up_proj, FP8GroupedLinear)
-                and isinstance(self.down_proj, FP8GroupedLinear)
-                and fused_experts.supported(x, self.gate_up_proj.weight, self.down_proj.weight)):
+        if fuse_activation and x.shape[0] > 0 and self.one_node(x):
             return fused_experts.FP8SwiGLUExpertsFunc.apply(
-                x, self.gate_up_proj.weight, self.down_proj.weight, grouped_mm_offs, ks, ks_tensor,
-                self.gate_up_proj._get_quantized_weight(), self.down_proj._get_quantized_weight(), row_map, expand_idx,
+                x, _weight(self._modules["gate_up_proj"]), _weight(self._modules["down_proj"]), grouped_mm_offs, ks, ks_tensor,
+                *self._quantized_weights(), row_map, expand_idx,
             )  # fmt: skip
         assert expand_idx is None, "expand_idx needs the one-node FP8 path"
         gi = precompute_group_indices(grouped_mm_offs, x.shape[0])
@@ -166,6 +224,15 @@ class GptOssExperts(nn.Module):
             cache[name] = fp8cast_grouped_weight(weight)
         return cache[name]
 
+    def _quantized_weights(self):
+        """Both operands, quantised by one launch when neither is cached."""
+        stale = self._wq_version != FP8WeightCacheControl.version or not self._wq_cache
+        if stale and not (torch.compiler.is_compiling() or weight_twin_enabled()):
+            gate_up, down = fp8cast_grouped_weights([[self.gate_up_proj], [self.down_proj]])
+            self._wq_cache = {"gate_up_proj": gate_up, "down_proj": down}
+            self._wq_version = FP8WeightCacheControl.version
+        return self._quantized_weight("gate_up_proj", self.gate_up_proj), self._quantized_weight("down_proj", self.down_proj)
+
     def _group_linear(self, x, weight, name, offs, ks, ks_tensor, group_indices_, in_rows=None, bias=None,
                       out_rows=None, out_m=None):
         if x.shape[0] == 0:
@@ -180,9 +247,10 @@ class GptOssExperts(nn.Module):
 
     def bias_fusable(self, x) -> bool:
         """Whether the two ``indexed_bias_add`` steps happen in the stores of the GEMMs."""
+        p = self._parameters
         return (self.fuse_bias and training.fp8 and x.shape[0] > 0 and x.dtype == torch.bfloat16
-                and self.gate_up_proj_bias.dtype == x.dtype and self.down_proj_bias.dtype == x.dtype
-                and self.gate_up_proj.shape[1] % 8 == 0 and self.down_proj.shape[1] % 8 == 0)
+                and p["gate_up_proj_bias"].dtype == x.dtype and p["down_proj_bias"].dtype == x.dtype
+                and p["gate_up_proj"].shape[1] % 8 == 0 and p["down_proj"].shape[1] % 8 == 0)
 
     def one_node(self, x) -> bool:
         """Whether the block runs as one autograd node (fused biases and activation).  That node
@@ -204,8 +272,7 @@ class GptOssExperts(nn.Module):
         if M % 128 == 0 and self.one_node(x):
             return fused_experts.FP8ClampedSwiGLUExpertsFunc.apply(
                 x, self.gate_up_proj, self.gate_up_proj_bias, self.down_proj, self.down_proj_bias, grouped_mm_offs,
-                self._quantized_weight("gate_up_proj", self.gate_up_proj), self._quantized_weight("down_proj", self.down_proj),
-                1.702, self.swiglu_limit, row_map, scatter_output,
+                *self._quantized_weights(), 1.702, self.swiglu_limit, row_map, scatter_output,
             )
         if fused:
             gate_up = self._group_linear(x, self.gate_up_proj, "gate_up_proj", grouped_mm_offs, ks, ks_tensor, None, row_map,
@@ -240,19 +307,15 @@ def forward_stage3(experts: nn.Module, gathered_tokens, expert_idxs, experts_per
     (each unique row is read once per use and no expanded copy is materialised); without it the
     two steps run separately as in the reference.
     """
-    if (fuse_permute and training.fp8 and expert_idxs.shape[0] > 0
-            and isinstance(experts, (Qwen3MoeExperts, Qwen35MoeExperts))
-            and isinstance(experts.down_proj, FP8GroupedLinear)
-            and experts.down_proj.out_features % 8 == 0 and experts.down_proj.in_features % 8 == 0):
-        if isinstance(experts, Qwen35MoeExperts):
-            fused_node = fused_experts.supported(gathered_tokens, experts.gate_up_proj.weight, experts.down_proj.weight)
-        else:
-            fused_node = (isinstance(experts.gate_proj, FP8GroupedLinear) and isinstance(experts.up_proj, FP8GroupedLinear)
-                          and fused_experts.supported_split(gathered_tokens, experts.gate_proj.weight,
-                                                            experts.up_proj.weight, experts.down_proj.weight))
-        if expand_idx is None or (fused_node and fuse_expand):
+    if fuse_permute and training.fp8 and expert_idxs.shape[0] > 0 and isinstance(experts, (Qwen3MoeExperts, Qwen35MoeExperts)):
+        fused_node = experts.one_node(gathered_tokens)
+        # the composition of separate operators can still take the row map when its layers are FP8 ones
+        down = experts._modules["down_proj"]
+        mapped = fused_node or (isinstance(down, FP8GroupedLinear) and down.out_features % 8 == 0 and down.in_features % 8 == 0)
+        if mapped and (expand_idx is None or (fused_node and fuse_expand)):
             _, grouped_mm_offs, ks, ks_tensor, src_of = group_rows_with_sizes(
-                expert_idxs, experts_per_rank, device=gathered_tokens.device, host_sizes=host_sizes or not fused_node)
+                expert_idxs, experts_per_rank, device=gathered_tokens.device, host_sizes=host_sizes or not fused_node,
+                need_reverse=False)
             if expand_idx is None:
                 return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of)
             # deduplicated rows: the first quantisation reads them through expand_idx composed with

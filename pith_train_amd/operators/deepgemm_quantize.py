@@ -8,6 +8,9 @@ here.
 
 from __future__ import annotations
 
+import os
+import struct
+
 import torch
 
 from .. import _lib
@@ -22,6 +25,7 @@ __all__ = [
     "fp8cast_blockwise_batched",
     "fp8cast_grouped_weight",
     "fp8cast_grouped_weight_cat",
+    "fp8cast_grouped_weights",
     "fp8cast_rowwise_colwise_t",
     "fp8cast_rowwise_colwise_t_rows",
 ]
@@ -46,7 +50,9 @@ def transposed_pitch(m: int) -> int:
     """Row pitch (bytes) of a transposed FP8 operand ``[N, m]`` of a dense linear.  The weight
     gradient reads these operands along rows, 128 bytes of every row per step; with a pitch that
     is a multiple of 256 the rows of a step fall onto few memory channels (measured: 25 % slower
-    at 5 * 2**14 than at 579 * 128), so such pitches get one more 128-byte column."""
+    at 5 * 2**14 than at 579 * 128), so such pitches get one more 128-byte column.  The reduction
+    is read in 16-byte chunks, so a ragged token count is padded to whole ones (with zeros)."""
+    m = (m + 15) // 16 * 16
     return m + 128 if (m >= 2048 and m % 256 == 0) else m
 
 
@@ -249,8 +255,6 @@ def fp8cast_blockwise_batched(x: torch.Tensor):
 def weight_twin_enabled() -> bool:
     """``PITHTRAIN_FP8_WEIGHT_TWIN=1`` keeps the transposed FP8 copy of the grouped-expert weights
     (the reference's data flow: the input-gradient GEMM then runs in the NT form on it)."""
-    import os
-
     return os.environ.get("PITHTRAIN_FP8_WEIGHT_TWIN", "0") == "1"
 
 
@@ -263,3 +267,40 @@ def fp8cast_grouped_weight(x: torch.Tensor):
 def fp8cast_grouped_weight_cat(parts):
     """:func:`fp8cast_grouped_weight` of ``torch.cat(parts, dim=1)`` without the concatenation."""
     return fp8cast_blockwise_transpose_batched_cat(parts, twin=weight_twin_enabled())
+
+
+_WEIGHT_PART = struct.Struct("=10q").pack
+
+
+def fp8cast_grouped_weights(weights):
+    """``[fp8cast_grouped_weight_cat(parts) for parts in weights]`` - the fused operand of every list of
+    ``[G, N_i, K]`` parts - with one launch for all of them when no twin is wanted: the projections of
+    an expert block after an optimizer step."""
+    flat = [p if p.is_cuda and p.stride(-1) == 1 else _prep2d(p.detach()) for parts in weights for p in parts]
+    dtype = flat[0].dtype
+    if weight_twin_enabled() or len(flat) > _lib.PT_QUANT_WEIGHTS_MAX or any(t.dtype != dtype for t in flat) or any(
+            len(parts) > 1 and t.shape[1] % 128 for parts in weights for t in parts):
+        return [fp8cast_grouped_weight(parts[0]) if len(parts) == 1 else fp8cast_grouped_weight_cat(parts) for parts in weights]
+    dev = flat[0].device
+    block, result, i = b"", [], 0
+    for parts in weights:
+        G, N, K = parts[0].shape
+        for p in parts[1:]:
+            assert p.ndim == 3 and p.shape[0] == G and p.shape[2] == K
+            N += p.shape[1]
+        nb, kb = _cdiv(N, 128), _cdiv(K, 128)
+        out = torch.empty((G, N, K), dtype=FP8, device=dev)
+        scale = torch.empty((G, nb, kb), dtype=torch.float32, device=dev)
+        row = 0
+        for _ in parts:
+            x3 = flat[i]
+            n = x3.shape[1]
+            block += _WEIGHT_PART(
+                x3.data_ptr(), G, n, K, x3.stride(0) if G > 1 else n * K, x3.stride(1) if n > 1 else K,
+                out.data_ptr() + row * K, N * K, scale.data_ptr() + 4 * (row // 128) * kb, nb * kb,
+            )  # fmt: skip
+            row += n
+            i += 1
+        result.append((out, scale, None, None))
+    _lib.call("pt_quant_weights", block, i, _lib.dtype_code(dtype), _lib.stream_ptr(dev))
+    return result

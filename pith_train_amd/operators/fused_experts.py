@@ -11,11 +11,15 @@ The token permutation can be folded in as well (``row_map``, see ``FP8GroupedLin
 
 from __future__ import annotations
 
+import functools
+import struct
+
 import torch
 
 from .. import _lib
-from .deepgemm_quantize import FP8, fp8cast_rowwise_colwise_t, fp8cast_rowwise_colwise_t_rows
-from .grouped_linear import dgrad_operand, m_grouped_fp8_dgrad, m_grouped_fp8_gemm_nt, schedule_wgrad
+from ..dualpipe_utils import WeightGradStore
+from .deepgemm_quantize import FP8
+from .grouped_linear import dgrad_operand, m_grouped_fp8_dgrad, schedule_wgrad, wgrad_target
 from .token_scatter import _GEMM_ALLOC_ALIGNMENT, _PaddedIndexGather
 
 
@@ -124,77 +128,167 @@ def compose_row_maps(row_map: torch.Tensor, expand_idx: torch.Tensor, n_src: int
     return out
 
 
-def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx=None):
-    """Shared forward of the two autograd nodes below.  ``gate_up_weights``: the parameters whose
-    gradients the gate_up weight gradient is written to, one fused ``[G, 2I, K]`` tensor or the
-    pair ``(gate [G, I, K], up [G, I, K])``.  ``expand_idx`` (with ``row_map``): ``x`` holds
-    deduplicated rows and routed row i is ``x[expand_idx[i]]``; the result has one row per routed
-    row, and the backward sums the gradients of the rows that share a source row."""
-    _lib.require_cuda(x)
-    gu_fp8, gu_scale, gu_t_fp8, gu_t_scale = q_gate_up
-    dn_fp8, dn_scale, dn_t_fp8, dn_t_scale = q_down
-    two_i = gu_fp8.shape[1]
-    H = w_down.shape[1]
-    out_m = x.shape[0]
-    if row_map is not None:
-        M = row_map.shape[0]
-        in_map = row_map
-        if expand_idx is not None:
-            in_map = compose_row_maps(row_map, expand_idx, x.shape[0])
-            out_m = expand_idx.shape[0]
-        x_fp8, x_s, x_ch_t, x_ch_s = fp8cast_rowwise_colwise_t_rows(x, in_map, grouped_mm_offs)
+_FORWARD_BLOCK = struct.Struct("=23q2d10q").pack
+_BACKWARD_BLOCK = struct.Struct("=35q2d5q").pack
+_ONE_BUFFER = 32 << 20  # bytes up to which the tensors of one kind share an allocation
+
+
+@functools.lru_cache(maxsize=256)
+def _sizes(M, K, half, H):
+    """Byte sizes of what a step allocates: kept activations (x^T, its scales, h^T, its scales), forward
+    temporaries (composed map, x, its scales, h, its scales), transposed gradients (dy^T, scales,
+    gate_up's^T, scales), backward temporaries (dy, scales, grad_h, column sums)."""
+    blocks = M // 128
+    return (
+        _offsets(K * M, 4 * blocks * K, half * M, 4 * blocks * half),
+        _offsets(4 * M, M * K, 4 * M * _cdiv(K, 128), M * half, 4 * M * _cdiv(half, 128)),
+        _offsets(H * M, 4 * blocks * H, 2 * half * M, 8 * blocks * half),
+        _offsets(M * H, 4 * M * _cdiv(H, 128), 2 * M * half, 8 * blocks * half),
+    )
+
+
+def _offsets(*sizes):
+    offsets, total = [], 0
+    for n in sizes:
+        offsets.append(total)
+        total += (n + 255) // 256 * 256
+    return sizes, tuple(offsets), total
+
+
+def _allocate(layout, dev):
+    """(tensors that own the memory, addresses of its pieces): one buffer for small pieces (an allocation
+    costs the host two microseconds), one each for large ones."""
+    sizes, offsets, total = layout
+    if total <= _ONE_BUFFER:
+        buffers = [torch.empty(total, dtype=torch.uint8, device=dev)]
     else:
-        assert expand_idx is None, "expand_idx needs the row map of the scatter"
-        M = x.shape[0]
-        x_fp8, x_s, x_ch_t, x_ch_s = fp8cast_rowwise_colwise_t(x)
-    gate_up = torch.empty((M, two_i), device=x.device, dtype=x.dtype)
-    m_grouped_fp8_gemm_nt((x_fp8, x_s), (gu_fp8, gu_scale), gate_up, grouped_mm_offs)
-    del x_fp8, x_s
-    h_fp8, h_s, h_ch_t, h_ch_s = silu_mul_quant(gate_up, grouped_mm_offs if row_map is not None else None)
-    out = torch.empty((out_m, H), device=x.device, dtype=x.dtype)
-    m_grouped_fp8_gemm_nt((h_fp8, h_s), (dn_fp8, dn_scale), out, grouped_mm_offs, row_map)
-    gu_dg, gu_dg_s, ctx.gu_forward_layout = dgrad_operand(q_gate_up, gate_up_weights, M)
-    dn_dg, dn_dg_s, ctx.dn_forward_layout = dgrad_operand(q_down, w_down, M)
-    ctx.save_for_backward(gu_dg, gu_dg_s, dn_dg, dn_dg_s, grouped_mm_offs, x_ch_t, x_ch_s,
-                          gate_up, h_ch_t, h_ch_s, row_map, expand_idx)
+        buffers = [torch.empty(n, dtype=torch.uint8, device=dev) for n in sizes]
+    return buffers, _addresses(layout, buffers)
+
+
+def _addresses(layout, buffers):
+    if len(buffers) > 1:
+        return [b.data_ptr() for b in buffers]
+    base = buffers[0].data_ptr()
+    return [base + o for o in layout[1]]
+
+
+def _piece(layout, buffers, i, rows, cols, dtype):
+    """Piece ``i`` as a ``[rows, cols]`` tensor."""
+    if len(buffers) > 1:
+        return buffers[i].view(dtype).view(rows, cols)
+    at = layout[1][i]
+    return buffers[0][at : at + layout[0][i]].view(dtype).view(rows, cols)
+
+
+def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx=None, scatter=True,
+             clamp=None, biases=(None, None)):
+    """Shared forward of the autograd nodes below: one library call queues every launch of it.
+    ``gate_up_weights``: the parameters whose gradients the gate_up weight gradient is written to, one
+    fused ``[G, 2I, K]`` tensor or the pair ``(gate [G, I, K], up [G, I, K])``.  ``expand_idx`` (with
+    ``row_map``): ``x`` holds deduplicated rows and routed row i is ``x[expand_idx[i]]``; the result
+    has one row per routed row, and the backward sums the gradients of the rows that share a source
+    row.  ``scatter`` (with ``row_map``): the result comes back un-permuted.  ``clamp``: ``(alpha,
+    limit)`` of the clamped SwiGLU, whose projections have the two ``biases``."""
+    _lib.require_cuda(x)
+    gu_fp8, gu_scale = q_gate_up[:2]
+    dn_fp8, dn_scale = q_down[:2]
+    G, H, half = w_down.shape
+    src_rows, K = x.shape
+    assert expand_idx is None or row_map is not None, "expand_idx needs the row map of the scatter"
+    scatter = scatter and row_map is not None
+    if row_map is not None:
+        assert row_map.dtype == torch.int32 and row_map.shape[0] % 128 == 0
+        row_map = row_map.contiguous()
+    M = src_rows if row_map is None else row_map.shape[0]
+    assert M % 128 == 0, f"grouped rows must be a multiple of 128, got {M}"
+    routed = src_rows
+    if expand_idx is not None:
+        assert expand_idx.dtype == torch.int64
+        expand_idx = expand_idx.contiguous()
+        routed = expand_idx.shape[0]
+    if x.stride(1) != 1:
+        x = x.contiguous()
+    dev = x.device
+    kept_layout, temp_layout, _, _ = _sizes(M, K, half, H)
+    _temp, temp_at = _allocate(temp_layout, dev)
+    kept, kept_at = _allocate(kept_layout, dev)
+    gate_up = torch.empty((M, 2 * half), device=dev, dtype=x.dtype)
+    out = torch.empty((routed if scatter else M, H), device=dev, dtype=x.dtype)
+    b_gate_up, b_down = biases if biases[0] is None else [b.detach().contiguous() for b in biases]
+    alpha, limit = clamp or (0.0, 0.0)
+    _lib.call("pt_experts_forward", _FORWARD_BLOCK(
+        x.data_ptr(), src_rows, x.stride(0) if src_rows > 1 else K, M, K, half, H, G, grouped_mm_offs.data_ptr(), _lib.ptr(row_map) or 0,
+        _lib.ptr(expand_idx) or 0, 0 if expand_idx is None else routed, gu_fp8.data_ptr(), gu_scale.data_ptr(), _lib.ptr(b_gate_up) or 0,
+        dn_fp8.data_ptr(), dn_scale.data_ptr(), _lib.ptr(b_down) or 0, gate_up.data_ptr(), out.data_ptr(), out.shape[0], scatter,
+        clamp is not None, alpha, limit, *kept_at, *temp_at, _lib.stream_ptr(dev),
+    ))  # fmt: skip
+    gu_dg, gu_dg_s, gu_forward = dgrad_operand(q_gate_up, gate_up_weights, M)
+    dn_dg, dn_dg_s, dn_forward = dgrad_operand(q_down, w_down, M)
+    ctx.save_for_backward(gu_dg, gu_dg_s, dn_dg, dn_dg_s, grouped_mm_offs, gate_up, row_map, expand_idx, *kept)
     ctx.gate_up_weights, ctx.w_down = gate_up_weights, w_down
-    ctx.rows = (M, out_m, x.shape[0])
+    ctx.clamp = clamp
+    ctx.bias_dtypes = tuple(None if b is None else b.dtype for b in biases)
+    ctx.dims = (M, K, half, H, G, routed, src_rows, gu_forward, dn_forward, scatter)
     return out
 
 
 def _backward(ctx, grad_out):
-    """Shared backward: returns the gradient of ``x``; the weight gradients go to ``.grad`` (or to
-    the ``WeightGradStore`` queue) through :func:`schedule_wgrad`."""
-    (gu_dg, gu_dg_s, dn_dg, dn_dg_s, offs, x_ch_t, x_ch_s, gate_up, h_ch_t, h_ch_s,
-     row_map, expand_idx) = ctx.saved_tensors  # fmt: skip
-    M, rows_x, rows_src = ctx.rows
-    half = gate_up.shape[1] // 2
-    K = gu_dg.shape[2] if ctx.gu_forward_layout else gu_dg.shape[1]
+    """Shared backward: returns the gradient of ``x`` and of the two biases (None without); the weight
+    gradients go to ``.grad``, or to the ``WeightGradStore`` queue."""
+    gu_dg, gu_dg_s, dn_dg, dn_dg_s, offs, gate_up, row_map, expand_idx, *kept = ctx.saved_tensors
+    M, K, half, H, G, routed, src_rows, gu_forward, dn_forward, scatter = ctx.dims
     grad_out = grad_out.contiguous()
-    if row_map is not None:
-        dy_fp8, dy_s, dy_ch_t, dy_ch_s = fp8cast_rowwise_colwise_t_rows(grad_out, row_map, offs)
-    else:
-        dy_fp8, dy_s, dy_ch_t, dy_ch_s = fp8cast_rowwise_colwise_t(grad_out)
-    grad_h = torch.empty((M, half), device=grad_out.device, dtype=grad_out.dtype)
-    m_grouped_fp8_dgrad((dy_fp8, dy_s), dn_dg, dn_dg_s, ctx.dn_forward_layout, grad_h, offs)
-    schedule_wgrad(ctx.w_down, (dy_ch_t, dy_ch_s), (h_ch_t, h_ch_s), offs)
-    del dy_fp8, dy_s
-    dgu_fp8, dgu_s, dgu_ch_t, dgu_ch_s = silu_mul_bwd_quant(grad_h, gate_up, offs if row_map is not None else None)
-    grad_x = torch.empty((rows_x, K), device=grad_out.device, dtype=grad_out.dtype)
-    m_grouped_fp8_dgrad((dgu_fp8, dgu_s), gu_dg, gu_dg_s, ctx.gu_forward_layout, grad_x, offs, row_map)
+    dev = grad_out.device
+    split = isinstance(ctx.gate_up_weights, tuple)
+    gu_weights = ctx.gate_up_weights if split else (ctx.gate_up_weights,)
+    deferred = WeightGradStore.enabled
+    # separate gate and up parameters: each gets its half of the gate_up weight gradient's rows
+    targets = [(None, False, None)] * 3 if deferred else [wgrad_target(w) for w in (ctx.w_down, *gu_weights)]
+    if len(targets) == 2:
+        targets.append((None, False, None))
+    kept_layout, _, twin_layout, temp_layout = _sizes(M, K, half, H)
+    twins, twins_at = _allocate(twin_layout, dev)
+    _temp, temp_at = _allocate(temp_layout, dev)
+    dgu = torch.empty((M, 2 * half), device=dev, dtype=FP8)
+    dgu_s = torch.empty((M, _cdiv(2 * half, 128)), device=dev, dtype=torch.float32)
+    d_gu, d_dn = ctx.bias_dtypes
+    d_gu_bias = None if d_gu is None else torch.empty((G, 2 * half), device=dev, dtype=d_gu)
+    d_dn_bias = None if d_dn is None else torch.empty((G, H), device=dev, dtype=d_dn)
+    (dw_down, add_down, _), (dw_gu, add_gu, _), (dw_up, add_up, _) = targets
+    alpha, limit = ctx.clamp or (0.0, 0.0)
+    block = _BACKWARD_BLOCK(
+        grad_out.data_ptr(), grad_out.shape[0], M, K, half, H, G, offs.data_ptr(), (_lib.ptr(row_map) or 0) if scatter else 0,
+        row_map is not None, dn_dg.data_ptr(), dn_dg_s.data_ptr(), dn_forward, gate_up.data_ptr(),
+        *_addresses(kept_layout, kept), dgu.data_ptr(), dgu_s.data_ptr(), *twins_at, *temp_at, _lib.ptr(dw_down) or 0, add_down, _lib.ptr(dw_gu) or 0, add_gu, _lib.ptr(dw_up) or 0, add_up,
+        ctx.clamp is not None, alpha, limit, _lib.ptr(d_gu_bias) or 0, 0 if d_gu is None else _lib.dtype_code(d_gu),
+        _lib.ptr(d_dn_bias) or 0, 0 if d_dn is None else _lib.dtype_code(d_dn), _lib.stream_ptr(dev),
+    )  # fmt: skip
+    _lib.call("pt_experts_backward", block)
+    grad_x = torch.empty((M if row_map is None else routed, K), device=dev, dtype=grad_out.dtype)
+    m_grouped_fp8_dgrad((dgu, dgu_s), gu_dg, gu_dg_s, gu_forward, grad_x, offs, row_map)
+    if not deferred:
+        _lib.call("pt_experts_weight_gradient", block)
+    for _, _, finish in targets:
+        if finish is not None:
+            finish()
+    if deferred:
+        blocks, f32 = M // 128, torch.float32
+        dy_t = _piece(twin_layout, twins, 0, H, M, FP8), _piece(twin_layout, twins, 1, blocks, H, f32)
+        gu, gus = _piece(twin_layout, twins, 2, 2 * half, M, FP8), _piece(twin_layout, twins, 3, blocks, 2 * half, f32)
+        x_t = _piece(kept_layout, kept, 0, K, M, FP8), _piece(kept_layout, kept, 1, blocks, K, f32)
+        h_t = _piece(kept_layout, kept, 2, half, M, FP8), _piece(kept_layout, kept, 3, blocks, half, f32)
+        schedule_wgrad(ctx.w_down, dy_t, h_t, offs)
+        if split:
+            schedule_wgrad(gu_weights[0], (gu[:half], gus[:, :half]), x_t, offs)
+            schedule_wgrad(gu_weights[1], (gu[half:], gus[:, half:]), x_t, offs)
+        else:
+            schedule_wgrad(gu_weights[0], (gu, gus), x_t, offs)
     if expand_idx is not None:
         # one gradient row per routed row so far: rows that expand the same source row are summed
         # (the backward of the expanding gather, token_scatter.py:311-325)
-        grad_x = _PaddedIndexGather.scatter_sum(grad_x, expand_idx, rows_src, _GEMM_ALLOC_ALIGNMENT)
-    if isinstance(ctx.gate_up_weights, tuple):
-        # separate gate and up parameters: each gets the weight-gradient GEMM of its half of the
-        # colwise twin (rows of the transposed bytes, columns of the scale array)
-        w_gate, w_up = ctx.gate_up_weights
-        schedule_wgrad(w_gate, (dgu_ch_t[:half], dgu_ch_s[:, :half]), (x_ch_t, x_ch_s), offs)
-        schedule_wgrad(w_up, (dgu_ch_t[half:], dgu_ch_s[:, half:]), (x_ch_t, x_ch_s), offs)
-    else:
-        schedule_wgrad(ctx.gate_up_weights, (dgu_ch_t, dgu_ch_s), (x_ch_t, x_ch_s), offs)
-    return grad_x
+        grad_x = _PaddedIndexGather.scatter_sum(grad_x, expand_idx, src_rows, _GEMM_ALLOC_ALIGNMENT)
+    return grad_x, d_gu_bias, d_dn_bias
 
 
 class FP8SwiGLUExpertsFunc(torch.autograd.Function):
@@ -208,7 +302,7 @@ class FP8SwiGLUExpertsFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        return _backward(ctx, grad_out), None, None, None, None, None, None, None, None, None
+        return _backward(ctx, grad_out)[0], None, None, None, None, None, None, None, None, None
 
 
 class FP8SwiGLUSplitExpertsFunc(torch.autograd.Function):
@@ -224,7 +318,7 @@ class FP8SwiGLUSplitExpertsFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        return _backward(ctx, grad_out), None, None, None, None, None, None, None, None
+        return _backward(ctx, grad_out)[0], None, None, None, None, None, None, None, None
 
 
 def supported_split(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor) -> bool:
@@ -250,64 +344,11 @@ class FP8ClampedSwiGLUExpertsFunc(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_gate_up, b_gate_up, w_down, b_down, grouped_mm_offs, q_gate_up, q_down, alpha, limit,
                 row_map=None, scatter_output=False):
-        _lib.require_cuda(x)
-        gu_fp8, gu_scale, gu_t_fp8, gu_t_scale = q_gate_up
-        dn_fp8, dn_scale, dn_t_fp8, dn_t_scale = q_down
-        two_i = gu_fp8.shape[1]
-        H = w_down.shape[1]
         assert not scatter_output or row_map is not None, "scatter_output needs the row map"
-        if row_map is not None:
-            M = row_map.shape[0]
-            # row_map may be sized for more rows than the routing produced (its tail negative):
-            # every kernel below takes the real row count from grouped_mm_offs on the device
-            x_fp8, x_s, x_ch_t, x_ch_s = fp8cast_rowwise_colwise_t_rows(x, row_map, grouped_mm_offs)
-        else:
-            M = x.shape[0]
-            x_fp8, x_s, x_ch_t, x_ch_s = fp8cast_rowwise_colwise_t(x)
-        limit_rows = grouped_mm_offs if row_map is not None else None
-        gate_up = torch.empty((M, two_i), device=x.device, dtype=x.dtype)
-        m_grouped_fp8_gemm_nt((x_fp8, x_s), (gu_fp8, gu_scale), gate_up, grouped_mm_offs, None,
-                              b_gate_up.detach().contiguous())
-        del x_fp8, x_s
-        h_fp8, h_s, h_ch_t, h_ch_s = clamped_swiglu_quant(gate_up, alpha, limit, limit_rows)
-        out_rows = row_map if scatter_output else None
-        out = torch.empty((x.shape[0] if scatter_output else M, H), device=x.device, dtype=x.dtype)
-        m_grouped_fp8_gemm_nt((h_fp8, h_s), (dn_fp8, dn_scale), out, grouped_mm_offs, out_rows,
-                              b_down.detach().contiguous())
-        gu_dg, gu_dg_s, ctx.gu_forward_layout = dgrad_operand(q_gate_up, w_gate_up, M)
-        dn_dg, dn_dg_s, ctx.dn_forward_layout = dgrad_operand(q_down, w_down, M)
-        ctx.save_for_backward(gu_dg, gu_dg_s, dn_dg, dn_dg_s, grouped_mm_offs, x_ch_t, x_ch_s,
-                              gate_up, h_ch_t, h_ch_s, row_map)
-        ctx.weights = (w_gate_up, w_down)
-        ctx.consts = (float(alpha), float(limit), bool(scatter_output), M, x.shape[0], b_gate_up.dtype, b_down.dtype)
-        return out
+        return _forward(ctx, x, w_gate_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, None, scatter_output,
+                        (float(alpha), float(limit)), (b_gate_up, b_down))
 
     @staticmethod
     def backward(ctx, grad_out):
-        from .indexed_bias_add import _segment_sum_along_rows
-
-        (gu_dg, gu_dg_s, dn_dg, dn_dg_s, offs, x_ch_t, x_ch_s, gate_up, h_ch_t, h_ch_s,
-         row_map) = ctx.saved_tensors  # fmt: skip
-        w_gate_up, w_down = ctx.weights
-        alpha, limit, scatter_output, M, rows_x, gu_bias_dtype, dn_bias_dtype = ctx.consts
-        half = gate_up.shape[1] // 2
-        K = gu_dg.shape[2] if ctx.gu_forward_layout else gu_dg.shape[1]
-        grad_out = grad_out.contiguous()
-        out_rows = row_map if scatter_output else None
-        if out_rows is not None:
-            dy_fp8, dy_s, dy_ch_t, dy_ch_s = fp8cast_rowwise_colwise_t_rows(grad_out, out_rows, offs)
-        else:
-            dy_fp8, dy_s, dy_ch_t, dy_ch_s = fp8cast_rowwise_colwise_t(grad_out)
-        grad_b_down = _segment_sum_along_rows(grad_out, offs, dn_bias_dtype, out_rows)
-        grad_h = torch.empty((M, half), device=grad_out.device, dtype=grad_out.dtype)
-        m_grouped_fp8_dgrad((dy_fp8, dy_s), dn_dg, dn_dg_s, ctx.dn_forward_layout, grad_h, offs)
-        schedule_wgrad(w_down, (dy_ch_t, dy_ch_s), (h_ch_t, h_ch_s), offs)
-        del dy_fp8, dy_s
-        dgu_fp8, dgu_s, dgu_ch_t, dgu_ch_s, col_sum = clamped_swiglu_bwd_quant(
-            grad_h, gate_up, alpha, limit, offs if row_map is not None else None)
-        # groups are whole 128-row tiles: their ends in tiles index the per-tile column sums
-        grad_b_gate_up = _segment_sum_along_rows(col_sum, offs // 128, gu_bias_dtype)
-        grad_x = torch.empty((rows_x if row_map is not None else M, K), device=grad_out.device, dtype=grad_out.dtype)
-        m_grouped_fp8_dgrad((dgu_fp8, dgu_s), gu_dg, gu_dg_s, ctx.gu_forward_layout, grad_x, offs, row_map)
-        schedule_wgrad(w_gate_up, (dgu_ch_t, dgu_ch_s), (x_ch_t, x_ch_s), offs)
+        grad_x, grad_b_gate_up, grad_b_down = _backward(ctx, grad_out)
         return grad_x, None, grad_b_gate_up, None, grad_b_down, None, None, None, None, None, None, None

@@ -203,25 +203,35 @@ def k_grouped_fp8_wgrad(dy_t, x_t, out: torch.Tensor, grouped_mm_offs, accumulat
     return out
 
 
+def wgrad_target(weight: torch.Tensor):
+    """Where the weight-gradient GEMM of one grouped linear writes now: ``(tensor, accumulate, finish)``;
+    ``finish()`` (or None) completes the update of ``weight.grad`` once the GEMM is queued.  bf16(sum) is
+    formed in the GEMM's store, and an existing bf16 grad is accumulated there too."""
+    grad = weight.grad
+    if grad is not None and grad.dtype == torch.bfloat16 and grad.is_contiguous():
+        return grad, True, None
+    wg = torch.empty(weight.shape, device=weight.device, dtype=torch.bfloat16)
+
+    def finish():
+        if weight.grad is None:
+            weight.grad = wg if weight.dtype == torch.bfloat16 else wg.to(weight.dtype)
+        else:
+            weight.grad += wg
+
+    return wg, False, finish
+
+
 def schedule_wgrad(weight: torch.Tensor, a_wgrad: tuple, b_wgrad: tuple, offs: torch.Tensor) -> None:
     """Run - or, when ``WeightGradStore`` is enabled, queue - the weight-gradient GEMM of one
     grouped linear (``grad_weight_fn``, grouped_linear.py:202-234): ``a_wgrad`` / ``b_wgrad`` are the
     colwise-quantised transposed copies (fp8 ``[N, M]`` / ``[K, M]`` and their scales).  The result is
     written to ``weight.grad`` (assigned if None, accumulated otherwise)."""
-    num_groups, N, K = weight.shape
 
     def grad_weight_fn(a, b, offs):
-        # bf16(sum) is formed in the GEMM epilogue; an existing grad is accumulated there too
-        if weight.grad is None:
-            wg = torch.empty((num_groups, N, K), device=a[0].device, dtype=torch.bfloat16)
-            k_grouped_fp8_wgrad(a, b, wg, offs, accumulate=False)
-            weight.grad = wg if weight.dtype == torch.bfloat16 else wg.to(weight.dtype)
-        elif weight.grad.dtype == torch.bfloat16 and weight.grad.is_contiguous():
-            k_grouped_fp8_wgrad(a, b, weight.grad, offs, accumulate=True)
-        else:
-            wg = torch.empty((num_groups, N, K), device=a[0].device, dtype=torch.bfloat16)
-            k_grouped_fp8_wgrad(a, b, wg, offs, accumulate=False)
-            weight.grad += wg
+        out, accumulate, finish = wgrad_target(weight)
+        k_grouped_fp8_wgrad(a, b, out, offs, accumulate)
+        if finish is not None:
+            finish()
 
     if WeightGradStore.enabled:
         WeightGradStore.put(

@@ -61,5 +61,5 @@ def mla_decompress_backward(
     out_features = dk_nope.shape[2] * (dk_nope.shape[3] + dvalue.shape[3])
     dy2d = torch.cat([dk_nope, dvalue], dim=-1).reshape(b * n, out_features).to(nkv_blk.dtype)
     _, _, x_t_fp8, scale_x_t = fp8cast_rowwise_blockwise_transpose(nkv_blk.reshape(b * n, lora_rank), _padded=True)
-    d_nkv_2d, dW_blk = fp8_dgrad_wgrad(dy2d, weight_t_fp8, scale_weight_t, x_t_fp8, scale_x_t, lora_rank)
+    d_nkv_2d, dW_blk = fp8_dgrad_wgrad(dy2d, weight_t_fp8, scale_weight_t, x_t_fp8, scale_x_t, lora_rank, _zero_padded=True)
     return d_nkv_2d.view(b, n, lora_rank).to(torch.float32), dW_blk.to(torch.float32)

@@ -34,29 +34,33 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
 
 
-def group_rows(expert_idxs: torch.Tensor, num_groups: int, padding_alignment: int, cap: int):
-    """Index half of the scatter: (reverse i64[m], offs i32[G], ks i32[G], src_of i32[cap])."""
+def group_rows(expert_idxs: torch.Tensor, num_groups: int, padding_alignment: int, cap: int, need_reverse: bool = True):
+    """Index half of the scatter: (reverse i64[m], offs i32[G], ks i32[G], src_of i32[cap]); ``reverse`` is
+    None unless it is needed."""
     m = expert_idxs.shape[0]
     dev = expert_idxs.device
-    reverse = torch.empty((m,), device=dev, dtype=torch.int64)
-    offs = torch.empty((num_groups,), device=dev, dtype=torch.int32)
-    ks_tensor = torch.empty((num_groups,), device=dev, dtype=torch.int32)
-    src_of = torch.empty((cap,), device=dev, dtype=torch.int32)
+    reverse = torch.empty((m,), device=dev, dtype=torch.int64) if need_reverse else None
     ws_bytes = _lib.query("pt_group_rows_workspace_bytes", m, num_groups)
-    ws = _workspace(ws_bytes, dev)
+    # one allocation for the four int32 results and the workspace; src_of first, its start aligned
+    pad = -cap % 4
+    words = torch.empty((cap + pad + 2 * num_groups + ws_bytes // 4 + 64,), device=dev, dtype=torch.int32)
+    at = words.data_ptr()
+    offs_at = at + 4 * (cap + pad)
+    ws_at = (offs_at + 8 * num_groups + 255) & ~255
     _lib.call(
-        "pt_group_rows", expert_idxs.data_ptr(), m, num_groups, padding_alignment, offs.data_ptr(),
-        ks_tensor.data_ptr(), reverse.data_ptr(), src_of.data_ptr(), cap, ws.data_ptr(), ws.numel(),
-        _lib.stream_ptr(dev),
+        "pt_group_rows", expert_idxs.data_ptr(), m, num_groups, padding_alignment, offs_at, offs_at + 4 * num_groups,
+        _lib.ptr(reverse), at, cap, ws_at if ws_bytes else None, ws_bytes, _lib.stream_ptr(dev),
     )  # fmt: skip
-    return reverse, offs, ks_tensor, src_of
+    o = cap + pad
+    return reverse, words[o : o + num_groups], words[o + num_groups : o + 2 * num_groups], words[:cap]
 
 
 def group_rows_with_sizes(expert_idxs: torch.Tensor, num_groups: int, padding_alignment: int = 128, device=None,
-                          host_sizes: bool = True):
+                          host_sizes: bool = True, need_reverse: bool = True):
     """The index half of :func:`scatter_for_grouped_gemm` on its own: returns ``(reverse i64[m],
     grouped_mm_offs i32[G], ks list[int], ks_tensor i32[G], src_of i32[sum(ks)])`` where
     ``src_of[r]`` is the source row of grouped row r (-1 for a padding row).  No rows are moved.
+    ``need_reverse=False`` leaves ``reverse`` out (None), for callers that store rows through ``src_of``.
 
     ``host_sizes=False`` skips the device-to-host copy of the group sizes and the stream
     synchronisation it needs: ``ks`` is None and ``src_of`` keeps its full capacity (the largest
@@ -78,10 +82,10 @@ def group_rows_with_sizes(expert_idxs: torch.Tensor, num_groups: int, padding_al
         if (cap // 128) % 2 == 0:
             cap += 128
         alloc = -(-cap // _GEMM_ALLOC_ALIGNMENT) * _GEMM_ALLOC_ALIGNMENT
-        reverse, offs, ks_tensor, src_of = group_rows(expert_idxs, num_groups, padding_alignment, alloc)
+        reverse, offs, ks_tensor, src_of = group_rows(expert_idxs, num_groups, padding_alignment, alloc, need_reverse)
         return reverse, offs, None, ks_tensor, src_of[:cap]
     max_m_padded = -(-max_m_padded // _GEMM_ALLOC_ALIGNMENT) * _GEMM_ALLOC_ALIGNMENT
-    reverse, offs, ks_tensor, src_of = group_rows(expert_idxs, num_groups, padding_alignment, max_m_padded)
+    reverse, offs, ks_tensor, src_of = group_rows(expert_idxs, num_groups, padding_alignment, max_m_padded, need_reverse)
     ks_cpu = get_pinned_buffer("ks", num_groups, torch.int32)
     ks_cpu.copy_(ks_tensor, non_blocking=True)
     torch.cuda.current_stream(dev).synchronize()
