@@ -64,6 +64,9 @@ int pt_quant_rowwise_colwise_rows(const void* x, int dtype, int64_t M, int64_t N
                                   void* ch_fp8, float* ch_scale, int ch_layout,
                                   const int32_t* offs, int32_t num_groups, pt_stream_t stream);
 
+/* The transposed / column-scaled results (ch_fp8, ch_scale) of the row-scaled quantisers above and of the
+ * fused SwiGLU forwards below may be left out (both NULL) when no backward reads them. */
+
 /* SwiGLU fused into the activation quantisation (bf16 only).  Forward: h = bf16(silu(gate) * up)
  * with gate = gate_up[:, :half], up = gate_up[:, half:], quantised as pt_quant_rowwise_colwise
  * with the PT_CH_TRANSPOSED twin: tok_fp8[M,half], tok_scale[M,ceil(half/128)], ch_t_fp8[half,M],
@@ -119,12 +122,20 @@ int pt_quant_rowwise_transpose_ld(const void* x, int dtype, int64_t M, int64_t N
                                   void* tok_fp8, float* tok_scale, void* t_fp8, int64_t ld_t,
                                   float* t_scale, pt_stream_t stream);
 
+/* The same of a bf16 matrix [M, heads * (head_a + head_b)] given as two packed tensors x [M, heads, head_a] and
+ * x2 [M, heads, head_b] (dK and dV of an attention's latent projection, ring_attention.py:636-652)
+ * instead of their concatenation per head.  Head widths are multiples of 8. */
+int pt_quant_heads_rowwise_transpose_ld(const void* x, const void* x2, int64_t M, int64_t heads,
+                                        int64_t head_a, int64_t head_b, void* tok_fp8, float* tok_scale,
+                                        void* t_fp8, int64_t ld_t, float* t_scale, pt_stream_t stream);
+
 /* rowwise(x) + 128x128 blockwise(x^T): blk_t_fp8[K,M], blk_t_scale[ceil(K/128),ceil(M/128)].
  * fp8cast_rowwise_blockwise_transpose, deepgemm_quantize.py:575-629 */
 int pt_quant_rowwise_blockwise_transpose(const void* x, int dtype, int64_t M, int64_t K,
                                          int64_t ldx, void* tok_fp8, float* tok_scale,
                                          void* blk_t_fp8, float* blk_t_scale, pt_stream_t stream);
-/* The same with a row pitch ld_t >= M (bytes) for blk_t_fp8 (see pt_quant_rowwise_transpose_ld). */
+/* The same with a row pitch ld_t >= M (bytes) for blk_t_fp8 (see pt_quant_rowwise_transpose_ld).  One of
+ * the two results may be left out (NULL for its bytes and scales). */
 int pt_quant_rowwise_blockwise_transpose_ld(const void* x, int dtype, int64_t M, int64_t K,
                                             int64_t ldx, void* tok_fp8, float* tok_scale,
                                             void* blk_t_fp8, int64_t ld_t, float* blk_t_scale,
@@ -181,6 +192,14 @@ int pt_gemm_nt_dense(const void* a_fp8, const float* a_scale, const void* b_fp8,
 int pt_gemm_nt_dense_ld(const void* a_fp8, int64_t lda, const float* a_scale, const void* b_fp8,
                         int64_t ldb, const float* b_scale, void* out, int out_dtype, int64_t M,
                         int64_t N, int64_t K, pt_stream_t stream);
+/* pt_gemm_nt_dense (packed operands, bf16 result) whose columns go to two tensors, head by head: result
+ * column h * (head_a + head_b) + c is out[:, h * head_a + c] for c < head_a and
+ * out2[:, h * head_b + c - head_a] behind it; out [M, heads * head_a], out2 [M, heads * head_b] packed.
+ * out2 lies behind out in one allocation, together below 2 GiB; head widths are multiples of 8.
+ * The kv split of the MLA decompression (operators/ring_attention.py:428-457) without its copy. */
+int pt_gemm_nt_dense_heads(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,
+                           void* out, void* out2, int64_t head_a, int64_t head_b, int64_t M, int64_t N,
+                           int64_t K, pt_stream_t stream);
 /* Split-K form of pt_gemm_nt_dense for outputs with too few 256 x 256 tiles to fill the GPU (the
  * weight gradient of a dense linear, linear.py:61-83: M, N = weight dims, K = tokens): the
  * reduction is cut into `splits` ranges of split_len (a multiple of 128), range s is reduced into
@@ -579,13 +598,15 @@ int pt_experts_backward(const pt_experts_backward_args* args /* host */);
 int pt_experts_weight_gradient(const pt_experts_backward_args* args /* host */);
 /* Forward of a dense FP8 linear (fp8_act_weight_gemm, operators/linear.py:44-60): x [M, K] in dtype,
  * y [M, N] in y_dtype (PT_BF16 or PT_F32); x_t (row pitch ld_t >= M bytes) and x_t_scale are the transposed
- * operand the weight gradient reads.  K % 16 == 0. */
+ * operand the weight gradient reads (both NULL: not written).  K % 16 == 0.  y2 != NULL (bf16, splits == 1):
+ * the outputs of pt_gemm_nt_dense_heads. */
 typedef struct {
   const void* x; int64_t dtype, M, K, ldx;
   const void* w_fp8; const float* w_scale; int64_t N;
   void* y; int64_t y_dtype;
   void* x_t; int64_t ld_t; float* x_t_scale;
   int64_t splits, split_len;
+  void* y2; int64_t head_a, head_b;
   void* workspace;
   pt_stream_t stream;
 } pt_linear_forward_args;
@@ -596,17 +617,22 @@ int pt_linear_forward(const pt_linear_forward_args* args /* host */);
  * the transposed weight w_t [K, N], grad_w [N, K] through x_t [K, M]; both in out_dtype.  N % 16 == 0;
  * M % 16 == 0 unless x_t was written by pt_linear_forward with a pitch of at least M rounded up to 16
  * (its columns past M are zero).  splits / split_len per GEMM: the reduction ranges of
- * pt_gemm_nt_dense_splitk (1 = not split). */
+ * pt_gemm_nt_dense_splitk (1 = not split).  x_t NULL: the input x [M, K] (dtype, row stride ldx) is
+ * quantised here (workspace query with from_x != 0).  grad2 != NULL: the gradient's columns come from two
+ * tensors as in pt_quant_heads_rowwise_transpose_ld. */
 typedef struct {
   const void* grad; int64_t dtype, M, N, ldg;
   const void* w_t_fp8; const float* w_t_scale; int64_t K;
   const void* x_t; int64_t ld_xt; const float* x_t_scale;
   void* grad_x; void* grad_w; int64_t out_dtype;
   int64_t x_splits, x_split_len, w_splits, w_split_len;
+  const void* x; int64_t ldx;
+  const void* grad2; int64_t head_a, head_b;
   void* workspace;
   pt_stream_t stream;
 } pt_linear_backward_args;
-int64_t pt_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t x_splits, int64_t w_splits);
+int64_t pt_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t x_splits, int64_t w_splits,
+                                           int64_t from_x);
 int pt_linear_backward(const pt_linear_backward_args* args /* host */);
 
 /* Measurement: `fn`, when not NULL, is called on the host before (begin = 1) and after (begin = 0) every

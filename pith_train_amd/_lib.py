@@ -38,6 +38,7 @@ SIGNATURES = {
     "pt_quant_rowwise_blockwise_transpose": (c_int, [P, c_int, I64, I64, I64, P, P, P, P, P]),
     "pt_quant_rowwise_transpose_ld": (c_int, [P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_rowwise_blockwise_transpose_ld": (c_int, [P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
+    "pt_quant_heads_rowwise_transpose_ld": (c_int, [P, P, I64, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_blockwise_transpose_batched": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, P, P, P, P]),
     "pt_quant_blockwise_transpose_batched_into": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, I64, P, I64, P, I64, I64, P, I64,
                                                           I64, P]),
@@ -46,6 +47,7 @@ SIGNATURES = {
     "pt_gemm_nt_dense_splitk": (c_int, [P, P, P, P, P, I32, I64, I64, I64, I64, P]),
     "pt_gemm_nt_dense_ld": (c_int, [P, I64, P, P, I64, P, P, c_int, I64, I64, I64, P]),
     "pt_gemm_nt_dense_splitk_ld": (c_int, [P, I64, P, P, I64, P, P, I32, I64, I64, I64, I64, P]),
+    "pt_gemm_nt_dense_heads": (c_int, [P, P, P, P, P, P, I64, I64, I64, I64, I64, P]),
     "pt_sum_partials": (c_int, [P, I32, I64, P, c_int, P]),
     "pt_gemm_m_grouped_nt": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P]),
     "pt_gemm_m_grouped_nn": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P]),
@@ -95,7 +97,7 @@ SIGNATURES = {
     "pt_experts_weight_gradient": (c_int, [c_char_p]),
     "pt_linear_forward_workspace_bytes": (I64, [I64, I64, I64, I64]),
     "pt_linear_forward": (c_int, [c_char_p]),
-    "pt_linear_backward_workspace_bytes": (I64, [I64, I64, I64, I64, I64]),
+    "pt_linear_backward_workspace_bytes": (I64, [I64, I64, I64, I64, I64, I64]),
     "pt_linear_backward": (c_int, [c_char_p]),
     "pt_set_observer": (None, [P]),
 }

@@ -338,8 +338,8 @@ static int dispatch_gemm(const GemmArgs& g, hipStream_t stream) {
     const int rows = impl >= IMPL_SMALL ? impl - IMPL_SMALL : impl == IMPL_AUTO ? small_tile_rows(g) : 0;
     return rows ? launch_gemm_small(g, rows, stream) : launch_gemm_rowsplit(g, 0, stream);
   }
-  PT_REQUIRE((!g.out_row_index && !g.bias) || (impl != IMPL_TILE && fits),
-             "gemm: scattered output rows and the fused bias need the persistent kernels, which address every operand and "
+  PT_REQUIRE((!g.out_row_index && !g.bias && !g.head_a) || (impl != IMPL_TILE && fits),
+             "gemm: scattered output rows, per-head outputs and the fused bias need the persistent kernels, which address every operand and "
              "the output (one group's block of it in the k-grouped mode) through 32-bit byte offsets: operands below 2 GiB, "
              "output below 4 GiB");
   if (impl == IMPL_TILE || !fits) return launch_gemm<128, 128, 2, 2>(g, stream);
@@ -372,7 +372,7 @@ static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 static int gemm_nt_dense_impl(const void* a_fp8, int64_t lda, const float* a_scale, const void* b_fp8, int64_t ldb,
                               const float* b_scale, void* out, int out_dtype, int64_t M, int64_t N, int64_t K,
-                              pt_stream_t stream) {
+                              pt_stream_t stream, void* out2 = nullptr, int64_t head_a = 0, int64_t head_b = 0, int64_t extent = 0) {
   PT_REQUIRE(M >= 0 && N >= 0 && K >= 0, "gemm_nt_dense: negative size");
   if (M == 0 || N == 0) return PT_OK;
   PT_REQUIRE(K > 0 && K % 16 == 0, "gemm_nt_dense: K=%lld must be a positive multiple of 16", (long long)K);
@@ -389,6 +389,7 @@ static int gemm_nt_dense_impl(const void* a_fp8, int64_t lda, const float* a_sca
   g.a_bytes = (M - 1) * lda + K; g.b_bytes = (N - 1) * ldb + K; g.sa_bytes = M * KB * 4; g.sb_bytes = cdiv(N, 128) * KB * 4;
   g.tiles_a = (int)cdiv(M, 128); g.tiles_b = (int)cdiv(N, 128);
   g.total_tiles = (int64_t)g.tiles_a * g.tiles_b;
+  g.out2 = out2; g.head_a = (int)head_a; g.head_b = (int)head_b; g.out_extent = extent;
   return dispatch_gemm(g, (hipStream_t)stream);
 }
 
@@ -401,6 +402,19 @@ extern "C" int pt_gemm_nt_dense_ld(const void* a_fp8, int64_t lda, const float* 
                                    const float* b_scale, void* out, int out_dtype, int64_t M, int64_t N, int64_t K,
                                    pt_stream_t stream) {
   return gemm_nt_dense_impl(a_fp8, lda, a_scale, b_fp8, ldb, b_scale, out, out_dtype, M, N, K, stream);
+}
+
+extern "C" int pt_gemm_nt_dense_heads(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale, void* out, void* out2,
+                                      int64_t head_a, int64_t head_b, int64_t M, int64_t N, int64_t K, pt_stream_t stream) {
+  if (M == 0 || N == 0) return PT_OK;
+  PT_REQUIRE(head_a > 0 && head_b > 0 && head_a % 8 == 0 && head_b % 8 == 0 && N % (head_a + head_b) == 0,
+             "gemm_nt_dense_heads: head widths must be multiples of 8 that make up N");
+  const int64_t heads = N / (head_a + head_b);
+  PT_REQUIRE(out && out2 && al16(out) && al16(out2) && (char*)out2 >= (char*)out + M * heads * head_a * 2,
+             "gemm_nt_dense_heads: the second output lies behind the first, both 16-byte aligned");
+  const int64_t extent = ((char*)out2 - (char*)out) + M * heads * head_b * 2;
+  PT_REQUIRE(extent < (1ll << 31), "gemm_nt_dense_heads: outputs are stored through 32-bit byte offsets (below 2 GiB)");
+  return gemm_nt_dense_impl(a_fp8, K, a_scale, b_fp8, K, b_scale, out, PT_BF16, M, N, K, stream, out2, head_a, head_b, extent);
 }
 
 // ---- split-K: a dense GEMM whose output has too few tiles to fill the GPU ------------------------

@@ -27,6 +27,9 @@ struct GemmArgs {
   void* out2; int64_t split_row;          // k-grouped: result rows from split_row on (a multiple of 128; 0 = none) go to out2, a second
                                           // parameter's gradient (group stride out2_stride_g) whose row 0 is row split_row
   int64_t out2_stride_g;
+  int head_a, head_b;                     // dense only: result column h * (head_a + head_b) + c is out[h * head_a + c] for c < head_a, else
+                                          // out2[h * head_b + c - head_a]; out2 lies behind out in one allocation (head_a == 0: one output)
+  int64_t out_extent;                     // with head_a: bytes from out to the end of out2, below 2 GiB
   int b_kmajor;                           // m-grouped, row-split kernel: b is [red, rows_b] per group (row pitch ldb) instead of [rows_b, red]
 };
 

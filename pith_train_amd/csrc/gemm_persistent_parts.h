@@ -446,7 +446,31 @@ __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& 
   const uint32_t s_tile = (uint32_t)row0 * pitch + (uint32_t)(T.b_row0 + wn0) * esz;
   const int colw = T.b_row0 + wn0 + (lane & 31);
   static_assert(TN % 2 == 0, "the wide stores take column blocks in pairs");
-  if (MODE == GEMM_M_GROUPED && p.out_row_index) {
+  if (MODE == GEMM_DENSE && p.head_a) {
+    // Per-head halves in two tensors: a lane's eight columns lie in one of them (both widths are multiples
+    // of 8), so its offset from `out` and its row pitch are all that differ.
+    const __amdgpu_buffer_rsrc_t rs_heads = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, kAblateStores ? 0 : (int)p.out_extent, kRsrcFlags);
+    const int width = p.head_a + p.head_b, heads = (int)p.rows_b / width;
+#pragma unroll
+    for (int j = 0; j < TN; j += 2) {
+      const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;
+      const int h = colc / width, c = colc - h * width;
+      const bool second = c >= p.head_a;
+      const uint32_t at = second ? (uint32_t)((char*)p.out2 - (char*)p.out) + (uint32_t)(h * p.head_b + c - p.head_a) * 2 : (uint32_t)(h * p.head_a + c) * 2;
+      const uint32_t pitch_h = (uint32_t)(heads * (second ? p.head_b : p.head_a)) * 2;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        uint32_t voff[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int r = row0 + i * 32 + q * 8 + (lane >> 3);
+          voff[q] = colc < T.b_lim && r < row_lim ? (uint32_t)r * pitch_h + at : kOob;
+        }
+        pin_acc<PIN>(acc[i][j]); pin_acc<PIN>(acc[i][j + 1]);
+        store_staged_bf16_lines<kStoreAux<MODE>>(acc[i][j], acc[i][j + 1], rs_heads, stg, voff, 0, false, lane);
+      }
+    }
+  } else if (MODE == GEMM_M_GROUPED && p.out_row_index) {
     // Result row r goes to output row out_row_index[r] (the un-permute folded into the store);
     // rows of the group's padding map to a negative index and are dropped.
     const __amdgpu_buffer_rsrc_t rs_sc = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, kAblateStores ? 0 : (int)((uint32_t)p.out_rows * pitch), kRsrcFlags);

@@ -170,36 +170,59 @@ extern "C" int pt_linear_forward(const pt_linear_forward_args* args) {
   Carve ws(a.workspace);
   void* x_fp8 = ws.bytes(a.M * a.K);
   float* x_s = ws.floats(a.M * cdiv(a.K, 128));
-  PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, x_fp8, x_s, a.x_t, a.ld_t,
+  PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, x_fp8, x_s, a.x_t, a.x_t ? a.ld_t : a.M,
           a.x_t_scale, a.stream);
+  if (a.y2) {
+    PT_STEP(pt_gemm_nt_dense_heads, a.M, a.N, a.K, x_fp8, x_s, a.w_fp8, a.w_scale, a.y, a.y2, a.head_a, a.head_b, a.M, a.N, a.K, a.stream);
+    return PT_OK;
+  }
   return dense_gemm(x_fp8, a.K, x_s, a.w_fp8, a.K, a.w_scale, a.y, (int)a.y_dtype, a.M, a.N, a.K, a.splits, a.split_len,
                     (float*)(void*)ws.p, a.stream);
 }
 
-// workspace: gradient bytes and scales | its transposed form and scales | slabs of whichever GEMM is split
-extern "C" int64_t pt_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t x_splits, int64_t w_splits) {
+// a pitch that is no multiple of 256 bytes spreads the rows of a reduction step over the memory channels
+static int64_t transposed_pitch(int64_t red) { return red >= 2048 && red % 256 == 0 ? red + 128 : red; }
+
+// workspace: gradient bytes and scales | its transposed form and scales | the input's transposed form and
+// scales when it is quantised here | slabs of whichever GEMM is split
+extern "C" int64_t pt_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t x_splits, int64_t w_splits, int64_t from_x) {
   const int64_t sx = x_splits > 1 ? 4 * x_splits * M * K : 0, sw = w_splits > 1 ? 4 * w_splits * N * K : 0;
-  return up(M * N) + up(4 * M * cdiv(N, 128)) + up(N * (M + 256)) + up(4 * N * cdiv(M, 128)) + up(sx > sw ? sx : sw);
+  return up(M * N) + up(4 * M * cdiv(N, 128)) + up(N * (M + 256)) + up(4 * N * cdiv(M, 128)) + up(sx > sw ? sx : sw) +
+         (from_x ? up(K * (M + 256)) + up(4 * cdiv(K, 128) * cdiv(M, 128)) : 0);
 }
 
 extern "C" int pt_linear_backward(const pt_linear_backward_args* args) {
   PT_REQUIRE(args, "linear_backward: null arguments");
   const pt_linear_backward_args& a = *args;
-  PT_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0 && a.grad && a.workspace, "linear_backward: bad arguments");
+  PT_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0 && a.grad && a.workspace && (a.x_t || a.x), "linear_backward: bad arguments");
   const int64_t red = (a.M + 15) & ~(int64_t)15;  // the weight gradient's reduction, zero-filled to whole 16-byte chunks
-  PT_REQUIRE(a.ld_xt >= red && a.ld_xt % 16 == 0, "linear_backward: the transposed input needs a row pitch of %lld or more, a multiple of 16",
-             (long long)red);
-  // a pitch that is no multiple of 256 bytes spreads the rows of a reduction step over the memory channels
-  const int64_t ld_t = red >= 2048 && red % 256 == 0 ? red + 128 : red;
+  PT_REQUIRE(!a.x_t || (a.ld_xt >= red && a.ld_xt % 16 == 0),
+             "linear_backward: the transposed input needs a row pitch of %lld or more, a multiple of 16", (long long)red);
+  const int64_t ld_t = transposed_pitch(red);
   Carve ws(a.workspace);
   void* g_fp8 = ws.bytes(a.M * a.N);
   float* g_s = ws.floats(a.M * cdiv(a.N, 128));
   void* g_t = ws.bytes(a.N * (a.M + 256));
   float* g_ts = ws.floats(a.N * cdiv(a.M, 128));
+  const void* x_t = a.x_t;
+  const float* x_ts = a.x_t_scale;
+  int64_t ld_xt = a.ld_xt;
+  if (!x_t) {
+    void* t = ws.bytes(a.K * (a.M + 256));
+    float* ts = ws.floats(cdiv(a.K, 128) * cdiv(a.M, 128));
+    ld_xt = ld_t;
+    PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, nullptr, nullptr, t, ld_xt, ts, a.stream);
+    x_t = t;
+    x_ts = ts;
+  }
   float* slabs = (float*)(void*)ws.p;
-  PT_STEP(pt_quant_rowwise_transpose_ld, a.M, a.N, a.M, a.grad, (int)a.dtype, a.M, a.N, a.ldg, g_fp8, g_s, g_t, ld_t, g_ts, a.stream);
+  if (a.grad2)
+    PT_STEP(pt_quant_heads_rowwise_transpose_ld, a.M, a.N, a.M, a.grad, a.grad2, a.M, a.N / (a.head_a + a.head_b), a.head_a, a.head_b, g_fp8,
+            g_s, g_t, ld_t, g_ts, a.stream);
+  else
+    PT_STEP(pt_quant_rowwise_transpose_ld, a.M, a.N, a.M, a.grad, (int)a.dtype, a.M, a.N, a.ldg, g_fp8, g_s, g_t, ld_t, g_ts, a.stream);
   if (int rc = dense_gemm(g_fp8, a.N, g_s, a.w_t_fp8, a.N, a.w_t_scale, a.grad_x, (int)a.out_dtype, a.M, a.K, a.N, a.x_splits,
                           a.x_split_len, slabs, a.stream)) return rc;
-  return dense_gemm(g_t, ld_t, g_ts, a.x_t, a.ld_xt, a.x_t_scale, a.grad_w, (int)a.out_dtype, a.N, a.K, red, a.w_splits, a.w_split_len,
+  return dense_gemm(g_t, ld_t, g_ts, x_t, ld_xt, x_ts, a.grad_w, (int)a.out_dtype, a.N, a.K, red, a.w_splits, a.w_split_len,
                     slabs, a.stream);
 }

@@ -64,9 +64,9 @@ enum { BS_MB_N = 0, BS_N_MB = 1 };                     // twin scale layout for 
 struct QuantArgs {
   const void* x;
   int64_t M, N, ldx, x_stride_g;
-  uint8_t* a_out;  int64_t a_stride_g;   // [M,N] bytes, ld = N
+  uint8_t* a_out;  int64_t a_stride_g;   // [M,N] bytes, ld = N; row-scaled launches: null = not written
   float* a_scale;  int64_t a_scale_stride_g;
-  uint8_t* b_out;  int64_t b_stride_g;   // rowmajor [M,N] / transposed [N,M] / kmajor flat
+  uint8_t* b_out;  int64_t b_stride_g;   // rowmajor [M,N] / transposed [N,M] / kmajor flat; row-scaled launches: null = not written
   float* b_scale;  int64_t b_scale_stride_g;
   int32_t tiles_m, tiles_n;
   const int32_t* offs; int32_t num_groups;  // KMAJOR only
@@ -81,6 +81,7 @@ struct QuantArgs {
   int64_t bs_ld;                 // row length of the twin's block-scale grid; tiles_m unless it is a column slice
   float alpha, limit;            // fused clamped SwiGLU: its two constants
   float* col_sum;                // fused clamped SwiGLU backward: [tiles_m, N] column sums of each 128-row tile
+  int32_t head_a, head_b;        // per-head halves in two tensors: column h * (head_a + head_b) + c is x[h * head_a + c] or x2[h * head_b + c - head_a]
 };
 
 template <typename T> struct Loader;
@@ -187,7 +188,8 @@ template <> struct Frag<float> {
 };
 
 // what the tile is computed from
-enum { PRO_NONE = 0, PRO_SILU_FWD = 1, PRO_SILU_BWD = 2, PRO_SILU_BWD_PAIR = 3, PRO_CSWIGLU_FWD = 4, PRO_CSWIGLU_BWD = 5 };
+enum { PRO_NONE = 0, PRO_SILU_FWD = 1, PRO_SILU_BWD = 2, PRO_SILU_BWD_PAIR = 3, PRO_CSWIGLU_FWD = 4, PRO_CSWIGLU_BWD = 5,
+       PRO_HEADS = 6 };
 
 // ---- packed-bf16 arithmetic of the interior-tile path -------------------------------------------
 // |x| of a bf16 is its low 15 bits, and for non-negative floats the integer order of the bits is
@@ -305,6 +307,21 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
       } else {
         f.zero_row(i);
       }
+    }
+  } else if constexpr (PRO == PRO_HEADS) {
+    // The columns of every head come from two tensors (dK | dV of an attention's latent projection): the
+    // thread's eight columns lie in one of them, so only its base and pitch differ.
+    const int64_t width = p.head_a + p.head_b, heads = p.N / width;
+    const int64_t h = col0 / width, c = col0 - h * width;
+    const bool second = c >= p.head_a;
+    const char* base = second ? (const char*)p.x2 + (h * p.head_b + c - p.head_a) * 2 : xb + (h * p.head_a + c) * 2;
+    const int64_t pitch = heads * (second ? p.head_b : p.head_a) * 2;
+    base += row0 * pitch;
+    const bool col_ok = FULL || col0 < p.N;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (FULL || (col_ok && row0 + i < p.M)) f.load_row(i, base + i * pitch);
+      else f.zero_row(i);
     }
   } else if constexpr (PRO != PRO_NONE) {
     // The quantised tensor is the bf16-rounded SwiGLU output (forward: h = silu(gate) * up from
@@ -457,7 +474,8 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
   };
   // Row-scaled output needs nothing from the other phases: write it now so that the row maxima
   // are dead before the column phase starts (fewer live registers, more resident waves).
-  if (AM == A_ROW) write_same_orientation(0.f, 0.f);
+  if (AM == A_ROW && p.a_out) write_same_orientation(0.f, 0.f);
+  if (AM == A_ROW && !p.b_out) return;  // nobody reads the twin (no backward follows)
 
   f.fence();
   float colmax[8];
@@ -789,6 +807,7 @@ static void fill_common(QuantArgs& a, const void* x, int dtype, int64_t M, int64
   a.tiles_m = (int32_t)cdiv(M, 128); a.tiles_n = (int32_t)cdiv(N, 128);
   a.offs = nullptr; a.num_groups = 0; a.row_index = nullptr; a.x2 = nullptr; a.ldx2 = 0; a.half = 0;
   a.row_limit = nullptr; a.ld_t = M; a.bs_ld = a.tiles_m; a.alpha = 0.f; a.limit = 0.f; a.col_sum = nullptr;
+  a.head_a = a.head_b = 0;
   const int eb = dtype == PT_F32 ? 4 : 2;
   a.vec_in = (N % 8 == 0) && ((ldx * eb) % 16 == 0) && (((uintptr_t)x) % 16 == 0);
   a.vec_out = (N % 8 == 0);
@@ -826,7 +845,7 @@ static int quant_rowwise_colwise_impl(const void* x, int dtype, int64_t M, int64
   PT_REQUIRE(M >= 0 && N >= 0 && M % 128 == 0, "quant_rowwise_colwise: M=%lld must be a multiple of 128", (long long)M);
   PT_REQUIRE(ldx >= N, "quant_rowwise_colwise: ldx < N");
   if (M == 0 || N == 0) return PT_OK;
-  PT_REQUIRE(x && tok_fp8 && tok_scale && ch_fp8 && ch_scale, "quant_rowwise_colwise: null pointer");
+  PT_REQUIRE(x && tok_fp8 && tok_scale && (ch_fp8 == nullptr) == (ch_scale == nullptr), "quant_rowwise_colwise: null pointer");
   QuantArgs a;
   fill_common(a, x, dtype, M, N, ldx);
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_fp8; a.b_scale = ch_scale;
@@ -876,12 +895,35 @@ extern "C" int pt_quant_rowwise_transpose_ld(const void* x, int dtype, int64_t M
   return quant_rowwise_transpose_impl(x, dtype, M, N, ldx, tok_fp8, tok_scale, t_fp8, ld_t, t_scale, stream);
 }
 
+extern "C" int pt_quant_heads_rowwise_transpose_ld(const void* x, const void* x2, int64_t M, int64_t heads, int64_t head_a, int64_t head_b,
+                                                   void* tok_fp8, float* tok_scale, void* t_fp8, int64_t ld_t, float* t_scale,
+                                                   pt_stream_t stream) {
+  const int64_t N = heads * (head_a + head_b);
+  PT_REQUIRE(M >= 0 && heads >= 0 && head_a > 0 && head_b > 0 && N < (1ll << 31) && ld_t >= M, "quant_heads_rowwise_transpose: bad shape");
+  if (M == 0 || N == 0) return PT_OK;
+  PT_REQUIRE(x && x2 && tok_fp8 && tok_scale && t_fp8 && t_scale, "quant_heads_rowwise_transpose: null pointer");
+  PT_REQUIRE(head_a % 8 == 0 && head_b % 8 == 0 && (((uintptr_t)x | (uintptr_t)x2) & 15) == 0,
+             "quant_heads_rowwise_transpose: head widths must be multiples of 8 elements, pointers 16-byte aligned");
+  QuantArgs a;
+  fill_common(a, x, PT_BF16, M, N, N);
+  a.x2 = x2; a.head_a = (int32_t)head_a; a.head_b = (int32_t)head_b;
+  a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)t_fp8; a.b_scale = t_scale;
+  a.ld_t = ld_t;
+  a.vec_out_t = whole_chunks(M, ld_t, t_fp8);
+  const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
+  PT_REQUIRE(blocks < (1ll << 31), "quant: grid too large (%lld tiles)", (long long)blocks);
+  hipLaunchKernelGGL((quant_tile_kernel<bf16_tag, A_ROW, B_COL, BL_TRANSPOSED, BS_N_MB, PRO_HEADS>), dim3((unsigned)blocks), dim3(256), 0,
+                     (hipStream_t)stream, a);
+  return check_launch("quant_tile_kernel(heads)");
+}
+
 static int quant_rowwise_blockwise_transpose_impl(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, void* tok_fp8,
                                                   float* tok_scale, void* blk_t_fp8, int64_t ld_t, float* blk_t_scale,
                                                   pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && K >= 0 && ldx >= K && ld_t >= M, "quant_rowwise_blockwise_transpose: bad shape");
   if (M == 0 || K == 0) return PT_OK;
-  PT_REQUIRE(x && tok_fp8 && tok_scale && blk_t_fp8 && blk_t_scale, "quant_rowwise_blockwise_transpose: null pointer");
+  PT_REQUIRE(x && (tok_fp8 == nullptr) == (tok_scale == nullptr) && (blk_t_fp8 == nullptr) == (blk_t_scale == nullptr) && (tok_fp8 || blk_t_fp8),
+             "quant_rowwise_blockwise_transpose: null pointer");
   QuantArgs a;
   fill_common(a, x, dtype, M, K, ldx);
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)blk_t_fp8; a.b_scale = blk_t_scale;
@@ -999,7 +1041,7 @@ extern "C" int pt_silu_mul_quant_rowwise_colwise(const void* gate_up, int64_t M,
                                                  const int32_t* valid_rows, pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half, "silu_mul_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
-  PT_REQUIRE(gate_up && tok_fp8 && tok_scale && ch_t_fp8 && ch_scale, "silu_mul_quant: null pointer");
+  PT_REQUIRE(gate_up && tok_fp8 && tok_scale && (ch_t_fp8 == nullptr) == (ch_scale == nullptr), "silu_mul_quant: null pointer");
   PT_REQUIRE(half % 8 == 0 && ld_gate_up % 8 == 0 && ((uintptr_t)gate_up) % 16 == 0,
              "silu_mul_quant: the half width and the row stride must be multiples of 8 elements, the pointer 16-byte aligned");
   QuantArgs a;
@@ -1035,7 +1077,7 @@ extern "C" int pt_clamped_swiglu_quant_rowwise_colwise(const void* gate_up, int6
                                                        pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half, "clamped_swiglu_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
-  PT_REQUIRE(gate_up && tok_fp8 && tok_scale && ch_t_fp8 && ch_scale, "clamped_swiglu_quant: null pointer");
+  PT_REQUIRE(gate_up && tok_fp8 && tok_scale && (ch_t_fp8 == nullptr) == (ch_scale == nullptr), "clamped_swiglu_quant: null pointer");
   PT_REQUIRE(half % 8 == 0 && ld_gate_up % 8 == 0 && ((uintptr_t)gate_up) % 16 == 0,
              "clamped_swiglu_quant: the output width and the row stride must be multiples of 8 elements, the pointer 16-byte aligned");
   QuantArgs a;

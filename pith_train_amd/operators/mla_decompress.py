@@ -18,7 +18,7 @@ import torch
 import torch.nn.functional as F
 
 from .deepgemm_quantize import fp8cast_rowwise_blockwise_transpose
-from .linear import fp8_act_weight_gemm, fp8_dgrad_wgrad
+from .linear import fp8_act_weight_gemm, fp8_act_weight_gemm_heads, fp8_dgrad_wgrad, fp8_dgrad_wgrad_heads
 
 
 def mla_decompress(
@@ -37,6 +37,10 @@ def mla_decompress(
     b, n, _ = normed_kv.shape
     if use_fp8:
         x2d = normed_kv.reshape(b * n, normed_kv.shape[-1])
+        # the GEMM stores both parts where they belong (4096 rows: the copy of the values took 10 us)
+        parts = fp8_act_weight_gemm_heads(x2d, weight_fp8, scale_weight, num_heads, qk_nope_head_dim, v_head_dim)
+        if parts is not None:
+            return parts[0].view(b, n, num_heads, qk_nope_head_dim), parts[1].view(b, n, num_heads, v_head_dim)
         kv2d, _, _ = fp8_act_weight_gemm(x2d, weight_fp8, scale_weight)
         kv = kv2d.view(b, n, num_heads, qk_nope_head_dim + v_head_dim)
     else:
@@ -59,6 +63,11 @@ def mla_decompress_backward(
     fp32)`` through the FP8 dgrad / wgrad of the dense linear."""
     b, n, lora_rank = nkv_blk.shape
     out_features = dk_nope.shape[2] * (dk_nope.shape[3] + dvalue.shape[3])
+    # the quantiser reads both parts in place and the GEMMs store fp32 (4096 rows: concatenation and casts took 37 us)
+    grads = fp8_dgrad_wgrad_heads(dk_nope.flatten(0, 1), dvalue.flatten(0, 1), weight_t_fp8, scale_weight_t,
+                                  nkv_blk.reshape(b * n, lora_rank), lora_rank)  # fmt: skip
+    if grads is not None:
+        return grads[0].view(b, n, lora_rank), grads[1]
     dy2d = torch.cat([dk_nope, dvalue], dim=-1).reshape(b * n, out_features).to(nkv_blk.dtype)
     _, _, x_t_fp8, scale_x_t = fp8cast_rowwise_blockwise_transpose(nkv_blk.reshape(b * n, lora_rank), _padded=True)
     d_nkv_2d, dW_blk = fp8_dgrad_wgrad(dy2d, weight_t_fp8, scale_weight_t, x_t_fp8, scale_x_t, lora_rank, _zero_padded=True)

@@ -47,3 +47,33 @@ def test_decompress_forward_backward(b, n, heads, nope, vdim, rank):
     assert d_nkv.shape == (b, n, rank) and dW.shape == (out_features, rank)
     _close(d_nkv, gi_ref.view(b, n, rank), "d_nkv")
     _close(dW, gw_ref, "dW")
+
+
+@pytest.mark.parametrize("rows,heads,nope,vdim,rank,fused", [
+    (16, 1, 8, 8, 128, True), (129, 3, 24, 40, 144, True), (1000, 4, 64, 32, 256, True), (384, 4, 128, 128, 512, True),
+    (520, 16, 128, 64, 512, True), (200, 2, 20, 44, 128, False)])
+def test_per_head_halves_have_the_bits_of_the_concatenated_tensors(rows, heads, nope, vdim, rank, fused):
+    """The GEMM that stores both halves of every head and the quantiser that reads them, against the dense
+    linear on the concatenated tensors: ragged rows, widths below and across a tile's columns, and a
+    width that is no multiple of 8, which goes the concatenated way."""
+    from pith_train_amd.operators import linear as L
+    from pith_train_amd.operators.deepgemm_quantize import fp8cast_blockwise_transpose, fp8cast_rowwise_blockwise_transpose
+    from pith_train_amd.operators.mla_decompress import mla_decompress, mla_decompress_backward
+
+    n = heads * (nope + vdim)
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn((rows, rank), generator=g).bfloat16().cuda()
+    w_fp8, w_s, w_t, w_t_s = fp8cast_blockwise_transpose((torch.randn((n, rank), generator=g) * 0.02).bfloat16().cuda())
+    dk = torch.randn((rows, heads, nope), generator=g).bfloat16().cuda()
+    dv = torch.randn((rows, heads, vdim), generator=g).bfloat16().cuda()
+
+    assert (L.fp8_act_weight_gemm_heads(x, w_fp8, w_s, heads, nope, vdim) is not None) == fused
+    k_nope, value = mla_decompress(x[None], None, heads, nope, vdim, use_fp8=True, weight_fp8=w_fp8, scale_weight=w_s)
+    kv = L.fp8_act_weight_gemm(x, w_fp8, w_s)[0].view(rows, heads, nope + vdim)
+    assert torch.equal(k_nope[0], kv[..., :nope]) and torch.equal(value[0], kv[..., nope:])
+
+    d_x, d_w = mla_decompress_backward(dk[None], dv[None], x[None], w_t, w_t_s)
+    x_t, x_t_s = fp8cast_rowwise_blockwise_transpose(x, _padded=True)[2:]
+    want = L.fp8_dgrad_wgrad(torch.cat([dk, dv], -1).view(rows, n), w_t, w_t_s, x_t, x_t_s, rank, _zero_padded=True)
+    # the concatenated way rounds to bf16 before it widens
+    assert torch.equal(d_x[0].bfloat16(), want[0]) and torch.equal(d_w.bfloat16(), want[1])
