@@ -300,18 +300,38 @@ static int preferred_kernel(const GemmArgs& g) {
   return g.red >= 512 ? KERNEL_PIPELINED : KERNEL_TWO_PHASE;
 }
 
-// Problems too small for 256 x 256 tiles to fill 256 compute units go to the kernel with one 64 x 128 or
-// 128 x 128 tile per workgroup (gemm_small.hip): tile rows, or 0 when the persistent kernels are the
-// better choice.  While all 64-row tiles run at once the smaller tile wins (1001 x 512 x 2048: 10.5 us
-// against 13.1 with 128 rows and 25.0 for the pipelined kernel; 4096 x 512 x 4096: 18.5, 23.4, 46.0);
-// with more of them, 128-row tiles do up to two rounds of workgroups (2048 x 2048 x 2816, 256 tiles: 19.0
-// against 35.4; 4096 x 2048 x 2048, 512 tiles: 27.8 against 28.8; 4352 x 2048 x 1536 in 16 groups, 544
-// tiles: 31.9 against 27.5), past which the persistent kernels' overlap of one tile's stores with the
-// next tile's loads counts for more.
+// Problems too small for 256 x 256 tiles to fill 256 compute units evenly go to the kernel with one 64 x 128
+// or 128 x 128 tile per workgroup and two workgroups per compute unit (gemm_small.hip): tile rows, or 0
+// when the persistent kernels are the better choice.  While all 64-row tiles run at once the smaller tile
+// wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 25.0 for the pipelined kernel).  Then both
+// kinds are priced in rounds of the GPU: a round of 256 large tiles is the unit, a round of 512 small ones
+// (a quarter of the area each, half of it in all) costs 0.57 of it in the m-grouped mode, 0.65 in
+// the dense one, where the large tiles have the better loop (0.45 up to a reduction of 512, most of it
+// filling and draining), 0.43 for a weight gradient over groups of up to 1024 rows (mostly stores, which
+// one workgroup of a unit does while the other loads; longer ones are like dense products).  A partly filled round of small tiles costs half of what it leaves idle.  Us,
+// large / small: m-grouped, K 2048, N 1536: 16 groups of 256 rows 26.1 / 18.0, of 512 33.3 / 32.1, of 640
+// 60.4 / 36.4, of 1024 62.9 / 56.0; 64 groups of 128 51.5 / 40.7, of 384 90 / 85, of 512 105 / 115.  Dense
+// 4096 x 2048 x 2048 28.7 / 19.3, 4096 x 4096 x 2048 32.7 / 38.0.  Weight gradients 1536 x 2048 of 16
+// groups of 128 rows 28.2 / 23.1, of 1024 61.1 / 57.1; of 64 groups 73 / 83.  Past three to four rounds
+// large tiles have no round to waste and need half of the operand traffic.
 static int small_tile_rows(const GemmArgs& g) {
-  const int64_t cols = cdiv(g.rows_b, 128) * (g.mode == GEMM_K_GROUPED ? g.G : 1);
+  const int64_t groups = g.mode == GEMM_K_GROUPED ? g.G : 1;
+  const int64_t cols = cdiv(g.rows_b, 128) * groups, cols_large = cdiv(g.rows_b, 256) * groups;
   if (cdiv(g.rows_a, 64) * cols <= 256) return 64;
-  return cdiv(g.rows_a, 128) * cols <= 512 ? 128 : 0;
+  const int64_t small = cdiv(g.rows_a, 128) * cols;
+  if (small <= 512) return 128;
+  int64_t rows_large = cdiv(g.rows_a, 256);
+  if (g.mode == GEMM_M_GROUPED) {  // half of the groups end in half a tile
+    const int64_t blocks = g.rows_a / 128, least = blocks < g.G ? blocks : g.G;
+    rows_large = (blocks + g.G / 2) / 2;
+    if (rows_large < least) rows_large = least;
+  }
+  const int64_t large = rows_large * cols_large;
+  if (large > (g.mode == GEMM_K_GROUPED ? 1024 : 768)) return 0;
+  const int64_t depth = g.mode == GEMM_K_GROUPED ? g.red / g.G : g.red;
+  const int64_t price = g.mode == GEMM_M_GROUPED ? 57 : g.mode == GEMM_K_GROUPED ? (depth <= 1024 ? 43 : 65) : depth <= 512 ? 45 : 65;
+  // in units of 1 / (100 * 512 * 2) of a round of large tiles, five percent in favour of those
+  return (small + cdiv(small, 512) * 512) * price * 105 < cdiv(large, 256) * (2 * 512 * 100) * 100 ? 128 : 0;
 }
 
 // The persistent kernels address operands through 32-bit buffer offsets (signed range for the

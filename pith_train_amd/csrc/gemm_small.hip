@@ -2,12 +2,14 @@
 //
 // A layer with few tokens has a handful of large tiles: most compute units stay idle, and the ones
 // that work spend their time waiting for one operand stage after the other.  Here a workgroup of
-// four waves owns one BM x 128 tile (BM = 64 or 128), so there are four to eight times as many
-// workgroups, and the LDS holds a ring of four or five 128-deep stages, all of them requested
-// ahead: a step waits only for the stage requested three or four steps earlier.  There is no
-// persistent loop, no tile table and no scan over the groups (a tile finds its group with one
-// ballot over the group ends), which keeps the time before the first load and the code that has to
-// be fetched short.
+// four waves owns one BM x 128 tile (BM = 64 or 128) with a ring of two or three 128-deep stages, small
+// enough that a compute unit holds two workgroups: while one waits for its first stage, drains its
+// pipeline or stores its result, the other multiplies.  (One workgroup per unit with four to five stages
+// in flight is level while there is only one tile per unit, and slower with more: 512 tiles of
+// 4096 x 2048 x 2048 28.7 us against 19.3, 128 groups of 128 rows with 1536 x 2048 weights 105 against 95.)
+// There is no persistent loop, no tile table and no scan over the groups (a tile finds its group with
+// one ballot over the group ends), which keeps the time before the first load and the code that has to
+// be fetched short.  Operand traffic bounds it from the L2 on: 10 to 14 TB/s.
 //
 // Operand layouts in LDS, direct-to-LDS loads, scale handling and result stores are those of the
 // persistent kernels (gemm_persistent_parts.h); the MFMAs run in the same order, so the results have
@@ -16,17 +18,22 @@
 
 namespace pt {
 
+// LDS of a workgroup: the ring of stages, their scales, a sink for scale loads that nobody needs
+// (65.3 or 74.5 KiB: two workgroups share a compute unit)
+template <int BM> static constexpr int kSmallStages = BM == 64 ? 3 : 2;
+template <int BM> static constexpr size_t kSmallLds = (size_t)kSmallStages<BM> * (BM + 128) * (128 + 4) + 256;
+
 template <int MODE, int BM, bool ACC, bool BT>
-__global__ __launch_bounds__(256, 1) void fp8_gemm_small_kernel(GemmArgs p) {
-  constexpr int BN = 128, BK = 128;
-  constexpr int NS = BM == 64 ? 5 : 4;  // stages in the LDS ring: 120 or 128 KiB
+__global__ __launch_bounds__(256, 2) void fp8_gemm_small_kernel(GemmArgs p) {
+  constexpr int BN = 128, BK = 128, NS = kSmallStages<BM>;
+  static_assert(2 * kSmallLds<BM> <= 160 * 1024, "two workgroups per compute unit");
   constexpr int TM = BM / 64, TN = 2;   // waves 2 x 2, each TM x 2 blocks of 32 x 32
   constexpr int STAGE = (BM + BN) * BK;
   constexpr int LA = BM / 32, LB = BN / 32;  // 1 KiB loads of a and of b per wave and stage
   constexpr int NP = LA + LB + 1;            // and one of scales
   constexpr int kWait = (NS - 2) * NP;       // loads of the stages after the one a step needs
   static_assert(kWait < 64, "vmcnt is a 6-bit counter");
-  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // [NS][STAGE] | [NS][BM + BN] scales | 256 B sink | staging
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // [NS][STAGE] | [NS][BM + BN] scales | 256 B sink; the stores' staging takes the first 8 KiB afterwards
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -43,15 +50,20 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_small_kernel(GemmArgs p) {
   if (idx >= per_xcd || t >= total) return;
   Tile T;
   if (MODE == GEMM_M_GROUPED) {
-    const int tr = t / p.tiles_b;
-    T.a_row0 = tr * BM;
-    T.b_row0 = (t - tr * p.tiles_b) * BN;
-    int g = 0;  // groups that end at or before the tile's first row; groups are multiples of 128 rows
+    // Row tile t / tiles_b names the group; inside a group the row tiles of one b panel come first, so
+    // that they run together and the panel comes from HBM once.
+    const int row = t / p.tiles_b * BM;
+    int g = 0;  // groups that end at or before that row; groups are whole tiles
     for (int g0 = 0; g0 < p.G; g0 += 64) {
       const int q = g0 + lane;
-      g += __popcll(__ballot(q < p.G && p.offs[q < p.G ? q : 0] <= T.a_row0));
+      g += __popcll(__ballot(q < p.G && p.offs[q < p.G ? q : 0] <= row));
     }
     T.g = __builtin_amdgcn_readfirstlane(g);
+    const int first = __builtin_amdgcn_readfirstlane(T.g ? p.offs[T.g - 1] : 0);
+    const int rows_g = (__builtin_amdgcn_readfirstlane(p.offs[T.g]) - first) / BM;
+    const int i = t - first / BM * p.tiles_b, col = i / rows_g;
+    T.a_row0 = first + (i - col * rows_g) * BM;
+    T.b_row0 = col * BN;
     T.a_lim = T.a_row0 + BM; T.b_lim = (int)p.rows_b;
     T.k_begin = 0; T.k_len = (int)p.red; T.kb0 = 0;
   } else {
@@ -189,13 +201,13 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_small_kernel(GemmArgs p) {
   }
   wait_all_vmem();  // nothing may still be writing into this workgroup's LDS when it retires
   if (MODE == GEMM_K_GROUPED && nk == 0 && ACC) return;
-  store_tile<MODE, TM, TN, ACC, 0, MODE == GEMM_K_GROUPED>(acc, p, T, wm0, wn0, lane, lds + NS * STAGE + NS * (BM + BN) * 4 + 256 + wave * 2048);
+  __syncthreads();  // every wave has read its last stage and has nothing in flight: the ring's memory is free
+  store_tile<MODE, TM, TN, ACC, 0, MODE == GEMM_K_GROUPED>(acc, p, T, wm0, wn0, lane, lds + wave * 2048);
 }
 
 template <int MODE, int BM, bool ACC, bool BT>
 static int launch_small(GemmArgs a, hipStream_t stream) {
-  constexpr int NS = BM == 64 ? 5 : 4;
-  constexpr size_t lds = (size_t)NS * (BM + 128) * 128 + NS * (BM + 128) * 4 + 256 + 4 * 2048;
+  constexpr size_t lds = kSmallLds<BM>;
   static bool attr_set = false;
   auto kernel = fp8_gemm_small_kernel<MODE, BM, ACC, BT>;
   if (!attr_set) {
