@@ -64,6 +64,15 @@ int pt_quant_rowwise_colwise_rows(const void* x, int dtype, int64_t M, int64_t N
                                   void* ch_fp8, float* ch_scale, int ch_layout,
                                   const int32_t* offs, int32_t num_groups, pt_stream_t stream);
 
+/* pt_quant_rowwise_colwise_rows with row r read from x[row_index[r] / repeat]: x [rows, N] holds one row per
+ * token and routed row i is token i / repeat (the expand of the models' reference_forward,
+ * qwen3_moe.py:104-108, without the copies).  rows * repeat^2 < 2^32. */
+int pt_quant_rowwise_colwise_rows_repeat(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M,
+                                         int64_t N, int64_t ldx, const int32_t* row_index,
+                                         void* tok_fp8, float* tok_scale, void* ch_fp8, float* ch_scale,
+                                         int ch_layout, const int32_t* offs, int32_t num_groups,
+                                         pt_stream_t stream);
+
 /* The transposed / column-scaled results (ch_fp8, ch_scale) of the row-scaled quantisers above and of the
  * fused SwiGLU forwards below may be left out (both NULL) when no backward reads them. */
 
@@ -233,6 +242,15 @@ int pt_gemm_m_grouped_nt_scatter(const void* a_fp8, const float* a_scale, const 
                                  const int32_t* offs, int32_t num_groups, int64_t M, int64_t N,
                                  int64_t K, const int32_t* out_row_index, int64_t out_rows,
                                  pt_stream_t stream);
+
+/* pt_gemm_m_grouped_nt and its _scatter / _bias forms (out_row_index, bias: may be NULL) for groups of a few
+ * rows each: every offs[g] is a multiple of 64 only, so that less padding is computed (a forward
+ * without a backward, whose groups need not be whole 128-row scale blocks). */
+int pt_gemm_m_grouped_nt_few_rows(const void* a_fp8, const float* a_scale, const void* b_fp8,
+                                  const float* b_scale, void* out, int out_dtype, const int32_t* offs,
+                                  int32_t num_groups, int64_t M, int64_t N, int64_t K,
+                                  const int32_t* out_row_index, int64_t out_rows, const void* bias,
+                                  pt_stream_t stream);
 
 /* pt_gemm_m_grouped_nt with the b operand given reduction-major: b[g] is [K, N] (K = the reduction,
  * row pitch N, N % 16 == 0) with scales [ceil(K/128), ceil(N/128)], i.e. a weight and its
@@ -478,6 +496,13 @@ int pt_moe_combine_bwd(const void* grad_out, int64_t ld_go, const void* moe, int
                        const float* topk_weight, void* d_moe, int64_t ld_dmoe, float* d_weight,
                        int64_t T, int32_t k, int64_t H, int dtype, pt_stream_t stream);
 
+/* Gradient of a tensor [T, H] that several branches read: out[t] = sum_j rows[t * k + j] + g0[t] + g1[t] + g2[t]
+ * (rows [T * k, H] or NULL, g0 .. g2 [T, H] or NULL), all in dtype, added in fp32 in that order and rounded
+ * once.  Replaces the reduction of the expand's backward and the additions autograd does between branches
+ * (qwen3_moe.py:104-119).  H % 8 == 0, 16-byte aligned. */
+int pt_sum_branches(const void* rows, int32_t k, const void* g0, const void* g1, const void* g2, void* out,
+                    int64_t T, int64_t H, int dtype, pt_stream_t stream);
+
 /* Expert-parallel branch of forward_stage5 (models/qwen3_moe.py:238-245, same lines in
  * deepseek_v2.py:351-357, qwen35_moe.py:334-340, gpt_oss.py:334-340): row r of moe [rows,H] belongs
  * to the flat top-k slot local_idxs[r] (token local_idxs[r] / k), every weighted row is rounded to
@@ -542,7 +567,9 @@ int pt_router_topk_bwd(const void* logits, int64_t ld_logits, int dtype, int64_t
  * [out_rows, H] when scatter != 0, else [M, H].  clamped != 0: the clamped SwiGLU on interleaved pairs
  * (alpha, limit) with the biases gu_bias [G, 2*half] and dn_bias [G, H] (may be NULL) added by the
  * GEMMs' stores; otherwise silu(gate) * up on concatenated halves.  x_t [K, M] and h_t [half, M] bytes with
- * scales [M/128, K] and [M/128, half]: the transposed activations that the weight gradients read.  Not
+ * scales [M/128, K] and [M/128, half]: the transposed activations that the weight gradients read (all four
+ * NULL: no backward follows).  repeat > 1 (with row_map, without expand_idx): grouped row r is
+ * x[row_map[r] / repeat].  few_rows != 0 (no backward): the groups are multiples of 64 rows.  Not
  * needed afterwards: composed_map int32 [M] (with expand_idx), x_fp8 [M, K] and h_fp8 [M, half] with
  * their 1x128 scales. */
 typedef struct {
@@ -551,6 +578,7 @@ typedef struct {
   const int32_t* offs;
   const int32_t* row_map;
   const int64_t* expand_idx; int64_t n_expand;
+  int64_t repeat, few_rows;
   const void* gu_fp8; const float* gu_scale; const void* gu_bias;
   const void* dn_fp8; const float* dn_scale; const void* dn_bias;
   void* gate_up;

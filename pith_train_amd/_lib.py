@@ -30,6 +30,7 @@ SIGNATURES = {
     "pt_abi_version": (c_int, []),
     "pt_quant_rowwise_colwise": (c_int, [P, c_int, I64, I64, I64, P, P, P, P, c_int, P, I32, P]),
     "pt_quant_rowwise_colwise_rows": (c_int, [P, c_int, I64, I64, I64, P, P, P, P, P, c_int, P, I32, P]),
+    "pt_quant_rowwise_colwise_rows_repeat": (c_int, [P, I64, I64, c_int, I64, I64, I64, P, P, P, P, P, c_int, P, I32, P]),
     "pt_silu_mul_quant_rowwise_colwise": (c_int, [P, I64, I64, I64, P, P, P, P, P, P]),
     "pt_silu_mul_bwd_quant_rowwise_colwise": (c_int, [P, I64, P, I64, I64, I64, P, P, P, P, P, P]),
     "pt_clamped_swiglu_quant_rowwise_colwise": (c_int, [P, I64, I64, I64, F, F, P, P, P, P, P, P]),
@@ -50,6 +51,7 @@ SIGNATURES = {
     "pt_gemm_nt_dense_heads": (c_int, [P, P, P, P, P, P, I64, I64, I64, I64, I64, P]),
     "pt_sum_partials": (c_int, [P, I32, I64, P, c_int, P]),
     "pt_gemm_m_grouped_nt": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P]),
+    "pt_gemm_m_grouped_nt_few_rows": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P, P]),
     "pt_gemm_m_grouped_nn": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P]),
     "pt_gemm_m_grouped_nn_scatter": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P]),
     "pt_gemm_m_grouped_nt_bias": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, P]),
@@ -66,6 +68,7 @@ SIGNATURES = {
     "pt_compose_row_map": (c_int, [P, I64, P, I64, I64, P, P]),
     "pt_cross_entropy_fwd": (c_int, [P, I64, c_int, P, I64, I64, I64, P, P, P, P]),
     "pt_cross_entropy_bwd": (c_int, [P, I64, c_int, I64, I64, P, P]),
+    "pt_sum_branches": (c_int, [P, I32, P, P, P, P, I64, I64, c_int, P]),
     "pt_moe_combine_ep_index": (c_int, [P, I64, I64, P, P]),
     "pt_moe_combine_ep_fwd": (c_int, [P, I64, I64, P, P, P, I64, P, I64, I64, I32, I64, c_int, P]),
     "pt_moe_combine_ep_bwd": (c_int, [P, I64, P, I64, I64, P, P, P, I64, P, I64, I32, I64, c_int, P]),

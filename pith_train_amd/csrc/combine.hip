@@ -341,6 +341,64 @@ extern "C" int pt_moe_combine_bwd(const void* grad_out, int64_t ld_go, const voi
   return launch_combine<true>(a, T, dtype, (hipStream_t)stream);
 }
 
+namespace pt {
+// Gradient of a tensor that several branches read (see the header).  Bound by HBM: every operand is read
+// once, k + 4 rows in flight per thread; one thread per 16 bytes of the result.
+struct BranchArgs {
+  const char* rows; const char* g[3]; char* out;
+  int32_t k; uint32_t chunks; int64_t n;  // chunks of 8 elements per row, threads
+};
+template <typename S>
+__global__ __launch_bounds__(256) void sum_branches_kernel(BranchArgs p) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.n) return;
+  const int64_t t = i / p.chunks;
+  const uint32_t c = (uint32_t)(i - t * p.chunks);
+  constexpr int64_t kChunk = 8 * S::kBytes;
+  float acc[8] = {};
+  float v[3][8];
+#pragma unroll
+  for (int q = 0; q < 3; ++q)  // requested first, added last
+    if (p.g[q]) S::load8(p.g[q] + i * kChunk, v[q]);
+  if (p.rows) {
+    for (int j0 = 0; j0 < p.k; j0 += 4) {
+      float m[4][8];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        load8_policy<S, (PT_COMBINE_NT & 1) != 0>(p.rows + ((t * p.k + (j0 + u < p.k ? j0 + u : j0)) * p.chunks + c) * kChunk, m[u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = j0 + u < p.k ? acc[e] + m[u][e] : acc[e];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+    if (p.g[q]) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += v[q][e];
+    }
+  S::store8(p.out + i * kChunk, acc);
+}
+}  // namespace pt
+
+extern "C" int pt_sum_branches(const void* rows, int32_t k, const void* g0, const void* g1, const void* g2, void* out, int64_t T, int64_t H,
+                               int dtype, pt_stream_t stream) {
+  PT_REQUIRE(T >= 0 && H >= 0 && H % 8 == 0 && H < (1ll << 31) && (!rows || k >= 1), "sum_branches: bad sizes");
+  if (T == 0 || H == 0) return PT_OK;
+  PT_REQUIRE(out && al16(rows) && al16(g0) && al16(g1) && al16(g2) && al16(out), "sum_branches: null or misaligned pointer");
+  BranchArgs a = {(const char*)rows, {(const char*)g0, (const char*)g1, (const char*)g2}, (char*)out, k, (uint32_t)(H / 8), T * (H / 8)};
+  PT_REQUIRE(cdiv(a.n, 256) < (1ll << 31), "sum_branches: too many elements");
+  const dim3 grid((unsigned)cdiv(a.n, 256));
+  switch (dtype) {
+    case PT_BF16: hipLaunchKernelGGL(sum_branches_kernel<st_bf16>, grid, dim3(256), 0, (hipStream_t)stream, a); break;
+    case PT_F16: hipLaunchKernelGGL(sum_branches_kernel<st_f16>, grid, dim3(256), 0, (hipStream_t)stream, a); break;
+    case PT_F32: hipLaunchKernelGGL(sum_branches_kernel<st_f32>, grid, dim3(256), 0, (hipStream_t)stream, a); break;
+    default: PT_REQUIRE(false, "sum_branches: unsupported dtype %d", dtype);
+  }
+  return check_launch("sum_branches_kernel");
+}
+
 extern "C" int pt_moe_combine_ep_index(const int64_t* local_idxs, int64_t rows, int64_t slots, int32_t* slot_row,
                                        pt_stream_t stream) {
   PT_REQUIRE(rows >= 0 && slots >= 0 && rows < (1ll << 31) && slots < (1ll << 31), "moe_combine_ep_index: bad sizes");

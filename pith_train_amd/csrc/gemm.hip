@@ -351,6 +351,10 @@ static bool fits_persistent(const GemmArgs& g) {
 static int dispatch_gemm(const GemmArgs& g, hipStream_t stream) {
   const int impl = gemm_impl();
   const bool fits = fits_persistent(g);
+  if (g.few_rows) {  // only tiles of 64 rows end where these groups end
+    PT_REQUIRE(fits, "gemm_m_grouped_nt_few_rows: operands below 2 GiB, output below 4 GiB");
+    return launch_gemm_small(g, 64, stream);
+  }
   if (g.b_kmajor) {  // two kernels read this layout, whatever kernel was selected for the others
     PT_REQUIRE(fits, "gemm: the reduction-major b operand needs the row-split kernel, which addresses operands below 2 GiB "
                      "and an output below 4 GiB through 32-bit byte offsets; larger problems take the NT entry point on the "
@@ -514,10 +518,10 @@ extern "C" int pt_sum_partials(const float* partial, int32_t splits, int64_t n, 
 static int gemm_m_grouped_impl(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale, void* out,
                                int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K,
                                const int32_t* out_row_index, int64_t out_rows, const void* bias, pt_stream_t stream,
-                               bool b_kmajor = false) {
+                               bool b_kmajor = false, bool few_rows = false) {
   PT_REQUIRE(M >= 0 && N >= 0 && K >= 0 && G > 0, "gemm_m_grouped_nt: bad sizes");
   if (M == 0 || N == 0) return PT_OK;
-  PT_REQUIRE(M % 128 == 0, "gemm_m_grouped_nt: M=%lld must be a multiple of 128", (long long)M);
+  PT_REQUIRE(M % (few_rows ? 64 : 128) == 0, "gemm_m_grouped_nt: M=%lld must be a multiple of %d", (long long)M, few_rows ? 64 : 128);
   PT_REQUIRE(K > 0 && K % 16 == 0, "gemm_m_grouped_nt: K=%lld must be a positive multiple of 16", (long long)K);
   PT_REQUIRE(a_fp8 && a_scale && b_fp8 && b_scale && out && offs && al16(a_fp8) && al16(b_fp8), "gemm_m_grouped_nt: null or misaligned pointer");
   PT_REQUIRE(out_dtype == PT_BF16, "gemm_m_grouped_nt: out_dtype must be bf16");
@@ -529,7 +533,7 @@ static int gemm_m_grouped_impl(const void* a_fp8, const float* a_scale, const vo
   g.sb = b_scale; g.sb_rs = KB; g.sb_ks = 1; g.sb_shift = 7;
   g.out = out; g.ldo = N; g.out_dtype = out_dtype; g.accumulate = 0;
   g.rows_a = M; g.rows_b = N; g.red = K; g.mode = GEMM_M_GROUPED; g.offs = offs; g.G = G;
-  g.b_stride_g = N * K; g.sb_stride_g = NB * KB;
+  g.b_stride_g = N * K; g.sb_stride_g = NB * KB; g.few_rows = few_rows;
   g.a_bytes = M * K; g.b_bytes = N * K; g.sa_bytes = M * KB * 4; g.sb_bytes = NB * KB * 4;
   g.tiles_a = (int)(M / 128); g.tiles_b = (int)NB;
   g.total_tiles = (int64_t)g.tiles_a * g.tiles_b;
@@ -574,6 +578,13 @@ extern "C" int pt_gemm_m_grouped_nt_scatter_bias(const void* a_fp8, const float*
   PT_REQUIRE(out_row_index && bias, "gemm_m_grouped_nt_scatter_bias: null out_row_index or bias");
   return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, bias,
                              stream);
+}
+
+extern "C" int pt_gemm_m_grouped_nt_few_rows(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale, void* out,
+                                             int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K,
+                                             const int32_t* out_row_index, int64_t out_rows, const void* bias, pt_stream_t stream) {
+  return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, bias, stream,
+                             false, true);
 }
 
 extern "C" int pt_gemm_m_grouped_nn(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,

@@ -30,6 +30,7 @@ struct GemmArgs {
   int head_a, head_b;                     // dense only: result column h * (head_a + head_b) + c is out[h * head_a + c] for c < head_a, else
                                           // out2[h * head_b + c - head_a]; out2 lies behind out in one allocation (head_a == 0: one output)
   int64_t out_extent;                     // with head_a: bytes from out to the end of out2, below 2 GiB
+  int few_rows;                           // m-grouped: the group ends are multiples of 64, not of 128
   int b_kmajor;                           // m-grouped, row-split kernel: b is [red, rows_b] per group (row pitch ldb) instead of [rows_b, red]
 };
 

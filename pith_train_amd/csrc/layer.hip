@@ -39,8 +39,11 @@ extern "C" int pt_experts_forward(const pt_experts_forward_args* args) {
   PT_REQUIRE(args, "experts_forward: null arguments");
   const pt_experts_forward_args& a = *args;
   PT_REQUIRE(a.M >= 0 && a.M % 128 == 0 && a.K > 0 && a.half > 0 && a.H > 0 && a.G > 0 && a.G < (1ll << 31), "experts_forward: bad sizes");
-  PT_REQUIRE(a.offs && a.gate_up && a.out && a.x_fp8 && a.x_scale && a.x_t && a.x_t_scale && a.h_fp8 && a.h_scale && a.h_t && a.h_t_scale,
-             "experts_forward: null pointer");
+  const bool keep = a.x_t != nullptr;  // a backward will read the transposed activations
+  PT_REQUIRE(a.offs && a.gate_up && a.out && a.x_fp8 && a.x_scale && a.h_fp8 && a.h_scale && keep == (a.h_t != nullptr) &&
+                 keep == (a.x_t_scale != nullptr) && keep == (a.h_t_scale != nullptr), "experts_forward: null pointer");
+  PT_REQUIRE(a.repeat >= 1 && (a.repeat == 1 || (a.row_map && !a.expand_idx)), "experts_forward: repeat needs row_map and no expand_idx");
+  PT_REQUIRE(!a.few_rows || !keep, "experts_forward: a backward needs groups of whole 128-row blocks");
   PT_REQUIRE(!a.expand_idx || a.composed_map, "experts_forward: expand_idx needs composed_map");
   PT_REQUIRE(a.row_map || (!a.expand_idx && !a.scatter), "experts_forward: expand_idx and scatter need row_map");
   if (a.M == 0) return PT_OK;
@@ -51,13 +54,19 @@ extern "C" int pt_experts_forward(const pt_experts_forward_args* args) {
     PT_STEP(pt_compose_row_map, a.M, 0, 0, a.row_map, a.M, a.expand_idx, a.n_expand, a.x_rows, a.composed_map, a.stream);
     in_map = a.composed_map;
   }
-  if (in_map)
+  if (a.repeat > 1)
+    PT_STEP(pt_quant_rowwise_colwise_rows_repeat, a.M, a.K, a.x_rows, a.x, a.x_rows, a.repeat, PT_BF16, a.M, a.K, a.ldx, in_map, a.x_fp8,
+            a.x_scale, a.x_t, a.x_t_scale, PT_CH_TRANSPOSED, a.offs, G, a.stream);
+  else if (in_map)
     PT_STEP(pt_quant_rowwise_colwise_rows, a.M, a.K, a.x_rows, a.x, PT_BF16, a.M, a.K, a.ldx, in_map, a.x_fp8, a.x_scale, a.x_t, a.x_t_scale,
             PT_CH_TRANSPOSED, a.offs, G, a.stream);
   else
     PT_STEP(pt_quant_rowwise_colwise, a.M, a.K, a.x_rows, a.x, PT_BF16, a.M, a.K, a.ldx, a.x_fp8, a.x_scale, a.x_t, a.x_t_scale, PT_CH_TRANSPOSED,
             nullptr, 0, a.stream);
-  if (a.gu_bias)
+  if (a.few_rows)
+    PT_STEP(pt_gemm_m_grouped_nt_few_rows, a.M, 2 * a.half, a.K, a.x_fp8, a.x_scale, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M,
+            2 * a.half, a.K, nullptr, 0, a.gu_bias, a.stream);
+  else if (a.gu_bias)
     PT_STEP(pt_gemm_m_grouped_nt_bias, a.M, 2 * a.half, a.K, a.x_fp8, a.x_scale, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M,
             2 * a.half, a.K, a.gu_bias, a.stream);
   else
@@ -69,7 +78,10 @@ extern "C" int pt_experts_forward(const pt_experts_forward_args* args) {
   else
     PT_STEP(pt_silu_mul_quant_rowwise_colwise, a.M, a.half, 0, a.gate_up, a.M, a.half, 2 * a.half, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit,
             a.stream);
-  if (a.scatter && a.dn_bias)
+  if (a.few_rows)
+    PT_STEP(pt_gemm_m_grouped_nt_few_rows, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H,
+            a.half, a.scatter ? a.row_map : nullptr, a.out_rows, a.dn_bias, a.stream);
+  else if (a.scatter && a.dn_bias)
     PT_STEP(pt_gemm_m_grouped_nt_scatter_bias, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M,
             a.H, a.half, a.row_map, a.out_rows, a.dn_bias, a.stream);
   else if (a.scatter)

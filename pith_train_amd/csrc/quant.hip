@@ -74,6 +74,7 @@ struct QuantArgs {
   int32_t vec_out;    // 8-byte row-major stores legal (N % 8 == 0)
   int32_t vec_out_t;  // 16-byte transposed stores legal
   const int32_t* row_index;  // optional [M]: source row of output row r (negative: a zero row); null = identity
+  uint32_t row_mul;          // with row_index: the source row is floor(row_index * row_mul / 2^32) (every source row stands for several); 0 = row_index itself
   const void* x2; int64_t ldx2;  // fused SwiGLU backward: the saved gate_up [M, 2*half]
   int64_t half;                  // fused SwiGLU: width of one half of gate_up
   const int32_t* row_limit;      // optional device scalar: row tiles at or past *row_limit are skipped (nothing written)
@@ -375,6 +376,10 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
         for (int i = 0; i < 8; ++i)
           if (row0 + i < p.M) src[i] = p.row_index[row0 + i];
       }
+      if (p.row_mul) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) src[i] = src[i] >= 0 ? (int32_t)__umulhi((uint32_t)src[i], p.row_mul) : src[i];
+      }
     }
     if (FULL && !p.row_index) {
       const char* base = xb + (row0 * p.ldx + col0) * Loader<T>::kBytes;
@@ -403,7 +408,10 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
     for (int i = 0; i < 8; ++i) {
       f.zero_row(i);
       int64_t sr = row0 + i;
-      if (p.row_index && sr < p.M) sr = p.row_index[sr];
+      if (p.row_index && sr < p.M) {
+        sr = p.row_index[sr];
+        if (p.row_mul && sr >= 0) sr = __umulhi((uint32_t)sr, p.row_mul);
+      }
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         if (row0 + i < p.M && sr >= 0 && col0 + j < p.N) f.set(i, j, xb + (sr * p.ldx + col0 + j) * Loader<T>::kBytes);
@@ -805,7 +813,7 @@ static void fill_common(QuantArgs& a, const void* x, int dtype, int64_t M, int64
   a.x = x; a.M = M; a.N = N; a.ldx = ldx; a.x_stride_g = 0;
   a.a_stride_g = 0; a.a_scale_stride_g = 0; a.b_stride_g = 0; a.b_scale_stride_g = 0;
   a.tiles_m = (int32_t)cdiv(M, 128); a.tiles_n = (int32_t)cdiv(N, 128);
-  a.offs = nullptr; a.num_groups = 0; a.row_index = nullptr; a.x2 = nullptr; a.ldx2 = 0; a.half = 0;
+  a.offs = nullptr; a.num_groups = 0; a.row_index = nullptr; a.row_mul = 0; a.x2 = nullptr; a.ldx2 = 0; a.half = 0;
   a.row_limit = nullptr; a.ld_t = M; a.bs_ld = a.tiles_m; a.alpha = 0.f; a.limit = 0.f; a.col_sum = nullptr;
   a.head_a = a.head_b = 0;
   const int eb = dtype == PT_F32 ? 4 : 2;
@@ -820,7 +828,7 @@ using namespace pt;
 
 static int quant_rowwise_colwise_impl(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
                                       void* tok_fp8, float* tok_scale, void* ch_fp8, float* ch_scale, int ch_layout,
-                                      const int32_t* offs, int32_t num_groups, pt_stream_t stream);
+                                      const int32_t* offs, int32_t num_groups, pt_stream_t stream, int64_t repeat = 1);
 
 extern "C" int pt_quant_rowwise_colwise(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx,
                                         void* tok_fp8, float* tok_scale, void* ch_fp8,
@@ -839,9 +847,21 @@ extern "C" int pt_quant_rowwise_colwise_rows(const void* x, int dtype, int64_t M
                                     num_groups, stream);
 }
 
+extern "C" int pt_quant_rowwise_colwise_rows_repeat(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M, int64_t N, int64_t ldx,
+                                                    const int32_t* row_index, void* tok_fp8, float* tok_scale, void* ch_fp8,
+                                                    float* ch_scale, int ch_layout, const int32_t* offs, int32_t num_groups,
+                                                    pt_stream_t stream) {
+  PT_REQUIRE(row_index || M == 0, "quant_rowwise_colwise_rows_repeat: null row_index");
+  // floor(i / repeat) = floor(i * m / 2^32) with m = ceil(2^32 / repeat) is exact while i * repeat stays below 2^32
+  PT_REQUIRE(rows >= 0 && repeat >= 1 && repeat < (1 << 16) && rows * repeat * repeat < (1ll << 32) && rows * repeat < (1ll << 31),
+             "quant_rowwise_colwise_rows_repeat: %lld rows, each %lld times, are too many", (long long)rows, (long long)repeat);
+  return quant_rowwise_colwise_impl(x, dtype, M, N, ldx, row_index, tok_fp8, tok_scale, ch_fp8, ch_scale, ch_layout, offs,
+                                    num_groups, stream, repeat);
+}
+
 static int quant_rowwise_colwise_impl(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
                                       void* tok_fp8, float* tok_scale, void* ch_fp8, float* ch_scale, int ch_layout,
-                                      const int32_t* offs, int32_t num_groups, pt_stream_t stream) {
+                                      const int32_t* offs, int32_t num_groups, pt_stream_t stream, int64_t repeat) {
   PT_REQUIRE(M >= 0 && N >= 0 && M % 128 == 0, "quant_rowwise_colwise: M=%lld must be a multiple of 128", (long long)M);
   PT_REQUIRE(ldx >= N, "quant_rowwise_colwise: ldx < N");
   if (M == 0 || N == 0) return PT_OK;
@@ -850,6 +870,7 @@ static int quant_rowwise_colwise_impl(const void* x, int dtype, int64_t M, int64
   fill_common(a, x, dtype, M, N, ldx);
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_fp8; a.b_scale = ch_scale;
   a.row_index = row_index;
+  if (repeat > 1) a.row_mul = (uint32_t)(((1ull << 32) + repeat - 1) / repeat);
   if (offs && num_groups > 0) a.row_limit = offs + (num_groups - 1);
   hipStream_t s = (hipStream_t)stream;
   switch (ch_layout) {

@@ -97,20 +97,24 @@ class Qwen3MoeExperts(nn.Module):
         return self._gu_cache, down._wq_cache
 
     def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, fuse_activation: bool = True,
-                expand_idx=None):
+                expand_idx=None, few_rows: bool = False):
         """``row_map`` (extension, FP8 layers only): the scatter's int32 source-row map.  ``x`` is
         then the un-permuted ``[m, H]`` token tensor and the result comes back un-permuted; the
         permutation happens inside the first quantisation and the last GEMM's store.
         ``expand_idx`` (one-node path only): ``x`` holds deduplicated rows, see
-        :func:`fused_experts.compose_row_maps`.  With
-        ``fuse_activation`` (FP8 layers, intermediate size a multiple of 128) the block runs as one
+        :func:`fused_experts.compose_row_maps`.  One-node path with ``row_map`` only: ``x`` may be an expanded
+        ``[T, k, H]`` view of the tokens, and ``few_rows`` says that the groups are multiples of 64 rows (no
+        backward may follow).  With ``fuse_activation`` (FP8 layers, intermediate size a multiple of 128) the block runs as one
         autograd node on a fused gate_up operand: the tokens are quantised once instead of once
         per projection, one GEMM serves both, and the SwiGLU and its gradient are computed inside
         the kernels that quantise them (same bits as the three-operator composition)."""
         if fuse_activation and x.shape[0] > 0 and self.one_node(x):
-            gate, up, down = self._projections()
+            gate, up, down = map(_weight, self._projections())
+            if not fused_experts.wants_backward(x, gate, up, down):
+                return fused_experts.forward_only(x, (gate, up), down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
+                                                  few_rows=few_rows)  # fmt: skip
             return fused_experts.FP8SwiGLUSplitExpertsFunc.apply(
-                x, _weight(gate), _weight(up), _weight(down), grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
+                x, gate, up, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
             )  # fmt: skip
         assert expand_idx is None, "expand_idx needs the one-node FP8 path"
         gi = precompute_group_indices(grouped_mm_offs, x.shape[0])
@@ -174,13 +178,17 @@ class Qwen35MoeExperts(nn.Module):
         return gu._get_quantized_weight(), down._get_quantized_weight()
 
     def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, fuse_activation: bool = True,
-                expand_idx=None):
+                expand_idx=None, few_rows: bool = False):
         """``row_map`` / ``expand_idx``: see :meth:`Qwen3MoeExperts.forward`.  With ``fuse_activation`` (FP8 layers)
         the block runs as one autograd node whose SwiGLU output and SwiGLU gradient are computed
         inside the kernels that quantise them (same bits as the three-operator composition)."""
         if fuse_activation and x.shape[0] > 0 and self.one_node(x):
+            gate_up, down = _weight(self._modules["gate_up_proj"]), _weight(self._modules["down_proj"])
+            if not fused_experts.wants_backward(x, gate_up, down):
+                return fused_experts.forward_only(x, gate_up, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
+                                                  few_rows=few_rows)  # fmt: skip
             return fused_experts.FP8SwiGLUExpertsFunc.apply(
-                x, _weight(self._modules["gate_up_proj"]), _weight(self._modules["down_proj"]), grouped_mm_offs, ks, ks_tensor,
+                x, gate_up, down, grouped_mm_offs, ks, ks_tensor,
                 *self._quantized_weights(), row_map, expand_idx,
             )  # fmt: skip
         assert expand_idx is None, "expand_idx needs the one-node FP8 path"
@@ -258,7 +266,8 @@ class GptOssExperts(nn.Module):
         sized for more rows than the routing produced."""
         return self.bias_fusable(x) and self.fuse_activation and self.down_proj.shape[2] % 8 == 0
 
-    def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, scatter_output: bool = False):
+    def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, scatter_output: bool = False,
+                few_rows: bool = False):
         """``row_map`` (extension, FP8 only): the scatter's int32 source-row map; ``x`` is then the
         un-permuted token tensor and the first quantisation gathers its rows.  The result stays
         in the grouped layout unless ``scatter_output`` is set (with ``row_map`` and the fused
@@ -269,6 +278,11 @@ class GptOssExperts(nn.Module):
         M = x.shape[0] if row_map is None else row_map.shape[0]
         fused = self.bias_fusable(x)
         assert not scatter_output or (fused and row_map is not None), "scatter_output needs row_map and the fused biases"
+        if M % 128 == 0 and self.one_node(x) and not fused_experts.wants_backward(x, *self._parameters.values()):
+            return fused_experts.forward_only(
+                x, self.gate_up_proj, self.down_proj, grouped_mm_offs, *self._quantized_weights(), row_map, None, scatter_output,
+                (1.702, self.swiglu_limit), (self.gate_up_proj_bias, self.down_proj_bias), few_rows,
+            )
         if M % 128 == 0 and self.one_node(x):
             return fused_experts.FP8ClampedSwiGLUExpertsFunc.apply(
                 x, self.gate_up_proj, self.gate_up_proj_bias, self.down_proj, self.down_proj_bias, grouped_mm_offs,
@@ -289,6 +303,14 @@ class GptOssExperts(nn.Module):
         return indexed_bias_add(out, self.down_proj_bias, group_ids, grouped_mm_offs)
 
 
+_ONE_NODE_BLOCKS = (Qwen3MoeExperts, Qwen35MoeExperts, GptOssExperts)
+
+
+def _few_rows(experts: nn.Module, x, expert_idxs, experts_per_rank: int) -> bool:
+    return (fused_experts.few_rows_per_expert(expert_idxs.shape[0], experts_per_rank)
+            and not fused_experts.wants_backward(x, *experts.parameters()))
+
+
 def forward_stage3(experts: nn.Module, gathered_tokens, expert_idxs, experts_per_rank: int, expand_idx=None,
                    fuse_expand: bool = True, fuse_permute: bool = True, host_sizes: bool = False):
     """Expert compute between the dispatch and combine all-to-alls.
@@ -306,32 +328,46 @@ def forward_stage3(experts: nn.Module, gathered_tokens, expert_idxs, experts_per
     (token, expert) pair.  With ``fuse_expand`` that gather is folded into the scatter's row copy
     (each unique row is read once per use and no expanded copy is materialised); without it the
     two steps run separately as in the reference.
+
+    ``gathered_tokens`` may also be an expanded ``[T, k, H]`` view of one row per token (stride 0 along k):
+    the one-node blocks then read every token where it is, and its gradient comes back as ``[T, k, H]``.
     """
+    if gathered_tokens.dim() == 3:
+        T, k = gathered_tokens.shape[:2]
+        one = (fuse_permute and training.fp8 and expand_idx is None and T > 0 and isinstance(experts, _ONE_NODE_BLOCKS)
+               and experts.one_node(gathered_tokens[:, 0]) and gathered_tokens.stride(1) == 0 and T * k * k < 2**32)
+        if not one:
+            gathered_tokens = gathered_tokens.reshape(T * k, -1)
     if fuse_permute and training.fp8 and expert_idxs.shape[0] > 0 and isinstance(experts, (Qwen3MoeExperts, Qwen35MoeExperts)):
         fused_node = experts.one_node(gathered_tokens)
         # the composition of separate operators can still take the row map when its layers are FP8 ones
         down = experts._modules["down_proj"]
         mapped = fused_node or (isinstance(down, FP8GroupedLinear) and down.out_features % 8 == 0 and down.in_features % 8 == 0)
         if mapped and (expand_idx is None or (fused_node and fuse_expand)):
+            few = fused_node and not host_sizes and _few_rows(experts, gathered_tokens, expert_idxs, experts_per_rank)
             _, grouped_mm_offs, ks, ks_tensor, src_of = group_rows_with_sizes(
-                expert_idxs, experts_per_rank, device=gathered_tokens.device, host_sizes=host_sizes or not fused_node,
-                need_reverse=False)
+                expert_idxs, experts_per_rank, fused_experts.FEW_ROWS if few else 128, device=gathered_tokens.device,
+                host_sizes=host_sizes or not fused_node, need_reverse=False)
             if expand_idx is None:
-                return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of)
+                return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of,
+                               **({"few_rows": True} if few else {}))
             # deduplicated rows: the first quantisation reads them through expand_idx composed with
             # the scatter's map, so neither the expanded nor the permuted copy exists
             return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of,
-                           expand_idx=expand_idx)
+                           expand_idx=expand_idx, **({"few_rows": True} if few else {}))
     if (fuse_permute and expand_idx is None and training.fp8 and expert_idxs.shape[0] > 0
             and isinstance(experts, GptOssExperts)):
         # the one-node block needs no host-side sizes (see the SwiGLU branch above)
+        fused_node = experts.one_node(gathered_tokens)
+        few = fused_node and not host_sizes and _few_rows(experts, gathered_tokens, expert_idxs, experts_per_rank)
         reverse_shuffle_idxs, grouped_mm_offs, ks, ks_tensor, src_of = group_rows_with_sizes(
-            expert_idxs, experts_per_rank, device=gathered_tokens.device,
-            host_sizes=host_sizes or not experts.one_node(gathered_tokens))
+            expert_idxs, experts_per_rank, fused_experts.FEW_ROWS if few else 128, device=gathered_tokens.device,
+            host_sizes=host_sizes or not fused_node, need_reverse=not fused_node)
         if experts.bias_fusable(gathered_tokens):
             # both sides: rows gathered by the first quantisation, stored un-permuted (bias added)
             # by the last GEMM; the bias gradients are summed through the same map
-            return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of, scatter_output=True)
+            return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of, scatter_output=True,
+                           few_rows=few)
         # input side only: the unfused bias add wants the grouped layout
         outs = experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of)
         return padded_index_gather(outs, reverse_shuffle_idxs)

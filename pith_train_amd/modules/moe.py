@@ -17,7 +17,7 @@ from typing import List, Tuple
 import torch
 import torch.nn as nn
 
-from ..operators.moe_combine import moe_combine
+from ..operators.moe_combine import moe_combine, token_branches
 from . import training
 from .experts import DeepSeekV2Experts, DeepSeekV2MLP, GptOssExperts, Qwen3MoeExperts, Qwen35MoeExperts, forward_stage3
 from .gates import DeepSeekV2MoEGate, GptOssTopKRouter, Qwen3MoeGate, Qwen35MoeTopKRouter
@@ -57,15 +57,17 @@ class _RoutedExperts(nn.Module):
     num_experts_per_tok: int
     experts_per_rank: int
 
-    def _routed(self, hidden_states: torch.Tensor, gate: nn.Module) -> torch.Tensor:
-        topk_idx, topk_weight, lb_loss = gate(hidden_states)
+    def _routed(self, hidden_states: torch.Tensor, gate: nn.Module, shared=None) -> torch.Tensor:
+        """The experts' weighted sum, plus ``shared(hidden_states)`` when given."""
+        k = self.num_experts_per_tok
+        flat = hidden_states.view(-1, hidden_states.shape[-1])
+        replicated, for_gate, *for_shared = token_branches(flat, k, 1 if shared is None else 2)
+        topk_idx, topk_weight, lb_loss = gate(for_gate.view(hidden_states.shape))
         if lb_loss is not None:
             MoELoadBalanceLossTracker.add(lb_loss)
-        flat = hidden_states.view(-1, hidden_states.shape[-1])
-        k = self.num_experts_per_tok
-        replicated = flat.unsqueeze(1).expand(-1, k, -1).reshape(-1, flat.shape[-1])
         outs = forward_stage3(self.experts, replicated, topk_idx.reshape(-1), self.experts_per_rank)
-        return moe_combine(outs, topk_weight).view(hidden_states.shape)
+        routed = moe_combine(outs, topk_weight).view(hidden_states.shape)
+        return routed if shared is None else routed + shared(for_shared[0].view(hidden_states.shape))
 
 
 class Qwen3MoeMoE(_RoutedExperts):
@@ -95,7 +97,7 @@ class DeepSeekV2MoE(_RoutedExperts):
         self.shared_experts = DeepSeekV2MLP(hidden_size, moe_intermediate_size * n_shared_experts)
 
     def reference_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
-        return self._routed(hidden_states, self.gate) + self.shared_experts(hidden_states)
+        return self._routed(hidden_states, self.gate, self.shared_experts)
 
 
 class GptOssMoE(_RoutedExperts):
@@ -130,7 +132,7 @@ class Qwen35MoeSparseMoeBlock(_RoutedExperts):
         return torch.sigmoid(self.shared_expert_gate(hidden_states)) * self.shared_expert(hidden_states)
 
     def reference_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
-        return self._routed(hidden_states, self.gate) + self.shared_out(hidden_states)
+        return self._routed(hidden_states, self.gate, self.shared_out)
 
 
 __all__ = ["MoELoadBalanceLossTracker", "Qwen3MoeMoE", "DeepSeekV2MoE", "GptOssMoE", "Qwen35MoeSparseMoeBlock", "training"]

@@ -128,7 +128,7 @@ def compose_row_maps(row_map: torch.Tensor, expand_idx: torch.Tensor, n_src: int
     return out
 
 
-_FORWARD_BLOCK = struct.Struct("=23q2d10q").pack
+_FORWARD_BLOCK = struct.Struct("=14q11q2d10q").pack
 _BACKWARD_BLOCK = struct.Struct("=35q2d5q").pack
 _ONE_BUFFER = 32 << 20  # bytes up to which the tensors of one kind share an allocation
 
@@ -181,16 +181,33 @@ def _piece(layout, buffers, i, rows, cols, dtype):
     return buffers[0][at : at + layout[0][i]].view(dtype).view(rows, cols)
 
 
+FEW_ROWS = 64  # group alignment of forwards that no backward follows, see few_rows_per_expert
+
+
+def few_rows_per_expert(rows: int, num_groups: int) -> bool:
+    """Whether a forward without a backward pads its groups to 64 rows instead of 128 and takes the GEMM tiles
+    of that height.  Such a forward reads every expert's weights for a handful of rows, and half of a
+    128-row tile would be padding; with more rows than this most groups need a second 64-row tile,
+    which reads the weight panel again."""
+    return rows <= 48 * num_groups
+
+
 def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx=None, scatter=True,
-             clamp=None, biases=(None, None)):
+             clamp=None, biases=(None, None), few_rows=False):
     """Shared forward of the autograd nodes below: one library call queues every launch of it.
     ``gate_up_weights``: the parameters whose gradients the gate_up weight gradient is written to, one
     fused ``[G, 2I, K]`` tensor or the pair ``(gate [G, I, K], up [G, I, K])``.  ``expand_idx`` (with
     ``row_map``): ``x`` holds deduplicated rows and routed row i is ``x[expand_idx[i]]``; the result
     has one row per routed row, and the backward sums the gradients of the rows that share a source
     row.  ``scatter`` (with ``row_map``): the result comes back un-permuted.  ``clamp``: ``(alpha,
-    limit)`` of the clamped SwiGLU, whose projections have the two ``biases``."""
+    limit)`` of the clamped SwiGLU, whose projections have the two ``biases``.  ``x`` may be an expanded
+    ``[T, k, K]`` view of one row per token (routed row i is token i // k).  Without a ``ctx`` nothing is
+    kept for a backward, and the groups may be multiples of 64 rows (``few_rows``)."""
     _lib.require_cuda(x)
+    repeat = 1
+    if x.dim() == 3:
+        repeat = x.shape[1]
+        x = x[:, 0]
     gu_fp8, gu_scale = q_gate_up[:2]
     dn_fp8, dn_scale = q_down[:2]
     G, H, half = w_down.shape
@@ -202,7 +219,7 @@ def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down
         row_map = row_map.contiguous()
     M = src_rows if row_map is None else row_map.shape[0]
     assert M % 128 == 0, f"grouped rows must be a multiple of 128, got {M}"
-    routed = src_rows
+    routed = src_rows * repeat
     if expand_idx is not None:
         assert expand_idx.dtype == torch.int64
         expand_idx = expand_idx.contiguous()
@@ -211,18 +228,20 @@ def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down
         x = x.contiguous()
     dev = x.device
     kept_layout, temp_layout, _, _ = _sizes(M, K, half, H)
+    kept, kept_at = _allocate(kept_layout, dev) if ctx is not None else ((), (0, 0, 0, 0))
     _temp, temp_at = _allocate(temp_layout, dev)
-    kept, kept_at = _allocate(kept_layout, dev)
     gate_up = torch.empty((M, 2 * half), device=dev, dtype=x.dtype)
     out = torch.empty((routed if scatter else M, H), device=dev, dtype=x.dtype)
     b_gate_up, b_down = biases if biases[0] is None else [b.detach().contiguous() for b in biases]
     alpha, limit = clamp or (0.0, 0.0)
     _lib.call("pt_experts_forward", _FORWARD_BLOCK(
         x.data_ptr(), src_rows, x.stride(0) if src_rows > 1 else K, M, K, half, H, G, grouped_mm_offs.data_ptr(), _lib.ptr(row_map) or 0,
-        _lib.ptr(expand_idx) or 0, 0 if expand_idx is None else routed, gu_fp8.data_ptr(), gu_scale.data_ptr(), _lib.ptr(b_gate_up) or 0,
+        _lib.ptr(expand_idx) or 0, 0 if expand_idx is None else routed, repeat, few_rows, gu_fp8.data_ptr(), gu_scale.data_ptr(), _lib.ptr(b_gate_up) or 0,
         dn_fp8.data_ptr(), dn_scale.data_ptr(), _lib.ptr(b_down) or 0, gate_up.data_ptr(), out.data_ptr(), out.shape[0], scatter,
         clamp is not None, alpha, limit, *kept_at, *temp_at, _lib.stream_ptr(dev),
     ))  # fmt: skip
+    if ctx is None:
+        return out
     gu_dg, gu_dg_s, gu_forward = dgrad_operand(q_gate_up, gate_up_weights, M)
     dn_dg, dn_dg_s, dn_forward = dgrad_operand(q_down, w_down, M)
     ctx.save_for_backward(gu_dg, gu_dg_s, dn_dg, dn_dg_s, grouped_mm_offs, gate_up, row_map, expand_idx, *kept)
@@ -230,6 +249,7 @@ def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down
     ctx.clamp = clamp
     ctx.bias_dtypes = tuple(None if b is None else b.dtype for b in biases)
     ctx.dims = (M, K, half, H, G, routed, src_rows, gu_forward, dn_forward, scatter)
+    ctx.repeat = repeat
     return out
 
 
@@ -288,7 +308,21 @@ def _backward(ctx, grad_out):
         # one gradient row per routed row so far: rows that expand the same source row are summed
         # (the backward of the expanding gather, token_scatter.py:311-325)
         grad_x = _PaddedIndexGather.scatter_sum(grad_x, expand_idx, src_rows, _GEMM_ALLOC_ALIGNMENT)
+    if ctx.repeat > 1:
+        grad_x = grad_x.view(src_rows, ctx.repeat, K)
     return grad_x, d_gu_bias, d_dn_bias
+
+
+def wants_backward(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+    """Whether a backward can follow a forward on these tensors."""
+    return torch.is_grad_enabled() and (x.requires_grad or any(w.requires_grad for w in weights))
+
+
+def forward_only(x, w_gate_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map=None, expand_idx=None, scatter=True,
+                 clamp=None, biases=(None, None), few_rows=False):
+    """The forward of the nodes below when no backward follows: nothing is kept, and the quantisers leave out
+    the transposed operands of the weight gradients."""
+    return _forward(None, x, w_gate_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx, scatter, clamp, biases, few_rows)
 
 
 class FP8SwiGLUExpertsFunc(torch.autograd.Function):

@@ -127,3 +127,41 @@ def moe_combine_ep(moe_outs: torch.Tensor, moe_local_idxs: torch.Tensor, topk_we
     rounded, a token's rows are added in ascending r with every partial sum rounded to the
     storage type (a sequential ``scatter_add_``), and the residual is added last."""
     return _MoeCombineEP.apply(moe_outs, moe_local_idxs, topk_weight, residual)
+
+
+class _Branches(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x: torch.Tensor, k: int, n: int):
+        ctx.set_materialize_grads(False)
+        ctx.shape = x.shape
+        return (x.unsqueeze(1).expand(-1, k, -1), *(x.view_as(x) for _ in range(n)))
+
+    @staticmethod
+    def backward(ctx, rows, *others):
+        T, H = ctx.shape
+        given = [g for g in (rows, *others) if g is not None]
+        if not given:
+            return None, None, None
+        if H % 8 or len(others) > 3 or len({g.dtype for g in given}) > 1:
+            total = None if rows is None else rows.sum(1)
+            for g in others:
+                if g is not None:
+                    total = g if total is None else total + g
+            return total, None, None
+        given = [g.contiguous() for g in given]
+        others = given if rows is None else given[1:]
+        out = torch.empty((T, H), dtype=given[0].dtype, device=given[0].device)
+        at = [g.data_ptr() for g in others] + [0] * (3 - len(others))
+        _lib.call("pt_sum_branches", 0 if rows is None else given[0].data_ptr(), 0 if rows is None else rows.shape[1], *at,
+                  out.data_ptr(), T, H, _lib.dtype_code(out.dtype), _lib.stream_ptr(out.device))  # fmt: skip
+        return out, None, None
+
+
+def token_branches(x: torch.Tensor, k: int, n: int):
+    """``x`` ``[T, H]`` for a MoE block's branches: the expanded view ``[T, k, H]`` with one row per (token,
+    choice) for the experts, and ``n`` (up to 3) times ``x`` itself.  The backward adds the branches'
+    gradients, the k rows of the experts' included, in one pass with one rounding, where a reduction and an
+    addition per branch would each read and write the whole tensor."""
+    if not (torch.is_grad_enabled() and x.requires_grad):
+        return (x.unsqueeze(1).expand(-1, k, -1), *([x] * n))
+    return _Branches.apply(x, k, n)
