@@ -204,3 +204,18 @@ def test_receiver_simulation_roundtrip():
         assert torch.equal(torch.cat(rows)[adj], torch.cat(refs))
         ref_e, ref_adj, _, _ = OD.simulate_receiver_expand_idx(ids, recv, ep, epr)
         assert torch.equal(adj.cpu(), ref_adj) and torch.equal(eidx[: ref_e.numel()].cpu(), ref_e)
+
+
+@pytest.mark.parametrize("copies", [7, 8, 9, 63, 64, 65, 200])
+def test_gather_backward_with_rows_at_the_edges_of_the_source_lists(copies):
+    """Rows gathered about as often as their slots hold, as a wave's registers sort, and more often; a row
+    that is never gathered, and one that only the last index names."""
+    T = _ts()
+    g = torch.Generator().manual_seed(copies)
+    rows, H = 40, 264
+    idx = torch.arange(rows - 2).repeat(copies)
+    idx = torch.cat([idx[torch.randperm(idx.numel(), generator=g)], torch.tensor([rows - 1])])
+    x = torch.randn((rows, H), generator=g).bfloat16().cuda().requires_grad_(True)
+    go = torch.randn((idx.numel(), H), generator=g).bfloat16()
+    T.padded_index_gather(x, idx.cuda()).backward(go.cuda())
+    assert torch.equal(x.grad.cpu().view(torch.uint8), OP.padded_index_gather_backward(go, idx, rows).view(torch.uint8))
