@@ -260,6 +260,10 @@ class GemmTimer:
                 return r * cols * (4 + 2 * sc)
             if name == "pt_quant_rowwise_blockwise_transpose_ld":
                 return r * cols * (4 + sc)
+            if name == "pt_quant_weights":
+                return 3 * r * cols
+            if name == "pt_quant_blockwise_transpose_batched":
+                return 4 * r * cols
             return None
 
         def nbytes(name, a):

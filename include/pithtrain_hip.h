@@ -668,6 +668,8 @@ int pt_linear_backward(const pt_linear_backward_args* args /* host */);
  * {rows, columns, source rows} of a quantisation. */
 typedef void (*pt_observer_t)(const char* name, int begin, int64_t a, int64_t b, int64_t c);
 void pt_set_observer(pt_observer_t fn);
+/* Reports an entry point that a caller outside this library runs as part of a whole step of its own. */
+void pt_observe(const char* name, int begin, int64_t a, int64_t b, int64_t c);
 
 /* In-place fused cross-entropy with mean reduction (CrossEntropy.forward and its Triton kernel
  * cross_entropy_fwd, operators/cross_entropy.py:16-78,86-118): logits [N,V] in dtype are

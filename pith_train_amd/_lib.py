@@ -103,6 +103,7 @@ SIGNATURES = {
     "pt_linear_backward_workspace_bytes": (I64, [I64, I64, I64, I64, I64, I64]),
     "pt_linear_backward": (c_int, [c_char_p]),
     "pt_set_observer": (None, [P]),
+    "pt_observe": (None, [c_char_p, c_int, I64, I64, I64]),
 }
 
 _lib = None
@@ -130,6 +131,26 @@ def load() -> ctypes.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The C++ host side (``_host.so``, built from ``csrc/host.cpp``): loaded once, bound to the same library."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as exc:
+            raise PithTrainHipError(
+                f"{os.path.join(_HERE, '_host.so')} is missing or was built for another torch: build it with "
+                "`make -C pith_train_amd/csrc`"
+            ) from exc
+        module.init(LIB_PATH, PithTrainHipError)
+        _host = module
+    return _host
 
 
 def dtype_code(dtype: torch.dtype) -> int:

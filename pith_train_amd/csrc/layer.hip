@@ -34,6 +34,9 @@ struct Carve {
 using namespace pt;
 
 extern "C" void pt_set_observer(pt_observer_t fn) { g_observer = fn; }
+extern "C" void pt_observe(const char* name, int begin, int64_t a, int64_t b, int64_t c) {
+  if (g_observer) g_observer(name, begin, a, b, c);
+}
 
 extern "C" int pt_experts_forward(const pt_experts_forward_args* args) {
   PT_REQUIRE(args, "experts_forward: null arguments");

@@ -9,7 +9,6 @@ here.
 from __future__ import annotations
 
 import os
-import struct
 
 import torch
 
@@ -269,9 +268,6 @@ def fp8cast_grouped_weight_cat(parts):
     return fp8cast_blockwise_transpose_batched_cat(parts, twin=weight_twin_enabled())
 
 
-_WEIGHT_PART = struct.Struct("=10q").pack
-
-
 def fp8cast_grouped_weights(weights):
     """``[fp8cast_grouped_weight_cat(parts) for parts in weights]`` - the fused operand of every list of
     ``[G, N_i, K]`` parts - with one launch for all of them when no twin is wanted: the projections of
@@ -281,26 +277,4 @@ def fp8cast_grouped_weights(weights):
     if weight_twin_enabled() or len(flat) > _lib.PT_QUANT_WEIGHTS_MAX or any(t.dtype != dtype for t in flat) or any(
             len(parts) > 1 and t.shape[1] % 128 for parts in weights for t in parts):
         return [fp8cast_grouped_weight(parts[0]) if len(parts) == 1 else fp8cast_grouped_weight_cat(parts) for parts in weights]
-    dev = flat[0].device
-    block, result, i = b"", [], 0
-    for parts in weights:
-        G, N, K = parts[0].shape
-        for p in parts[1:]:
-            assert p.ndim == 3 and p.shape[0] == G and p.shape[2] == K
-            N += p.shape[1]
-        nb, kb = _cdiv(N, 128), _cdiv(K, 128)
-        out = torch.empty((G, N, K), dtype=FP8, device=dev)
-        scale = torch.empty((G, nb, kb), dtype=torch.float32, device=dev)
-        row = 0
-        for _ in parts:
-            x3 = flat[i]
-            n = x3.shape[1]
-            block += _WEIGHT_PART(
-                x3.data_ptr(), G, n, K, x3.stride(0) if G > 1 else n * K, x3.stride(1) if n > 1 else K,
-                out.data_ptr() + row * K, N * K, scale.data_ptr() + 4 * (row // 128) * kb, nb * kb,
-            )  # fmt: skip
-            row += n
-            i += 1
-        result.append((out, scale, None, None))
-    _lib.call("pt_quant_weights", block, i, _lib.dtype_code(dtype), _lib.stream_ptr(dev))
-    return result
+    return [(q, scale, None, None) for q, scale in _lib.host().quant_grouped_weights(weights, _lib.stream_ptr(flat[0].device))]

@@ -11,15 +11,12 @@ The token permutation can be folded in as well (``row_map``, see ``FP8GroupedLin
 
 from __future__ import annotations
 
-import functools
-import struct
-
 import torch
 
 from .. import _lib
 from ..dualpipe_utils import WeightGradStore
 from .deepgemm_quantize import FP8
-from .grouped_linear import dgrad_operand, m_grouped_fp8_dgrad, schedule_wgrad, wgrad_target
+from .grouped_linear import dgrad_operand, m_grouped_fp8_dgrad, schedule_wgrad
 from .token_scatter import _GEMM_ALLOC_ALIGNMENT, _PaddedIndexGather
 
 
@@ -128,59 +125,6 @@ def compose_row_maps(row_map: torch.Tensor, expand_idx: torch.Tensor, n_src: int
     return out
 
 
-_FORWARD_BLOCK = struct.Struct("=14q11q2d10q").pack
-_BACKWARD_BLOCK = struct.Struct("=35q2d5q").pack
-_ONE_BUFFER = 32 << 20  # bytes up to which the tensors of one kind share an allocation
-
-
-@functools.lru_cache(maxsize=256)
-def _sizes(M, K, half, H):
-    """Byte sizes of what a step allocates: kept activations (x^T, its scales, h^T, its scales), forward
-    temporaries (composed map, x, its scales, h, its scales), transposed gradients (dy^T, scales,
-    gate_up's^T, scales), backward temporaries (dy, scales, grad_h, column sums)."""
-    blocks = M // 128
-    return (
-        _offsets(K * M, 4 * blocks * K, half * M, 4 * blocks * half),
-        _offsets(4 * M, M * K, 4 * M * _cdiv(K, 128), M * half, 4 * M * _cdiv(half, 128)),
-        _offsets(H * M, 4 * blocks * H, 2 * half * M, 8 * blocks * half),
-        _offsets(M * H, 4 * M * _cdiv(H, 128), 2 * M * half, 8 * blocks * half),
-    )
-
-
-def _offsets(*sizes):
-    offsets, total = [], 0
-    for n in sizes:
-        offsets.append(total)
-        total += (n + 255) // 256 * 256
-    return sizes, tuple(offsets), total
-
-
-def _allocate(layout, dev):
-    """(tensors that own the memory, addresses of its pieces): one buffer for small pieces (an allocation
-    costs the host two microseconds), one each for large ones."""
-    sizes, offsets, total = layout
-    if total <= _ONE_BUFFER:
-        buffers = [torch.empty(total, dtype=torch.uint8, device=dev)]
-    else:
-        buffers = [torch.empty(n, dtype=torch.uint8, device=dev) for n in sizes]
-    return buffers, _addresses(layout, buffers)
-
-
-def _addresses(layout, buffers):
-    if len(buffers) > 1:
-        return [b.data_ptr() for b in buffers]
-    base = buffers[0].data_ptr()
-    return [base + o for o in layout[1]]
-
-
-def _piece(layout, buffers, i, rows, cols, dtype):
-    """Piece ``i`` as a ``[rows, cols]`` tensor."""
-    if len(buffers) > 1:
-        return buffers[i].view(dtype).view(rows, cols)
-    at = layout[1][i]
-    return buffers[0][at : at + layout[0][i]].view(dtype).view(rows, cols)
-
-
 FEW_ROWS = 64  # group alignment of forwards that no backward follows, see few_rows_per_expert
 
 
@@ -226,20 +170,11 @@ def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down
         routed = expand_idx.shape[0]
     if x.stride(1) != 1:
         x = x.contiguous()
-    dev = x.device
-    kept_layout, temp_layout, _, _ = _sizes(M, K, half, H)
-    kept, kept_at = _allocate(kept_layout, dev) if ctx is not None else ((), (0, 0, 0, 0))
-    _temp, temp_at = _allocate(temp_layout, dev)
-    gate_up = torch.empty((M, 2 * half), device=dev, dtype=x.dtype)
-    out = torch.empty((routed if scatter else M, H), device=dev, dtype=x.dtype)
     b_gate_up, b_down = biases if biases[0] is None else [b.detach().contiguous() for b in biases]
-    alpha, limit = clamp or (0.0, 0.0)
-    _lib.call("pt_experts_forward", _FORWARD_BLOCK(
-        x.data_ptr(), src_rows, x.stride(0) if src_rows > 1 else K, M, K, half, H, G, grouped_mm_offs.data_ptr(), _lib.ptr(row_map) or 0,
-        _lib.ptr(expand_idx) or 0, 0 if expand_idx is None else routed, repeat, few_rows, gu_fp8.data_ptr(), gu_scale.data_ptr(), _lib.ptr(b_gate_up) or 0,
-        dn_fp8.data_ptr(), dn_scale.data_ptr(), _lib.ptr(b_down) or 0, gate_up.data_ptr(), out.data_ptr(), out.shape[0], scatter,
-        clamp is not None, alpha, limit, *kept_at, *temp_at, _lib.stream_ptr(dev),
-    ))  # fmt: skip
+    out, gate_up, kept = _lib.host().experts_forward(
+        x, repeat, row_map, expand_idx, grouped_mm_offs, gu_fp8, gu_scale, dn_fp8, dn_scale, half, b_gate_up, b_down, scatter,
+        clamp is not None, *(clamp or (0.0, 0.0)), ctx is not None, few_rows, _lib.stream_ptr(x.device),
+    )  # fmt: skip
     if ctx is None:
         return out
     gu_dg, gu_dg_s, gu_forward = dgrad_operand(q_gate_up, gate_up_weights, M)
@@ -247,7 +182,7 @@ def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down
     ctx.save_for_backward(gu_dg, gu_dg_s, dn_dg, dn_dg_s, grouped_mm_offs, gate_up, row_map, expand_idx, *kept)
     ctx.gate_up_weights, ctx.w_down = gate_up_weights, w_down
     ctx.clamp = clamp
-    ctx.bias_dtypes = tuple(None if b is None else b.dtype for b in biases)
+    ctx.biases = biases
     ctx.dims = (M, K, half, H, G, routed, src_rows, gu_forward, dn_forward, scatter)
     ctx.repeat = repeat
     return out
@@ -258,52 +193,27 @@ def _backward(ctx, grad_out):
     gradients go to ``.grad``, or to the ``WeightGradStore`` queue."""
     gu_dg, gu_dg_s, dn_dg, dn_dg_s, offs, gate_up, row_map, expand_idx, *kept = ctx.saved_tensors
     M, K, half, H, G, routed, src_rows, gu_forward, dn_forward, scatter = ctx.dims
-    grad_out = grad_out.contiguous()
-    dev = grad_out.device
     split = isinstance(ctx.gate_up_weights, tuple)
     gu_weights = ctx.gate_up_weights if split else (ctx.gate_up_weights,)
     deferred = WeightGradStore.enabled
     # separate gate and up parameters: each gets its half of the gate_up weight gradient's rows
-    targets = [(None, False, None)] * 3 if deferred else [wgrad_target(w) for w in (ctx.w_down, *gu_weights)]
-    if len(targets) == 2:
-        targets.append((None, False, None))
-    kept_layout, _, twin_layout, temp_layout = _sizes(M, K, half, H)
-    twins, twins_at = _allocate(twin_layout, dev)
-    _temp, temp_at = _allocate(temp_layout, dev)
-    dgu = torch.empty((M, 2 * half), device=dev, dtype=FP8)
-    dgu_s = torch.empty((M, _cdiv(2 * half, 128)), device=dev, dtype=torch.float32)
-    d_gu, d_dn = ctx.bias_dtypes
-    d_gu_bias = None if d_gu is None else torch.empty((G, 2 * half), device=dev, dtype=d_gu)
-    d_dn_bias = None if d_dn is None else torch.empty((G, H), device=dev, dtype=d_dn)
-    (dw_down, add_down, _), (dw_gu, add_gu, _), (dw_up, add_up, _) = targets
-    alpha, limit = ctx.clamp or (0.0, 0.0)
-    block = _BACKWARD_BLOCK(
-        grad_out.data_ptr(), grad_out.shape[0], M, K, half, H, G, offs.data_ptr(), (_lib.ptr(row_map) or 0) if scatter else 0,
-        row_map is not None, dn_dg.data_ptr(), dn_dg_s.data_ptr(), dn_forward, gate_up.data_ptr(),
-        *_addresses(kept_layout, kept), dgu.data_ptr(), dgu_s.data_ptr(), *twins_at, *temp_at, _lib.ptr(dw_down) or 0, add_down, _lib.ptr(dw_gu) or 0, add_gu, _lib.ptr(dw_up) or 0, add_up,
-        ctx.clamp is not None, alpha, limit, _lib.ptr(d_gu_bias) or 0, 0 if d_gu is None else _lib.dtype_code(d_gu),
-        _lib.ptr(d_dn_bias) or 0, 0 if d_dn is None else _lib.dtype_code(d_dn), _lib.stream_ptr(dev),
+    step = _lib.host().ExpertsBackward(
+        grad_out, (M, K, half, H, G), offs, row_map, scatter, dn_dg, dn_dg_s, dn_forward, gate_up, kept, ctx.clamp is not None,
+        *(ctx.clamp or (0.0, 0.0)), *ctx.biases, [] if deferred else [ctx.w_down, *gu_weights], _lib.stream_ptr(grad_out.device),
     )  # fmt: skip
-    _lib.call("pt_experts_backward", block)
-    grad_x = torch.empty((M if row_map is None else routed, K), device=dev, dtype=grad_out.dtype)
-    m_grouped_fp8_dgrad((dgu, dgu_s), gu_dg, gu_dg_s, gu_forward, grad_x, offs, row_map)
+    grad_x = torch.empty((M if row_map is None else routed, K), device=grad_out.device, dtype=grad_out.dtype)
+    m_grouped_fp8_dgrad((step.dgu, step.dgu_s), gu_dg, gu_dg_s, gu_forward, grad_x, offs, row_map)
     if not deferred:
-        _lib.call("pt_experts_weight_gradient", block)
-    for _, _, finish in targets:
-        if finish is not None:
-            finish()
-    if deferred:
-        blocks, f32 = M // 128, torch.float32
-        dy_t = _piece(twin_layout, twins, 0, H, M, FP8), _piece(twin_layout, twins, 1, blocks, H, f32)
-        gu, gus = _piece(twin_layout, twins, 2, 2 * half, M, FP8), _piece(twin_layout, twins, 3, blocks, 2 * half, f32)
-        x_t = _piece(kept_layout, kept, 0, K, M, FP8), _piece(kept_layout, kept, 1, blocks, K, f32)
-        h_t = _piece(kept_layout, kept, 2, half, M, FP8), _piece(kept_layout, kept, 3, blocks, half, f32)
+        step.weight_gradient()
+    else:
+        dy_t, (gu, gus), x_t, h_t = step.operands()
         schedule_wgrad(ctx.w_down, dy_t, h_t, offs)
         if split:
             schedule_wgrad(gu_weights[0], (gu[:half], gus[:, :half]), x_t, offs)
             schedule_wgrad(gu_weights[1], (gu[half:], gus[:, half:]), x_t, offs)
         else:
             schedule_wgrad(gu_weights[0], (gu, gus), x_t, offs)
+    d_gu_bias, d_dn_bias = step.d_gu_bias, step.d_dn_bias
     if expand_idx is not None:
         # one gradient row per routed row so far: rows that expand the same source row are summed
         # (the backward of the expanding gather, token_scatter.py:311-325)

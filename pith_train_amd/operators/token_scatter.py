@@ -37,22 +37,7 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
 def group_rows(expert_idxs: torch.Tensor, num_groups: int, padding_alignment: int, cap: int, need_reverse: bool = True):
     """Index half of the scatter: (reverse i64[m], offs i32[G], ks i32[G], src_of i32[cap]); ``reverse`` is
     None unless it is needed."""
-    m = expert_idxs.shape[0]
-    dev = expert_idxs.device
-    reverse = torch.empty((m,), device=dev, dtype=torch.int64) if need_reverse else None
-    ws_bytes = _lib.query("pt_group_rows_workspace_bytes", m, num_groups)
-    # one allocation for the four int32 results and the workspace; src_of first, its start aligned
-    pad = -cap % 4
-    words = torch.empty((cap + pad + 2 * num_groups + ws_bytes // 4 + 64,), device=dev, dtype=torch.int32)
-    at = words.data_ptr()
-    offs_at = at + 4 * (cap + pad)
-    ws_at = (offs_at + 8 * num_groups + 255) & ~255
-    _lib.call(
-        "pt_group_rows", expert_idxs.data_ptr(), m, num_groups, padding_alignment, offs_at, offs_at + 4 * num_groups,
-        _lib.ptr(reverse), at, cap, ws_at if ws_bytes else None, ws_bytes, _lib.stream_ptr(dev),
-    )  # fmt: skip
-    o = cap + pad
-    return reverse, words[o : o + num_groups], words[o + num_groups : o + 2 * num_groups], words[:cap]
+    return _lib.host().group_rows(expert_idxs, num_groups, padding_alignment, cap, need_reverse, _lib.stream_ptr(expert_idxs.device))
 
 
 def group_rows_with_sizes(expert_idxs: torch.Tensor, num_groups: int, padding_alignment: int = 128, device=None,
