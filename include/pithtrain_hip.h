@@ -201,6 +201,17 @@ int pt_gemm_nt_dense(const void* a_fp8, const float* a_scale, const void* b_fp8,
 int pt_gemm_nt_dense_ld(const void* a_fp8, int64_t lda, const float* a_scale, const void* b_fp8,
                         int64_t ldb, const float* b_scale, void* out, int out_dtype, int64_t M,
                         int64_t N, int64_t K, pt_stream_t stream);
+/* Two products in the form of pt_gemm_nt_dense_ld that do not depend on each other (the input and the weight
+ * gradient of a dense linear, linear.py:77-80), in one launch where they are small.  All fields are 8
+ * bytes wide. */
+typedef struct {
+  const void* a_fp8; int64_t lda; const float* a_scale;
+  const void* b_fp8; int64_t ldb; const float* b_scale;
+  void* out;
+  int64_t M, N, K;
+} pt_dense_gemm;
+int pt_gemm_nt_dense_pair(const pt_dense_gemm* two /* host, [2] */, int out_dtype, pt_stream_t stream);
+
 /* pt_gemm_nt_dense (packed operands, bf16 result) whose columns go to two tensors, head by head: result
  * column h * (head_a + head_b) + c is out[:, h * head_a + c] for c < head_a and
  * out2[:, h * head_b + c - head_a] behind it; out [M, heads * head_a], out2 [M, heads * head_b] packed.

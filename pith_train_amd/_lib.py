@@ -48,6 +48,7 @@ SIGNATURES = {
     "pt_gemm_nt_dense_splitk": (c_int, [P, P, P, P, P, I32, I64, I64, I64, I64, P]),
     "pt_gemm_nt_dense_ld": (c_int, [P, I64, P, P, I64, P, P, c_int, I64, I64, I64, P]),
     "pt_gemm_nt_dense_splitk_ld": (c_int, [P, I64, P, P, I64, P, P, I32, I64, I64, I64, I64, P]),
+    "pt_gemm_nt_dense_pair": (c_int, [c_char_p, c_int, P]),
     "pt_gemm_nt_dense_heads": (c_int, [P, P, P, P, P, P, I64, I64, I64, I64, I64, P]),
     "pt_sum_partials": (c_int, [P, I32, I64, P, c_int, P]),
     "pt_gemm_m_grouped_nt": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P]),

@@ -394,17 +394,15 @@ extern "C" int pt_gemm_select_kernel(const char* name) {
 
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-static int gemm_nt_dense_impl(const void* a_fp8, int64_t lda, const float* a_scale, const void* b_fp8, int64_t ldb,
+static int fill_dense(GemmArgs& g, const void* a_fp8, int64_t lda, const float* a_scale, const void* b_fp8, int64_t ldb,
                               const float* b_scale, void* out, int out_dtype, int64_t M, int64_t N, int64_t K,
-                              pt_stream_t stream, void* out2 = nullptr, int64_t head_a = 0, int64_t head_b = 0, int64_t extent = 0) {
+                              void* out2, int64_t head_a, int64_t head_b, int64_t extent) {
   PT_REQUIRE(M >= 0 && N >= 0 && K >= 0, "gemm_nt_dense: negative size");
-  if (M == 0 || N == 0) return PT_OK;
   PT_REQUIRE(K > 0 && K % 16 == 0, "gemm_nt_dense: K=%lld must be a positive multiple of 16", (long long)K);
   PT_REQUIRE(lda >= K && ldb >= K && lda % 16 == 0 && ldb % 16 == 0, "gemm_nt_dense: row pitches must be multiples of 16 and at least K");
   PT_REQUIRE(a_fp8 && a_scale && b_fp8 && b_scale && out && al16(a_fp8) && al16(b_fp8), "gemm_nt_dense: null or misaligned pointer");
   PT_REQUIRE(out_dtype == PT_BF16 || out_dtype == PT_F32, "gemm_nt_dense: out_dtype must be bf16 or fp32");
   const int64_t KB = cdiv(K, 128);
-  GemmArgs g = {};
   g.a = (const uint8_t*)a_fp8; g.lda = lda; g.b = (const uint8_t*)b_fp8; g.ldb = ldb;
   g.sa = a_scale; g.sa_rs = KB; g.sa_ks = 1; g.sa_shift = 0;
   g.sb = b_scale; g.sb_rs = KB; g.sb_ks = 1; g.sb_shift = 7;
@@ -414,7 +412,36 @@ static int gemm_nt_dense_impl(const void* a_fp8, int64_t lda, const float* a_sca
   g.tiles_a = (int)cdiv(M, 128); g.tiles_b = (int)cdiv(N, 128);
   g.total_tiles = (int64_t)g.tiles_a * g.tiles_b;
   g.out2 = out2; g.head_a = (int)head_a; g.head_b = (int)head_b; g.out_extent = extent;
+  return PT_OK;
+}
+
+static int gemm_nt_dense_impl(const void* a_fp8, int64_t lda, const float* a_scale, const void* b_fp8, int64_t ldb,
+                              const float* b_scale, void* out, int out_dtype, int64_t M, int64_t N, int64_t K,
+                              pt_stream_t stream, void* out2 = nullptr, int64_t head_a = 0, int64_t head_b = 0, int64_t extent = 0) {
+  if (M == 0 || N == 0) return PT_OK;
+  GemmArgs g = {};
+  if (int rc = fill_dense(g, a_fp8, lda, a_scale, b_fp8, ldb, b_scale, out, out_dtype, M, N, K, out2, head_a, head_b, extent)) return rc;
   return dispatch_gemm(g, (hipStream_t)stream);
+}
+
+extern "C" int pt_gemm_nt_dense_pair(const pt_dense_gemm* two, int out_dtype, pt_stream_t stream) {
+  PT_REQUIRE(two, "gemm_nt_dense_pair: null arguments");
+  GemmArgs g[2] = {};
+  for (int i = 0; i < 2; ++i) {
+    const pt_dense_gemm& q = two[i];
+    PT_REQUIRE(q.M > 0 && q.N > 0, "gemm_nt_dense_pair: empty product");
+    if (int rc = fill_dense(g[i], q.a_fp8, q.lda, q.a_scale, q.b_fp8, q.ldb, q.b_scale, q.out, out_dtype, q.M, q.N, q.K, nullptr, 0, 0, 0)) return rc;
+  }
+  // One launch where each would take the small-tile kernel and their tiles together still make one round
+  // of two workgroups per compute unit, 64-row tiles if those do (4096 x 512 x 4096 twice, 256 tiles
+  // each: 39.7 us in two launches, 11 less in one).
+  if (gemm_impl() == IMPL_AUTO && fits_persistent(g[0]) && fits_persistent(g[1]) && small_tile_rows(g[0]) && small_tile_rows(g[1])) {
+    for (int rows : {64, 128})
+      if (cdiv(g[0].rows_a, rows) * cdiv(g[0].rows_b, 128) + cdiv(g[1].rows_a, rows) * cdiv(g[1].rows_b, 128) <= 512)
+        return launch_gemm_small_pair(g[0], g[1], rows, (hipStream_t)stream);
+  }
+  if (int rc = dispatch_gemm(g[0], (hipStream_t)stream)) return rc;
+  return dispatch_gemm(g[1], (hipStream_t)stream);
 }
 
 extern "C" int pt_gemm_nt_dense(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale, void* out,

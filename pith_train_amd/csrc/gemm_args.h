@@ -50,5 +50,7 @@ int launch_gemm_pipelined(const GemmArgs& a, int variant, hipStream_t stream);
 int launch_gemm_rowsplit(const GemmArgs& a, int variant, hipStream_t stream);
 // one tile of 64 or 128 rows x 128 columns per workgroup, for small problems (gemm_small.hip)
 int launch_gemm_small(const GemmArgs& a, int rows, hipStream_t stream);
+// the tiles of two independent dense products in one launch of that kernel
+int launch_gemm_small_pair(const GemmArgs& a, const GemmArgs& b, int rows, hipStream_t stream);
 
 }  // namespace pt

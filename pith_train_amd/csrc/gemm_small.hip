@@ -24,7 +24,7 @@ template <int BM> static constexpr int kSmallStages = BM == 64 ? 3 : 2;
 template <int BM> static constexpr size_t kSmallLds = (size_t)kSmallStages<BM> * (BM + 128) * (128 + 4) + 256;
 
 template <int MODE, int BM, bool ACC, bool BT>
-__global__ __launch_bounds__(256, 2) void fp8_gemm_small_kernel(GemmArgs p) {
+__device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
   constexpr int BN = 128, BK = 128, NS = kSmallStages<BM>;
   static_assert(2 * kSmallLds<BM> <= 160 * 1024, "two workgroups per compute unit");
   constexpr int TM = BM / 64, TN = 2;   // waves 2 x 2, each TM x 2 blocks of 32 x 32
@@ -45,8 +45,8 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_small_kernel(GemmArgs p) {
   // The m-grouped row count is known on the device only; workgroups past the real list end here. ----
   const int total = MODE == GEMM_M_GROUPED ? p.offs[p.G - 1] / BM * p.tiles_b : (int)p.total_tiles;
   const int per_xcd = (total + 7) >> 3;
-  const int idx = blockIdx.x >> 3;
-  const int t = (blockIdx.x & 7) * per_xcd + idx;
+  const int idx = block >> 3;
+  const int t = (block & 7) * per_xcd + idx;
   if (idx >= per_xcd || t >= total) return;
   Tile T;
   if (MODE == GEMM_M_GROUPED) {
@@ -206,18 +206,60 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_small_kernel(GemmArgs p) {
 }
 
 template <int MODE, int BM, bool ACC, bool BT>
-static int launch_small(GemmArgs a, hipStream_t stream) {
-  constexpr size_t lds = kSmallLds<BM>;
-  static bool attr_set = false;
-  auto kernel = fp8_gemm_small_kernel<MODE, BM, ACC, BT>;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) { set_error("gemm: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e)); return PT_ERR_LAUNCH; }
-    attr_set = true;
-  }
+__global__ __launch_bounds__(256, 2) void fp8_gemm_small_kernel(GemmArgs p) {
+  small_tile_body<MODE, BM, ACC, BT>(p, blockIdx.x);
+}
+
+// Two products that do not depend on each other (the input and the weight gradient of a dense linear): the
+// workgroups past `second` (a multiple of 8) take the second one's tiles, so that compute units which
+// either would leave with one workgroup or none hold two.
+struct GemmPair { GemmArgs g[2]; int second; };
+template <int BM>
+__global__ __launch_bounds__(256, 2) void fp8_gemm_small_pair_kernel(GemmPair q) {
+  const bool late = (int)blockIdx.x >= q.second;
+  small_tile_body<GEMM_DENSE, BM, false, false>(late ? q.g[1] : q.g[0], (int)blockIdx.x - (late ? q.second : 0));
+}
+
+template <int MODE, int BM>
+static void count_small_tiles(GemmArgs& a) {
   a.tiles_a = (int)cdiv(a.rows_a, BM);
   a.tiles_b = (int)cdiv(a.rows_b, 128);
   a.total_tiles = (int64_t)a.tiles_a * a.tiles_b * (MODE == GEMM_K_GROUPED ? a.G : 1);
+}
+
+template <class Kernel>
+static int reserve_lds(Kernel kernel, size_t lds, bool& done) {
+  if (done) return PT_OK;
+  hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) { set_error("gemm: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e)); return PT_ERR_LAUNCH; }
+  done = true;
+  return PT_OK;
+}
+
+template <int BM>
+static int launch_pair(const GemmArgs& a, const GemmArgs& b, hipStream_t stream) {
+  static bool reserved = false;
+  if (int rc = reserve_lds(fp8_gemm_small_pair_kernel<BM>, kSmallLds<BM>, reserved)) return rc;
+  GemmPair q = {{a, b}, 0};
+  count_small_tiles<GEMM_DENSE, BM>(q.g[0]);
+  count_small_tiles<GEMM_DENSE, BM>(q.g[1]);
+  q.second = (int)(cdiv(q.g[0].total_tiles, 8) * 8);
+  hipLaunchKernelGGL(fp8_gemm_small_pair_kernel<BM>, dim3((unsigned)(q.second + cdiv(q.g[1].total_tiles, 8) * 8)), dim3(256), kSmallLds<BM>, stream, q);
+  return check_launch("fp8_gemm_small_pair_kernel");
+}
+
+int launch_gemm_small_pair(const GemmArgs& a, const GemmArgs& b, int rows, hipStream_t stream) {
+  PT_REQUIRE(rows == 64 || rows == 128, "gemm: the small-problem kernel has tiles of 64 or 128 rows");
+  return rows == 64 ? launch_pair<64>(a, b, stream) : launch_pair<128>(a, b, stream);
+}
+
+template <int MODE, int BM, bool ACC, bool BT>
+static int launch_small(GemmArgs a, hipStream_t stream) {
+  constexpr size_t lds = kSmallLds<BM>;
+  static bool reserved = false;
+  auto kernel = fp8_gemm_small_kernel<MODE, BM, ACC, BT>;
+  if (int rc = reserve_lds(kernel, lds, reserved)) return rc;
+  count_small_tiles<MODE, BM>(a);
   if (a.total_tiles == 0) return PT_OK;
   PT_REQUIRE(a.total_tiles < (1ll << 28), "gemm: too many tiles");
   hipLaunchKernelGGL(kernel, dim3((unsigned)(cdiv(a.total_tiles, 8) * 8)), dim3(256), lds, stream, a);

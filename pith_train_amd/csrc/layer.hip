@@ -236,6 +236,12 @@ extern "C" int pt_linear_backward(const pt_linear_backward_args* args) {
             g_s, g_t, ld_t, g_ts, a.stream);
   else
     PT_STEP(pt_quant_rowwise_transpose_ld, a.M, a.N, a.M, a.grad, (int)a.dtype, a.M, a.N, a.ldg, g_fp8, g_s, g_t, ld_t, g_ts, a.stream);
+  if (a.x_splits <= 1 && a.w_splits <= 1) {
+    const pt_dense_gemm two[2] = {{g_fp8, a.N, g_s, a.w_t_fp8, a.N, a.w_t_scale, a.grad_x, a.M, a.K, a.N},
+                                  {g_t, ld_t, g_ts, x_t, ld_xt, x_ts, a.grad_w, a.N, a.K, red}};
+    PT_STEP(pt_gemm_nt_dense_pair, 2 * a.M, a.K, a.N, two, (int)a.out_dtype, a.stream);
+    return PT_OK;
+  }
   if (int rc = dense_gemm(g_fp8, a.N, g_s, a.w_t_fp8, a.N, a.w_t_scale, a.grad_x, (int)a.out_dtype, a.M, a.K, a.N, a.x_splits,
                           a.x_split_len, slabs, a.stream)) return rc;
   return dense_gemm(g_t, ld_t, g_ts, x_t, ld_xt, x_ts, a.grad_w, (int)a.out_dtype, a.N, a.K, red, a.w_splits, a.w_split_len,

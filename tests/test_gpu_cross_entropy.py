@@ -128,3 +128,29 @@ def test_full_size_rows_sum_to_zero_and_loss_matches_torch():
     sums = a.float().sum(-1) * n
     assert sums[y == -100].abs().max() == 0
     assert sums[y != -100].abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("N,V,dtype", [(256, 264, torch.bfloat16), (257, 8, torch.bfloat16), (515, 125000, torch.float16), (600, 122880, torch.bfloat16)])
+def test_more_rows_than_workgroups(N, V, dtype):
+    """A workgroup that walks several rows gives each of them what a workgroup of its own gives: rows within
+    the registers, exactly as long as they hold, and past them; ignored rows in every position."""
+    from pith_train_amd.operators.cross_entropy import cross_entropy
+
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = (torch.randn((N, V), device="cuda", generator=g) * 2).to(dtype)
+    y = torch.randint(0, V, (N,), device="cuda", generator=g)
+    y[::5] = -100
+    whole = x.clone()
+    loss = cross_entropy(whole, y)
+    total = torch.zeros((), dtype=torch.float64, device="cuda")
+    n = int((y != -100).sum())
+    for r0 in range(0, N, 128):
+        part, yp = x[r0 : r0 + 128].clone(), y[r0 : r0 + 128]
+        np_ = max(1, int((yp != -100).sum()))
+        total += cross_entropy(part, yp).double() * np_
+        a, b = whole[r0 : r0 + 128].float() * n, part.float() * np_  # both rounded after the division by their own n
+        step = 2.0 ** (-6 if dtype == torch.bfloat16 else -9)
+        at_target = torch.zeros_like(b)  # there the softmax term was rounded before 1 was taken off
+        at_target[torch.arange(len(yp), device="cuda"), yp.clamp(min=0)] = step
+        assert ((a - b).abs() <= step * b.abs() + at_target + (2.0 ** -20 if dtype == torch.float16 else 1e-20) * n).all()
+    torch.testing.assert_close(loss.double(), total / n, rtol=1e-5, atol=1e-6)

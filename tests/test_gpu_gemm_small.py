@@ -77,3 +77,57 @@ def test_grouped(rows, n, k, form):
         index[::7] = -1
         index = index.cuda()
     _same_bits(lambda: m_grouped_fp8_gemm_nn((a, sa), (b, sb), out, offs, index), out, "r0")
+
+
+@pytest.mark.parametrize("first,second", [((1, 16, 16), (70, 24, 144)), ((1001, 2048, 512), (512, 2048, 1008)), ((640, 264, 400), (129, 1000, 272)),
+                                          ((2048, 2048, 256), (2048, 2048, 128)), ((4096, 2048, 128), (128, 128, 128))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_two_products_in_one_launch(first, second, dtype):
+    """Pairs that share a launch of 64- or 128-row tiles, and pairs that are too large for one."""
+    import struct
+
+    from pith_train_amd import _lib
+
+    g = torch.Generator().manual_seed(first[0])
+    block, got, want, keep = b"", [], [], []
+    for m, n, k in (first, second):
+        a, sa, b, sb = _fp8(g, m, k), _scale(g, m, _cdiv(k, 128)), _fp8(g, n, k), _scale(g, _cdiv(n, 128), _cdiv(k, 128))
+        keep.append((a, sa, b, sb))
+        got.append(torch.full((m, n), 0.5, device="cuda", dtype=dtype))
+        want.append(torch.empty((m, n), device="cuda", dtype=dtype))
+        _lib.call("pt_gemm_nt_dense", a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), want[-1].data_ptr(), _lib.dtype_code(dtype),
+                  m, n, k, _lib.stream_ptr())
+        block += struct.pack("=10q", a.data_ptr(), k, sa.data_ptr(), b.data_ptr(), k, sb.data_ptr(), got[-1].data_ptr(), m, n, k)
+    _lib.call("pt_gemm_nt_dense_pair", block, _lib.dtype_code(dtype), _lib.stream_ptr())
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("rows,n,k", [([64, 0, 192, 128, 64], 264, 400), ([64] * 70, 72, 1040), ([0, 64], 8, 16)])
+@pytest.mark.parametrize("scatter,bias", [(False, False), (True, False), (False, True), (True, True)])
+def test_groups_of_a_few_rows(rows, n, k, scatter, bias):
+    """Group ends at odd multiples of 64, against one dense product per group."""
+    from pith_train_amd import _lib
+
+    g = torch.Generator().manual_seed(n + k)
+    G, M, cap = len(rows), sum(rows), sum(rows) + 128
+    offs = torch.tensor(rows).cumsum(0).to(torch.int32).cuda()
+    a, sa = _fp8(g, cap, k), _scale(g, cap, _cdiv(k, 128))
+    b, sb = _fp8(g, G, n, k), _scale(g, G, _cdiv(n, 128), _cdiv(k, 128))
+    bias_rows = torch.randn((G, n), generator=g).bfloat16().cuda() if bias else None
+    index = torch.randperm(cap, generator=g).to(torch.int32).cuda() if scatter else None
+    out = torch.zeros((cap, n), device="cuda", dtype=torch.bfloat16)
+    _lib.call("pt_gemm_m_grouped_nt_few_rows", a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), out.data_ptr(), _lib.PT_BF16,
+              offs.data_ptr(), G, cap, n, k, _lib.ptr(index), cap, _lib.ptr(bias_rows), _lib.stream_ptr())
+    want, row = torch.zeros_like(out), 0
+    for q, r in enumerate(rows):
+        if r:
+            y = torch.empty((r, n), device="cuda", dtype=torch.bfloat16)
+            _lib.call("pt_gemm_nt_dense", a[row:].data_ptr(), sa[row:].data_ptr(), b[q].data_ptr(), sb[q].data_ptr(), y.data_ptr(),
+                      _lib.PT_BF16, r, n, k, _lib.stream_ptr())
+            y = y + bias_rows[q] if bias else y
+            if scatter:
+                want[index[row : row + r].long()] = y
+            else:
+                want[row : row + r] = y
+        row += r
+    assert row == M and torch.equal(out, want)
