@@ -286,18 +286,23 @@ static int gemm_impl() {
   return g_impl;
 }
 
-// Choice of the persistent kernel, from measurements on MI355X inside a training step (operands
-// freshly written, i.e. partly cache-resident):
-//   m-grouped, k-grouped  the row-split loop: its loads never pause, which matters most where
-//              operands come from HBM (every group has its own b operand), and waves of a half-empty
-//              tile skip their MFMAs.  +1..5 % per layer over the better of the other two.
+// Choice of the persistent kernel, from measurements on MI355X:
+//   m-grouped  the row-split loop: its loads never pause, which matters most where operands come from
+//              HBM (every group has its own b operand), and waves of a half-empty tile skip their
+//              MFMAs (us, against the software-pipelined loop: 32 groups of about 2048 rows, 5760 x
+//              2880 weights 1194 / 1250, of 1000 rows 602 / 645, 128 groups 873 / 880).
+//   k-grouped  the software-pipelined loop: both operands are shared by a whole group, there are no
+//              half-empty tiles, and one barrier per block counts for more (us, against the row-split
+//              loop: 32 groups of about 2048 rows 5760 x 2880 1165 / 1218, 64 Zipf-distributed groups
+//              of 768 in the mean 2816 x 2048 420 / 459 and 2048 x 1408 198 / 233, split reductions
+//              4096 x 2048 x 32768 240 / 253 and 2816 x 2048 x 8192 56 / 64; 128 groups of 512 level).
 //   dense      the software-pipelined loop from K = 512 on (+5 % at 512, +13..20 % from 2048 on
 //              over the two-phase loop, +5..8 % over the row-split loop); below, the two-phase loop,
 //              which has no fill/drain of one 128-block per tile.
 enum { KERNEL_TWO_PHASE, KERNEL_PIPELINED, KERNEL_ROWSPLIT };
 static int preferred_kernel(const GemmArgs& g) {
-  if (g.mode != GEMM_DENSE) return KERNEL_ROWSPLIT;
-  return g.red >= 512 ? KERNEL_PIPELINED : KERNEL_TWO_PHASE;
+  if (g.mode == GEMM_M_GROUPED) return KERNEL_ROWSPLIT;
+  return g.mode == GEMM_K_GROUPED || g.red >= 512 ? KERNEL_PIPELINED : KERNEL_TWO_PHASE;
 }
 
 // Problems too small for 256 x 256 tiles to fill 256 compute units evenly go to the kernel with one 64 x 128
