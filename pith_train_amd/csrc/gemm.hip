@@ -291,18 +291,22 @@ static int gemm_impl() {
 //              HBM (every group has its own b operand), and waves of a half-empty tile skip their
 //              MFMAs (us, against the software-pipelined loop: 32 groups of about 2048 rows, 5760 x
 //              2880 weights 1194 / 1250, of 1000 rows 602 / 645, 128 groups 873 / 880).
-//   k-grouped  the software-pipelined loop: both operands are shared by a whole group, there are no
-//              half-empty tiles, and one barrier per block counts for more (us, against the row-split
-//              loop: 32 groups of about 2048 rows 5760 x 2880 1165 / 1218, 64 Zipf-distributed groups
-//              of 768 in the mean 2816 x 2048 420 / 459 and 2048 x 1408 198 / 233, split reductions
-//              4096 x 2048 x 32768 240 / 253 and 2816 x 2048 x 8192 56 / 64; 128 groups of 512 level).
+//   k-grouped  the software-pipelined loop from 768 rows a group on and for split reductions: both
+//              operands are shared by a whole group, there are no half-empty tiles, and one barrier per
+//              block counts for more (us, against the row-split loop: 32 groups of about 2048 rows 5760 x
+//              2880 1165 / 1218, 64 Zipf-distributed groups of 768 in the mean 2816 x 2048 420 / 459 and
+//              2048 x 1408 198 / 233, split reductions 4096 x 2048 x 32768 240 / 253 and 2816 x 2048 x
+//              8192 56 / 64).  With fewer rows the stores weigh more and the row-split loop is level or
+//              ahead (inside a step, 128 Zipf-distributed groups of 420 in the mean 2048 x 512 208 / 223
+//              and 1024 x 2048 290 / 312).
 //   dense      the software-pipelined loop from K = 512 on (+5 % at 512, +13..20 % from 2048 on
 //              over the two-phase loop, +5..8 % over the row-split loop); below, the two-phase loop,
 //              which has no fill/drain of one 128-block per tile.
 enum { KERNEL_TWO_PHASE, KERNEL_PIPELINED, KERNEL_ROWSPLIT };
 static int preferred_kernel(const GemmArgs& g) {
   if (g.mode == GEMM_M_GROUPED) return KERNEL_ROWSPLIT;
-  return g.mode == GEMM_K_GROUPED || g.red >= 512 ? KERNEL_PIPELINED : KERNEL_TWO_PHASE;
+  if (g.mode == GEMM_K_GROUPED) return !g.offs || g.red >= 768 * (int64_t)g.G ? KERNEL_PIPELINED : KERNEL_ROWSPLIT;
+  return g.red >= 512 ? KERNEL_PIPELINED : KERNEL_TWO_PHASE;
 }
 
 // Problems too small for 256 x 256 tiles to fill 256 compute units evenly go to the kernel with one 64 x 128
@@ -310,12 +314,14 @@ static int preferred_kernel(const GemmArgs& g) {
 // when the persistent kernels are the better choice.  While all 64-row tiles run at once the smaller tile
 // wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 25.0 for the pipelined kernel).  Then both
 // kinds are priced in rounds of the GPU: a round of 256 large tiles is the unit, a round of 512 small ones
-// (a quarter of the area each, half of it in all) costs 0.57 of it in the m-grouped mode, 0.65 in
+// (a quarter of the area each, half of it in all) costs 0.57 of it in the m-grouped mode (0.68 with a
+// reduction-major b, whose fragments take twice the LDS reads), 0.65 in
 // the dense one, where the large tiles have the better loop (0.45 up to a reduction of 512, most of it
 // filling and draining), 0.43 for a weight gradient over groups of up to 1024 rows (mostly stores, which
 // one workgroup of a unit does while the other loads; longer ones are like dense products).  A partly filled round of small tiles costs half of what it leaves idle.  Us,
 // large / small: m-grouped, K 2048, N 1536: 16 groups of 256 rows 26.1 / 18.0, of 512 33.3 / 32.1, of 640
-// 60.4 / 36.4, of 1024 62.9 / 56.0; 64 groups of 128 51.5 / 40.7, of 384 90 / 85, of 512 105 / 115.  Dense
+// 60.4 / 36.4, of 1024 62.9 / 56.0; 64 groups of 128 51.5 / 40.7, of 384 90 / 85, of 512 105 / 115;
+// reduction-major b, K 1536, N 2048: 16 groups of 512 32.3 / 29.9, of 1024 54.5 / 57.3.  Dense
 // 4096 x 2048 x 2048 28.7 / 19.3, 4096 x 4096 x 2048 32.7 / 38.0.  Weight gradients 1536 x 2048 of 16
 // groups of 128 rows 28.2 / 23.1, of 1024 61.1 / 57.1; of 64 groups 73 / 83.  Past three to four rounds
 // large tiles have no round to waste and need half of the operand traffic.
@@ -323,18 +329,23 @@ static int small_tile_rows(const GemmArgs& g) {
   const int64_t groups = g.mode == GEMM_K_GROUPED ? g.G : 1;
   const int64_t cols = cdiv(g.rows_b, 128) * groups, cols_large = cdiv(g.rows_b, 256) * groups;
   if (cdiv(g.rows_a, 64) * cols <= 256) return 64;
-  const int64_t small = cdiv(g.rows_a, 128) * cols;
+  int64_t small = cdiv(g.rows_a, 128) * cols;
   if (small <= 512) return 128;
   int64_t rows_large = cdiv(g.rows_a, 256);
-  if (g.mode == GEMM_M_GROUPED) {  // half of the groups end in half a tile
+  if (g.mode == GEMM_M_GROUPED) {
+    // Half of the groups end in half a large tile.  The row count may be a capacity, which exceeds the real
+    // one by half a block per group in the mean, or exact: half of that is taken off.
     const int64_t blocks = g.rows_a / 128, least = blocks < g.G ? blocks : g.G;
     rows_large = (blocks + g.G / 2) / 2;
     if (rows_large < least) rows_large = least;
+    const int64_t fewer = blocks - g.G / 4;
+    small = (fewer > least ? fewer : least) * cols;
   }
   const int64_t large = rows_large * cols_large;
-  if (large > (g.mode == GEMM_K_GROUPED ? 1024 : 768)) return 0;
+  if (large > (g.mode == GEMM_K_GROUPED ? 1024 : g.b_kmajor ? 512 : 768)) return 0;
   const int64_t depth = g.mode == GEMM_K_GROUPED ? g.red / g.G : g.red;
-  const int64_t price = g.mode == GEMM_M_GROUPED ? 57 : g.mode == GEMM_K_GROUPED ? (depth <= 1024 ? 43 : 65) : depth <= 512 ? 45 : 65;
+  const int64_t price = g.mode == GEMM_M_GROUPED ? (g.b_kmajor ? 68 : 57)
+                        : g.mode == GEMM_K_GROUPED ? (depth <= 1024 ? 43 : 65) : depth <= 512 ? 45 : 65;
   // in units of 1 / (100 * 512 * 2) of a round of large tiles, five percent in favour of those
   return (small + cdiv(small, 512) * 512) * price * 105 < cdiv(large, 256) * (2 * 512 * 100) * 100 ? 128 : 0;
 }
