@@ -150,6 +150,10 @@ def host():
                 "`make -C pith_train_amd/csrc`"
             ) from exc
         module.init(LIB_PATH, PithTrainHipError)
+        from .dualpipe_utils import WeightGradStore
+        from .operators.grouped_linear import m_grouped_fp8_dgrad, schedule_wgrad
+
+        module.set_callbacks(WeightGradStore, schedule_wgrad, m_grouped_fp8_dgrad)
         _host = module
     return _host
 

@@ -1,13 +1,15 @@
-// Host side of the hot operators as a Python extension: allocations, argument blocks and the dense linear's
-// autograd node in C++, the kernels behind the C-ABI of libpithtrain_hip.so as everywhere else.
+// Host side of the hot operators as a Python extension: allocations, argument blocks and autograd nodes in C++, the kernels behind the C-ABI of libpithtrain_hip.so as everywhere else.
 //
 // Layers of a few thousand tokens are bound by what the host does per step.  Written in Python, preparing
 // the launches of an expert block's forward and backward took about 90 us and of a dense linear's 40 us,
 // on top of 3.5 us per launch in the runtime; torch's allocator alone costs 1.5 us per tensor from Python
-// and 0.7 us from here.
+// and 0.7 us from here, an autograd node written in Python 10 to 15 us a direction.
 //
 // No HIP header and no stream query here: the caller passes the stream it is on, and a backward runs on
 // the stream of its forward.
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/extension.h>
 
 #include <dlfcn.h>
@@ -43,6 +45,28 @@ struct Library {
   PT_FN(pt_linear_forward);
   PT_FN(pt_linear_backward_workspace_bytes);
   PT_FN(pt_linear_backward);
+  PT_FN(pt_gather_rows);
+  PT_FN(pt_gather_rows_backward_workspace_bytes);
+  PT_FN(pt_gather_rows_backward);
+  PT_FN(pt_permute_rows);
+  PT_FN(pt_silu_mul_fwd);
+  PT_FN(pt_silu_mul_bwd);
+  PT_FN(pt_moe_combine_fwd);
+  PT_FN(pt_moe_combine_bwd);
+  PT_FN(pt_moe_combine_ep_index);
+  PT_FN(pt_moe_combine_ep_fwd);
+  PT_FN(pt_moe_combine_ep_bwd);
+  PT_FN(pt_router_topk_fwd);
+  PT_FN(pt_router_topk_bwd);
+  PT_FN(pt_dedup_workspace_bytes);
+  PT_FN(pt_dedup_prepare_dispatch);
+  PT_FN(pt_build_expert_idxs);
+  PT_FN(pt_adjust_expand_idx);
+  PT_FN(pt_quant_rowwise_colwise);
+  PT_FN(pt_gemm_m_grouped_nt);
+  PT_FN(pt_gemm_m_grouped_nn);
+  PT_FN(pt_gemm_k_grouped_wgrad);
+  PT_FN(pt_sum_branches);
 #undef PT_FN
 } lib;
 
@@ -68,6 +92,28 @@ void init(const std::string& path) {
   PT_FN(pt_linear_forward);
   PT_FN(pt_linear_backward_workspace_bytes);
   PT_FN(pt_linear_backward);
+  PT_FN(pt_gather_rows);
+  PT_FN(pt_gather_rows_backward_workspace_bytes);
+  PT_FN(pt_gather_rows_backward);
+  PT_FN(pt_permute_rows);
+  PT_FN(pt_silu_mul_fwd);
+  PT_FN(pt_silu_mul_bwd);
+  PT_FN(pt_moe_combine_fwd);
+  PT_FN(pt_moe_combine_bwd);
+  PT_FN(pt_moe_combine_ep_index);
+  PT_FN(pt_moe_combine_ep_fwd);
+  PT_FN(pt_moe_combine_ep_bwd);
+  PT_FN(pt_router_topk_fwd);
+  PT_FN(pt_router_topk_bwd);
+  PT_FN(pt_dedup_workspace_bytes);
+  PT_FN(pt_dedup_prepare_dispatch);
+  PT_FN(pt_build_expert_idxs);
+  PT_FN(pt_adjust_expand_idx);
+  PT_FN(pt_quant_rowwise_colwise);
+  PT_FN(pt_gemm_m_grouped_nt);
+  PT_FN(pt_gemm_m_grouped_nn);
+  PT_FN(pt_gemm_k_grouped_wgrad);
+  PT_FN(pt_sum_branches);
 #undef PT_FN
 }
 
@@ -446,7 +492,561 @@ struct ExpertsBackward {
   }
 };
 
-PyObject* g_error = nullptr;
+// ---------------------------------------------------------------------------------------------------------
+// autograd nodes
+// ---------------------------------------------------------------------------------------------------------
+// Python objects the nodes call back into (never released: they live as long as the process)
+PyObject *g_error = nullptr, *g_store = nullptr, *g_schedule = nullptr, *g_dgrad = nullptr;
+
+struct HipNode : torch::autograd::Node {
+  pt_stream_t stream = nullptr;
+  bool released = false;
+  virtual variable_list run(variable_list&& grads) = 0;
+  virtual void drop() = 0;
+  variable_list apply(variable_list&& grads) override {
+    TORCH_CHECK(!released, "the saved tensors of ", name(), " are gone: a second backward needs retain_graph=True for the first one");
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return run(std::move(grads));
+  }
+  void release_variables() override {
+    released = true;
+    drop();
+  }
+};
+
+template <class N, class... Inputs>
+std::shared_ptr<N> make_node(int64_t stream, const Inputs&... inputs) {
+  std::shared_ptr<N> node(new N(), torch::autograd::deleteNode);
+  node->stream = (pt_stream_t)stream;
+  node->set_next_edges(torch::autograd::collect_next_edges(inputs...));
+  return node;
+}
+
+// Runs `compute` below autograd and, when one of the inputs wants a gradient, hangs its result (a fresh
+// tensor) on a node that `fill` completes.
+template <class N, class Compute, class Fill, class... Inputs>
+Tensor with_node(int64_t stream, Compute compute, Fill fill, const Inputs&... inputs) {
+  const bool wants = torch::autograd::compute_requires_grad(inputs...);
+  Tensor out;
+  {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    out = compute();
+  }
+  if (wants) {
+    auto node = make_node<N>(stream, inputs...);
+    fill(*node);
+    torch::autograd::set_history(out, node);
+  }
+  return out;
+}
+
+Tensor or_zeros(const Tensor& grad, at::IntArrayRef shape, at::ScalarType type, const at::Device& dev) {
+  return grad.defined() ? grad : at::zeros(shape, at::TensorOptions().dtype(type).device(dev));
+}
+
+bool deferred_gradients() {  // WeightGradStore.enabled; needs the GIL
+  return py::handle(g_store).attr("enabled").cast<bool>();
+}
+
+// ---- rows moved through an index --------------------------------------------------------------------------
+constexpr int64_t kRowAlignment = 1024;
+
+Tensor gather_into(const Tensor& src, const Tensor& index, const Tensor& out, pt_stream_t stream) {
+  const int64_t n = index.size(0);
+  if (n > 0 && src.size(1) > 0)
+    check(lib.pt_gather_rows(ptr(src), src.stride(0), ptr(out), out.stride(0), (const int64_t*)ptr(index), n, src.size(1), (int32_t)src.element_size(),
+                             stream), "pt_gather_rows");
+  return out;
+}
+
+// Sum of the rows of `grad` that share an index, in a buffer of whole 1024 rows.
+Tensor scatter_sum(const Tensor& grad, const Tensor& index, int64_t rows, int64_t alignment, int64_t stream) {
+  std::vector<int64_t> shape = grad.sizes().vec();
+  shape[0] = cdiv(rows, alignment) * alignment;
+  Tensor out = empty(shape, grad.scalar_type(), grad.device());
+  const int64_t n = index.size(0);
+  int64_t H = 1;
+  for (size_t i = 1; i < shape.size(); ++i) H *= shape[i];
+  if (rows && H) {
+    const Tensor go = grad.contiguous(), idx = index.contiguous();
+    const int64_t bytes = lib.pt_gather_rows_backward_workspace_bytes(n, rows);
+    Tensor ws = empty({std::max<int64_t>(bytes, 256)}, at::kByte, grad.device());
+    check(lib.pt_gather_rows_backward(ptr(go), H, ptr(out), H, (const int64_t*)ptr(idx), n, rows, H, dtype_code(grad.scalar_type()), ptr(ws),
+                                      ws.numel(), (pt_stream_t)stream), "pt_gather_rows_backward");
+  }
+  return out.narrow(0, 0, rows);
+}
+
+struct GatherNode : HipNode {
+  Tensor index;
+  int64_t rows, alignment;
+  void drop() override { index.reset(); }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor()};
+    return {scatter_sum(g[0], index, rows, alignment, (int64_t)stream)};
+  }
+};
+
+Tensor index_gather(const Tensor& input, const Tensor& index, int64_t alignment, int64_t stream) {
+  require_cuda(input);
+  require_cuda(index);
+  return with_node<GatherNode>(
+      stream,
+      [&] {
+        const int64_t n = index.size(0);
+        std::vector<int64_t> shape = input.sizes().vec();
+        shape[0] = cdiv(n, alignment) * alignment;
+        Tensor buf = empty(shape, input.scalar_type(), input.device());
+        Tensor out = buf.narrow(0, 0, n);
+        if (n) {
+          const Tensor src = row_major(input.reshape({input.size(0), -1}));
+          gather_into(src, index.contiguous(), out.view({n, -1}), (pt_stream_t)stream);
+        }
+        return out;
+      },
+      [&](GatherNode& node) {
+        node.index = index;
+        node.rows = input.size(0);
+        node.alignment = alignment;
+      },
+      input);
+}
+
+// Rows grouped by expert (ScatterForGroupedGemm): the caller sorted the indices; backward: gather.
+struct PermuteNode : HipNode {
+  Tensor reverse;
+  Maybe pre;
+  int64_t in_rows;
+  void drop() override { reverse.reset(); pre.reset(); }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor()};
+    const Tensor go = g[0].contiguous();
+    Tensor grad = gather_into(go, reverse, empty({reverse.size(0), go.size(1)}, go.scalar_type(), go.device()), stream);
+    return {pre ? scatter_sum(grad, *pre, in_rows, kRowAlignment, (int64_t)stream) : grad};
+  }
+};
+
+Tensor permute_rows(const Tensor& input, const Tensor& src_of, const Tensor& offs, const Tensor& reverse, const Maybe& pre, const Tensor& buffer,
+                    int64_t rows, int64_t stream) {
+  return with_node<PermuteNode>(
+      stream, [&] { return buffer.narrow(0, 0, rows); },
+      [&](PermuteNode& node) {
+        node.reverse = reverse;
+        node.pre = pre;
+        node.in_rows = input.size(0);
+      },
+      input);
+}
+// The row copy itself, queued before the caller waits for the group sizes.
+Tensor permute_into_buffer(const Tensor& input, const Tensor& src_of, const Tensor& offs, const Maybe& pre, int64_t stream) {
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor in = row_major(input);
+  Tensor buf = empty({src_of.size(0), in.size(1)}, in.scalar_type(), in.device());
+  check(lib.pt_permute_rows(ptr(in), in.stride(0), ptr(buf), buf.stride(0), (const int32_t*)ptr(src_of), (const int64_t*)ptr(pre),
+                            (const int32_t*)ptr(offs) + offs.size(0) - 1, (int32_t)kRowAlignment, buf.size(0), in.size(1), (int32_t)in.element_size(),
+                            (pt_stream_t)stream), "pt_permute_rows");
+  return buf;
+}
+
+// ---- SwiGLU -----------------------------------------------------------------------------------------------
+struct SiluMulNode : HipNode {
+  torch::autograd::SavedVariable gate, up;
+  void drop() override { gate.reset_data(); up.reset_data(); }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor()};
+    const Tensor a = gate.unpack(), b = up.unpack();
+    TORCH_CHECK(g[0].sizes() == a.sizes(), "grad_output shape ", g[0].sizes(), " != gate shape ", a.sizes());
+    TORCH_CHECK(g[0].scalar_type() == a.scalar_type(), "grad_output dtype differs from gate's");
+    TORCH_CHECK(g[0].is_contiguous(), "grad_output must be contiguous");
+    Tensor da = empty(a.sizes(), a.scalar_type(), a.device()), db = empty(a.sizes(), a.scalar_type(), a.device());
+    check(lib.pt_silu_mul_bwd(ptr(g[0]), ptr(a), ptr(b), ptr(da), ptr(db), a.numel(), dtype_code(a.scalar_type()), stream), "pt_silu_mul_bwd");
+    return {da, db};
+  }
+};
+
+Tensor silu_mul(const Tensor& gate, const Tensor& up, int64_t stream) {
+  require_cuda(gate);
+  require_cuda(up);
+  return with_node<SiluMulNode>(
+      stream,
+      [&] {
+        Tensor out = empty(gate.sizes(), gate.scalar_type(), gate.device());
+        check(lib.pt_silu_mul_fwd(ptr(gate), ptr(up), ptr(out), gate.numel(), dtype_code(gate.scalar_type()), (pt_stream_t)stream), "pt_silu_mul_fwd");
+        return out;
+      },
+      [&](SiluMulNode& node) {
+        node.gate = torch::autograd::SavedVariable(gate, false);
+        node.up = torch::autograd::SavedVariable(up, false);
+      },
+      gate, up);
+}
+
+// ---- grouped linear ---------------------------------------------------------------------------------------
+// Row- and column-scaled FP8 forms of x [M, N], M % 128 == 0: bytes, scales, transposed bytes, their scales
+struct Quantised {
+  Tensor q, s, q_t, s_t;
+  Quantised() = default;
+  Quantised(const Tensor& input, pt_stream_t stream) {
+    const Tensor x = row_major(input);
+    const int64_t M = x.size(0), N = x.size(1);
+    const auto dev = x.device();
+    q = empty({M, N}, kFp8, dev);
+    s = empty({M, cdiv(N, 128)}, at::kFloat, dev);
+    q_t = empty({N, M}, kFp8, dev);
+    s_t = empty({M / 128, N}, at::kFloat, dev);
+    lib.pt_observe("pt_quant_rowwise_colwise", 1, M, N, M);
+    check(lib.pt_quant_rowwise_colwise(ptr(x), dtype_code(x.scalar_type()), M, N, M > 1 ? x.stride(0) : N, ptr(q), (float*)ptr(s), ptr(q_t),
+                                       (float*)ptr(s_t), PT_CH_TRANSPOSED, nullptr, 0, stream), "pt_quant_rowwise_colwise");
+    lib.pt_observe("pt_quant_rowwise_colwise", 0, M, N, M);
+  }
+};
+
+struct GroupedLinearNode : HipNode {
+  Tensor weight, dg, dg_s, offs, x_t, x_ts;
+  bool forward_layout;
+  void drop() override { dg.reset(); dg_s.reset(); offs.reset(); x_t.reset(); x_ts.reset(); }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor()};
+    const Tensor go = g[0].contiguous();
+    const int64_t M = go.size(0), N = go.size(1), K = x_t.size(0), G = offs.size(0);
+    Quantised d(go, stream);
+    Tensor gx = empty({M, K}, go.scalar_type(), go.device());
+    const auto o = (const int32_t*)ptr(offs);
+    const char* what = forward_layout ? "pt_gemm_m_grouped_nn" : "pt_gemm_m_grouped_nt";
+    lib.pt_observe(what, 1, M, K, N);
+    check((forward_layout ? lib.pt_gemm_m_grouped_nn : lib.pt_gemm_m_grouped_nt)(ptr(d.q), (const float*)ptr(d.s), ptr(dg), (const float*)ptr(dg_s), ptr(gx),
+                                                                                 dtype_code(gx.scalar_type()), o, (int32_t)G, M, K, N, stream), what);
+    lib.pt_observe(what, 0, M, K, N);
+    {
+      py::gil_scoped_acquire gil;
+      if (deferred_gradients()) {
+        const py::handle schedule(g_schedule);
+        schedule(weight, py::make_tuple(d.q_t, d.s_t), py::make_tuple(x_t, x_ts), offs);
+        return {gx, Tensor()};
+      }
+    }
+    Target t;
+    t.aim(weight);
+    lib.pt_observe("pt_gemm_k_grouped_wgrad", 1, M, N, K);
+    check(lib.pt_gemm_k_grouped_wgrad(ptr(d.q_t), (const float*)ptr(d.s_t), ptr(x_t), (const float*)ptr(x_ts), t.at(), PT_BF16, t.add, o, (int32_t)G, M, N,
+                                      K, stream), "pt_gemm_k_grouped_wgrad");
+    lib.pt_observe("pt_gemm_k_grouped_wgrad", 0, M, N, K);
+    t.finish();
+    return {gx, Tensor()};  // the weight's gradient went to .grad
+  }
+};
+
+Tensor grouped_linear(const Tensor& x, const Tensor& weight, const Tensor& offs, const Tensor& w, const Tensor& w_s, const Tensor& dg, const Tensor& dg_s,
+                      bool forward_layout, int64_t stream) {
+  require_cuda(x);
+  Quantised q;
+  return with_node<GroupedLinearNode>(
+      stream,
+      [&] {
+        q = Quantised(x, (pt_stream_t)stream);
+        const int64_t M = x.size(0), K = x.size(1), N = w.size(1), G = w.size(0);
+        Tensor y = empty({M, N}, x.scalar_type(), x.device());
+        lib.pt_observe("pt_gemm_m_grouped_nt", 1, M, N, K);
+        check(lib.pt_gemm_m_grouped_nt(ptr(q.q), (const float*)ptr(q.s), ptr(w), (const float*)ptr(w_s), ptr(y), dtype_code(y.scalar_type()),
+                                       (const int32_t*)ptr(offs), (int32_t)G, M, N, K, (pt_stream_t)stream), "pt_gemm_m_grouped_nt");
+        lib.pt_observe("pt_gemm_m_grouped_nt", 0, M, N, K);
+        return y;
+      },
+      [&](GroupedLinearNode& node) {
+        node.weight = weight; node.dg = dg; node.dg_s = dg_s; node.offs = offs;
+        node.x_t = q.q_t; node.x_ts = q.s_t; node.forward_layout = forward_layout;
+      },
+      x, weight);
+}
+
+// ---- expert block -----------------------------------------------------------------------------------------
+struct ExpertsNode : HipNode {
+  Dims d;
+  Tensor w_gate, w_up, w_down;  // w_gate: the fused gate_up weight when w_up is not there
+  Tensor gu_dg, gu_dg_s, dn_dg, dn_dg_s, offs, gate_up;
+  Maybe row_map, expand_idx, gu_bias, dn_bias;
+  std::vector<Tensor> kept;
+  bool gu_forward, dn_forward, scatter, clamped;
+  double alpha, limit;
+  int64_t src_rows, routed, repeat;
+  void drop() override {
+    for (Tensor* t : {&gu_dg, &gu_dg_s, &dn_dg, &dn_dg_s, &offs, &gate_up}) t->reset();
+    row_map.reset(); expand_idx.reset();
+    kept.clear();
+  }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    bool deferred;
+    {
+      py::gil_scoped_acquire gil;
+      deferred = deferred_gradients();
+    }
+    std::vector<Tensor> weights;
+    if (!deferred) {
+      weights = {w_down, w_gate};
+      if (w_up.defined()) weights.push_back(w_up);
+    }
+    ExpertsBackward step(g[0], d, offs, row_map, scatter, dn_dg, dn_dg_s, dn_forward, gate_up, kept, clamped, alpha, limit, gu_bias, dn_bias, weights,
+                         (int64_t)stream);
+    Tensor gx = empty({row_map ? routed : d.M, d.K}, g[0].scalar_type(), g[0].device());
+    {
+      py::gil_scoped_acquire gil;
+      const py::handle dgrad(g_dgrad);
+      dgrad(py::make_tuple(step.dgu, step.dgu_s), gu_dg, gu_dg_s, gu_forward, gx, offs, row_map);
+      if (deferred) {
+        const auto op = step.operands();
+        auto pair = [](const std::pair<Tensor, Tensor>& p) { return py::make_tuple(p.first, p.second); };
+        py::handle schedule(g_schedule);
+        schedule(w_down, pair(op[0]), pair(op[3]), offs);
+        if (w_up.defined()) {
+          const Tensor &q = op[1].first, &sc = op[1].second;
+          schedule(w_gate, py::make_tuple(q.narrow(0, 0, d.half), sc.narrow(1, 0, d.half)), pair(op[2]), offs);
+          schedule(w_up, py::make_tuple(q.narrow(0, d.half, d.half), sc.narrow(1, d.half, d.half)), pair(op[2]), offs);
+        } else {
+          schedule(w_gate, pair(op[1]), pair(op[2]), offs);
+        }
+      }
+    }
+    if (!deferred) step.weight_gradient();
+    // rows that expand the same source row are summed (the backward of the expanding gather)
+    if (expand_idx) gx = scatter_sum(gx, *expand_idx, src_rows, kRowAlignment, (int64_t)stream);
+    if (repeat > 1) gx = gx.view({src_rows, repeat, d.K});
+    return {gx, Tensor(), Tensor(), Tensor(), step.d_gu_bias.value_or(Tensor()), step.d_dn_bias.value_or(Tensor())};
+  }
+};
+
+// (fp8, scale) of the forward operand and (fp8, scale, forward_layout) of the input gradient's
+typedef std::tuple<Tensor, Tensor> Operand;
+typedef std::tuple<Tensor, Tensor, bool> DgradOperand;
+
+Tensor experts(const Tensor& input, const Tensor& w_gate, const Maybe& w_up, const Tensor& w_down, const Maybe& gu_bias, const Maybe& dn_bias,
+               const Tensor& offs, const Operand& gu, const Operand& dn, const DgradOperand& gu_dg, const DgradOperand& dn_dg, const Maybe& row_map,
+               const Maybe& expand_idx, bool scatter, std::optional<std::pair<double, double>> clamp, int64_t stream) {
+  require_cuda(input);
+  const Tensor up = w_up.value_or(Tensor()), b0 = gu_bias.value_or(Tensor()), b1 = dn_bias.value_or(Tensor());
+  std::tuple<Tensor, Tensor, std::vector<Tensor>> done;
+  Tensor x;
+  int64_t repeat = 1;
+  const auto [alpha, limit] = clamp.value_or(std::pair<double, double>{0.0, 0.0});
+  return with_node<ExpertsNode>(
+      stream,
+      [&] {
+        x = input;
+        if (x.dim() == 3) {
+          repeat = x.size(1);
+          x = x.select(1, 0);
+        }
+        x = row_major(x);
+        Maybe c0, c1;
+        if (gu_bias) c0 = gu_bias->contiguous();
+        if (dn_bias) c1 = dn_bias->contiguous();
+        done = experts_forward(x, repeat, row_map, expand_idx, offs, std::get<0>(gu), std::get<1>(gu), std::get<0>(dn), std::get<1>(dn), w_down.size(2), c0,
+                               c1, scatter, (bool)clamp, alpha, limit, true, false, stream);
+        return std::get<0>(done);
+      },
+      [&](ExpertsNode& n) {
+        n.src_rows = x.size(0);
+        n.repeat = repeat;
+        n.routed = expand_idx ? expand_idx->size(0) : n.src_rows * repeat;
+        n.d = Dims{row_map ? row_map->size(0) : n.src_rows, x.size(1), w_down.size(2), w_down.size(1), w_down.size(0)};
+        n.w_gate = w_gate; n.w_up = up; n.w_down = w_down;
+        std::tie(n.gu_dg, n.gu_dg_s, n.gu_forward) = gu_dg;
+        std::tie(n.dn_dg, n.dn_dg_s, n.dn_forward) = dn_dg;
+        n.offs = offs; n.gate_up = std::get<1>(done); n.kept = std::get<2>(done);
+        n.row_map = row_map; n.expand_idx = expand_idx; n.gu_bias = gu_bias; n.dn_bias = dn_bias;
+        n.scatter = scatter; n.clamped = (bool)clamp; n.alpha = alpha; n.limit = limit;
+      },
+      input, w_gate, up, w_down, b0, b1);
+}
+
+// ---- combine ----------------------------------------------------------------------------------------------
+struct CombineNode : HipNode {
+  Tensor moe, w;
+  bool residual;
+  void drop() override { moe.reset(); w.reset(); }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    const int64_t T = w.size(0), k = w.size(1), H = moe.size(1);
+    const Tensor go = g[0].reshape({T, H}).contiguous();
+    Tensor dm = empty(moe.sizes(), moe.scalar_type(), moe.device()), dw = empty({T, k}, at::kFloat, moe.device());
+    check(lib.pt_moe_combine_bwd(ptr(go), H, ptr(moe), H, (const float*)ptr(w), ptr(dm), H, (float*)ptr(dw), T, (int32_t)k, H,
+                                 dtype_code(moe.scalar_type()), stream), "pt_moe_combine_bwd");
+    return {dm, dw, residual ? g[0] : Tensor()};
+  }
+};
+
+Tensor combine(const Tensor& outs, const Tensor& weight, const Maybe& residual, int64_t stream) {
+  const int64_t T = weight.size(0), k = weight.size(1), H = outs.size(1);
+  Tensor moe, w;
+  const Tensor res = residual.value_or(Tensor());
+  return with_node<CombineNode>(
+      stream,
+      [&] {
+        moe = outs.contiguous();
+        w = weight.contiguous();
+        Tensor r;
+        if (residual) r = res.reshape({T, H}).contiguous();
+        Tensor out = empty({T, H}, moe.scalar_type(), moe.device());
+        check(lib.pt_moe_combine_fwd(ptr(moe), H, (const float*)ptr(w), residual ? ptr(r) : nullptr, H, ptr(out), H, T, (int32_t)k, H,
+                                     dtype_code(moe.scalar_type()), (pt_stream_t)stream), "pt_moe_combine_fwd");
+        return residual ? out.view(res.sizes()) : out;
+      },
+      [&](CombineNode& n) { n.moe = moe.detach(); n.w = w.detach(); n.residual = (bool)residual; }, outs, weight, res);
+}
+
+struct CombineEpNode : HipNode {
+  Tensor moe, w, slots;
+  void drop() override { moe.reset(); w.reset(); slots.reset(); }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    const int64_t T = w.size(0), k = w.size(1), R = moe.size(0), H = moe.size(1);
+    const Tensor go = g[0].reshape({T, H}).contiguous();
+    // rows no slot points to (none when the indices are a permutation) get a zero gradient
+    Tensor dm = R == T * k ? empty(moe.sizes(), moe.scalar_type(), moe.device()) : at::zeros_like(moe);
+    Tensor dw = empty({T, k}, at::kFloat, moe.device());
+    check(lib.pt_moe_combine_ep_bwd(ptr(go), H, ptr(moe), H, R, (const int32_t*)ptr(slots), (const float*)ptr(w), ptr(dm), H, (float*)ptr(dw), T,
+                                    (int32_t)k, H, dtype_code(moe.scalar_type()), stream), "pt_moe_combine_ep_bwd");
+    return {dm, dw, g[0]};
+  }
+};
+
+Tensor combine_ep(const Tensor& outs, const Tensor& local_idxs, const Tensor& weight, const Tensor& residual, int64_t stream) {
+  const int64_t T = weight.size(0), k = weight.size(1), R = outs.size(0), H = outs.size(1);
+  const auto st = (pt_stream_t)stream;
+  Tensor moe, w, slots;
+  return with_node<CombineEpNode>(
+      stream,
+      [&] {
+        moe = outs.contiguous();
+        w = weight.contiguous();
+        const Tensor r = residual.reshape({T, H}).contiguous(), idx = local_idxs.contiguous();
+        slots = empty({T * k}, at::kInt, moe.device());
+        check(lib.pt_moe_combine_ep_index((const int64_t*)ptr(idx), R, T * k, (int32_t*)ptr(slots), st), "pt_moe_combine_ep_index");
+        Tensor out = empty({T, H}, moe.scalar_type(), moe.device());
+        check(lib.pt_moe_combine_ep_fwd(ptr(moe), H, R, (const int32_t*)ptr(slots), (const float*)ptr(w), ptr(r), H, ptr(out), H, T, (int32_t)k, H,
+                                        dtype_code(moe.scalar_type()), st), "pt_moe_combine_ep_fwd");
+        return out.view(residual.sizes());
+      },
+      [&](CombineEpNode& n) { n.moe = moe.detach(); n.w = w.detach(); n.slots = slots; }, outs, weight, residual);
+}
+
+// ---- a MoE block's branches (see moe_combine.token_branches) ------------------------------------------------
+struct BranchesNode : HipNode {
+  int64_t T, H;
+  void drop() override {}
+  variable_list run(variable_list&& g) override {
+    std::vector<Tensor> given;
+    bool same = H % 8 == 0 && g.size() <= 4;
+    for (const Tensor& t : g)
+      if (t.defined()) {
+        given.push_back(t);
+        same = same && t.scalar_type() == given[0].scalar_type();
+      }
+    if (given.empty()) return {Tensor()};
+    const bool rows = g[0].defined();
+    if (!same) {
+      Tensor total = rows ? g[0].sum(1) : Tensor();
+      for (size_t i = 1; i < g.size(); ++i)
+        if (g[i].defined()) total = total.defined() ? total + g[i] : g[i];
+      return {total};
+    }
+    for (Tensor& t : given) t = t.contiguous();
+    const void* at[3] = {};
+    for (size_t i = rows, n = 0; i < given.size(); ++i) at[n++] = ptr(given[i]);
+    Tensor out = empty({T, H}, given[0].scalar_type(), given[0].device());
+    check(lib.pt_sum_branches(rows ? ptr(given[0]) : nullptr, rows ? (int32_t)given[0].size(1) : 0, at[0], at[1], at[2], ptr(out), T, H,
+                              dtype_code(out.scalar_type()), stream), "pt_sum_branches");
+    return {out};
+  }
+};
+
+variable_list branches(const Tensor& x, int64_t k, int64_t n, int64_t stream) {
+  variable_list out;
+  {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    const Tensor base = x.detach();
+    out.push_back(base.unsqueeze(1).expand({-1, k, -1}));
+    for (int64_t i = 0; i < n; ++i) out.push_back(x.detach());
+  }
+  auto node = make_node<BranchesNode>(stream, x);
+  node->T = x.size(0);
+  node->H = x.size(1);
+  for (Tensor& t : out) torch::autograd::set_history(t, node);
+  return out;
+}
+
+// ---- router gate ------------------------------------------------------------------------------------------
+struct RouterNode : HipNode {
+  Tensor logits, idx;
+  int64_t mode, k, norm, num_group, topk_group;
+  double scale;
+  void drop() override { logits.reset(); idx.reset(); }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor()};
+    const int64_t T = logits.size(0), E = logits.size(1);
+    const Tensor dw = g[0].to(at::kFloat).contiguous();
+    Tensor d = empty({T, E}, logits.scalar_type(), logits.device());
+    check(lib.pt_router_topk_bwd(ptr(logits), logits.stride(0), dtype_code(logits.scalar_type()), T, (int32_t)E, (int32_t)k, (int)mode, (int)norm,
+                                 (float)scale, (int32_t)num_group, (int32_t)topk_group, (const int64_t*)ptr(idx), (const float*)ptr(dw), nullptr, ptr(d), E,
+                                 stream), "pt_router_topk_bwd");
+    return {d};
+  }
+};
+
+// (topk_idx, topk_weight), without forced choices and without the scores
+std::pair<Tensor, Tensor> router_topk(const Tensor& input, int64_t mode, int64_t k, bool norm, double scale, int64_t num_group, int64_t topk_group,
+                                      int64_t stream) {
+  require_cuda(input);
+  Tensor logits, idx;
+  Tensor weight = with_node<RouterNode>(
+      stream,
+      [&] {
+        logits = row_major(input);
+        const int64_t T = logits.size(0), E = logits.size(1);
+        idx = empty({T, k}, at::kLong, logits.device());
+        Tensor w = empty({T, k}, at::kFloat, logits.device());
+        check(lib.pt_router_topk_fwd(ptr(logits), logits.stride(0), dtype_code(logits.scalar_type()), T, (int32_t)E, (int32_t)k, (int)mode, (int)norm,
+                                     (float)scale, (int32_t)num_group, (int32_t)topk_group, nullptr, (int64_t*)ptr(idx), (float*)ptr(w), nullptr,
+                                     (pt_stream_t)stream), "pt_router_topk_fwd");
+        return w;
+      },
+      [&](RouterNode& n) {
+        n.logits = logits.detach(); n.idx = idx;
+        n.mode = mode; n.k = k; n.norm = norm; n.scale = scale; n.num_group = num_group; n.topk_group = topk_group;
+      },
+      input);
+  return {idx, weight};
+}
+
+// ---- dispatch of an expert-parallel rank --------------------------------------------------------------------
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> dedup_prepare_dispatch(const Tensor& ids, int64_t E, int64_t ep, int64_t epr, int64_t stream) {
+  const int64_t m = ids.size(0), k = ids.size(1);
+  const auto dev = ids.device();
+  auto i64 = [&](int64_t n) { return empty({n}, at::kLong, dev); };
+  Tensor per_rank = i64(ep), unique = i64(ep), dispatch = i64(m * ep), idxs = i64(m * k), expand = i64(m * k), meta = i64(ep * (epr + 1));
+  Tensor ws = empty({std::max<int64_t>(lib.pt_dedup_workspace_bytes(m, (int32_t)k, (int32_t)E, (int32_t)ep), 256)}, at::kByte, dev);
+  auto p = [](const Tensor& t) { return (int64_t*)ptr(t); };
+  check(lib.pt_dedup_prepare_dispatch(p(ids), ids.stride(0), m, (int32_t)k, (int32_t)E, (int32_t)ep, (int32_t)epr, p(per_rank), p(unique), p(dispatch),
+                                      p(idxs), p(expand), p(meta), ptr(ws), ws.numel(), (pt_stream_t)stream), "pt_dedup_prepare_dispatch");
+  return {per_rank, unique, dispatch, idxs, expand, meta};
+}
+
+std::pair<Tensor, Tensor> build_expert_idxs(const Tensor& counts, int64_t ep, int64_t epr, int64_t max_total, int64_t stream) {
+  const Tensor c = counts.to(at::kLong).contiguous();
+  Tensor idxs = empty({max_total}, at::kLong, c.device()), splits = empty({ep}, at::kLong, c.device());
+  check(lib.pt_build_expert_idxs((const int64_t*)ptr(c), (int32_t)c.size(0), (int32_t)ep, (int32_t)epr, max_total, max_total ? (int64_t*)ptr(idxs) : nullptr,
+                                 (int64_t*)ptr(splits), (pt_stream_t)stream), "pt_build_expert_idxs");
+  return {idxs, splits};
+}
+
+Tensor adjust_expand_idx(const Tensor& received, const Tensor& dedup, const Tensor& splits, int64_t stream) {
+  const Tensor r = received.contiguous(), sp = splits.contiguous();
+  Tensor out = empty(r.sizes(), at::kLong, r.device());
+  if (r.size(0))
+    check(lib.pt_adjust_expand_idx((const int64_t*)ptr(r), (int64_t*)ptr(out), (const int64_t*)ptr(dedup), dedup.stride(0), (const int64_t*)ptr(sp),
+                                   (int32_t)dedup.size(0), r.size(0), (pt_stream_t)stream), "pt_adjust_expand_idx");
+  return out;
+}
 
 }  // namespace
 
@@ -462,6 +1062,25 @@ PYBIND11_MODULE(_host, m) {
     g_error = error.release().ptr();
     init(path);
   });
+  m.def("set_callbacks", [](py::object store, py::object schedule, py::object dgrad) {
+    g_store = store.release().ptr();
+    g_schedule = schedule.release().ptr();
+    g_dgrad = dgrad.release().ptr();
+  });
+  m.def("index_gather", &index_gather);
+  m.def("scatter_sum", &scatter_sum);
+  m.def("permute_into_buffer", &permute_into_buffer);
+  m.def("permute_rows", &permute_rows);
+  m.def("silu_mul", &silu_mul);
+  m.def("grouped_linear", &grouped_linear);
+  m.def("experts", &experts);
+  m.def("combine", &combine);
+  m.def("combine_ep", &combine_ep);
+  m.def("branches", &branches);
+  m.def("router_topk", &router_topk);
+  m.def("dedup_prepare_dispatch", &dedup_prepare_dispatch);
+  m.def("build_expert_idxs", &build_expert_idxs);
+  m.def("adjust_expand_idx", &adjust_expand_idx);
   m.def("split_k", &split_k);
   m.def("quant_weight", &quant_weight);
   m.def("quant_grouped_weights", &quant_grouped_weights);
@@ -470,19 +1089,4 @@ PYBIND11_MODULE(_host, m) {
   m.def("linear_heads_backward", &linear_heads_backward);
   m.def("group_rows", &group_rows);
   m.def("experts_forward", &experts_forward);
-  py::class_<ExpertsBackward>(m, "ExpertsBackward")
-      .def(py::init([](const Tensor& grad, std::tuple<int64_t, int64_t, int64_t, int64_t, int64_t> dims, const Tensor& offs, const Maybe& row_map,
-                       bool scatter, const Tensor& dn_dg, const Tensor& dn_dg_s, bool dn_forward, const Tensor& gate_up, std::vector<Tensor> kept,
-                       bool clamped, double alpha, double limit, const Maybe& gu_bias_like, const Maybe& dn_bias_like,
-                       const std::vector<Tensor>& weights, int64_t stream) {
-        const auto [M, K, half, H, G] = dims;
-        return std::make_unique<ExpertsBackward>(grad, Dims{M, K, half, H, G}, offs, row_map, scatter, dn_dg, dn_dg_s, dn_forward, gate_up,
-                                                 std::move(kept), clamped, alpha, limit, gu_bias_like, dn_bias_like, weights, stream);
-      }))
-      .def("weight_gradient", &ExpertsBackward::weight_gradient)
-      .def("operands", &ExpertsBackward::operands)
-      .def_readonly("dgu", &ExpertsBackward::dgu)
-      .def_readonly("dgu_s", &ExpertsBackward::dgu_s)
-      .def_readonly("d_gu_bias", &ExpertsBackward::d_gu_bias)
-      .def_readonly("d_dn_bias", &ExpertsBackward::d_dn_bias);
 }

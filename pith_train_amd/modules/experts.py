@@ -111,7 +111,7 @@ class Qwen3MoeExperts(nn.Module):
         if fuse_activation and x.shape[0] > 0 and self.one_node(x):
             gate, up, down = map(_weight, self._projections())
             if not fused_experts.wants_backward(x, gate, up, down):
-                return fused_experts.forward_only(x, (gate, up), down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
+                return fused_experts.forward_only(x, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
                                                   few_rows=few_rows)  # fmt: skip
             return fused_experts.FP8SwiGLUSplitExpertsFunc.apply(
                 x, gate, up, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
@@ -185,7 +185,7 @@ class Qwen35MoeExperts(nn.Module):
         if fuse_activation and x.shape[0] > 0 and self.one_node(x):
             gate_up, down = _weight(self._modules["gate_up_proj"]), _weight(self._modules["down_proj"])
             if not fused_experts.wants_backward(x, gate_up, down):
-                return fused_experts.forward_only(x, gate_up, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
+                return fused_experts.forward_only(x, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
                                                   few_rows=few_rows)  # fmt: skip
             return fused_experts.FP8SwiGLUExpertsFunc.apply(
                 x, gate_up, down, grouped_mm_offs, ks, ks_tensor,
@@ -280,7 +280,7 @@ class GptOssExperts(nn.Module):
         assert not scatter_output or (fused and row_map is not None), "scatter_output needs row_map and the fused biases"
         if M % 128 == 0 and self.one_node(x) and not fused_experts.wants_backward(x, *self._parameters.values()):
             return fused_experts.forward_only(
-                x, self.gate_up_proj, self.down_proj, grouped_mm_offs, *self._quantized_weights(), row_map, None, scatter_output,
+                x, self.down_proj, grouped_mm_offs, *self._quantized_weights(), row_map, None, scatter_output,
                 (1.702, self.swiglu_limit), (self.gate_up_proj_bias, self.down_proj_bias), few_rows,
             )
         if M % 128 == 0 and self.one_node(x):

@@ -18,7 +18,7 @@ from typing import List, NamedTuple, Optional
 import torch
 
 from .. import _lib
-from .token_scatter import _workspace, get_pinned_buffer, padded_index_gather
+from .token_scatter import get_pinned_buffer, padded_index_gather
 
 
 class AllToAllSplits(NamedTuple):
@@ -58,53 +58,22 @@ def fused_dedup_prepare_dispatch(topk_ids: torch.Tensor, num_experts: int, ep_si
     assert topk_ids.dtype == torch.int64
     if topk_ids.stride(1) != 1:
         topk_ids = topk_ids.contiguous()
-    tokens_per_ep_rank = torch.empty(ep_size, **i64)
-    dedup_tokens_per_gpu = torch.empty(ep_size, **i64)
-    dispatch_token_idxs = torch.empty(m * ep_size, **i64)
-    idxs = torch.empty(m * k, **i64)
-    expand_idx = torch.empty(m * k, **i64)
-    send_meta = torch.empty(ep_size * (experts_per_rank + 1), **i64)
-    ws = _workspace(_lib.query("pt_dedup_workspace_bytes", m, k, num_experts, ep_size), device)
-    _lib.call(
-        "pt_dedup_prepare_dispatch", topk_ids.data_ptr(), topk_ids.stride(0), m, k, num_experts,
-        ep_size, experts_per_rank, tokens_per_ep_rank.data_ptr(), dedup_tokens_per_gpu.data_ptr(),
-        dispatch_token_idxs.data_ptr(), idxs.data_ptr(), expand_idx.data_ptr(), send_meta.data_ptr(),
-        ws.data_ptr(), ws.numel(), _lib.stream_ptr(device),
-    )  # fmt: skip
-    return tokens_per_ep_rank, dedup_tokens_per_gpu, dispatch_token_idxs, idxs, expand_idx, send_meta
+    return _lib.host().dedup_prepare_dispatch(topk_ids, num_experts, ep_size, experts_per_rank, _lib.stream_ptr(device))
 
 
 def build_expert_idxs(tokens_per_expert_group: torch.Tensor, ep_size: int, experts_per_rank: int, max_total: int):
     """(expert_idxs[max_total] over-allocated, output_splits[ep]); the caller trims expert_idxs to
     ``sum(output_splits)``."""
     _lib.require_cuda(tokens_per_expert_group)
-    num_experts = tokens_per_expert_group.shape[0]
-    device = tokens_per_expert_group.device
-    expert_idxs = torch.empty(max_total, dtype=torch.int64, device=device)
-    output_splits = torch.empty(ep_size, dtype=torch.int64, device=device)
-    counts = tokens_per_expert_group.to(torch.int64).contiguous()
-    _lib.call(
-        "pt_build_expert_idxs", counts.data_ptr(), num_experts, ep_size, experts_per_rank,
-        max_total, _lib.ptr(expert_idxs) if max_total else None, output_splits.data_ptr(),
-        _lib.stream_ptr(device),
-    )  # fmt: skip
-    return expert_idxs, output_splits
+    return _lib.host().build_expert_idxs(tokens_per_expert_group, ep_size, experts_per_rank, max_total,
+                                         _lib.stream_ptr(tokens_per_expert_group.device))  # fmt: skip
 
 
 def adjust_expand_idx(received_expand_idx, dedup_tokens_from_each_gpu, output_splits_tensor):
     """received + exclusive_cumsum(dedup counts)[sender of each slot]."""
     _lib.require_cuda(received_expand_idx)
-    N = received_expand_idx.shape[0]
-    ep_size = dedup_tokens_from_each_gpu.shape[0]
-    out = torch.empty_like(received_expand_idx)
-    if N == 0:
-        return out
-    _lib.call(
-        "pt_adjust_expand_idx", received_expand_idx.contiguous().data_ptr(), out.data_ptr(),
-        dedup_tokens_from_each_gpu.data_ptr(), dedup_tokens_from_each_gpu.stride(0),
-        output_splits_tensor.contiguous().data_ptr(), ep_size, N, _lib.stream_ptr(out.device),
-    )  # fmt: skip
-    return out
+    return _lib.host().adjust_expand_idx(received_expand_idx, dedup_tokens_from_each_gpu, output_splits_tensor,
+                                         _lib.stream_ptr(received_expand_idx.device))  # fmt: skip
 
 
 @torch.compiler.disable

@@ -14,10 +14,8 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ..dualpipe_utils import WeightGradStore
 from .deepgemm_quantize import FP8
-from .grouped_linear import dgrad_operand, m_grouped_fp8_dgrad, schedule_wgrad
-from .token_scatter import _GEMM_ALLOC_ALIGNMENT, _PaddedIndexGather
+from .grouped_linear import dgrad_operand
 
 
 def _cdiv(a: int, b: int) -> int:
@@ -136,91 +134,40 @@ def few_rows_per_expert(rows: int, num_groups: int) -> bool:
     return rows <= 48 * num_groups
 
 
-def _forward(ctx, x, gate_up_weights, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx=None, scatter=True,
-             clamp=None, biases=(None, None), few_rows=False):
-    """Shared forward of the autograd nodes below: one library call queues every launch of it.
-    ``gate_up_weights``: the parameters whose gradients the gate_up weight gradient is written to, one
-    fused ``[G, 2I, K]`` tensor or the pair ``(gate [G, I, K], up [G, I, K])``.  ``expand_idx`` (with
+def _prepare(x, grouped_mm_offs, row_map, expand_idx, scatter):
+    """The checked ``(row_map, expand_idx, scatter)`` of a block on ``x`` (a ``[T, k, K]`` view of one row per
+    token counts as its T * k rows)."""
+    _lib.require_cuda(x)
+    assert expand_idx is None or row_map is not None, "expand_idx needs the row map of the scatter"
+    if row_map is not None:
+        assert row_map.dtype == torch.int32 and row_map.shape[0] % 128 == 0
+        row_map = row_map.contiguous()
+    else:
+        assert x.dim() == 2 and x.shape[0] % 128 == 0, f"grouped rows must be a multiple of 128, got {x.shape[0]}"
+    if expand_idx is not None:
+        assert expand_idx.dtype == torch.int64
+        expand_idx = expand_idx.contiguous()
+    return row_map, expand_idx, scatter and row_map is not None
+
+
+def _node(x, w_gate, w_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx=None, scatter=True, clamp=None, biases=(None, None)):
+    """The autograd node of the three functions below (``csrc/host.cpp``): the forward is one library call that
+    queues every launch of it, and so is the backward but for its input gradient.  ``w_gate`` and
+    ``w_up`` are the parameters whose gradients the gate_up weight gradient is written to; without
+    ``w_up`` the former is the fused ``[G, 2I, K]`` one.  ``expand_idx`` (with
     ``row_map``): ``x`` holds deduplicated rows and routed row i is ``x[expand_idx[i]]``; the result
     has one row per routed row, and the backward sums the gradients of the rows that share a source
     row.  ``scatter`` (with ``row_map``): the result comes back un-permuted.  ``clamp``: ``(alpha,
     limit)`` of the clamped SwiGLU, whose projections have the two ``biases``.  ``x`` may be an expanded
-    ``[T, k, K]`` view of one row per token (routed row i is token i // k).  Without a ``ctx`` nothing is
-    kept for a backward, and the groups may be multiples of 64 rows (``few_rows``)."""
-    _lib.require_cuda(x)
-    repeat = 1
-    if x.dim() == 3:
-        repeat = x.shape[1]
-        x = x[:, 0]
-    gu_fp8, gu_scale = q_gate_up[:2]
-    dn_fp8, dn_scale = q_down[:2]
-    G, H, half = w_down.shape
-    src_rows, K = x.shape
-    assert expand_idx is None or row_map is not None, "expand_idx needs the row map of the scatter"
-    scatter = scatter and row_map is not None
-    if row_map is not None:
-        assert row_map.dtype == torch.int32 and row_map.shape[0] % 128 == 0
-        row_map = row_map.contiguous()
-    M = src_rows if row_map is None else row_map.shape[0]
-    assert M % 128 == 0, f"grouped rows must be a multiple of 128, got {M}"
-    routed = src_rows * repeat
-    if expand_idx is not None:
-        assert expand_idx.dtype == torch.int64
-        expand_idx = expand_idx.contiguous()
-        routed = expand_idx.shape[0]
-    if x.stride(1) != 1:
-        x = x.contiguous()
-    b_gate_up, b_down = biases if biases[0] is None else [b.detach().contiguous() for b in biases]
-    out, gate_up, kept = _lib.host().experts_forward(
-        x, repeat, row_map, expand_idx, grouped_mm_offs, gu_fp8, gu_scale, dn_fp8, dn_scale, half, b_gate_up, b_down, scatter,
-        clamp is not None, *(clamp or (0.0, 0.0)), ctx is not None, few_rows, _lib.stream_ptr(x.device),
+    ``[T, k, K]`` view of one row per token (routed row i is token i // k).  The weight gradients go to
+    ``.grad``, or to the ``WeightGradStore`` queue."""
+    row_map, expand_idx, scatter = _prepare(x, grouped_mm_offs, row_map, expand_idx, scatter)
+    M = x.shape[0] if row_map is None else row_map.shape[0]
+    weights = w_gate if w_up is None else (w_gate, w_up)
+    return _lib.host().experts(
+        x, w_gate, w_up, w_down, *biases, grouped_mm_offs, q_gate_up[:2], q_down[:2], dgrad_operand(q_gate_up, weights, M),
+        dgrad_operand(q_down, w_down, M), row_map, expand_idx, scatter, clamp, _lib.stream_ptr(x.device),
     )  # fmt: skip
-    if ctx is None:
-        return out
-    gu_dg, gu_dg_s, gu_forward = dgrad_operand(q_gate_up, gate_up_weights, M)
-    dn_dg, dn_dg_s, dn_forward = dgrad_operand(q_down, w_down, M)
-    ctx.save_for_backward(gu_dg, gu_dg_s, dn_dg, dn_dg_s, grouped_mm_offs, gate_up, row_map, expand_idx, *kept)
-    ctx.gate_up_weights, ctx.w_down = gate_up_weights, w_down
-    ctx.clamp = clamp
-    ctx.biases = biases
-    ctx.dims = (M, K, half, H, G, routed, src_rows, gu_forward, dn_forward, scatter)
-    ctx.repeat = repeat
-    return out
-
-
-def _backward(ctx, grad_out):
-    """Shared backward: returns the gradient of ``x`` and of the two biases (None without); the weight
-    gradients go to ``.grad``, or to the ``WeightGradStore`` queue."""
-    gu_dg, gu_dg_s, dn_dg, dn_dg_s, offs, gate_up, row_map, expand_idx, *kept = ctx.saved_tensors
-    M, K, half, H, G, routed, src_rows, gu_forward, dn_forward, scatter = ctx.dims
-    split = isinstance(ctx.gate_up_weights, tuple)
-    gu_weights = ctx.gate_up_weights if split else (ctx.gate_up_weights,)
-    deferred = WeightGradStore.enabled
-    # separate gate and up parameters: each gets its half of the gate_up weight gradient's rows
-    step = _lib.host().ExpertsBackward(
-        grad_out, (M, K, half, H, G), offs, row_map, scatter, dn_dg, dn_dg_s, dn_forward, gate_up, kept, ctx.clamp is not None,
-        *(ctx.clamp or (0.0, 0.0)), *ctx.biases, [] if deferred else [ctx.w_down, *gu_weights], _lib.stream_ptr(grad_out.device),
-    )  # fmt: skip
-    grad_x = torch.empty((M if row_map is None else routed, K), device=grad_out.device, dtype=grad_out.dtype)
-    m_grouped_fp8_dgrad((step.dgu, step.dgu_s), gu_dg, gu_dg_s, gu_forward, grad_x, offs, row_map)
-    if not deferred:
-        step.weight_gradient()
-    else:
-        dy_t, (gu, gus), x_t, h_t = step.operands()
-        schedule_wgrad(ctx.w_down, dy_t, h_t, offs)
-        if split:
-            schedule_wgrad(gu_weights[0], (gu[:half], gus[:, :half]), x_t, offs)
-            schedule_wgrad(gu_weights[1], (gu[half:], gus[:, half:]), x_t, offs)
-        else:
-            schedule_wgrad(gu_weights[0], (gu, gus), x_t, offs)
-    d_gu_bias, d_dn_bias = step.d_gu_bias, step.d_dn_bias
-    if expand_idx is not None:
-        # one gradient row per routed row so far: rows that expand the same source row are summed
-        # (the backward of the expanding gather, token_scatter.py:311-325)
-        grad_x = _PaddedIndexGather.scatter_sum(grad_x, expand_idx, src_rows, _GEMM_ALLOC_ALIGNMENT)
-    if ctx.repeat > 1:
-        grad_x = grad_x.view(src_rows, ctx.repeat, K)
-    return grad_x, d_gu_bias, d_dn_bias
 
 
 def wants_backward(x: torch.Tensor, *weights: torch.Tensor) -> bool:
@@ -228,28 +175,36 @@ def wants_backward(x: torch.Tensor, *weights: torch.Tensor) -> bool:
     return torch.is_grad_enabled() and (x.requires_grad or any(w.requires_grad for w in weights))
 
 
-def forward_only(x, w_gate_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map=None, expand_idx=None, scatter=True,
+def forward_only(x, w_down, grouped_mm_offs, q_gate_up, q_down, row_map=None, expand_idx=None, scatter=True,
                  clamp=None, biases=(None, None), few_rows=False):
-    """The forward of the nodes below when no backward follows: nothing is kept, and the quantisers leave out
-    the transposed operands of the weight gradients."""
-    return _forward(None, x, w_gate_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx, scatter, clamp, biases, few_rows)
+    """The forward of the nodes below when no backward follows: nothing is kept, the quantisers leave out
+    the transposed operands of the weight gradients, and the groups may be multiples of 64 rows
+    (``few_rows``)."""
+    row_map, expand_idx, scatter = _prepare(x, grouped_mm_offs, row_map, expand_idx, scatter)
+    repeat = 1
+    if x.dim() == 3:
+        repeat, x = x.shape[1], x[:, 0]
+    if x.stride(1) != 1:
+        x = x.contiguous()
+    if biases[0] is not None:
+        biases = [b.detach().contiguous() for b in biases]
+    return _lib.host().experts_forward(
+        x, repeat, row_map, expand_idx, grouped_mm_offs, *q_gate_up[:2], *q_down[:2], w_down.shape[2], *biases, scatter, clamp is not None,
+        *(clamp or (0.0, 0.0)), False, few_rows, _lib.stream_ptr(x.device),
+    )[0]  # fmt: skip
 
 
-class FP8SwiGLUExpertsFunc(torch.autograd.Function):
+class FP8SwiGLUExpertsFunc:
     @staticmethod
-    def forward(ctx, x, w_gate_up, w_down, grouped_mm_offs, ks, ks_tensor, q_gate_up, q_down, row_map=None, expand_idx=None):
+    def apply(x, w_gate_up, w_down, grouped_mm_offs, ks, ks_tensor, q_gate_up, q_down, row_map=None, expand_idx=None):
         """``x`` is ``[M, K]`` grouped rows, or with ``row_map`` (int32 ``[M]``) the un-permuted
         ``[m, K]`` tokens; the result has the same row layout as ``x``.  ``row_map`` may be longer
         than the grouped rows (its tail negative): every kernel takes the real row count from
         ``grouped_mm_offs`` on the device, so no host-side size is needed (``ks`` may be None)."""
-        return _forward(ctx, x, w_gate_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx)
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        return _backward(ctx, grad_out)[0], None, None, None, None, None, None, None, None, None
+        return _node(x, w_gate_up, None, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx)
 
 
-class FP8SwiGLUSplitExpertsFunc(torch.autograd.Function):
+class FP8SwiGLUSplitExpertsFunc:
     """The same node for experts that keep gate and up as separate parameters
     (``Qwen3MoeExperts`` / ``DeepSeekV2Experts``, models/qwen3_moe.py:45-65): ``q_gate_up`` is the
     two weights quantised into one fused operand (:func:`fp8cast_blockwise_transpose_batched_cat`),
@@ -257,12 +212,8 @@ class FP8SwiGLUSplitExpertsFunc(torch.autograd.Function):
     gradients are written to the two parameters separately."""
 
     @staticmethod
-    def forward(ctx, x, w_gate, w_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map=None, expand_idx=None):
-        return _forward(ctx, x, (w_gate, w_up), w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx)
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        return _backward(ctx, grad_out)[0], None, None, None, None, None, None, None, None
+    def apply(x, w_gate, w_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map=None, expand_idx=None):
+        return _node(x, w_gate, w_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx)
 
 
 def supported_split(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor) -> bool:
@@ -272,7 +223,7 @@ def supported_split(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w
             and w_down.shape[1] % 8 == 0 and w_down.shape[2] == half)
 
 
-class FP8ClampedSwiGLUExpertsFunc(torch.autograd.Function):
+class FP8ClampedSwiGLUExpertsFunc:
     """The GPT-OSS expert block (models/gpt_oss.py:139-157: gate_up projection + bias, clamped
     SwiGLU on interleaved pairs, down projection + bias) as one node.  Outputs, input gradient,
     weight gradients and the down bias gradient have the bits of the composition of
@@ -286,13 +237,8 @@ class FP8ClampedSwiGLUExpertsFunc(torch.autograd.Function):
     with ``scatter_output`` the result comes back un-permuted as well."""
 
     @staticmethod
-    def forward(ctx, x, w_gate_up, b_gate_up, w_down, b_down, grouped_mm_offs, q_gate_up, q_down, alpha, limit,
+    def apply(x, w_gate_up, b_gate_up, w_down, b_down, grouped_mm_offs, q_gate_up, q_down, alpha, limit,
                 row_map=None, scatter_output=False):
         assert not scatter_output or row_map is not None, "scatter_output needs the row map"
-        return _forward(ctx, x, w_gate_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, None, scatter_output,
-                        (float(alpha), float(limit)), (b_gate_up, b_down))
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        grad_x, grad_b_gate_up, grad_b_down = _backward(ctx, grad_out)
-        return grad_x, None, grad_b_gate_up, None, grad_b_down, None, None, None, None, None, None, None
+        return _node(x, w_gate_up, None, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, None, scatter_output,
+                     (float(alpha), float(limit)), (b_gate_up, b_down))

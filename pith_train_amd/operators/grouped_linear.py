@@ -309,6 +309,9 @@ def m_grouped_fp8_dgrad(grad, w_fp8: torch.Tensor, w_scale: torch.Tensor, forwar
     return m_grouped_fp8_gemm_nt(grad, (w_fp8, w_scale), out, grouped_mm_offs, out_rows)
 
 
+_GEMM_OUT = (torch.bfloat16,)  # activations the grouped GEMMs store; the C++ node (``csrc/host.cpp``) takes these
+
+
 class FP8GroupedLinearFunc(torch.autograd.Function):
     """FP8 grouped linear (grouped_linear.py:104-236): forward and dgrad are m-grouped NT GEMMs on
     1x128-scaled activations against 128x128-scaled weights, wgrad a k-grouped GEMM on the colwise
@@ -432,7 +435,15 @@ class FP8GroupedLinear(nn.Module):
     ) -> torch.Tensor:
         if input.shape[0] == 0:
             return input @ self.weight[0].T  # keeps a grad_fn with zero rows
+        quantized = self._get_quantized_weight()
+        if (in_rows is None and out_rows is None and input.dim() == 2 and input.shape[0] % 128 == 0 and input.dtype in _GEMM_OUT
+                and input.shape[1] % 16 == 0 and not torch.compiler.is_compiling()):
+            weight = self._parameters.get("weight")
+            if weight is not None and not weight.shape[1] % 16:
+                dg_fp8, dg_scale, forward_layout = dgrad_operand(quantized, weight, input.shape[0])
+                return _lib.host().grouped_linear(input, weight, grouped_mm_offs, quantized[0], quantized[1], dg_fp8, dg_scale,
+                                                  forward_layout, _lib.stream_ptr(input.device))  # fmt: skip
         return FP8GroupedLinearFunc.apply(
-            input, self.weight, grouped_mm_offs, ks, ks_tensor, self._get_quantized_weight(),
+            input, self.weight, grouped_mm_offs, ks, ks_tensor, quantized,
             group_indices, in_rows, out_rows, out_m,
         )  # fmt: skip

@@ -70,6 +70,13 @@ class _RouterTopK(torch.autograd.Function):
         return d_logits, None, None, None, None, None, None, None, None
 
 
+def _plain(logits, mode, k, norm, scale, num_group, topk_group):
+    """The gate without forced choices and without the scores: one autograd node in ``csrc/host.cpp``."""
+    _lib.require_cuda(logits)
+    assert logits.ndim == 2, "logits must be [T, E]"
+    return _lib.host().router_topk(logits, mode, k, norm, float(scale), num_group, topk_group, _lib.stream_ptr(logits.device))
+
+
 def softmax_topk(logits: torch.Tensor, k: int, *, norm_topk_prob: bool = False, scale: float = 1.0,
                  num_group: int = 1, topk_group: int = 1, forced_idx: Optional[torch.Tensor] = None,
                  return_scores: bool = False):
@@ -77,6 +84,8 @@ def softmax_topk(logits: torch.Tensor, k: int, *, norm_topk_prob: bool = False, 
     [``/ sum``] ``* scale``.  With ``num_group > 1`` only the ``topk_group`` groups of
     ``E / num_group`` contiguous experts with the largest maximum score keep their scores; the
     returned ``scores`` are the limited ones, as in the reference."""
+    if forced_idx is None and not return_scores:
+        return _plain(logits, 0, k, norm_topk_prob, scale, num_group, topk_group if num_group > 1 else 1)
     return _RouterTopK.apply(logits, 0, k, norm_topk_prob, scale, num_group, topk_group if num_group > 1 else 1,
                              forced_idx, return_scores)
 
@@ -85,4 +94,6 @@ def topk_softmax(logits: torch.Tensor, k: int, *, forced_idx: Optional[torch.Ten
                  return_scores: bool = False):
     """Top-k of the logits, then the fp32 softmax over the k chosen logits; ``scores`` (when asked
     for) is the softmax over all experts."""
+    if forced_idx is None and not return_scores:
+        return _plain(logits, 1, k, False, 1.0, 1, 1)
     return _RouterTopK.apply(logits, 1, k, False, 1.0, 1, 1, forced_idx, return_scores)

@@ -101,129 +101,63 @@ def gather_rows(input: torch.Tensor, index: torch.Tensor, out: torch.Tensor) -> 
     return out
 
 
-class ScatterForGroupedGemm(torch.autograd.Function):
+class ScatterForGroupedGemm:
     """Forward: rows grouped by expert, groups zero-padded to the alignment.  Backward: gather."""
 
     @staticmethod
-    def forward(ctx, input_tokens, expert_idxs, num_groups, padding_alignment=128, pre_index=None):
+    def apply(input_tokens, expert_idxs, num_groups, padding_alignment=128, pre_index=None):
         _lib.require_cuda(input_tokens, expert_idxs)
         m = expert_idxs.shape[0]
-        hidden_size = input_tokens.shape[1]
         device = input_tokens.device
-        ctx.pre_index = pre_index
-        ctx.in_rows = input_tokens.shape[0]
         if m == 0:
-            output_tokens = torch.empty((0, hidden_size), device=device, dtype=input_tokens.dtype)
+            output_tokens = torch.empty((0, input_tokens.shape[1]), device=device, dtype=input_tokens.dtype)
             reverse = torch.empty((0,), device=device, dtype=torch.int64)
             offs = torch.empty((0,), device=device, dtype=torch.int32)
             ks_tensor = torch.empty((0,), device=device, dtype=torch.int32)
-            ctx.save_for_backward(reverse)
-            ctx.src_of = None
             return output_tokens, reverse, offs, ks_tensor, []
-        if input_tokens.stride(1) != 1:
-            input_tokens = input_tokens.contiguous()
         expert_idxs = expert_idxs.contiguous()
         assert expert_idxs.dtype == torch.int64, "expert_idxs must be int64"
 
         max_m_padded = m + num_groups * (padding_alignment - 1)
         max_m_padded = -(-max_m_padded // _GEMM_ALLOC_ALIGNMENT) * _GEMM_ALLOC_ALIGNMENT
-        reverse, offs, ks_tensor, src_of = group_rows(
-            expert_idxs, num_groups, padding_alignment, max_m_padded
-        )
-        # ks goes to the host on a side stream while the row copy runs
+        host, stream = _lib.host(), _lib.stream_ptr(device)
+        reverse, offs, ks_tensor, src_of = group_rows(expert_idxs, num_groups, padding_alignment, max_m_padded)
+        # The group sizes go to the host ahead of the row copy, and only they are waited for.
         ks_cpu = get_pinned_buffer("ks", num_groups, torch.int32)
-        copy_stream, copy_event = _copy_stream_and_event(device)
-        copy_event.record()
-        output_tokens = torch.empty((max_m_padded, hidden_size), device=device, dtype=input_tokens.dtype)
-        permute_rows(input_tokens, src_of, output_tokens, offs[num_groups - 1 :], pre_index)
-        with torch.cuda.stream(copy_stream):
-            copy_stream.wait_event(copy_event)
-            ks_cpu.copy_(ks_tensor, non_blocking=True)
-        copy_stream.synchronize()
+        copied = _copy_event()
+        ks_cpu.copy_(ks_tensor, non_blocking=True)
+        copied.record()
+        buffer = host.permute_into_buffer(input_tokens, src_of, offs, pre_index, stream)
+        copied.synchronize()
         ks = ks_cpu.tolist()
-        actual_M = sum(ks)
-        output_tokens = output_tokens[:actual_M]
-        ctx.save_for_backward(reverse)
-        ctx.mark_non_differentiable(reverse, offs, ks_tensor)
+        output_tokens = host.permute_rows(input_tokens, src_of, offs, reverse, pre_index, buffer, sum(ks), stream)
         return output_tokens, reverse, offs, ks_tensor, ks
 
-    @staticmethod
-    def backward(ctx, grad_output_tokens, *unused):
-        (reverse,) = ctx.saved_tensors
-        m = reverse.shape[0]
-        grad_output_tokens = grad_output_tokens.contiguous()
-        H = grad_output_tokens.shape[1]
-        grad = torch.empty((m, H), device=grad_output_tokens.device, dtype=grad_output_tokens.dtype)
-        gather_rows(grad_output_tokens, reverse, grad)
-        if ctx.pre_index is not None:
-            grad = _PaddedIndexGather.scatter_sum(grad, ctx.pre_index, ctx.in_rows, _GEMM_ALLOC_ALIGNMENT)
-        return grad, None, None, None, None
+
+_copy_events: dict[int, torch.cuda.Event] = {}
 
 
-_copy_stream: Optional[torch.cuda.Stream] = None
-_copy_event: Optional[torch.cuda.Event] = None
+def _copy_event() -> torch.cuda.Event:
+    device = torch.cuda.current_device()
+    event = _copy_events.get(device)
+    if event is None:
+        event = _copy_events[device] = torch.cuda.Event()
+    return event
 
 
-def _copy_stream_and_event(device):
-    global _copy_stream, _copy_event
-    if _copy_stream is None:
-        _copy_stream = torch.cuda.Stream(device=device)
-        _copy_event = torch.cuda.Event()
-    return _copy_stream, _copy_event
-
-
-class _PaddedIndexGather(torch.autograd.Function):
+class _PaddedIndexGather:
     """``input[index]`` into a buffer whose row count is padded; the input is not saved, backward
     sums the rows that share an index."""
 
     @staticmethod
-    def forward(ctx, input: torch.Tensor, index: torch.Tensor, pad_to_multiple: int):
-        _lib.require_cuda(input, index)
-        ctx.save_for_backward(index)
-        ctx.input_shape = input.shape
-        ctx.pad_to_multiple = pad_to_multiple
-        actual = index.shape[0]
-        padded = -(-actual // pad_to_multiple) * pad_to_multiple
-        buf = input.new_empty(padded, *input.shape[1:])
-        if actual:
-            src = input.reshape(input.shape[0], -1)
-            if src.stride(-1) != 1:
-                src = src.contiguous()
-            gather_rows(src, index.contiguous(), buf[:actual].view(actual, -1))
-        return buf[:actual]
-
-    @staticmethod
     def scatter_sum(grad_output, index, rows: int, pad_to_multiple: int):
-        padded_rows = -(-rows // pad_to_multiple) * pad_to_multiple
-        tail = tuple(grad_output.shape[1:])
-        grad_buf = torch.empty((padded_rows,) + tail, dtype=grad_output.dtype, device=grad_output.device)
-        n = index.shape[0]
-        H = 1
-        for d in tail:
-            H *= d
-        if rows and H:
-            go = grad_output.contiguous().view(n, H)
-            ws_bytes = _lib.query("pt_gather_rows_backward_workspace_bytes", n, rows)
-            ws = _workspace(ws_bytes, grad_output.device)
-            _lib.call(
-                "pt_gather_rows_backward", go.data_ptr(), H, grad_buf.data_ptr(), H,
-                index.contiguous().data_ptr(), n, rows, H, _lib.dtype_code(grad_output.dtype),
-                ws.data_ptr(), ws.numel(), _lib.stream_ptr(grad_output.device),
-            )  # fmt: skip
-        return grad_buf[:rows]
-
-    @staticmethod
-    def backward(ctx, grad_output: torch.Tensor):
-        (index,) = ctx.saved_tensors
-        grad = _PaddedIndexGather.scatter_sum(
-            grad_output, index, ctx.input_shape[0], ctx.pad_to_multiple
-        )
-        return grad, None, None
+        return _lib.host().scatter_sum(grad_output, index, rows, pad_to_multiple, _lib.stream_ptr(grad_output.device))
 
 
 def padded_index_gather(input: torch.Tensor, index: torch.Tensor, pad_to_multiple: int = 1024):
     """Memory-lean ``input[index]`` with a padded allocation."""
-    return _PaddedIndexGather.apply(input, index, pad_to_multiple)
+    _lib.require_cuda(input, index)
+    return _lib.host().index_gather(input, index, pad_to_multiple, _lib.stream_ptr(input.device))
 
 
 def scatter_for_grouped_gemm(
