@@ -145,8 +145,9 @@ void require_cuda(const Tensor& t) {
 
 // Row pitch of a transposed operand: the rule of deepgemm_quantize.transposed_pitch.
 int64_t transposed_pitch(int64_t m) {
-  m = (m + 15) / 16 * 16;
-  return m >= 2048 && m % 256 == 0 ? m + 128 : m;
+  if (m < 2048) return (m + 15) / 16 * 16;
+  m = (m + 127) / 128 * 128;
+  return m % 256 == 0 ? m + 128 : m;
 }
 
 constexpr int64_t kWorkgroups = 256;  // compute units of the MI355X

@@ -195,15 +195,20 @@ extern "C" int pt_linear_forward(const pt_linear_forward_args* args) {
                     (float*)(void*)ws.p, a.stream);
 }
 
-// a pitch that is no multiple of 256 bytes spreads the rows of a reduction step over the memory channels
-static int64_t transposed_pitch(int64_t red) { return red >= 2048 && red % 256 == 0 ? red + 128 : red; }
+// Row pitch of a transposed operand (`red` = its length, a multiple of 16): whole 128-byte lines, and no
+// multiple of 256 bytes, which would put the rows of a reduction step onto few memory channels.
+static int64_t transposed_pitch(int64_t red) {
+  if (red < 2048) return red;
+  red = (red + 127) & ~(int64_t)127;
+  return red % 256 == 0 ? red + 128 : red;
+}
 
 // workspace: gradient bytes and scales | its transposed form and scales | the input's transposed form and
 // scales when it is quantised here | slabs of whichever GEMM is split
 extern "C" int64_t pt_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t x_splits, int64_t w_splits, int64_t from_x) {
   const int64_t sx = x_splits > 1 ? 4 * x_splits * M * K : 0, sw = w_splits > 1 ? 4 * w_splits * N * K : 0;
-  return up(M * N) + up(4 * M * cdiv(N, 128)) + up(N * (M + 256)) + up(4 * N * cdiv(M, 128)) + up(sx > sw ? sx : sw) +
-         (from_x ? up(K * (M + 256)) + up(4 * cdiv(K, 128) * cdiv(M, 128)) : 0);
+  return up(M * N) + up(4 * M * cdiv(N, 128)) + up(N * (M + 384)) + up(4 * N * cdiv(M, 128)) + up(sx > sw ? sx : sw) +
+         (from_x ? up(K * (M + 384)) + up(4 * cdiv(K, 128) * cdiv(M, 128)) : 0);
 }
 
 extern "C" int pt_linear_backward(const pt_linear_backward_args* args) {
@@ -217,13 +222,13 @@ extern "C" int pt_linear_backward(const pt_linear_backward_args* args) {
   Carve ws(a.workspace);
   void* g_fp8 = ws.bytes(a.M * a.N);
   float* g_s = ws.floats(a.M * cdiv(a.N, 128));
-  void* g_t = ws.bytes(a.N * (a.M + 256));
+  void* g_t = ws.bytes(a.N * (a.M + 384));
   float* g_ts = ws.floats(a.N * cdiv(a.M, 128));
   const void* x_t = a.x_t;
   const float* x_ts = a.x_t_scale;
   int64_t ld_xt = a.ld_xt;
   if (!x_t) {
-    void* t = ws.bytes(a.K * (a.M + 256));
+    void* t = ws.bytes(a.K * (a.M + 384));
     float* ts = ws.floats(cdiv(a.K, 128) * cdiv(a.M, 128));
     ld_xt = ld_t;
     PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, nullptr, nullptr, t, ld_xt, ts, a.stream);
