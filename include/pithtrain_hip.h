@@ -150,6 +150,15 @@ int pt_quant_rowwise_blockwise_transpose_ld(const void* x, int dtype, int64_t M,
                                             void* blk_t_fp8, int64_t ld_t, float* blk_t_scale,
                                             pt_stream_t stream);
 
+/* pt_quant_rowwise_blockwise_transpose_ld of x [M, K] and pt_quant_blockwise_transpose_batched of one weight
+ * w [N, K], both in dtype (bf16 or fp32), with one launch while they have up to
+ * PT_QUANT_LINEAR_MAX_TILES 128 x 128 tiles together. */
+#define PT_QUANT_LINEAR_MAX_TILES 1024
+int pt_quant_linear_operands(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K,
+                             int64_t ldx, int64_t ldw, void* tok_fp8, float* tok_scale, void* blk_t_fp8,
+                             int64_t ld_t, float* blk_t_scale, void* w_fp8, float* w_scale,
+                             void* w_t_fp8, float* w_t_scale, pt_stream_t stream);
+
 /* 128x128 blockwise(x) + blockwise(x^T) for x[G,N,K] (element strides stride_g, stride_row):
  * fp8[G,N,K], scale[G,ceil(N/128),ceil(K/128)], fp8_t[G,K,N], scale_t[G,ceil(K/128),ceil(N/128)].
  * fp8cast_blockwise_transpose (:709-756, G == 1) and fp8cast_blockwise_transpose_batched
@@ -638,9 +647,11 @@ int pt_experts_weight_gradient(const pt_experts_backward_args* args /* host */);
 /* Forward of a dense FP8 linear (fp8_act_weight_gemm, operators/linear.py:44-60): x [M, K] in dtype,
  * y [M, N] in y_dtype (PT_BF16 or PT_F32); x_t (row pitch ld_t >= M bytes) and x_t_scale are the transposed
  * operand the weight gradient reads (both NULL: not written).  K % 16 == 0.  y2 != NULL (bf16, splits == 1):
- * the outputs of pt_gemm_nt_dense_heads. */
+ * the outputs of pt_gemm_nt_dense_heads.  w != NULL (in dtype, row stride ldw): the weight itself, quantised
+ * here into w_fp8 [N, K], w_scale, w_t_fp8 [K, N] and w_t_scale (then outputs, with x_t). */
 typedef struct {
   const void* x; int64_t dtype, M, K, ldx;
+  const void* w; int64_t ldw; void* w_t_fp8; float* w_t_scale;
   const void* w_fp8; const float* w_scale; int64_t N;
   void* y; int64_t y_dtype;
   void* x_t; int64_t ld_t; float* x_t_scale;

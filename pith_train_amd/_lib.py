@@ -40,6 +40,7 @@ SIGNATURES = {
     "pt_quant_rowwise_transpose_ld": (c_int, [P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_rowwise_blockwise_transpose_ld": (c_int, [P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_heads_rowwise_transpose_ld": (c_int, [P, P, I64, I64, I64, I64, P, P, P, I64, P, P]),
+    "pt_quant_linear_operands": (c_int, [P, P, c_int, I64, I64, I64, I64, I64, P, P, P, I64, P, P, P, P, P, P]),
     "pt_quant_blockwise_transpose_batched": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, P, P, P, P]),
     "pt_quant_blockwise_transpose_batched_into": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, I64, P, I64, P, I64, I64, P, I64,
                                                           I64, P]),

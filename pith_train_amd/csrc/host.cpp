@@ -227,13 +227,16 @@ std::vector<std::pair<Tensor, Tensor>> quant_grouped_weights(const std::vector<s
 // dense linear
 // ---------------------------------------------------------------------------------------------------------
 // Whether the whole-step entry points take both directions of y[m, n] = x[m, k] W^T.
-bool linear_supported(const Tensor& x, const Tensor& w_fp8, const Tensor& w_t) {
-  const int64_t m = x.size(0), k = x.size(1), n = w_fp8.size(0);
-  return (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat) && m > 0 && n > 0 && k > 0 && k % 16 == 0 && n % 16 == 0 &&
-         w_fp8.is_contiguous() && w_t.is_contiguous();
+bool linear_supported(const Tensor& x, int64_t n) {
+  const int64_t m = x.size(0), k = x.size(1);
+  return (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat) && m > 0 && n > 0 && k > 0 && k % 16 == 0 && n % 16 == 0;
 }
 
-std::tuple<Tensor, Tensor, Tensor> linear_forward(const Tensor& input, const Tensor& w_fp8, const Tensor& w_s, int64_t stream) {
+typedef std::tuple<Tensor, Tensor, Tensor, Tensor> QuantisedWeight;  // bytes, scales, transposed bytes, their scales
+
+// (y, x^T, its scales); `fresh`: the weight itself, to be quantised into `q` in the same call
+std::tuple<Tensor, Tensor, Tensor> linear_forward(const Tensor& input, const QuantisedWeight& q, const Tensor* fresh, int64_t stream) {
+  const auto& [w_fp8, w_s, w_t, w_ts] = q;
   const Tensor x = row_major(input);
   const int64_t m = x.size(0), k = x.size(1), n = w_fp8.size(0);
   const auto dev = x.device();
@@ -242,7 +245,9 @@ std::tuple<Tensor, Tensor, Tensor> linear_forward(const Tensor& input, const Ten
   const auto [splits, len] = split_k(m, n, k);
   Tensor ws = empty({lib.pt_linear_forward_workspace_bytes(m, n, k, splits)}, at::kByte, dev);
   const int code = dtype_code(x.scalar_type());
-  const pt_linear_forward_args a = {ptr(x), code, m, k, m > 1 ? x.stride(0) : k, ptr(w_fp8), (const float*)ptr(w_s), n, ptr(y), code, ptr(x_t), ld_t,
+  const pt_linear_forward_args a = {ptr(x), code, m, k, m > 1 ? x.stride(0) : k,
+                                    fresh ? ptr(*fresh) : nullptr, fresh ? (n > 1 ? fresh->stride(0) : k) : 0, fresh ? ptr(w_t) : nullptr,
+                                    fresh ? (float*)ptr(w_ts) : nullptr, ptr(w_fp8), (const float*)ptr(w_s), n, ptr(y), code, ptr(x_t), ld_t,
                                     (float*)ptr(x_ts), splits, len, nullptr, 0, 0, ptr(ws), (pt_stream_t)stream};
   check(lib.pt_linear_forward(&a), "pt_linear_forward");
   return {y, x_t, x_ts};
@@ -250,10 +255,9 @@ std::tuple<Tensor, Tensor, Tensor> linear_forward(const Tensor& input, const Ten
 
 struct LinearFunction : torch::autograd::Function<LinearFunction> {
   // weight is an argument for its gradient's sake; the quantised forms are what is read
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const Tensor& w_s, const Tensor& w_t,
-                        const Tensor& w_ts, int64_t stream) {
-    auto [y, x_t, x_ts] = linear_forward(x, w_fp8, w_s, stream);
-    ctx->save_for_backward({w_t, w_ts, x_t, x_ts});
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const QuantisedWeight& q, const Tensor* fresh, int64_t stream) {
+    auto [y, x_t, x_ts] = linear_forward(x, q, fresh, stream);
+    ctx->save_for_backward({std::get<2>(q), std::get<3>(q), x_t, x_ts});
     ctx->saved_data["stream"] = stream;
     return y;
   }
@@ -277,15 +281,27 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
       gx = gx.to(g.scalar_type());
       gw = gw.to(g.scalar_type());
     }
-    return {gx, gw, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    return {gx, gw, Tensor(), Tensor(), Tensor()};
   }
 };
 
 // None where the whole-step entry points do not take the shape.
 Maybe linear(const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const Tensor& w_s, const Tensor& w_t, const Tensor& w_ts, int64_t stream) {
   require_cuda(x);
-  if (!linear_supported(x, w_fp8, w_t)) return std::nullopt;
-  return LinearFunction::apply(x, weight, w_fp8, w_s, w_t, w_ts, stream);
+  if (!linear_supported(x, w_fp8.size(0)) || !w_fp8.is_contiguous() || !w_t.is_contiguous()) return std::nullopt;
+  return LinearFunction::apply(x, weight, QuantisedWeight{w_fp8, w_s, w_t, w_ts}, (const Tensor*)nullptr, stream);
+}
+
+// The same with a weight that has not been quantised yet: (result, its quantised forms), or two Nones.
+std::pair<Maybe, std::optional<QuantisedWeight>> linear_fresh(const Tensor& x, const Tensor& weight, int64_t stream) {
+  require_cuda(x);
+  if (weight.dim() != 2 || !linear_supported(x, weight.size(0))) return {std::nullopt, std::nullopt};
+  const Tensor w = row_major(weight.detach());
+  const int64_t N = w.size(0), K = w.size(1), nb = cdiv(N, 128), kb = cdiv(K, 128);
+  const auto dev = w.device();
+  QuantisedWeight q{empty({N, K}, kFp8, dev), empty({nb, kb}, at::kFloat, dev), empty({K, N}, kFp8, dev), empty({kb, nb}, at::kFloat, dev)};
+  Tensor y = LinearFunction::apply(x, weight, q, &w, stream);
+  return {y, q};
 }
 
 // Dense linear on two per-head halves (see operators/linear.py).
@@ -295,7 +311,8 @@ std::pair<Tensor, Tensor> linear_heads_forward(const Tensor& input, const Tensor
   const int64_t m = x.size(0), k = x.size(1), n = w_fp8.size(0), na = m * heads * head_a, nb = m * heads * head_b;
   Tensor y = empty({na + nb}, at::kBFloat16, x.device());  // one allocation: the GEMM stores through one descriptor
   Tensor ws = empty({lib.pt_linear_forward_workspace_bytes(m, n, k, 1)}, at::kByte, x.device());
-  const pt_linear_forward_args a = {ptr(x), PT_BF16, m, k, m > 1 ? x.stride(0) : k, ptr(w_fp8), (const float*)ptr(w_s), n, ptr(y), PT_BF16, nullptr, 0,
+  const pt_linear_forward_args a = {ptr(x), PT_BF16, m, k, m > 1 ? x.stride(0) : k, nullptr, 0, nullptr, nullptr,
+                                    ptr(w_fp8), (const float*)ptr(w_s), n, ptr(y), PT_BF16, nullptr, 0,
                                     nullptr, 1, k, (char*)ptr(y) + 2 * na, head_a, head_b, ptr(ws), (pt_stream_t)stream};
   check(lib.pt_linear_forward(&a), "pt_linear_forward");
   return {y.narrow(0, 0, na).view({m, heads, head_a}), y.narrow(0, na, nb).view({m, heads, head_b})};
@@ -1086,6 +1103,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("quant_weight", &quant_weight);
   m.def("quant_grouped_weights", &quant_grouped_weights);
   m.def("linear", &linear);
+  m.def("linear_fresh", &linear_fresh);
   m.def("linear_heads_forward", &linear_heads_forward);
   m.def("linear_heads_backward", &linear_heads_backward);
   m.def("group_rows", &group_rows);

@@ -182,11 +182,20 @@ extern "C" int pt_linear_forward(const pt_linear_forward_args* args) {
   PT_REQUIRE(args, "linear_forward: null arguments");
   const pt_linear_forward_args& a = *args;
   PT_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0 && a.x && a.workspace, "linear_forward: bad arguments");
+  PT_REQUIRE(!a.w || a.x_t, "linear_forward: a weight is quantised together with the transposed input");
   Carve ws(a.workspace);
   void* x_fp8 = ws.bytes(a.M * a.K);
   float* x_s = ws.floats(a.M * cdiv(a.K, 128));
-  PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, x_fp8, x_s, a.x_t, a.x_t ? a.ld_t : a.M,
-          a.x_t_scale, a.stream);
+  const bool together = a.w && cdiv(a.K, 128) * (cdiv(a.M, 128) + cdiv(a.N, 128)) <= PT_QUANT_LINEAR_MAX_TILES;
+  if (together)
+    PT_STEP(pt_quant_linear_operands, a.M, a.N, a.K, a.x, a.w, (int)a.dtype, a.M, a.N, a.K, a.ldx, a.ldw, x_fp8, x_s, a.x_t, a.ld_t, a.x_t_scale,
+            const_cast<void*>(a.w_fp8), const_cast<float*>(a.w_scale), a.w_t_fp8, a.w_t_scale, a.stream);
+  else if (a.w)
+    PT_STEP(pt_quant_blockwise_transpose_batched, a.N, a.K, 0, a.w, (int)a.dtype, 1, a.N, a.K, a.N * a.K, a.ldw, const_cast<void*>(a.w_fp8),
+            const_cast<float*>(a.w_scale), a.w_t_fp8, a.w_t_scale, a.stream);
+  if (!together)
+    PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, x_fp8, x_s, a.x_t, a.x_t ? a.ld_t : a.M,
+            a.x_t_scale, a.stream);
   if (a.y2) {
     PT_STEP(pt_gemm_nt_dense_heads, a.M, a.N, a.K, x_fp8, x_s, a.w_fp8, a.w_scale, a.y, a.y2, a.head_a, a.head_b, a.M, a.N, a.K, a.stream);
     return PT_OK;

@@ -781,6 +781,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void q
   else      quant_tile_body<T, A_BLOCK, B_BLOCK, BL_NONE, BS_MB_N, PRO_NONE, false>(p, s_colmax, s_blk, nullptr, nullptr, tc, tr, g);
 }
 
+// The weight and the input of a small dense linear in one launch: the first `weight_tiles` workgroups take
+// the weight's tiles (128 x 128 scales both ways), the others the input's (row scales and the transposed
+// 128 x 128 form).  Either alone is a few microseconds of latency, and a launch costs the host four.
+struct QuantLinearArgs { QuantArgs w, x; int weight_tiles; };
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void quant_linear_kernel(QuantLinearArgs q) {
+  __shared__ float s_colmax[4][128];
+  __shared__ float s_blk[4];
+  __shared__ __attribute__((aligned(16))) uint8_t s_t[128 * 128];
+  const bool weight = (int)blockIdx.x < q.weight_tiles;
+  const QuantArgs& p = weight ? q.w : q.x;
+  const int b = (int)blockIdx.x - (weight ? 0 : q.weight_tiles);
+  const int tr = b / p.tiles_n, tc = b - tr * p.tiles_n;
+  const bool full = (int64_t)tr * 128 + 128 <= p.M && (int64_t)tc * 128 + 128 <= p.N && p.vec_in && p.vec_out && p.vec_out_t;
+  if (weight) {
+    if (full) quant_tile_body<T, A_BLOCK, B_BLOCK, BL_TRANSPOSED, BS_MB_N, PRO_NONE, true>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
+    else      quant_tile_body<T, A_BLOCK, B_BLOCK, BL_TRANSPOSED, BS_MB_N, PRO_NONE, false>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
+  } else {
+    if (full) quant_tile_body<T, A_ROW, B_BLOCK, BL_TRANSPOSED, BS_MB_N, PRO_NONE, true>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
+    else      quant_tile_body<T, A_ROW, B_BLOCK, BL_TRANSPOSED, BS_MB_N, PRO_NONE, false>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
+  }
+}
+
 static int launch_quant_weights(const QuantWeightsArgs& w, int dtype, hipStream_t stream) {
   const int64_t blocks = w.n ? w.end[w.n - 1] : 0;
   if (blocks == 0) return PT_OK;
@@ -1044,6 +1067,33 @@ extern "C" int pt_quant_blockwise_transpose_batched_into(const void* x, int dtyp
   return quant_blockwise_transpose_batched_impl(x, dtype, G, N, K, stride_g, stride_row, fp8, fp8_stride_g, scale,
                                                 scale_stride_g, fp8_t, t_ld, t_stride_g, scale_t, scale_t_ld,
                                                 scale_t_stride_g, stream);
+}
+
+extern "C" int pt_quant_linear_operands(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                                        void* tok_fp8, float* tok_scale, void* blk_t_fp8, int64_t ld_t, float* blk_t_scale, void* w_fp8,
+                                        float* w_scale, void* w_t_fp8, float* w_t_scale, pt_stream_t stream) {
+  PT_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldw >= K && ld_t >= M, "quant_linear_operands: bad shape");
+  PT_REQUIRE(x && w && tok_fp8 && tok_scale && blk_t_fp8 && blk_t_scale && w_fp8 && w_scale && w_t_fp8 && w_t_scale,
+             "quant_linear_operands: null pointer");
+  const int64_t weight_tiles = cdiv(N, 128) * cdiv(K, 128), tiles = weight_tiles + cdiv(M, 128) * cdiv(K, 128);
+  if (tiles > PT_QUANT_LINEAR_MAX_TILES) {
+    if (int rc = pt_quant_blockwise_transpose_batched(w, dtype, 1, N, K, N * K, ldw, w_fp8, w_scale, w_t_fp8, w_t_scale, stream)) return rc;
+    return pt_quant_rowwise_blockwise_transpose_ld(x, dtype, M, K, ldx, tok_fp8, tok_scale, blk_t_fp8, ld_t, blk_t_scale, stream);
+  }
+  QuantLinearArgs q;
+  if (int rc = fill_blockwise(q.w, w, dtype, 1, N, K, N * K, ldw, w_fp8, N * K, w_scale, cdiv(N, 128) * cdiv(K, 128))) return rc;
+  q.w.b_out = (uint8_t*)w_t_fp8; q.w.b_scale = w_t_scale;
+  q.w.vec_out_t = q.w.vec_out_t && ((uintptr_t)w_t_fp8) % 16 == 0;
+  fill_common(q.x, x, dtype, M, K, ldx);
+  q.x.a_out = (uint8_t*)tok_fp8; q.x.a_scale = tok_scale; q.x.b_out = (uint8_t*)blk_t_fp8; q.x.b_scale = blk_t_scale;
+  q.x.ld_t = ld_t;
+  q.x.vec_out_t = whole_chunks(M, ld_t, blk_t_fp8);
+  q.weight_tiles = (int)weight_tiles;
+  const dim3 grid((unsigned)tiles), block(256);
+  if (dtype == PT_BF16) hipLaunchKernelGGL(quant_linear_kernel<bf16_tag>, grid, block, 0, (hipStream_t)stream, q);
+  else if (dtype == PT_F32) hipLaunchKernelGGL(quant_linear_kernel<float>, grid, block, 0, (hipStream_t)stream, q);
+  else PT_REQUIRE(false, "quant_linear_operands: unsupported dtype %d (bf16 and fp32 only)", dtype);
+  return check_launch("quant_linear_kernel");
 }
 
 // ---- SwiGLU fused into the activation quantisation --------------------------------------------

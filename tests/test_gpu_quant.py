@@ -313,3 +313,26 @@ def test_blockwise_batched_without_the_twin_is_the_first_half_of_the_transposing
         parts = (w[:, : N // 2].contiguous(), w[:, N // 2 :].contiguous())
         cat = D.fp8cast_blockwise_transpose_batched_cat(parts, twin=False)
         assert cat[2] is None and torch.equal(cat[0].view(torch.uint8), full[0].view(torch.uint8)) and torch.equal(cat[1], full[1])
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (130, 200, 144), (129, 128, 1003), (1001, 512, 2048), (4096, 1024, 4096)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_weight_and_input_of_a_linear_in_one_launch(M, N, K, dtype):
+    """One tile each, ragged edges both ways, widths without vector accesses, and more tiles than one launch
+    takes: the bits of the two quantisers on their own."""
+    from pith_train_amd import _lib
+    from pith_train_amd.operators import deepgemm_quantize as DQ
+
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn((M, K), generator=g).to(dtype).cuda()
+    w = (torch.randn((N, K), generator=g) * 0.02).to(dtype).cuda()
+    want = (*DQ.fp8cast_rowwise_blockwise_transpose(x, _padded=True), *DQ.fp8cast_blockwise_transpose(w))
+    ld_t = DQ.transposed_pitch(M)
+    got = [torch.zeros((K, ld_t) if i == 2 else t.shape, dtype=torch.uint8 if t.element_size() == 1 else t.dtype, device="cuda")
+           for i, t in enumerate(want)]
+    at = [t.data_ptr() for t in got]
+    _lib.call("pt_quant_linear_operands", x.data_ptr(), w.data_ptr(), _lib.dtype_code(dtype), M, N, K, K, K, at[0], at[1], at[2], ld_t, *at[3:],
+              _lib.stream_ptr(x.device))
+    for i, (a, b) in enumerate(zip(got, want)):
+        b = b.view(torch.uint8) if b.element_size() == 1 else b
+        assert torch.equal(a[:, :M] if i == 2 else a, b), i
