@@ -95,6 +95,17 @@ int pt_silu_mul_bwd_quant_rowwise_colwise(const void* grad_h, int64_t ld_grad_h,
                                           int64_t half, void* tok_fp8, float* tok_scale,
                                           void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows,
                                           pt_stream_t stream);
+/* The same pair in the scalings of the dense linears, for any M: forward h as
+ * pt_quant_rowwise_blockwise_transpose_ld (blk_t_fp8 and blk_t_scale may both be NULL), backward
+ * [dgate | dup] as pt_quant_rowwise_transpose_ld, half a multiple of 128. */
+int pt_silu_mul_quant_rowwise_blockwise_transpose_ld(const void* gate_up, int64_t M, int64_t half,
+                                                     int64_t ld_gate_up, void* tok_fp8, float* tok_scale,
+                                                     void* blk_t_fp8, int64_t ld_t, float* blk_t_scale,
+                                                     pt_stream_t stream);
+int pt_silu_mul_bwd_quant_rowwise_transpose_ld(const void* grad_h, int64_t ld_grad_h, const void* gate_up,
+                                               int64_t ld_gate_up, int64_t M, int64_t half, void* tok_fp8,
+                                               float* tok_scale, void* t_fp8, int64_t ld_t, float* t_scale,
+                                               pt_stream_t stream);
 /* The same pair for the clamped SwiGLU of GPT-OSS (interleaved (gate, up) pairs, alpha, limit):
  * quantises h = clamped_swiglu(gate_up[M,2*half]) (clamped_swiglu.py:18-46) as
  * fp8cast_rowwise_colwise (deepgemm_quantize.py:204-259) would, without writing h:
@@ -150,10 +161,21 @@ int pt_quant_rowwise_blockwise_transpose_ld(const void* x, int dtype, int64_t M,
                                             void* blk_t_fp8, int64_t ld_t, float* blk_t_scale,
                                             pt_stream_t stream);
 
-/* pt_quant_rowwise_blockwise_transpose_ld of x [M, K] and pt_quant_blockwise_transpose_batched of one weight
- * w [N, K], both in dtype (bf16 or fp32), with one launch while they have up to
- * PT_QUANT_LINEAR_MAX_TILES 128 x 128 tiles together. */
-#define PT_QUANT_LINEAR_MAX_TILES 1024
+/* pt_quant_rowwise_blockwise_transpose_ld of x [M, K] and pt_quant_blockwise_transpose_batched of up to
+ * PT_QUANT_DENSE_MAX weights, all in dtype (bf16 or fp32): one launch, or two when x has more than
+ * PT_QUANT_DENSE_INPUT_TILES 128 x 128 tiles.  fp8_t and scale_t of a weight have row pitches t_ld and
+ * scale_t_ld (weights side by side in one transposed operand).  blk_t_fp8 and blk_t_scale may both be NULL. */
+#define PT_QUANT_DENSE_MAX 3
+#define PT_QUANT_DENSE_INPUT_TILES 512
+typedef struct {
+  const void* w; int64_t N, K, ldw;
+  void* fp8; float* scale;
+  void* fp8_t; int64_t t_ld; float* scale_t; int64_t scale_t_ld;
+} pt_quant_dense_weight;
+int pt_quant_dense_operands(const pt_quant_dense_weight* weights /* host */, int32_t n, const void* x,
+                            int dtype, int64_t M, int64_t K, int64_t ldx, void* tok_fp8, float* tok_scale,
+                            void* blk_t_fp8, int64_t ld_t, float* blk_t_scale, pt_stream_t stream);
+/* The same for one weight w [N, K]. */
 int pt_quant_linear_operands(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K,
                              int64_t ldx, int64_t ldw, void* tok_fp8, float* tok_scale, void* blk_t_fp8,
                              int64_t ld_t, float* blk_t_scale, void* w_fp8, float* w_scale,
@@ -684,6 +706,41 @@ typedef struct {
 int64_t pt_linear_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t x_splits, int64_t w_splits,
                                            int64_t from_x);
 int pt_linear_backward(const pt_linear_backward_args* args /* host */);
+
+/* Forward of a dense SwiGLU MLP (DeepseekV2MLP, models/deepseek_v2.py:94-108), all bf16:
+ * gate_up [M, 2 half] = x [M, K] (gate | up)^T, y [M, H] = (silu(gate) * up) down^T.  The gate and up weights
+ * [half, K] are one quantised operand gu_fp8 [2 half, K] with scales [2 half / 128, K / 128] and its
+ * transposed form gu_t [K, 2 half]; down [H, half] has dn_*.  w_gate, w_up, w_down (row strides ld_*; all or
+ * none): the weights, quantised here into those operands.  x_t [K, ld_t], h_t [half, ld_t] and their scales:
+ * what the weight gradients read (all NULL: not written).  half % 128 == 0, K % 16 == 0, H % 16 == 0. */
+typedef struct {
+  const void* x; int64_t M, K, ldx, half, H;
+  const void* w_gate; int64_t ld_gate; const void* w_up; int64_t ld_up; const void* w_down; int64_t ld_down;
+  void* gu_fp8; float* gu_scale; void* gu_t; float* gu_t_scale;
+  void* dn_fp8; float* dn_scale; void* dn_t; float* dn_t_scale;
+  void* gate_up; void* y;
+  void* x_t; float* x_t_scale; void* h_t; float* h_t_scale; int64_t ld_t;
+  int64_t gu_splits, gu_split_len, dn_splits, dn_split_len;
+  void* workspace;
+  pt_stream_t stream;
+} pt_mlp_forward_args;
+int64_t pt_mlp_forward_workspace_bytes(int64_t M, int64_t K, int64_t half, int64_t H, int64_t gu_splits,
+                                       int64_t dn_splits);
+int pt_mlp_forward(const pt_mlp_forward_args* args /* host */);
+/* Its backward: grad [M, H] -> grad_x [M, K], grad_gu [2 half, K] (gate | up), grad_dn [H, half], all bf16.
+ * splits of the four GEMMs (grad_h, grad_dn, grad_x, grad_gu) as in pt_linear_backward. */
+typedef struct {
+  const void* grad; int64_t M, K, half, H, ldg;
+  const void* gu_t; const float* gu_t_scale; const void* dn_t; const float* dn_t_scale;
+  const void* gate_up;
+  const void* x_t; const float* x_t_scale; const void* h_t; const float* h_t_scale; int64_t ld_t;
+  void* grad_x; void* grad_gu; void* grad_dn;
+  int64_t splits[4], split_len[4];
+  void* workspace;
+  pt_stream_t stream;
+} pt_mlp_backward_args;
+int64_t pt_mlp_backward_workspace_bytes(int64_t M, int64_t K, int64_t half, int64_t H, const int64_t* splits /* host [4] */);
+int pt_mlp_backward(const pt_mlp_backward_args* args /* host */);
 
 /* Measurement: `fn`, when not NULL, is called on the host before (begin = 1) and after (begin = 0) every
  * entry point that the whole-step functions above run, with its name and {M, N, K} of a GEMM or

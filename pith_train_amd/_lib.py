@@ -33,6 +33,8 @@ SIGNATURES = {
     "pt_quant_rowwise_colwise_rows_repeat": (c_int, [P, I64, I64, c_int, I64, I64, I64, P, P, P, P, P, c_int, P, I32, P]),
     "pt_silu_mul_quant_rowwise_colwise": (c_int, [P, I64, I64, I64, P, P, P, P, P, P]),
     "pt_silu_mul_bwd_quant_rowwise_colwise": (c_int, [P, I64, P, I64, I64, I64, P, P, P, P, P, P]),
+    "pt_silu_mul_quant_rowwise_blockwise_transpose_ld": (c_int, [P, I64, I64, I64, P, P, P, I64, P, P]),
+    "pt_silu_mul_bwd_quant_rowwise_transpose_ld": (c_int, [P, I64, P, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_clamped_swiglu_quant_rowwise_colwise": (c_int, [P, I64, I64, I64, F, F, P, P, P, P, P, P]),
     "pt_clamped_swiglu_bwd_quant_rowwise_colwise": (c_int, [P, I64, P, I64, I64, I64, F, F, P, P, P, P, P, P, P]),
     "pt_quant_rowwise_transpose": (c_int, [P, c_int, I64, I64, I64, P, P, P, P, P]),
@@ -40,6 +42,7 @@ SIGNATURES = {
     "pt_quant_rowwise_transpose_ld": (c_int, [P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_rowwise_blockwise_transpose_ld": (c_int, [P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_heads_rowwise_transpose_ld": (c_int, [P, P, I64, I64, I64, I64, P, P, P, I64, P, P]),
+    "pt_quant_dense_operands": (c_int, [c_char_p, I32, P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_linear_operands": (c_int, [P, P, c_int, I64, I64, I64, I64, I64, P, P, P, I64, P, P, P, P, P, P]),
     "pt_quant_blockwise_transpose_batched": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, P, P, P, P]),
     "pt_quant_blockwise_transpose_batched_into": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, I64, P, I64, P, I64, I64, P, I64,
@@ -104,6 +107,10 @@ SIGNATURES = {
     "pt_linear_forward": (c_int, [c_char_p]),
     "pt_linear_backward_workspace_bytes": (I64, [I64, I64, I64, I64, I64, I64]),
     "pt_linear_backward": (c_int, [c_char_p]),
+    "pt_mlp_forward_workspace_bytes": (I64, [I64, I64, I64, I64, I64, I64]),
+    "pt_mlp_forward": (c_int, [c_char_p]),
+    "pt_mlp_backward_workspace_bytes": (I64, [I64, I64, I64, I64, P]),
+    "pt_mlp_backward": (c_int, [c_char_p]),
     "pt_set_observer": (None, [P]),
     "pt_observe": (None, [c_char_p, c_int, I64, I64, I64]),
 }

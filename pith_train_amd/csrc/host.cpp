@@ -45,6 +45,10 @@ struct Library {
   PT_FN(pt_linear_forward);
   PT_FN(pt_linear_backward_workspace_bytes);
   PT_FN(pt_linear_backward);
+  PT_FN(pt_mlp_forward_workspace_bytes);
+  PT_FN(pt_mlp_forward);
+  PT_FN(pt_mlp_backward_workspace_bytes);
+  PT_FN(pt_mlp_backward);
   PT_FN(pt_gather_rows);
   PT_FN(pt_gather_rows_backward_workspace_bytes);
   PT_FN(pt_gather_rows_backward);
@@ -92,6 +96,10 @@ void init(const std::string& path) {
   PT_FN(pt_linear_forward);
   PT_FN(pt_linear_backward_workspace_bytes);
   PT_FN(pt_linear_backward);
+  PT_FN(pt_mlp_forward_workspace_bytes);
+  PT_FN(pt_mlp_forward);
+  PT_FN(pt_mlp_backward_workspace_bytes);
+  PT_FN(pt_mlp_backward);
   PT_FN(pt_gather_rows);
   PT_FN(pt_gather_rows_backward_workspace_bytes);
   PT_FN(pt_gather_rows_backward);
@@ -699,6 +707,92 @@ Tensor silu_mul(const Tensor& gate, const Tensor& up, int64_t stream) {
       gate, up);
 }
 
+// ---- dense SwiGLU MLP -------------------------------------------------------------------------------------
+struct QuantisedMlp {
+  Tensor gu, gu_s, gu_t, gu_ts, dn, dn_s, dn_t, dn_ts;  // gate | up as one operand, and down: bytes, scales and their transposed forms
+};
+
+struct MlpNode : HipNode {
+  QuantisedMlp q;
+  Tensor gate_up, x_t, x_ts, h_t, h_ts;
+  int64_t M;
+  void drop() override { gate_up = x_t = x_ts = h_t = h_ts = Tensor(); q = QuantisedMlp(); }
+  variable_list run(variable_list&& grads) override {
+    if (!grads[0].defined()) return variable_list(4);
+    const Tensor g = row_major(grads[0]);
+    const int64_t K = x_t.size(0), half = h_t.size(0), H = q.dn.size(0);
+    const auto dev = g.device();
+    Tensor gx = empty({M, K}, at::kBFloat16, dev), ggu = empty({2 * half, K}, at::kBFloat16, dev), gdn = empty({H, half}, at::kBFloat16, dev);
+    pt_mlp_backward_args a = {ptr(g), M, K, half, H, M > 1 ? g.stride(0) : H, ptr(q.gu_t), (const float*)ptr(q.gu_ts), ptr(q.dn_t),
+                              (const float*)ptr(q.dn_ts), ptr(gate_up), ptr(x_t), (const float*)ptr(x_ts), ptr(h_t), (const float*)ptr(h_ts),
+                              x_t.size(1), ptr(gx), ptr(ggu), ptr(gdn), {}, {}, nullptr, stream};
+    const int64_t red = cdiv(M, 16) * 16, shapes[4][3] = {{M, half, H}, {H, half, red}, {M, K, 2 * half}, {2 * half, K, red}};
+    for (int i = 0; i < 4; ++i) std::tie(a.splits[i], a.split_len[i]) = split_k(shapes[i][0], shapes[i][1], shapes[i][2]);
+    Tensor ws = empty({lib.pt_mlp_backward_workspace_bytes(M, K, half, H, a.splits)}, at::kByte, dev);
+    a.workspace = ptr(ws);
+    check(lib.pt_mlp_backward(&a), "pt_mlp_backward");
+    return {gx, ggu.narrow(0, 0, half), ggu.narrow(0, half, half), gdn};
+  }
+};
+
+// y = down(silu(gate(x)) * up(x)) for bf16 x [M, K]; `cached`: the eight tensors of a QuantisedMlp when the weights have been
+// quantised before, else they are quantised in the same call.  (y, those tensors), or two Nones where the
+// library does not take the shapes.
+std::pair<Maybe, std::optional<std::vector<Tensor>>> mlp(const Tensor& input, const Tensor& w_gate, const Tensor& w_up, const Tensor& w_down,
+                                                         const std::optional<std::vector<Tensor>>& cached, int64_t stream) {
+  require_cuda(input);
+  const int64_t M = input.size(0), K = input.size(1), half = w_gate.size(0), H = w_down.size(0);
+  const auto bf16 = at::kBFloat16;
+  if (input.scalar_type() != bf16 || w_gate.scalar_type() != bf16 || w_up.scalar_type() != bf16 || w_down.scalar_type() != bf16 || w_gate.dim() != 2 ||
+      w_up.sizes() != w_gate.sizes() || w_gate.size(1) != K || w_down.size(1) != half || M == 0 || half == 0 || half % 128 || K == 0 || K % 16 || H == 0 || H % 16)
+    return {std::nullopt, std::nullopt};
+  const bool keep = torch::autograd::compute_requires_grad(input, w_gate, w_up, w_down);
+  std::vector<Tensor> t;
+  auto node = keep ? make_node<MlpNode>(stream, input, w_gate, w_up, w_down) : nullptr;
+  Tensor y;
+  {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    const auto dev = input.device();
+    const int64_t N = 2 * half, nb = cdiv(N, 128), kb = cdiv(K, 128), hb = half / 128, Hb = cdiv(H, 128);
+    const Tensor x = row_major(input), wg = row_major(w_gate), wu = row_major(w_up), wd = row_major(w_down);
+    if (cached) t = *cached;
+    else t = {empty({N, K}, kFp8, dev), empty({nb, kb}, at::kFloat, dev), empty({K, N}, kFp8, dev), empty({kb, nb}, at::kFloat, dev),
+              empty({H, half}, kFp8, dev), empty({Hb, hb}, at::kFloat, dev), empty({half, H}, kFp8, dev), empty({hb, Hb}, at::kFloat, dev)};
+    TORCH_CHECK(t.size() == 8, "mlp: eight quantised tensors");
+    const int64_t ld_t = transposed_pitch(M);
+    Tensor gate_up = empty({M, N}, bf16, dev), x_t, x_ts, h_t, h_ts;
+    y = empty({M, H}, bf16, dev);
+    if (keep) {
+      x_t = empty({K, ld_t}, kFp8, dev);
+      x_ts = empty({kb, cdiv(M, 128)}, at::kFloat, dev);
+      h_t = empty({half, ld_t}, kFp8, dev);
+      h_ts = empty({hb, cdiv(M, 128)}, at::kFloat, dev);
+    }
+    const auto [gs, gl] = split_k(M, N, K);
+    const auto [ds, dl] = split_k(M, H, half);
+    Tensor ws = empty({lib.pt_mlp_forward_workspace_bytes(M, K, half, H, gs, ds)}, at::kByte, dev);
+    auto opt = [](const Tensor& v) { return v.defined() ? v.data_ptr() : nullptr; };
+    auto pitch = [](const Tensor& v) { return v.size(0) > 1 ? v.stride(0) : v.size(1); };
+    const pt_mlp_forward_args a = {ptr(x), M, K, pitch(x), half, H,
+                                   cached ? nullptr : ptr(wg), pitch(wg), cached ? nullptr : ptr(wu), pitch(wu), cached ? nullptr : ptr(wd), pitch(wd),
+                                   ptr(t[0]), (float*)ptr(t[1]), ptr(t[2]), (float*)ptr(t[3]), ptr(t[4]), (float*)ptr(t[5]), ptr(t[6]), (float*)ptr(t[7]),
+                                   ptr(gate_up), ptr(y), opt(x_t), (float*)opt(x_ts), opt(h_t), (float*)opt(h_ts), ld_t, gs, gl, ds, dl, ptr(ws),
+                                   (pt_stream_t)stream};
+    check(lib.pt_mlp_forward(&a), "pt_mlp_forward");
+    if (keep) {
+      node->q = {t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7]};
+      node->gate_up = gate_up;
+      node->x_t = x_t;
+      node->x_ts = x_ts;
+      node->h_t = h_t;
+      node->h_ts = h_ts;
+      node->M = M;
+    }
+  }
+  if (keep) torch::autograd::set_history(y, node);
+  return {y, t};
+}
+
 // ---- grouped linear ---------------------------------------------------------------------------------------
 // Row- and column-scaled FP8 forms of x [M, N], M % 128 == 0: bytes, scales, transposed bytes, their scales
 struct Quantised {
@@ -1102,6 +1196,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("split_k", &split_k);
   m.def("quant_weight", &quant_weight);
   m.def("quant_grouped_weights", &quant_grouped_weights);
+  m.def("mlp", &mlp);
   m.def("linear", &linear);
   m.def("linear_fresh", &linear_fresh);
   m.def("linear_heads_forward", &linear_heads_forward);

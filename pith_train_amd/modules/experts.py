@@ -19,12 +19,14 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from .. import _lib
 from ..dualpipe_utils import FP8WeightCacheControl
 from ..operators import fused_experts
 from ..operators.clamped_swiglu import clamped_swiglu
 from ..operators.deepgemm_quantize import fp8cast_grouped_weight, fp8cast_grouped_weight_cat, fp8cast_grouped_weights, weight_twin_enabled
 from ..operators.grouped_linear import FP8GroupedLinear, FP8GroupedLinearFunc, GroupedLinearFunc
 from ..operators.indexed_bias_add import indexed_bias_add
+from ..operators.linear import FP8Linear
 from ..operators.silu_mul import silu_mul, silu_mul_halves
 from ..operators.token_scatter import (
     group_indices,
@@ -140,9 +142,31 @@ class DeepSeekV2MLP(nn.Module):
         self.gate_proj = training.Linear(hidden_size, intermediate_size, bias=False)
         self.up_proj = training.Linear(hidden_size, intermediate_size, bias=False)
         self.down_proj = training.Linear(intermediate_size, hidden_size, bias=False)
+        self._q_cache = None  # the quantised weights of the one-node path, once per FP8WeightCacheControl version
+        self._q_version = -1
+
+    def _one_node(self, x: torch.Tensor):
+        """The layer as one autograd node (gate and up as one fused operand, the SwiGLU and its gradient inside the
+        quantisers), or None: not three plain FP8 linears, or shapes and types that the node does not take."""
+        weights = []
+        for m in self._modules.values():
+            if (type(m) is not FP8Linear or m.bias is not None or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                    or m._backward_pre_hooks):
+                return None
+            weights.append(_weight(m))
+        if len(weights) != 3 or x.dtype != torch.bfloat16 or not x.is_cuda or x.numel() == 0 or torch.compiler.is_compiling():
+            return None
+        ver = FP8WeightCacheControl.version
+        x_2d = x if x.dim() == 2 else x.flatten(0, -2)
+        out, quantised = _lib.host().mlp(x_2d, *weights, self._q_cache if self._q_version == ver else None, _lib.stream_ptr(x.device))
+        if out is None:
+            return None
+        self._q_cache, self._q_version = quantised, ver
+        return out if x.dim() == 2 else out.view(*x.shape[:-1], out.shape[-1])
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down_proj(silu_mul(self.gate_proj(x), self.up_proj(x)))
+        out = self._one_node(x)
+        return self.down_proj(silu_mul(self.gate_proj(x), self.up_proj(x))) if out is None else out
 
 
 class Qwen35MoeExperts(nn.Module):

@@ -81,3 +81,32 @@ def test_branch_gradients_are_summed_once(dtype, T, H, k, n):
         assert ((got.double() - want).abs() <= tol * (want.abs() + 4)).all()
         if H % 8 == 0 and dtype == torch.bfloat16:
             assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("rows,hidden,width", [(1, 16, 128), (17, 144, 384), (129, 272, 128), (1000, 256, 640), (2049, 2048, 128), (4100, 512, 1408)])
+def test_mlp_as_one_node(rows, hidden, width):
+    """One row, ragged rows and widths, an input that is quantised with the weights and one that is not, split
+    reductions: the result of the three linears, their weight gradients, and the input gradient up to the
+    rounding of one addition; then again with the weights kept, and without a backward."""
+    from pith_train_amd.modules import experts as X
+    from pith_train_amd.operators.silu_mul import silu_mul
+
+    g = torch.Generator().manual_seed(rows)
+    mlp = X.DeepSeekV2MLP(hidden, width).cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        for p in mlp.parameters():
+            p.copy_((torch.randn(p.shape, generator=g) * 0.05).to(p.dtype))
+    x = torch.randn((rows, hidden), generator=g).bfloat16().cuda().requires_grad_(True)
+    dy = torch.randn((rows, hidden), generator=g).bfloat16().cuda()
+    params = list(mlp.parameters())
+    want = mlp.down_proj(silu_mul(mlp.gate_proj(x), mlp.up_proj(x)))
+    want_grads = torch.autograd.grad(want, [x, *params], dy)
+    for _ in range(2):  # weights quantised in the call, then kept
+        got = mlp(x)
+        grads = torch.autograd.grad(got, [x, *params], dy)
+        assert got.grad_fn.name() != want.grad_fn.name()
+        torch.testing.assert_close(got, want, rtol=0.01, atol=0.01 * want.float().abs().max().item())
+        for a, b in zip(grads, want_grads):
+            torch.testing.assert_close(a, b, rtol=0.01, atol=0.01 * b.float().abs().max().item())
+    with torch.no_grad():
+        assert torch.equal(mlp(x.view(1, rows, hidden))[0], got)
