@@ -62,6 +62,8 @@ struct Library {
   PT_FN(pt_moe_combine_ep_bwd);
   PT_FN(pt_router_topk_fwd);
   PT_FN(pt_router_topk_bwd);
+  PT_FN(pt_gate_linear_bwd_workspace_bytes);
+  PT_FN(pt_gate_linear_bwd);
   PT_FN(pt_dedup_workspace_bytes);
   PT_FN(pt_dedup_prepare_dispatch);
   PT_FN(pt_build_expert_idxs);
@@ -113,6 +115,8 @@ void init(const std::string& path) {
   PT_FN(pt_moe_combine_ep_bwd);
   PT_FN(pt_router_topk_fwd);
   PT_FN(pt_router_topk_bwd);
+  PT_FN(pt_gate_linear_bwd_workspace_bytes);
+  PT_FN(pt_gate_linear_bwd);
   PT_FN(pt_dedup_workspace_bytes);
   PT_FN(pt_dedup_prepare_dispatch);
   PT_FN(pt_build_expert_idxs);
@@ -1130,6 +1134,39 @@ std::pair<Tensor, Tensor> router_topk(const Tensor& input, int64_t mode, int64_t
   return {idx, weight};
 }
 
+// fp32 logits of a gate on bf16 inputs; its backward is one pass over them (csrc/gate.hip)
+struct GateLinearNode : HipNode {
+  torch::autograd::SavedVariable input, weight;
+  void drop() override { input.reset_data(); weight.reset_data(); }
+  variable_list run(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor()};
+    const Tensor x = input.unpack(), w = weight.unpack();
+    const int64_t T = x.size(0), H = x.size(1), E = w.size(0);
+    const Tensor dl = g[0].to(at::kFloat).contiguous();
+    Tensor dx = empty({T, H}, at::kBFloat16, x.device()), dw = empty({E, H}, at::kBFloat16, x.device());
+    Tensor ws = empty({lib.pt_gate_linear_bwd_workspace_bytes(T, (int32_t)E, H)}, at::kByte, x.device());
+    check(lib.pt_gate_linear_bwd((const float*)ptr(dl), ptr(x), ptr(w), ptr(dx), ptr(dw), T, (int32_t)E, H, ptr(ws), stream), "pt_gate_linear_bwd");
+    return {dx, dw};
+  }
+};
+
+// None where the backward kernel does not take the shapes and types.
+Maybe gate_linear(const Tensor& input, const Tensor& weight, int64_t stream) {
+  if (!input.is_cuda() || input.dim() != 2 || weight.dim() != 2 || input.scalar_type() != at::kBFloat16 || weight.scalar_type() != at::kBFloat16)
+    return std::nullopt;
+  const int64_t E = weight.size(0);
+  const auto plain = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)ptr(t) % 16 == 0; };
+  if (input.numel() == 0 || E % 8 || E > 256 || E == 0 || input.size(1) % 8 || input.size(1) != weight.size(1) || !plain(input) || !plain(weight))
+    return std::nullopt;
+  return with_node<GateLinearNode>(
+      stream, [&] { return at::linear(input.to(at::kFloat), weight.to(at::kFloat)); },
+      [&](GateLinearNode& n) {
+        n.input = torch::autograd::SavedVariable(input, false);
+        n.weight = torch::autograd::SavedVariable(weight, false);
+      },
+      input, weight);
+}
+
 // ---- dispatch of an expert-parallel rank --------------------------------------------------------------------
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> dedup_prepare_dispatch(const Tensor& ids, int64_t E, int64_t ep, int64_t epr, int64_t stream) {
   const int64_t m = ids.size(0), k = ids.size(1);
@@ -1196,6 +1233,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("split_k", &split_k);
   m.def("quant_weight", &quant_weight);
   m.def("quant_grouped_weights", &quant_grouped_weights);
+  m.def("gate_linear", &gate_linear);
   m.def("mlp", &mlp);
   m.def("linear", &linear);
   m.def("linear_fresh", &linear_fresh);

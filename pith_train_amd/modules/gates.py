@@ -14,6 +14,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import _lib
 from ..operators.router_topk import softmax_topk, topk_softmax
 
 
@@ -94,7 +95,11 @@ class DeepSeekV2MoEGate(_Gate):
 
     def forward(self, hidden_states: torch.Tensor):
         hidden_states = hidden_states.view(-1, hidden_states.shape[-1])
-        logits = F.linear(hidden_states.type(torch.float32), self.weight.type(torch.float32), None)
+        logits = None
+        if hidden_states.is_cuda and not torch.compiler.is_compiling():
+            logits = _lib.host().gate_linear(hidden_states, self.weight, _lib.stream_ptr(hidden_states.device))
+        if logits is None:
+            logits = F.linear(hidden_states.type(torch.float32), self.weight.type(torch.float32), None)
         limited = self.topk_method == "group_limited_greedy"
         return self._route(logits, softmax_topk, scale=self.routed_scaling_factor,
                            num_group=self.num_group if limited else 1, topk_group=self.topk_group if limited else 1)

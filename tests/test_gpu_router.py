@@ -221,3 +221,22 @@ def test_gate_modules_against_the_tensor_expressions(kind, with_lb, dtype):
     torch.testing.assert_close(xa.grad, xb.grad, rtol=1e-3, atol=1e-4 * float(xb.grad.abs().max()))
     if kind == "gpt_oss":
         torch.testing.assert_close(mod.bias.grad, bb.grad, rtol=1e-3, atol=1e-4 * float(bb.grad.abs().max()))
+
+
+@pytest.mark.parametrize("T,E,H", [(1, 8, 8), (33, 24, 136), (128, 64, 256), (129, 72, 264), (1000, 256, 512), (8192, 64, 2048)])
+def test_gate_linear_gradients(T, E, H):
+    """One token, ragged tokens, experts and columns, more than 64 experts and several token ranges, against
+    double precision; and the logits of torch's product of the fp32 copies."""
+    from pith_train_amd import _lib
+
+    g = torch.Generator().manual_seed(T + E)
+    x = torch.randn((T, H), generator=g).bfloat16().cuda().requires_grad_(True)
+    w = (torch.randn((E, H), generator=g) * 0.05).bfloat16().cuda().requires_grad_(True)
+    dl = (torch.randn((T, E), generator=g) * torch.randn((T, 1), generator=g).exp()).cuda()
+    logits = _lib.host().gate_linear(x, w, _lib.stream_ptr(x.device))
+    assert torch.equal(logits, torch.nn.functional.linear(x.detach().float(), w.detach().float()))
+    dx, dw = torch.autograd.grad(logits, [x, w], dl)
+    for got, want in ((dx, dl.double() @ w.detach().double()), (dw, dl.double().T @ x.detach().double())):
+        assert got.dtype == torch.bfloat16
+        # half a unit of bf16, plus fp32 summation error relative to the largest value
+        assert bool(((got.double() - want).abs() <= want.abs() * 2.0**-8 + 1e-5 * want.abs().max()).all())
