@@ -66,8 +66,12 @@ class _RoutedExperts(nn.Module):
         if lb_loss is not None:
             MoELoadBalanceLossTracker.add(lb_loss)
         outs = forward_stage3(self.experts, replicated, topk_idx.reshape(-1), self.experts_per_rank)
-        routed = moe_combine(outs, topk_weight).view(hidden_states.shape)
-        return routed if shared is None else routed + shared(for_shared[0].view(hidden_states.shape))
+        if shared is None:
+            return moe_combine(outs, topk_weight).view(hidden_states.shape)
+        beside = shared(for_shared[0].view(hidden_states.shape))
+        if beside.dtype == outs.dtype:  # added by the kernel that sums the experts' rows, after the same rounding
+            return moe_combine(outs, topk_weight, beside)
+        return moe_combine(outs, topk_weight).view(hidden_states.shape) + beside
 
 
 class Qwen3MoeMoE(_RoutedExperts):
