@@ -595,12 +595,12 @@ int pt_router_topk_bwd(const void* logits, int64_t ld_logits, int dtype, int64_t
                        const float* d_scores, void* d_logits, int64_t ld_dlogits,
                        pt_stream_t stream);
 
-/* Gradients of a gate whose logits are the fp32 product of bf16 x [T,H] and w [E,H] (DeepseekV2MoEGate,
- * models/deepseek_v2.py:145-147): d_x = d_logits w and d_w = d_logits^T x from fp32 d_logits [T,E], summed
- * in fp32 and rounded to bf16.  E and H multiples of 8, E <= 256. */
+/* Gradients of a gate's logits = x w^T for bf16 x [T,H] and w [E,H] (models/qwen3_moe.py:79; as an fp32 product
+ * models/deepseek_v2.py:145-147): d_x = d_logits w and d_w = d_logits^T x from d_logits [T,E] in dtype (fp32
+ * or bf16), summed in fp32 and rounded to bf16.  E and H multiples of 8, E <= 256. */
 int64_t pt_gate_linear_bwd_workspace_bytes(int64_t T, int32_t E, int64_t H);
-int pt_gate_linear_bwd(const float* d_logits, const void* x, const void* w, void* d_x, void* d_w, int64_t T,
-                       int32_t E, int64_t H, void* workspace, pt_stream_t stream);
+int pt_gate_linear_bwd(const void* d_logits, int dtype, const void* x, const void* w, void* d_x, void* d_w,
+                       int64_t T, int32_t E, int64_t H, void* workspace, pt_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------
  * Whole steps as one call: the launches of a forward or a backward are prepared and queued here

@@ -71,7 +71,7 @@ SIGNATURES = {
     "pt_router_topk_fwd": (c_int, [P, I64, c_int, I64, I32, I32, c_int, c_int, F, I32, I32, P, P, P, P, P]),
     "pt_router_topk_bwd": (c_int, [P, I64, c_int, I64, I32, I32, c_int, c_int, F, I32, I32, P, P, P, P, I64, P]),
     "pt_gate_linear_bwd_workspace_bytes": (I64, [I64, I32, I64]),
-    "pt_gate_linear_bwd": (c_int, [P, P, P, P, P, I64, I32, I64, P, P]),
+    "pt_gate_linear_bwd": (c_int, [P, c_int, P, P, P, P, I64, I32, I64, P, P]),
     "pt_compose_row_map": (c_int, [P, I64, P, I64, I64, P, P]),
     "pt_cross_entropy_fwd": (c_int, [P, I64, c_int, P, I64, I64, I64, P, P, P, P]),
     "pt_cross_entropy_bwd": (c_int, [P, I64, c_int, I64, I64, P, P]),

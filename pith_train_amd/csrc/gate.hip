@@ -1,12 +1,16 @@
-// Backward of a router gate whose logits are an fp32 product of bf16 inputs (logits = float(x) float(w)^T):
-// d_x = bf16(d_logits w) and d_w = bf16(d_logits^T x) in one pass over x.
+// Backward of a router gate: d_x = bf16(d_logits w) and d_w = bf16(d_logits^T x) in one pass over x, for bf16
+// logits and for fp32 logits of bf16 inputs (logits = float(x) float(w)^T).
 //
-// The fp32 matrix products that autograd ran for this read fp32 copies of x and wrote an fp32 d_x before its
-// conversion: 8192 tokens x 2048, 64 experts took 84 us for d_w (64 workgroups over the whole token
+// The two matrix products that autograd ran for fp32 logits read fp32 copies of x and wrote an fp32 d_x before
+// its conversion: 8192 tokens x 2048, 64 experts took 84 us for d_w (64 workgroups over the whole token
 // range), 38 us for d_x, 20 us for conversions.  What has to move is x, d_x and the small rest, 70 MB: this
-// kernel and the sum of its slabs take 36 + 11 us (block of that size: 3593 -> 3532 us).  Both products run on the bf16 matrix instructions without losing
-// anything: x and w are bf16 already, and an fp32 gradient is the exact sum of three bf16 numbers (its
-// 24 significant bits cut in three), so the products are exact and are added in fp32 as before.
+// kernel and the sum of its slabs take 36 + 11 us (block of that size: 3593 -> 3532 us).  With bf16 logits and
+// few tokens it was the host that the two library products cost: a block step on 512 tokens x 256 took 300 us
+// and takes 260.
+//
+// Both products run on the bf16 matrix instructions without losing anything: x and w are bf16 already, and an
+// fp32 gradient is the exact sum of three bf16 numbers (its 24 significant bits cut in three), so the
+// products are exact and are added in fp32 as before.
 //
 // A workgroup takes 128 columns and a range of tokens, a wave 32 tokens of it at a time:
 //   - lane (q, c) = (lane / 16, lane % 16) loads eight 16-byte pieces (columns 8c..8c+7) of eight rows, so a
@@ -25,7 +29,7 @@ typedef float gate_f32x4 __attribute__((ext_vector_type(4)));
 static constexpr int kGateCols = 128, kGateExperts = 64, kGateMaxExperts = 256;
 
 struct GateArgs {
-  const float* dl;
+  const void* dl;  // [T][E], fp32 or bf16
   const uint16_t *x, *w;
   uint16_t* dx;
   float* partial;  // [ranges][E][H]
@@ -52,27 +56,59 @@ __device__ __forceinline__ GateFrag gate_column(const uint4 (&rows)[8], int j) {
   return f;
 }
 
-// v = hi + mid + lo exactly, each with at most eight significant bits
-struct GateSplit { GateFrag hi, mid, lo; };
-__device__ __forceinline__ GateSplit gate_split(const float (&v)[8]) {
-  GateSplit s;
+// The gradients of the logits as operands.  fp32: v = hi + mid + lo exactly, each with at most eight significant
+// bits; bf16: as they are.
+template <typename D> struct GateOperand;
+template <> struct GateOperand<float> {
+  GateFrag hi, mid, lo;
+  __device__ __forceinline__ void set(const float (&v)[8]) {
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    uint32_t h[2], d[2], l[2];
+    for (int m = 0; m < 4; ++m) {
+      uint32_t h[2], d[2], l[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const float f = v[2 * m + u];
-      h[u] = __float_as_uint(f);
-      const float r = f - __uint_as_float(h[u] & 0xFFFF0000u);
-      d[u] = __float_as_uint(r);
-      l[u] = __float_as_uint(r - __uint_as_float(d[u] & 0xFFFF0000u));
+      for (int u = 0; u < 2; ++u) {
+        const float f = v[2 * m + u];
+        h[u] = __float_as_uint(f);
+        const float r = f - __uint_as_float(h[u] & 0xFFFF0000u);
+        d[u] = __float_as_uint(r);
+        l[u] = __float_as_uint(r - __uint_as_float(d[u] & 0xFFFF0000u));
+      }
+      hi.w[m] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
+      mid.w[m] = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
+      lo.w[m] = __builtin_amdgcn_perm(l[1], l[0], 0x07060302u);
     }
-    s.hi.w[m] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
-    s.mid.w[m] = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
-    s.lo.w[m] = __builtin_amdgcn_perm(l[1], l[0], 0x07060302u);
   }
-  return s;
-}
+  __device__ __forceinline__ void load_row(const float* p, bool ok) {  // eight neighbours
+    float v[8] = {};
+    if (ok) {
+      const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    }
+    set(v);
+  }
+  __device__ __forceinline__ void load_column(const float* p, int64_t pitch, int n) {  // n of eight, one per row
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = k < n ? p[k * pitch] : 0.f;
+    set(v);
+  }
+  __device__ __forceinline__ gate_f32x4 times(const GateFrag& b, gate_f32x4 c) const { return gate_mfma(hi, b, gate_mfma(mid, b, gate_mfma(lo, b, c))); }
+};
+template <> struct GateOperand<uint16_t> {
+  GateFrag v;
+  __device__ __forceinline__ void load_row(const uint16_t* p, bool ok) {
+    const uint4 u = ok ? *reinterpret_cast<const uint4*>(p) : make_uint4(0, 0, 0, 0);
+    v = {{u.x, u.y, u.z, u.w}};
+  }
+  __device__ __forceinline__ void load_column(const uint16_t* p, int64_t pitch, int n) {
+    uint32_t b[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) b[k] = k < n ? p[k * pitch] : 0u;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) v.w[m] = b[2 * m] | (b[2 * m + 1] << 16);
+  }
+  __device__ __forceinline__ gate_f32x4 times(const GateFrag& b, gate_f32x4 c) const { return gate_mfma(v, b, c); }
+};
 
 __device__ __forceinline__ void gate_rows(uint4 (&rows)[8], const uint16_t* base, int64_t row0, int64_t n_rows, int64_t H, bool col_ok) {
 #pragma unroll
@@ -80,7 +116,9 @@ __device__ __forceinline__ void gate_rows(uint4 (&rows)[8], const uint16_t* base
     rows[k] = col_ok && row0 + k < n_rows ? *reinterpret_cast<const uint4*>(base + (row0 + k) * H) : make_uint4(0, 0, 0, 0);
 }
 
+template <typename D>
 __global__ __launch_bounds__(256, 2) void gate_linear_bwd_kernel(GateArgs p) {
+  const D* dl = reinterpret_cast<const D*>(p.dl);
   extern __shared__ __attribute__((aligned(16))) uint8_t s_mem[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
   const int col_tile = blockIdx.x % p.col_tiles;
@@ -124,17 +162,13 @@ __global__ __launch_bounds__(256, 2) void gate_linear_bwd_kernel(GateArgs p) {
         for (int j = 0; j < 8; ++j) acc[j] = gate_f32x4{0.f, 0.f, 0.f, 0.f};
         for (int s = 0; s < steps; ++s) {
           const int e = 32 * s + 8 * q;
-          float v[8] = {};
-          if (token < end && e < p.E) {  // E % 8 == 0
-            const float4 a = reinterpret_cast<const float4*>(p.dl + token * p.E + e)[0], b = reinterpret_cast<const float4*>(p.dl + token * p.E + e)[1];
-            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-          }
-          const GateSplit g = gate_split(v);
+          GateOperand<D> g;
+          g.load_row(dl + token * p.E + e, token < end && e < p.E);  // E % 8 == 0
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
             const uint4 u = s_w[(s * 8 + j) * 64 + lane];
             const GateFrag f = {{u.x, u.y, u.z, u.w}};
-            acc[j] = gate_mfma(g.hi, f, gate_mfma(g.mid, f, gate_mfma(g.lo, f, acc[j])));
+            acc[j] = g.times(f, acc[j]);
           }
         }
 #pragma unroll
@@ -152,12 +186,12 @@ __global__ __launch_bounds__(256, 2) void gate_linear_bwd_kernel(GateArgs p) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int e = e0 + 16 * i + c;
-      float v[8];
+      const int64_t row = t0 + 8 * q;
+      const int n = e >= p.E || row >= end ? 0 : end - row < 8 ? (int)(end - row) : 8;
+      GateOperand<D> g;
+      g.load_column(dl + row * p.E + e, p.E, n);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = e < p.E && t0 + 8 * q + k < end ? p.dl[(t0 + 8 * q + k) * p.E + e] : 0.f;
-      const GateSplit g = gate_split(v);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) dw[i][j] = gate_mfma(g.hi, fx[j], gate_mfma(g.mid, fx[j], gate_mfma(g.lo, fx[j], dw[i][j])));
+      for (int j = 0; j < 8; ++j) dw[i][j] = g.times(fx[j], dw[i][j]);
     }
   }
 
@@ -203,7 +237,7 @@ extern "C" int64_t pt_gate_linear_bwd_workspace_bytes(int64_t T, int32_t E, int6
   return 4 * cdiv(T, gate_range(T, E, H)) * E * H;
 }
 
-extern "C" int pt_gate_linear_bwd(const float* d_logits, const void* x, const void* w, void* d_x, void* d_w, int64_t T, int32_t E, int64_t H,
+extern "C" int pt_gate_linear_bwd(const void* d_logits, int dtype, const void* x, const void* w, void* d_x, void* d_w, int64_t T, int32_t E, int64_t H,
                                   void* workspace, pt_stream_t stream) {
   PT_REQUIRE(T > 0 && E > 0 && H > 0 && E % 8 == 0 && E <= kGateMaxExperts && H % 8 == 0,
              "gate_linear_bwd: %d experts and a width of %lld: both multiples of 8, at most %d experts", E, (long long)H, kGateMaxExperts);
@@ -216,8 +250,11 @@ extern "C" int pt_gate_linear_bwd(const float* d_logits, const void* x, const vo
   const int64_t ranges = cdiv(T, a.range);
   PT_REQUIRE(ranges * a.col_tiles < (1ll << 31), "gate_linear_bwd: too many tokens");
   const int weights = (int)cdiv(E, 32) * 8 * 64 * 16, sums = kGateExperts * kGateCols * 4;
-  hipLaunchKernelGGL(gate_linear_bwd_kernel, dim3((unsigned)(ranges * a.col_tiles), (unsigned)cdiv(E, kGateExperts)), dim3(256),
-                     weights > sums ? weights : sums, (hipStream_t)stream, a);
+  const dim3 grid((unsigned)(ranges * a.col_tiles), (unsigned)cdiv(E, kGateExperts)), block(256);
+  const int lds = weights > sums ? weights : sums;
+  if (dtype == PT_F32) hipLaunchKernelGGL(gate_linear_bwd_kernel<float>, grid, block, lds, (hipStream_t)stream, a);
+  else if (dtype == PT_BF16) hipLaunchKernelGGL(gate_linear_bwd_kernel<uint16_t>, grid, block, lds, (hipStream_t)stream, a);
+  else PT_REQUIRE(false, "gate_linear_bwd: unsupported dtype %d (fp32 and bf16 only)", dtype);
   if (int rc = check_launch("gate_linear_bwd_kernel")) return rc;
   return pt_sum_partials(a.partial, (int32_t)ranges, (int64_t)E * H, d_w, PT_BF16, stream);
 }

@@ -1134,7 +1134,7 @@ std::pair<Tensor, Tensor> router_topk(const Tensor& input, int64_t mode, int64_t
   return {idx, weight};
 }
 
-// fp32 logits of a gate on bf16 inputs; its backward is one pass over them (csrc/gate.hip)
+// logits of a gate on bf16 inputs, bf16 or as the product of fp32 copies; the backward is one pass over them (csrc/gate.hip)
 struct GateLinearNode : HipNode {
   torch::autograd::SavedVariable input, weight;
   void drop() override { input.reset_data(); weight.reset_data(); }
@@ -1142,16 +1142,16 @@ struct GateLinearNode : HipNode {
     if (!g[0].defined()) return {Tensor(), Tensor()};
     const Tensor x = input.unpack(), w = weight.unpack();
     const int64_t T = x.size(0), H = x.size(1), E = w.size(0);
-    const Tensor dl = g[0].to(at::kFloat).contiguous();
+    const Tensor dl = (g[0].scalar_type() == at::kBFloat16 ? g[0] : g[0].to(at::kFloat)).contiguous();
     Tensor dx = empty({T, H}, at::kBFloat16, x.device()), dw = empty({E, H}, at::kBFloat16, x.device());
     Tensor ws = empty({lib.pt_gate_linear_bwd_workspace_bytes(T, (int32_t)E, H)}, at::kByte, x.device());
-    check(lib.pt_gate_linear_bwd((const float*)ptr(dl), ptr(x), ptr(w), ptr(dx), ptr(dw), T, (int32_t)E, H, ptr(ws), stream), "pt_gate_linear_bwd");
+    check(lib.pt_gate_linear_bwd(ptr(dl), dtype_code(dl.scalar_type()), ptr(x), ptr(w), ptr(dx), ptr(dw), T, (int32_t)E, H, ptr(ws), stream), "pt_gate_linear_bwd");
     return {dx, dw};
   }
 };
 
 // None where the backward kernel does not take the shapes and types.
-Maybe gate_linear(const Tensor& input, const Tensor& weight, int64_t stream) {
+Maybe gate_linear(const Tensor& input, const Tensor& weight, bool fp32, int64_t stream) {
   if (!input.is_cuda() || input.dim() != 2 || weight.dim() != 2 || input.scalar_type() != at::kBFloat16 || weight.scalar_type() != at::kBFloat16)
     return std::nullopt;
   const int64_t E = weight.size(0);
@@ -1159,7 +1159,7 @@ Maybe gate_linear(const Tensor& input, const Tensor& weight, int64_t stream) {
   if (input.numel() == 0 || E % 8 || E > 256 || E == 0 || input.size(1) % 8 || input.size(1) != weight.size(1) || !plain(input) || !plain(weight))
     return std::nullopt;
   return with_node<GateLinearNode>(
-      stream, [&] { return at::linear(input.to(at::kFloat), weight.to(at::kFloat)); },
+      stream, [&] { return fp32 ? at::linear(input.to(at::kFloat), weight.to(at::kFloat)) : at::linear(input, weight); },
       [&](GateLinearNode& n) {
         n.input = torch::autograd::SavedVariable(input, false);
         n.weight = torch::autograd::SavedVariable(weight, false);

@@ -64,6 +64,17 @@ class _Gate(nn.Module):
         return self._finish(res[0], res[1], res[2] if want else None)
 
 
+    def _logits(self, hidden_states: torch.Tensor, fp32: bool = False) -> torch.Tensor:
+        """``F.linear`` without a bias (``fp32``: on fp32 copies), for bf16 inputs with a backward of its own that
+        makes both gradients in one pass."""
+        weight = self._parameters["weight"]
+        if hidden_states.is_cuda and not torch.compiler.is_compiling():
+            logits = _lib.host().gate_linear(hidden_states, weight, fp32, _lib.stream_ptr(hidden_states.device))
+            if logits is not None:
+                return logits
+        return F.linear(hidden_states.type(torch.float32), weight.type(torch.float32)) if fp32 else F.linear(hidden_states, weight)
+
+
 class Qwen3MoeGate(_Gate):
     def __init__(self, num_experts: int, hidden_size: int, num_experts_per_tok: int, norm_topk_prob: bool = True):
         super().__init__(num_experts, hidden_size, num_experts_per_tok)
@@ -71,7 +82,7 @@ class Qwen3MoeGate(_Gate):
 
     def forward(self, hidden_states: torch.Tensor):
         hidden_states = hidden_states.view(-1, hidden_states.shape[-1])
-        logits = F.linear(hidden_states, self.weight, None)
+        logits = self._logits(hidden_states)
         return self._route(logits, softmax_topk, norm_topk_prob=self.norm_topk_prob)
 
 
@@ -95,11 +106,7 @@ class DeepSeekV2MoEGate(_Gate):
 
     def forward(self, hidden_states: torch.Tensor):
         hidden_states = hidden_states.view(-1, hidden_states.shape[-1])
-        logits = None
-        if hidden_states.is_cuda and not torch.compiler.is_compiling():
-            logits = _lib.host().gate_linear(hidden_states, self.weight, _lib.stream_ptr(hidden_states.device))
-        if logits is None:
-            logits = F.linear(hidden_states.type(torch.float32), self.weight.type(torch.float32), None)
+        logits = self._logits(hidden_states, fp32=True)
         limited = self.topk_method == "group_limited_greedy"
         return self._route(logits, softmax_topk, scale=self.routed_scaling_factor,
                            num_group=self.num_group if limited else 1, topk_group=self.topk_group if limited else 1)

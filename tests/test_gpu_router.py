@@ -224,17 +224,19 @@ def test_gate_modules_against_the_tensor_expressions(kind, with_lb, dtype):
 
 
 @pytest.mark.parametrize("T,E,H", [(1, 8, 8), (33, 24, 136), (128, 64, 256), (129, 72, 264), (1000, 256, 512), (8192, 64, 2048)])
-def test_gate_linear_gradients(T, E, H):
+@pytest.mark.parametrize("fp32", [True, False])
+def test_gate_linear_gradients(T, E, H, fp32):
     """One token, ragged tokens, experts and columns, more than 64 experts and several token ranges, against
-    double precision; and the logits of torch's product of the fp32 copies."""
+    double precision; and the logits of torch's product."""
     from pith_train_amd import _lib
 
     g = torch.Generator().manual_seed(T + E)
     x = torch.randn((T, H), generator=g).bfloat16().cuda().requires_grad_(True)
     w = (torch.randn((E, H), generator=g) * 0.05).bfloat16().cuda().requires_grad_(True)
-    dl = (torch.randn((T, E), generator=g) * torch.randn((T, 1), generator=g).exp()).cuda()
-    logits = _lib.host().gate_linear(x, w, _lib.stream_ptr(x.device))
-    assert torch.equal(logits, torch.nn.functional.linear(x.detach().float(), w.detach().float()))
+    kind = torch.float32 if fp32 else torch.bfloat16
+    dl = (torch.randn((T, E), generator=g) * torch.randn((T, 1), generator=g).exp()).cuda().to(kind)
+    logits = _lib.host().gate_linear(x, w, fp32, _lib.stream_ptr(x.device))
+    assert torch.equal(logits, torch.nn.functional.linear(x.detach().to(kind), w.detach().to(kind)))
     dx, dw = torch.autograd.grad(logits, [x, w], dl)
     for got, want in ((dx, dl.double() @ w.detach().double()), (dw, dl.double().T @ x.detach().double())):
         assert got.dtype == torch.bfloat16
