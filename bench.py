@@ -360,7 +360,7 @@ def hbm_kernel_report(H, I, E, rows, eidx, top_k=8, kind="fused", extras=None):
     from pith_train_amd.operators import token_scatter as TS
     from pith_train_amd.operators.silu_mul import silu_mul_halves
 
-    def timeit(fn, iters=10):
+    def timeit(fn, iters=10, graph=True):
         for _ in range(2):
             fn()
         torch.cuda.synchronize()
@@ -371,7 +371,9 @@ def hbm_kernel_report(H, I, E, rows, eidx, top_k=8, kind="fused", extras=None):
         b.record()
         torch.cuda.synchronize()
         us = a.elapsed_time(b) / iters * 1e3
-        if us >= 30.0:
+        # (graph=False: an autograd backward runs on the stream of its forward, here the default stream, which
+        # must not be made to wait for the capturing one)
+        if us >= 30.0 or not graph:
             return us
         # A call this short is bound by the host's launch path when timed in a Python loop: record
         # 25 calls into a HIP graph and time replays, i.e. 100 back-to-back launches on the device.
@@ -436,14 +438,14 @@ def hbm_kernel_report(H, I, E, rows, eidx, top_k=8, kind="fused", extras=None):
     gur = gu.clone().requires_grad_(True)
     rep("silu_mul_2d_kernel fwd [Mp,I]", timeit(lambda: silu_mul_halves(gur)), Mp * I * 6)
     o = silu_mul_halves(gur)
-    rep("silu_mul_2d_kernel bwd [Mp,I]", timeit(lambda: torch.autograd.grad(o, gur, dh, retain_graph=True)), Mp * I * 10)
+    rep("silu_mul_2d_kernel bwd [Mp,I]", timeit(lambda: torch.autograd.grad(o, gur, dh, retain_graph=True), graph=False), Mp * I * 10)
     del gu, dh, gur, o
     pbuf = torch.empty((src_of.shape[0], H), device="cuda", dtype=torch.bfloat16)
     rep("permute_rows_kernel alone (row copy of the scatter, indices given) [rows,H]",
         timeit(lambda: TS.permute_rows(src, src_of, pbuf, offs[E - 1:])), (rows + Mp) * H * 2 + 4 * src_of.shape[0])
     del pbuf
     rep("group_rows + permute_rows_kernel + host copy of the group sizes (scatter_for_grouped_gemm) [rows,H]",
-        timeit(lambda: TS.scatter_for_grouped_gemm(src, eidx, E)), (rows + Mp) * H * 2 + 16 * rows)
+        timeit(lambda: TS.scatter_for_grouped_gemm(src, eidx, E), graph=False), (rows + Mp) * H * 2 + 16 * rows)
     rep("gather_rows_kernel (padded_index_gather) [rows,H]", timeit(lambda: TS.padded_index_gather(xp, reverse)),
         2 * rows * H * 2 + 8 * rows)
     rep("gb_* kernels (padded_index_gather backward) [rows,H]",
@@ -458,7 +460,7 @@ def hbm_kernel_report(H, I, E, rows, eidx, top_k=8, kind="fused", extras=None):
     twg = tw.clone().requires_grad_(True)
     rep("moe_combine_fwd_kernel [T,k,H]", timeit(lambda: moe_combine(srcg, twg, res)), (rows + 2 * T) * H * 2 + 4 * rows)
     o = moe_combine(srcg, twg, res)
-    rep("moe_combine_bwd_kernel [T,k,H]", timeit(lambda: torch.autograd.grad(o, [srcg, twg], res, retain_graph=True)),
+    rep("moe_combine_bwd_kernel [T,k,H]", timeit(lambda: torch.autograd.grad(o, [srcg, twg], res, retain_graph=True), graph=False),
         (2 * rows + T) * H * 2 + 8 * rows)
     # the expert-parallel branch of the same step: rows arrive in the dispatch sort's order
     from pith_train_amd.operators.moe_combine import moe_combine_ep
@@ -468,20 +470,25 @@ def hbm_kernel_report(H, I, E, rows, eidx, top_k=8, kind="fused", extras=None):
         (rows + 2 * T) * H * 2 + 20 * rows)
     o = moe_combine_ep(srcg, local_idxs, twg, res)
     rep("moe_combine_bwd_kernel, rows through the slot index [T,k,H]",
-        timeit(lambda: torch.autograd.grad(o, [srcg, twg], res, retain_graph=True)), (2 * rows + T) * H * 2 + 12 * rows)
+        timeit(lambda: torch.autograd.grad(o, [srcg, twg], res, retain_graph=True), graph=False), (2 * rows + T) * H * 2 + 12 * rows)
     del srcg, twg, o, res, tw, local_idxs
     # the step before the path: softmax / top-k / weights of the router gate (after its logits GEMM)
+    from pith_train_amd import _lib
     from pith_train_amd.operators.router_topk import softmax_topk, topk_softmax
 
     lg = (torch.randn((T, E), device="cuda", generator=g) * 2).bfloat16().requires_grad_(True)
     route = (lambda: topk_softmax(lg, top_k)) if kind == "gpt_oss" else (lambda: softmax_topk(lg, top_k, norm_topk_prob=True))
     rep("router_topk_fwd_kernel [T,E] -> [T,k]", timeit(route), T * E * 2 + T * top_k * 12)
-    o = route()[1]
-    rep("router_topk_bwd_kernel [T,k] -> [T,E]", timeit(lambda: torch.autograd.grad(o, lg, o.detach(), retain_graph=True)),
+    lg = lg.detach()
+    chosen, weight = route()
+    d_lg = torch.empty_like(lg)
+    mode, norm = (1, 0) if kind == "gpt_oss" else (0, 1)
+    rep("router_topk_bwd_kernel [T,k] -> [T,E]",
+        timeit(lambda: _lib.call("pt_router_topk_bwd", lg.data_ptr(), E, _lib.dtype_code(lg.dtype), T, E, top_k, mode, norm, 1.0, 1, 1,
+                                 chosen.data_ptr(), weight.data_ptr(), None, d_lg.data_ptr(), E, _lib.stream_ptr(lg.device))),
         2 * T * E * 2 + T * top_k * 12)
-    del lg, o
+    del lg, d_lg, chosen, weight
     # the loss head: in-place fused cross-entropy over a 151 936-entry vocabulary (Qwen3), 4096 rows
-    from pith_train_amd import _lib
     from pith_train_amd.operators.cross_entropy import cross_entropy
 
     Nce, Vce = 4096, 151936
@@ -509,12 +516,12 @@ def hbm_kernel_report(H, I, E, rows, eidx, top_k=8, kind="fused", extras=None):
         ob = indexed_bias_add(gu, bias, gids, offs)
         dgu = torch.randn((Mp, 2 * I), device="cuda", generator=g).bfloat16()
         rep("segment_sum_kernel (indexed_bias_add bwd: bias gradient) [Mp,2I]",
-            timeit(lambda: torch.autograd.grad(ob, bias, dgu, retain_graph=True)), Mp * 2 * I * 2 + E * 2 * I * 4)
+            timeit(lambda: torch.autograd.grad(ob, bias, dgu, retain_graph=True), graph=False), Mp * 2 * I * 2 + E * 2 * I * 4)
         del ob
         rep("clamped_swiglu_fwd_kernel [Mp,I]", timeit(lambda: clamped_swiglu(gu, 1.702, 7.0)), Mp * I * 6)
         oc = clamped_swiglu(gu, 1.702, 7.0)
         dhh = torch.randn((Mp, I), device="cuda", generator=g).bfloat16()
-        rep("clamped_swiglu_bwd_kernel [Mp,I]", timeit(lambda: torch.autograd.grad(oc, gu, dhh, retain_graph=True)), Mp * I * 10)
+        rep("clamped_swiglu_bwd_kernel [Mp,I]", timeit(lambda: torch.autograd.grad(oc, gu, dhh, retain_graph=True), graph=False), Mp * I * 10)
         gq = gu.detach()
         rep("quant_tile_kernel clamped SwiGLU fwd + quant (the step's kernel) [Mp,I]",
             timeit(lambda: FE.clamped_swiglu_quant(gq, 1.702, 7.0)), Mp * I * (4 + 2 + 2 * sc))
