@@ -151,6 +151,11 @@ int dtype_code(at::ScalarType t) {
   }
 }
 Tensor row_major(const Tensor& t) { return t.size(-1) > 0 && t.stride(-1) != 1 ? t.contiguous() : t; }
+// contiguous and on a 16-byte boundary, for kernels that take nothing else (a gradient may be a piece of a wider buffer)
+Tensor packed(const Tensor& t) {
+  const Tensor c = t.contiguous();
+  return (uintptr_t)c.data_ptr() % 16 ? c.clone() : c;
+}
 void require_cuda(const Tensor& t) {
   if (!t.is_cuda()) throw HipError("pith_train_amd operators run on the GPU only (got a tensor on " + t.device().str() + "); there is no CPU path");
 }
@@ -1047,49 +1052,48 @@ Tensor combine_ep(const Tensor& outs, const Tensor& local_idxs, const Tensor& we
 }
 
 // ---- a MoE block's branches (see moe_combine.token_branches) ------------------------------------------------
-struct BranchesNode : HipNode {
-  int64_t T, H;
-  void drop() override {}
-  variable_list run(variable_list&& g) override {
+// The branches are views of x in autograd's eyes as well: they share its version counter, so a branch that
+// something saved for its backward is found out when x is written afterwards (hidden += block(hidden)), and
+// writing to a branch is refused.  That is what torch's own function template does with views that a
+// forward returns; a node of this file would leave it out.
+struct BranchesFunction : torch::autograd::Function<BranchesFunction> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, int64_t k, int64_t n, int64_t stream) {
+    ctx->set_materialize_grads(false);
+    ctx->saved_data["stream"] = stream;
+    variable_list out;
+    out.push_back(x.unsqueeze(1).expand({-1, k, -1}));
+    for (int64_t i = 0; i < n; ++i) out.push_back(x.view_as(x));
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
     std::vector<Tensor> given;
-    bool same = H % 8 == 0 && g.size() <= 4;
+    bool same = g.size() <= 4;
     for (const Tensor& t : g)
       if (t.defined()) {
         given.push_back(t);
-        same = same && t.scalar_type() == given[0].scalar_type();
+        same = same && t.is_cuda() && t.size(-1) % 8 == 0 && t.scalar_type() == given[0].scalar_type();
       }
-    if (given.empty()) return {Tensor()};
+    if (given.empty()) return variable_list(4);
     const bool rows = g[0].defined();
-    if (!same) {
+    if (!same || at::GradMode::is_enabled()) {  // a backward that is itself differentiated adds with torch's operators
       Tensor total = rows ? g[0].sum(1) : Tensor();
       for (size_t i = 1; i < g.size(); ++i)
         if (g[i].defined()) total = total.defined() ? total + g[i] : g[i];
-      return {total};
+      return {total, Tensor(), Tensor(), Tensor()};
     }
-    for (Tensor& t : given) t = t.contiguous();
+    for (Tensor& t : given) t = packed(t);
     const void* at[3] = {};
     for (size_t i = rows, n = 0; i < given.size(); ++i) at[n++] = ptr(given[i]);
+    const int64_t T = given[0].size(0), H = given[0].size(-1);
     Tensor out = empty({T, H}, given[0].scalar_type(), given[0].device());
     check(lib.pt_sum_branches(rows ? ptr(given[0]) : nullptr, rows ? (int32_t)given[0].size(1) : 0, at[0], at[1], at[2], ptr(out), T, H,
-                              dtype_code(out.scalar_type()), stream), "pt_sum_branches");
-    return {out};
+                              dtype_code(out.scalar_type()), (pt_stream_t)ctx->saved_data["stream"].toInt()), "pt_sum_branches");
+    return {out, Tensor(), Tensor(), Tensor()};
   }
 };
 
-variable_list branches(const Tensor& x, int64_t k, int64_t n, int64_t stream) {
-  variable_list out;
-  {
-    at::AutoDispatchBelowADInplaceOrView guard;
-    const Tensor base = x.detach();
-    out.push_back(base.unsqueeze(1).expand({-1, k, -1}));
-    for (int64_t i = 0; i < n; ++i) out.push_back(x.detach());
-  }
-  auto node = make_node<BranchesNode>(stream, x);
-  node->T = x.size(0);
-  node->H = x.size(1);
-  for (Tensor& t : out) torch::autograd::set_history(t, node);
-  return out;
-}
+variable_list branches(const Tensor& x, int64_t k, int64_t n, int64_t stream) { return BranchesFunction::apply(x, k, n, stream); }
 
 // ---- router gate ------------------------------------------------------------------------------------------
 struct RouterNode : HipNode {

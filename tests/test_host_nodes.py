@@ -1,0 +1,38 @@
+"""What the C++ autograd nodes (``csrc/host.cpp``) owe a caller besides their numbers: the errors, hooks and links of
+an ordinary autograd node.  Everything here runs without a GPU: no launch is reached."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+
+def _host():
+    from pith_train_amd import _lib
+
+    return _lib.host()
+
+
+def test_input_of_a_block_written_before_its_backward_is_found_out():
+    """hidden += block(hidden): the gate saved its branch of ``hidden``, whose values are gone."""
+    x = torch.randn((6, 16), requires_grad=True)
+    w = torch.randn((4, 16), requires_grad=True)
+    hidden = x * 1.0
+    _, for_gate, _ = _host().branches(hidden, 3, 2, 0)
+    logits = F.linear(for_gate, w)
+    hidden += 100.0
+    assert for_gate._version == hidden._version
+    with pytest.raises(RuntimeError, match="inplace"):
+        torch.autograd.grad(logits.sum(), w)
+
+
+def test_a_branch_of_a_block_cannot_be_written():
+    for i in range(3):
+        branch = _host().branches(torch.randn((6, 16), requires_grad=True) * 1.0, 3, 2, 0)[i]
+        with pytest.raises(RuntimeError, match="inplace"):
+            branch += 1.0
+
+
+def test_branches_are_differentiable_twice():
+    x = torch.randn((5, 8), dtype=torch.float64, requires_grad=True)
+    assert torch.autograd.gradcheck(lambda t: _host().branches(t, 3, 2, 0), x)
+    assert torch.autograd.gradgradcheck(lambda t: [b * b for b in _host().branches(t, 3, 2, 0)], x)
