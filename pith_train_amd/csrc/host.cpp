@@ -366,6 +366,7 @@ std::tuple<Maybe, Tensor, Tensor, Tensor> group_rows(const Tensor& keys, int64_t
   check(lib.pt_group_rows((const int64_t*)ptr(keys), m, (int32_t)G, (int32_t)alignment, at + o, at + o + G, (int64_t*)ptr(reverse), at, cap,
                           bytes ? at + ws : nullptr, bytes, (pt_stream_t)stream), "pt_group_rows");
   lib.pt_observe("pt_group_rows", 0, m, G, 0);
+  at::AutoDispatchBelowADInplaceOrView separate;  // a caller that writes to one of them does not touch the others
   return {reverse, words.narrow(0, o, G), words.narrow(0, o + G, G), words.narrow(0, 0, cap)};
 }
 
@@ -533,6 +534,16 @@ struct ExpertsBackward {
 // Python objects the nodes call back into (never released: they live as long as the process)
 PyObject *g_error = nullptr, *g_store = nullptr, *g_schedule = nullptr, *g_dgrad = nullptr;
 
+// A tensor kept for the backward as autograd keeps its own: a write to it before the backward is found out, and
+// saved-tensor hooks see it.
+struct Saved {
+  torch::autograd::SavedVariable v;
+  Saved() = default;
+  Saved(const Tensor& t) : v(t, false) {}
+  Tensor get() const { return v.unpack(); }
+  void reset() { v.reset_data(); }
+};
+
 struct HipNode : torch::autograd::Node {
   pt_stream_t stream = nullptr;
   bool released = false;
@@ -613,12 +624,12 @@ Tensor scatter_sum(const Tensor& grad, const Tensor& index, int64_t rows, int64_
 }
 
 struct GatherNode : HipNode {
-  Tensor index;
+  Saved index;
   int64_t rows, alignment;
   void drop() override { index.reset(); }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor()};
-    return {scatter_sum(g[0], index, rows, alignment, (int64_t)stream)};
+    return {scatter_sum(g[0], index.get(), rows, alignment, (int64_t)stream)};
   }
 };
 
@@ -640,7 +651,7 @@ Tensor index_gather(const Tensor& input, const Tensor& index, int64_t alignment,
         return out;
       },
       [&](GatherNode& node) {
-        node.index = index;
+        node.index = Saved(index);
         node.rows = input.size(0);
         node.alignment = alignment;
       },
@@ -649,15 +660,15 @@ Tensor index_gather(const Tensor& input, const Tensor& index, int64_t alignment,
 
 // Rows grouped by expert (ScatterForGroupedGemm): the caller sorted the indices; backward: gather.
 struct PermuteNode : HipNode {
-  Tensor reverse;
-  Maybe pre;
+  Saved reverse, pre;
+  bool expanded;
   int64_t in_rows;
   void drop() override { reverse.reset(); pre.reset(); }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor()};
-    const Tensor go = g[0].contiguous();
-    Tensor grad = gather_into(go, reverse, empty({reverse.size(0), go.size(1)}, go.scalar_type(), go.device()), stream);
-    return {pre ? scatter_sum(grad, *pre, in_rows, kRowAlignment, (int64_t)stream) : grad};
+    const Tensor go = g[0].contiguous(), index = reverse.get();
+    Tensor grad = gather_into(go, index, empty({index.size(0), go.size(1)}, go.scalar_type(), go.device()), stream);
+    return {expanded ? scatter_sum(grad, pre.get(), in_rows, kRowAlignment, (int64_t)stream) : grad};
   }
 };
 
@@ -666,8 +677,9 @@ Tensor permute_rows(const Tensor& input, const Tensor& src_of, const Tensor& off
   return with_node<PermuteNode>(
       stream, [&] { return buffer.narrow(0, 0, rows); },
       [&](PermuteNode& node) {
-        node.reverse = reverse;
-        node.pre = pre;
+        node.reverse = Saved(reverse);
+        node.expanded = (bool)pre;
+        if (pre) node.pre = Saved(*pre);
         node.in_rows = input.size(0);
       },
       input);
@@ -685,11 +697,11 @@ Tensor permute_into_buffer(const Tensor& input, const Tensor& src_of, const Tens
 
 // ---- SwiGLU -----------------------------------------------------------------------------------------------
 struct SiluMulNode : HipNode {
-  torch::autograd::SavedVariable gate, up;
-  void drop() override { gate.reset_data(); up.reset_data(); }
+  Saved gate, up;
+  void drop() override { gate.reset(); up.reset(); }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor()};
-    const Tensor a = gate.unpack(), b = up.unpack();
+    const Tensor a = gate.get(), b = up.get();
     TORCH_CHECK(g[0].sizes() == a.sizes(), "grad_output shape ", g[0].sizes(), " != gate shape ", a.sizes());
     TORCH_CHECK(g[0].scalar_type() == a.scalar_type(), "grad_output dtype differs from gate's");
     TORCH_CHECK(g[0].is_contiguous(), "grad_output must be contiguous");
@@ -710,8 +722,8 @@ Tensor silu_mul(const Tensor& gate, const Tensor& up, int64_t stream) {
         return out;
       },
       [&](SiluMulNode& node) {
-        node.gate = torch::autograd::SavedVariable(gate, false);
-        node.up = torch::autograd::SavedVariable(up, false);
+        node.gate = Saved(gate);
+        node.up = Saved(up);
       },
       gate, up);
 }
@@ -982,11 +994,12 @@ Tensor experts(const Tensor& input, const Tensor& w_gate, const Maybe& w_up, con
 
 // ---- combine ----------------------------------------------------------------------------------------------
 struct CombineNode : HipNode {
-  Tensor moe, w;
+  Saved outs, weight;
   bool residual;
-  void drop() override { moe.reset(); w.reset(); }
+  void drop() override { outs.reset(); weight.reset(); }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    const Tensor moe = outs.get(), w = weight.get();
     const int64_t T = w.size(0), k = w.size(1), H = moe.size(1);
     const Tensor go = g[0].reshape({T, H}).contiguous();
     Tensor dm = empty(moe.sizes(), moe.scalar_type(), moe.device()), dw = empty({T, k}, at::kFloat, moe.device());
@@ -1012,14 +1025,15 @@ Tensor combine(const Tensor& outs, const Tensor& weight, const Maybe& residual, 
                                      dtype_code(moe.scalar_type()), (pt_stream_t)stream), "pt_moe_combine_fwd");
         return residual ? out.view(res.sizes()) : out;
       },
-      [&](CombineNode& n) { n.moe = moe.detach(); n.w = w.detach(); n.residual = (bool)residual; }, outs, weight, res);
+      [&](CombineNode& n) { n.outs = Saved(moe); n.weight = Saved(w); n.residual = (bool)residual; }, outs, weight, res);
 }
 
 struct CombineEpNode : HipNode {
-  Tensor moe, w, slots;
-  void drop() override { moe.reset(); w.reset(); slots.reset(); }
+  Saved outs, weight, slot_row;
+  void drop() override { outs.reset(); weight.reset(); slot_row.reset(); }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    const Tensor moe = outs.get(), w = weight.get(), slots = slot_row.get();
     const int64_t T = w.size(0), k = w.size(1), R = moe.size(0), H = moe.size(1);
     const Tensor go = g[0].reshape({T, H}).contiguous();
     // rows no slot points to (none when the indices are a permutation) get a zero gradient
@@ -1048,7 +1062,7 @@ Tensor combine_ep(const Tensor& outs, const Tensor& local_idxs, const Tensor& we
                                         dtype_code(moe.scalar_type()), st), "pt_moe_combine_ep_fwd");
         return out.view(residual.sizes());
       },
-      [&](CombineEpNode& n) { n.moe = moe.detach(); n.w = w.detach(); n.slots = slots; }, outs, weight, residual);
+      [&](CombineEpNode& n) { n.outs = Saved(moe); n.weight = Saved(w); n.slot_row = Saved(slots); }, outs, weight, residual);
 }
 
 // ---- a MoE block's branches (see moe_combine.token_branches) ------------------------------------------------
@@ -1097,12 +1111,13 @@ variable_list branches(const Tensor& x, int64_t k, int64_t n, int64_t stream) { 
 
 // ---- router gate ------------------------------------------------------------------------------------------
 struct RouterNode : HipNode {
-  Tensor logits, idx;
+  Saved input, choice;
   int64_t mode, k, norm, num_group, topk_group;
   double scale;
-  void drop() override { logits.reset(); idx.reset(); }
+  void drop() override { input.reset(); choice.reset(); }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor()};
+    const Tensor logits = input.get(), idx = choice.get();
     const int64_t T = logits.size(0), E = logits.size(1);
     const Tensor dw = g[0].to(at::kFloat).contiguous();
     Tensor d = empty({T, E}, logits.scalar_type(), logits.device());
@@ -1131,7 +1146,7 @@ std::pair<Tensor, Tensor> router_topk(const Tensor& input, int64_t mode, int64_t
         return w;
       },
       [&](RouterNode& n) {
-        n.logits = logits.detach(); n.idx = idx;
+        n.input = Saved(logits); n.choice = Saved(idx);
         n.mode = mode; n.k = k; n.norm = norm; n.scale = scale; n.num_group = num_group; n.topk_group = topk_group;
       },
       input);
@@ -1140,11 +1155,11 @@ std::pair<Tensor, Tensor> router_topk(const Tensor& input, int64_t mode, int64_t
 
 // logits of a gate on bf16 inputs, bf16 or as the product of fp32 copies; the backward is one pass over them (csrc/gate.hip)
 struct GateLinearNode : HipNode {
-  torch::autograd::SavedVariable input, weight;
-  void drop() override { input.reset_data(); weight.reset_data(); }
+  Saved input, weight;
+  void drop() override { input.reset(); weight.reset(); }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor()};
-    const Tensor x = input.unpack(), w = weight.unpack();
+    const Tensor x = input.get(), w = weight.get();
     const int64_t T = x.size(0), H = x.size(1), E = w.size(0);
     const Tensor dl = (g[0].scalar_type() == at::kBFloat16 ? g[0] : g[0].to(at::kFloat)).contiguous();
     Tensor dx = empty({T, H}, at::kBFloat16, x.device()), dw = empty({E, H}, at::kBFloat16, x.device());
@@ -1165,8 +1180,8 @@ Maybe gate_linear(const Tensor& input, const Tensor& weight, bool fp32, int64_t 
   return with_node<GateLinearNode>(
       stream, [&] { return fp32 ? at::linear(input.to(at::kFloat), weight.to(at::kFloat)) : at::linear(input, weight); },
       [&](GateLinearNode& n) {
-        n.input = torch::autograd::SavedVariable(input, false);
-        n.weight = torch::autograd::SavedVariable(weight, false);
+        n.input = Saved(input);
+        n.weight = Saved(weight);
       },
       input, weight);
 }
