@@ -305,6 +305,10 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
 // None where the whole-step entry points do not take the shape.
 Maybe linear(const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const Tensor& w_s, const Tensor& w_t, const Tensor& w_ts, int64_t stream) {
   require_cuda(x);
+  // the GEMM walks the weight at x's width: a wider input would be multiplied with memory past it
+  if (x.size(1) != w_fp8.size(1) || w_t.size(0) != x.size(1) || w_t.size(1) != w_fp8.size(0))
+    throw HipError("linear: an input of width " + std::to_string(x.size(1)) + " for a weight of " + std::to_string(w_fp8.size(0)) + " x " +
+                   std::to_string(w_fp8.size(1)));
   if (!linear_supported(x, w_fp8.size(0)) || !w_fp8.is_contiguous() || !w_t.is_contiguous()) return std::nullopt;
   return LinearFunction::apply(x, weight, QuantisedWeight{w_fp8, w_s, w_t, w_ts}, (const Tensor*)nullptr, stream);
 }
@@ -312,7 +316,7 @@ Maybe linear(const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const T
 // The same with a weight that has not been quantised yet: (result, its quantised forms), or two Nones.
 std::pair<Maybe, std::optional<QuantisedWeight>> linear_fresh(const Tensor& x, const Tensor& weight, int64_t stream) {
   require_cuda(x);
-  if (weight.dim() != 2 || !linear_supported(x, weight.size(0))) return {std::nullopt, std::nullopt};
+  if (weight.dim() != 2 || weight.size(1) != x.size(1) || !linear_supported(x, weight.size(0))) return {std::nullopt, std::nullopt};
   const Tensor w = row_major(weight.detach());
   const int64_t N = w.size(0), K = w.size(1), nb = cdiv(N, 128), kb = cdiv(K, 128);
   const auto dev = w.device();

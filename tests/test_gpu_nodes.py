@@ -69,3 +69,23 @@ def test_results_of_the_scatter_are_written_independently():
     ks_tensor.add_(1)
     assert offs._version == version and int(offs[-1]) == sum(ks)
     rows.sum().backward()
+
+
+@pytest.mark.parametrize("width", [272, 512, 128])
+def test_dense_linear_refuses_an_input_of_another_width(width):
+    """With the weight quantised in the call and with a kept one; the backward's operands likewise."""
+    from pith_train_amd._lib import PithTrainHipError
+    from pith_train_amd.operators import linear as L
+
+    m = L.FP8Linear(256, 128, bias=False, device="cuda", dtype=torch.bfloat16)
+    for _ in range(2):
+        with pytest.raises(PithTrainHipError, match="width"):
+            m(_randn(32, width))
+        m(_randn(32, 256)).sum().backward()
+    _, _, w_t, w_ts = m._get_quantized_weight()
+    heads = [_randn(32, 2, 32, grad=False), _randn(32, 2, 32, grad=False)]
+    with pytest.raises(PithTrainHipError, match="transposed weight"):
+        L.fp8_dgrad_wgrad_heads(*heads, w_t, w_ts, _randn(32, width, grad=False), width)
+    x_t = torch.empty((256, 32), dtype=torch.float8_e4m3fn, device="cuda")
+    with pytest.raises(PithTrainHipError, match="transposed weight"):
+        L.fp8_dgrad_wgrad(_randn(32, 128, grad=False), w_t, w_ts, x_t, w_ts, 512)
