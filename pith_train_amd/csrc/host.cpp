@@ -159,6 +159,13 @@ Tensor packed(const Tensor& t) {
 void require_cuda(const Tensor& t) {
   if (!t.is_cuda()) throw HipError("pith_train_amd operators run on the GPU only (got a tensor on " + t.device().str() + "); there is no CPU path");
 }
+// Every other operand of a call lives where its input does (undefined: not given): a kernel gets their addresses.
+void require_same_device(const Tensor& x, std::initializer_list<const Tensor*> others) {
+  require_cuda(x);
+  for (const Tensor* t : others)
+    if (t->defined() && t->device() != x.device())
+      throw HipError("pith_train_amd operators take all of their tensors on one GPU (got " + x.device().str() + " and " + t->device().str() + ")");
+}
 
 // Row pitch of a transposed operand: the rule of deepgemm_quantize.transposed_pitch.
 int64_t transposed_pitch(int64_t m) {
@@ -304,7 +311,7 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
 
 // None where the whole-step entry points do not take the shape.
 Maybe linear(const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const Tensor& w_s, const Tensor& w_t, const Tensor& w_ts, int64_t stream) {
-  require_cuda(x);
+  require_same_device(x, {&weight, &w_fp8, &w_s, &w_t, &w_ts});
   // the GEMM walks the weight at x's width: a wider input would be multiplied with memory past it
   if (x.size(1) != w_fp8.size(1) || w_t.size(0) != x.size(1) || w_t.size(1) != w_fp8.size(0))
     throw HipError("linear: an input of width " + std::to_string(x.size(1)) + " for a weight of " + std::to_string(w_fp8.size(0)) + " x " +
@@ -315,7 +322,7 @@ Maybe linear(const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const T
 
 // The same with a weight that has not been quantised yet: (result, its quantised forms), or two Nones.
 std::pair<Maybe, std::optional<QuantisedWeight>> linear_fresh(const Tensor& x, const Tensor& weight, int64_t stream) {
-  require_cuda(x);
+  require_same_device(x, {&weight});
   if (weight.dim() != 2 || weight.size(1) != x.size(1) || !linear_supported(x, weight.size(0))) return {std::nullopt, std::nullopt};
   const Tensor w = row_major(weight.detach());
   const int64_t N = w.size(0), K = w.size(1), nb = cdiv(N, 128), kb = cdiv(K, 128);
@@ -328,6 +335,7 @@ std::pair<Maybe, std::optional<QuantisedWeight>> linear_fresh(const Tensor& x, c
 // Dense linear on two per-head halves (see operators/linear.py).
 std::pair<Tensor, Tensor> linear_heads_forward(const Tensor& input, const Tensor& w_fp8, const Tensor& w_s, int64_t heads, int64_t head_a, int64_t head_b,
                                                int64_t stream) {
+  require_same_device(input, {&w_fp8, &w_s});
   const Tensor x = row_major(input);
   const int64_t m = x.size(0), k = x.size(1), n = w_fp8.size(0), na = m * heads * head_a, nb = m * heads * head_b;
   Tensor y = empty({na + nb}, at::kBFloat16, x.device());  // one allocation: the GEMM stores through one descriptor
@@ -341,6 +349,7 @@ std::pair<Tensor, Tensor> linear_heads_forward(const Tensor& input, const Tensor
 
 std::pair<Tensor, Tensor> linear_heads_backward(const Tensor& grad_a, const Tensor& grad_b, const Tensor& w_t, const Tensor& w_ts, const Tensor& input,
                                                 int64_t stream) {
+  require_same_device(input, {&grad_a, &grad_b, &w_t, &w_ts});
   const Tensor x = row_major(input);
   const int64_t m = grad_a.size(0), heads = grad_a.size(1), head_a = grad_a.size(2), head_b = grad_b.size(2), n = heads * (head_a + head_b), k = x.size(1);
   Tensor gx = empty({m, k}, at::kFloat, x.device()), gw = empty({n, k}, at::kFloat, x.device());
@@ -423,6 +432,9 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x,
                                                                 const Tensor& offs, const Tensor& gu, const Tensor& gu_s, const Tensor& dn,
                                                                 const Tensor& dn_s, int64_t half, const Maybe& gu_bias, const Maybe& dn_bias, bool scatter,
                                                                 bool clamped, double alpha, double limit, bool keep, bool few_rows, int64_t stream) {
+  const auto given = [](const Maybe& t) { return t.value_or(Tensor()); };
+  const Tensor maps[] = {given(row_map), given(expand_idx), given(gu_bias), given(dn_bias)};
+  require_same_device(x, {&offs, &gu, &gu_s, &dn, &dn_s, &maps[0], &maps[1], &maps[2], &maps[3]});
   const int64_t src_rows = x.size(0), K = x.size(1);
   const Dims d{row_map ? row_map->size(0) : src_rows, K, half, dn.size(1), dn.size(0)};
   const int64_t routed = expand_idx ? expand_idx->size(0) : src_rows * repeat;
@@ -638,8 +650,7 @@ struct GatherNode : HipNode {
 };
 
 Tensor index_gather(const Tensor& input, const Tensor& index, int64_t alignment, int64_t stream) {
-  require_cuda(input);
-  require_cuda(index);
+  require_same_device(input, {&index});
   return with_node<GatherNode>(
       stream,
       [&] {
@@ -690,6 +701,8 @@ Tensor permute_rows(const Tensor& input, const Tensor& src_of, const Tensor& off
 }
 // The row copy itself, queued before the caller waits for the group sizes.
 Tensor permute_into_buffer(const Tensor& input, const Tensor& src_of, const Tensor& offs, const Maybe& pre, int64_t stream) {
+  const Tensor index = pre.value_or(Tensor());
+  require_same_device(input, {&src_of, &offs, &index});
   at::AutoDispatchBelowADInplaceOrView guard;
   const Tensor in = row_major(input);
   Tensor buf = empty({src_of.size(0), in.size(1)}, in.scalar_type(), in.device());
@@ -716,8 +729,7 @@ struct SiluMulNode : HipNode {
 };
 
 Tensor silu_mul(const Tensor& gate, const Tensor& up, int64_t stream) {
-  require_cuda(gate);
-  require_cuda(up);
+  require_same_device(gate, {&up});
   return with_node<SiluMulNode>(
       stream,
       [&] {
@@ -765,7 +777,9 @@ struct MlpNode : HipNode {
 // library does not take the shapes.
 std::pair<Maybe, std::optional<std::vector<Tensor>>> mlp(const Tensor& input, const Tensor& w_gate, const Tensor& w_up, const Tensor& w_down,
                                                          const std::optional<std::vector<Tensor>>& cached, int64_t stream) {
-  require_cuda(input);
+  require_same_device(input, {&w_gate, &w_up, &w_down});
+  if (cached)
+    for (const Tensor& q : *cached) require_same_device(input, {&q});
   const int64_t M = input.size(0), K = input.size(1), half = w_gate.size(0), H = w_down.size(0);
   const auto bf16 = at::kBFloat16;
   if (input.scalar_type() != bf16 || w_gate.scalar_type() != bf16 || w_up.scalar_type() != bf16 || w_down.scalar_type() != bf16 || w_gate.dim() != 2 ||
@@ -875,7 +889,7 @@ struct GroupedLinearNode : HipNode {
 
 Tensor grouped_linear(const Tensor& x, const Tensor& weight, const Tensor& offs, const Tensor& w, const Tensor& w_s, const Tensor& dg, const Tensor& dg_s,
                       bool forward_layout, int64_t stream) {
-  require_cuda(x);
+  require_same_device(x, {&weight, &offs, &w, &w_s, &dg, &dg_s});
   Quantised q;
   return with_node<GroupedLinearNode>(
       stream,
@@ -959,8 +973,8 @@ typedef std::tuple<Tensor, Tensor, bool> DgradOperand;
 Tensor experts(const Tensor& input, const Tensor& w_gate, const Maybe& w_up, const Tensor& w_down, const Maybe& gu_bias, const Maybe& dn_bias,
                const Tensor& offs, const Operand& gu, const Operand& dn, const DgradOperand& gu_dg, const DgradOperand& dn_dg, const Maybe& row_map,
                const Maybe& expand_idx, bool scatter, std::optional<std::pair<double, double>> clamp, int64_t stream) {
-  require_cuda(input);
   const Tensor up = w_up.value_or(Tensor()), b0 = gu_bias.value_or(Tensor()), b1 = dn_bias.value_or(Tensor());
+  require_same_device(input, {&w_gate, &up, &w_down, &std::get<0>(gu_dg), &std::get<1>(gu_dg), &std::get<0>(dn_dg), &std::get<1>(dn_dg)});
   std::tuple<Tensor, Tensor, std::vector<Tensor>> done;
   Tensor x;
   int64_t repeat = 1;
@@ -1014,9 +1028,10 @@ struct CombineNode : HipNode {
 };
 
 Tensor combine(const Tensor& outs, const Tensor& weight, const Maybe& residual, int64_t stream) {
+  const Tensor res = residual.value_or(Tensor());
+  require_same_device(outs, {&weight, &res});
   const int64_t T = weight.size(0), k = weight.size(1), H = outs.size(1);
   Tensor moe, w;
-  const Tensor res = residual.value_or(Tensor());
   return with_node<CombineNode>(
       stream,
       [&] {
@@ -1050,6 +1065,7 @@ struct CombineEpNode : HipNode {
 };
 
 Tensor combine_ep(const Tensor& outs, const Tensor& local_idxs, const Tensor& weight, const Tensor& residual, int64_t stream) {
+  require_same_device(outs, {&local_idxs, &weight, &residual});
   const int64_t T = weight.size(0), k = weight.size(1), R = outs.size(0), H = outs.size(1);
   const auto st = (pt_stream_t)stream;
   Tensor moe, w, slots;
@@ -1175,7 +1191,7 @@ struct GateLinearNode : HipNode {
 
 // None where the backward kernel does not take the shapes and types.
 Maybe gate_linear(const Tensor& input, const Tensor& weight, bool fp32, int64_t stream) {
-  if (!input.is_cuda() || input.dim() != 2 || weight.dim() != 2 || input.scalar_type() != at::kBFloat16 || weight.scalar_type() != at::kBFloat16)
+  if (!input.is_cuda() || input.device() != weight.device() || input.dim() != 2 || weight.dim() != 2 || input.scalar_type() != at::kBFloat16 || weight.scalar_type() != at::kBFloat16)
     return std::nullopt;
   const int64_t E = weight.size(0);
   const auto plain = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)ptr(t) % 16 == 0; };
@@ -1212,6 +1228,7 @@ std::pair<Tensor, Tensor> build_expert_idxs(const Tensor& counts, int64_t ep, in
 }
 
 Tensor adjust_expand_idx(const Tensor& received, const Tensor& dedup, const Tensor& splits, int64_t stream) {
+  require_same_device(received, {&dedup, &splits});
   const Tensor r = received.contiguous(), sp = splits.contiguous();
   Tensor out = empty(r.sizes(), at::kLong, r.device());
   if (r.size(0))

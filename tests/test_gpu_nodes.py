@@ -89,3 +89,21 @@ def test_dense_linear_refuses_an_input_of_another_width(width):
     x_t = torch.empty((256, 32), dtype=torch.float8_e4m3fn, device="cuda")
     with pytest.raises(PithTrainHipError, match="transposed weight"):
         L.fp8_dgrad_wgrad(_randn(32, 128, grad=False), w_t, w_ts, x_t, w_ts, 512)
+
+
+def test_weights_and_indices_on_the_host_are_refused():
+    from pith_train_amd._lib import PithTrainHipError
+    from pith_train_amd.modules.experts import DeepSeekV2MLP, Qwen3MoeExperts, forward_stage3
+    from pith_train_amd.operators.linear import FP8Linear
+    from pith_train_amd.operators.token_scatter import scatter_for_grouped_gemm
+
+    x = _randn(32, 128)
+    for m in (DeepSeekV2MLP(128, 128).to(torch.bfloat16), FP8Linear(128, 128, bias=False, dtype=torch.bfloat16)):
+        with pytest.raises(PithTrainHipError, match="GPU"):
+            m(x)
+    keys, pre = torch.randint(0, 4, (48,), device="cuda"), torch.randint(0, 32, (48,))
+    with pytest.raises(PithTrainHipError, match="GPU"):
+        scatter_for_grouped_gemm(x, keys, 4, pre_index=pre)
+    experts = Qwen3MoeExperts(128, 128, 4).cuda().to(torch.bfloat16)
+    with pytest.raises(PithTrainHipError, match="GPU"):
+        forward_stage3(experts, x, keys, 4, expand_idx=pre)
