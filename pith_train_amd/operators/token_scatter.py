@@ -110,7 +110,8 @@ class ScatterForGroupedGemm:
         m = expert_idxs.shape[0]
         device = input_tokens.device
         if m == 0:
-            output_tokens = torch.empty((0, input_tokens.shape[1]), device=device, dtype=input_tokens.dtype)
+            # linked to the input: a collective before it runs its backward on every rank, also on those without rows
+            output_tokens = input_tokens.narrow(0, 0, 0).clone()
             reverse = torch.empty((0,), device=device, dtype=torch.int64)
             offs = torch.empty((0,), device=device, dtype=torch.int32)
             ks_tensor = torch.empty((0,), device=device, dtype=torch.int32)

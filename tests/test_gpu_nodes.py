@@ -107,3 +107,19 @@ def test_weights_and_indices_on_the_host_are_refused():
     experts = Qwen3MoeExperts(128, 128, 4).cuda().to(torch.bfloat16)
     with pytest.raises(PithTrainHipError, match="GPU"):
         forward_stage3(experts, x, keys, 4, expand_idx=pre)
+
+
+@pytest.mark.parametrize("rows", [0, 5])
+@pytest.mark.parametrize("expand", [False, True])
+@pytest.mark.parametrize("family", ["Qwen3MoeExperts", "Qwen35MoeExperts"])
+def test_a_rank_without_rows_stays_in_the_graph(rows, expand, family):
+    """The gradient of what it received is a zero tensor, so a linked all-to-all runs its backward there too."""
+    from pith_train_amd.modules import experts as X
+
+    m = getattr(X, family)(128, 128, 4).cuda().to(torch.bfloat16)
+    received = _randn(rows, 128)
+    none = torch.zeros((0,), dtype=torch.int64, device="cuda")
+    out = X.forward_stage3(m, received * 1.0, none, 4, expand_idx=none if expand else None)
+    assert out.shape == (0, 128) and out.requires_grad
+    (grad,) = torch.autograd.grad(out, received, torch.zeros_like(out))
+    assert grad.shape == received.shape and not grad.any()
