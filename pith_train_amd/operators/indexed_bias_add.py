@@ -46,7 +46,7 @@ class _IndexedBiasAdd(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, bias, group_ids, grouped_mm_offs):
         _lib.require_cuda(x, bias, group_ids)
-        ctx.bias_dtype = bias.dtype
+        ctx.bias_dtype, ctx.bias_shape = bias.dtype, bias.shape
         ctx.save_for_backward(grouped_mm_offs)
         if x.dtype != bias.dtype or x.dim() != 2 or not x.is_contiguous():
             return x + bias[group_ids]  # mixed-dtype promotion is left to torch
@@ -64,6 +64,8 @@ class _IndexedBiasAdd(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out):
         (offs,) = ctx.saved_tensors
+        if grad_out.shape[0] == 0 and offs.shape[0] == 0:  # a scatter of no rows gives no group ends
+            return grad_out, torch.zeros(ctx.bias_shape, dtype=ctx.bias_dtype, device=grad_out.device), None, None
         bias_grad = _segment_sum_along_rows(grad_out.contiguous(), offs, ctx.bias_dtype)
         return grad_out, bias_grad, None, None
 

@@ -111,7 +111,7 @@ def test_weights_and_indices_on_the_host_are_refused():
 
 @pytest.mark.parametrize("rows", [0, 5])
 @pytest.mark.parametrize("expand", [False, True])
-@pytest.mark.parametrize("family", ["Qwen3MoeExperts", "Qwen35MoeExperts"])
+@pytest.mark.parametrize("family", ["Qwen3MoeExperts", "Qwen35MoeExperts", "GptOssExperts"])
 def test_a_rank_without_rows_stays_in_the_graph(rows, expand, family):
     """The gradient of what it received is a zero tensor, so a linked all-to-all runs its backward there too."""
     from pith_train_amd.modules import experts as X
