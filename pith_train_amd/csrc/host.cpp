@@ -15,6 +15,7 @@
 #include <dlfcn.h>
 
 #include <optional>
+#include <sstream>
 
 #include "../../include/pithtrain_hip.h"
 
@@ -165,6 +166,21 @@ void require_same_device(const Tensor& x, std::initializer_list<const Tensor*> o
   for (const Tensor* t : others)
     if (t->defined() && t->device() != x.device())
       throw HipError("pith_train_amd operators take all of their tensors on one GPU (got " + x.device().str() + " and " + t->device().str() + ")");
+}
+
+// A tensor whose address goes to a kernel that derives every index from the sizes given here.
+void require_shape(const Tensor& t, at::IntArrayRef shape, at::ScalarType type, const char* what) {
+  if (t.sizes() != shape || t.scalar_type() != type || !t.is_contiguous()) {
+    std::ostringstream s;
+    s << what << ": expected a contiguous " << c10::toString(type) << " tensor of " << shape << ", got " << c10::toString(t.scalar_type()) << ' '
+      << t.sizes() << " with strides " << t.strides();
+    throw HipError(s.str());
+  }
+}
+// the FP8 bytes [G, N, K] of a grouped weight and the scales of its 128 x 128 blocks
+void require_operand(const Tensor& q, const Tensor& scale, int64_t G, int64_t N, int64_t K, const char* what) {
+  require_shape(q, {G, N, K}, kFp8, what);
+  require_shape(scale, {G, cdiv(N, 128), cdiv(K, 128)}, at::kFloat, what);
 }
 
 // Row pitch of a transposed operand: the rule of deepgemm_quantize.transposed_pitch.
@@ -438,6 +454,14 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x,
   const int64_t src_rows = x.size(0), K = x.size(1);
   const Dims d{row_map ? row_map->size(0) : src_rows, K, half, dn.size(1), dn.size(0)};
   const int64_t routed = expand_idx ? expand_idx->size(0) : src_rows * repeat;
+  if (x.scalar_type() != at::kBFloat16) throw HipError("expert block: bf16 rows only");
+  require_operand(gu, gu_s, d.G, 2 * half, K, "gate_up weight");
+  require_operand(dn, dn_s, d.G, d.H, half, "down weight");
+  require_shape(offs, {d.G}, at::kInt, "group ends");
+  if (gu_bias) require_shape(*gu_bias, {d.G, 2 * half}, x.scalar_type(), "gate_up bias");
+  if (dn_bias) require_shape(*dn_bias, {d.G, d.H}, x.scalar_type(), "down bias");
+  if (row_map) require_shape(*row_map, {d.M}, at::kInt, "row map");
+  if (expand_idx) require_shape(*expand_idx, {routed}, at::kLong, "expanding index");
   const auto dev = x.device();
   Pieces kept = d.kept(), temp = d.forward_temp((bool)expand_idx);
   if (keep) kept.allocate(dev);
@@ -894,8 +918,11 @@ Tensor grouped_linear(const Tensor& x, const Tensor& weight, const Tensor& offs,
   return with_node<GroupedLinearNode>(
       stream,
       [&] {
-        q = Quantised(x, (pt_stream_t)stream);
         const int64_t M = x.size(0), K = x.size(1), N = w.size(1), G = w.size(0);
+        require_operand(w, w_s, G, N, K, "grouped weight");
+        require_operand(dg, dg_s, G, forward_layout ? N : K, forward_layout ? K : N, "grouped weight of the input gradient");
+        require_shape(offs, {G}, at::kInt, "group ends");
+        q = Quantised(x, (pt_stream_t)stream);
         Tensor y = empty({M, N}, x.scalar_type(), x.device());
         lib.pt_observe("pt_gemm_m_grouped_nt", 1, M, N, K);
         check(lib.pt_gemm_m_grouped_nt(ptr(q.q), (const float*)ptr(q.s), ptr(w), (const float*)ptr(w_s), ptr(y), dtype_code(y.scalar_type()),
@@ -991,6 +1018,13 @@ Tensor experts(const Tensor& input, const Tensor& w_gate, const Maybe& w_up, con
         Maybe c0, c1;
         if (gu_bias) c0 = gu_bias->contiguous();
         if (dn_bias) c1 = dn_bias->contiguous();
+        const int64_t G = w_down.size(0), H = w_down.size(1), half = w_down.size(2), K = x.size(1), N = 2 * half;
+        const auto dgrad = [&](const DgradOperand& q, int64_t rows, int64_t cols, const char* what) {  // W as it is, or its transposed twin
+          if (!std::get<2>(q)) std::swap(rows, cols);
+          require_operand(std::get<0>(q), std::get<1>(q), G, rows, cols, what);
+        };
+        dgrad(gu_dg, N, K, "gate_up weight of the input gradient");
+        dgrad(dn_dg, H, half, "down weight of the input gradient");
         done = experts_forward(x, repeat, row_map, expand_idx, offs, std::get<0>(gu), std::get<1>(gu), std::get<0>(dn), std::get<1>(dn), w_down.size(2), c0,
                                c1, scatter, (bool)clamp, alpha, limit, true, false, stream);
         return std::get<0>(done);

@@ -150,6 +150,14 @@ def _prepare(x, grouped_mm_offs, row_map, expand_idx, scatter):
     return row_map, expand_idx, scatter and row_map is not None
 
 
+def _check_biases(x, w_down, biases):
+    """The GEMM stores add a row of the bias per group, addressed by the weights' sizes."""
+    G, H, half = w_down.shape
+    for bias, width in zip(biases, (2 * half, H)):
+        assert bias is None or (bias.shape == (G, width) and bias.dtype == x.dtype), (
+            f"bias must be {x.dtype} {(G, width)}, got {bias.dtype} {tuple(bias.shape)}")
+
+
 def _node(x, w_gate, w_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, expand_idx=None, scatter=True, clamp=None, biases=(None, None)):
     """The autograd node of the three functions below (``csrc/host.cpp``): the forward is one library call that
     queues every launch of it, and so is the backward but for its input gradient.  ``w_gate`` and
@@ -162,6 +170,7 @@ def _node(x, w_gate, w_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, 
     ``[T, k, K]`` view of one row per token (routed row i is token i // k).  The weight gradients go to
     ``.grad``, or to the ``WeightGradStore`` queue."""
     row_map, expand_idx, scatter = _prepare(x, grouped_mm_offs, row_map, expand_idx, scatter)
+    _check_biases(x, w_down, biases)
     M = x.shape[0] if row_map is None else row_map.shape[0]
     weights = w_gate if w_up is None else (w_gate, w_up)
     return _lib.host().experts(
@@ -186,6 +195,7 @@ def forward_only(x, w_down, grouped_mm_offs, q_gate_up, q_down, row_map=None, ex
         repeat, x = x.shape[1], x[:, 0]
     if x.stride(1) != 1:
         x = x.contiguous()
+    _check_biases(x, w_down, biases)
     if biases[0] is not None:
         biases = [b.detach().contiguous() for b in biases]
     return _lib.host().experts_forward(

@@ -123,3 +123,23 @@ def test_a_rank_without_rows_stays_in_the_graph(rows, expand, family):
     assert out.shape == (0, 128) and out.requires_grad
     (grad,) = torch.autograd.grad(out, received, torch.zeros_like(out))
     assert grad.shape == received.shape and not grad.any()
+
+
+@pytest.mark.parametrize("train", [True, False])
+def test_gpt_oss_block_refuses_biases_and_weights_of_other_shapes(train):
+    from pith_train_amd._lib import PithTrainHipError
+    from pith_train_amd.modules.experts import GptOssExperts, Qwen3MoeExperts, forward_stage3
+
+    keys = torch.randint(0, 4, (48,), device="cuda")
+
+    def refused(error, m, width=128):
+        with torch.set_grad_enabled(train), pytest.raises(error):
+            forward_stage3(m, _randn(48, width, grad=train), keys, 4)
+
+    for name, shape in (("gate_up_proj_bias", (4, 128)), ("gate_up_proj_bias", (3, 256)), ("down_proj_bias", (4, 64)), ("down_proj_bias", (1, 128))):
+        m = GptOssExperts(128, 128, 4).cuda().to(torch.bfloat16)
+        setattr(m, name, torch.nn.Parameter(torch.zeros(shape, device="cuda", dtype=torch.bfloat16)))
+        refused(AssertionError, m)
+    refused(PithTrainHipError, GptOssExperts(128, 128, 4).cuda().to(torch.bfloat16), 256)
+    refused(PithTrainHipError, Qwen3MoeExperts(128, 128, 4).cuda().to(torch.bfloat16), 256)
+    refused(PithTrainHipError, Qwen3MoeExperts(128, 128, 3).cuda().to(torch.bfloat16))
