@@ -293,61 +293,6 @@ std::tuple<Tensor, Tensor, Tensor> linear_forward(const Tensor& input, const Qua
   return {y, x_t, x_ts};
 }
 
-struct LinearFunction : torch::autograd::Function<LinearFunction> {
-  // weight is an argument for its gradient's sake; the quantised forms are what is read
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const QuantisedWeight& q, const Tensor* fresh, int64_t stream) {
-    auto [y, x_t, x_ts] = linear_forward(x, q, fresh, stream);
-    ctx->save_for_backward({std::get<2>(q), std::get<3>(q), x_t, x_ts});
-    ctx->saved_data["stream"] = stream;
-    return y;
-  }
-
-  static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const auto saved = ctx->get_saved_variables();
-    const Tensor &w_t = saved[0], &w_ts = saved[1], &x_t = saved[2], &x_ts = saved[3];
-    const Tensor g = row_major(grads[0]);
-    const int64_t m = g.size(0), n = g.size(1), k = w_t.size(0);
-    const auto dev = g.device();
-    const auto type = g.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
-    Tensor gx = empty({m, k}, type, dev), gw = empty({n, k}, type, dev);
-    const auto [xs, xl] = split_k(m, k, n);
-    const auto [ws, wl] = split_k(n, k, cdiv(m, 16) * 16);
-    Tensor work = empty({lib.pt_linear_backward_workspace_bytes(m, n, k, xs, ws, 0)}, at::kByte, dev);
-    const pt_linear_backward_args a = {ptr(g), dtype_code(g.scalar_type()), m, n, m > 1 ? g.stride(0) : n, ptr(w_t), (const float*)ptr(w_ts), k, ptr(x_t),
-                                       x_t.size(1), (const float*)ptr(x_ts), ptr(gx), ptr(gw), dtype_code(type), xs, xl, ws, wl, nullptr, 0,
-                                       nullptr, 0, 0, ptr(work), (pt_stream_t)ctx->saved_data["stream"].toInt()};
-    check(lib.pt_linear_backward(&a), "pt_linear_backward");
-    if (type != g.scalar_type()) {
-      gx = gx.to(g.scalar_type());
-      gw = gw.to(g.scalar_type());
-    }
-    return {gx, gw, Tensor(), Tensor(), Tensor()};
-  }
-};
-
-// None where the whole-step entry points do not take the shape.
-Maybe linear(const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const Tensor& w_s, const Tensor& w_t, const Tensor& w_ts, int64_t stream) {
-  require_same_device(x, {&weight, &w_fp8, &w_s, &w_t, &w_ts});
-  // the GEMM walks the weight at x's width: a wider input would be multiplied with memory past it
-  if (x.size(1) != w_fp8.size(1) || w_t.size(0) != x.size(1) || w_t.size(1) != w_fp8.size(0))
-    throw HipError("linear: an input of width " + std::to_string(x.size(1)) + " for a weight of " + std::to_string(w_fp8.size(0)) + " x " +
-                   std::to_string(w_fp8.size(1)));
-  if (!linear_supported(x, w_fp8.size(0)) || !w_fp8.is_contiguous() || !w_t.is_contiguous()) return std::nullopt;
-  return LinearFunction::apply(x, weight, QuantisedWeight{w_fp8, w_s, w_t, w_ts}, (const Tensor*)nullptr, stream);
-}
-
-// The same with a weight that has not been quantised yet: (result, its quantised forms), or two Nones.
-std::pair<Maybe, std::optional<QuantisedWeight>> linear_fresh(const Tensor& x, const Tensor& weight, int64_t stream) {
-  require_same_device(x, {&weight});
-  if (weight.dim() != 2 || weight.size(1) != x.size(1) || !linear_supported(x, weight.size(0))) return {std::nullopt, std::nullopt};
-  const Tensor w = row_major(weight.detach());
-  const int64_t N = w.size(0), K = w.size(1), nb = cdiv(N, 128), kb = cdiv(K, 128);
-  const auto dev = w.device();
-  QuantisedWeight q{empty({N, K}, kFp8, dev), empty({nb, kb}, at::kFloat, dev), empty({K, N}, kFp8, dev), empty({kb, nb}, at::kFloat, dev)};
-  Tensor y = LinearFunction::apply(x, weight, q, &w, stream);
-  return {y, q};
-}
-
 // Dense linear on two per-head halves (see operators/linear.py).
 std::pair<Tensor, Tensor> linear_heads_forward(const Tensor& input, const Tensor& w_fp8, const Tensor& w_s, int64_t heads, int64_t head_a, int64_t head_b,
                                                int64_t stream) {
@@ -575,12 +520,27 @@ struct ExpertsBackward {
 PyObject *g_error = nullptr, *g_store = nullptr, *g_schedule = nullptr, *g_dgrad = nullptr;
 
 // A tensor kept for the backward as autograd keeps its own: a write to it before the backward is found out, and
-// saved-tensor hooks see it.
+// saved-tensor hooks see it.  What a hook gives back goes to kernels by address, so it has to be what was saved.
 struct Saved {
   torch::autograd::SavedVariable v;
+  std::vector<int64_t> sizes, strides;  // with hooks only
+  at::TensorOptions options;
   Saved() = default;
-  Saved(const Tensor& t) : v(t, false) {}
-  Tensor get() const { return v.unpack(); }
+  Saved(const Tensor& t) : v(t, false) {
+    if (!v.has_hooks()) return;
+    sizes = t.sizes().vec();
+    strides = t.strides().vec();
+    options = t.options();
+  }
+  Tensor get() const {
+    const Tensor t = v.unpack();
+    if (!v.has_hooks()) return t;
+    TORCH_CHECK(t.defined() && t.sizes() == sizes && t.scalar_type() == c10::typeMetaToScalarType(options.dtype()) && t.device() == options.device(),
+                "a saved-tensor hook gave back another size, type or device than it was given");
+    if (t.strides() == strides) return t;
+    Tensor same = at::empty_strided(sizes, strides, options);
+    return same.copy_(t.detach());
+  }
   void reset() { v.reset_data(); }
 };
 
@@ -768,24 +728,90 @@ Tensor silu_mul(const Tensor& gate, const Tensor& up, int64_t stream) {
       gate, up);
 }
 
-// ---- dense SwiGLU MLP -------------------------------------------------------------------------------------
-struct QuantisedMlp {
-  Tensor gu, gu_s, gu_t, gu_ts, dn, dn_s, dn_t, dn_ts;  // gate | up as one operand, and down: bytes, scales and their transposed forms
+// ---- dense linear -----------------------------------------------------------------------------------------
+struct LinearNode : HipNode {
+  Saved weight_t, weight_ts, input_t, input_ts;
+  void drop() override { for (Saved* s : {&weight_t, &weight_ts, &input_t, &input_ts}) s->reset(); }
+  variable_list run(variable_list&& grads) override {
+    if (!grads[0].defined()) return {Tensor(), Tensor()};
+    const Tensor w_t = weight_t.get(), w_ts = weight_ts.get(), x_t = input_t.get(), x_ts = input_ts.get(), g = row_major(grads[0]);
+    const int64_t m = g.size(0), n = g.size(1), k = w_t.size(0);
+    const auto dev = g.device();
+    const auto type = g.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
+    Tensor gx = empty({m, k}, type, dev), gw = empty({n, k}, type, dev);
+    const auto [xs, xl] = split_k(m, k, n);
+    const auto [ws, wl] = split_k(n, k, cdiv(m, 16) * 16);
+    Tensor work = empty({lib.pt_linear_backward_workspace_bytes(m, n, k, xs, ws, 0)}, at::kByte, dev);
+    const pt_linear_backward_args a = {ptr(g), dtype_code(g.scalar_type()), m, n, m > 1 ? g.stride(0) : n, ptr(w_t), (const float*)ptr(w_ts), k, ptr(x_t),
+                                       x_t.size(1), (const float*)ptr(x_ts), ptr(gx), ptr(gw), dtype_code(type), xs, xl, ws, wl, nullptr, 0,
+                                       nullptr, 0, 0, ptr(work), stream};
+    check(lib.pt_linear_backward(&a), "pt_linear_backward");
+    if (type != g.scalar_type()) {
+      gx = gx.to(g.scalar_type());
+      gw = gw.to(g.scalar_type());
+    }
+    return {gx, gw};
+  }
 };
 
+// weight is an argument for its gradient's sake; the quantised forms are what is read
+Tensor linear_node(const Tensor& x, const Tensor& weight, const QuantisedWeight& q, const Tensor* fresh, int64_t stream) {
+  Tensor x_t, x_ts;
+  return with_node<LinearNode>(
+      stream,
+      [&] {
+        Tensor y;
+        std::tie(y, x_t, x_ts) = linear_forward(x, q, fresh, stream);
+        return y;
+      },
+      [&](LinearNode& node) {
+        node.weight_t = Saved(std::get<2>(q));
+        node.weight_ts = Saved(std::get<3>(q));
+        node.input_t = Saved(x_t);
+        node.input_ts = Saved(x_ts);
+      },
+      x, weight);
+}
+
+// None where the whole-step entry points do not take the shape.
+Maybe linear(const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const Tensor& w_s, const Tensor& w_t, const Tensor& w_ts, int64_t stream) {
+  require_same_device(x, {&weight, &w_fp8, &w_s, &w_t, &w_ts});
+  // the GEMM walks the weight at x's width: a wider input would be multiplied with memory past it
+  if (x.size(1) != w_fp8.size(1) || w_t.size(0) != x.size(1) || w_t.size(1) != w_fp8.size(0))
+    throw HipError("linear: an input of width " + std::to_string(x.size(1)) + " for a weight of " + std::to_string(w_fp8.size(0)) + " x " +
+                   std::to_string(w_fp8.size(1)));
+  if (!linear_supported(x, w_fp8.size(0)) || !w_fp8.is_contiguous() || !w_t.is_contiguous()) return std::nullopt;
+  return linear_node(x, weight, QuantisedWeight{w_fp8, w_s, w_t, w_ts}, nullptr, stream);
+}
+
+// The same with a weight that has not been quantised yet: (result, its quantised forms), or two Nones.
+std::pair<Maybe, std::optional<QuantisedWeight>> linear_fresh(const Tensor& x, const Tensor& weight, int64_t stream) {
+  require_same_device(x, {&weight});
+  if (weight.dim() != 2 || weight.size(1) != x.size(1) || !linear_supported(x, weight.size(0))) return {std::nullopt, std::nullopt};
+  const Tensor w = row_major(weight.detach());
+  const int64_t N = w.size(0), K = w.size(1), nb = cdiv(N, 128), kb = cdiv(K, 128);
+  const auto dev = w.device();
+  QuantisedWeight q{empty({N, K}, kFp8, dev), empty({nb, kb}, at::kFloat, dev), empty({K, N}, kFp8, dev), empty({kb, nb}, at::kFloat, dev)};
+  Tensor y = linear_node(x, weight, q, &w, stream);
+  return {y, q};
+}
+
+// ---- dense SwiGLU MLP -------------------------------------------------------------------------------------
 struct MlpNode : HipNode {
-  QuantisedMlp q;
-  Tensor gate_up, x_t, x_ts, h_t, h_ts;
+  enum { GU_T, GU_TS, DN_T, DN_TS, GATE_UP, X_T, X_TS, H_T, H_TS, COUNT };  // transposed weights, gate_up, transposed activations; scales
+  Saved kept[COUNT];
   int64_t M;
-  void drop() override { gate_up = x_t = x_ts = h_t = h_ts = Tensor(); q = QuantisedMlp(); }
+  void drop() override { for (Saved& s : kept) s.reset(); }
   variable_list run(variable_list&& grads) override {
     if (!grads[0].defined()) return variable_list(4);
-    const Tensor g = row_major(grads[0]);
-    const int64_t K = x_t.size(0), half = h_t.size(0), H = q.dn.size(0);
+    Tensor t[COUNT];
+    for (int i = 0; i < COUNT; ++i) t[i] = kept[i].get();
+    const Tensor &x_t = t[X_T], &h_t = t[H_T], g = row_major(grads[0]);
+    const int64_t K = x_t.size(0), half = h_t.size(0), H = t[DN_T].size(1);
     const auto dev = g.device();
     Tensor gx = empty({M, K}, at::kBFloat16, dev), ggu = empty({2 * half, K}, at::kBFloat16, dev), gdn = empty({H, half}, at::kBFloat16, dev);
-    pt_mlp_backward_args a = {ptr(g), M, K, half, H, M > 1 ? g.stride(0) : H, ptr(q.gu_t), (const float*)ptr(q.gu_ts), ptr(q.dn_t),
-                              (const float*)ptr(q.dn_ts), ptr(gate_up), ptr(x_t), (const float*)ptr(x_ts), ptr(h_t), (const float*)ptr(h_ts),
+    pt_mlp_backward_args a = {ptr(g), M, K, half, H, M > 1 ? g.stride(0) : H, ptr(t[GU_T]), (const float*)ptr(t[GU_TS]), ptr(t[DN_T]),
+                              (const float*)ptr(t[DN_TS]), ptr(t[GATE_UP]), ptr(x_t), (const float*)ptr(t[X_TS]), ptr(h_t), (const float*)ptr(t[H_TS]),
                               x_t.size(1), ptr(gx), ptr(ggu), ptr(gdn), {}, {}, nullptr, stream};
     const int64_t red = cdiv(M, 16) * 16, shapes[4][3] = {{M, half, H}, {H, half, red}, {M, K, 2 * half}, {2 * half, K, red}};
     for (int i = 0; i < 4; ++i) std::tie(a.splits[i], a.split_len[i]) = split_k(shapes[i][0], shapes[i][1], shapes[i][2]);
@@ -796,8 +822,8 @@ struct MlpNode : HipNode {
   }
 };
 
-// y = down(silu(gate(x)) * up(x)) for bf16 x [M, K]; `cached`: the eight tensors of a QuantisedMlp when the weights have been
-// quantised before, else they are quantised in the same call.  (y, those tensors), or two Nones where the
+// y = down(silu(gate(x)) * up(x)) for bf16 x [M, K]; `cached`: the quantised weights (gate | up as one operand, and down:
+// bytes, scales and their transposed forms, eight tensors) when there are any, else they are quantised in the same call.  (y, those tensors), or two Nones where the
 // library does not take the shapes.
 std::pair<Maybe, std::optional<std::vector<Tensor>>> mlp(const Tensor& input, const Tensor& w_gate, const Tensor& w_up, const Tensor& w_down,
                                                          const std::optional<std::vector<Tensor>>& cached, int64_t stream) {
@@ -843,12 +869,8 @@ std::pair<Maybe, std::optional<std::vector<Tensor>>> mlp(const Tensor& input, co
                                    (pt_stream_t)stream};
     check(lib.pt_mlp_forward(&a), "pt_mlp_forward");
     if (keep) {
-      node->q = {t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7]};
-      node->gate_up = gate_up;
-      node->x_t = x_t;
-      node->x_ts = x_ts;
-      node->h_t = h_t;
-      node->h_ts = h_ts;
+      const Tensor kept[MlpNode::COUNT] = {t[2], t[3], t[6], t[7], gate_up, x_t, x_ts, h_t, h_ts};
+      for (int i = 0; i < MlpNode::COUNT; ++i) node->kept[i] = Saved(kept[i]);
       node->M = M;
     }
   }
@@ -877,11 +899,13 @@ struct Quantised {
 };
 
 struct GroupedLinearNode : HipNode {
-  Tensor weight, dg, dg_s, offs, x_t, x_ts;
+  Tensor weight;  // its gradient is written to; its values are not read
+  Saved operand, operand_scale, ends, input_t, input_ts;
   bool forward_layout;
-  void drop() override { dg.reset(); dg_s.reset(); offs.reset(); x_t.reset(); x_ts.reset(); }
+  void drop() override { for (Saved* s : {&operand, &operand_scale, &ends, &input_t, &input_ts}) s->reset(); }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor()};
+    const Tensor dg = operand.get(), dg_s = operand_scale.get(), offs = ends.get(), x_t = input_t.get(), x_ts = input_ts.get();
     const Tensor go = g[0].contiguous();
     const int64_t M = go.size(0), N = go.size(1), K = x_t.size(0), G = offs.size(0);
     Quantised d(go, stream);
@@ -931,8 +955,8 @@ Tensor grouped_linear(const Tensor& x, const Tensor& weight, const Tensor& offs,
         return y;
       },
       [&](GroupedLinearNode& node) {
-        node.weight = weight; node.dg = dg; node.dg_s = dg_s; node.offs = offs;
-        node.x_t = q.q_t; node.x_ts = q.s_t; node.forward_layout = forward_layout;
+        node.weight = weight; node.operand = Saved(dg); node.operand_scale = Saved(dg_s); node.ends = Saved(offs);
+        node.input_t = Saved(q.q_t); node.input_ts = Saved(q.s_t); node.forward_layout = forward_layout;
       },
       x, weight);
 }
@@ -941,19 +965,25 @@ Tensor grouped_linear(const Tensor& x, const Tensor& weight, const Tensor& offs,
 struct ExpertsNode : HipNode {
   Dims d;
   Tensor w_gate, w_up, w_down;  // w_gate: the fused gate_up weight when w_up is not there
-  Tensor gu_dg, gu_dg_s, dn_dg, dn_dg_s, offs, gate_up;
-  Maybe row_map, expand_idx, gu_bias, dn_bias;
-  std::vector<Tensor> kept;
-  bool gu_forward, dn_forward, scatter, clamped;
+  enum { GU_DG, GU_DG_S, DN_DG, DN_DG_S, OFFS, GATE_UP, ROW_MAP, EXPAND_IDX, COUNT };
+  Saved saved[COUNT];
+  std::vector<Saved> activations;  // x^T, h^T with scales
+  Maybe gu_bias, dn_bias;
+  bool has_map, has_expand, gu_forward, dn_forward, scatter, clamped;
   double alpha, limit;
   int64_t src_rows, routed, repeat;
   void drop() override {
-    for (Tensor* t : {&gu_dg, &gu_dg_s, &dn_dg, &dn_dg_s, &offs, &gate_up}) t->reset();
-    row_map.reset(); expand_idx.reset();
-    kept.clear();
+    for (Saved& s : saved) s.reset();
+    activations.clear();
   }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    const Tensor offs = saved[OFFS].get(), gu_dg = saved[GU_DG].get(), gu_dg_s = saved[GU_DG_S].get();
+    Maybe row_map, expand_idx;
+    if (has_map) row_map = saved[ROW_MAP].get();
+    if (has_expand) expand_idx = saved[EXPAND_IDX].get();
+    std::vector<Tensor> kept;
+    for (const Saved& s : activations) kept.push_back(s.get());
     bool deferred;
     {
       py::gil_scoped_acquire gil;
@@ -964,8 +994,8 @@ struct ExpertsNode : HipNode {
       weights = {w_down, w_gate};
       if (w_up.defined()) weights.push_back(w_up);
     }
-    ExpertsBackward step(g[0], d, offs, row_map, scatter, dn_dg, dn_dg_s, dn_forward, gate_up, kept, clamped, alpha, limit, gu_bias, dn_bias, weights,
-                         (int64_t)stream);
+    ExpertsBackward step(g[0], d, offs, row_map, scatter, saved[DN_DG].get(), saved[DN_DG_S].get(), dn_forward, saved[GATE_UP].get(), std::move(kept),
+                         clamped, alpha, limit, gu_bias, dn_bias, weights, (int64_t)stream);
     Tensor gx = empty({row_map ? routed : d.M, d.K}, g[0].scalar_type(), g[0].device());
     {
       py::gil_scoped_acquire gil;
@@ -1035,10 +1065,16 @@ Tensor experts(const Tensor& input, const Tensor& w_gate, const Maybe& w_up, con
         n.routed = expand_idx ? expand_idx->size(0) : n.src_rows * repeat;
         n.d = Dims{row_map ? row_map->size(0) : n.src_rows, x.size(1), w_down.size(2), w_down.size(1), w_down.size(0)};
         n.w_gate = w_gate; n.w_up = up; n.w_down = w_down;
-        std::tie(n.gu_dg, n.gu_dg_s, n.gu_forward) = gu_dg;
-        std::tie(n.dn_dg, n.dn_dg_s, n.dn_forward) = dn_dg;
-        n.offs = offs; n.gate_up = std::get<1>(done); n.kept = std::get<2>(done);
-        n.row_map = row_map; n.expand_idx = expand_idx; n.gu_bias = gu_bias; n.dn_bias = dn_bias;
+        n.gu_forward = std::get<2>(gu_dg);
+        n.dn_forward = std::get<2>(dn_dg);
+        n.has_map = (bool)row_map;
+        n.has_expand = (bool)expand_idx;
+        const Tensor keep[] = {std::get<0>(gu_dg), std::get<1>(gu_dg), std::get<0>(dn_dg), std::get<1>(dn_dg), offs, std::get<1>(done),
+                               row_map.value_or(Tensor()), expand_idx.value_or(Tensor())};
+        for (int i = 0; i < ExpertsNode::COUNT; ++i)
+          if (keep[i].defined()) n.saved[i] = Saved(keep[i]);
+        for (const Tensor& t : std::get<2>(done)) n.activations.emplace_back(t);
+        n.gu_bias = gu_bias; n.dn_bias = dn_bias;
         n.scatter = scatter; n.clamped = (bool)clamp; n.alpha = alpha; n.limit = limit;
       },
       input, w_gate, up, w_down, b0, b1);

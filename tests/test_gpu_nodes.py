@@ -143,3 +143,71 @@ def test_gpt_oss_block_refuses_biases_and_weights_of_other_shapes(train):
     refused(PithTrainHipError, GptOssExperts(128, 128, 4).cuda().to(torch.bfloat16), 256)
     refused(PithTrainHipError, Qwen3MoeExperts(128, 128, 4).cuda().to(torch.bfloat16), 256)
     refused(PithTrainHipError, Qwen3MoeExperts(128, 128, 3).cuda().to(torch.bfloat16))
+
+
+def _hidden_activations(kind):
+    """(module call, input, bytes of the activations that the backward needs besides weights)"""
+    from pith_train_amd.modules import experts as X
+    from pith_train_amd.operators.linear import FP8Linear
+    from pith_train_amd.operators.token_scatter import scatter_for_grouped_gemm
+
+    T, H, half, E = 300, 256, 384, 4
+    if kind == "mlp":
+        m = X.DeepSeekV2MLP(H, half)
+        return m, m, T * (H + 2 * 2 * half + half)
+    if kind == "linear":
+        m = FP8Linear(H, half, bias=False)
+        return m, m, T * H
+    keys = torch.randint(0, E, (T,), device="cuda")
+    if kind == "grouped":
+        m = X.Qwen3MoeExperts(H, half, E)
+
+        def call(x):
+            rows, reverse, offs, ks, ks_t = scatter_for_grouped_gemm(x, keys, E)
+            return m.gate_proj(rows, grouped_mm_offs=offs, ks=ks, ks_tensor=ks_t)
+
+        return m, call, T * H
+    m = getattr(X, kind)(H, half, E)
+    return m, lambda x: X.forward_stage3(m, x, keys, E), T * (H + 2 * 2 * half + half)
+
+
+@pytest.mark.parametrize("kind", ["Qwen3MoeExperts", "Qwen35MoeExperts", "GptOssExperts", "grouped", "mlp", "linear"])
+def test_hooks_on_saved_tensors_see_the_activations(kind):
+    """save_on_cpu and checkpointing without re-entry can let go of what a layer keeps: same gradients, nothing of it
+    left on the GPU in between."""
+    from torch.utils.checkpoint import checkpoint
+
+    m, call, nbytes = _hidden_activations(kind)
+    m.cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.normal_(0.0, 0.05)
+    x = _randn(300, 256)
+
+    def step(forward):
+        m.zero_grad(set_to_none=True)
+        out = forward(x)
+        dy = torch.linspace(-1, 1, out.numel(), device="cuda").view(out.shape).to(out.dtype)
+        grads = torch.autograd.grad(out, [x, *m.parameters()], dy, allow_unused=True)
+        return [out.detach(), *[p.grad if g is None else g for p, g in zip([None, *m.parameters()], grads) if g is not None or p.grad is not None]]
+
+    def offloaded(x):
+        seen = []
+
+        def pack(t):
+            seen.append(t.numel() * t.element_size())
+            return t.cpu()
+
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+            out = call(x)
+        assert sum(seen) >= nbytes
+        return out
+
+    want = step(call)
+    for forward in (offloaded, lambda x: checkpoint(call, x, use_reentrant=False)):
+        got = step(forward)
+        assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.reshape(-1)[:1]):
+        out = call(x)
+    with pytest.raises(RuntimeError):
+        out.sum().backward()
