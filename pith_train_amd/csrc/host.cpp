@@ -151,7 +151,11 @@ int dtype_code(at::ScalarType t) {
     default: throw py::type_error(std::string("unsupported dtype ") + c10::toString(t));
   }
 }
-Tensor row_major(const Tensor& t) { return t.size(-1) > 0 && t.stride(-1) != 1 ? t.contiguous() : t; }
+// Rows that do not overlap, each contiguous: a sum over the rows hands one row of gradients to all of them (pitch 0).
+Tensor row_major(const Tensor& t) {
+  const bool overlap = t.dim() == 2 && t.size(0) > 1 && t.stride(0) < t.size(1);
+  return t.size(-1) > 0 && (t.stride(-1) != 1 || overlap) ? t.contiguous() : t;
+}
 // contiguous and on a 16-byte boundary, for kernels that take nothing else (a gradient may be a piece of a wider buffer)
 Tensor packed(const Tensor& t) {
   const Tensor c = t.contiguous();

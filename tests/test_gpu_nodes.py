@@ -211,3 +211,33 @@ def test_hooks_on_saved_tensors_see_the_activations(kind):
         out = call(x)
     with pytest.raises(RuntimeError):
         out.sum().backward()
+
+
+@pytest.mark.parametrize("kind", ["linear", "mlp", "grouped"])
+@pytest.mark.parametrize("fresh", [True, False])
+def test_rows_that_share_memory(kind, fresh):
+    """An input and a gradient of one row for all: a broadcast, and a sum over the rows."""
+    from pith_train_amd.dualpipe_utils import FP8WeightCacheControl
+    from pith_train_amd.modules import experts as X
+    from pith_train_amd.operators.linear import FP8Linear
+
+    offs = torch.tensor([128, 256], dtype=torch.int32, device="cuda")
+    m = {"linear": lambda: FP8Linear(256, 128, bias=False), "mlp": lambda: X.DeepSeekV2MLP(256, 256),
+         "grouped": lambda: X.FP8GroupedLinear(2, 256, 128)}[kind]().cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.normal_(0.0, 0.05)
+    call = (lambda x: m(x, grouped_mm_offs=offs)) if kind == "grouped" else m
+
+    def step(shared):
+        if fresh:
+            FP8WeightCacheControl.step()
+        m.zero_grad(set_to_none=True)
+        x = _randn(1, 256).detach().fill_(0.5).requires_grad_(True)
+        rows = x.expand(256, 256)
+        out = call(rows if shared else rows.contiguous())
+        dy = torch.linspace(-1, 1, out.shape[1], device="cuda").bfloat16().expand(out.shape)
+        out.backward(dy if shared else dy.contiguous())
+        return [out.detach(), x.grad, *(p.grad for p in m.parameters())]
+
+    assert all(torch.equal(a, b) for a, b in zip(step(True), step(False)))
