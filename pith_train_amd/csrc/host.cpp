@@ -1255,7 +1255,7 @@ struct GateLinearNode : HipNode {
     if (!g[0].defined()) return {Tensor(), Tensor()};
     const Tensor x = input.get(), w = weight.get();
     const int64_t T = x.size(0), H = x.size(1), E = w.size(0);
-    const Tensor dl = (g[0].scalar_type() == at::kBFloat16 ? g[0] : g[0].to(at::kFloat)).contiguous();
+    const Tensor dl = packed(g[0].scalar_type() == at::kBFloat16 ? g[0] : g[0].to(at::kFloat));
     Tensor dx = empty({T, H}, at::kBFloat16, x.device()), dw = empty({E, H}, at::kBFloat16, x.device());
     Tensor ws = empty({lib.pt_gate_linear_bwd_workspace_bytes(T, (int32_t)E, H)}, at::kByte, x.device());
     check(lib.pt_gate_linear_bwd(ptr(dl), dtype_code(dl.scalar_type()), ptr(x), ptr(w), ptr(dx), ptr(dw), T, (int32_t)E, H, ptr(ws), stream), "pt_gate_linear_bwd");

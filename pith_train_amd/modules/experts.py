@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from .. import _lib
 from ..dualpipe_utils import FP8WeightCacheControl
@@ -38,11 +39,11 @@ from ..operators.token_scatter import (
 from . import training
 
 
-def _weight(linear: nn.Module) -> torch.Tensor:
-    """``linear.weight`` without the module's attribute search (a microsecond each, and a step of a small
-    layer makes twenty of them)."""
-    w = linear._parameters.get("weight")
-    return w if w is not None else linear.weight
+def _weight(module: nn.Module, name: str = "weight") -> torch.Tensor:
+    """``module.weight`` without the module's attribute search (a microsecond each, and a step of a small
+    layer makes twenty of them).  A parametrised, pruned or sharded weight is no parameter of that name."""
+    w = module._parameters.get(name)
+    return w if w is not None else getattr(module, name)
 
 
 def _cached(cache, version: int, now: int, twin: bool) -> bool:
@@ -151,7 +152,7 @@ class DeepSeekV2MLP(nn.Module):
         weights = []
         for m in self._modules.values():
             if (type(m) is not FP8Linear or m.bias is not None or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                    or m._backward_pre_hooks):
+                    or m._backward_pre_hooks or _has_any_global_hook()):
                 return None
             weights.append(_weight(m))
         if len(weights) != 3 or x.dtype != torch.bfloat16 or not x.is_cuda or x.numel() == 0 or torch.compiler.is_compiling():
@@ -279,10 +280,9 @@ class GptOssExperts(nn.Module):
 
     def bias_fusable(self, x) -> bool:
         """Whether the two ``indexed_bias_add`` steps happen in the stores of the GEMMs."""
-        p = self._parameters
         return (self.fuse_bias and training.fp8 and x.shape[0] > 0 and x.dtype == torch.bfloat16
-                and p["gate_up_proj_bias"].dtype == x.dtype and p["down_proj_bias"].dtype == x.dtype
-                and p["gate_up_proj"].shape[1] % 8 == 0 and p["down_proj"].shape[1] % 8 == 0)
+                and _weight(self, "gate_up_proj_bias").dtype == x.dtype and _weight(self, "down_proj_bias").dtype == x.dtype
+                and _weight(self, "gate_up_proj").shape[1] % 8 == 0 and _weight(self, "down_proj").shape[1] % 8 == 0)
 
     def one_node(self, x) -> bool:
         """Whether the block runs as one autograd node (fused biases and activation).  That node
@@ -302,14 +302,15 @@ class GptOssExperts(nn.Module):
         M = x.shape[0] if row_map is None else row_map.shape[0]
         fused = self.bias_fusable(x)
         assert not scatter_output or (fused and row_map is not None), "scatter_output needs row_map and the fused biases"
-        if M % 128 == 0 and self.one_node(x) and not fused_experts.wants_backward(x, *self._parameters.values()):
-            return fused_experts.forward_only(
-                x, self.down_proj, grouped_mm_offs, *self._quantized_weights(), row_map, None, scatter_output,
-                (1.702, self.swiglu_limit), (self.gate_up_proj_bias, self.down_proj_bias), few_rows,
-            )
         if M % 128 == 0 and self.one_node(x):
+            gate_up, gate_up_bias, down, down_bias = (_weight(self, n) for n in ("gate_up_proj", "gate_up_proj_bias", "down_proj", "down_proj_bias"))
+            if not fused_experts.wants_backward(x, gate_up, gate_up_bias, down, down_bias):
+                return fused_experts.forward_only(
+                    x, down, grouped_mm_offs, *self._quantized_weights(), row_map, None, scatter_output,
+                    (1.702, self.swiglu_limit), (gate_up_bias, down_bias), few_rows,
+                )
             return fused_experts.FP8ClampedSwiGLUExpertsFunc.apply(
-                x, self.gate_up_proj, self.gate_up_proj_bias, self.down_proj, self.down_proj_bias, grouped_mm_offs,
+                x, gate_up, gate_up_bias, down, down_bias, grouped_mm_offs,
                 *self._quantized_weights(), 1.702, self.swiglu_limit, row_map, scatter_output,
             )
         if fused:

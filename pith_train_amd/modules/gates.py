@@ -67,7 +67,9 @@ class _Gate(nn.Module):
     def _logits(self, hidden_states: torch.Tensor, fp32: bool = False) -> torch.Tensor:
         """``F.linear`` without a bias (``fp32``: on fp32 copies), for bf16 inputs with a backward of its own that
         makes both gradients in one pass."""
-        weight = self._parameters["weight"]
+        weight = self._parameters.get("weight")
+        if weight is None:  # parametrised, pruned or sharded: an attribute, or computed by one
+            weight = self.weight
         if hidden_states.is_cuda and not torch.compiler.is_compiling():
             logits = _lib.host().gate_linear(hidden_states, weight, fp32, _lib.stream_ptr(hidden_states.device))
             if logits is not None:

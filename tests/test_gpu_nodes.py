@@ -241,3 +241,41 @@ def test_rows_that_share_memory(kind, fresh):
         return [out.detach(), x.grad, *(p.grad for p in m.parameters())]
 
     assert all(torch.equal(a, b) for a, b in zip(step(True), step(False)))
+
+
+class _Doubled(torch.nn.Module):
+    def forward(self, w):
+        return 2.0 * w
+
+
+@pytest.mark.parametrize("family,names", [("Qwen3MoeMoE", ["gate.weight"]), ("DeepSeekV2MoE", ["gate.weight", "shared_experts.up_proj.weight"]),
+                                          ("GptOssMoE", ["router.weight", "experts.down_proj_bias"])])
+def test_block_with_parametrised_weights(family, names):
+    """Twice the stored weight equals a block that stores twice the weight; the gradient reaches the stored one."""
+    from torch.nn.utils import parametrize
+
+    from pith_train_amd.dualpipe_utils import FP8WeightCacheControl
+    from pith_train_amd.modules import moe
+
+    torch.manual_seed(1)
+    block = getattr(moe, family)(128, 128, 8, 2).cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        for p in block.parameters():
+            p.normal_(0.0, 0.05)
+    x = _randn(64, 128, grad=False)
+    for name in names:
+        module, attr = block.get_submodule(name.rpartition(".")[0]), name.rpartition(".")[2]
+        w = getattr(module, attr)
+        with torch.no_grad():
+            w.mul_(2.0)
+        FP8WeightCacheControl.step()
+        want = block.reference_forward(x)
+        with torch.no_grad():
+            w.mul_(0.5)
+        parametrize.register_parametrization(module, attr, _Doubled())
+        FP8WeightCacheControl.step()
+        got = block.reference_forward(x)
+        torch.testing.assert_close(got, want, rtol=2.0**-7, atol=2.0**-7 * want.float().abs().max().item())
+        (grad,) = torch.autograd.grad(got.float().square().sum(), getattr(module.parametrizations, attr).original, allow_unused=False)
+        assert grad.abs().sum() > 0
+        parametrize.remove_parametrizations(module, attr, leave_parametrized=False)

@@ -36,3 +36,27 @@ def test_branches_are_differentiable_twice():
     x = torch.randn((5, 8), dtype=torch.float64, requires_grad=True)
     assert torch.autograd.gradcheck(lambda t: _host().branches(t, 3, 2, 0), x)
     assert torch.autograd.gradgradcheck(lambda t: [b * b for b in _host().branches(t, 3, 2, 0)], x)
+
+
+class _Doubled(torch.nn.Module):
+    def forward(self, w):
+        return 2.0 * w
+
+
+def test_gates_and_experts_with_a_parametrised_weight():
+    """The parameter is then no entry of that name, and the attribute computes the weight."""
+    from torch.nn.utils import parametrize
+
+    from pith_train_amd.modules.experts import GptOssExperts
+    from pith_train_amd.modules.gates import Qwen3MoeGate
+
+    gate = Qwen3MoeGate(4, 16, 2)
+    torch.nn.init.normal_(gate.weight)
+    x, w = torch.randn((6, 16)), gate.weight.detach().clone()
+    parametrize.register_parametrization(gate, "weight", _Doubled())
+    torch.testing.assert_close(gate._logits(x), F.linear(x, 2.0 * w))
+    experts = GptOssExperts(16, 16, 2).to(torch.bfloat16)
+    fusable = experts.bias_fusable(x.bfloat16())
+    for name in ("gate_up_proj", "down_proj_bias"):
+        parametrize.register_parametrization(experts, name, _Doubled())
+    assert experts.bias_fusable(x.bfloat16()) == fusable
