@@ -8,12 +8,14 @@
 // No HIP header and no stream query here: the caller passes the stream it is on, and a backward runs on
 // the stream of its forward.
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/extension.h>
 
 #include <dlfcn.h>
 
+#include <algorithm>
 #include <optional>
 #include <sstream>
 
@@ -170,6 +172,11 @@ void require_same_device(const Tensor& x, std::initializer_list<const Tensor*> o
   for (const Tensor* t : others)
     if (t->defined() && t->device() != x.device())
       throw HipError("pith_train_amd operators take all of their tensors on one GPU (got " + x.device().str() + " and " + t->device().str() + ")");
+}
+
+bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(0).defined(); }
+void refuse_tangent(const Tensor& t) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!has_tangent(t), "pith_train_amd operators have no forward-mode derivative");
 }
 
 // A tensor whose address goes to a kernel that derives every index from the sizes given here.
@@ -404,6 +411,7 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x,
   const Dims d{row_map ? row_map->size(0) : src_rows, K, half, dn.size(1), dn.size(0)};
   const int64_t routed = expand_idx ? expand_idx->size(0) : src_rows * repeat;
   if (x.scalar_type() != at::kBFloat16) throw HipError("expert block: bf16 rows only");
+  refuse_tangent(x);
   require_operand(gu, gu_s, d.G, 2 * half, K, "gate_up weight");
   require_operand(dn, dn_s, d.G, d.H, half, "down weight");
   require_shape(offs, {d.G}, at::kInt, "group ends");
@@ -552,11 +560,31 @@ struct HipNode : torch::autograd::Node {
   pt_stream_t stream = nullptr;
   bool released = false;
   virtual variable_list run(variable_list&& grads) = 0;
+  // the gradients as torch's operators make them, for nodes whose backward can be differentiated
+  virtual std::optional<variable_list> differentiable(const variable_list& grads) { return std::nullopt; }
   virtual void drop() = 0;
   variable_list apply(variable_list&& grads) override {
     TORCH_CHECK(!released, "the saved tensors of ", name(), " are gone: a second backward needs retain_graph=True for the first one");
-    at::AutoDispatchBelowADInplaceOrView guard;
-    return run(std::move(grads));
+    const bool twice = at::GradMode::is_enabled();  // create_graph=True
+    if (twice)
+      if (auto result = differentiable(grads)) return *result;
+    const variable_list given = twice ? grads : variable_list();
+    variable_list result;
+    {
+      at::AutoDispatchBelowADInplaceOrView guard;
+      result = run(std::move(grads));
+    }
+    if (twice) refuse_second(result, given);
+    return result;
+  }
+  // A kernel's result has no graph: differentiating it again raises instead of passing for a constant.
+  void refuse_second(variable_list& result, const variable_list& given) {
+    for (Tensor& t : result) {
+      if (!t.defined() || std::any_of(given.begin(), given.end(), [&](const Tensor& g) { return g.is_same(t); })) continue;
+      std::shared_ptr<torch::autograd::Error> error(new torch::autograd::Error("the backward of " + name() + " cannot be differentiated"),
+                                                    torch::autograd::deleteNode);
+      torch::autograd::set_history(t, error);
+    }
   }
   void release_variables() override {
     released = true;
@@ -577,6 +605,7 @@ std::shared_ptr<N> make_node(int64_t stream, const Inputs&... inputs) {
 template <class N, class Compute, class Fill, class... Inputs>
 Tensor with_node(int64_t stream, Compute compute, Fill fill, const Inputs&... inputs) {
   const bool wants = torch::autograd::compute_requires_grad(inputs...);
+  (refuse_tangent(inputs), ...);
   Tensor out;
   {
     at::AutoDispatchBelowADInplaceOrView guard;
@@ -840,6 +869,7 @@ std::pair<Maybe, std::optional<std::vector<Tensor>>> mlp(const Tensor& input, co
       w_up.sizes() != w_gate.sizes() || w_gate.size(1) != K || w_down.size(1) != half || M == 0 || half == 0 || half % 128 || K == 0 || K % 16 || H == 0 || H % 16)
     return {std::nullopt, std::nullopt};
   const bool keep = torch::autograd::compute_requires_grad(input, w_gate, w_up, w_down);
+  if (has_tangent(input) || has_tangent(w_gate) || has_tangent(w_up) || has_tangent(w_down)) return {std::nullopt, std::nullopt};
   std::vector<Tensor> t;
   auto node = keep ? make_node<MlpNode>(stream, input, w_gate, w_up, w_down) : nullptr;
   Tensor y;
@@ -1251,6 +1281,13 @@ std::pair<Tensor, Tensor> router_topk(const Tensor& input, int64_t mode, int64_t
 struct GateLinearNode : HipNode {
   Saved input, weight;
   void drop() override { input.reset(); weight.reset(); }
+  std::optional<variable_list> differentiable(const variable_list& g) override {
+    if (!g[0].defined()) return variable_list(2);
+    const Tensor x = input.get(), w = weight.get();
+    const Tensor dl = g[0].scalar_type() == at::kBFloat16 ? g[0] : g[0].to(at::kFloat);
+    const auto type = dl.scalar_type();
+    return variable_list{at::matmul(dl, w.to(type)).to(at::kBFloat16), at::matmul(dl.t(), x.to(type)).to(at::kBFloat16)};
+  }
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor()};
     const Tensor x = input.get(), w = weight.get();
@@ -1271,6 +1308,7 @@ Maybe gate_linear(const Tensor& input, const Tensor& weight, bool fp32, int64_t 
   const auto plain = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)ptr(t) % 16 == 0; };
   if (input.numel() == 0 || E % 8 || E > 256 || E == 0 || input.size(1) % 8 || input.size(1) != weight.size(1) || !plain(input) || !plain(weight))
     return std::nullopt;
+  if (has_tangent(input) || has_tangent(weight)) return std::nullopt;
   return with_node<GateLinearNode>(
       stream, [&] { return fp32 ? at::linear(input.to(at::kFloat), weight.to(at::kFloat)) : at::linear(input, weight); },
       [&](GateLinearNode& n) {

@@ -22,6 +22,7 @@ likewise (:func:`moe_combine_ep`), with the order of the adds fixed: ascending r
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _lib
 
@@ -67,6 +68,7 @@ def token_branches(x: torch.Tensor, k: int, n: int):
     choice) for the experts, and ``n`` (up to 3) times ``x`` itself.  The backward adds the branches'
     gradients, the k rows of the experts' included, in one pass with one rounding, where a reduction and an
     addition per branch would each read and write the whole tensor."""
-    if not (torch.is_grad_enabled() and x.requires_grad):
+    plain = not (torch.is_grad_enabled() and x.requires_grad) or torch.compiler.is_compiling() or torch._C._functorch.is_functorch_wrapped_tensor(x)
+    if plain or forward_ad.unpack_dual(x).tangent is not None:
         return (x.unsqueeze(1).expand(-1, k, -1), *([x] * n))
     return _lib.host().branches(x, k, n, _lib.stream_ptr(x.device))

@@ -279,3 +279,50 @@ def test_block_with_parametrised_weights(family, names):
         (grad,) = torch.autograd.grad(got.float().square().sum(), getattr(module.parametrizations, attr).original, allow_unused=False)
         assert grad.abs().sum() > 0
         parametrize.remove_parametrizations(module, attr, leave_parametrized=False)
+
+
+def test_gate_and_branches_are_differentiable_twice_and_forward():
+    """As the torch expressions they stand for: the gate's product, and the input handed to several consumers."""
+    import torch.nn.functional as F
+    from torch.autograd import forward_ad
+
+    from pith_train_amd.modules.gates import DeepSeekV2MoEGate, Qwen3MoeGate
+    from pith_train_amd.operators.moe_combine import token_branches
+
+    for make, fp32 in ((Qwen3MoeGate, False), (DeepSeekV2MoEGate, True)):
+        gate = make(8, 64, 2).cuda().to(torch.bfloat16)
+        torch.nn.init.normal_(gate.weight)
+        x, up = _randn(40, 64), torch.randn((40, 8), device="cuda")
+        results = []
+        for logits in (gate._logits(x, fp32), F.linear(x.float(), gate.weight.float()) if fp32 else F.linear(x, gate.weight)):
+            gx, gw = torch.autograd.grad(logits, [x, gate.weight], (up.to(logits.dtype) * logits), create_graph=True)
+            results.append([logits, gx, gw, *torch.autograd.grad(gx.float().square().sum() + gw.float().square().sum(), [x, gate.weight])])
+        for got, want in zip(*results):
+            torch.testing.assert_close(got, want, rtol=0.02, atol=0.02 * want.float().abs().max().item())
+        with forward_ad.dual_level():
+            dual = forward_ad.make_dual(x.detach(), torch.ones_like(x))
+            tangent = forward_ad.unpack_dual(gate._logits(dual, fp32)).tangent
+            assert tangent is not None and torch.equal(tangent[0], tangent[1])
+            assert all(forward_ad.unpack_dual(b).tangent is not None for b in token_branches(dual.requires_grad_(True), 2, 1))
+
+
+@pytest.mark.parametrize("kind", ["Qwen3MoeExperts", "grouped", "mlp", "linear"])
+def test_what_a_kernel_cannot_differentiate_is_refused(kind):
+    """Not dropped: a second derivative, and a forward-mode one."""
+    from torch.autograd import forward_ad
+
+    m, call, _ = _hidden_activations(kind)
+    m.cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.normal_(0.0, 0.05)
+    x = _randn(300, 256)
+    out = call(x)
+    (grad,) = torch.autograd.grad(out, x, torch.ones_like(out), create_graph=True)
+    assert grad.requires_grad
+    with pytest.raises(RuntimeError, match="cannot be differentiated"):
+        grad.sum().backward()
+    with forward_ad.dual_level(), pytest.raises(RuntimeError, match="forward-mode|forward mode|forward AD"):
+        call(forward_ad.make_dual(x.detach(), torch.ones_like(x)).requires_grad_(True))
+    with torch.no_grad(), forward_ad.dual_level(), pytest.raises(RuntimeError, match="forward-mode|forward mode|forward AD"):
+        call(forward_ad.make_dual(x.detach(), torch.ones_like(x)))
