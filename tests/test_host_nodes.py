@@ -60,3 +60,25 @@ def test_gates_and_experts_with_a_parametrised_weight():
     for name in ("gate_up_proj", "down_proj_bias"):
         parametrize.register_parametrization(experts, name, _Doubled())
     assert experts.bias_fusable(x.bfloat16()) == fusable
+
+
+def test_import_leaves_the_process_as_it_is():
+    """A library that is imported changes no setting of autograd's, nor of anything else the whole program uses."""
+    import os
+    import subprocess
+    import sys
+
+    code = """
+import torch
+def state():
+    return (torch._C._is_multithreading_enabled(), torch.is_grad_enabled(), torch.get_num_threads(), torch.get_default_dtype(),
+            torch.backends.cuda.matmul.allow_tf32, torch.are_deterministic_algorithms_enabled(), torch.is_anomaly_enabled())
+before = state()
+import pith_train_amd
+from pith_train_amd import _lib
+from pith_train_amd.modules import moe
+_lib.host()
+assert state() == before, (before, state())
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=root)
