@@ -7,6 +7,7 @@
 //
 // No HIP header and no stream query here: the caller passes the stream it is on, and a backward runs on
 // the stream of its forward.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -32,6 +33,38 @@ namespace {
 struct HipError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
+struct AssertionError : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
+PyObject* g_error = nullptr;  // PithTrainHipError (never released)
+
+// Runs a backward and turns what it throws into the Python error that a node written in Python would raise: the
+// engine carries nothing but torch's own exceptions over to the caller's thread unchanged.
+template <class F>
+auto as_python_errors(F f) {
+  const auto carry = [](PyObject* type, const char* what) {
+    py::gil_scoped_acquire gil;
+    if (type) PyErr_SetString(type, what);
+    python_error e;
+    e.persist();
+    throw std::move(e);
+  };
+  try {
+    return f();
+  } catch (const HipError& e) {
+    carry(g_error ? g_error : PyExc_RuntimeError, e.what());
+  } catch (const AssertionError& e) {
+    carry(PyExc_AssertionError, e.what());
+  } catch (const py::type_error& e) {
+    carry(PyExc_TypeError, e.what());
+  } catch (py::error_already_set& e) {  // from a callback
+    py::gil_scoped_acquire gil;
+    e.restore();
+    carry(nullptr, nullptr);
+  }
+  return decltype(f())();
+}
 
 struct Library {
 #define PT_FN(NAME) decltype(&::NAME) NAME = nullptr
@@ -529,7 +562,7 @@ struct ExpertsBackward {
 // autograd nodes
 // ---------------------------------------------------------------------------------------------------------
 // Python objects the nodes call back into (never released: they live as long as the process)
-PyObject *g_error = nullptr, *g_store = nullptr, *g_schedule = nullptr, *g_dgrad = nullptr;
+PyObject *g_store = nullptr, *g_schedule = nullptr, *g_dgrad = nullptr;
 
 // A tensor kept for the backward as autograd keeps its own: a write to it before the backward is found out, and
 // saved-tensor hooks see it.  What a hook gives back goes to kernels by address, so it has to be what was saved.
@@ -564,6 +597,9 @@ struct HipNode : torch::autograd::Node {
   virtual std::optional<variable_list> differentiable(const variable_list& grads) { return std::nullopt; }
   virtual void drop() = 0;
   variable_list apply(variable_list&& grads) override {
+    return as_python_errors([&] { return backward(std::move(grads)); });
+  }
+  variable_list backward(variable_list&& grads) {
     TORCH_CHECK(!released, "the saved tensors of ", name(), " are gone: a second backward needs retain_graph=True for the first one");
     const bool twice = at::GradMode::is_enabled();  // create_graph=True
     if (twice)
@@ -736,9 +772,9 @@ struct SiluMulNode : HipNode {
   variable_list run(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor()};
     const Tensor a = gate.get(), b = up.get();
-    TORCH_CHECK(g[0].sizes() == a.sizes(), "grad_output shape ", g[0].sizes(), " != gate shape ", a.sizes());
-    TORCH_CHECK(g[0].scalar_type() == a.scalar_type(), "grad_output dtype differs from gate's");
-    TORCH_CHECK(g[0].is_contiguous(), "grad_output must be contiguous");
+    if (g[0].sizes() != a.sizes()) throw AssertionError("grad_output shape != gate shape");
+    if (g[0].scalar_type() != a.scalar_type()) throw AssertionError("grad_output dtype differs from gate's");
+    if (!g[0].is_contiguous()) throw AssertionError("grad_output must be contiguous");
     Tensor da = empty(a.sizes(), a.scalar_type(), a.device()), db = empty(a.sizes(), a.scalar_type(), a.device());
     check(lib.pt_silu_mul_bwd(ptr(g[0]), ptr(a), ptr(b), ptr(da), ptr(db), a.numel(), dtype_code(a.scalar_type()), stream), "pt_silu_mul_bwd");
     return {da, db};
@@ -1205,12 +1241,17 @@ struct BranchesFunction : torch::autograd::Function<BranchesFunction> {
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    return as_python_errors([&] { return sum(ctx, g); });
+  }
+
+  static variable_list sum(AutogradContext* ctx, const variable_list& g) {
     std::vector<Tensor> given;
     bool same = g.size() <= 4;
     for (const Tensor& t : g)
       if (t.defined()) {
         given.push_back(t);
-        same = same && t.is_cuda() && t.size(-1) % 8 == 0 && t.scalar_type() == given[0].scalar_type();
+        const auto type = t.scalar_type();
+        same = same && t.is_cuda() && t.size(-1) % 8 == 0 && type == given[0].scalar_type() && (type == at::kBFloat16 || type == at::kFloat || type == at::kHalf);
       }
     if (given.empty()) return variable_list(4);
     const bool rows = g[0].defined();
@@ -1357,6 +1398,10 @@ PYBIND11_MODULE(_host, m) {
       if (p) std::rethrow_exception(p);
     } catch (const HipError& e) {
       PyErr_SetString(g_error ? g_error : PyExc_RuntimeError, e.what());
+    } catch (python_error& e) {  // a saved-tensor hook's
+      e.restore();
+    } catch (const c10::Error&) {  // by its kind: NotImplementedError, IndexError, ...
+      torch::translate_exception_to_python(p);
     }
   });
   m.def("init", [](const std::string& path, py::object error) {
@@ -1368,29 +1413,31 @@ PYBIND11_MODULE(_host, m) {
     g_schedule = schedule.release().ptr();
     g_dgrad = dgrad.release().ptr();
   });
-  m.def("index_gather", &index_gather);
-  m.def("scatter_sum", &scatter_sum);
-  m.def("permute_into_buffer", &permute_into_buffer);
-  m.def("permute_rows", &permute_rows);
-  m.def("silu_mul", &silu_mul);
-  m.def("grouped_linear", &grouped_linear);
-  m.def("experts", &experts);
-  m.def("combine", &combine);
-  m.def("combine_ep", &combine_ep);
-  m.def("branches", &branches);
-  m.def("router_topk", &router_topk);
-  m.def("dedup_prepare_dispatch", &dedup_prepare_dispatch);
-  m.def("build_expert_idxs", &build_expert_idxs);
-  m.def("adjust_expand_idx", &adjust_expand_idx);
+  // without the GIL, as ctypes calls the library: other threads run while a step's launches are queued
+  const auto launch = [&m](const char* name, auto* f) { m.def(name, f, py::call_guard<py::gil_scoped_release>()); };
+  launch("index_gather", &index_gather);
+  launch("scatter_sum", &scatter_sum);
+  launch("permute_into_buffer", &permute_into_buffer);
+  launch("permute_rows", &permute_rows);
+  launch("silu_mul", &silu_mul);
+  launch("grouped_linear", &grouped_linear);
+  launch("experts", &experts);
+  launch("combine", &combine);
+  launch("combine_ep", &combine_ep);
+  launch("branches", &branches);
+  launch("router_topk", &router_topk);
+  launch("dedup_prepare_dispatch", &dedup_prepare_dispatch);
+  launch("build_expert_idxs", &build_expert_idxs);
+  launch("adjust_expand_idx", &adjust_expand_idx);
   m.def("split_k", &split_k);
-  m.def("quant_weight", &quant_weight);
-  m.def("quant_grouped_weights", &quant_grouped_weights);
-  m.def("gate_linear", &gate_linear);
-  m.def("mlp", &mlp);
-  m.def("linear", &linear);
-  m.def("linear_fresh", &linear_fresh);
-  m.def("linear_heads_forward", &linear_heads_forward);
-  m.def("linear_heads_backward", &linear_heads_backward);
-  m.def("group_rows", &group_rows);
-  m.def("experts_forward", &experts_forward);
+  launch("quant_weight", &quant_weight);
+  launch("quant_grouped_weights", &quant_grouped_weights);
+  launch("gate_linear", &gate_linear);
+  launch("mlp", &mlp);
+  launch("linear", &linear);
+  launch("linear_fresh", &linear_fresh);
+  launch("linear_heads_forward", &linear_heads_forward);
+  launch("linear_heads_backward", &linear_heads_backward);
+  launch("group_rows", &group_rows);
+  launch("experts_forward", &experts_forward);
 }

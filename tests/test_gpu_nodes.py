@@ -326,3 +326,35 @@ def test_what_a_kernel_cannot_differentiate_is_refused(kind):
         call(forward_ad.make_dual(x.detach(), torch.ones_like(x)).requires_grad_(True))
     with torch.no_grad(), forward_ad.dual_level(), pytest.raises(RuntimeError, match="forward-mode|forward mode|forward AD"):
         call(forward_ad.make_dual(x.detach(), torch.ones_like(x)))
+
+
+def test_errors_of_a_backward_keep_their_types(monkeypatch):
+    from pith_train_amd import _lib
+    from pith_train_amd.dualpipe_utils import WeightGradStore
+    from pith_train_amd.modules.experts import Qwen3MoeExperts, forward_stage3
+    from pith_train_amd.operators.silu_mul import silu_mul
+    from pith_train_amd.operators.token_scatter import padded_index_gather
+
+    out = padded_index_gather(_randn(6, 16, dtype=torch.float64), torch.randint(0, 6, (10,), device="cuda"))
+    with pytest.raises(TypeError, match="dtype"):  # rows of any type are copied, but not summed
+        out.sum().backward()
+    out = silu_mul(_randn(4, 16), _randn(4, 16))
+    with pytest.raises(AssertionError, match="contiguous"):
+        out.backward(torch.ones((16, 4), device="cuda", dtype=torch.bfloat16).t())
+    keys = torch.randint(0, 4, (48,), device="cuda")
+    monkeypatch.setenv("PITHTRAIN_FP8_WEIGHT_TWIN", "1")
+    out = forward_stage3(Qwen3MoeExperts(128, 128, 4).cuda().to(torch.bfloat16), _randn(48, 128), keys, 4)
+    _lib.call("pt_gemm_select_kernel", b"t")  # a kernel that has no scattered store, which the host says
+    try:
+        with pytest.raises(_lib.PithTrainHipError, match="scattered"):
+            out.sum().backward(retain_graph=True)
+    finally:
+        _lib.call("pt_gemm_select_kernel", None)
+
+    def full(_):
+        raise KeyError("queue")
+
+    monkeypatch.setattr(WeightGradStore, "enabled", True)
+    monkeypatch.setattr(WeightGradStore, "put", full)
+    with pytest.raises(KeyError, match="queue"):
+        out.sum().backward()
