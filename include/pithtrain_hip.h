@@ -647,6 +647,8 @@ int pt_experts_forward(const pt_experts_forward_args* args /* host */);
  * for the transposed twin.  dy_t [H, M] and dgu_t [2*half, M] bytes with scales [M/128, .]: the transposed
  * gradients of the weight-gradient GEMMs (kept by the caller when it runs those later).  Not needed
  * afterwards: dy_fp8 [M, H] with 1x128 scales, grad_h bf16 [M, half], col_sum fp32 [M/128, 2*half].
+ * dy_fp8 and dy_scale may be the memory of dgu_fp8 and dgu_scale (of the larger size): they have been read
+ * before those are written.
  * dw_down [G, H, half] bf16 (NULL = not computed here), dw_gate_up [G, 2*half, K] or, when dw_up is given,
  * [G, half, K] each (pt_experts_weight_gradient only); *_add != 0: added to what is there.  d_gu_bias / d_dn_bias [G, 2*half] /
  * [G, H] in the types given: NULL = none. */

@@ -427,9 +427,7 @@ struct Dims {
     return Pieces({map ? 4 * M : 0, M * K, 4 * M * cdiv(K, 128), M * half, 4 * M * cdiv(half, 128)});
   }
   Pieces twins() const { return Pieces({H * M, M / 128 * H * 4, 2 * half * M, M / 128 * half * 8}); }      // dy^T, d(gate_up)^T with scales
-  Pieces backward_temp(bool sums) const {                                                                  // dy with scales, grad_h, column sums
-    return Pieces({M * H, 4 * M * cdiv(H, 128), 2 * M * half, sums ? M / 128 * half * 8 : 0});
-  }
+  Pieces backward_temp(bool sums) const { return Pieces({2 * M * half, sums ? M / 128 * half * 8 : 0}); }  // grad_h, column sums
 };
 
 // Forward of an expert block (see fused_experts._forward): (out, gate_up, kept buffers).
@@ -495,33 +493,41 @@ struct Target {
   }
 };
 
+// [rows, cols] of `type` in a new buffer that holds at least `other` columns
+Tensor shared_rows(int64_t rows, int64_t cols, int64_t other, at::ScalarType type, const at::Device& dev) {
+  if (cols >= other) return empty({rows, cols}, type, dev);
+  return empty({rows * other}, type, dev).narrow(0, 0, rows * cols).view({rows, cols});
+}
+
 // Backward of an expert block up to the quantised gradient of gate_up; the caller queues the input gradient from
-// it and then weight_gradient().
+// it and then weight_gradient().  A buffer goes back to the allocator when its last reader is queued (the next
+// user is behind it on the stream), and the gradient of gate_up is written over the one of the output, which only
+// the GEMM before it reads: at 32k tokens these are 0.6 GB each.
 struct ExpertsBackward {
   Dims d;
   pt_experts_backward_args a = {};
-  Pieces kept, twins, temp;
+  Pieces kept, twins;
+  std::vector<Tensor> weights;
   Tensor grad_out, dgu, dgu_s;
   Maybe d_gu_bias, d_dn_bias;
   Target down, gate_up, up;
 
   ExpertsBackward(const Tensor& grad, const Dims& dims, const Tensor& offs, const Maybe& row_map, bool scatter, const Tensor& dn_dg, const Tensor& dn_dg_s,
                   bool dn_forward, const Tensor& gate_up_saved, std::vector<Tensor> kept_buffers, bool clamped, double alpha, double limit,
-                  const Maybe& gu_bias_like, const Maybe& dn_bias_like, const std::vector<Tensor>& weights /* down, gate_up or gate, up; empty: deferred */,
+                  const Maybe& gu_bias_like, const Maybe& dn_bias_like, std::vector<Tensor> weights_ /* down, gate_up or gate, up; empty: deferred */,
                   int64_t stream)
-      : d(dims), kept(d.kept()), twins(d.twins()), temp(d.backward_temp(clamped)) {
+      : d(dims), kept(d.kept()), twins(d.twins()), weights(std::move(weights_)) {
+    Pieces temp = d.backward_temp(clamped);
     grad_out = grad.contiguous();
     const auto dev = grad_out.device();
     kept.buffers = std::move(kept_buffers);
     twins.allocate(dev);
     temp.allocate(dev);
-    dgu = empty({d.M, 2 * d.half}, kFp8, dev);
-    dgu_s = empty({d.M, cdiv(2 * d.half, 128)}, at::kFloat, dev);
+    dgu = shared_rows(d.M, 2 * d.half, d.H, kFp8, dev);
+    dgu_s = shared_rows(d.M, cdiv(2 * d.half, 128), cdiv(d.H, 128), at::kFloat, dev);
     if (gu_bias_like) d_gu_bias = empty({d.G, 2 * d.half}, gu_bias_like->scalar_type(), dev);
     if (dn_bias_like) d_dn_bias = empty({d.G, d.H}, dn_bias_like->scalar_type(), dev);
     if (weights.size() > 0) down.aim(weights[0]);
-    if (weights.size() > 1) gate_up.aim(weights[1]);
-    if (weights.size() > 2) up.aim(weights[2]);
     a.grad_out = ptr(grad_out); a.grad_rows = grad_out.size(0);
     a.M = d.M; a.K = d.K; a.half = d.half; a.H = d.H; a.G = d.G;
     a.offs = (const int32_t*)ptr(offs); a.out_map = scatter ? (const int32_t*)ptr(row_map) : nullptr; a.limit_rows = (bool)row_map;
@@ -530,18 +536,21 @@ struct ExpertsBackward {
     a.x_t = kept.at(0); a.x_t_scale = (const float*)kept.at(1); a.h_t = kept.at(2); a.h_t_scale = (const float*)kept.at(3);
     a.dgu_fp8 = ptr(dgu); a.dgu_scale = (float*)ptr(dgu_s);
     a.dy_t = twins.at(0); a.dy_t_scale = (float*)twins.at(1); a.dgu_t = twins.at(2); a.dgu_t_scale = (float*)twins.at(3);
-    a.dy_fp8 = temp.at(0); a.dy_scale = (float*)temp.at(1); a.grad_h = temp.at(2); a.col_sum = (float*)temp.at(3);
+    a.dy_fp8 = ptr(dgu); a.dy_scale = (float*)ptr(dgu_s); a.grad_h = temp.at(0); a.col_sum = (float*)temp.at(1);
     a.dw_down = down.at(); a.dw_down_add = down.add;
-    a.dw_gate_up = gate_up.at(); a.dw_gate_up_add = gate_up.add;
-    a.dw_up = up.at(); a.dw_up_add = up.add;
     a.clamped = clamped; a.alpha = alpha; a.limit = limit;
     a.d_gu_bias = ptr(d_gu_bias); a.d_gu_bias_dtype = d_gu_bias ? dtype_code(d_gu_bias->scalar_type()) : 0;
     a.d_dn_bias = ptr(d_dn_bias); a.d_dn_bias_dtype = d_dn_bias ? dtype_code(d_dn_bias->scalar_type()) : 0;
     a.stream = (pt_stream_t)stream;
     check(lib.pt_experts_backward(&a), "pt_experts_backward");
+    grad_out.reset();
   }
 
   void weight_gradient() {
+    gate_up.aim(weights[1]);
+    if (weights.size() > 2) up.aim(weights[2]);
+    a.dw_gate_up = gate_up.at(); a.dw_gate_up_add = gate_up.add;
+    a.dw_up = up.at(); a.dw_up_add = up.add;
     check(lib.pt_experts_weight_gradient(&a), "pt_experts_weight_gradient");
     down.finish();
     gate_up.finish();
@@ -1065,7 +1074,7 @@ struct ExpertsNode : HipNode {
       if (w_up.defined()) weights.push_back(w_up);
     }
     ExpertsBackward step(g[0], d, offs, row_map, scatter, saved[DN_DG].get(), saved[DN_DG_S].get(), dn_forward, saved[GATE_UP].get(), std::move(kept),
-                         clamped, alpha, limit, gu_bias, dn_bias, weights, (int64_t)stream);
+                         clamped, alpha, limit, gu_bias, dn_bias, std::move(weights), (int64_t)stream);
     Tensor gx = empty({row_map ? routed : d.M, d.K}, g[0].scalar_type(), g[0].device());
     {
       py::gil_scoped_acquire gil;
@@ -1085,6 +1094,8 @@ struct ExpertsNode : HipNode {
         }
       }
     }
+    step.dgu.reset();
+    step.dgu_s.reset();
     if (!deferred) step.weight_gradient();
     // rows that expand the same source row are summed (the backward of the expanding gather)
     if (expand_idx) gx = scatter_sum(gx, *expand_idx, src_rows, kRowAlignment, (int64_t)stream);

@@ -358,3 +358,30 @@ def test_errors_of_a_backward_keep_their_types(monkeypatch):
     monkeypatch.setattr(WeightGradStore, "put", full)
     with pytest.raises(KeyError, match="queue"):
         out.sum().backward()
+
+
+@pytest.mark.parametrize("hidden,inter", [(1024, 256), (512, 1024)])
+def test_peak_memory_of_an_expert_block_backward(hidden, inter):
+    """The row-scaled gradients and the activation's gradient are not held at once, nor with the last weight gradients:
+    the largest phase is the activation's backward (its own buffers, both transposed gradients, the first weight
+    gradient) or the one after it (the input gradient and the other weight gradients beside the transposed ones)."""
+    from pith_train_amd.modules.experts import Qwen35MoeExperts, forward_stage3
+
+    E, T = 4, 16384
+    m = Qwen35MoeExperts(hidden, inter, E).cuda().to(torch.bfloat16)
+    x, keys = _randn(T, hidden), torch.randint(0, E, (T,), device="cuda")
+    out = forward_stage3(m, x, keys, E)
+    dy = torch.ones_like(out)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    grad = torch.autograd.grad(out, x, dy)
+    torch.cuda.synchronize()
+    peak = torch.cuda.max_memory_allocated() - before
+    rows = -(-(T + 127 * E) // 128) * 128 + 128
+    transposed, down = rows * (hidden + 2 * inter), 2 * E * hidden * inter
+    first = rows * (max(hidden, 2 * inter) + 2 * inter) + down
+    second = rows * max(hidden, 2 * inter) + 2 * T * hidden + down
+    third = 2 * T * hidden + 3 * down
+    assert peak <= 1.05 * (transposed + max(first, second, third)) + (4 << 20), (peak, transposed, first, second, third)
+    assert grad[0].shape == x.shape
