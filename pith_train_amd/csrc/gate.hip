@@ -57,7 +57,7 @@ __device__ __forceinline__ GateFrag gate_column(const uint4 (&rows)[8], int j) {
 }
 
 // The gradients of the logits as operands.  fp32: v = hi + mid + lo exactly, each with at most eight significant
-// bits; bf16: as they are.
+// bits (a NaN stays one in all three, an infinity in the first); bf16: as they are.
 template <typename D> struct GateOperand;
 template <> struct GateOperand<float> {
   GateFrag hi, mid, lo;
@@ -69,7 +69,7 @@ template <> struct GateOperand<float> {
       for (int u = 0; u < 2; ++u) {
         const float f = v[2 * m + u];
         h[u] = __float_as_uint(f);
-        const float r = f - __uint_as_float(h[u] & 0xFFFF0000u);
+        const float r = __builtin_isinf(f) ? 0.f : f - __uint_as_float(h[u] & 0xFFFF0000u);  // an infinity is its own first part
         d[u] = __float_as_uint(r);
         l[u] = __float_as_uint(r - __uint_as_float(d[u] & 0xFFFF0000u));
       }

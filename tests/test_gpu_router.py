@@ -242,3 +242,27 @@ def test_gate_linear_gradients(T, E, H, fp32):
         assert got.dtype == torch.bfloat16
         # half a unit of bf16, plus fp32 summation error relative to the largest value
         assert bool(((got.double() - want).abs() <= want.abs() * 2.0**-8 + 1e-5 * want.abs().max()).all())
+
+
+@pytest.mark.parametrize("fp32", [True, False])
+def test_gate_linear_gradients_of_overflowed_logits(fp32):
+    """Infinities and NaN stay what they are in the row and the column they reach, and reach no other; values at
+    either end of the type's range."""
+    from pith_train_amd import _lib
+
+    g = torch.Generator().manual_seed(3)
+    T, E, H = 70, 24, 136
+    x = torch.randn((T, H), generator=g).bfloat16().cuda().requires_grad_(True)
+    w = torch.randn((E, H), generator=g).bfloat16().cuda().requires_grad_(True)
+    kind = torch.float32 if fp32 else torch.bfloat16
+    dl = torch.randn((T, E), generator=g).to(kind)
+    for i, v in enumerate((float("inf"), float("-inf"), float("nan"), 1e30, -1e30, 1e-38)):
+        dl[11 * i, 3 * i] = v
+    dl = dl.cuda()
+    dx, dw = torch.autograd.grad(_lib.host().gate_linear(x, w, fp32, _lib.stream_ptr(x.device)), [x, w], dl)
+    for got, want in ((dx, dl.double() @ w.detach().double()), (dw, dl.double().T @ x.detach().double())):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf()) and want.isinf().any()
+        assert torch.equal(got[want.isinf()].double(), want[want.isinf()])
+        fin = want.isfinite()
+        scale = torch.where(fin, want.abs(), 0.0).amax(1, keepdim=True)  # rows differ by 30 orders of magnitude
+        assert bool(((got.double() - want).abs() <= want.abs() * 2.0**-8 + 1e-5 * scale)[fin].all())
