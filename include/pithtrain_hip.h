@@ -675,6 +675,9 @@ int pt_experts_backward(const pt_experts_backward_args* args /* host */);
 /* The gate_up weight gradient of the same block from the same arguments (dw_gate_up, dw_up): the last
  * launch of a backward, after the caller has queued the input gradient. */
 int pt_experts_weight_gradient(const pt_experts_backward_args* args /* host */);
+/* Row pitch (bytes) of a transposed FP8 operand of `rows` columns in a dense linear: what the backward entry points
+ * below use for their own, and callers for the ones they keep. */
+int64_t pt_transposed_pitch(int64_t rows);
 /* Forward of a dense FP8 linear (fp8_act_weight_gemm, operators/linear.py:44-60): x [M, K] in dtype,
  * y [M, N] in y_dtype (PT_BF16 or PT_F32); x_t (row pitch ld_t >= M bytes) and x_t_scale are the transposed
  * operand the weight gradient reads (both NULL: not written).  K % 16 == 0.  y2 != NULL (bf16, splits == 1):

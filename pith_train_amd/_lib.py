@@ -105,6 +105,7 @@ SIGNATURES = {
     "pt_experts_forward": (c_int, [c_char_p]),
     "pt_experts_backward": (c_int, [c_char_p]),
     "pt_experts_weight_gradient": (c_int, [c_char_p]),
+    "pt_transposed_pitch": (I64, [I64]),
     "pt_linear_forward_workspace_bytes": (I64, [I64, I64, I64, I64]),
     "pt_linear_forward": (c_int, [c_char_p]),
     "pt_linear_backward_workspace_bytes": (I64, [I64, I64, I64, I64, I64, I64]),

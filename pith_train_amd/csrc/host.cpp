@@ -77,6 +77,7 @@ struct Library {
   PT_FN(pt_experts_forward);
   PT_FN(pt_experts_backward);
   PT_FN(pt_experts_weight_gradient);
+  PT_FN(pt_transposed_pitch);
   PT_FN(pt_linear_forward_workspace_bytes);
   PT_FN(pt_linear_forward);
   PT_FN(pt_linear_backward_workspace_bytes);
@@ -130,6 +131,7 @@ void init(const std::string& path) {
   PT_FN(pt_experts_forward);
   PT_FN(pt_experts_backward);
   PT_FN(pt_experts_weight_gradient);
+  PT_FN(pt_transposed_pitch);
   PT_FN(pt_linear_forward_workspace_bytes);
   PT_FN(pt_linear_forward);
   PT_FN(pt_linear_backward_workspace_bytes);
@@ -227,13 +229,6 @@ void require_operand(const Tensor& q, const Tensor& scale, int64_t G, int64_t N,
   require_shape(scale, {G, cdiv(N, 128), cdiv(K, 128)}, at::kFloat, what);
 }
 
-// Row pitch of a transposed operand: the rule of deepgemm_quantize.transposed_pitch.
-int64_t transposed_pitch(int64_t m) {
-  if (m < 2048) return (m + 15) / 16 * 16;
-  m = (m + 127) / 128 * 128;
-  return m % 256 == 0 ? m + 128 : m;
-}
-
 constexpr int64_t kWorkgroups = 256;  // compute units of the MI355X
 
 // (splits, split_len) for out[m, n] = a[m, k] b[n, k]^T.  An output with fewer 256 x 256 tiles than the GPU
@@ -324,7 +319,7 @@ std::tuple<Tensor, Tensor, Tensor> linear_forward(const Tensor& input, const Qua
   const Tensor x = row_major(input);
   const int64_t m = x.size(0), k = x.size(1), n = w_fp8.size(0);
   const auto dev = x.device();
-  const int64_t ld_t = transposed_pitch(m);
+  const int64_t ld_t = lib.pt_transposed_pitch(m);
   Tensor y = empty({m, n}, x.scalar_type(), dev), x_t = empty({k, ld_t}, kFp8, dev), x_ts = empty({cdiv(k, 128), cdiv(m, 128)}, at::kFloat, dev);
   const auto [splits, len] = split_k(m, n, k);
   Tensor ws = empty({lib.pt_linear_forward_workspace_bytes(m, n, k, splits)}, at::kByte, dev);
@@ -927,7 +922,7 @@ std::pair<Maybe, std::optional<std::vector<Tensor>>> mlp(const Tensor& input, co
     else t = {empty({N, K}, kFp8, dev), empty({nb, kb}, at::kFloat, dev), empty({K, N}, kFp8, dev), empty({kb, nb}, at::kFloat, dev),
               empty({H, half}, kFp8, dev), empty({Hb, hb}, at::kFloat, dev), empty({half, H}, kFp8, dev), empty({hb, Hb}, at::kFloat, dev)};
     TORCH_CHECK(t.size() == 8, "mlp: eight quantised tensors");
-    const int64_t ld_t = transposed_pitch(M);
+    const int64_t ld_t = lib.pt_transposed_pitch(M);
     Tensor gate_up = empty({M, N}, bf16, dev), x_t, x_ts, h_t, h_ts;
     y = empty({M, H}, bf16, dev);
     if (keep) {

@@ -213,12 +213,13 @@ extern "C" int pt_linear_forward(const pt_linear_forward_args* args) {
                     (float*)(void*)ws.p, a.stream);
 }
 
-// Row pitch of a transposed operand (`red` = its length, a multiple of 16): whole 128-byte lines, and no
-// multiple of 256 bytes, which would put the rows of a reduction step onto few memory channels.
-static int64_t transposed_pitch(int64_t red) {
+// Whole 16-byte chunks; from 2048 on whole 128-byte lines, and no multiple of 256 bytes, which would put the rows
+// of a reduction step onto few memory channels.
+extern "C" int64_t pt_transposed_pitch(int64_t rows) {
+  const int64_t red = (rows + 15) & ~(int64_t)15;
   if (red < 2048) return red;
-  red = (red + 127) & ~(int64_t)127;
-  return red % 256 == 0 ? red + 128 : red;
+  const int64_t lines = (red + 127) & ~(int64_t)127;
+  return lines % 256 == 0 ? lines + 128 : lines;
 }
 
 // workspace: gradient bytes and scales | its transposed form and scales | the input's transposed form and
@@ -236,7 +237,7 @@ extern "C" int pt_linear_backward(const pt_linear_backward_args* args) {
   const int64_t red = (a.M + 15) & ~(int64_t)15;  // the weight gradient's reduction, zero-filled to whole 16-byte chunks
   PT_REQUIRE(!a.x_t || (a.ld_xt >= red && a.ld_xt % 16 == 0),
              "linear_backward: the transposed input needs a row pitch of %lld or more, a multiple of 16", (long long)red);
-  const int64_t ld_t = transposed_pitch(red);
+  const int64_t ld_t = pt_transposed_pitch(a.M);
   Carve ws(a.workspace);
   void* g_fp8 = ws.bytes(a.M * a.N);
   float* g_s = ws.floats(a.M * cdiv(a.N, 128));
@@ -351,7 +352,7 @@ extern "C" int pt_mlp_backward(const pt_mlp_backward_args* args) {
   PT_REQUIRE(a.M > 0 && a.K > 0 && a.half > 0 && a.H > 0 && a.half % 128 == 0 && a.K % 16 == 0 && a.H % 16 == 0 && a.ldg >= a.H, "mlp_backward: bad sizes");
   PT_REQUIRE(a.grad && a.gu_t && a.gu_t_scale && a.dn_t && a.dn_t_scale && a.gate_up && a.x_t && a.x_t_scale && a.h_t && a.h_t_scale && a.grad_x &&
                  a.grad_gu && a.grad_dn && a.workspace, "mlp_backward: null pointer");
-  const int64_t red = (a.M + 15) & ~(int64_t)15, ld_t = transposed_pitch(red), N = 2 * a.half;
+  const int64_t red = (a.M + 15) & ~(int64_t)15, ld_t = pt_transposed_pitch(a.M), N = 2 * a.half;
   PT_REQUIRE(a.ld_t >= red && a.ld_t % 16 == 0, "mlp_backward: the transposed operands need a row pitch of %lld or more, a multiple of 16", (long long)red);
   const MlpBackwardBuffers b(a.workspace, a.M, a.K, a.half, a.H, a.splits);
   PT_STEP(pt_quant_rowwise_transpose_ld, a.M, a.H, a.M, a.grad, PT_BF16, a.M, a.H, a.ldg, b.dy, b.dy_s, b.dy_t, ld_t, b.dy_ts, a.stream);

@@ -52,9 +52,10 @@ def transposed_pitch(m: int) -> int:
     gradient: 202 us against 241 at the packed pitch); with one that is a multiple of 256 the rows of a step fall
     onto few memory channels (measured: 25 % slower at 5 * 2**14 than at 579 * 128), so such pitches
     get one more line.  The reduction is read in 16-byte chunks, so a ragged token count is padded to
-    whole ones (with zeros)."""
+    whole ones (with zeros).  The library's ``pt_transposed_pitch``, spelled so that traced sizes pass."""
+    m = (m + 15) // 16 * 16
     if m < 2048:
-        return (m + 15) // 16 * 16
+        return m
     m = (m + 127) // 128 * 128
     return m + 128 if m % 256 == 0 else m
 

@@ -46,6 +46,18 @@ def test_workspace_queries_need_no_gpu():
     assert _lib.query("pt_dedup_workspace_bytes", 2048, 8, 128, 8) > 0
 
 
+def test_pitch_of_transposed_operands_is_one_rule():
+    """What the operators allocate is what the library's backward writes: a multiple of 16 that holds the rows, and
+    from 2048 on an odd number of 128-byte lines."""
+    from pith_train_amd import _lib
+    from pith_train_amd.operators.deepgemm_quantize import transposed_pitch
+
+    for m in (*range(1, 4700), 8191, 8192, 32767, 32768, 65537):
+        p = transposed_pitch(m)
+        assert p == _lib.query("pt_transposed_pitch", m), m
+        assert m <= p < m + 384 and (p % 256 == 128 if p >= 2048 else p == -(-m // 16) * 16)
+
+
 def test_gemm_kernel_selection_validates_names_without_a_gpu():
     from pith_train_amd import _lib
 
