@@ -1091,9 +1091,10 @@ struct ExpertsNode : HipNode {
     }
     step.dgu.reset();
     step.dgu_s.reset();
-    if (!deferred) step.weight_gradient();
-    // rows that expand the same source row are summed (the backward of the expanding gather)
+    // rows that expand the same source row are summed (the backward of the expanding gather), right behind the GEMM
+    // that wrote them: after the weight gradient they come from HBM
     if (expand_idx) gx = scatter_sum(gx, *expand_idx, src_rows, kRowAlignment, (int64_t)stream);
+    if (!deferred) step.weight_gradient();
     if (repeat > 1) gx = gx.view({src_rows, repeat, d.K});
     return {gx, Tensor(), Tensor(), Tensor(), step.d_gu_bias.value_or(Tensor()), step.d_dn_bias.value_or(Tensor())};
   }
