@@ -130,7 +130,10 @@ def few_rows_per_expert(rows: int, num_groups: int) -> bool:
     """Whether a forward without a backward pads its groups to 64 rows instead of 128 and takes the GEMM tiles
     of that height.  Such a forward reads every expert's weights for a handful of rows, and half of a
     128-row tile would be padding; with more rows than this most groups need a second 64-row tile,
-    which reads the weight panel again."""
+    which reads the weight panel again.  Expert blocks (2048 x 768 x 128, 2048 x 1408 x 64 and 2880 x 2880 x 32
+    hidden x width x experts, equal popularity), us with 64 / 128 rows: 16 rows an expert 163 / 211, 143 / 174,
+    221 / 261; 48 178 / 217, 151 / 178, 224 / 264; 64 208 / 220, 175 / 181, 273 / 263; 80 237 / 225, 200 / 184,
+    301 / 273.  With Zipf-distributed popularity the gain ends between 40 and 80."""
     return rows <= 48 * num_groups
 
 
