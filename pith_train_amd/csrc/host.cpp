@@ -223,6 +223,11 @@ void require_shape(const Tensor& t, at::IntArrayRef shape, at::ScalarType type, 
     throw HipError(s.str());
   }
 }
+// An index that a kernel reads as 64-bit numbers.
+void require_index(const Tensor& t, const char* what) {
+  if (t.numel() > 0 && (t.dim() != 1 || t.scalar_type() != at::kLong))
+    throw py::type_error(std::string(what) + ": expected a one-dimensional int64 index, got " + c10::toString(t.scalar_type()));
+}
 // the FP8 bytes [G, N, K] of a grouped weight and the scales of its 128 x 128 blocks
 void require_operand(const Tensor& q, const Tensor& scale, int64_t G, int64_t N, int64_t K, const char* what) {
   require_shape(q, {G, N, K}, kFp8, what);
@@ -659,10 +664,6 @@ Tensor with_node(int64_t stream, Compute compute, Fill fill, const Inputs&... in
   return out;
 }
 
-Tensor or_zeros(const Tensor& grad, at::IntArrayRef shape, at::ScalarType type, const at::Device& dev) {
-  return grad.defined() ? grad : at::zeros(shape, at::TensorOptions().dtype(type).device(dev));
-}
-
 bool deferred_gradients() {  // WeightGradStore.enabled; needs the GIL
   return py::handle(g_store).attr("enabled").cast<bool>();
 }
@@ -708,6 +709,7 @@ struct GatherNode : HipNode {
 
 Tensor index_gather(const Tensor& input, const Tensor& index, int64_t alignment, int64_t stream) {
   require_same_device(input, {&index});
+  require_index(index, "padded_index_gather");
   return with_node<GatherNode>(
       stream,
       [&] {
@@ -760,10 +762,11 @@ Tensor permute_rows(const Tensor& input, const Tensor& src_of, const Tensor& off
 Tensor permute_into_buffer(const Tensor& input, const Tensor& src_of, const Tensor& offs, const Maybe& pre, int64_t stream) {
   const Tensor index = pre.value_or(Tensor());
   require_same_device(input, {&src_of, &offs, &index});
+  if (pre) require_index(*pre, "scatter_for_grouped_gemm: pre_index");
   at::AutoDispatchBelowADInplaceOrView guard;
-  const Tensor in = row_major(input);
+  const Tensor in = row_major(input), through = index.defined() ? index.contiguous() : Tensor();
   Tensor buf = empty({src_of.size(0), in.size(1)}, in.scalar_type(), in.device());
-  check(lib.pt_permute_rows(ptr(in), in.stride(0), ptr(buf), buf.stride(0), (const int32_t*)ptr(src_of), (const int64_t*)ptr(pre),
+  check(lib.pt_permute_rows(ptr(in), in.stride(0), ptr(buf), buf.stride(0), (const int32_t*)ptr(src_of), index.defined() ? (const int64_t*)ptr(through) : nullptr,
                             (const int32_t*)ptr(offs) + offs.size(0) - 1, (int32_t)kRowAlignment, buf.size(0), in.size(1), (int32_t)in.element_size(),
                             (pt_stream_t)stream), "pt_permute_rows");
   return buf;
@@ -1389,6 +1392,10 @@ std::pair<Tensor, Tensor> build_expert_idxs(const Tensor& counts, int64_t ep, in
 
 Tensor adjust_expand_idx(const Tensor& received, const Tensor& dedup, const Tensor& splits, int64_t stream) {
   require_same_device(received, {&dedup, &splits});
+  require_index(received, "adjust_expand_idx");
+  require_index(dedup, "adjust_expand_idx: rows from each rank");
+  require_index(splits, "adjust_expand_idx: splits");
+  if (splits.size(0) < dedup.size(0)) throw HipError("adjust_expand_idx: fewer splits than ranks");
   const Tensor r = received.contiguous(), sp = splits.contiguous();
   Tensor out = empty(r.sizes(), at::kLong, r.device());
   if (r.size(0))

@@ -118,6 +118,8 @@ class ScatterForGroupedGemm:
             return output_tokens, reverse, offs, ks_tensor, []
         expert_idxs = expert_idxs.contiguous()
         assert expert_idxs.dtype == torch.int64, "expert_idxs must be int64"
+        source = input_tokens if pre_index is None else pre_index
+        assert source.shape[0] >= m, f"{m} routed rows, {source.shape[0]} rows to take them from"
 
         max_m_padded = m + num_groups * (padding_alignment - 1)
         max_m_padded = -(-max_m_padded // _GEMM_ALLOC_ALIGNMENT) * _GEMM_ALLOC_ALIGNMENT

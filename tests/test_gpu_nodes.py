@@ -385,3 +385,26 @@ def test_peak_memory_of_an_expert_block_backward(hidden, inter):
     third = 2 * T * hidden + 3 * down
     assert peak <= 1.05 * (transposed + max(first, second, third)) + (4 << 20), (peak, transposed, first, second, third)
     assert grad[0].shape == x.shape
+
+
+def test_indices_of_other_types_and_lengths_are_refused():
+    """They go to kernels by address."""
+    from pith_train_amd.operators.ep_dispatch import adjust_expand_idx
+    from pith_train_amd.operators.token_scatter import padded_index_gather, scatter_for_grouped_gemm
+
+    x = _randn(6, 16)
+    index = torch.randint(0, 6, (20,), device="cuda")
+    with pytest.raises(TypeError, match="int64"):
+        padded_index_gather(x, index.int())
+    with pytest.raises(TypeError, match="int64"):
+        scatter_for_grouped_gemm(x, index % 4, 4, pre_index=index.int())
+    for keys, pre in ((index % 4, None), (index % 4, index[:10])):
+        with pytest.raises(AssertionError, match="rows"):
+            scatter_for_grouped_gemm(x, keys, 4, pre_index=pre)
+    counts = torch.tensor([2, 4], device="cuda")
+    with pytest.raises(TypeError, match="int64"):
+        adjust_expand_idx(index[:6].int(), counts, counts)
+    # a strided index is read as what it is
+    rows, reverse, *_ = scatter_for_grouped_gemm(x, index[::2] % 4, 4, pre_index=index[::2])
+    want = scatter_for_grouped_gemm(x, index[::2].contiguous() % 4, 4, pre_index=index[::2].contiguous())
+    assert torch.equal(rows, want[0]) and torch.equal(reverse, want[1])
