@@ -857,6 +857,9 @@ Maybe linear(const Tensor& x, const Tensor& weight, const Tensor& w_fp8, const T
     throw HipError("linear: an input of width " + std::to_string(x.size(1)) + " for a weight of " + std::to_string(w_fp8.size(0)) + " x " +
                    std::to_string(w_fp8.size(1)));
   if (!linear_supported(x, w_fp8.size(0)) || !w_fp8.is_contiguous() || !w_t.is_contiguous()) return std::nullopt;
+  const int64_t nb = cdiv(w_fp8.size(0), 128), kb = cdiv(w_fp8.size(1), 128);
+  require_shape(w_s, {nb, kb}, at::kFloat, "linear: scales of the quantised weight");
+  require_shape(w_ts, {kb, nb}, at::kFloat, "linear: scales of the transposed weight");
   return linear_node(x, weight, QuantisedWeight{w_fp8, w_s, w_t, w_ts}, nullptr, stream);
 }
 
@@ -921,10 +924,16 @@ std::pair<Maybe, std::optional<std::vector<Tensor>>> mlp(const Tensor& input, co
     const auto dev = input.device();
     const int64_t N = 2 * half, nb = cdiv(N, 128), kb = cdiv(K, 128), hb = half / 128, Hb = cdiv(H, 128);
     const Tensor x = row_major(input), wg = row_major(w_gate), wu = row_major(w_up), wd = row_major(w_down);
-    if (cached) t = *cached;
-    else t = {empty({N, K}, kFp8, dev), empty({nb, kb}, at::kFloat, dev), empty({K, N}, kFp8, dev), empty({kb, nb}, at::kFloat, dev),
+    if (cached) {
+      t = *cached;
+      if (t.size() != 8) throw HipError("mlp: eight quantised tensors");
+      const int64_t sizes[4][2] = {{N, K}, {K, N}, {H, half}, {half, H}};
+      for (int i = 0; i < 4; ++i) {
+        require_shape(t[2 * i], {sizes[i][0], sizes[i][1]}, kFp8, "mlp: quantised weight");
+        require_shape(t[2 * i + 1], {cdiv(sizes[i][0], 128), cdiv(sizes[i][1], 128)}, at::kFloat, "mlp: scales of a quantised weight");
+      }
+    } else t = {empty({N, K}, kFp8, dev), empty({nb, kb}, at::kFloat, dev), empty({K, N}, kFp8, dev), empty({kb, nb}, at::kFloat, dev),
               empty({H, half}, kFp8, dev), empty({Hb, hb}, at::kFloat, dev), empty({half, H}, kFp8, dev), empty({hb, Hb}, at::kFloat, dev)};
-    TORCH_CHECK(t.size() == 8, "mlp: eight quantised tensors");
     const int64_t ld_t = lib.pt_transposed_pitch(M);
     Tensor gate_up = empty({M, N}, bf16, dev), x_t, x_ts, h_t, h_ts;
     y = empty({M, H}, bf16, dev);

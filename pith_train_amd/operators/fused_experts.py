@@ -141,6 +141,9 @@ def _prepare(x, grouped_mm_offs, row_map, expand_idx, scatter):
     """The checked ``(row_map, expand_idx, scatter)`` of a block on ``x`` (a ``[T, k, K]`` view of one row per
     token counts as its T * k rows)."""
     _lib.require_cuda(x)
+    # three dimensions: one row per token, seen k times
+    assert x.dim() == 2 or (x.dim() == 3 and row_map is not None and expand_idx is None and (x.stride(1) == 0 or x.shape[1] == 1)), (
+        f"expected [rows, width] or an expanded [tokens, k, width] view, got {tuple(x.shape)} with strides {x.stride()}")
     assert expand_idx is None or row_map is not None, "expand_idx needs the row map of the scatter"
     if row_map is not None:
         assert row_map.dtype == torch.int32 and row_map.shape[0] % 128 == 0

@@ -408,3 +408,32 @@ def test_indices_of_other_types_and_lengths_are_refused():
     rows, reverse, *_ = scatter_for_grouped_gemm(x, index[::2] % 4, 4, pre_index=index[::2])
     want = scatter_for_grouped_gemm(x, index[::2].contiguous() % 4, 4, pre_index=index[::2].contiguous())
     assert torch.equal(rows, want[0]) and torch.equal(reverse, want[1])
+
+
+def test_kept_weights_and_repeated_rows_of_other_shapes_are_refused():
+    """A weight replaced under a cache that still counts as fresh; [T, k, H] rows that are not one row k times."""
+    from pith_train_amd._lib import PithTrainHipError
+    from pith_train_amd.modules.experts import DeepSeekV2MLP, Qwen3MoeExperts, forward_stage3
+    from pith_train_amd.operators.linear import FP8Linear
+    from pith_train_amd.operators.token_scatter import group_rows_with_sizes
+
+    mlp = DeepSeekV2MLP(128, 256).cuda().to(torch.bfloat16)
+    mlp(_randn(32, 128))
+    for m in (mlp.gate_proj, mlp.up_proj, mlp.down_proj):
+        m.weight = torch.nn.Parameter(torch.zeros((128, 128), device="cuda", dtype=torch.bfloat16))
+    with pytest.raises(PithTrainHipError, match="quantised"):
+        mlp(_randn(32, 128))
+    lin = FP8Linear(128, 64, bias=False, device="cuda", dtype=torch.bfloat16)
+    lin(_randn(32, 128))
+    q = list(lin._wq_cache)
+    q[1] = q[1][:, :0]
+    lin._wq_cache = tuple(q)
+    with pytest.raises(PithTrainHipError, match="scales"):
+        lin(_randn(32, 128))
+    experts, x = Qwen3MoeExperts(128, 128, 4).cuda().to(torch.bfloat16), _randn(24, 2, 128)
+    keys = torch.randint(0, 4, (48,), device="cuda")
+    _, offs, _, ks, src = group_rows_with_sizes(keys, 4, host_sizes=False)
+    for grad in (True, False):
+        with torch.set_grad_enabled(grad), pytest.raises(AssertionError, match="expanded"):
+            experts(x, offs, row_map=src)
+    assert forward_stage3(experts, x, keys, 4).shape == (48, 128)  # there such rows are copied
