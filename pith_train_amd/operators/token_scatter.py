@@ -127,9 +127,9 @@ class ScatterForGroupedGemm:
         reverse, offs, ks_tensor, src_of = group_rows(expert_idxs, num_groups, padding_alignment, max_m_padded)
         # The group sizes go to the host ahead of the row copy, and only they are waited for.
         ks_cpu = get_pinned_buffer("ks", num_groups, torch.int32)
-        copied = _copy_event()
+        copied = _copy_event(device)
         ks_cpu.copy_(ks_tensor, non_blocking=True)
-        copied.record()
+        copied.record(torch.cuda.current_stream(device))
         buffer = host.permute_into_buffer(input_tokens, src_of, offs, pre_index, stream)
         copied.synchronize()
         ks = ks_cpu.tolist()
@@ -140,11 +140,10 @@ class ScatterForGroupedGemm:
 _copy_events: dict[int, torch.cuda.Event] = {}
 
 
-def _copy_event() -> torch.cuda.Event:
-    device = torch.cuda.current_device()
-    event = _copy_events.get(device)
+def _copy_event(device: torch.device) -> torch.cuda.Event:
+    event = _copy_events.get(device.index)
     if event is None:
-        event = _copy_events[device] = torch.cuda.Event()
+        event = _copy_events[device.index] = torch.cuda.Event()
     return event
 
 
