@@ -1029,6 +1029,7 @@ Tensor grouped_linear(const Tensor& x, const Tensor& weight, const Tensor& offs,
       stream,
       [&] {
         const int64_t M = x.size(0), K = x.size(1), N = w.size(1), G = w.size(0);
+        if (weight.sizes() != w.sizes()) throw HipError("grouped linear: the quantised weight has another size than the weight");
         require_operand(w, w_s, G, N, K, "grouped weight");
         require_operand(dg, dg_s, G, forward_layout ? N : K, forward_layout ? K : N, "grouped weight of the input gradient");
         require_shape(offs, {G}, at::kInt, "group ends");
@@ -1142,6 +1143,10 @@ Tensor experts(const Tensor& input, const Tensor& w_gate, const Maybe& w_up, con
           if (!std::get<2>(q)) std::swap(rows, cols);
           require_operand(std::get<0>(q), std::get<1>(q), G, rows, cols, what);
         };
+        // the weight gradients are written to tensors of the parameters' sizes
+        const bool split = up.defined();
+        if (w_gate.sizes() != at::IntArrayRef({G, split ? half : N, K}) || (split && up.sizes() != w_gate.sizes()))
+          throw HipError("expert block: gate and up weights of other sizes than the down weight and the rows");
         dgrad(gu_dg, N, K, "gate_up weight of the input gradient");
         dgrad(dn_dg, H, half, "down weight of the input gradient");
         done = experts_forward(x, repeat, row_map, expand_idx, offs, std::get<0>(gu), std::get<1>(gu), std::get<0>(dn), std::get<1>(dn), w_down.size(2), c0,

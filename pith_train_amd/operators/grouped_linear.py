@@ -144,7 +144,8 @@ def m_grouped_fp8_gemm_nt(a, b, out: torch.Tensor, grouped_mm_offs: torch.Tensor
     may be given."""
     (a_fp8, a_s), (b_fp8, b_s) = a, b
     M, K = a_fp8.shape
-    G, N, _ = b_fp8.shape
+    G, N, Kb = b_fp8.shape
+    assert Kb == K, (b_fp8.shape, a_fp8.shape)
     if bias is not None:
         assert bias.shape == (G, N) and bias.dtype == out.dtype and bias.is_contiguous()
     if bias is not None and out_rows is not None:
@@ -185,6 +186,7 @@ def k_grouped_fp8_wgrad(dy_t, x_t, out: torch.Tensor, grouped_mm_offs, accumulat
     N, M = dy_fp8.shape
     K = x_fp8.shape[0]
     G = out.shape[0]
+    assert x_fp8.shape[1] == M and out.shape == (G, N, K) and out.is_contiguous(), (out.shape, dy_fp8.shape, x_fp8.shape)
     assert dy_fp8.is_contiguous() and x_fp8.is_contiguous() and dy_s.stride(-1) == 1 and x_s.stride(-1) == 1
     ld_dy = dy_s.stride(0) if dy_s.shape[0] > 1 else N
     ld_x = x_s.stride(0) if x_s.shape[0] > 1 else K

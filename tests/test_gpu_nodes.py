@@ -437,3 +437,24 @@ def test_kept_weights_and_repeated_rows_of_other_shapes_are_refused():
         with torch.set_grad_enabled(grad), pytest.raises(AssertionError, match="expanded"):
             experts(x, offs, row_map=src)
     assert forward_stage3(experts, x, keys, 4).shape == (48, 128)  # there such rows are copied
+
+
+def test_weights_replaced_under_a_kept_quantisation_are_refused():
+    """Their gradients would be written past a smaller tensor."""
+    from pith_train_amd._lib import PithTrainHipError
+    from pith_train_amd.modules.experts import Qwen3MoeExperts, Qwen35MoeExperts, forward_stage3
+
+    keys = torch.randint(0, 4, (48,), device="cuda")
+    for make, name, shape in ((Qwen3MoeExperts, "gate_proj", (4, 128, 64)), (Qwen3MoeExperts, "up_proj", (4, 128, 64)), (Qwen35MoeExperts, "gate_up_proj", (2, 256, 128))):
+        m = make(128, 128, 4).cuda().to(torch.bfloat16)
+        forward_stage3(m, _randn(48, 128), keys, 4)
+        for p in ("gate_proj", "up_proj") if make is Qwen3MoeExperts and name == "gate_proj" else (name,):
+            getattr(m, p).weight = torch.nn.Parameter(torch.zeros(shape, device="cuda", dtype=torch.bfloat16))
+        with pytest.raises((PithTrainHipError, AssertionError, RuntimeError)):
+            forward_stage3(m, _randn(48, 128), keys, 4)
+    m = Qwen3MoeExperts(128, 128, 2).cuda().to(torch.bfloat16)
+    kw = dict(grouped_mm_offs=torch.tensor([128, 256], dtype=torch.int32, device="cuda"))
+    m.gate_proj(_randn(256, 128), **kw)
+    m.gate_proj.weight = torch.nn.Parameter(torch.zeros((2, 64, 128), device="cuda", dtype=torch.bfloat16))
+    with pytest.raises(PithTrainHipError, match="another size"):
+        m.gate_proj(_randn(256, 128), **kw)
