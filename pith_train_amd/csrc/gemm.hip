@@ -286,37 +286,6 @@ static int gemm_impl() {
   return g_impl;
 }
 
-// Choice of the persistent kernel, from measurements on MI355X:
-//   m-grouped  the row-split loop: its loads never pause, which matters most where operands come from
-//              HBM (every group has its own b operand), and waves of a half-empty tile skip their
-//              MFMAs (us, against the software-pipelined loop: 32 groups of about 2048 rows, 5760 x
-//              2880 weights 1194 / 1250, of 1000 rows 602 / 645, 128 groups 873 / 880).
-//   k-grouped  the software-pipelined loop where a tile's reduction is long enough for its one barrier per
-//              block to count (both operands are shared by a whole group, no tile is half-empty): from
-//              768 rows a group on with up to 32 groups, from 1792 with more, where skewed groups leave
-//              many short tiles and the row-split loop, whose loads run on across tiles, is ahead.  Inside a
-//              step (us, row-split / pipelined): 16 Zipf-distributed groups of 896 rows in the mean 2048 x
-//              768 77 / 65 and 1536 x 2048 93 / 89; 32 equal groups of 1024 5760 x 2880 664 / 650, of 2048
-//              1230 / 1120; 64 Zipf-distributed groups of 768 2048 x 1408 298 / 311 and 2816 x 2048 454 / 471,
-//              of 1536 414 / 444 and 707 / 764, of 2048 562 / 557 and 1009 / 981; 128 of 1536 2048 x 512
-//              388 / 427; 128 equal groups of 768 1536 x 2048 421 / 420, of 2048 868 / 823.
-//              Split reductions: the pipelined loop for ranges up to 14336 (whole step of a linear, us:
-//              ranges of 12288 4096 -> 2048 700 / 688, 2048 -> 2816 570 / 561; of 14336 828 / 827 and 654 /
-//              657), the row-split one past it (16384: 2048 -> 4096 924-942 / 935-952, 4096 -> 2048
-//              918-924 / 919-928, 2048 -> 2816 723-729 / 739-745).
-//   dense      the software-pipelined loop from K = 512 on (+5 % at 512, +13..20 % from 2048 on
-//              over the two-phase loop, +5..8 % over the row-split loop); below, the two-phase loop,
-//              which has no fill/drain of one 128-block per tile.
-enum { KERNEL_TWO_PHASE, KERNEL_PIPELINED, KERNEL_ROWSPLIT };
-static int preferred_kernel(const GemmArgs& g) {
-  if (g.mode == GEMM_M_GROUPED) return KERNEL_ROWSPLIT;
-  if (g.mode == GEMM_K_GROUPED) {
-    const bool pipelined = g.offs ? g.red >= (g.G <= 32 ? 768 : 1792) * (int64_t)g.G : g.split_len <= 14336;
-    return pipelined ? KERNEL_PIPELINED : KERNEL_ROWSPLIT;
-  }
-  return g.red >= 512 ? KERNEL_PIPELINED : KERNEL_TWO_PHASE;
-}
-
 // Problems too small for 256 x 256 tiles to fill 256 compute units evenly go to the kernel with one 64 x 128
 // or 128 x 128 tile per workgroup and two workgroups per compute unit (gemm_small.hip): tile rows, or 0
 // when the persistent kernels are the better choice.  While all 64-row tiles run at once the smaller tile
@@ -393,11 +362,7 @@ static int dispatch_gemm(const GemmArgs& g, hipStream_t stream) {
   if (impl == IMPL_TILE || !fits) return launch_gemm<128, 128, 2, 2>(g, stream);
   if (impl == IMPL_AUTO) {
     if (const int rows = small_tile_rows(g)) return launch_gemm_small(g, rows, stream);
-    switch (preferred_kernel(g)) {
-      case KERNEL_ROWSPLIT: return launch_gemm_rowsplit(g, 0, stream);
-      case KERNEL_PIPELINED: return launch_gemm_pipelined(g, 0, stream);
-      default: return launch_gemm_persistent(g, 0, stream);
-    }
+    return launch_gemm_rowsplit(g, 0, stream);
   }
   if (impl >= IMPL_SMALL) return launch_gemm_small(g, impl - IMPL_SMALL, stream);
   if (impl >= IMPL_ROWSPLIT) return launch_gemm_rowsplit(g, impl - IMPL_ROWSPLIT, stream);

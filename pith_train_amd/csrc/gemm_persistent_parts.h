@@ -77,6 +77,20 @@ __device__ __forceinline__ void dma16_op(v4i rsrc, uint32_t voff, uint32_t soff,
                  "s"(soff), "s"(lds_off)
                  : "memory");
 }
+// the same at LDS byte lds_off + OFF
+template <int OPERAND, int OFF>
+__device__ __forceinline__ void dma16_at(v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds_off) {
+  soff = (uint32_t)__builtin_amdgcn_readfirstlane((int)soff);
+  lds_off = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_off);
+  if (OPERAND == 0)
+    asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen" PT_GEMM_LOAD_A_MOD " lds" ::"v"(voff), "s"(rsrc),
+                 "s"(soff), "s"(lds_off), "n"(OFF)
+                 : "memory", "scc");
+  else
+    asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen" PT_GEMM_LOAD_B_MOD " lds" ::"v"(voff), "s"(rsrc),
+                 "s"(soff), "s"(lds_off), "n"(OFF)
+                 : "memory", "scc");
+}
 __device__ __forceinline__ void dma4(v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds_off) {
   soff = (uint32_t)__builtin_amdgcn_readfirstlane((int)soff);
   lds_off = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_off);
@@ -210,6 +224,20 @@ __device__ __forceinline__ void store_single_bf16(const v16f& a, __amdgpu_buffer
     }
     __builtin_amdgcn_raw_buffer_store_b16((short)r, out, voff, s, 0);
   }
+}
+
+// The kernel's arguments read anew from where the launch left them (the kernel takes the block by value as its
+// only argument).  What a tile needs once need not stay in scalar registers during its main loop, nor be
+// spilled to vector registers: the compiler cannot see that these loads return what it has read before.
+__device__ __forceinline__ GemmArgs reload_args() {
+#ifdef __HIP_DEVICE_COMPILE__
+  typedef const GemmArgs __attribute__((address_space(4))) * ArgsPtr;
+  ArgsPtr q = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(q));
+  return *q;
+#else
+  return GemmArgs{};
+#endif
 }
 
 // One tile of the work list; everything is wave-uniform (SGPRs).
@@ -421,9 +449,11 @@ __device__ __forceinline__ void pin_acc(v16f& a) {
 // tile).  `stg` is the wave's 2 KiB LDS staging area.  PIN != 0: the accumulators were produced by
 // inline-assembly MFMAs; each block is handed to the compiler only right before its store, so
 // that it is converted and copied out one block at a time.
-template <int MODE, int TM, int TN, bool ACC, int PIN, bool PAIR = false>
+// EXTRAS: the output rows (out_row_index) and the bias of the tile lie in LDS, row wm0 and column wn0 of
+// the tile's at rows_lds[wm0] and bias_lds + 2 wn0: a load here would wait for every store before it.
+template <int MODE, int TM, int TN, bool ACC, int PIN, bool PAIR = false, bool EXTRAS = false>
 __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& p, const Tile& T, int wm0, int wn0, int lane,
-                                           uint8_t* stg) {
+                                           uint8_t* stg, const int* rows_lds = nullptr, const uint8_t* bias_lds = nullptr) {
   const uint32_t esz = p.out_dtype == PT_F32 ? 4 : 2;
   const uint32_t pitch = (uint32_t)p.ldo * esz;
   const bool pair_ok = p.out_dtype != PT_F32 && (p.ldo & 1) == 0 && (((uintptr_t)p.out) & 3) == 0;
@@ -478,7 +508,9 @@ __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& 
     for (int i = 0; i < TM; ++i) {
       // one index load for the block row (lane -> row lane%32), handed to the lanes that store the row
       const int r = T.a_row0 + wm0 + i * 32 + (lane & 31);
-      const int dst_of_lane = r < T.a_lim ? p.out_row_index[r] : -1;
+      int dst_of_lane = -1;
+      if (EXTRAS) { dst_of_lane = rows_lds[wm0 + i * 32 + (lane & 31)]; if (r >= T.a_lim) dst_of_lane = -1; }
+      else if (r < T.a_lim) dst_of_lane = p.out_row_index[r];
       uint32_t vrow[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -492,7 +524,8 @@ __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& 
 #pragma unroll
         for (int q = 0; q < 4; ++q) voff[q] = colc < T.b_lim ? vrow[q] : kOob;
         v4i bias = v4i{0, 0, 0, 0};
-        if (p.bias != nullptr && colc < T.b_lim) bias = *(const v4i*)((const char*)p.bias + ((int64_t)T.g * p.rows_b + colc) * 2);
+        if (EXTRAS) { if (p.bias != nullptr) bias = *(const v4i*)(bias_lds + (wn0 + j * 32 + (lane & 7) * 8) * 2); }
+        else if (p.bias != nullptr && colc < T.b_lim) bias = *(const v4i*)((const char*)p.bias + ((int64_t)T.g * p.rows_b + colc) * 2);
         pin_acc<PIN>(acc[i][j]); pin_acc<PIN>(acc[i][j + 1]);
         store_staged_bf16_lines<kStoreAux<MODE>>(acc[i][j], acc[i][j + 1], rs_sc, stg, voff, (uint32_t)(T.b_row0 + wn0 + j * 32) * 2, false, lane,
                                 p.bias != nullptr, bias);
@@ -504,7 +537,8 @@ __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& 
     for (int j = 0; j < TN; j += 2) {
       const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;
       v4i bias = v4i{0, 0, 0, 0};
-      if (has_bias && colc < T.b_lim) bias = *(const v4i*)((const char*)p.bias + ((int64_t)T.g * p.rows_b + colc) * 2);
+      if (EXTRAS) { if (has_bias) bias = *(const v4i*)(bias_lds + (wn0 + j * 32 + (lane & 7) * 8) * 2); }
+      else if (has_bias && colc < T.b_lim) bias = *(const v4i*)((const char*)p.bias + ((int64_t)T.g * p.rows_b + colc) * 2);
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         uint32_t voff[4];

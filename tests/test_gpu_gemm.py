@@ -408,3 +408,76 @@ def test_k_grouped_wgrad_on_column_slices_of_the_scale_array():
         out = torch.full((Gn, half, K), float("nan"), dtype=torch.bfloat16, device="cuda")
         k_grouped_fp8_wgrad((dy_t[lo : lo + half], dy_sc[:, lo : lo + half]), (x_t, x_sc), out, offs.cuda(), False)
         _check(out, ref, f"wgrad on scale columns {lo}..{lo + half}")
+
+
+@pytest.mark.parametrize("K", [128, 144, 256, 400])
+@pytest.mark.parametrize("sizes,N", [([128, 0, 384, 250], 8), ([300, 128], 264), ([640, 1], 520)])
+def test_m_grouped_scattered_rows_with_bias_of_short_reductions(sizes, N, K, gemm_kernel):
+    """Output rows and bias of a tile are fetched during its first reduction block, which here is the
+    only one or one of two to four; tiles end inside the columns.  Same bits as adding the bias to the
+    plain result and moving the rows."""
+    from pith_train_amd import _lib
+
+    if gemm_kernel == "t":
+        pytest.skip("the tile-per-workgroup kernel has no scattered store (the library refuses it)")
+    ks, offs = _groups(sizes)
+    M, Gn = int(offs[-1]), len(sizes)
+    a, sa, _, _ = Q.fp8cast_rowwise_colwise(_rand((M, K), M + K))
+    b, sb, _, _ = Q.fp8cast_blockwise_transpose_batched(_rand((Gn, N, K), N + K, 0.02))
+    a, sa, b, sb, offs, bias = a.cuda(), sa.cuda(), b.cuda(), sb.cuda(), offs.cuda(), _rand((Gn, N), K).cuda()
+    rows = torch.randperm(M, generator=torch.Generator().manual_seed(K)).int().cuda()
+    plain, out = (torch.empty((M, N), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    args = [_lib.ptr(a), _lib.ptr(sa), _lib.ptr(b), _lib.ptr(sb)]
+    dims = [_lib.dtype_code(torch.bfloat16), _lib.ptr(offs), Gn, M, N, K]
+    _lib.call("pt_gemm_m_grouped_nt", *args, _lib.ptr(plain), *dims, _lib.stream_ptr())
+    _lib.call("pt_gemm_m_grouped_nt_scatter_bias", *args, _lib.ptr(out), *dims, _lib.ptr(rows), M, _lib.ptr(bias), _lib.stream_ptr())
+    group = torch.repeat_interleave(torch.arange(Gn, device="cuda"), torch.diff(offs, prepend=offs.new_zeros(1)).long())
+    assert torch.equal(out[rows.long()], plain + bias[group])
+
+
+def test_grouped_work_lists_longer_than_the_tile_table(gemm_kernel):
+    """12800 large tiles, 50 for every workgroup, so that the table is filled a second time and the groups
+    are scanned again: the bits of the kernel that takes one small tile per workgroup.  m-grouped, then
+    k-grouped with empty groups among them."""
+    from pith_train_amd import _lib
+
+    if gemm_kernel != "auto":
+        pytest.skip("the test selects the kernels itself; run once")
+
+    def both(make):
+        out = []
+        for kernel in (b"r0", b"s128"):
+            _lib.call("pt_gemm_select_kernel", kernel)
+            out.append(make())
+        assert torch.equal(*out)
+
+    def fp8(*shape, seed):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        return torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # finite values below 2
+
+    def scale(*shape, seed):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        return torch.exp2(torch.randint(-6, 3, shape, device="cuda", generator=g).float())
+
+    G_, N, K = 100, 32768, 128
+    a, sa, b, sb = fp8(G_ * 128, K, seed=1), scale(G_ * 128, 1, seed=2), fp8(G_, N, K, seed=3), scale(G_, N // 128, 1, seed=4)
+    offs = torch.arange(1, G_ + 1, dtype=torch.int32, device="cuda") * 128
+
+    def m_grouped():
+        o = torch.empty((G_ * 128, N), dtype=torch.bfloat16, device="cuda")
+        _lib.call("pt_gemm_m_grouped_nt", _lib.ptr(a), _lib.ptr(sa), _lib.ptr(b), _lib.ptr(sb), _lib.ptr(o), _lib.dtype_code(o.dtype),
+                  _lib.ptr(offs), G_, G_ * 128, N, K, _lib.stream_ptr())
+        return o
+
+    both(m_grouped)
+    ks = torch.tensor([128, 0, 256, 128] * 32, dtype=torch.int32)
+    offs_k, M, W = torch.cumsum(ks, 0).int().cuda(), int(ks.sum()), 2560
+    d, sd, x, sx = fp8(W, M, seed=5), scale(M // 128, W, seed=6), fp8(W, M, seed=7), scale(M // 128, W, seed=8)
+
+    def k_grouped():
+        o = torch.empty((128, W, W), dtype=torch.bfloat16, device="cuda")
+        _lib.call("pt_gemm_k_grouped_wgrad", _lib.ptr(d), _lib.ptr(sd), _lib.ptr(x), _lib.ptr(sx), _lib.ptr(o), _lib.dtype_code(o.dtype), 0,
+                  _lib.ptr(offs_k), 128, M, W, W, _lib.stream_ptr())
+        return o
+
+    both(k_grouped)
