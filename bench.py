@@ -894,7 +894,7 @@ def main():
         },
         "roofline": {
             "bound": "mfma",
-            "kernel": "fp8_gemm_nt_rowsplit_kernel (grouped launches) / fp8_gemm_nt_pipelined_kernel (dense launches): every GEMM launch of the step, fwd, dgrad, wgrad; the library picks the main loop per mode and shape",
+            "kernel": "fp8_gemm_nt_rowsplit_kernel: every GEMM launch of the step, fwd, dgrad, wgrad",
             "achieved": achieved,
             "peak": FP8_DENSE_PEAK_TFLOPS,
             "unit": "TFLOP/s",

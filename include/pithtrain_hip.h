@@ -357,8 +357,9 @@ int pt_gemm_k_grouped_wgrad_pair(const void* dy_t_fp8, const float* dy_scale, co
 
 /* Which GEMM kernel the three entry points above launch: "auto" (or NULL: per call from the
  * shape; the default unless the environment variable PT_GEMM_IMPL names one of the others),
- * "p0" persistent kernel with the two-phase main loop, "q0" / "q1" persistent kernel with the
- * software-pipelined main loop (8 / 4 waves per workgroup), "t" one 128x128 tile per workgroup.
+ * "r0" persistent kernel, one 256x256 tile after the other per compute unit ("p0", "q0" and "q1", names of
+ * main loops that it has replaced, mean the same), "s64" / "s128" one 64x128 / 128x128 tile per workgroup
+ * (small problems), "t" one 128x128 tile per workgroup through 64-bit addresses.
  * Every choice computes the same function; this exists for measurements and for tests that
  * cover each kernel.  Process-wide, not synchronised with concurrent GEMM calls.
  * No counterpart in the reference (DeepGEMM selects its kernels internally). */

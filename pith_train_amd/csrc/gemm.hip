@@ -262,17 +262,15 @@ static int launch_gemm(const GemmArgs& a, hipStream_t stream) {
 }
 
 // PT_GEMM_IMPL overrides the choice of kernel for measurements: "t" = one 128x128 tile per
-// workgroup, "p0" = persistent two-phase kernel, "q0" / "q1" = persistent software-pipelined kernel
-// (8 / 4 waves), "r0" = persistent kernel with the row-split loop, "s64" / "s128" = one 64 / 128 x 128
-// tile per workgroup with a deep load ring.  Unset: chosen per call from the shape (below).
-enum { IMPL_UNSET = -3, IMPL_AUTO = -2, IMPL_TILE = -1, IMPL_PIPELINED = 100, IMPL_ROWSPLIT = 200, IMPL_SMALL = 1000 };
+// workgroup, "r0" = persistent kernel with the row-split loop ("p0", "q0", "q1", names of main loops that it
+// has replaced, mean the same), "s64" / "s128" = one 64 / 128 x 128 tile per workgroup with a deep load
+// ring.  Unset: chosen per call from the shape (below).
+enum { IMPL_UNSET = -3, IMPL_AUTO = -2, IMPL_TILE = -1, IMPL_ROWSPLIT = 0, IMPL_SMALL = 1000 };
 static int g_impl = IMPL_UNSET;
 static bool parse_impl(const char* e, int& impl) {
   if (!e || !*e || !strcmp(e, "auto")) impl = IMPL_AUTO;
   else if (!strcmp(e, "t")) impl = IMPL_TILE;
-  else if (!strcmp(e, "p0")) impl = 0;
-  else if (!strcmp(e, "q0") || !strcmp(e, "q1")) impl = IMPL_PIPELINED + (e[1] - '0');
-  else if (!strcmp(e, "r0")) impl = IMPL_ROWSPLIT;
+  else if (!strcmp(e, "r0") || !strcmp(e, "p0") || !strcmp(e, "q0") || !strcmp(e, "q1")) impl = IMPL_ROWSPLIT;
   else if (!strcmp(e, "s64")) impl = IMPL_SMALL + 64;
   else if (!strcmp(e, "s128")) impl = IMPL_SMALL + 128;
   else return false;
@@ -288,8 +286,8 @@ static int gemm_impl() {
 
 // Problems too small for 256 x 256 tiles to fill 256 compute units evenly go to the kernel with one 64 x 128
 // or 128 x 128 tile per workgroup and two workgroups per compute unit (gemm_small.hip): tile rows, or 0
-// when the persistent kernels are the better choice.  While all 64-row tiles run at once the smaller tile
-// wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 25.0 for the pipelined kernel).  Then both
+// when the persistent kernel is the better choice.  While all 64-row tiles run at once the smaller tile
+// wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 25.0 for the large one).  Then both
 // kinds are priced in rounds of the GPU: a round of 256 large tiles is the unit, a round of 512 small ones
 // (a quarter of the area each, half of it in all) costs 0.57 of it in the m-grouped mode (0.68 with a
 // reduction-major b, whose fragments take twice the LDS reads), 0.65 in
@@ -327,7 +325,7 @@ static int small_tile_rows(const GemmArgs& g) {
   return (small + cdiv(small, 512) * 512) * price * 105 < cdiv(large, 256) * (2 * 512 * 100) * 100 ? 128 : 0;
 }
 
-// The persistent kernels address operands through 32-bit buffer offsets (signed range for the
+// The persistent kernel addresses operands through 32-bit buffer offsets (signed range for the
 // loads, whose out-of-range marker is bit 31) and the result through an unsigned 32-bit byte
 // offset from the start of the output (of one group's block in the k-grouped mode, of the
 // scattered output when rows are stored through an index).  Larger problems go to the
@@ -353,7 +351,7 @@ static int dispatch_gemm(const GemmArgs& g, hipStream_t stream) {
                      "and an output below 4 GiB through 32-bit byte offsets; larger problems take the NT entry point on the "
                      "transposed operand");
     const int rows = impl >= IMPL_SMALL ? impl - IMPL_SMALL : impl == IMPL_AUTO ? small_tile_rows(g) : 0;
-    return rows ? launch_gemm_small(g, rows, stream) : launch_gemm_rowsplit(g, 0, stream);
+    return rows ? launch_gemm_small(g, rows, stream) : launch_gemm_rowsplit(g, stream);
   }
   PT_REQUIRE((!g.out_row_index && !g.bias && !g.head_a) || (impl != IMPL_TILE && fits),
              "gemm: scattered output rows, per-head outputs and the fused bias need the persistent kernels, which address every operand and "
@@ -362,12 +360,8 @@ static int dispatch_gemm(const GemmArgs& g, hipStream_t stream) {
   if (impl == IMPL_TILE || !fits) return launch_gemm<128, 128, 2, 2>(g, stream);
   if (impl == IMPL_AUTO) {
     if (const int rows = small_tile_rows(g)) return launch_gemm_small(g, rows, stream);
-    return launch_gemm_rowsplit(g, 0, stream);
   }
-  if (impl >= IMPL_SMALL) return launch_gemm_small(g, impl - IMPL_SMALL, stream);
-  if (impl >= IMPL_ROWSPLIT) return launch_gemm_rowsplit(g, impl - IMPL_ROWSPLIT, stream);
-  if (impl >= IMPL_PIPELINED) return launch_gemm_pipelined(g, impl - IMPL_PIPELINED, stream);
-  return launch_gemm_persistent(g, impl, stream);
+  return impl >= IMPL_SMALL ? launch_gemm_small(g, impl - IMPL_SMALL, stream) : launch_gemm_rowsplit(g, stream);
 }
 
 }  // namespace pt
@@ -376,7 +370,7 @@ using namespace pt;
 
 extern "C" int pt_gemm_select_kernel(const char* name) {
   int impl;
-  PT_REQUIRE(parse_impl(name, impl), "gemm_select_kernel: unknown kernel '%s' (auto, p0, q0, q1, r0, s64, s128, t)", name);
+  PT_REQUIRE(parse_impl(name, impl), "gemm_select_kernel: unknown kernel '%s' (auto, r0, s64, s128, t; p0, q0 and q1 mean r0)", name);
   g_impl = impl;
   return PT_OK;
 }

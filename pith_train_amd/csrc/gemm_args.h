@@ -42,12 +42,8 @@ __device__ __forceinline__ int k_group_end(const GemmArgs& p, int g) {
 }
 
 
-// persistent kernel with the two-phase main loop (gemm_persistent.hip); variant selects the wave layout
-int launch_gemm_persistent(const GemmArgs& a, int variant, hipStream_t stream);
-// persistent kernel with the software-pipelined main loop (gemm_pipelined.hip)
-int launch_gemm_pipelined(const GemmArgs& a, int variant, hipStream_t stream);
 // persistent kernel whose two steps per 128-block split the tile by rows (gemm_rowsplit.hip)
-int launch_gemm_rowsplit(const GemmArgs& a, int variant, hipStream_t stream);
+int launch_gemm_rowsplit(const GemmArgs& a, hipStream_t stream);
 // one tile of 64 or 128 rows x 128 columns per workgroup, for small problems (gemm_small.hip)
 int launch_gemm_small(const GemmArgs& a, int rows, hipStream_t stream);
 // the tiles of two independent dense products in one launch of that kernel

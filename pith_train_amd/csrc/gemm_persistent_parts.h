@@ -1,6 +1,6 @@
-// Parts shared by the two persistent FP8 GEMM kernels (two-phase and software-pipelined main
-// loops): buffer descriptors and direct-to-LDS loads, the work list (group scan, tile geometry),
-// the result stores, and the launch of one workgroup per CU.
+// Parts of the persistent FP8 GEMM kernel (gemm_rowsplit.hip), some of them shared with the kernel for small
+// problems (gemm_small.hip): buffer descriptors and direct-to-LDS loads, the work list (group scan, tile
+// geometry), the result stores, and the launch of one workgroup per CU.
 #pragma once
 #include "common.h"
 #include "gemm_args.h"
@@ -64,20 +64,7 @@ __device__ __forceinline__ void dma16(v4i rsrc, uint32_t voff, uint32_t soff, ui
                "s"(lds_off)
                : "memory");
 }
-template <int OPERAND>  // 0: a, 1: b
-__device__ __forceinline__ void dma16_op(v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds_off) {
-  soff = (uint32_t)__builtin_amdgcn_readfirstlane((int)soff);
-  lds_off = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_off);
-  if (OPERAND == 0)
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen" PT_GEMM_LOAD_A_MOD " lds" ::"v"(voff), "s"(rsrc),
-                 "s"(soff), "s"(lds_off)
-                 : "memory");
-  else
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen" PT_GEMM_LOAD_B_MOD " lds" ::"v"(voff), "s"(rsrc),
-                 "s"(soff), "s"(lds_off)
-                 : "memory");
-}
-// the same at LDS byte lds_off + OFF
+// the same at LDS byte lds_off + OFF; OPERAND 0: a, 1: b
 template <int OPERAND, int OFF>
 __device__ __forceinline__ void dma16_at(v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds_off) {
   soff = (uint32_t)__builtin_amdgcn_readfirstlane((int)soff);
@@ -249,17 +236,14 @@ struct Tile {
 // 2 * op_sel_hi bit, one pair per operand).  Issued as volatile inline assembly with a memory
 // clobber: the compiler keeps such statements, and every memory operation between them, in source
 // order, which is what pins the interleaving of MFMAs, LDS reads and direct-to-LDS loads in the
-// main loop.  AGPR: the accumulator lives in the accumulation registers ("a" constraint), which a
-// wave with 256 accumulator values needs; with 128 it lives in ordinary registers ("v"), where the
-// epilogue reads it without a copy and shares one register pool with everything else.
-template <bool AGPR>
+// main loop.  The accumulators live in ordinary registers ("v"; 128 of them fit next to everything else in the
+// 256 a wave has at two waves per SIMD), where the epilogue reads them without a copy.
 __device__ __forceinline__ void mfma_sel(const v8i& a, const v8i& b, v16f& c, int ia, int sa, int ib, int sb) {
 #define PT_MFMA_TEXT(S0, S1, H0, H1) \
   "v_mfma_scale_f32_32x32x64_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[" #S0 "," #S1 ",0] op_sel_hi:[" #H0 "," #H1 ",0]"
 #define PT_MFMA(IA, IB, S0, S1, H0, H1)                                                                                  \
   case IA * 4 + IB:                                                                                                      \
-    if constexpr (AGPR) asm volatile(PT_MFMA_TEXT(S0, S1, H0, H1) : "+a"(c) : "v"(a), "v"(b), "v"(sa), "v"(sb) : "memory"); \
-    else asm volatile(PT_MFMA_TEXT(S0, S1, H0, H1) : "+v"(c) : "v"(a), "v"(b), "v"(sa), "v"(sb) : "memory");               \
+    asm volatile(PT_MFMA_TEXT(S0, S1, H0, H1) : "+v"(c) : "v"(a), "v"(b), "v"(sa), "v"(sb) : "memory");                  \
     break;
   switch (ia * 4 + ib) {
     PT_MFMA(0, 0, 0, 0, 0, 0) PT_MFMA(0, 1, 0, 1, 0, 0) PT_MFMA(0, 2, 0, 0, 0, 1) PT_MFMA(0, 3, 0, 1, 0, 1)
@@ -437,21 +421,20 @@ __device__ __forceinline__ void decode_tile(const GemmArgs& p, const int* s_pref
   }
 }
 
-// Hands one accumulator block produced by inline-assembly MFMAs to the compiler: PIN 1 = it lives
-// in the accumulation registers, 2 = in ordinary registers, 0 = the compiler produced it itself.
-template <int PIN>
+// Hands one accumulator block produced by inline-assembly MFMAs to the compiler (PIN; otherwise the compiler
+// produced it itself).
+template <bool PIN>
 __device__ __forceinline__ void pin_acc(v16f& a) {
-  if constexpr (PIN == 1) asm volatile("" : "+a"(a));
-  else if constexpr (PIN == 2) asm volatile("" : "+v"(a));
+  if constexpr (PIN) asm volatile("" : "+v"(a));
 }
 
 // Writes one wave's TM x TN blocks of 32 x 32 results of tile T (rows wm0.., columns wn0.. of the
-// tile).  `stg` is the wave's 2 KiB LDS staging area.  PIN != 0: the accumulators were produced by
+// tile).  `stg` is the wave's 2 KiB LDS staging area.  PIN: the accumulators were produced by
 // inline-assembly MFMAs; each block is handed to the compiler only right before its store, so
 // that it is converted and copied out one block at a time.
 // EXTRAS: the output rows (out_row_index) and the bias of the tile lie in LDS, row wm0 and column wn0 of
 // the tile's at rows_lds[wm0] and bias_lds + 2 wn0: a load here would wait for every store before it.
-template <int MODE, int TM, int TN, bool ACC, int PIN, bool PAIR = false, bool EXTRAS = false>
+template <int MODE, int TM, int TN, bool ACC, bool PIN, bool PAIR = false, bool EXTRAS = false>
 __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& p, const Tile& T, int wm0, int wn0, int lane,
                                            uint8_t* stg, const int* rows_lds = nullptr, const uint8_t* bias_lds = nullptr) {
   const uint32_t esz = p.out_dtype == PT_F32 ? 4 : 2;

@@ -366,7 +366,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
           const int i = m & 1, j = (m >> 1) & 1, ks = m >> 2;
           const int late = BT ? ks : j, early = BT ? j : ks;
           if (wave_active) {
-            mfma_sel<false>(fa[2 * ks + i], fb[late][early], acc[i][j], i, sca, j, scb);
+            mfma_sel(fa[2 * ks + i], fb[late][early], acc[i][j], i, sca, j, scb);
           }
           if (m < NX) issue_o(m);
           if (m == 0) { if (BT) fa[2] = read_a(0, 1); else fb[1][0] = read_b(1, 0); }
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
           const int i = m & 1, j = (m >> 1) & 1, ks = m >> 2;
           const int late = BT ? ks : j, early = BT ? j : ks;
           if (wave_active) {
-            mfma_sel<false>(fa[2 * ks + i], fb[late][early], acc[2 + i][j], 2 + i, sca, j, scb);
+            mfma_sel(fa[2 * ks + i], fb[late][early], acc[2 + i][j], 2 + i, sca, j, scb);
           }
           if (m < NY) issue_e(m);
           if (m == 0) fa[2] = read_a(2, 1);
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
       // not kept (or spilled, and reloaded behind a wait for every store so far) across the main loop
       int el = lane;
       asm volatile("" : "+v"(el));
-      store_tile<MODE, TM, TN, ACC, 2, PAIR, true>(acc, reload_args(), C, wm0, wn0, el, lds + kRsStaging + wave * 2048,
+      store_tile<MODE, TM, TN, ACC, true, PAIR, true>(acc, reload_args(), C, wm0, wn0, el, lds + kRsStaging + wave * 2048,
                                                    (const int*)(lds + kRsIndex), lds + kRsBias);
     }
   }
@@ -454,13 +454,10 @@ static int launch_mode(const GemmArgs& a, hipStream_t stream) {
   }
 }
 
-int launch_gemm_rowsplit(const GemmArgs& a, int variant, hipStream_t stream) {
+int launch_gemm_rowsplit(const GemmArgs& a, hipStream_t stream) {
   PT_REQUIRE(a.mode == GEMM_DENSE || a.G <= kMaxGroupsGemm, "gemm: at most %d groups", kMaxGroupsGemm);
   PT_REQUIRE(!a.b_kmajor || a.mode == GEMM_M_GROUPED, "gemm: a reduction-major b operand is built for the m-grouped mode only");
-  switch (variant) {
-    case 0: return launch_mode<256, 256, 2, 4>(a, stream);  // 8 waves, 128 x 64 per wave
-  }
-  PT_REQUIRE(false, "gemm: unknown variant %d", variant);
+  return launch_mode<256, 256, 2, 4>(a, stream);  // 8 waves, 128 x 64 per wave
 }
 
 }  // namespace pt

@@ -13,7 +13,7 @@
 // 2048 268 MB in 19.3 us, 4096 x 512 x 4096 201 MB in 18.5, 4096 x 4096 x 512 134 MB in 15.1: 9 to 14 TB/s.
 //
 // Operand layouts in LDS, direct-to-LDS loads, scale handling and result stores are those of the
-// persistent kernels (gemm_persistent_parts.h); the MFMAs run in the same order, so the results have
+// persistent kernel (gemm_rowsplit.hip, gemm_persistent_parts.h); the MFMAs run in the same order, so the results have
 // the same bits.
 #include "gemm_persistent_parts.h"
 
@@ -203,7 +203,7 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
   wait_all_vmem();  // nothing may still be writing into this workgroup's LDS when it retires
   if (MODE == GEMM_K_GROUPED && nk == 0 && ACC) return;
   __syncthreads();  // every wave has read its last stage and has nothing in flight: the ring's memory is free
-  store_tile<MODE, TM, TN, ACC, 0, MODE == GEMM_K_GROUPED>(acc, p, T, wm0, wn0, lane, lds + wave * 2048);
+  store_tile<MODE, TM, TN, ACC, false, MODE == GEMM_K_GROUPED>(acc, p, T, wm0, wn0, lane, lds + wave * 2048);
 }
 
 template <int MODE, int BM, bool ACC, bool BT>
