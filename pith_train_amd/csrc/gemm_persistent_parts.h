@@ -92,124 +92,116 @@ __device__ __forceinline__ uint32_t pack2_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, h);
 }
 
-// ---- epilogue of one 32x32 accumulator tile.  The lane holds column (lane&31) and rows
-// 8*(v/4) + 4*(lane>>5) + (v&3).  voff is the lane's byte offset inside the tile (kOob if its
-// column is out of range); soff the uniform byte offset of the tile's row 0, column 0; pitch the
-// row pitch in bytes. ----
-__device__ __forceinline__ void store_f32(const v16f& a, __amdgpu_buffer_rsrc_t out, uint32_t voff, uint32_t soff,
-                                          uint32_t pitch, bool accumulate) {
+// ---- result stores -------------------------------------------------------------------------
+// The products are computed with the b fragment as the first MFMA operand, so that a lane holds one row of
+// the result: row lane % 32 of a 32x32 block, columns 8 (v / 4) + 4 (lane / 32) + v % 4, i.e. four
+// neighbouring columns per register quad.  A wave turns 32 rows x 128 bytes (two blocks of bf16, one of
+// fp32) into whole lines through a 4 KiB staging area of its own, four pieces of 8 rows: 8- or 16-byte LDS
+// writes, then four times a 16-byte read and a store of eight full lines.  With a lane per column every bf16 pair
+// had to be traded with the neighbouring lane first and went to LDS in 4-byte writes: us with that / with
+// this / with raw accumulator bits stored instead, 128 groups of 512 rows 1536 x 2048 243 / 238 / 233, 2048 x
+// 768 137 / 132 / 128, their weight gradients 297 / 291 / 290 and 135 / 127 / 119.  (Half lines cost a
+// tenth of the dense and a quarter of the weight-gradient GEMM's time in the write path; the memory
+// pipeline spends the same time on a 4-byte and on a 16-byte store.)
+// Only this wave touches its staging area, and the LDS executes one wave's operations in order, so the
+// phases need compiler fences only.
+struct Staging {
+  uint32_t wr;     // the lane's place for row lane % 32, chunk 0 of the swizzle (LDS byte address)
+  uint32_t rd[4];  // the lane's 16 bytes of piece q: row 8 q + lane / 8, chunk lane % 8
+};
+// Chunk c (16 bytes) of row m lies at position c ^ (m / 2) % 8: the 16 rows that an 8-byte write touches
+// at a time spread over all banks, and so do the 8 of a 16-byte one.
+__device__ __forceinline__ Staging make_staging(const uint32_t (&piece)[4], int lane) {
+  Staging s;
+  const int m = lane & 31, r = lane >> 3;
+  const uint32_t lo = lane & 8 ? piece[1] : piece[0], hi = lane & 8 ? piece[3] : piece[2];
+  s.wr = (lane & 16 ? hi : lo) + (m & 7) * 128 + (((m >> 1) & 7) << 4);
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const uint32_t s = soff + (8 * (v >> 2) + (v & 3)) * pitch;
-    float x = a[v];
-    if (accumulate) x += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(out, voff, s, 0));
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, x), out, voff, s, 0);
-  }
+  for (int q = 0; q < 4; ++q) s.rd[q] = piece[q] + r * 128 + (((lane & 7) ^ ((4 * q + (r >> 1)) & 7)) << 4);
+  return s;
 }
-// bf16: lanes 2c and 2c+1 trade one value of each register pair so that each stores two adjacent
-// columns of one row as a dword (the odd lane writes one row below the even lane; voff already
-// says so).  Needs an even row pitch in elements.
-__device__ __forceinline__ void store_pairs_bf16(const v16f& a, __amdgpu_buffer_rsrc_t out, uint32_t voff, uint32_t soff,
-                                                 uint32_t pitch, bool accumulate, bool odd) {
-#pragma unroll
-  for (int v = 0; v < 16; v += 2) {
-    const float x0 = a[v], x1 = a[v + 1];
-    const float send = odd ? x0 : x1;
-    const float recv = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), 0xB1, 0xF, 0xF, false));
-    const uint32_t s = soff + (8 * (v >> 2) + (v & 3)) * pitch;
-    // round the GEMM result to bf16 first, then add: the two roundings of `grad += wgrad.to(bf16)`
-    uint32_t w = odd ? pack2_bf16(recv, x1) : pack2_bf16(x0, recv);
-    if (accumulate) {
-      const uint32_t old = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(out, voff, s, 0);
-      w = pack2_bf16(bf16_lo(old) + bf16_lo(w), bf16_hi(old) + bf16_hi(w));
-    }
-    __builtin_amdgcn_raw_buffer_store_b32((int)w, out, voff, s, 0);
-  }
-}
-// bf16 through a per-wave LDS staging tile: the accumulator layout (a lane owns one column) is
-// turned into rows so that every lane stores 16 contiguous bytes.  Two horizontally adjacent
-// 32x32 blocks (64 columns: one 128-byte line per row) go through the 2 KiB tile 16 rows at a
-// time, and each store instruction then writes 8 whole 128-byte lines.  (Half lines - one block,
-// 16 rows x 64 B per instruction - cost a tenth of the dense and a quarter of the weight-gradient
-// GEMM's time in the write path; the memory pipeline spends the same time on a 4-byte and on a
-// 16-byte store instruction, which is why the stores are wide in the first place.)  Only this wave
-// touches its staging tile, and the LDS executes one wave's operations in order, so the phases
-// need compiler fences only.
-// voff[q]: the lane's byte offset for tile rows 8q + lane/8, q = 0..3 (row start + 16-byte chunk
-// lane%8, or kOob); soff: uniform byte offset added to all of them.
-// bias (with has_bias): the 8 values of the lane's columns, added in the output type after the
-// result has been rounded to it (x + bias[group] as a second operation on the rounded x).
-template <int AUX = 0>
-__device__ __forceinline__ void store_staged_bf16_lines(const v16f& a0, const v16f& a1, __amdgpu_buffer_rsrc_t out, uint8_t* stg,
-                                                        const uint32_t (&voff)[4], uint32_t soff, bool accumulate, int lane,
-                                                        bool has_bias = false, v4i bias = v4i{0, 0, 0, 0}) {
-  const bool odd = lane & 1;
-  uint8_t* wr = stg + (4 * (lane >> 5) + (odd ? 1 : 0)) * 128 + ((lane & 31) >> 1) * 4;
-  const uint8_t* rd = stg + (lane >> 3) * 128 + (lane & 7) * 16;
-  // p = (row r | row r+1) of the lane's column; the even lane of a pair takes both low halves (row r,
-  // columns c and c+1), the odd lane both high halves (row r+1): one byte permute of own and neighbour
-  const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
-#ifdef PT_GEMM_ABLATE_STAGING
-  // measurement build: the stores carry raw accumulator bits, no conversion and no staging
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const v16f& a = hf ? a1 : a0;
-      v4i w = v4i{__float_as_int(a[8 * h]), __float_as_int(a[8 * h + 1]), __float_as_int(a[8 * h + 2]), __float_as_int(a[8 * h + 3])};
-      __builtin_amdgcn_raw_buffer_store_b128(w, out, voff[2 * hf + h], soff, AUX);
-      asm volatile("s_nop 4" ::"v"(w) : "memory");
-    }
-  return;
-#endif
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {  // tile rows 0-15, then 16-31
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const v16f& a = b ? a1 : a0;
-#pragma unroll
-      for (int v = 8 * hf; v < 8 * hf + 8; v += 2) {
-        const uint32_t pk = pack2_bf16(a[v], a[v + 1]);
-        const uint32_t nb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)pk, 0xB1, 0xF, 0xF, false);
-        *(uint32_t*)(wr + (8 * ((v >> 2) & 1) + (v & 3)) * 128 + b * 64) = __builtin_amdgcn_perm(nb, pk, sel);
-      }
-    }
-    asm volatile("" ::: "memory");  // the reads below alias the writes above
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      v4i w = *(const v4i*)(rd + h * 1024);
-      const uint32_t vo = voff[2 * hf + h];
-      if (has_bias) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          w[q] = (int)pack2_bf16(bf16_lo((uint32_t)w[q]) + bf16_lo((uint32_t)bias[q]), bf16_hi((uint32_t)w[q]) + bf16_hi((uint32_t)bias[q]));
-      }
-      if (accumulate) {
-        const v4i old = __builtin_amdgcn_raw_buffer_load_b128(out, vo, soff, 0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          w[q] = (int)pack2_bf16(bf16_lo((uint32_t)old[q]) + bf16_lo((uint32_t)w[q]), bf16_hi((uint32_t)old[q]) + bf16_hi((uint32_t)w[q]));
-      }
-      __builtin_amdgcn_raw_buffer_store_b128(w, out, vo, soff, AUX);
-      // A 16-byte store reads its data registers for a few cycles after it issues; the compiler
-      // only guards that window for stores without a scalar offset, so hold the registers here.
-      asm volatile("s_nop 4" ::"v"(w) : "memory");
-    }
-    asm volatile("" ::: "memory");  // the next half's writes alias these reads
-  }
+typedef int v2i __attribute__((ext_vector_type(2)));
+#define PT_LDS(TYPE, ADDR) (*(TYPE __attribute__((address_space(3)))*)(uintptr_t)(ADDR))
+
+// A 16-byte store reads its data registers for a few cycles after it issues; the compiler only guards that
+// window for stores without a scalar offset, so the registers are held here.
+template <int AUX>
+__device__ __forceinline__ void store16(v4i w, __amdgpu_buffer_rsrc_t out, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_buffer_store_b128(w, out, voff, soff, AUX);
+  asm volatile("s_nop 4" ::"v"(w) : "memory");
 }
 
-__device__ __forceinline__ void store_single_bf16(const v16f& a, __amdgpu_buffer_rsrc_t out, uint32_t voff, uint32_t soff,
-                                                  uint32_t pitch, bool accumulate) {
+// Writes two horizontally adjacent blocks as bf16 (one block as fp32) to the staging area, and reads back the
+// lane's 16 bytes of each piece.
+__device__ __forceinline__ void stage_bf16(const v16f& a0, const v16f& a1, const Staging& stg, int lane) {
+  const uint32_t wr = stg.wr + (lane >> 5) * 8;
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const v16f& a = b ? a1 : a0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      PT_LDS(v2i, wr ^ ((4 * b + q) << 4)) = v2i{(int)pack2_bf16(a[4 * q], a[4 * q + 1]), (int)pack2_bf16(a[4 * q + 2], a[4 * q + 3])};
+  }
+}
+__device__ __forceinline__ void stage_f32(const v16f& a, const Staging& stg, int lane) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    PT_LDS(v4i, stg.wr ^ ((2 * q + (lane >> 5)) << 4)) =
+        v4i{__float_as_int(a[4 * q]), __float_as_int(a[4 * q + 1]), __float_as_int(a[4 * q + 2]), __float_as_int(a[4 * q + 3])};
+}
+// A column of TM blocks (pairs of them as bf16) through the staging area: emit(i, q, w) gets the 16 bytes of rows
+// 8 q + lane / 8 of block row i.  One block row after the other (scheduling barriers: converted all at once they
+// would not fit next to the accumulators).
+template <bool F32, int TM, int TN, class Emit>
+__device__ __forceinline__ void stage_column(const v16f (&acc)[TM][TN], int j, const Staging& stg, int lane, Emit emit) {
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    if (F32) stage_f32(acc[i][j], stg, lane);
+    else     stage_bf16(acc[i][j], acc[i][j + 1], stg, lane);
+    asm volatile("" ::: "memory");  // the reads alias the writes before and behind them
+    v4i w[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = PT_LDS(const v4i, stg.rd[q]);
+#ifdef PT_GEMM_ABLATE_STAGING
+    // measurement build: the stores carry raw accumulator bits, no conversion and no staging
+    for (int q = 0; q < 4; ++q) w[q] = v4i{__float_as_int(acc[i][j][4 * q]), __float_as_int(acc[i][j][4 * q + 1]), __float_as_int(acc[i][j][4 * q + 2]), __float_as_int(acc[i][j][4 * q + 3])};
+#endif
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) emit(i, q, w[q]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// x + y on packed bf16 pairs
+__device__ __forceinline__ v4i add_bf16(v4i x, v4i y) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    x[k] = (int)pack2_bf16(bf16_lo((uint32_t)x[k]) + bf16_lo((uint32_t)y[k]), bf16_hi((uint32_t)x[k]) + bf16_hi((uint32_t)y[k]));
+  return x;
+}
+
+// One block element by element, for outputs that the wide stores cannot write (a pitch, an end or a base that is
+// no multiple of 16 bytes).  voff: byte offset of the lane's row and first column (kOob: no such row); cols:
+// columns from the lane's first on that exist.
+template <bool F32>
+__device__ __forceinline__ void store_elements(const v16f& a, __amdgpu_buffer_rsrc_t out, uint32_t voff, uint32_t soff, int cols, bool accumulate) {
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
-    const uint32_t s = soff + (8 * (v >> 2) + (v & 3)) * pitch;
-    uint32_t r = f32_to_bf16_bits(a[v]);
-    if (accumulate) {
-      const uint32_t old = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(out, voff, s, 0);
-      r = f32_to_bf16_bits(bf16_bits_to_f32(old) + bf16_bits_to_f32(r));
+    const int c = 8 * (v >> 2) + (v & 3);
+    const uint32_t vo = c < cols ? voff : kOob, so = soff + c * (F32 ? 4 : 2);
+    if (F32) {
+      float x = a[v];
+      if (accumulate) x += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(out, vo, so, 0));
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, x), out, vo, so, 0);
+    } else {
+      uint32_t r = f32_to_bf16_bits(a[v]);
+      if (accumulate) {
+        const uint32_t old = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(out, vo, so, 0);
+        r = f32_to_bf16_bits(bf16_bits_to_f32(old) + bf16_bits_to_f32(r));
+      }
+      __builtin_amdgcn_raw_buffer_store_b16((short)r, out, vo, so, 0);
     }
-    __builtin_amdgcn_raw_buffer_store_b16((short)r, out, voff, s, 0);
   }
 }
 
@@ -421,27 +413,19 @@ __device__ __forceinline__ void decode_tile(const GemmArgs& p, const int* s_pref
   }
 }
 
-// Hands one accumulator block produced by inline-assembly MFMAs to the compiler (PIN; otherwise the compiler
-// produced it itself).
-template <bool PIN>
-__device__ __forceinline__ void pin_acc(v16f& a) {
-  if constexpr (PIN) asm volatile("" : "+v"(a));
-}
-
 // Writes one wave's TM x TN blocks of 32 x 32 results of tile T (rows wm0.., columns wn0.. of the
-// tile).  `stg` is the wave's 2 KiB LDS staging area.  PIN: the accumulators were produced by
-// inline-assembly MFMAs; each block is handed to the compiler only right before its store, so
-// that it is converted and copied out one block at a time.
+// tile).  `piece`: the LDS addresses of the wave's four 1 KiB pieces of staging.
 // EXTRAS: the output rows (out_row_index) and the bias of the tile lie in LDS, row wm0 and column wn0 of
-// the tile's at rows_lds[wm0] and bias_lds + 2 wn0: a load here would wait for every store before it.
-template <int MODE, int TM, int TN, bool ACC, bool PIN, bool PAIR = false, bool EXTRAS = false>
-__device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& p, const Tile& T, int wm0, int wn0, int lane,
-                                           uint8_t* stg, const int* rows_lds = nullptr, const uint8_t* bias_lds = nullptr) {
+// the tile's at LDS bytes rows_lds + 4 wm0 and bias_lds + 2 wn0: a load here would wait for every store before it.
+template <int MODE, int TM, int TN, bool ACC, bool PAIR = false, bool EXTRAS = false>
+__device__ __forceinline__ void store_tile(const v16f (&acc)[TM][TN], const GemmArgs& p, const Tile& T, int wm0, int wn0, int lane,
+                                           const uint32_t (&piece)[4], uint32_t rows_lds = 0, uint32_t bias_lds = 0) {
+  const Staging stg = make_staging(piece, lane);
   const uint32_t esz = p.out_dtype == PT_F32 ? 4 : 2;
   const uint32_t pitch = (uint32_t)p.ldo * esz;
-  const bool pair_ok = p.out_dtype != PT_F32 && (p.ldo & 1) == 0 && (((uintptr_t)p.out) & 3) == 0;
-  const bool wide_ok = p.out_dtype != PT_F32 && (p.ldo & 7) == 0 && (((uintptr_t)p.out) & 15) == 0 &&
-                       (MODE != GEMM_K_GROUPED || (p.out_stride_g & 7) == 0);
+  const int whole = p.out_dtype == PT_F32 ? 3 : 7;  // elements of 16 bytes, less one
+  const bool wide_ok = (p.ldo & whole) == 0 && (((uintptr_t)p.out) & 15) == 0 && (MODE != GEMM_K_GROUPED || (p.out_stride_g & whole) == 0) &&
+                       (T.b_lim & whole) == 0;
   // The descriptor ends after the tile's last valid row: stores to ragged rows are dropped.
   // (PT_GEMM_ABLATE_STORES, measurement builds only: it ends before the first, so every store
   // instruction runs and nothing is written.)
@@ -457,8 +441,15 @@ __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& 
   }
   const __amdgpu_buffer_rsrc_t rs_out = __builtin_amdgcn_make_buffer_rsrc(outp, 0, kAblateStores ? 0 : (int)((uint32_t)row_lim * pitch), kRsrcFlags);
   const uint32_t s_tile = (uint32_t)row0 * pitch + (uint32_t)(T.b_row0 + wn0) * esz;
-  const int colw = T.b_row0 + wn0 + (lane & 31);
-  static_assert(TN % 2 == 0, "the wide stores take column blocks in pairs");
+  static_assert(TN % 2 == 0, "the bf16 stores take column blocks in pairs");
+  constexpr int AUX = kStoreAux<MODE>;
+  // bias: the 8 values of the lane's columns, added in the output type after the result has been rounded to it
+  // (x + bias[group] as a second operation on the rounded x)
+  auto bias_of = [&](int j, int colc) -> v4i {
+    if (MODE != GEMM_M_GROUPED || p.bias == nullptr || colc >= T.b_lim) return v4i{0, 0, 0, 0};
+    if (EXTRAS) return PT_LDS(const v4i, bias_lds + (wn0 + j * 32 + (lane & 7) * 8) * 2);
+    return *(const v4i*)((const char*)p.bias + ((int64_t)T.g * p.rows_b + colc) * 2);
+  };
   if (MODE == GEMM_DENSE && p.head_a) {
     // Per-head halves in two tensors: a lane's eight columns lie in one of them (both widths are multiples
     // of 8), so its offset from `out` and its row pitch are all that differ.
@@ -471,88 +462,77 @@ __device__ __forceinline__ void store_tile(v16f (&acc)[TM][TN], const GemmArgs& 
       const bool second = c >= p.head_a;
       const uint32_t at = second ? (uint32_t)((char*)p.out2 - (char*)p.out) + (uint32_t)(h * p.head_b + c - p.head_a) * 2 : (uint32_t)(h * p.head_a + c) * 2;
       const uint32_t pitch_h = (uint32_t)(heads * (second ? p.head_b : p.head_a)) * 2;
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        uint32_t voff[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int r = row0 + i * 32 + q * 8 + (lane >> 3);
-          voff[q] = colc < T.b_lim && r < row_lim ? (uint32_t)r * pitch_h + at : kOob;
-        }
-        pin_acc<PIN>(acc[i][j]); pin_acc<PIN>(acc[i][j + 1]);
-        store_staged_bf16_lines<kStoreAux<MODE>>(acc[i][j], acc[i][j + 1], rs_heads, stg, voff, 0, false, lane);
-      }
+      stage_column<false>(acc, j, stg, lane, [&](int i, int q, v4i w) {
+        const int r = row0 + i * 32 + q * 8 + (lane >> 3);
+        store16<AUX>(w, rs_heads, colc < T.b_lim && r < row_lim ? (uint32_t)r * pitch_h + at : kOob, 0);
+      });
     }
   } else if (MODE == GEMM_M_GROUPED && p.out_row_index) {
     // Result row r goes to output row out_row_index[r] (the un-permute folded into the store);
     // rows of the group's padding map to a negative index and are dropped.
     const __amdgpu_buffer_rsrc_t rs_sc = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, kAblateStores ? 0 : (int)((uint32_t)p.out_rows * pitch), kRsrcFlags);
+    // one index per lane and block row (lane -> row lane % 32), handed to the lanes that store the row
+    int dst[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      // one index load for the block row (lane -> row lane%32), handed to the lanes that store the row
       const int r = T.a_row0 + wm0 + i * 32 + (lane & 31);
-      int dst_of_lane = -1;
-      if (EXTRAS) { dst_of_lane = rows_lds[wm0 + i * 32 + (lane & 31)]; if (r >= T.a_lim) dst_of_lane = -1; }
-      else if (r < T.a_lim) dst_of_lane = p.out_row_index[r];
-      uint32_t vrow[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int dst = __shfl(dst_of_lane, q * 8 + (lane >> 3));
-        vrow[q] = dst >= 0 ? (uint32_t)dst * pitch + (uint32_t)(lane & 7) * 16 : kOob;
-      }
-#pragma unroll
-      for (int j = 0; j < TN; j += 2) {
-        const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;
-        uint32_t voff[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) voff[q] = colc < T.b_lim ? vrow[q] : kOob;
-        v4i bias = v4i{0, 0, 0, 0};
-        if (EXTRAS) { if (p.bias != nullptr) bias = *(const v4i*)(bias_lds + (wn0 + j * 32 + (lane & 7) * 8) * 2); }
-        else if (p.bias != nullptr && colc < T.b_lim) bias = *(const v4i*)((const char*)p.bias + ((int64_t)T.g * p.rows_b + colc) * 2);
-        pin_acc<PIN>(acc[i][j]); pin_acc<PIN>(acc[i][j + 1]);
-        store_staged_bf16_lines<kStoreAux<MODE>>(acc[i][j], acc[i][j + 1], rs_sc, stg, voff, (uint32_t)(T.b_row0 + wn0 + j * 32) * 2, false, lane,
-                                p.bias != nullptr, bias);
-      }
+      if (EXTRAS) dst[i] = PT_LDS(const int, rows_lds + (wm0 + i * 32 + (lane & 31)) * 4);
+      else dst[i] = p.out_row_index[r < T.a_lim ? r : T.a_row0];
+      if (r >= T.a_lim) dst[i] = -1;
     }
-  } else if (p.out_dtype != PT_F32 && wide_ok && (T.b_lim & 7) == 0) {
+#pragma unroll
+    for (int j = 0; j < TN; j += 2) {
+      const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;
+      const v4i bias = bias_of(j, colc);
+      stage_column<false>(acc, j, stg, lane, [&](int i, int q, v4i w) {
+        const int row = __shfl(dst[i], q * 8 + (lane >> 3));
+        store16<AUX>(p.bias ? add_bf16(w, bias) : w, rs_sc, row >= 0 && colc < T.b_lim ? (uint32_t)row * pitch + (uint32_t)(lane & 7) * 16 : kOob,
+                     (uint32_t)(T.b_row0 + wn0 + j * 32) * 2);
+      });
+    }
+  } else if (p.out_dtype != PT_F32 && wide_ok) {
     const bool has_bias = MODE == GEMM_M_GROUPED && p.bias != nullptr;
 #pragma unroll
     for (int j = 0; j < TN; j += 2) {
       const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;
-      v4i bias = v4i{0, 0, 0, 0};
-      if (EXTRAS) { if (has_bias) bias = *(const v4i*)(bias_lds + (wn0 + j * 32 + (lane & 7) * 8) * 2); }
-      else if (has_bias && colc < T.b_lim) bias = *(const v4i*)((const char*)p.bias + ((int64_t)T.g * p.rows_b + colc) * 2);
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        uint32_t voff[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          voff[q] = colc < T.b_lim ? (uint32_t)(q * 8 + (lane >> 3)) * pitch + (uint32_t)(lane & 7) * 16 : kOob;
-        pin_acc<PIN>(acc[i][j]); pin_acc<PIN>(acc[i][j + 1]);
-        store_staged_bf16_lines<kStoreAux<MODE>>(acc[i][j], acc[i][j + 1], rs_out, stg, voff, s_tile + i * 32 * pitch + j * 64, ACC, lane, has_bias, bias);
-      }
+      const v4i bias = bias_of(j, colc);
+      const uint32_t v0 = (uint32_t)(lane >> 3) * pitch + (uint32_t)(lane & 7) * 16;
+      stage_column<false>(acc, j, stg, lane, [&](int i, int q, v4i w) {
+        const uint32_t soff = s_tile + i * 32 * pitch + j * 64;
+        const uint32_t voff = colc < T.b_lim ? v0 + q * 8 * pitch : kOob;
+        v4i x = has_bias ? add_bf16(w, bias) : w;
+        // the result is rounded to bf16 first, then added: the two roundings of `grad += wgrad.to(bf16)`
+        if (ACC) x = add_bf16(__builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs_out, voff, soff, 0)), x);
+        store16<AUX>(x, rs_out, voff, soff);
+      });
     }
-  } else if (p.out_dtype != PT_F32 && pair_ok && (T.b_lim & 1) == 0) {
-    const bool odd = lane & 1;
+  } else if (wide_ok) {
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const uint32_t voff = colw + j * 32 < T.b_lim ? (uint32_t)(4 * (lane >> 5) + odd) * pitch + (uint32_t)(((lane & 31) & ~1) + j * 32) * 2 : kOob;
+      const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 4;
+      const uint32_t v0 = (uint32_t)(lane >> 3) * pitch + (uint32_t)(lane & 7) * 16;
+      stage_column<true>(acc, j, stg, lane, [&](int i, int q, v4i w) {
+        const uint32_t soff = s_tile + i * 32 * pitch + j * 128;
+        const uint32_t voff = colc < T.b_lim ? v0 + q * 8 * pitch : kOob;
+        v4i x = w;
+        if (ACC) {
+          const v4i old = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs_out, voff, soff, 0));
 #pragma unroll
-      for (int i = 0; i < TM; ++i) { pin_acc<PIN>(acc[i][j]); store_pairs_bf16(acc[i][j], rs_out, voff, s_tile + i * 32 * pitch, pitch, ACC, odd); }
-    }
-  } else if (p.out_dtype == PT_F32) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const uint32_t voff = colw + j * 32 < T.b_lim ? (uint32_t)(4 * (lane >> 5)) * pitch + (uint32_t)((lane & 31) + j * 32) * 4 : kOob;
-#pragma unroll
-      for (int i = 0; i < TM; ++i) { pin_acc<PIN>(acc[i][j]); store_f32(acc[i][j], rs_out, voff, s_tile + i * 32 * pitch, pitch, ACC); }
+          for (int k = 0; k < 4; ++k) x[k] = __float_as_int(__int_as_float(x[k]) + __int_as_float(old[k]));
+        }
+        store16<0>(x, rs_out, voff, soff);
+      });
     }
   } else {
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const uint32_t voff = colw + j * 32 < T.b_lim ? (uint32_t)(4 * (lane >> 5)) * pitch + (uint32_t)((lane & 31) + j * 32) * 2 : kOob;
+      const int col = T.b_row0 + wn0 + j * 32 + 4 * (lane >> 5);
+      const uint32_t voff = (uint32_t)(lane & 31) * pitch + (uint32_t)(4 * (lane >> 5) + j * 32) * esz;
 #pragma unroll
-      for (int i = 0; i < TM; ++i) { pin_acc<PIN>(acc[i][j]); store_single_bf16(acc[i][j], rs_out, voff, s_tile + i * 32 * pitch, pitch, ACC); }
+      for (int i = 0; i < TM; ++i) {
+        if (p.out_dtype == PT_F32) store_elements<true>(acc[i][j], rs_out, voff, s_tile + i * 32 * pitch, T.b_lim - col, ACC);
+        else store_elements<false>(acc[i][j], rs_out, voff, s_tile + i * 32 * pitch, T.b_lim - col, ACC);
+      }
     }
   }
 }

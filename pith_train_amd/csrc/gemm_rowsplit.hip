@@ -48,17 +48,17 @@
 namespace pt {
 
 // LDS of a workgroup, all of it dynamic, so that the ring starts at byte 0 and a slot is bit 16 of an address:
-// two operand stages, two stages of scales, the tile table, the waves' result staging (which the group scan
-// of the work list borrows before the first tile), the scatter indices and the bias of the current tile.
+// two operand stages, two stages of scales, the tile table, the group scan of the work list, the scatter
+// indices and the bias of the current tile.  (The waves stage their results in the ring itself.)
 static constexpr int kRsStage = 512 * 128;
 static constexpr int kRsScales = 2 * kRsStage;
 static constexpr int kRsTable = kRsScales + 2 * 512 * 4;
 static constexpr int kRsTiles = 48, kRsEntry = 48;
-static constexpr int kRsStaging = kRsTable + kRsTiles * kRsEntry;
-static constexpr int kRsIndex = kRsStaging + 8 * 2048;
+static constexpr int kRsPref = kRsTable + kRsTiles * kRsEntry;
+static constexpr int kRsIndex = kRsPref + ((kMaxGroupsGemm + 2) * 4 + 15) / 16 * 16;
 static constexpr int kRsBias = kRsIndex + 256 * 4;
 static constexpr int kRsLds = kRsBias + 256 * 2;
-static_assert((kMaxGroupsGemm + 2) * 4 <= 8 * 2048 && kRsLds <= 160 * 1024 && kRsStaging % 16 == 0 && kRsIndex % 16 == 0, "LDS map");
+static_assert(kRsLds <= 160 * 1024 && kRsPref % 16 == 0, "LDS map");
 
 // BT: the b operand is given reduction-major, [red][rows_b] with row pitch ldb (the forward layout of
 // a weight, read by its input-gradient GEMM), instead of [rows_b][red].
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm0 = (wave / WGN) * WM, wn0 = (wave % WGN) * WN;
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
-  int* const s_pref = (int*)(lds + kRsStaging);
+  int* const s_pref = (int*)(lds + kRsPref);
 
   // ---- tile list ----
   const GemmArgs p = reload_args();
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
           const int i = m & 1, j = (m >> 1) & 1, ks = m >> 2;
           const int late = BT ? ks : j, early = BT ? j : ks;
           if (wave_active) {
-            mfma_sel(fa[2 * ks + i], fb[late][early], acc[i][j], i, sca, j, scb);
+            mfma_sel(fb[late][early], fa[2 * ks + i], acc[i][j], j, scb, i, sca);
           }
           if (m < NX) issue_o(m);
           if (m == 0) { if (BT) fa[2] = read_a(0, 1); else fb[1][0] = read_b(1, 0); }
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
           const int i = m & 1, j = (m >> 1) & 1, ks = m >> 2;
           const int late = BT ? ks : j, early = BT ? j : ks;
           if (wave_active) {
-            mfma_sel(fa[2 * ks + i], fb[late][early], acc[2 + i][j], 2 + i, sca, j, scb);
+            mfma_sel(fb[late][early], fa[2 * ks + i], acc[2 + i][j], j, scb, 2 + i, sca);
           }
           if (m < NY) issue_e(m);
           if (m == 0) fa[2] = read_a(2, 1);
@@ -414,7 +414,11 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
       }
       // the compiler does not see the MFMAs inside the assembly statements: cover the result latency
       // of the last one before the epilogue reads the accumulators
-      asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+      static_assert(TM == 4 && TN == 2, "all accumulators are operands");
+      asm volatile("s_nop 15\n\ts_nop 15"
+                   : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[1][0]), "+v"(acc[1][1]), "+v"(acc[2][0]), "+v"(acc[2][1]), "+v"(acc[3][0]), "+v"(acc[3][1])
+                   :
+                   : "memory");
 
       // ---- epilogue ----
       if (!wave_active) continue;
@@ -423,8 +427,11 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
       // not kept (or spilled, and reloaded behind a wait for every store so far) across the main loop
       int el = lane;
       asm volatile("" : "+v"(el));
-      store_tile<MODE, TM, TN, ACC, true, PAIR, true>(acc, reload_args(), C, wm0, wn0, el, lds + kRsStaging + wave * 2048,
-                                                   (const int*)(lds + kRsIndex), lds + kRsBias);
+      // staging: the part of the ring that this wave itself refills next (the O half that its step Y has just
+      // released), with loads that it issues behind these stores
+      const uint32_t piece[4] = {to_a + l_slot + kToAO, to_a + l_slot + kToAO + kToA2, to_b + l_slot + kToBO, to_b + l_slot + kToBO + kToB2};
+      store_tile<MODE, TM, TN, ACC, PAIR, true>(acc, reload_args(), C, wm0, wn0, el, piece,
+                                                   lds_base + kRsIndex, lds_base + kRsBias);
     }
   }
   wait_all_vmem();  // nothing may still be writing into this workgroup's LDS when it retires

@@ -34,7 +34,7 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
   constexpr int NP = LA + LB + 1;            // and one of scales
   constexpr int kWait = (NS - 2) * NP;       // loads of the stages after the one a step needs
   static_assert(kWait < 64, "vmcnt is a 6-bit counter");
-  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // [NS][STAGE] | [NS][BM + BN] scales | 256 B sink; the stores' staging takes the first 8 KiB afterwards
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // [NS][STAGE] | [NS][BM + BN] scales | 256 B sink; the stores' staging takes the first 16 KiB afterwards
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -190,20 +190,21 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
     for (int ks = 0; ks < 2; ++ks) {
       v8i fa[TM], fb[TN];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) fa[i] = read_frag(sA + (wm0 + 32 * i) * BK, ks);
-#pragma unroll
       for (int j = 0; j < TN; ++j) fb[j] = read_b(sB, j, ks);
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < TM; ++i) fa[i] = read_frag(sA + (wm0 + 32 * i) * BK, ks);
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[i], fb[j], acc[i][j], 0, 0, 0, sca[i], 0, scb[j]);
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[j], fa[i], acc[i][j], 0, 0, 0, scb[j], 0, sca[i]);
     }
   }
   wait_all_vmem();  // nothing may still be writing into this workgroup's LDS when it retires
   if (MODE == GEMM_K_GROUPED && nk == 0 && ACC) return;
   __syncthreads();  // every wave has read its last stage and has nothing in flight: the ring's memory is free
-  store_tile<MODE, TM, TN, ACC, false, MODE == GEMM_K_GROUPED>(acc, p, T, wm0, wn0, lane, lds + wave * 2048);
+  const uint32_t stg = lds_base + wave * 4096, piece[4] = {stg, stg + 1024, stg + 2048, stg + 3072};
+  store_tile<MODE, TM, TN, ACC, MODE == GEMM_K_GROUPED>(acc, p, T, wm0, wn0, lane, piece);
 }
 
 template <int MODE, int BM, bool ACC, bool BT>

@@ -61,6 +61,20 @@ def test_dense_nt(M, N, K):
     _check(out32, ref, f"dense fp32 {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("N", [1, 3, 4, 130, 259, 516])
+def test_dense_nt_with_rows_that_are_no_whole_16_bytes(N):
+    """Result rows that the 16-byte stores cannot write (as bf16, fp32 or both), ending inside a tile's first,
+    second and third columns of blocks."""
+    from pith_train_amd.operators.linear import _fp8_gemm_nt
+
+    M, K = 300, 144
+    a, sa, _, _ = Q.fp8cast_rowwise_transpose(_rand((M, K), N))
+    b, sb, _, _ = Q.fp8cast_blockwise_transpose(_rand((N, K), N + 1, 0.02))
+    ref = G.gemm_nt_dense(a, sa, b, sb, torch.float64)
+    for dtype in (torch.bfloat16, torch.float32):
+        _check(_fp8_gemm_nt(a.cuda(), sa.cuda(), b.cuda(), sb.cuda(), M, N, "cuda", dtype), ref, f"dense {M}x{N}x{K} {dtype}")
+
+
 @pytest.mark.parametrize("M,N,K", [(512, 256, 4096), (300, 200, 4000), (128, 128, 20000), (256, 1024, 2048)])
 def test_dense_nt_with_the_reduction_split_over_workgroups(M, N, K):
     """Small outputs with a long reduction (a dense weight gradient) are computed as several
