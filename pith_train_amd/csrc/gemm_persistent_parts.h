@@ -57,12 +57,18 @@ __device__ __forceinline__ v4i make_rsrc(const void* base, uint32_t bytes) {
 #ifndef PT_GEMM_LOAD_B_MOD
 #define PT_GEMM_LOAD_B_MOD ""
 #endif
+template <bool NT = false>  // NT: non-temporal
 __device__ __forceinline__ void dma16(v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds_off) {
   soff = (uint32_t)__builtin_amdgcn_readfirstlane((int)soff);  // uniform by construction; pin them to SGPRs
   lds_off = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_off);
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rsrc), "s"(soff),
-               "s"(lds_off)
-               : "memory");
+  if (NT)
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(voff), "s"(rsrc), "s"(soff),
+                 "s"(lds_off)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rsrc), "s"(soff),
+                 "s"(lds_off)
+                 : "memory");
 }
 // the same at LDS byte lds_off + OFF; OPERAND 0: a, 1: b
 template <int OPERAND, int OFF>
