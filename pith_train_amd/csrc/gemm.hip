@@ -287,19 +287,20 @@ static int gemm_impl() {
 // Problems too small for 256 x 256 tiles to fill 256 compute units evenly go to the kernel with one 64 x 128
 // or 128 x 128 tile per workgroup and two workgroups per compute unit (gemm_small.hip): tile rows, or 0
 // when the persistent kernel is the better choice.  While all 64-row tiles run at once the smaller tile
-// wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 25.0 for the large one).  Then both
+// wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 21.5 for the large one).  Then both
 // kinds are priced in rounds of the GPU: a round of 256 large tiles is the unit, a round of 512 small ones
-// (a quarter of the area each, half of it in all) costs 0.57 of it in the m-grouped mode (0.68 with a
-// reduction-major b, whose fragments take twice the LDS reads), 0.65 in
-// the dense one, where the large tiles have the better loop (0.45 up to a reduction of 512, most of it
-// filling and draining), 0.43 for a weight gradient over groups of up to 1024 rows (mostly stores, which
-// one workgroup of a unit does while the other loads; longer ones are like dense products).  A partly filled round of small tiles costs half of what it leaves idle.  Us,
-// large / small: m-grouped, K 2048, N 1536: 16 groups of 256 rows 26.1 / 18.0, of 512 33.3 / 32.1, of 640
-// 60.4 / 36.4, of 1024 62.9 / 56.0; 64 groups of 128 51.5 / 40.7, of 384 90 / 85, of 512 105 / 115;
-// reduction-major b, K 1536, N 2048: 16 groups of 512 32.3 / 29.9, of 1024 54.5 / 57.3.  Dense
-// 4096 x 2048 x 2048 28.7 / 19.3, 4096 x 4096 x 2048 32.7 / 38.0.  Weight gradients 1536 x 2048 of 16
-// groups of 128 rows 28.2 / 23.1, of 1024 61.1 / 57.1; of 64 groups 73 / 83.  Past three to four rounds
-// large tiles have no round to waste and need half of the operand traffic.
+// (a quarter of the area each, half of it in all) costs 0.72 of it in the m-grouped mode, 0.68 in
+// the dense one (0.45 up to a reduction of 512, most of it filling and draining), 0.36 for a weight gradient
+// over groups of up to 1024 rows (mostly stores, which one workgroup of a unit does while the other loads), 0.65
+// over longer ones (16 Zipf-distributed groups of 7600 rows 768 x 2048 and 1536 x 2048: whole step 2540 us, 2623 at
+// 0.56).  A partly filled round of small tiles costs half of what it leaves idle.  Fitted to 270
+// shapes timed with both kernels, where the choice now loses 0.9 % to the better one in the mean (m-grouped), 0.2 %
+// (weight gradients) and nothing (dense).  Us, large / small: m-grouped, K 2048, N 1536: 16 groups of 256 rows
+// 25.4 / 19.7, of 512 30.5 / 34.9, of 640 50.1 / 37.4, of 1024 53.0 / 62.8; 64 groups of 128 49.6 / 52.7, of 384
+// 89 / 108; reduction-major b, K 1536, N 2048: 16 groups of 256 24.5 / 25.2, of 640 42.2 / 41.2.  Dense
+// 4096 x 2048 x 2048 26 / 20, 4096 x 4096 x 512 15.0 / 13.6.  Weight gradients 1536 x 2048 of 8 groups of 512
+// rows 26.6 / 23.4, of 1024 35.1 / 32.7; of 16 groups of 512 37.8 / 40.9.  Past two rounds large tiles have
+// no round to waste and need half of the operand traffic.
 static int small_tile_rows(const GemmArgs& g) {
   const int64_t groups = g.mode == GEMM_K_GROUPED ? g.G : 1;
   const int64_t cols = cdiv(g.rows_b, 128) * groups, cols_large = cdiv(g.rows_b, 256) * groups;
@@ -317,10 +318,9 @@ static int small_tile_rows(const GemmArgs& g) {
     small = (fewer > least ? fewer : least) * cols;
   }
   const int64_t large = rows_large * cols_large;
-  if (large > (g.mode == GEMM_K_GROUPED ? 1024 : g.b_kmajor ? 512 : 768)) return 0;
+  if (large > 512) return 0;
   const int64_t depth = g.mode == GEMM_K_GROUPED ? g.red / g.G : g.red;
-  const int64_t price = g.mode == GEMM_M_GROUPED ? (g.b_kmajor ? 68 : 57)
-                        : g.mode == GEMM_K_GROUPED ? (depth <= 1024 ? 43 : 65) : depth <= 512 ? 45 : 65;
+  const int64_t price = g.mode == GEMM_M_GROUPED ? 72 : g.mode == GEMM_K_GROUPED ? (depth <= 1024 ? 36 : 65) : depth <= 512 ? 45 : 68;
   // in units of 1 / (100 * 512 * 2) of a round of large tiles, five percent in favour of those
   return (small + cdiv(small, 512) * 512) * price * 105 < cdiv(large, 256) * (2 * 512 * 100) * 100 ? 128 : 0;
 }
