@@ -371,24 +371,35 @@ __device__ __forceinline__ int xcd_first_tile(const GemmArgs& p, const int* s_pr
 // Geometry of logical tile t; plain per-lane arithmetic (every lane may ask for a different t).
 template <int MODE, int BM, int BN>
 __device__ __forceinline__ void decode_tile(const GemmArgs& p, const int* s_pref, int t, Tile& T) {
-  // The 32 CUs of an XCD work on 32 consecutive logical tiles at a time.  The b-tiles are cut into
-  // strips of at most 8 (of nearly equal width), and a strip is walked row by row: 32 consecutive
-  // tiles then share 32 / w a-tiles and w b-tiles in that XCD's L2 (4 and 8 for a full strip)
-  // instead of 32 a-tiles and 1 b-tile, whatever the number of b-tiles is.
-  auto blocked = [&](int t, int& ta, int& tb) {
-    const int ns = (p.tiles_b + 7) >> 3;           // strips
-    const int w0 = p.tiles_b / ns, wide = p.tiles_b - w0 * ns;  // the first `wide` strips have w0 + 1 b-tiles
-    const int per_wide = p.tiles_a * (w0 + 1);
-    int s, r, w, b0;
-    if (t < wide * per_wide) { s = t / per_wide; r = t - s * per_wide; w = w0 + 1; b0 = s * w; }
-    else { const int t2 = t - wide * per_wide; s = t2 / (p.tiles_a * w0); r = t2 - s * p.tiles_a * w0; w = w0; b0 = wide * (w0 + 1) + s * w0; }
-    ta = r / w;
-    tb = b0 + r - ta * w;
+  // The 32 CUs of an XCD work on 32 consecutive logical tiles at a time.  One side of the tile grid is cut into
+  // strips of at most `width` tiles (of nearly equal width), and a strip is walked line by line along the other
+  // side: 32 consecutive tiles then share 32 / w tiles of one operand and w of the other in that XCD's L2
+  // instead of 32 and 1, whatever the two counts are.
+  auto strips = [](int t, int n, int lines, int width, int& tn, int& tl) {  // t -> place tn of the n that are cut, line tl
+    const int ns = (n + width - 1) / width;
+    const int w0 = n / ns, wide = n - w0 * ns;  // the first `wide` strips have w0 + 1 tiles
+    const int per_wide = lines * (w0 + 1);
+    int s, r, w, n0;
+    if (t < wide * per_wide) { s = t / per_wide; r = t - s * per_wide; w = w0 + 1; n0 = s * w; }
+    else { const int t2 = t - wide * per_wide; s = t2 / (lines * w0); r = t2 - s * lines * w0; w = w0; n0 = wide * (w0 + 1) + s * w0; }
+    tl = r / w;
+    tn = n0 + r - tl * w;
+  };
+  // A group's tiles: the longer side is cut, so that the operand that is read once per strip is the smaller one, and
+  // into strips of 3.  Against row tile by row tile down one column after the other, us: 32 groups of 2048 rows 5760 x
+  // 2880 1103 -> 994, their input gradient 1015 -> 974, weight gradient 994 -> 949, 2880 x 2880 586 -> 531; 8 groups of
+  // 8192 rows 1178 -> 930, 1251 -> 942, 994 -> 869, 1536 x 2048 193 -> 180; 128 groups of 512 rows level.  Strips
+  // of 4 of the columns (windows of 32 tiles are then whole lines and move on all at once) give 1066, 1013 and 601 for the
+  // first two and the 2880 x 2880, of 6 997, 989 and 545; the shorter side cut instead loses 2..10 % on 8192 rows.
+  // Dense products, which do not change operands every few tiles, are level with 3 and with 8.
+  auto group_strips = [&](int t, int na, int nb, int& ta, int& tb) {
+    if (na > nb) strips(t, na, nb, 3, ta, tb);
+    else strips(t, nb, na, 3, tb, ta);
   };
   if (MODE == GEMM_DENSE) {
     T.g = 0;
     int ta, tb;
-    blocked(t, ta, tb);
+    strips(t, p.tiles_b, p.tiles_a, 8, tb, ta);
     T.a_row0 = ta * BM; T.b_row0 = tb * BN;
     T.a_lim = (int)p.rows_a; T.b_lim = (int)p.rows_b; T.k_begin = 0; T.k_len = (int)p.red; T.kb0 = 0;
   } else if (MODE == GEMM_M_GROUPED) {
@@ -404,15 +415,18 @@ __device__ __forceinline__ void decode_tile(const GemmArgs& p, const int* s_pref
     const int m_tiles = pg1 - pg;
     const int idx = t - pg * p.tiles_b;
     T.g = g;
-    T.a_row0 = gs + (idx % m_tiles) * BM; T.b_row0 = (idx / m_tiles) * BN;
+    int ta, tb;
+    group_strips(idx, m_tiles, p.tiles_b, ta, tb);
+    T.a_row0 = gs + ta * BM; T.b_row0 = tb * BN;
     T.a_lim = p.offs[g]; T.b_lim = (int)p.rows_b; T.k_begin = 0; T.k_len = (int)p.red; T.kb0 = 0;
   } else {
     const int per_g = p.tiles_a * p.tiles_b;
     const int g = t / per_g;
     const int idx = t % per_g;
     T.g = g;
-    int ta = idx % p.tiles_a, tb = idx / p.tiles_a;
-    if (!p.offs) blocked(idx, ta, tb);  // split-K of a dense product: the dense order inside every range
+    int ta, tb;
+    if (p.offs) group_strips(idx, p.tiles_a, p.tiles_b, ta, tb);
+    else strips(idx, p.tiles_b, p.tiles_a, 8, tb, ta);  // split-K of a dense product: the dense order inside every range
     T.a_row0 = ta * BM; T.b_row0 = tb * BN;
     T.a_lim = (int)p.rows_a; T.b_lim = (int)p.rows_b;
     T.k_begin = g ? k_group_end(p, g - 1) : 0; T.k_len = k_group_end(p, g) - T.k_begin; T.kb0 = T.k_begin >> 7;

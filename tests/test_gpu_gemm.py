@@ -449,6 +449,54 @@ def test_m_grouped_scattered_rows_with_bias_of_short_reductions(sizes, N, K, gem
     assert torch.equal(out[rows.long()], plain + bias[group])
 
 
+@pytest.mark.parametrize("tiles", [1, 3, 4, 10])
+def test_grouped_tile_order_at_the_edges_of_its_strips(gemm_kernel, tiles):
+    """Groups with more row tiles than column tiles and the other way round, one strip and several of unequal
+    width, empty groups among them: the bits of the kernel that takes one small tile per workgroup, whatever
+    place the order gives a tile."""
+    from pith_train_amd import _lib
+
+    if gemm_kernel != "auto":
+        pytest.skip("the test selects the kernels itself; run once")
+    g = torch.Generator(device="cuda").manual_seed(tiles)
+
+    def fp8(*shape):
+        return torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # finite values below 2
+
+    def scale(*shape):
+        return torch.exp2(torch.randint(-6, 3, shape, device="cuda", generator=g).float())
+
+    def both(make):
+        out = []
+        for kernel in (b"r0", b"s128"):
+            _lib.call("pt_gemm_select_kernel", kernel)
+            out.append(make())
+        assert torch.equal(*out)
+
+    rows = torch.tensor([128, 0, 640, 1024, 1152, 0, 2688], dtype=torch.int32)  # 1, 3, 4, 5 and 11 row tiles
+    G_, M, N, K = len(rows), int(rows.sum()), 256 * tiles - 112, 256
+    offs = torch.cumsum(rows, 0).int().cuda()
+    a, sa, b, sb = fp8(M, K), scale(M, K // 128), fp8(G_, N, K), scale(G_, (N + 127) // 128, K // 128)
+
+    def m_grouped():
+        o = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
+        _lib.call("pt_gemm_m_grouped_nt", _lib.ptr(a), _lib.ptr(sa), _lib.ptr(b), _lib.ptr(sb), _lib.ptr(o), _lib.dtype_code(o.dtype),
+                  _lib.ptr(offs), G_, M, N, K, _lib.stream_ptr())
+        return o
+
+    both(m_grouped)
+    for W in (256 * 4, 256 * 11 - 128):  # the other side of a weight gradient
+        d, sd, x, sx = fp8(N, M), scale(M // 128, N), fp8(W, M), scale(M // 128, W)
+
+        def k_grouped():
+            o = torch.zeros((G_, N, W), dtype=torch.bfloat16, device="cuda")
+            _lib.call("pt_gemm_k_grouped_wgrad", _lib.ptr(d), _lib.ptr(sd), _lib.ptr(x), _lib.ptr(sx), _lib.ptr(o), _lib.dtype_code(o.dtype), 0,
+                      _lib.ptr(offs), G_, M, N, W, _lib.stream_ptr())
+            return o
+
+        both(k_grouped)
+
+
 def test_grouped_work_lists_longer_than_the_tile_table(gemm_kernel):
     """12800 large tiles, 50 for every workgroup, so that the table is filled a second time and the groups
     are scanned again: the bits of the kernel that takes one small tile per workgroup.  m-grouped, then
