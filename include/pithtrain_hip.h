@@ -53,6 +53,9 @@ int pt_quant_rowwise_colwise(const void* x, int dtype, int64_t M, int64_t N, int
                              void* tok_fp8, float* tok_scale, void* ch_fp8, float* ch_scale,
                              int ch_layout, const int32_t* offs, int32_t num_groups,
                              pt_stream_t stream);
+/* The same (PT_CH_TRANSPOSED, all M rows) with tok_scale [ceil(N/128), M], as pt_gemm_m_grouped_by_block reads it. */
+int pt_quant_rowwise_colwise_by_block(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx, void* tok_fp8,
+                                      float* tok_scale, void* ch_t_fp8, float* ch_scale, pt_stream_t stream);
 
 /* pt_quant_rowwise_colwise on gathered rows: output row r is quantised from source row
  * row_index[r] of x (a negative index gives an all-zero row: zero bytes, the scale of amax 0).
@@ -309,6 +312,12 @@ int pt_gemm_m_grouped_nn_scatter(const void* a_fp8, const float* a_scale, const 
                                  const int32_t* offs, int32_t num_groups, int64_t M, int64_t N,
                                  int64_t K, const int32_t* out_row_index, int64_t out_rows,
                                  pt_stream_t stream);
+/* The same products from a_scale [ceil(K/128), M]: b as pt_gemm_m_grouped_nt has it, or with b_reduction_major != 0 as
+ * pt_gemm_m_grouped_nn; stored through out_row_index (with out_rows) when that is not NULL. */
+int pt_gemm_m_grouped_by_block(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,
+                               int b_reduction_major, void* out, int out_dtype, const int32_t* offs, int32_t num_groups,
+                               int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows,
+                               pt_stream_t stream);
 
 /* pt_gemm_m_grouped_nt followed by `out + bias[group of the row]` in the output type (the result
  * is rounded to bf16, then the bias row of its group is added and the sum rounded again): the
@@ -639,6 +648,9 @@ typedef struct {
   pt_stream_t stream;
 } pt_experts_forward_args;
 int pt_experts_forward(const pt_experts_forward_args* args /* host */);
+/* The same step with the scales of its row-scaled operands (x_scale, h_scale; in the backward dy_scale and dgu_scale) as
+ * [K/128, M] instead of [M, K/128]: the GEMMs read them in whole lines. */
+int pt_experts_forward_by_block(const pt_experts_forward_args* args /* host */);
 
 /* Backward of the same block, up to the quantised gradient of gate_up: dgu_fp8 [M, 2*half] and dgu_scale
  * [M, ceil(2*half/128)], from which the input gradient follows with one pt_gemm_m_grouped_nn(_scatter) on
@@ -673,6 +685,7 @@ typedef struct {
   pt_stream_t stream;
 } pt_experts_backward_args;
 int pt_experts_backward(const pt_experts_backward_args* args /* host */);
+int pt_experts_backward_by_block(const pt_experts_backward_args* args /* host */); /* see pt_experts_forward_by_block; the input gradient is pt_gemm_m_grouped_by_block's */
 /* The gate_up weight gradient of the same block from the same arguments (dw_gate_up, dw_up): the last
  * launch of a backward, after the caller has queued the input gradient. */
 int pt_experts_weight_gradient(const pt_experts_backward_args* args /* host */);

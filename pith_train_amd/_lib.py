@@ -29,6 +29,7 @@ SIGNATURES = {
     "pt_last_error": (c_char_p, []),
     "pt_abi_version": (c_int, []),
     "pt_quant_rowwise_colwise": (c_int, [P, c_int, I64, I64, I64, P, P, P, P, c_int, P, I32, P]),
+    "pt_quant_rowwise_colwise_by_block": (c_int, [P, c_int, I64, I64, I64, P, P, P, P, P]),
     "pt_quant_rowwise_colwise_rows": (c_int, [P, c_int, I64, I64, I64, P, P, P, P, P, c_int, P, I32, P]),
     "pt_quant_rowwise_colwise_rows_repeat": (c_int, [P, I64, I64, c_int, I64, I64, I64, P, P, P, P, P, c_int, P, I32, P]),
     "pt_silu_mul_quant_rowwise_colwise": (c_int, [P, I64, I64, I64, P, P, P, P, P, P]),
@@ -59,6 +60,7 @@ SIGNATURES = {
     "pt_gemm_m_grouped_nt_few_rows": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P, P]),
     "pt_gemm_m_grouped_nn": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P]),
     "pt_gemm_m_grouped_nn_scatter": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P]),
+    "pt_gemm_m_grouped_by_block": (c_int, [P, P, P, P, c_int, P, c_int, P, I32, I64, I64, I64, P, I64, P]),
     "pt_gemm_m_grouped_nt_bias": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, P]),
     "pt_gemm_m_grouped_nt_scatter_bias": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P, P]),
     "pt_gemm_m_grouped_nt_scatter": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P]),
@@ -103,7 +105,9 @@ SIGNATURES = {
     "pt_segment_sum_tiles": (c_int, [P, P, I32, I32, P, I64, I64, c_int, P]),
     # whole steps: one host block of 8-byte fields (struct.pack) instead of an argument each
     "pt_experts_forward": (c_int, [c_char_p]),
+    "pt_experts_forward_by_block": (c_int, [c_char_p]),
     "pt_experts_backward": (c_int, [c_char_p]),
+    "pt_experts_backward_by_block": (c_int, [c_char_p]),
     "pt_experts_weight_gradient": (c_int, [c_char_p]),
     "pt_transposed_pitch": (I64, [I64]),
     "pt_linear_forward_workspace_bytes": (I64, [I64, I64, I64, I64]),

@@ -207,4 +207,29 @@ __device__ __forceinline__ float row16_allmax(float v) {
   return v;
 }
 
+// Where the scales of a row-scaled FP8 operand [M, K] lie: [M, K/128] floats, as the operators hand them out, or
+// [K/128, M], for operands that a step makes and reads itself.  A GEMM loads the scales of 64 rows of one block at a
+// time: 64 lines of the first form (a quarter as many requests to L2 as the operands themselves, more with ragged
+// rows), two of the second.  GEMMs alone, us: 32 groups of 2048 rows 5760 x 2880 1022 -> 964, their input gradient 1004 ->
+// 954, 2880 x 2880 545 -> 512; 128 groups of 512 rows 1536 x 2048 241 -> 228, input gradient 245 -> 229.  (Dense
+// products, which meet the same rows' scales again before they leave L1, gain 0..2 %, and keep the first form.)
+enum class RowScales { BY_ROW, BY_BLOCK };
+
+// The entry points of the same names (with pt_ in front) with the scales in either form
+int quant_rowwise_colwise(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
+                          void* tok_fp8, float* tok_scale, RowScales order, void* ch_fp8, float* ch_scale, int ch_layout, const int32_t* offs,
+                          int32_t num_groups, pt_stream_t stream);
+int silu_mul_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up, void* tok_fp8, float* tok_scale, void* ch_t_fp8, float* ch_scale,
+                   const int32_t* valid_rows, RowScales order, pt_stream_t stream);
+int silu_mul_bwd_quant(const void* grad_h, int64_t ld_grad_h, const void* gate_up, int64_t ld_gate_up, int64_t M, int64_t half, void* tok_fp8,
+                       float* tok_scale, void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream);
+int clamped_swiglu_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up, float alpha, float limit, void* tok_fp8, float* tok_scale,
+                         void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream);
+int clamped_swiglu_bwd_quant(const void* grad_h, int64_t ld_grad_h, const void* gate_up, int64_t ld_gate_up, int64_t M, int64_t half, float alpha,
+                             float limit, void* tok_fp8, float* tok_scale, void* ch_t_fp8, float* ch_scale, float* col_sum, const int32_t* valid_rows,
+                             RowScales order, pt_stream_t stream);
+int gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order, const void* b_fp8, const float* b_scale, void* out, int out_dtype,
+                   const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows, const void* bias,
+                   pt_stream_t stream, bool b_kmajor = false, bool few_rows = false);
+
 }  // namespace pt

@@ -525,10 +525,9 @@ extern "C" int pt_sum_partials(const float* partial, int32_t splits, int64_t n, 
   return check_launch("sum_partials_kernel");
 }
 
-static int gemm_m_grouped_impl(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale, void* out,
-                               int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K,
-                               const int32_t* out_row_index, int64_t out_rows, const void* bias, pt_stream_t stream,
-                               bool b_kmajor = false, bool few_rows = false) {
+int pt::gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order, const void* b_fp8, const float* b_scale, void* out, int out_dtype,
+                       const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows,
+                       const void* bias, pt_stream_t stream, bool b_kmajor, bool few_rows) {
   PT_REQUIRE(M >= 0 && N >= 0 && K >= 0 && G > 0, "gemm_m_grouped_nt: bad sizes");
   if (M == 0 || N == 0) return PT_OK;
   PT_REQUIRE(M % (few_rows ? 64 : 128) == 0, "gemm_m_grouped_nt: M=%lld must be a multiple of %d", (long long)M, few_rows ? 64 : 128);
@@ -539,7 +538,8 @@ static int gemm_m_grouped_impl(const void* a_fp8, const float* a_scale, const vo
   const int64_t KB = cdiv(K, 128), NB = cdiv(N, 128);
   GemmArgs g = {};
   g.a = (const uint8_t*)a_fp8; g.lda = K; g.b = (const uint8_t*)b_fp8; g.ldb = K;
-  g.sa = a_scale; g.sa_rs = KB; g.sa_ks = 1; g.sa_shift = 0;
+  g.sa = a_scale; g.sa_shift = 0;
+  g.sa_rs = order == RowScales::BY_BLOCK ? 1 : KB; g.sa_ks = order == RowScales::BY_BLOCK ? M : 1;
   g.sb = b_scale; g.sb_rs = KB; g.sb_ks = 1; g.sb_shift = 7;
   g.out = out; g.ldo = N; g.out_dtype = out_dtype; g.accumulate = 0;
   g.rows_a = M; g.rows_b = N; g.red = K; g.mode = GEMM_M_GROUPED; g.offs = offs; g.G = G;
@@ -570,15 +570,15 @@ static int gemm_m_grouped_impl(const void* a_fp8, const float* a_scale, const vo
 extern "C" int pt_gemm_m_grouped_nt(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,
                                     void* out, int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K,
                                     pt_stream_t stream) {
-  return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, nullptr, 0, nullptr, stream);
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_ROW, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int pt_gemm_m_grouped_nt_scatter(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,
                                             void* out, int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N,
                                             int64_t K, const int32_t* out_row_index, int64_t out_rows, pt_stream_t stream) {
   PT_REQUIRE(out_row_index, "gemm_m_grouped_nt_scatter: null out_row_index");
-  return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, nullptr,
-                             stream);
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_ROW, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, nullptr,
+                        stream);
 }
 
 extern "C" int pt_gemm_m_grouped_nt_scatter_bias(const void* a_fp8, const float* a_scale, const void* b_fp8,
@@ -586,36 +586,43 @@ extern "C" int pt_gemm_m_grouped_nt_scatter_bias(const void* a_fp8, const float*
                                                  int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows,
                                                  const void* bias, pt_stream_t stream) {
   PT_REQUIRE(out_row_index && bias, "gemm_m_grouped_nt_scatter_bias: null out_row_index or bias");
-  return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, bias,
-                             stream);
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_ROW, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, bias,
+                        stream);
 }
 
 extern "C" int pt_gemm_m_grouped_nt_few_rows(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale, void* out,
                                              int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K,
                                              const int32_t* out_row_index, int64_t out_rows, const void* bias, pt_stream_t stream) {
-  return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, bias, stream,
-                             false, true);
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_ROW, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, bias, stream,
+                        false, true);
 }
 
 extern "C" int pt_gemm_m_grouped_nn(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,
                                     void* out, int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K,
                                     pt_stream_t stream) {
-  return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, nullptr, 0, nullptr, stream, true);
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_ROW, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, nullptr, 0, nullptr, stream, true);
 }
 
 extern "C" int pt_gemm_m_grouped_nn_scatter(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,
                                             void* out, int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N,
                                             int64_t K, const int32_t* out_row_index, int64_t out_rows, pt_stream_t stream) {
   PT_REQUIRE(out_row_index, "gemm_m_grouped_nn_scatter: null out_row_index");
-  return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, nullptr,
-                             stream, true);
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_ROW, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, nullptr,
+                        stream, true);
 }
 
 extern "C" int pt_gemm_m_grouped_nt_bias(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,
                                          void* out, int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N,
                                          int64_t K, const void* bias, pt_stream_t stream) {
   PT_REQUIRE(bias, "gemm_m_grouped_nt_bias: null bias");
-  return gemm_m_grouped_impl(a_fp8, a_scale, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, nullptr, 0, bias, stream);
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_ROW, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, nullptr, 0, bias, stream);
+}
+
+extern "C" int pt_gemm_m_grouped_by_block(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale, int b_reduction_major,
+                                          void* out, int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K,
+                                          const int32_t* out_row_index, int64_t out_rows, pt_stream_t stream) {
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_BLOCK, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, nullptr,
+                        stream, b_reduction_major != 0);
 }
 
 static int gemm_k_grouped_wgrad_impl(const void* dy_t_fp8, const float* dy_scale, int64_t ld_dy_scale, const void* x_t_fp8,

@@ -74,8 +74,8 @@ struct Library {
   PT_FN(pt_quant_weights);
   PT_FN(pt_group_rows_workspace_bytes);
   PT_FN(pt_group_rows);
-  PT_FN(pt_experts_forward);
-  PT_FN(pt_experts_backward);
+  PT_FN(pt_experts_forward_by_block);
+  PT_FN(pt_experts_backward_by_block);
   PT_FN(pt_experts_weight_gradient);
   PT_FN(pt_transposed_pitch);
   PT_FN(pt_linear_forward_workspace_bytes);
@@ -105,9 +105,8 @@ struct Library {
   PT_FN(pt_dedup_prepare_dispatch);
   PT_FN(pt_build_expert_idxs);
   PT_FN(pt_adjust_expand_idx);
-  PT_FN(pt_quant_rowwise_colwise);
-  PT_FN(pt_gemm_m_grouped_nt);
-  PT_FN(pt_gemm_m_grouped_nn);
+  PT_FN(pt_quant_rowwise_colwise_by_block);
+  PT_FN(pt_gemm_m_grouped_by_block);
   PT_FN(pt_gemm_k_grouped_wgrad);
   PT_FN(pt_sum_branches);
 #undef PT_FN
@@ -128,8 +127,8 @@ void init(const std::string& path) {
   PT_FN(pt_quant_weights);
   PT_FN(pt_group_rows_workspace_bytes);
   PT_FN(pt_group_rows);
-  PT_FN(pt_experts_forward);
-  PT_FN(pt_experts_backward);
+  PT_FN(pt_experts_forward_by_block);
+  PT_FN(pt_experts_backward_by_block);
   PT_FN(pt_experts_weight_gradient);
   PT_FN(pt_transposed_pitch);
   PT_FN(pt_linear_forward_workspace_bytes);
@@ -159,9 +158,8 @@ void init(const std::string& path) {
   PT_FN(pt_dedup_prepare_dispatch);
   PT_FN(pt_build_expert_idxs);
   PT_FN(pt_adjust_expand_idx);
-  PT_FN(pt_quant_rowwise_colwise);
-  PT_FN(pt_gemm_m_grouped_nt);
-  PT_FN(pt_gemm_m_grouped_nn);
+  PT_FN(pt_quant_rowwise_colwise_by_block);
+  PT_FN(pt_gemm_m_grouped_by_block);
   PT_FN(pt_gemm_k_grouped_wgrad);
   PT_FN(pt_sum_branches);
 #undef PT_FN
@@ -469,7 +467,7 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x,
   if (keep) { a.x_t = kept.at(0); a.x_t_scale = (float*)kept.at(1); a.h_t = kept.at(2); a.h_t_scale = (float*)kept.at(3); }
   a.composed_map = (int32_t*)temp.at(0); a.x_fp8 = temp.at(1); a.x_scale = (float*)temp.at(2); a.h_fp8 = temp.at(3); a.h_scale = (float*)temp.at(4);
   a.stream = (pt_stream_t)stream;
-  check(lib.pt_experts_forward(&a), "pt_experts_forward");
+  check(lib.pt_experts_forward_by_block(&a), "pt_experts_forward_by_block");
   return {out, gate_up, kept.buffers};
 }
 
@@ -499,6 +497,13 @@ Tensor shared_rows(int64_t rows, int64_t cols, int64_t other, at::ScalarType typ
   return empty({rows * other}, type, dev).narrow(0, 0, rows * cols).view({rows, cols});
 }
 
+// [rows, blocks] scales that lie as [blocks, rows], in a new buffer that holds at least `other` blocks
+Tensor scales_by_block(int64_t rows, int64_t blocks, int64_t other, const at::Device& dev) {
+  const auto options = at::TensorOptions().dtype(at::kFloat).device(dev);
+  if (blocks >= other) return at::empty_strided({rows, blocks}, {1, rows}, options);
+  return empty({other, rows}, at::kFloat, dev).narrow(0, 0, blocks).t();
+}
+
 // Backward of an expert block up to the quantised gradient of gate_up; the caller queues the input gradient from
 // it and then weight_gradient().  A buffer goes back to the allocator when its last reader is queued (the next
 // user is behind it on the stream), and the gradient of gate_up is written over the one of the output, which only
@@ -524,7 +529,7 @@ struct ExpertsBackward {
     twins.allocate(dev);
     temp.allocate(dev);
     dgu = shared_rows(d.M, 2 * d.half, d.H, kFp8, dev);
-    dgu_s = shared_rows(d.M, cdiv(2 * d.half, 128), cdiv(d.H, 128), at::kFloat, dev);
+    dgu_s = scales_by_block(d.M, cdiv(2 * d.half, 128), cdiv(d.H, 128), dev);
     if (gu_bias_like) d_gu_bias = empty({d.G, 2 * d.half}, gu_bias_like->scalar_type(), dev);
     if (dn_bias_like) d_dn_bias = empty({d.G, d.H}, dn_bias_like->scalar_type(), dev);
     if (weights.size() > 0) down.aim(weights[0]);
@@ -542,7 +547,7 @@ struct ExpertsBackward {
     a.d_gu_bias = ptr(d_gu_bias); a.d_gu_bias_dtype = d_gu_bias ? dtype_code(d_gu_bias->scalar_type()) : 0;
     a.d_dn_bias = ptr(d_dn_bias); a.d_dn_bias_dtype = d_dn_bias ? dtype_code(d_dn_bias->scalar_type()) : 0;
     a.stream = (pt_stream_t)stream;
-    check(lib.pt_experts_backward(&a), "pt_experts_backward");
+    check(lib.pt_experts_backward_by_block(&a), "pt_experts_backward_by_block");
     grad_out.reset();
   }
 
@@ -965,7 +970,7 @@ std::pair<Maybe, std::optional<std::vector<Tensor>>> mlp(const Tensor& input, co
 }
 
 // ---- grouped linear ---------------------------------------------------------------------------------------
-// Row- and column-scaled FP8 forms of x [M, N], M % 128 == 0: bytes, scales, transposed bytes, their scales
+// Row- and column-scaled FP8 forms of x [M, N], M % 128 == 0: bytes, scales [N/128, M], transposed bytes, their scales
 struct Quantised {
   Tensor q, s, q_t, s_t;
   Quantised() = default;
@@ -974,12 +979,12 @@ struct Quantised {
     const int64_t M = x.size(0), N = x.size(1);
     const auto dev = x.device();
     q = empty({M, N}, kFp8, dev);
-    s = empty({M, cdiv(N, 128)}, at::kFloat, dev);
+    s = empty({cdiv(N, 128), M}, at::kFloat, dev);
     q_t = empty({N, M}, kFp8, dev);
     s_t = empty({M / 128, N}, at::kFloat, dev);
     lib.pt_observe("pt_quant_rowwise_colwise", 1, M, N, M);
-    check(lib.pt_quant_rowwise_colwise(ptr(x), dtype_code(x.scalar_type()), M, N, M > 1 ? x.stride(0) : N, ptr(q), (float*)ptr(s), ptr(q_t),
-                                       (float*)ptr(s_t), PT_CH_TRANSPOSED, nullptr, 0, stream), "pt_quant_rowwise_colwise");
+    check(lib.pt_quant_rowwise_colwise_by_block(ptr(x), dtype_code(x.scalar_type()), M, N, M > 1 ? x.stride(0) : N, ptr(q), (float*)ptr(s), ptr(q_t),
+                                                (float*)ptr(s_t), stream), "pt_quant_rowwise_colwise");
     lib.pt_observe("pt_quant_rowwise_colwise", 0, M, N, M);
   }
 };
@@ -999,8 +1004,8 @@ struct GroupedLinearNode : HipNode {
     const auto o = (const int32_t*)ptr(offs);
     const char* what = forward_layout ? "pt_gemm_m_grouped_nn" : "pt_gemm_m_grouped_nt";
     lib.pt_observe(what, 1, M, K, N);
-    check((forward_layout ? lib.pt_gemm_m_grouped_nn : lib.pt_gemm_m_grouped_nt)(ptr(d.q), (const float*)ptr(d.s), ptr(dg), (const float*)ptr(dg_s), ptr(gx),
-                                                                                 dtype_code(gx.scalar_type()), o, (int32_t)G, M, K, N, stream), what);
+    check(lib.pt_gemm_m_grouped_by_block(ptr(d.q), (const float*)ptr(d.s), ptr(dg), (const float*)ptr(dg_s), forward_layout, ptr(gx),
+                                         dtype_code(gx.scalar_type()), o, (int32_t)G, M, K, N, nullptr, 0, stream), what);
     lib.pt_observe(what, 0, M, K, N);
     {
       py::gil_scoped_acquire gil;
@@ -1036,8 +1041,8 @@ Tensor grouped_linear(const Tensor& x, const Tensor& weight, const Tensor& offs,
         q = Quantised(x, (pt_stream_t)stream);
         Tensor y = empty({M, N}, x.scalar_type(), x.device());
         lib.pt_observe("pt_gemm_m_grouped_nt", 1, M, N, K);
-        check(lib.pt_gemm_m_grouped_nt(ptr(q.q), (const float*)ptr(q.s), ptr(w), (const float*)ptr(w_s), ptr(y), dtype_code(y.scalar_type()),
-                                       (const int32_t*)ptr(offs), (int32_t)G, M, N, K, (pt_stream_t)stream), "pt_gemm_m_grouped_nt");
+        check(lib.pt_gemm_m_grouped_by_block(ptr(q.q), (const float*)ptr(q.s), ptr(w), (const float*)ptr(w_s), 0, ptr(y), dtype_code(y.scalar_type()),
+                                             (const int32_t*)ptr(offs), (int32_t)G, M, N, K, nullptr, 0, (pt_stream_t)stream), "pt_gemm_m_grouped_nt");
         lib.pt_observe("pt_gemm_m_grouped_nt", 0, M, N, K);
         return y;
       },

@@ -21,6 +21,14 @@ static pt_observer_t g_observer = nullptr;
     if (g_observer) g_observer(#NAME, 0, (A), (B), (C));    \
   } while (0)
 
+// the same around an internal form of that entry point
+#define PT_STEP_AS(NAME, A, B, C, CALL)                     \
+  do {                                                      \
+    if (g_observer) g_observer(#NAME, 1, (A), (B), (C));    \
+    if (int rc_ = CALL) return rc_;                         \
+    if (g_observer) g_observer(#NAME, 0, (A), (B), (C));    \
+  } while (0)
+
 // Carves consecutive 256-byte aligned pieces out of a buffer (a null buffer gives offsets).
 struct Carve {
   uintptr_t p;
@@ -38,7 +46,7 @@ extern "C" void pt_observe(const char* name, int begin, int64_t a, int64_t b, in
   if (g_observer) g_observer(name, begin, a, b, c);
 }
 
-extern "C" int pt_experts_forward(const pt_experts_forward_args* args) {
+static int experts_forward(const pt_experts_forward_args* args, RowScales order) {
   PT_REQUIRE(args, "experts_forward: null arguments");
   const pt_experts_forward_args& a = *args;
   PT_REQUIRE(a.M >= 0 && a.M % 128 == 0 && a.K > 0 && a.half > 0 && a.H > 0 && a.G > 0 && a.G < (1ll << 31), "experts_forward: bad sizes");
@@ -57,49 +65,52 @@ extern "C" int pt_experts_forward(const pt_experts_forward_args* args) {
     PT_STEP(pt_compose_row_map, a.M, 0, 0, a.row_map, a.M, a.expand_idx, a.n_expand, a.x_rows, a.composed_map, a.stream);
     in_map = a.composed_map;
   }
+  const auto quant_x = [&](int64_t repeat, const int32_t* rows_of, const int32_t* ends) {
+    return quant_rowwise_colwise(a.x, a.x_rows, repeat, PT_BF16, a.M, a.K, a.ldx, rows_of, a.x_fp8, a.x_scale, order, a.x_t, a.x_t_scale,
+                                 PT_CH_TRANSPOSED, ends, ends ? G : 0, a.stream);
+  };
   if (a.repeat > 1)
-    PT_STEP(pt_quant_rowwise_colwise_rows_repeat, a.M, a.K, a.x_rows, a.x, a.x_rows, a.repeat, PT_BF16, a.M, a.K, a.ldx, in_map, a.x_fp8,
-            a.x_scale, a.x_t, a.x_t_scale, PT_CH_TRANSPOSED, a.offs, G, a.stream);
+    PT_STEP_AS(pt_quant_rowwise_colwise_rows_repeat, a.M, a.K, a.x_rows, quant_x(a.repeat, in_map, a.offs));
   else if (in_map)
-    PT_STEP(pt_quant_rowwise_colwise_rows, a.M, a.K, a.x_rows, a.x, PT_BF16, a.M, a.K, a.ldx, in_map, a.x_fp8, a.x_scale, a.x_t, a.x_t_scale,
-            PT_CH_TRANSPOSED, a.offs, G, a.stream);
+    PT_STEP_AS(pt_quant_rowwise_colwise_rows, a.M, a.K, a.x_rows, quant_x(1, in_map, a.offs));
   else
-    PT_STEP(pt_quant_rowwise_colwise, a.M, a.K, a.x_rows, a.x, PT_BF16, a.M, a.K, a.ldx, a.x_fp8, a.x_scale, a.x_t, a.x_t_scale, PT_CH_TRANSPOSED,
-            nullptr, 0, a.stream);
+    PT_STEP_AS(pt_quant_rowwise_colwise, a.M, a.K, a.x_rows, quant_x(1, nullptr, nullptr));
+  const int64_t N = 2 * a.half;
+  const auto gate_up = [&](const void* bias) {
+    return gemm_m_grouped(a.x_fp8, a.x_scale, order, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M, N, a.K, nullptr, 0, bias, a.stream,
+                          false, a.few_rows != 0);
+  };
   if (a.few_rows)
-    PT_STEP(pt_gemm_m_grouped_nt_few_rows, a.M, 2 * a.half, a.K, a.x_fp8, a.x_scale, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M,
-            2 * a.half, a.K, nullptr, 0, a.gu_bias, a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt_few_rows, a.M, N, a.K, gate_up(a.gu_bias));
   else if (a.gu_bias)
-    PT_STEP(pt_gemm_m_grouped_nt_bias, a.M, 2 * a.half, a.K, a.x_fp8, a.x_scale, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M,
-            2 * a.half, a.K, a.gu_bias, a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt_bias, a.M, N, a.K, gate_up(a.gu_bias));
   else
-    PT_STEP(pt_gemm_m_grouped_nt, a.M, 2 * a.half, a.K, a.x_fp8, a.x_scale, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M,
-            2 * a.half, a.K, a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt, a.M, N, a.K, gate_up(nullptr));
   if (a.clamped)
-    PT_STEP(pt_clamped_swiglu_quant_rowwise_colwise, a.M, a.half, 0, a.gate_up, a.M, a.half, 2 * a.half, (float)a.alpha,
-            (float)a.limit, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit, a.stream);
+    PT_STEP_AS(pt_clamped_swiglu_quant_rowwise_colwise, a.M, a.half, 0,
+               clamped_swiglu_quant(a.gate_up, a.M, a.half, N, (float)a.alpha, (float)a.limit, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit, order,
+                                    a.stream));
   else
-    PT_STEP(pt_silu_mul_quant_rowwise_colwise, a.M, a.half, 0, a.gate_up, a.M, a.half, 2 * a.half, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit,
-            a.stream);
+    PT_STEP_AS(pt_silu_mul_quant_rowwise_colwise, a.M, a.half, 0,
+               silu_mul_quant(a.gate_up, a.M, a.half, N, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit, order, a.stream));
+  const auto down = [&](const void* bias) {
+    return gemm_m_grouped(a.h_fp8, a.h_scale, order, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H, a.half, a.scatter ? a.row_map : nullptr,
+                          a.scatter ? a.out_rows : 0, bias, a.stream, false, a.few_rows != 0);
+  };
   if (a.few_rows)
-    PT_STEP(pt_gemm_m_grouped_nt_few_rows, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H,
-            a.half, a.scatter ? a.row_map : nullptr, a.out_rows, a.dn_bias, a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt_few_rows, a.M, a.H, a.half, down(a.dn_bias));
   else if (a.scatter && a.dn_bias)
-    PT_STEP(pt_gemm_m_grouped_nt_scatter_bias, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M,
-            a.H, a.half, a.row_map, a.out_rows, a.dn_bias, a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt_scatter_bias, a.M, a.H, a.half, down(a.dn_bias));
   else if (a.scatter)
-    PT_STEP(pt_gemm_m_grouped_nt_scatter, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H,
-            a.half, a.row_map, a.out_rows, a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt_scatter, a.M, a.H, a.half, down(nullptr));
   else if (a.dn_bias)
-    PT_STEP(pt_gemm_m_grouped_nt_bias, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H,
-            a.half, a.dn_bias, a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt_bias, a.M, a.H, a.half, down(a.dn_bias));
   else
-    PT_STEP(pt_gemm_m_grouped_nt, a.M, a.H, a.half, a.h_fp8, a.h_scale, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H, a.half,
-            a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt, a.M, a.H, a.half, down(nullptr));
   return PT_OK;
 }
 
-extern "C" int pt_experts_backward(const pt_experts_backward_args* args) {
+static int experts_backward(const pt_experts_backward_args* args, RowScales order) {
   PT_REQUIRE(args, "experts_backward: null arguments");
   const pt_experts_backward_args& a = *args;
   PT_REQUIRE(a.M >= 0 && a.M % 128 == 0 && a.K > 0 && a.half > 0 && a.H > 0 && a.G > 0 && a.G < (1ll << 31), "experts_backward: bad sizes");
@@ -108,12 +119,14 @@ extern "C" int pt_experts_backward(const pt_experts_backward_args* args) {
   if (a.M == 0) return PT_OK;
   const int32_t G = (int32_t)a.G;
   const int32_t* limit = a.limit_rows ? a.offs + G - 1 : nullptr;
+  const auto quant_dy = [&](const int32_t* ends) {
+    return quant_rowwise_colwise(a.grad_out, a.grad_rows, 1, PT_BF16, a.M, a.H, a.H, a.out_map, a.dy_fp8, a.dy_scale, order, a.dy_t, a.dy_t_scale,
+                                 PT_CH_TRANSPOSED, ends, ends ? G : 0, a.stream);
+  };
   if (a.out_map)
-    PT_STEP(pt_quant_rowwise_colwise_rows, a.M, a.H, a.grad_rows, a.grad_out, PT_BF16, a.M, a.H, a.H, a.out_map, a.dy_fp8, a.dy_scale, a.dy_t,
-            a.dy_t_scale, PT_CH_TRANSPOSED, a.offs, G, a.stream);
+    PT_STEP_AS(pt_quant_rowwise_colwise_rows, a.M, a.H, a.grad_rows, quant_dy(a.offs));
   else
-    PT_STEP(pt_quant_rowwise_colwise, a.M, a.H, a.grad_rows, a.grad_out, PT_BF16, a.M, a.H, a.H, a.dy_fp8, a.dy_scale, a.dy_t, a.dy_t_scale,
-            PT_CH_TRANSPOSED, nullptr, 0, a.stream);
+    PT_STEP_AS(pt_quant_rowwise_colwise, a.M, a.H, a.grad_rows, quant_dy(nullptr));
   if (a.d_dn_bias) {
     if (a.out_map)
       PT_STEP(pt_segment_sum_rows, a.M, a.H, 0, a.grad_out, a.grad_rows, a.out_map, a.offs, G, a.d_dn_bias, a.M, a.H, PT_BF16,
@@ -121,26 +134,35 @@ extern "C" int pt_experts_backward(const pt_experts_backward_args* args) {
     else
       PT_STEP(pt_segment_sum, a.M, a.H, 0, a.grad_out, a.offs, G, a.d_dn_bias, a.M, a.H, PT_BF16, (int)a.d_dn_bias_dtype, a.stream);
   }
+  const auto grad_h = [&] {
+    return gemm_m_grouped(a.dy_fp8, a.dy_scale, order, a.dn_dg, a.dn_dg_scale, a.grad_h, PT_BF16, a.offs, G, a.M, a.half, a.H, nullptr, 0, nullptr,
+                          a.stream, a.dn_forward_layout != 0);
+  };
   if (a.dn_forward_layout)
-    PT_STEP(pt_gemm_m_grouped_nn, a.M, a.half, a.H, a.dy_fp8, a.dy_scale, a.dn_dg, a.dn_dg_scale, a.grad_h, PT_BF16, a.offs, G, a.M, a.half, a.H,
-            a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nn, a.M, a.half, a.H, grad_h());
   else
-    PT_STEP(pt_gemm_m_grouped_nt, a.M, a.half, a.H, a.dy_fp8, a.dy_scale, a.dn_dg, a.dn_dg_scale, a.grad_h, PT_BF16, a.offs, G, a.M, a.half, a.H,
-            a.stream);
+    PT_STEP_AS(pt_gemm_m_grouped_nt, a.M, a.half, a.H, grad_h());
   if (a.dw_down)
     PT_STEP(pt_gemm_k_grouped_wgrad, a.M, a.H, a.half, a.dy_t, a.dy_t_scale, a.h_t, a.h_t_scale, a.dw_down, PT_BF16, (int)a.dw_down_add, a.offs, G,
             a.M, a.H, a.half, a.stream);
   if (a.clamped)
-    PT_STEP(pt_clamped_swiglu_bwd_quant_rowwise_colwise, a.M, a.half, 0, a.grad_h, a.half, a.gate_up, 2 * a.half, a.M, a.half,
-            (float)a.alpha, (float)a.limit, a.dgu_fp8, a.dgu_scale, a.dgu_t, a.dgu_t_scale, a.col_sum, limit, a.stream);
+    PT_STEP_AS(pt_clamped_swiglu_bwd_quant_rowwise_colwise, a.M, a.half, 0,
+               clamped_swiglu_bwd_quant(a.grad_h, a.half, a.gate_up, 2 * a.half, a.M, a.half, (float)a.alpha, (float)a.limit, a.dgu_fp8, a.dgu_scale,
+                                        a.dgu_t, a.dgu_t_scale, a.col_sum, limit, order, a.stream));
   else
-    PT_STEP(pt_silu_mul_bwd_quant_rowwise_colwise, a.M, a.half, 0, a.grad_h, a.half, a.gate_up, 2 * a.half, a.M, a.half, a.dgu_fp8, a.dgu_scale,
-            a.dgu_t, a.dgu_t_scale, limit, a.stream);
+    PT_STEP_AS(pt_silu_mul_bwd_quant_rowwise_colwise, a.M, a.half, 0,
+               silu_mul_bwd_quant(a.grad_h, a.half, a.gate_up, 2 * a.half, a.M, a.half, a.dgu_fp8, a.dgu_scale, a.dgu_t, a.dgu_t_scale, limit, order,
+                                  a.stream));
   if (a.d_gu_bias)  // groups are whole 128-row tiles: their ends in tiles index the per-tile column sums
     PT_STEP(pt_segment_sum_tiles, a.M / 128, 2 * a.half, 0, a.col_sum, a.offs, 128, G, a.d_gu_bias, a.M / 128, 2 * a.half,
             (int)a.d_gu_bias_dtype, a.stream);
   return PT_OK;
 }
+
+extern "C" int pt_experts_forward(const pt_experts_forward_args* args) { return experts_forward(args, RowScales::BY_ROW); }
+extern "C" int pt_experts_forward_by_block(const pt_experts_forward_args* args) { return experts_forward(args, RowScales::BY_BLOCK); }
+extern "C" int pt_experts_backward(const pt_experts_backward_args* args) { return experts_backward(args, RowScales::BY_ROW); }
+extern "C" int pt_experts_backward_by_block(const pt_experts_backward_args* args) { return experts_backward(args, RowScales::BY_BLOCK); }
 
 extern "C" int pt_experts_weight_gradient(const pt_experts_backward_args* args) {
   PT_REQUIRE(args, "experts_weight_gradient: null arguments");

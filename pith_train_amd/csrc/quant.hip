@@ -66,6 +66,7 @@ struct QuantArgs {
   int64_t M, N, ldx, x_stride_g;
   uint8_t* a_out;  int64_t a_stride_g;   // [M,N] bytes, ld = N; row-scaled launches: null = not written
   float* a_scale;  int64_t a_scale_stride_g;
+  int64_t as_rs, as_ks;                  // row-scaled launches: the scale of row r, column tile c is a_scale[r * as_rs + c * as_ks]
   uint8_t* b_out;  int64_t b_stride_g;   // rowmajor [M,N] / transposed [N,M] / kmajor flat; row-scaled launches: null = not written
   float* b_scale;  int64_t b_scale_stride_g;
   int32_t tiles_m, tiles_n;
@@ -444,14 +445,13 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
   f.fence();
   {
     uint8_t* ab = p.a_out + g * p.a_stride_g;
-    const int64_t nb = p.tiles_n;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       f.fence_row(i);
       float rcp, s;
       if (AM == A_ROW) {
         s = fp8_scale_from_amax(rowmax[i], rcp);
-        if (cc == 0 && (FULL || row0 + i < p.M)) p.a_scale[(row0 + i) * nb + tc] = s;
+        if (cc == 0 && (FULL || row0 + i < p.M)) p.a_scale[(row0 + i) * p.as_rs + tc * p.as_ks] = s;
       } else {
         rcp = blk_rcp;
         s = blk_scale;
@@ -714,8 +714,8 @@ void quant_tile_kernel(QuantArgs p) {
   // tiles further right) from one read of grad_h, gate and up
   const int tiles_n_grid = PRO == PRO_SILU_BWD_PAIR ? p.tiles_n / 2 : p.tiles_n;
   // Row-scaled launches (one group): which XCD runs which tile decides whether the 4-byte scale
-  // writes merge into whole lines.  Row scales are [M, tiles_n] floats, so the column tiles of one
-  // row block write neighbouring floats; column scales in the [N, tiles_m] layout put the same
+  // writes merge into whole lines.  Row scales are [M, tiles_n] floats (or [tiles_n, M], whole lines of a tile), so the
+  // column tiles of one row block write neighbouring floats; column scales in the [N, tiles_m] layout put the same
   // column of neighbouring row blocks next to each other.  Workgroup b runs on XCD b % 8: with the
   // column tile as the fastest index all of those writes would meet in eight different L2s and
   // leave as one 32-byte sector per float (8x their bytes; 12 % of the kernel's write traffic).
@@ -843,6 +843,7 @@ static void fill_common(QuantArgs& a, const void* x, int dtype, int64_t M, int64
   a.x = x; a.M = M; a.N = N; a.ldx = ldx; a.x_stride_g = 0;
   a.a_stride_g = 0; a.a_scale_stride_g = 0; a.b_stride_g = 0; a.b_scale_stride_g = 0;
   a.tiles_m = (int32_t)cdiv(M, 128); a.tiles_n = (int32_t)cdiv(N, 128);
+  a.as_rs = a.tiles_n; a.as_ks = 1;
   a.offs = nullptr; a.num_groups = 0; a.row_index = nullptr; a.row_mul = 0; a.x2 = nullptr; a.ldx2 = 0; a.half = 0;
   a.row_limit = nullptr; a.ld_t = M; a.bs_ld = a.tiles_m; a.alpha = 0.f; a.limit = 0.f; a.col_sum = nullptr;
   a.head_a = a.head_b = 0;
@@ -852,53 +853,28 @@ static void fill_common(QuantArgs& a, const void* x, int dtype, int64_t M, int64
   a.vec_out_t = (M % 16 == 0);
 }
 
-}  // namespace pt
-
-using namespace pt;
-
-static int quant_rowwise_colwise_impl(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
-                                      void* tok_fp8, float* tok_scale, void* ch_fp8, float* ch_scale, int ch_layout,
-                                      const int32_t* offs, int32_t num_groups, pt_stream_t stream, int64_t repeat = 1);
-
-extern "C" int pt_quant_rowwise_colwise(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx,
-                                        void* tok_fp8, float* tok_scale, void* ch_fp8,
-                                        float* ch_scale, int ch_layout, const int32_t* offs,
-                                        int32_t num_groups, pt_stream_t stream) {
-  return quant_rowwise_colwise_impl(x, dtype, M, N, ldx, nullptr, tok_fp8, tok_scale, ch_fp8, ch_scale, ch_layout, offs,
-                                    num_groups, stream);
+static void order_scales(QuantArgs& a, RowScales order) {
+  if (order == RowScales::BY_BLOCK) { a.as_rs = 1; a.as_ks = a.M; }
 }
 
-extern "C" int pt_quant_rowwise_colwise_rows(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx,
-                                             const int32_t* row_index, void* tok_fp8, float* tok_scale,
-                                             void* ch_fp8, float* ch_scale, int ch_layout,
-                                             const int32_t* offs, int32_t num_groups, pt_stream_t stream) {
-  PT_REQUIRE(row_index || M == 0, "quant_rowwise_colwise_rows: null row_index");
-  return quant_rowwise_colwise_impl(x, dtype, M, N, ldx, row_index, tok_fp8, tok_scale, ch_fp8, ch_scale, ch_layout, offs,
-                                    num_groups, stream);
+// floor(i / repeat) = floor(i * m / 2^32) with m = ceil(2^32 / repeat) is exact while i * repeat stays below 2^32
+static bool repeat_fits(int64_t rows, int64_t repeat) {
+  return rows >= 0 && repeat >= 1 && repeat < (1 << 16) && rows * repeat * repeat < (1ll << 32) && rows * repeat < (1ll << 31);
 }
 
-extern "C" int pt_quant_rowwise_colwise_rows_repeat(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M, int64_t N, int64_t ldx,
-                                                    const int32_t* row_index, void* tok_fp8, float* tok_scale, void* ch_fp8,
-                                                    float* ch_scale, int ch_layout, const int32_t* offs, int32_t num_groups,
-                                                    pt_stream_t stream) {
-  PT_REQUIRE(row_index || M == 0, "quant_rowwise_colwise_rows_repeat: null row_index");
-  // floor(i / repeat) = floor(i * m / 2^32) with m = ceil(2^32 / repeat) is exact while i * repeat stays below 2^32
-  PT_REQUIRE(rows >= 0 && repeat >= 1 && repeat < (1 << 16) && rows * repeat * repeat < (1ll << 32) && rows * repeat < (1ll << 31),
-             "quant_rowwise_colwise_rows_repeat: %lld rows, each %lld times, are too many", (long long)rows, (long long)repeat);
-  return quant_rowwise_colwise_impl(x, dtype, M, N, ldx, row_index, tok_fp8, tok_scale, ch_fp8, ch_scale, ch_layout, offs,
-                                    num_groups, stream, repeat);
-}
-
-static int quant_rowwise_colwise_impl(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
-                                      void* tok_fp8, float* tok_scale, void* ch_fp8, float* ch_scale, int ch_layout,
-                                      const int32_t* offs, int32_t num_groups, pt_stream_t stream, int64_t repeat) {
+int quant_rowwise_colwise(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
+                          void* tok_fp8, float* tok_scale, RowScales order, void* ch_fp8, float* ch_scale, int ch_layout, const int32_t* offs,
+                          int32_t num_groups, pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && N >= 0 && M % 128 == 0, "quant_rowwise_colwise: M=%lld must be a multiple of 128", (long long)M);
   PT_REQUIRE(ldx >= N, "quant_rowwise_colwise: ldx < N");
+  PT_REQUIRE(repeat == 1 || (repeat_fits(rows, repeat) && (row_index || M == 0)), "quant_rowwise_colwise: %lld rows, each %lld times, are too many",
+             (long long)rows, (long long)repeat);
   if (M == 0 || N == 0) return PT_OK;
   PT_REQUIRE(x && tok_fp8 && tok_scale && (ch_fp8 == nullptr) == (ch_scale == nullptr), "quant_rowwise_colwise: null pointer");
   QuantArgs a;
   fill_common(a, x, dtype, M, N, ldx);
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_fp8; a.b_scale = ch_scale;
+  order_scales(a, order);
   a.row_index = row_index;
   if (repeat > 1) a.row_mul = (uint32_t)(((1ull << 32) + repeat - 1) / repeat);
   if (offs && num_groups > 0) a.row_limit = offs + (num_groups - 1);
@@ -912,6 +888,43 @@ static int quant_rowwise_colwise_impl(const void* x, int dtype, int64_t M, int64
       return launch_quant<A_ROW, B_COL, BL_KMAJOR, BS_N_MB>(a, dtype, 1, s);
   }
   PT_REQUIRE(false, "quant_rowwise_colwise: bad ch_layout %d", ch_layout);
+}
+
+}  // namespace pt
+
+using namespace pt;
+
+extern "C" int pt_quant_rowwise_colwise(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx,
+                                        void* tok_fp8, float* tok_scale, void* ch_fp8,
+                                        float* ch_scale, int ch_layout, const int32_t* offs,
+                                        int32_t num_groups, pt_stream_t stream) {
+  return quant_rowwise_colwise(x, 0, 1, dtype, M, N, ldx, nullptr, tok_fp8, tok_scale, RowScales::BY_ROW, ch_fp8, ch_scale, ch_layout, offs,
+                               num_groups, stream);
+}
+
+extern "C" int pt_quant_rowwise_colwise_rows(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx,
+                                             const int32_t* row_index, void* tok_fp8, float* tok_scale,
+                                             void* ch_fp8, float* ch_scale, int ch_layout,
+                                             const int32_t* offs, int32_t num_groups, pt_stream_t stream) {
+  PT_REQUIRE(row_index || M == 0, "quant_rowwise_colwise_rows: null row_index");
+  return quant_rowwise_colwise(x, 0, 1, dtype, M, N, ldx, row_index, tok_fp8, tok_scale, RowScales::BY_ROW, ch_fp8, ch_scale, ch_layout, offs,
+                               num_groups, stream);
+}
+
+extern "C" int pt_quant_rowwise_colwise_rows_repeat(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M, int64_t N, int64_t ldx,
+                                                    const int32_t* row_index, void* tok_fp8, float* tok_scale, void* ch_fp8,
+                                                    float* ch_scale, int ch_layout, const int32_t* offs, int32_t num_groups,
+                                                    pt_stream_t stream) {
+  PT_REQUIRE(row_index || M == 0, "quant_rowwise_colwise_rows_repeat: null row_index");
+  PT_REQUIRE(repeat_fits(rows, repeat), "quant_rowwise_colwise_rows_repeat: %lld rows, each %lld times, are too many", (long long)rows, (long long)repeat);
+  return quant_rowwise_colwise(x, rows, repeat, dtype, M, N, ldx, row_index, tok_fp8, tok_scale, RowScales::BY_ROW, ch_fp8, ch_scale, ch_layout,
+                               offs, num_groups, stream);
+}
+
+extern "C" int pt_quant_rowwise_colwise_by_block(const void* x, int dtype, int64_t M, int64_t N, int64_t ldx, void* tok_fp8, float* tok_scale,
+                                                 void* ch_t_fp8, float* ch_scale, pt_stream_t stream) {
+  return quant_rowwise_colwise(x, 0, 1, dtype, M, N, ldx, nullptr, tok_fp8, tok_scale, RowScales::BY_BLOCK, ch_t_fp8, ch_scale, PT_CH_TRANSPOSED,
+                               nullptr, 0, stream);
 }
 
 // The transposed twin of a dense linear's operand may be written in whole 16-byte chunks when its pitch has
@@ -1133,9 +1146,9 @@ static int launch_silu_quant(const QuantArgs& a, hipStream_t stream) {
   return pt::check_launch("quant_tile_kernel(fused SwiGLU)");
 }
 
-extern "C" int pt_silu_mul_quant_rowwise_colwise(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up,
-                                                 void* tok_fp8, float* tok_scale, void* ch_t_fp8, float* ch_scale,
-                                                 const int32_t* valid_rows, pt_stream_t stream) {
+namespace pt {
+int silu_mul_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up, void* tok_fp8, float* tok_scale, void* ch_t_fp8, float* ch_scale,
+                   const int32_t* valid_rows, RowScales order, pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half, "silu_mul_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
   PT_REQUIRE(gate_up && tok_fp8 && tok_scale && (ch_t_fp8 == nullptr) == (ch_scale == nullptr), "silu_mul_quant: null pointer");
@@ -1145,13 +1158,19 @@ extern "C" int pt_silu_mul_quant_rowwise_colwise(const void* gate_up, int64_t M,
   fill_common(a, gate_up, PT_BF16, M, half, ld_gate_up);
   a.half = half; a.row_limit = valid_rows;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_t_fp8; a.b_scale = ch_scale;
+  order_scales(a, order);
   return launch_silu_quant<PRO_SILU_FWD>(a, (hipStream_t)stream);
 }
+}  // namespace pt
+extern "C" int pt_silu_mul_quant_rowwise_colwise(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up,
+                                                 void* tok_fp8, float* tok_scale, void* ch_t_fp8, float* ch_scale,
+                                                 const int32_t* valid_rows, pt_stream_t stream) {
+  return silu_mul_quant(gate_up, M, half, ld_gate_up, tok_fp8, tok_scale, ch_t_fp8, ch_scale, valid_rows, RowScales::BY_ROW, stream);
+}
 
-extern "C" int pt_silu_mul_bwd_quant_rowwise_colwise(const void* grad_h, int64_t ld_grad_h, const void* gate_up,
-                                                     int64_t ld_gate_up, int64_t M, int64_t half, void* tok_fp8,
-                                                     float* tok_scale, void* ch_t_fp8, float* ch_scale,
-                                                     const int32_t* valid_rows, pt_stream_t stream) {
+namespace pt {
+int silu_mul_bwd_quant(const void* grad_h, int64_t ld_grad_h, const void* gate_up, int64_t ld_gate_up, int64_t M, int64_t half, void* tok_fp8,
+                       float* tok_scale, void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half && ld_grad_h >= half, "silu_mul_bwd_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
   PT_REQUIRE(grad_h && gate_up && tok_fp8 && tok_scale && ch_t_fp8 && ch_scale, "silu_mul_bwd_quant: null pointer");
@@ -1162,9 +1181,17 @@ extern "C" int pt_silu_mul_bwd_quant_rowwise_colwise(const void* grad_h, int64_t
   fill_common(a, grad_h, PT_BF16, M, 2 * half, ld_grad_h);
   a.half = half; a.x2 = gate_up; a.ldx2 = ld_gate_up; a.row_limit = valid_rows;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_t_fp8; a.b_scale = ch_scale;
+  order_scales(a, order);
   // with whole 128-column tiles per half, each workgroup makes a dgate tile and its dup twin
   if (half % 128 == 0) return launch_silu_quant<PRO_SILU_BWD_PAIR>(a, (hipStream_t)stream);
   return launch_silu_quant<PRO_SILU_BWD>(a, (hipStream_t)stream);
+}
+}  // namespace pt
+extern "C" int pt_silu_mul_bwd_quant_rowwise_colwise(const void* grad_h, int64_t ld_grad_h, const void* gate_up,
+                                                     int64_t ld_gate_up, int64_t M, int64_t half, void* tok_fp8,
+                                                     float* tok_scale, void* ch_t_fp8, float* ch_scale,
+                                                     const int32_t* valid_rows, pt_stream_t stream) {
+  return silu_mul_bwd_quant(grad_h, ld_grad_h, gate_up, ld_gate_up, M, half, tok_fp8, tok_scale, ch_t_fp8, ch_scale, valid_rows, RowScales::BY_ROW, stream);
 }
 
 // The same two steps inside a dense MLP: any row count, the twins with a pitch and in the scalings of the dense
@@ -1205,10 +1232,9 @@ extern "C" int pt_silu_mul_bwd_quant_rowwise_transpose_ld(const void* grad_h, in
 }
 
 // ---- clamped SwiGLU (interleaved gate/up) fused into the activation quantisation -----------------
-extern "C" int pt_clamped_swiglu_quant_rowwise_colwise(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up,
-                                                       float alpha, float limit, void* tok_fp8, float* tok_scale,
-                                                       void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows,
-                                                       pt_stream_t stream) {
+namespace pt {
+int clamped_swiglu_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up, float alpha, float limit, void* tok_fp8, float* tok_scale,
+                         void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half, "clamped_swiglu_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
   PT_REQUIRE(gate_up && tok_fp8 && tok_scale && (ch_t_fp8 == nullptr) == (ch_scale == nullptr), "clamped_swiglu_quant: null pointer");
@@ -1218,14 +1244,21 @@ extern "C" int pt_clamped_swiglu_quant_rowwise_colwise(const void* gate_up, int6
   fill_common(a, gate_up, PT_BF16, M, half, ld_gate_up);
   a.half = half; a.row_limit = valid_rows; a.alpha = alpha; a.limit = limit;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_t_fp8; a.b_scale = ch_scale;
+  order_scales(a, order);
   return launch_silu_quant<PRO_CSWIGLU_FWD>(a, (hipStream_t)stream);
 }
+}  // namespace pt
+extern "C" int pt_clamped_swiglu_quant_rowwise_colwise(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up,
+                                                       float alpha, float limit, void* tok_fp8, float* tok_scale,
+                                                       void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows,
+                                                       pt_stream_t stream) {
+  return clamped_swiglu_quant(gate_up, M, half, ld_gate_up, alpha, limit, tok_fp8, tok_scale, ch_t_fp8, ch_scale, valid_rows, RowScales::BY_ROW, stream);
+}
 
-extern "C" int pt_clamped_swiglu_bwd_quant_rowwise_colwise(const void* grad_h, int64_t ld_grad_h, const void* gate_up,
-                                                           int64_t ld_gate_up, int64_t M, int64_t half, float alpha,
-                                                           float limit, void* tok_fp8, float* tok_scale, void* ch_t_fp8,
-                                                           float* ch_scale, float* col_sum, const int32_t* valid_rows,
-                                                           pt_stream_t stream) {
+namespace pt {
+int clamped_swiglu_bwd_quant(const void* grad_h, int64_t ld_grad_h, const void* gate_up, int64_t ld_gate_up, int64_t M, int64_t half, float alpha,
+                             float limit, void* tok_fp8, float* tok_scale, void* ch_t_fp8, float* ch_scale, float* col_sum, const int32_t* valid_rows,
+                             RowScales order, pt_stream_t stream) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half && ld_grad_h >= half,
              "clamped_swiglu_bwd_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
@@ -1239,5 +1272,15 @@ extern "C" int pt_clamped_swiglu_bwd_quant_rowwise_colwise(const void* grad_h, i
   a.half = half; a.x2 = gate_up; a.ldx2 = ld_gate_up; a.row_limit = valid_rows; a.alpha = alpha; a.limit = limit;
   a.col_sum = col_sum;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_t_fp8; a.b_scale = ch_scale;
+  order_scales(a, order);
   return launch_silu_quant<PRO_CSWIGLU_BWD>(a, (hipStream_t)stream);
+}
+}  // namespace pt
+extern "C" int pt_clamped_swiglu_bwd_quant_rowwise_colwise(const void* grad_h, int64_t ld_grad_h, const void* gate_up,
+                                                           int64_t ld_gate_up, int64_t M, int64_t half, float alpha,
+                                                           float limit, void* tok_fp8, float* tok_scale, void* ch_t_fp8,
+                                                           float* ch_scale, float* col_sum, const int32_t* valid_rows,
+                                                           pt_stream_t stream) {
+  return clamped_swiglu_bwd_quant(grad_h, ld_grad_h, gate_up, ld_gate_up, M, half, alpha, limit, tok_fp8, tok_scale, ch_t_fp8, ch_scale, col_sum, valid_rows,
+                                  RowScales::BY_ROW, stream);
 }

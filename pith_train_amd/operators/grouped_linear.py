@@ -134,6 +134,21 @@ class GroupedLinear(nn.Module):
 # ------------------------------------------------------------------------------------------------
 # FP8
 # ------------------------------------------------------------------------------------------------
+def _scales_by_block(scale: torch.Tensor) -> bool:
+    """Whether row scales ``[M, K/128]`` lie in memory as ``[K/128, M]``: the form that a fused step makes for
+    its own GEMMs, which read it in whole lines."""
+    return not scale.is_contiguous() and scale.dim() == 2 and scale.stride() == (1, scale.shape[0])
+
+
+def _m_grouped_by_block(a, b, out, grouped_mm_offs, out_rows, sizes, reduction_major: bool) -> torch.Tensor:
+    _lib.call(
+        "pt_gemm_m_grouped_by_block", a[0].data_ptr(), a[1].data_ptr(), b[0].data_ptr(), b[1].data_ptr(), int(reduction_major),
+        out.data_ptr(), _lib.dtype_code(out.dtype), grouped_mm_offs.data_ptr(), b[0].shape[0], *sizes, _lib.ptr(out_rows),
+        0 if out_rows is None else out.shape[0], _lib.stream_ptr(out.device),
+    )  # fmt: skip
+    return out
+
+
 def m_grouped_fp8_gemm_nt(a, b, out: torch.Tensor, grouped_mm_offs: torch.Tensor,
                           out_rows: torch.Tensor | None = None, bias: torch.Tensor | None = None) -> torch.Tensor:
     """out[rows_g] = a[rows_g] @ b[g].T with a=(fp8[M,K], scale[M,K/128]), b=(fp8[G,N,K],
@@ -146,6 +161,10 @@ def m_grouped_fp8_gemm_nt(a, b, out: torch.Tensor, grouped_mm_offs: torch.Tensor
     M, K = a_fp8.shape
     G, N, Kb = b_fp8.shape
     assert Kb == K, (b_fp8.shape, a_fp8.shape)
+    if _scales_by_block(a_s):
+        if bias is None:
+            return _m_grouped_by_block(a, b, out, grouped_mm_offs, out_rows, (M, N, K), False)
+        a_s = a_s.contiguous()
     if bias is not None:
         assert bias.shape == (G, N) and bias.dtype == out.dtype and bias.is_contiguous()
     if bias is not None and out_rows is not None:
@@ -258,6 +277,8 @@ def m_grouped_fp8_gemm_nn(a, b, out: torch.Tensor, grouped_mm_offs: torch.Tensor
     M, K = a_fp8.shape
     G, Kb, N = b_fp8.shape
     assert Kb == K, (b_fp8.shape, a_fp8.shape)
+    if _scales_by_block(a_s):
+        return _m_grouped_by_block(a, b, out, grouped_mm_offs, out_rows, (M, N, K), True)
     if out_rows is not None:
         _lib.call(
             "pt_gemm_m_grouped_nn_scatter", a_fp8.data_ptr(), a_s.data_ptr(), b_fp8.data_ptr(),

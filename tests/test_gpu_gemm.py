@@ -449,6 +449,43 @@ def test_m_grouped_scattered_rows_with_bias_of_short_reductions(sizes, N, K, gem
     assert torch.equal(out[rows.long()], plain + bias[group])
 
 
+@pytest.mark.parametrize("N,K", [(256, 128), (272, 1408), (2880, 2880)])
+def test_row_scales_by_block(gemm_kernel, N, K):
+    """The quantiser writes the same scales as [K/128, M], and every grouped GEMM that reads them so has the bits of
+    the one that reads [M, K/128]: tiles past the last row and column, a reduction that ends inside a block."""
+    from pith_train_amd import _lib
+
+    g = torch.Generator(device="cuda").manual_seed(K)
+    rows = torch.tensor([128, 0, 384, 640], dtype=torch.int32)
+    G_, M, KB = len(rows), int(rows.sum()), (K + 127) // 128
+    offs = torch.cumsum(rows, 0).int().cuda()
+    x = torch.randn((M, K), device="cuda", generator=g).bfloat16() * torch.exp2(torch.randint(-9, 9, (M, 1), device="cuda", generator=g).float()).bfloat16()
+    q, q2 = (torch.empty((M, K), dtype=torch.uint8, device="cuda") for _ in range(2))
+    t, t2 = (torch.empty((K, M), dtype=torch.uint8, device="cuda") for _ in range(2))
+    s, s2 = torch.empty((M, KB), device="cuda"), torch.empty((KB, M), device="cuda")
+    ts, ts2 = (torch.empty((M // 128, K), device="cuda") for _ in range(2))
+    bf16 = _lib.dtype_code(torch.bfloat16)
+    _lib.call("pt_quant_rowwise_colwise", _lib.ptr(x), bf16, M, K, K, _lib.ptr(q), _lib.ptr(s), _lib.ptr(t), _lib.ptr(ts), _lib.PT_CH_TRANSPOSED, None, 0,
+              _lib.stream_ptr())
+    _lib.call("pt_quant_rowwise_colwise_by_block", _lib.ptr(x), bf16, M, K, K, _lib.ptr(q2), _lib.ptr(s2), _lib.ptr(t2), _lib.ptr(ts2), _lib.stream_ptr())
+    assert torch.equal(q, q2) and torch.equal(t, t2) and torch.equal(ts, ts2) and torch.equal(s, s2.t())
+    b = torch.randint(0, 256, (G_, N, K), dtype=torch.uint8, device="cuda", generator=g) & 0xBF
+    b_s = torch.exp2(torch.randint(-6, 3, (G_, (N + 127) // 128, KB), device="cuda", generator=g).float())
+    b_t, b_ts = b.transpose(1, 2).contiguous(), b_s.transpose(1, 2).contiguous()
+    to = torch.randperm(M, device="cuda", generator=g).int()
+    for reduction_major, scatter in ((0, False), (0, True), (1, False), (1, True)):
+        if gemm_kernel == "t" and scatter and not reduction_major:
+            continue  # refused: that kernel stores no scattered rows
+        w, w_s = (b_t, b_ts) if reduction_major else (b, b_s)
+        want, got = (torch.zeros((M, N), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        name = "pt_gemm_m_grouped_" + ("nn" if reduction_major else "nt") + ("_scatter" if scatter else "")
+        _lib.call(name, _lib.ptr(q), _lib.ptr(s), _lib.ptr(w), _lib.ptr(w_s), _lib.ptr(want), bf16, _lib.ptr(offs), G_, M, N, K,
+                  *((_lib.ptr(to), M) if scatter else ()), _lib.stream_ptr())
+        _lib.call("pt_gemm_m_grouped_by_block", _lib.ptr(q), _lib.ptr(s2), _lib.ptr(w), _lib.ptr(w_s), reduction_major, _lib.ptr(got), bf16, _lib.ptr(offs),
+                  G_, M, N, K, _lib.ptr(to) if scatter else None, M if scatter else 0, _lib.stream_ptr())
+        assert torch.equal(want, got)
+
+
 @pytest.mark.parametrize("tiles", [1, 3, 4, 10])
 def test_grouped_tile_order_at_the_edges_of_its_strips(gemm_kernel, tiles):
     """Groups with more row tiles than column tiles and the other way round, one strip and several of unequal
