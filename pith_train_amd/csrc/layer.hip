@@ -119,16 +119,23 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
   if (a.M == 0) return PT_OK;
   const int32_t G = (int32_t)a.G;
   const int32_t* limit = a.limit_rows ? a.offs + G - 1 : nullptr;
+  // The gradient of the down bias is the sum of the rows that are quantised here: the kernel that reads them adds up
+  // every 128 (groups are whole 128-row tiles) where col_sum, which the activation's backward fills afterwards, has
+  // room for those sums (16384 tokens x 4 of 2880 columns: a second pass over the rows took 110 us, the sums here cost
+  // 12 and their sum over the tiles 9).
+  float* const dy_sums = a.d_dn_bias && a.clamped && a.H <= 2 * a.half ? a.col_sum : nullptr;
   const auto quant_dy = [&](const int32_t* ends) {
     return quant_rowwise_colwise(a.grad_out, a.grad_rows, 1, PT_BF16, a.M, a.H, a.H, a.out_map, a.dy_fp8, a.dy_scale, order, a.dy_t, a.dy_t_scale,
-                                 PT_CH_TRANSPOSED, ends, ends ? G : 0, a.stream);
+                                 PT_CH_TRANSPOSED, ends, ends ? G : 0, a.stream, dy_sums);
   };
   if (a.out_map)
     PT_STEP_AS(pt_quant_rowwise_colwise_rows, a.M, a.H, a.grad_rows, quant_dy(a.offs));
   else
     PT_STEP_AS(pt_quant_rowwise_colwise, a.M, a.H, a.grad_rows, quant_dy(nullptr));
   if (a.d_dn_bias) {
-    if (a.out_map)
+    if (dy_sums)
+      PT_STEP(pt_segment_sum_tiles, a.M / 128, a.H, 0, dy_sums, a.offs, 128, G, a.d_dn_bias, a.M / 128, a.H, (int)a.d_dn_bias_dtype, a.stream);
+    else if (a.out_map)
       PT_STEP(pt_segment_sum_rows, a.M, a.H, 0, a.grad_out, a.grad_rows, a.out_map, a.offs, G, a.d_dn_bias, a.M, a.H, PT_BF16,
               (int)a.d_dn_bias_dtype, a.stream);
     else

@@ -82,7 +82,7 @@ struct QuantArgs {
   int64_t ld_t;                  // row pitch of the transposed twin (bytes = elements); M unless it is a column slice
   int64_t bs_ld;                 // row length of the twin's block-scale grid; tiles_m unless it is a column slice
   float alpha, limit;            // fused clamped SwiGLU: its two constants
-  float* col_sum;                // fused clamped SwiGLU backward: [tiles_m, N] column sums of each 128-row tile
+  float* col_sum;                // PRO_SUMS and fused clamped SwiGLU backward: [tiles_m, N] column sums of each 128-row tile
   int32_t head_a, head_b;        // per-head halves in two tensors: column h * (head_a + head_b) + c is x[h * head_a + c] or x2[h * head_b + c - head_a]
 };
 
@@ -191,7 +191,8 @@ template <> struct Frag<float> {
 
 // what the tile is computed from
 enum { PRO_NONE = 0, PRO_SILU_FWD = 1, PRO_SILU_BWD = 2, PRO_SILU_BWD_PAIR = 3, PRO_CSWIGLU_FWD = 4, PRO_CSWIGLU_BWD = 5,
-       PRO_HEADS = 6 };
+       PRO_HEADS = 6, PRO_SUMS = 7 };  // PRO_SUMS: nothing before, the tile's column sums beside
+constexpr bool writes_sums(int pro) { return pro == PRO_CSWIGLU_BWD || pro == PRO_SUMS; }
 
 // ---- packed-bf16 arithmetic of the interior-tile path -------------------------------------------
 // |x| of a bf16 is its low 15 bits, and for non-negative floats the integer order of the bits is
@@ -325,7 +326,7 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
       if (FULL || (col_ok && row0 + i < p.M)) f.load_row(i, base + i * pitch);
       else f.zero_row(i);
     }
-  } else if constexpr (PRO != PRO_NONE) {
+  } else if constexpr (PRO != PRO_NONE && PRO != PRO_SUMS) {
     // The quantised tensor is the bf16-rounded SwiGLU output (forward: h = silu(gate) * up from
     // gate_up = x) or its gradient (backward: [dgate | dup] from grad_h = x and gate_up = x2),
     // computed here instead of being written to memory and read back.  bf16 only, 16-byte loads.
@@ -516,9 +517,9 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
       }
     }
   }
-  if constexpr (PRO == PRO_CSWIGLU_BWD) {
-    // Column sums of the tile's bf16 values (the bias gradient of the projection before the
-    // activation is their sum over a group's tiles): rows of the thread in order, then the four
+  if constexpr (writes_sums(PRO)) {
+    // Column sums of the tile's bf16 values (the bias gradient of the projection whose gradient they
+    // are is their sum over a group's tiles): rows of the thread in order, then the four
     // row groups of a wave pairwise, then the four waves after the barrier.
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -541,7 +542,7 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
     if (lane == 0) s_blk[wave] = m;
   }
   __syncthreads();
-  if constexpr (PRO == PRO_CSWIGLU_BWD) {
+  if constexpr (writes_sums(PRO)) {
     if (rg == 0) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -707,7 +708,7 @@ void quant_tile_kernel(QuantArgs p) {
   __shared__ float s_colmax[4][128];
   __shared__ float s_blk[4];
   __shared__ __attribute__((aligned(16))) uint8_t s_t[128 * 128];
-  __shared__ float s_colsum[PRO == PRO_CSWIGLU_BWD ? 4 : 1][128];
+  __shared__ float s_colsum[writes_sums(PRO) ? 4 : 1][128];
 
   int64_t bid = blockIdx.x;
   // PRO_SILU_BWD_PAIR: one workgroup produces the dgate tile and its dup twin (half / 128 column
@@ -864,7 +865,7 @@ static bool repeat_fits(int64_t rows, int64_t repeat) {
 
 int quant_rowwise_colwise(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
                           void* tok_fp8, float* tok_scale, RowScales order, void* ch_fp8, float* ch_scale, int ch_layout, const int32_t* offs,
-                          int32_t num_groups, pt_stream_t stream) {
+                          int32_t num_groups, pt_stream_t stream, float* col_sum) {
   PT_REQUIRE(M >= 0 && N >= 0 && M % 128 == 0, "quant_rowwise_colwise: M=%lld must be a multiple of 128", (long long)M);
   PT_REQUIRE(ldx >= N, "quant_rowwise_colwise: ldx < N");
   PT_REQUIRE(repeat == 1 || (repeat_fits(rows, repeat) && (row_index || M == 0)), "quant_rowwise_colwise: %lld rows, each %lld times, are too many",
@@ -879,6 +880,14 @@ int quant_rowwise_colwise(const void* x, int64_t rows, int64_t repeat, int dtype
   if (repeat > 1) a.row_mul = (uint32_t)(((1ull << 32) + repeat - 1) / repeat);
   if (offs && num_groups > 0) a.row_limit = offs + (num_groups - 1);
   hipStream_t s = (hipStream_t)stream;
+  if (col_sum) {
+    PT_REQUIRE(dtype == PT_BF16 && ch_layout == PT_CH_TRANSPOSED && ch_fp8, "quant_rowwise_colwise: column sums go with bf16 rows and the transposed twin");
+    a.col_sum = col_sum;
+    const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
+    PT_REQUIRE(blocks < (1ll << 31), "quant: grid too large (%lld tiles)", (long long)blocks);
+    hipLaunchKernelGGL((quant_tile_kernel<bf16_tag, A_ROW, B_COL, BL_TRANSPOSED, BS_MB_N, PRO_SUMS>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+    return check_launch("quant_tile_kernel(column sums)");
+  }
   switch (ch_layout) {
     case PT_CH_ROWMAJOR:   return launch_quant<A_ROW, B_COL, BL_ROWMAJOR, BS_MB_N>(a, dtype, 1, s);
     case PT_CH_TRANSPOSED: return launch_quant<A_ROW, B_COL, BL_TRANSPOSED, BS_MB_N>(a, dtype, 1, s);

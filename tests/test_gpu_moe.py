@@ -478,6 +478,26 @@ def test_moe_block_reference_forward_against_the_oracle_chain(family):
         _close(gate.weight.grad, wg.grad, f"{family} gate weight gradient")
 
 
+@pytest.mark.parametrize("H,I", [(256, 384), (272, 136), (512, 128)])
+def test_down_bias_gradient_is_the_sum_of_its_group_s_rows(H, I):
+    """Summed by the kernel that quantises the rows (whole tiles; a last column tile of 16; up to 2 I columns), and in
+    a pass of its own past those: one rounding to bf16 of the sum of n rows in 32 bits, whose error stays below
+    n / 8 + 12 roundings of the sum of magnitudes (a thread adds 8 of a tile's rows, the rest is pairwise or 16 ways)."""
+    from pith_train_amd.modules.experts import forward_stage3
+
+    E, T, k = 8, 900, 2
+    ids = OM.make_routing(T, E, k, seed=5, zipf=1.2).reshape(-1).cuda()
+    mod, params = _build("gpt_oss", E, H, I, _weights("gpt_oss", E, H, I, 6))
+    g = torch.Generator().manual_seed(7)
+    x, dy = (torch.randn((T * k, H), generator=g).bfloat16().cuda() for _ in range(2))
+    forward_stage3(mod, x.requires_grad_(True), ids, E).backward(dy)
+    got = params["down_proj_bias"].grad.double()
+    for e in range(E):
+        rows = dy[ids == e].double()
+        want, magnitude = rows.sum(0), rows.abs().sum(0)
+        assert ((got[e] - want).abs() <= want.abs() * 2.0**-8 + magnitude * (len(rows) / 8 + 12) * 2.0**-24).all(), e
+
+
 @pytest.mark.parametrize("kind", ["fused", "split", "gpt_oss"])
 def test_stage3_builds_the_weight_twin_when_the_forward_layout_kernel_cannot_address_the_problem(kind, monkeypatch):
     """The input-gradient kernel on forward-layout weights has 32-bit limits; past them the forward
