@@ -478,7 +478,7 @@ def test_moe_block_reference_forward_against_the_oracle_chain(family):
         _close(gate.weight.grad, wg.grad, f"{family} gate weight gradient")
 
 
-@pytest.mark.parametrize("H,I", [(256, 384), (272, 136), (512, 128)])
+@pytest.mark.parametrize("H,I", [(256, 384), (272, 144), (512, 128)])
 def test_down_bias_gradient_is_the_sum_of_its_group_s_rows(H, I):
     """Summed by the kernel that quantises the rows (whole tiles; a last column tile of 16; up to 2 I columns), and in
     a pass of its own past those: one rounding to bf16 of the sum of n rows in 32 bits, whose error stays below
@@ -486,7 +486,7 @@ def test_down_bias_gradient_is_the_sum_of_its_group_s_rows(H, I):
     from pith_train_amd.modules.experts import forward_stage3
 
     E, T, k = 8, 900, 2
-    ids = OM.make_routing(T, E, k, seed=5, zipf=1.2).reshape(-1).cuda()
+    ids = OM.make_routing(T, E, k, seed=5, zipf_s=1.2).reshape(-1).cuda()
     mod, params = _build("gpt_oss", E, H, I, _weights("gpt_oss", E, H, I, 6))
     g = torch.Generator().manual_seed(7)
     x, dy = (torch.randn((T * k, H), generator=g).bfloat16().cuda() for _ in range(2))
