@@ -334,6 +334,12 @@ __device__ __forceinline__ void scan_group_costs(const GemmArgs& p, int* s_pref,
   scan_groups(p, s_pref, tid, lane, [&](int g) { return k_group_end(p, g); }, [](int rows) { return k_group_tile_cost(rows); });
 }
 
+// Groups of nearly equal cost (largest within a quarter of the mean): the plain cut by count, which
+// for a group count that is a multiple of eight also keeps whole groups on one XCD.
+__device__ __forceinline__ bool level_groups(const GemmArgs& p, const int* s_pref) {
+  return (int64_t)s_pref[p.G + 1] * p.G * 4 <= (int64_t)s_pref[p.G] * 5;
+}
+
 // First logical tile of XCD `x` (x in [0, 8]; x = 8 gives the end of the list).  Dense and
 // m-grouped tiles all cost the same, so the list is cut into eight equal counts.  k-grouped tiles
 // cost in proportion to their group's row count: the list (group-major) is cut where the summed
@@ -342,10 +348,7 @@ __device__ __forceinline__ void scan_group_costs(const GemmArgs& p, int* s_pref,
 // workgroups per XCD.
 template <int MODE>
 __device__ __forceinline__ int xcd_first_tile(const GemmArgs& p, const int* s_pref, int total_tiles, int x, int round) {
-  // Groups of nearly equal cost (largest within a quarter of the mean): the plain cut by count, which
-  // for a group count that is a multiple of eight also keeps whole groups on one XCD.
-  const bool by_count = MODE != GEMM_K_GROUPED || (int64_t)s_pref[p.G + 1] * p.G * 4 <= (int64_t)s_pref[p.G] * 5;
-  if (by_count) {
+  if (MODE != GEMM_K_GROUPED || level_groups(p, s_pref)) {
     const int per_xcd = (total_tiles + 7) / 8;
     const int t = x * per_xcd;
     return t < total_tiles ? t : total_tiles;
@@ -368,9 +371,178 @@ __device__ __forceinline__ int xcd_first_tile(const GemmArgs& p, const int* s_pr
   return t < total_tiles ? t : total_tiles;
 }
 
-// Geometry of logical tile t; plain per-lane arithmetic (every lane may ask for a different t).
+// ---- k-grouped tiles of skewed groups -------------------------------------------------------------
+// Tiles of groups of 64 blocks and of one stand in the same list, so a cut of the list by cost that rounds to whole
+// rounds of workgroups, and dealing it out by count, leave workgroups idle where the largest tile is a good part of
+// a workgroup's share.  There every XCD takes an eighth of every group of big tiles (more than an eighth of a share each;
+// neighbours in the group's order, the remainders of the eighths in turn), and deals them out one by one, largest
+// first, to the workgroup that has the least.  The other groups stay together: their list is cut by cost, and the
+// workgroups of an XCD take its part in turns, one that has less so far the earlier, as if each took the next
+// tile when it is done.  All of it is the same arithmetic in every workgroup (one wave).  Weight gradients with
+// Zipf-distributed popularity, us: 8192 tokens of 6 in 64 groups 2816 x 2048 372 -> 317, 2048 x 1408 229 -> 172, of 8 in
+// 128 groups 1536 x 2048 325 -> 291; 16384 of 8 in 64 groups 518 -> 425.
+static constexpr int kSchedGroups = 256;  // groups it is made for: four a lane
+static constexpr int kSchedPart = 8;
+static constexpr int kNoLoad = 0x3fffffff;
+struct KSchedule {  // in LDS
+  int tiles[kSchedGroups + 1], cost[kSchedGroups + 1];  // of the small groups before g: tiles, and their cost
+  int ahead[64];                                        // the XCD's workgroups: cost of their big tiles in small ones
+  int big[128];                                         // this workgroup's big tiles: group * 2^22 + place in the group
+  int n_big, first, last, n;                            // how many; the XCD's small tiles; how many tiles in all
+};
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_min(int v) {
+  const int o = __builtin_amdgcn_update_dpp(kNoLoad, v, CTRL, ROWS, 0xf, false);
+  return o < v ? o : v;
+}
+__device__ __forceinline__ int wave_min(int v) {
+  v = dpp_min<0x111, 0xf>(v); v = dpp_min<0x112, 0xf>(v); v = dpp_min<0x114, 0xf>(v); v = dpp_min<0x118, 0xf>(v);  // row_shr 1, 2, 4, 8
+  v = dpp_min<0x142, 0xa>(v);  // row_bcast 15
+  v = dpp_min<0x143, 0xc>(v);  // row_bcast 31
+  return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_scan(int v, int lane) {  // sum up to this lane
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) { const int y = __shfl_up(v, d); if (lane >= d) v += y; }
+  return v;
+}
+// an XCD's tiles of a big group: from .. from + number
+__device__ __forceinline__ void xcd_share(int per_g, int xcd, int g, int& from, int& number) {
+  const int y = (xcd + g) & 7;
+  from = per_g * y >> 3;
+  number = (per_g * (y + 1) >> 3) - from;
+}
+// Whether a launch is scheduled so: its largest tile makes a quarter of a workgroup's share, and that share 96 blocks (the
+// schedule takes 6 us and its rounds some more: shares of 60 and 87 blocks 87 -> 104 and 145 -> 163 us, of 15 40 -> 63;
+// largest tiles of 0.17 of a share 607 -> 719).  What the lists above can hold (a workgroup's share in big tiles
+// and one more); sums that stay below 2^29, a workgroup's below 2^22.
+__device__ __forceinline__ bool scheduled_groups(const GemmArgs& p, const int* s_pref, int workers) {
+  const int64_t per_g = (int64_t)p.tiles_a * p.tiles_b, total = s_pref[p.G] * per_g;
+  return p.offs && p.G <= kSchedGroups && workers <= 64 && per_g < (1 << 22) && total < (8ll << 22) * workers && total < (1ll << 29) && !level_groups(p, s_pref) &&
+         (int64_t)s_pref[p.G + 1] * 4 * 8 * workers >= total && total >= 96ll * 8 * workers;
+}
+// Place of workgroup `me`'s small tile j in the XCD's part of their list.  ahead: on lane w the big tiles of workgroup w
+// in small ones; tiles are taken in the order of (ahead + count so far, workgroup).
+__device__ __forceinline__ int small_place(int ahead, int me, int workers, int j) {
+  const int time = __builtin_amdgcn_readlane(ahead, me) + j;
+  int place = 0;
+  for (int w = 0; w < workers; ++w) {
+    const int before = time - __builtin_amdgcn_readlane(ahead, w) + (w < me);
+    place += before > 0 ? before : 0;
+  }
+  return place;
+}
+// By the first wave; the caller waits for the workgroup.  `workers` workgroups an XCD, this one is `me`.
+__device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* s_pref, KSchedule& s, int xcd, int me, int workers, int lane) {
+  const int per_g = p.tiles_a * p.tiles_b;
+  const int least = (int)((int64_t)s_pref[p.G] * per_g / (kSchedPart * 8 * workers)) + 1;  // cost of a big tile
+  int cost[4];
+  unsigned left = 0;  // the lane's groups of big tiles that have not been dealt out
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int g = 4 * lane + r;
+    cost[r] = g < p.G ? s_pref[g + 1] - s_pref[g] : 0;
+    if (cost[r] >= least) left |= 1u << r;
+  }
+  // ---- the others: their list, and this XCD's part of it ----
+  int tiles = 0, sum = 0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (!(left >> r & 1) && cost[r]) { tiles += per_g; sum += per_g * cost[r]; }
+  int tiles0 = wave_scan(tiles, lane), sum0 = wave_scan(sum, lane);
+  const int all_tiles = __builtin_amdgcn_readlane(tiles0, 63), all = __builtin_amdgcn_readlane(sum0, 63);
+  tiles0 -= tiles;
+  sum0 -= sum;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    s.tiles[4 * lane + r] = tiles0;
+    s.cost[4 * lane + r] = sum0;
+    if (!(left >> r & 1) && cost[r]) { tiles0 += per_g; sum0 += per_g * cost[r]; }
+  }
+  if (lane == 0) { s.tiles[kSchedGroups] = all_tiles; s.cost[kSchedGroups] = all; }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's own writes
+  int part;
+  {
+    // number of tiles whose middle lies below y, on lanes 0 and 1 for the two ends of the part
+    const int y = (int)((int64_t)all * (xcd + (lane & 1)) / 8);
+    int lo = 0, hi = kSchedGroups - 1;  // last g with cost[g] <= y
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (s.cost[mid] <= y) lo = mid; else hi = mid - 1;
+    }
+    const int n = s.tiles[lo + 1] - s.tiles[lo], c = n ? (s.cost[lo + 1] - s.cost[lo]) / n : 1;
+    const int b = (2 * (y - s.cost[lo]) + c - 1) / (2 * c), below = s.tiles[lo] + (b < n ? b : n);
+    const int first = __builtin_amdgcn_readlane(below, 0), last = xcd == 7 ? all_tiles : __builtin_amdgcn_readlane(below, 1);
+    part = last - first;
+    if (lane == 0) { s.first = first; s.last = last; }
+  }
+  // ---- the big ones ----
+  int load = lane < workers ? 0 : kNoLoad, n_big = 0;
+  while (__ballot(left != 0)) {
+    int most = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (left >> r & 1) most = cost[r] > most ? cost[r] : most;
+    const int c = -wave_min(-most);
+    int mine = 0;  // the lane's first group of that cost
+#pragma unroll
+    for (int r = 3; r >= 0; --r)
+      if ((left >> r & 1) && cost[r] == c) mine = r;
+    const int owner = __builtin_ctzll(__ballot(most == c));
+    if (lane == owner) left &= ~(1u << mine);
+    const int g = 4 * owner + __builtin_amdgcn_readlane(mine, owner);
+    int at, n;
+    xcd_share(per_g, xcd, g, at, n);
+    while (n > 0) {
+      // every workgroup that would still be ahead of another with one more takes one; if there are too few, those with the least
+      const int low = wave_min(load);
+      uint64_t takers = __ballot(load < low + c);
+      if (__popcll(takers) > n) takers = __ballot(load == low);
+      const int k = __popcll(takers), deal = k < n ? k : n;
+      const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(takers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)takers, 0));
+      if ((takers >> lane & 1) && rank < deal) {
+        if (lane == me) s.big[n_big] = g << 22 | (at + rank);
+        ++n_big;
+        load += c;
+      }
+      at += deal;
+      n -= deal;
+    }
+  }
+  const int ahead = all_tiles ? (int)((float)load * ((float)all_tiles / (float)all) + 0.5f) : 0;
+  s.ahead[lane] = ahead;
+  n_big = __builtin_amdgcn_readlane(n_big, me);
+  if (lane == 0) s.n_big = n_big;
+  int n = n_big;
+  for (int j = lane;; j += 64) {
+    const int k = __popcll(__ballot(small_place(ahead, me, workers, j) < part));
+    n += k;
+    if (k < 64) break;
+  }
+  if (lane == 0) s.n = n;
+}
+
+// the workgroup's tile i, one on every lane of the first wave: its group and its place in it
+__device__ __forceinline__ void scheduled_tile(const KSchedule& s, int me, int workers, int lane, int i, int& g, int& idx) {
+  const int t = s.first + small_place(s.ahead[lane], me, workers, i - s.n_big);
+  if (i < s.n_big) {
+    g = s.big[i] >> 22;
+    idx = s.big[i] & ((1 << 22) - 1);
+    return;
+  }
+  int lo = 0, hi = kSchedGroups - 1;  // last g with tiles[g] <= t
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (s.tiles[mid] <= t) lo = mid; else hi = mid - 1;
+  }
+  g = lo;
+  idx = t - s.tiles[lo];
+}
+
+// Geometry of logical tile t (k-grouped, with group >= 0: of that group's tile t); plain per-lane arithmetic (every lane
+// may ask for a different one).
 template <int MODE, int BM, int BN>
-__device__ __forceinline__ void decode_tile(const GemmArgs& p, const int* s_pref, int t, Tile& T) {
+__device__ __forceinline__ void decode_tile(const GemmArgs& p, const int* s_pref, int t, Tile& T, int group = -1) {
   // The 32 CUs of an XCD work on 32 consecutive logical tiles at a time.  One side of the tile grid is cut into
   // strips of at most `width` tiles (of nearly equal width), and a strip is walked line by line along the other
   // side: 32 consecutive tiles then share 32 / w tiles of one operand and w of the other in that XCD's L2
@@ -421,8 +593,8 @@ __device__ __forceinline__ void decode_tile(const GemmArgs& p, const int* s_pref
     T.a_lim = p.offs[g]; T.b_lim = (int)p.rows_b; T.k_begin = 0; T.k_len = (int)p.red; T.kb0 = 0;
   } else {
     const int per_g = p.tiles_a * p.tiles_b;
-    const int g = t / per_g;
-    const int idx = t % per_g;
+    const int g = group >= 0 ? group : t / per_g;
+    const int idx = group >= 0 ? t : t % per_g;
     T.g = g;
     int ta, tb;
     if (p.offs) group_strips(idx, p.tiles_a, p.tiles_b, ta, tb);

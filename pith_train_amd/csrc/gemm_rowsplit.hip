@@ -57,7 +57,8 @@ static constexpr int kRsTiles = 48, kRsEntry = 48;
 static constexpr int kRsPref = kRsTable + kRsTiles * kRsEntry;
 static constexpr int kRsIndex = kRsPref + ((kMaxGroupsGemm + 2) * 4 + 15) / 16 * 16;
 static constexpr int kRsBias = kRsIndex + 256 * 4;
-static constexpr int kRsLds = kRsBias + 256 * 2;
+static constexpr int kRsSched = kRsBias + 256 * 2;
+static constexpr int kRsLds = kRsSched + sizeof(KSchedule);
 static_assert(kRsLds <= 160 * 1024 && kRsPref % 16 == 0, "LDS map");
 
 // BT: the b operand is given reduction-major, [red][rows_b] with row pitch ldb (the forward layout of
@@ -92,10 +93,19 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
   }
   const int xcd = blockIdx.x & 7;
   // lanes 0 and 1 find the two ends of this XCD's share of the list side by side
-  const int t_step = gridDim.x >> 3;
+  int t_step = gridDim.x >> 3;
   const int t_cut = xcd_first_tile<MODE>(p, s_pref, total_tiles, xcd + (lane & 1), t_step);
-  const int t_end = __builtin_amdgcn_readlane(t_cut, 1);
+  int t_end = __builtin_amdgcn_readlane(t_cut, 1);
   int t_next = __builtin_amdgcn_readlane(t_cut, 0) + (blockIdx.x >> 3);
+  KSchedule& sched = *(KSchedule*)(lds + kRsSched);
+  const bool scheduled = MODE == GEMM_K_GROUPED && scheduled_groups(p, s_pref, t_step);
+  if (scheduled) {
+    if (tid < 64) schedule_k_groups(p, s_pref, sched, xcd, blockIdx.x >> 3, t_step, lane);
+    __syncthreads();
+    t_next = 0;
+    t_end = __builtin_amdgcn_readfirstlane(sched.n);
+    t_step = 1;
+  }
 
   // ---- LDS addressing ----
   // A stage holds rows of 128 bytes (8 chunks of 16).  Row r keeps logical chunk c at position
@@ -281,9 +291,11 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
     }
     n_tiles = (t_end - t_next + t_step - 1) / t_step;
     if (n_tiles > kRsTiles) n_tiles = kRsTiles;
+    int t = t_next + tid * t_step, group = -1;
+    if (scheduled && tid < 64) scheduled_tile(sched, blockIdx.x >> 3, gridDim.x >> 3, lane, t, group, t);
     if (tid < n_tiles) {
       Tile T;
-      decode_tile<MODE, BM, BN>(p, s_pref, t_next + tid * t_step, T);
+      decode_tile<MODE, BM, BN>(p, s_pref, t, T, group);
       const int64_t a_end = (int64_t)T.a_lim * p.lda < p.a_bytes ? (int64_t)T.a_lim * p.lda : p.a_bytes;
       const uint32_t soA = (uint32_t)T.a_row0 * lda + T.k_begin;
       const uint32_t soB = BT ? (uint32_t)T.k_begin * ldb + (uint32_t)T.b_row0 : (uint32_t)T.b_row0 * ldb + T.k_begin;

@@ -449,6 +449,44 @@ def test_m_grouped_scattered_rows_with_bias_of_short_reductions(sizes, N, K, gem
     assert torch.equal(out[rows.long()], plain + bias[group])
 
 
+@pytest.mark.parametrize("groups,N,W", [(3, 1024, 2048), (40, 1100, 1800), (256, 1024, 1280)])
+def test_k_grouped_schedule_of_skewed_groups(gemm_kernel, groups, N, W):
+    """A group of half of the rows, two of a quarter and so on, the others small or empty, so that workgroups are dealt the
+    big tiles one by one: every tile is computed, once (accumulating), with the bits of the kernel that takes one small
+    tile per workgroup."""
+    from pith_train_amd import _lib
+
+    if gemm_kernel != "auto":
+        pytest.skip("the test selects the kernels itself; run once")
+    g = torch.Generator(device="cuda").manual_seed(groups)
+    tiles = -(-N // 256) * -(-W // 256)
+    total = 1.3 * 96 * 256 / tiles  # blocks: a share of 125
+    blocks = torch.randint(0, 3, (groups,), generator=torch.Generator().manual_seed(groups))
+    for i, share in enumerate((2, 4, 4, 8, 8, 16, 32)[:groups]):
+        blocks[i * (groups // 7 or 1)] = int(total / share)
+    offs, M = torch.cumsum(blocks * 128, 0).int().cuda(), int(blocks.sum()) * 128
+    cost = blocks + 3
+    assert cost.sum() * tiles >= 96 * 256 and cost.max() * 4 * 256 >= cost.sum() * tiles  # what the rule asks for
+
+    def fp8(*shape):
+        return torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # finite values below 2
+
+    def scale(*shape):
+        return torch.exp2(torch.randint(-6, 3, shape, device="cuda", generator=g).float())
+
+    d, sd, x, sx = fp8(N, M), scale(M // 128, N), fp8(W, M), scale(M // 128, W)
+    start = torch.randn((groups, N, W), device="cuda", generator=g).bfloat16()
+    for add in (0, 1):
+        out = []
+        for kernel in (b"r0", b"s128"):
+            _lib.call("pt_gemm_select_kernel", kernel)
+            o = start.clone()
+            _lib.call("pt_gemm_k_grouped_wgrad", _lib.ptr(d), _lib.ptr(sd), _lib.ptr(x), _lib.ptr(sx), _lib.ptr(o), _lib.dtype_code(o.dtype), add,
+                      _lib.ptr(offs), groups, M, N, W, _lib.stream_ptr())
+            out.append(o)
+        assert torch.equal(*out)
+
+
 @pytest.mark.parametrize("N,K", [(256, 128), (272, 1408), (2880, 2880)])
 def test_row_scales_by_block(gemm_kernel, N, K):
     """The quantiser writes the same scales as [K/128, M], and every grouped GEMM that reads them so has the bits of
