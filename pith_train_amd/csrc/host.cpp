@@ -989,6 +989,20 @@ struct Quantised {
   }
 };
 
+// The GEMM of a fused step's own operand (its row scales lie as [K/128, M]), from Python: b [G, N, K], or reduction-major
+// [G, K, N]; result row r at out[rows[r]] when there is a map.
+void m_grouped_by_block(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, bool reduction_major, const Tensor& out, const Tensor& offs,
+                        const Maybe& rows, int64_t stream) {
+  const int64_t M = a.size(0), K = a.size(1), N = b.size(reduction_major ? 2 : 1), G = b.size(0);
+  const char* what = reduction_major ? rows ? "pt_gemm_m_grouped_nn_scatter" : "pt_gemm_m_grouped_nn"
+                                     : rows ? "pt_gemm_m_grouped_nt_scatter" : "pt_gemm_m_grouped_nt";
+  lib.pt_observe(what, 1, M, N, K);
+  check(lib.pt_gemm_m_grouped_by_block(ptr(a), (const float*)ptr(a_s), ptr(b), (const float*)ptr(b_s), reduction_major, ptr(out),
+                                       dtype_code(out.scalar_type()), (const int32_t*)ptr(offs), (int32_t)G, M, N, K, (const int32_t*)ptr(rows),
+                                       rows ? out.size(0) : 0, (pt_stream_t)stream), what);
+  lib.pt_observe(what, 0, M, N, K);
+}
+
 struct GroupedLinearNode : HipNode {
   Tensor weight;  // its gradient is written to; its values are not read
   Saved operand, operand_scale, ends, input_t, input_ts;
@@ -1002,11 +1016,7 @@ struct GroupedLinearNode : HipNode {
     Quantised d(go, stream);
     Tensor gx = empty({M, K}, go.scalar_type(), go.device());
     const auto o = (const int32_t*)ptr(offs);
-    const char* what = forward_layout ? "pt_gemm_m_grouped_nn" : "pt_gemm_m_grouped_nt";
-    lib.pt_observe(what, 1, M, K, N);
-    check(lib.pt_gemm_m_grouped_by_block(ptr(d.q), (const float*)ptr(d.s), ptr(dg), (const float*)ptr(dg_s), forward_layout, ptr(gx),
-                                         dtype_code(gx.scalar_type()), o, (int32_t)G, M, K, N, nullptr, 0, stream), what);
-    lib.pt_observe(what, 0, M, K, N);
+    m_grouped_by_block(d.q, d.s, dg, dg_s, forward_layout, gx, offs, std::nullopt, (int64_t)stream);
     {
       py::gil_scoped_acquire gil;
       if (deferred_gradients()) {
@@ -1453,6 +1463,7 @@ PYBIND11_MODULE(_host, m) {
   launch("permute_into_buffer", &permute_into_buffer);
   launch("permute_rows", &permute_rows);
   launch("silu_mul", &silu_mul);
+  launch("m_grouped_by_block", &m_grouped_by_block);
   launch("grouped_linear", &grouped_linear);
   launch("experts", &experts);
   launch("combine", &combine);

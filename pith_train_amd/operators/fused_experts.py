@@ -176,7 +176,8 @@ def _node(x, w_gate, w_up, w_down, grouped_mm_offs, q_gate_up, q_down, row_map, 
     ``[T, k, K]`` view of one row per token (routed row i is token i // k).  The weight gradients go to
     ``.grad``, or to the ``WeightGradStore`` queue."""
     row_map, expand_idx, scatter = _prepare(x, grouped_mm_offs, row_map, expand_idx, scatter)
-    _check_biases(x, w_down, biases)
+    if biases != (None, None):
+        _check_biases(x, w_down, biases)
     M = x.shape[0] if row_map is None else row_map.shape[0]
     weights = w_gate if w_up is None else (w_gate, w_up)
     return _lib.host().experts(
