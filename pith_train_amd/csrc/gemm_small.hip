@@ -179,27 +179,50 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
   for (int it = 0; it < nk; ++it) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kWait) : "memory");
     __syncthreads();  // stage `it` is complete, and every wave has read the stage whose slot is refilled next
-    issue_stage(it + NS - 1);
     const uint8_t* sA = lds + (it % NS) * STAGE;
     const uint8_t* sB = sA + BM * BK;
     const float* sc = (const float*)(lds + NS * STAGE) + (it % NS) * (BM + BN);
-    int sca[TM], scb[TN];
+    uint32_t sca[TM], scb[TN];
+    v8i fa[2][TM], fb[2][TN];
+    auto read_scales = [&]() {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) sca[i] = (int)(__float_as_uint(sc[wm0 + 32 * i + (lane & 31)]) >> 23);
+      for (int i = 0; i < TM; ++i) sca[i] = __float_as_uint(sc[wm0 + 32 * i + (lane & 31)]);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) scb[j] = (int)(__float_as_uint(sc[BM + wn0 + 32 * j + (lane & 31)]) >> 23);
+      for (int j = 0; j < TN; ++j) scb[j] = __float_as_uint(sc[BM + wn0 + 32 * j + (lane & 31)]);
+    };
+    auto read = [&](int ks) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      v8i fa[TM], fb[TN];
+      for (int j = 0; j < TN; ++j) fb[ks][j] = read_b(sB, j, ks);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) fb[j] = read_b(sB, j, ks);
-#pragma unroll
-      for (int i = 0; i < TM; ++i) fa[i] = read_frag(sA + (wm0 + 32 * i) * BK, ks);
+      for (int i = 0; i < TM; ++i) fa[ks][i] = read_frag(sA + (wm0 + 32 * i) * BK, ks);
+    };
+    auto multiply = [&](int ks) {
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int i = 0; i < TM; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[j], fa[i], acc[i][j], 0, 0, 0, scb[j], 0, sca[i]);
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[ks][j], fa[ks][i], acc[i][j], 0, 0, 0, (int)(scb[j] >> 23), 0, (int)(sca[i] >> 23));
+    };
+    // Dense products run few steps a workgroup from operands that lie in the L2, so a step is as long as its chain
+    // of barrier, reads and MFMAs: the reads go ahead of the next stage's loads, which have two steps to arrive (the
+    // gradients of an MLA block's latent projection as a pair, 2048 rows, 512 to 1024 wide: 12.9 -> 12.1 us; its
+    // forward product 6.5 -> 6.3).  Weights that come from HBM want their loads out first (few-row groups 74.7 us,
+    // 75.2 with the reads ahead; reduction-major 64 x 60 rows of 2048 x 2816: 90.0, 92.9).
+    if constexpr (MODE == GEMM_DENSE) {
+      read_scales();
+      read(0);
+      read(1);
+      __builtin_amdgcn_sched_barrier(0);
+      issue_stage(it + NS - 1);
+      multiply(0);
+      multiply(1);
+    } else {
+      issue_stage(it + NS - 1);
+      read_scales();
+      read(0);
+      multiply(0);
+      read(1);
+      multiply(1);
     }
   }
   wait_all_vmem();  // nothing may still be writing into this workgroup's LDS when it retires
