@@ -34,8 +34,8 @@
 #include <type_traits>
 
 // Measurement builds only (never defined by the Makefile's default target): parts of the main loop
-// compiled out to see what the rest costs.  PT_GEMM_ABLATE_MFMA: no MFMAs (the fragment reads go
-// with them, nothing consumes their results).  PT_GEMM_ABLATE_LOADS: 1 = every operand and scale
+// compiled out to see what the rest costs.  PT_GEMM_ABLATE_MFMA: no MFMAs, fragment reads or result
+// stores (every wave takes the path of one without rows).  PT_GEMM_ABLATE_LOADS: 1 = every operand and scale
 // load is issued out of range (the instruction runs, nothing is fetched), 2 = not issued at all.
 // The results of such builds are garbage; only their timing means something.
 #ifndef PT_GEMM_ABLATE_MFMA
