@@ -33,6 +33,7 @@
 namespace pt {
 
 static constexpr int kMaxTopK = 16;
+static constexpr int kCombineThreads = 384;  // most threads of a workgroup
 
 struct CombineArgs {
   const char *moe, *res, *go;
@@ -44,14 +45,16 @@ struct CombineArgs {
   int64_t ld_moe, ld_res, ld_out, ld_go, ld_dmoe;  // bytes
   int32_t k;
   uint32_t H, chunks;  // chunks of 8 elements per row
+  uint32_t threads;    // of a workgroup (launch_combine)
   int vec;
 };
 
 // Expert-parallel forward: sequential S-rounded accumulation over the token's rows in ascending
 // row order.  The first k threads rank the token's rows; everyone then walks the ranked list.
-template <typename S>
-__global__ __launch_bounds__(256) void moe_combine_ep_fwd_kernel(CombineArgs p) {
+template <typename S, bool FEW>
+__global__ __launch_bounds__(FEW ? kCombineThreads : 256) void moe_combine_ep_fwd_kernel(CombineArgs p) {
 #pragma clang fp contract(off)
+  constexpr int U = FEW ? 4 : 8;
   __shared__ int32_t s_row[kMaxTopK];
   __shared__ float s_w[kMaxTopK];
   __shared__ int s_n;
@@ -73,7 +76,7 @@ __global__ __launch_bounds__(256) void moe_combine_ep_fwd_kernel(CombineArgs p) 
   }
   __syncthreads();
   const int n = s_n;
-  for (uint32_t c = threadIdx.x; c < p.chunks; c += 256) {
+  for (uint32_t c = threadIdx.x; c < p.chunks; c += FEW ? p.threads : 256) {
     const uint32_t col = c * 8u;
     const int nval = (p.H - col) < 8u ? (int)(p.H - col) : 8;
     const int64_t cb = (int64_t)col * S::kBytes;
@@ -81,15 +84,15 @@ __global__ __launch_bounds__(256) void moe_combine_ep_fwd_kernel(CombineArgs p) 
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;
     if (p.vec) {
-      // Up to eight rows are requested together (a row past the list reads the first one again and
+      // Up to U rows are requested together (a row past the list reads the first one again and
       // is not used); the accumulation walks them in list order as before.
-      for (int j0 = 0; j0 < n; j0 += 8) {
-        float m[8][8];
+      for (int j0 = 0; j0 < n; j0 += U) {
+        float m[U][8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+        for (int u = 0; u < U; ++u)
           load8_policy<S, (PT_COMBINE_NT & 1) != 0>(p.moe + (int64_t)s_row[j0 + u < n ? j0 + u : j0] * p.ld_moe + cb, m[u]);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < U; ++u) {
           const bool ok = j0 + u < n;
           const float wj = s_w[ok ? j0 + u : j0];
 #pragma unroll
@@ -134,14 +137,15 @@ __global__ __launch_bounds__(256) void combine_slot_index_kernel(const int64_t* 
   if (s >= 0 && s < slots) slot_row[s] = (int32_t)r;  // an index outside the slots is dropped, never followed
 }
 
-template <typename S>
-__global__ __launch_bounds__(256) void moe_combine_fwd_kernel(CombineArgs p) {
+template <typename S, bool FEW>
+__global__ __launch_bounds__(FEW ? kCombineThreads : 256) void moe_combine_fwd_kernel(CombineArgs p) {
   // The product is rounded before it is added (the reference materialises the product tensor): a
   // fused multiply-add would differ in the last bit often enough to move the rounding of the sum.
 #pragma clang fp contract(off)
+  constexpr int U = FEW ? 4 : 8;
   const int64_t t = blockIdx.x;
   const float* w = p.w + t * p.k;
-  for (uint32_t c = threadIdx.x; c < p.chunks; c += 256) {
+  for (uint32_t c = threadIdx.x; c < p.chunks; c += FEW ? p.threads : 256) {
     const uint32_t col = c * 8u;
     const int nval = (p.H - col) < 8u ? (int)(p.H - col) : 8;
     const int64_t cb = (int64_t)col * S::kBytes;
@@ -149,14 +153,14 @@ __global__ __launch_bounds__(256) void moe_combine_fwd_kernel(CombineArgs p) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;
     if (p.vec) {
-      // up to eight rows requested together; the sum still runs over j = 0, 1, ... in order
-      for (int j0 = 0; j0 < p.k; j0 += 8) {
-        float m[8][8];
+      // up to U rows requested together; the sum still runs over j = 0, 1, ... in order
+      for (int j0 = 0; j0 < p.k; j0 += U) {
+        float m[U][8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+        for (int u = 0; u < U; ++u)
           load8_policy<S, (PT_COMBINE_NT & 1) != 0>(p.moe + (t * p.k + (j0 + u < p.k ? j0 + u : j0)) * p.ld_moe + cb, m[u]);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < U; ++u) {
           const bool ok = j0 + u < p.k;
           const float wj = w[ok ? j0 + u : j0];
 #pragma unroll
@@ -193,16 +197,17 @@ __global__ __launch_bounds__(256) void moe_combine_fwd_kernel(CombineArgs p) {
   }
 }
 
-template <typename S>
-__global__ __launch_bounds__(256) void moe_combine_bwd_kernel(CombineArgs p) {
-  __shared__ float s_part[4][kMaxTopK];
+template <typename S, bool FEW>
+__global__ __launch_bounds__(FEW ? kCombineThreads : 256) void moe_combine_bwd_kernel(CombineArgs p) {
+  constexpr int U = FEW ? 4 : 8, SLOTS = FEW ? 4 : kMaxTopK;
+  __shared__ float s_part[FEW ? kCombineThreads / 64 : 4][SLOTS];
   const int64_t t = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float* w = p.w + t * p.k;
-  float part[kMaxTopK];
+  float part[SLOTS];
 #pragma unroll
-  for (int j = 0; j < kMaxTopK; ++j) part[j] = 0.f;
-  for (uint32_t c = threadIdx.x; c < p.chunks; c += 256) {
+  for (int j = 0; j < SLOTS; ++j) part[j] = 0.f;
+  for (uint32_t c = threadIdx.x; c < p.chunks; c += FEW ? p.threads : 256) {
     const uint32_t col = c * 8u;
     const int nval = (p.H - col) < 8u ? (int)(p.H - col) : 8;
     const int64_t cb = (int64_t)col * S::kBytes;
@@ -214,15 +219,15 @@ __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(CombineArgs p) {
       for (int i = 0; i < 8; ++i) g[i] = i < nval ? S::load1(gp + i * S::kBytes) : 0.f;
     }
     if (p.vec) {
-      // The rows of eight slots are requested together (a slot without a row reads the gradient
+      // The rows of U slots are requested together (a slot without a row reads the gradient
       // chunk again, memory that certainly exists, and neither stores nor accumulates).
 #pragma unroll
-      for (int j0 = 0; j0 < kMaxTopK; j0 += 8) {
+      for (int j0 = 0; j0 < SLOTS; j0 += U) {
         if (j0 < p.k) {
-          int64_t row[8];
-          float m[8][8];
+          int64_t row[U];
+          float m[U][8];
 #pragma unroll
-          for (int u = 0; u < 8; ++u) {
+          for (int u = 0; u < U; ++u) {
             const int j = j0 + u;
             int64_t r = -1;
             if (j < p.k) r = p.slot_row ? (int64_t)p.slot_row[t * p.k + j] : t * p.k + j;
@@ -230,10 +235,10 @@ __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(CombineArgs p) {
             row[u] = r;
           }
 #pragma unroll
-          for (int u = 0; u < 8; ++u)
+          for (int u = 0; u < U; ++u)
             load8_policy<S, (PT_COMBINE_NT & 1) != 0>(row[u] >= 0 ? p.moe + row[u] * p.ld_moe + cb : gp, m[u]);
 #pragma unroll
-          for (int u = 0; u < 8; ++u) {
+          for (int u = 0; u < U; ++u) {
             const bool ok = row[u] >= 0;
             const float wj = w[j0 + u < p.k ? j0 + u : 0];
             float d[8];
@@ -250,7 +255,7 @@ __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(CombineArgs p) {
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < kMaxTopK; ++j) {
+      for (int j = 0; j < SLOTS; ++j) {
         if (j < p.k) {
           const int64_t row = p.slot_row ? (int64_t)p.slot_row[t * p.k + j] : t * p.k + j;
           if (row < 0 || (p.slot_row && row >= p.rows)) continue;  // slot without a row: its weight gradient stays zero
@@ -269,9 +274,9 @@ __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(CombineArgs p) {
       }
     }
   }
-  // fixed-order reduction: lanes of a wave (xor butterfly), then the four waves in order
+  // fixed-order reduction: lanes of a wave (xor butterfly), then the waves in order
 #pragma unroll
-  for (int j = 0; j < kMaxTopK; ++j) {
+  for (int j = 0; j < SLOTS; ++j) {
     if (j < p.k) {
       float v = part[j];
 #pragma unroll
@@ -280,22 +285,42 @@ __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(CombineArgs p) {
     }
   }
   __syncthreads();
-  if ((int)threadIdx.x < p.k)
-    p.dw[t * p.k + threadIdx.x] = ((s_part[0][threadIdx.x] + s_part[1][threadIdx.x]) + s_part[2][threadIdx.x]) + s_part[3][threadIdx.x];
+  if ((int)threadIdx.x < p.k) {
+    const int waves = FEW ? (int)p.threads >> 6 : 4;
+    float v = s_part[0][threadIdx.x];
+    for (int i = 1; i < (waves < 4 ? waves : 4); ++i) v += s_part[i][threadIdx.x];
+    if (FEW && waves > 4) v += waves > 5 ? s_part[4][threadIdx.x] + s_part[5][threadIdx.x] : s_part[4][threadIdx.x];
+    p.dw[t * p.k + threadIdx.x] = v;
+  }
 }
 
 static bool al16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
+// FEW: up to four slots, whose rows are requested together (a slot past k reads another row again: of eight
+// requests two or four were of use), by a workgroup of no more waves than the row has work for.  Us before / now,
+// backward and forward (residual included): 16384 tokens of 4 x 2880 188 / 146 and 94 / 82, 8192 of 4 x 1024 45 / 28 and 19.6 /
+// 17.5, 4096 of 2 x 1536 21 / 14 and 13.1 / 10.1, 16384 of 2 x 256 48 / 13 and 13.5 / 8.6.  More slots take eight at a time
+// and 256 threads: a width that is read from the arguments costs the backward of 8192 tokens of 8 x 2048 2 %.
+template <typename S, bool BWD, bool FEW>
+static void launch_combine_typed(const CombineArgs& a, int64_t T, hipStream_t stream) {
+  if (BWD) hipLaunchKernelGGL((moe_combine_bwd_kernel<S, FEW>), dim3((unsigned)T), dim3(a.threads), 0, stream, a);
+  else if (a.slot_row) hipLaunchKernelGGL((moe_combine_ep_fwd_kernel<S, FEW>), dim3((unsigned)T), dim3(a.threads), 0, stream, a);
+  else hipLaunchKernelGGL((moe_combine_fwd_kernel<S, FEW>), dim3((unsigned)T), dim3(a.threads), 0, stream, a);
+}
 template <typename S, bool BWD>
-static void launch_combine_typed(CombineArgs& a, int64_t T, hipStream_t stream) {
-  if (BWD) hipLaunchKernelGGL(moe_combine_bwd_kernel<S>, dim3((unsigned)T), dim3(256), 0, stream, a);
-  else if (a.slot_row) hipLaunchKernelGGL(moe_combine_ep_fwd_kernel<S>, dim3((unsigned)T), dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL(moe_combine_fwd_kernel<S>, dim3((unsigned)T), dim3(256), 0, stream, a);
+static void launch_combine_typed(const CombineArgs& a, int64_t T, hipStream_t stream) {
+  if (a.k <= 4) launch_combine_typed<S, BWD, true>(a, T, stream);
+  else          launch_combine_typed<S, BWD, false>(a, T, stream);
 }
 
 template <bool BWD>
 static int launch_combine(CombineArgs& a, int64_t T, int dtype, hipStream_t stream) {
   PT_REQUIRE(T < (1ll << 31), "moe_combine: too many tokens");
+  // As few passes over a row as there can be, and all of them full: a row of 2880 is 360 chunks, one pass of 384 threads
+  // (256 did two, the second 0.4 full; two of 192 take 162 us where this takes 146), 4096 two passes of 256 (one of 512 is
+  // 8 % slower), 256 one of a single wave.
+  const uint32_t passes = a.chunks ? (a.chunks + kCombineThreads - 1) / kCombineThreads : 1;
+  a.threads = a.k > 4 ? 256 : a.chunks ? ((a.chunks + passes - 1) / passes + 63) / 64 * 64 : 64;
   switch (dtype) {
     case PT_BF16: launch_combine_typed<st_bf16, BWD>(a, T, stream); break;
     case PT_F16: launch_combine_typed<st_f16, BWD>(a, T, stream); break;

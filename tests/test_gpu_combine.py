@@ -118,3 +118,27 @@ def test_combine_ep_full_size_against_the_tensor_expression():
     mag = torch.zeros((T, H), device="cuda").index_add_(0, idx // k, weighted.float().abs())
     assert ((a.float() - ref).abs() <= mag * 2.0**-5 + ref.abs() * 2.0**-7 + 1e-6).all()
     assert (a.float() == ref).float().mean().item() > 0.8
+
+
+@pytest.mark.parametrize("k,H", [(4, 8), (4, 512), (3, 520), (4, 2048), (2, 2056), (4, 2560), (4, 2880), (4, 3072), (1, 3080), (4, 6152), (4, 515), (5, 3080)])
+def test_combine_at_the_edges_of_its_workgroup(k, H):
+    """The width of a workgroup follows the row (one wave up to 512 columns, six up to 3072, then two passes) and four
+    or eight slots are requested together: both branches against the oracle, odd widths included.  A weight gradient is a sum of
+    H rounded products in fp32, in any order within H 2^-24 of the sum of their sizes."""
+    from pith_train_amd.operators.moe_combine import moe_combine, moe_combine_ep
+
+    T = 21
+    moe, idx, w, res, go = _ep_inputs(T, k, H, k + H, rows=T * k - 2)
+    full = torch.randn((T * k, H), generator=torch.Generator().manual_seed(H)).bfloat16()
+    bound = H * 2.0**-24 * (go.float().abs().repeat_interleave(k, 0) * full.float().abs()).sum(-1).view(T, k) + 1e-30
+    for ep in (False, True):
+        m, ww, r = (t.cuda().requires_grad_(True) for t in (moe if ep else full, w, res))
+        out = moe_combine_ep(m, idx.cuda(), ww, r) if ep else moe_combine(m, ww, r)
+        out.backward(go.cuda())
+        ref = C.combine_ep_fwd(moe, idx, w, res) if ep else C.combine_fwd(full, w, res)
+        d_moe, d_w, _ = C.combine_ep_bwd(go, moe, idx, w) if ep else C.combine_bwd(go, full, w)
+        assert torch.equal(out.detach().cpu(), ref) and torch.equal(m.grad.cpu(), d_moe)
+        if ep:
+            torch.testing.assert_close(ww.grad.cpu(), d_w, rtol=1e-5, atol=1e-5 * H**0.5)
+        else:
+            assert ((ww.grad.cpu() - d_w).abs() <= 2 * bound).all()
