@@ -100,18 +100,19 @@ class Qwen3MoeExperts(nn.Module):
         return self._gu_cache, down._wq_cache
 
     def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, fuse_activation: bool = True,
-                expand_idx=None, few_rows: bool = False, checked: bool = False):
+                expand_idx=None, few_rows: bool = False):
         """``row_map`` (extension, FP8 layers only): the scatter's int32 source-row map.  ``x`` is
         then the un-permuted ``[m, H]`` token tensor and the result comes back un-permuted; the
         permutation happens inside the first quantisation and the last GEMM's store.
         ``expand_idx`` (one-node path only): ``x`` holds deduplicated rows, see
         :func:`fused_experts.compose_row_maps`.  One-node path with ``row_map`` only: ``x`` may be an expanded
         ``[T, k, H]`` view of the tokens, and ``few_rows`` says that the groups are multiples of 64 rows (no
-        backward may follow).  ``checked``: the caller has asked :meth:`one_node`.  With ``fuse_activation`` (FP8 layers, intermediate size a multiple of 128) the block runs as one
+        backward may follow).  With ``fuse_activation`` (FP8 layers, intermediate size a multiple of 128) the block runs as one
         autograd node on a fused gate_up operand: the tokens are quantised once instead of once
         per projection, one GEMM serves both, and the SwiGLU and its gradient are computed inside
-        the kernels that quantise them (same bits as the three-operator composition)."""
-        if fuse_activation and x.shape[0] > 0 and (checked or self.one_node(x)):
+        the kernels that quantise them (same bits as the three-operator composition).  Asked here and not by the
+        caller: a forward pre-hook may have changed ``x``."""
+        if fuse_activation and x.shape[0] > 0 and self.one_node(x):
             gate, up, down = map(_weight, self._projections())
             if not fused_experts.wants_backward(x, gate, up, down):
                 return fused_experts.forward_only(x, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
@@ -203,11 +204,11 @@ class Qwen35MoeExperts(nn.Module):
         return gu._get_quantized_weight(), down._get_quantized_weight()
 
     def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, fuse_activation: bool = True,
-                expand_idx=None, few_rows: bool = False, checked: bool = False):
-        """``row_map`` / ``expand_idx`` / ``checked``: see :meth:`Qwen3MoeExperts.forward`.  With ``fuse_activation`` (FP8 layers)
+                expand_idx=None, few_rows: bool = False):
+        """``row_map`` / ``expand_idx``: see :meth:`Qwen3MoeExperts.forward`.  With ``fuse_activation`` (FP8 layers)
         the block runs as one autograd node whose SwiGLU output and SwiGLU gradient are computed
         inside the kernels that quantise them (same bits as the three-operator composition)."""
-        if fuse_activation and x.shape[0] > 0 and (checked or self.one_node(x)):
+        if fuse_activation and x.shape[0] > 0 and self.one_node(x):
             gate_up, down = _weight(self._modules["gate_up_proj"]), _weight(self._modules["down_proj"])
             if not fused_experts.wants_backward(x, gate_up, down):
                 return fused_experts.forward_only(x, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
@@ -375,8 +376,7 @@ def forward_stage3(experts: nn.Module, gathered_tokens, expert_idxs, experts_per
                 host_sizes=host_sizes or not fused_node, need_reverse=False)
             # deduplicated rows: the first quantisation reads them through expand_idx composed with
             # the scatter's map, so neither the expanded nor the permuted copy exists
-            return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of, expand_idx=expand_idx, few_rows=few,
-                           checked=fused_node)
+            return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of, expand_idx=expand_idx, few_rows=few)
     if (fuse_permute and expand_idx is None and training.fp8 and expert_idxs.shape[0] > 0
             and isinstance(experts, GptOssExperts)):
         # the one-node block needs no host-side sizes (see the SwiGLU branch above)

@@ -82,3 +82,54 @@ assert state() == before, (before, state())
 """
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     subprocess.run([sys.executable, "-c", code], check=True, cwd=root)
+
+
+def _grouped(expert_idxs, num_groups, alignment=128, **_):
+    """The scatter's index half in torch: (reverse, ends, sizes on the host and the device, source row of every grouped row)."""
+    sizes = torch.bincount(expert_idxs, minlength=num_groups)
+    ks = (sizes + alignment - 1) // alignment * alignment
+    ends = ks.cumsum(0).int()
+    src_of = torch.full((-(-int(ks.sum()) // 128) * 128,), -1, dtype=torch.int32)
+    for e in range(num_groups):
+        rows = (expert_idxs == e).nonzero().flatten().int()
+        src_of[int(ends[e] - ks[e]) :][: len(rows)] = rows
+    return None, ends, ks.tolist(), ks.int(), src_of
+
+
+class _InTorch:
+    """A user's projection: an ``FP8GroupedLinear`` by type, with a forward of its own that takes any floating type."""
+
+    def forward(self, input, grouped_mm_offs, ks=None, ks_tensor=None, group_indices=None, in_rows=None, out_rows=None, out_m=None):
+        rows = input if in_rows is None else input[in_rows.long().clamp(min=0)]
+        group = torch.searchsorted(grouped_mm_offs, torch.arange(len(rows), dtype=torch.int32), right=True).clamp(max=self.num_groups - 1)
+        y = torch.einsum("mk,mnk->mn", rows, self.weight[group].to(rows.dtype))
+        if out_rows is None:
+            return y
+        kept = (out_rows >= 0) & (torch.arange(len(out_rows)) < grouped_mm_offs[-1])
+        return y.new_zeros((out_m, y.shape[1])).index_copy(0, out_rows[kept].long(), y[kept])
+
+
+@pytest.mark.parametrize("family", ["Qwen3MoeExperts", "Qwen35MoeExperts"])
+def test_a_hook_that_changes_the_rows_type_gets_the_composition(family, monkeypatch):
+    """A block decides by the rows that its forward receives.  Behind this pre-hook they are no bf16 rows any more, so the
+    separate projections, which may take them, run in the place of the one node."""
+    from pith_train_amd.modules import experts as X
+    from pith_train_amd.operators.grouped_linear import FP8GroupedLinear
+
+    monkeypatch.setattr(X, "group_rows_with_sizes", _grouped)
+    monkeypatch.setattr(X, "silu_mul", lambda g, u: F.silu(g) * u)
+    monkeypatch.setattr(X, "silu_mul_halves", lambda y: F.silu(y[:, : y.shape[1] // 2]) * y[:, y.shape[1] // 2 :])
+    torch.manual_seed(0)
+    m = getattr(X, family)(16, 128, 3).to(torch.bfloat16)
+    projection = type("Projection", (_InTorch, FP8GroupedLinear), {})
+    for child in m.children():
+        child.__class__ = projection
+        torch.nn.init.normal_(child.weight, std=0.1)
+    m.register_forward_pre_hook(lambda module, args: (args[0].float(), *args[1:]))
+    x, expert_idxs = torch.randn((300, 16)).bfloat16(), torch.randint(0, 3, (300,))
+    assert m.one_node(x)
+    out = X.forward_stage3(m, x, expert_idxs, 3)
+    w = [p.float() for p in m.parameters()]
+    gate, up = (w[0], w[1]) if len(w) == 3 else (w[0][:, :128], w[0][:, 128:])
+    want = torch.stack([w[-1][e] @ (F.silu(gate[e] @ t) * (up[e] @ t)) for e, t in zip(expert_idxs, x.float())])
+    torch.testing.assert_close(out, want)
