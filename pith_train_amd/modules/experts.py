@@ -355,6 +355,9 @@ def forward_stage3(experts: nn.Module, gathered_tokens, expert_idxs, experts_per
     (each unique row is read once per use and no expanded copy is materialised); without it the
     two steps run separately as in the reference.
 
+    The block gets a keyword of an extension only in the calls that need it, so a subclass whose ``forward`` lacks
+    ``expand_idx`` or ``few_rows`` runs wherever there is nothing to expand and a backward follows.
+
     ``gathered_tokens`` may also be an expanded ``[T, k, H]`` view of one row per token (stride 0 along k):
     the one-node blocks then read every token where it is, and its gradient comes back as ``[T, k, H]``.
     """
@@ -376,7 +379,8 @@ def forward_stage3(experts: nn.Module, gathered_tokens, expert_idxs, experts_per
                 host_sizes=host_sizes or not fused_node, need_reverse=False)
             # deduplicated rows: the first quantisation reads them through expand_idx composed with
             # the scatter's map, so neither the expanded nor the permuted copy exists
-            return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of, expand_idx=expand_idx, few_rows=few)
+            return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of,
+                           **({} if expand_idx is None else {"expand_idx": expand_idx}), **({"few_rows": True} if few else {}))
     if (fuse_permute and expand_idx is None and training.fp8 and expert_idxs.shape[0] > 0
             and isinstance(experts, GptOssExperts)):
         # the one-node block needs no host-side sizes (see the SwiGLU branch above)
@@ -389,7 +393,7 @@ def forward_stage3(experts: nn.Module, gathered_tokens, expert_idxs, experts_per
             # both sides: rows gathered by the first quantisation, stored un-permuted (bias added)
             # by the last GEMM; the bias gradients are summed through the same map
             return experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of, scatter_output=True,
-                           few_rows=few)
+                           **({"few_rows": True} if few else {}))
         # input side only: the unfused bias add wants the grouped layout
         outs = experts(gathered_tokens, grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, row_map=src_of)
         return padded_index_gather(outs, reverse_shuffle_idxs)

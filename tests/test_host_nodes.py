@@ -133,3 +133,27 @@ def test_a_hook_that_changes_the_rows_type_gets_the_composition(family, monkeypa
     gate, up = (w[0], w[1]) if len(w) == 3 else (w[0][:, :128], w[0][:, 128:])
     want = torch.stack([w[-1][e] @ (F.silu(gate[e] @ t) * (up[e] @ t)) for e, t in zip(expert_idxs, x.float())])
     torch.testing.assert_close(out, want)
+
+
+@pytest.mark.parametrize("family", ["Qwen3MoeExperts", "Qwen35MoeExperts", "GptOssExperts"])
+def test_stage3_passes_an_extension_s_keyword_only_where_it_is_needed(family, monkeypatch):
+    """A subclass whose forward has fewer of them trains; evaluation with few rows and deduplicated rows name theirs."""
+    from pith_train_amd.modules import experts as X
+
+    seen = []
+
+    def forward(self, x, grouped_mm_offs, ks=None, ks_tensor=None, row_map=None, **extra):
+        seen.append(extra)
+        return x
+
+    m = type("Narrow", (getattr(X, family),), {"forward": forward})(16, 128, 3).to(torch.bfloat16)
+    monkeypatch.setattr(X, "group_rows_with_sizes", _grouped)
+    x, expert_idxs = torch.randn((30, 16)).bfloat16(), torch.randint(0, 3, (30,))
+    always = {"scatter_output": True} if family == "GptOssExperts" else {}
+    X.forward_stage3(m, x, expert_idxs, 3)
+    with torch.no_grad():
+        X.forward_stage3(m, x, expert_idxs, 3)
+    assert seen == [always, {**always, "few_rows": True}]
+    if not always:
+        X.forward_stage3(m, x, expert_idxs, 3, expand_idx=expert_idxs)
+        assert seen[2].keys() == {"expand_idx"}
