@@ -110,3 +110,30 @@ def test_mlp_as_one_node(rows, hidden, width):
             torch.testing.assert_close(a, b, rtol=0.01, atol=0.01 * b.float().abs().max().item())
     with torch.no_grad():
         assert torch.equal(mlp(x.view(1, rows, hidden))[0], got)
+
+
+@pytest.mark.parametrize("family", ["Qwen3MoeExperts", "Qwen35MoeExperts", "GptOssExperts"])
+def test_few_rows_whose_forward_turns_out_to_want_a_gradient(family):
+    """Frozen experts on a few rows are handed groups of 64; behind a pre-hook that makes its rows require a gradient the
+    forward keeps what the backward reads, in whole blocks of 128."""
+    from pith_train_amd.modules import experts as X
+
+    torch.manual_seed(5)
+    m = getattr(X, family)(256, 128, 8).cuda().to(torch.bfloat16).requires_grad_(False)
+    for p in m.parameters():
+        p.normal_(0.0, 0.05)
+    received = []
+
+    def attach(module, args):
+        received.append(args[0].detach().requires_grad_(True))
+        return (received[-1], *args[1:])
+
+    m.register_forward_pre_hook(attach)
+    x = torch.randn((300, 256), device="cuda").bfloat16()
+    idx, up = torch.randint(0, 7, (300,), device="cuda"), torch.randn((300, 256), device="cuda").bfloat16()
+    out = X.forward_stage3(m, x, idx, 8)
+    (grad,) = torch.autograd.grad(out, received[-1], up)
+    m._forward_pre_hooks.clear()
+    x.requires_grad_(True)
+    want = X.forward_stage3(m, x, idx, 8)
+    assert torch.equal(out, want) and torch.equal(grad, torch.autograd.grad(want, x, up)[0])

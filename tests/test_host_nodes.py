@@ -157,3 +157,16 @@ def test_stage3_passes_an_extension_s_keyword_only_where_it_is_needed(family, mo
     if not always:
         X.forward_stage3(m, x, expert_idxs, 3, expand_idx=expert_idxs)
         assert seen[2].keys() == {"expand_idx"}
+
+
+def test_groups_of_64_rows_spread_to_whole_blocks():
+    """Every group starts at the end of the last one, padded to 128 rows, and has the same rows in the same order."""
+    from pith_train_amd.modules.experts import _whole_blocks
+
+    expert_idxs = torch.cat([torch.full((n,), e) for e, n in enumerate((1, 0, 64, 65, 128, 0, 200, 3))])
+    expert_idxs = expert_idxs[torch.randperm(len(expert_idxs), generator=torch.Generator().manual_seed(0))]
+    _, ends, _, _, few = _grouped(expert_idxs, 8, 64)
+    _, want_ends, _, _, want = _grouped(expert_idxs, 8)
+    got, got_ends = _whole_blocks(torch.cat([few, few.new_full((256,), -1)]), ends)  # longer than the grouped rows
+    assert got_ends.dtype == torch.int32 and torch.equal(got_ends, want_ends) and len(got) % 128 == 0
+    assert torch.equal(got[: len(want)], want) and (got[len(want) :] == -1).all()
