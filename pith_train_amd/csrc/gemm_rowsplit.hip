@@ -283,11 +283,9 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
   // the two cursors (loader, MFMAs) fetch a tile with a few LDS reads; nothing in flight between two pieces ----
   for (bool first_piece = true; t_next < t_end; first_piece = false, t_next += kRsTiles * t_step) {
     const GemmArgs p = reload_args();
-    if (!first_piece) {
+    if (!first_piece) {  // the scan of the groups and the schedule have their own LDS and are still there
       wait_all_vmem();
       __syncthreads();
-      if (MODE == GEMM_M_GROUPED) scan_group_tiles<BM>(p, s_pref, tid, lane);
-      if (MODE == GEMM_K_GROUPED) scan_group_costs(p, s_pref, tid, lane);
     }
     n_tiles = (t_end - t_next + t_step - 1) / t_step;
     if (n_tiles > kRsTiles) n_tiles = kRsTiles;

@@ -573,8 +573,8 @@ def test_grouped_tile_order_at_the_edges_of_its_strips(gemm_kernel, tiles):
 
 
 def test_grouped_work_lists_longer_than_the_tile_table(gemm_kernel):
-    """12800 large tiles, 50 for every workgroup, so that the table is filled a second time and the groups
-    are scanned again: the bits of the kernel that takes one small tile per workgroup.  m-grouped, then
+    """12800 large tiles, 50 for every workgroup, so that the table is filled a second time from the scan that the
+    first one was made of: the bits of the kernel that takes one small tile per workgroup.  m-grouped, then
     k-grouped with empty groups among them."""
     from pith_train_amd import _lib
 
@@ -618,3 +618,45 @@ def test_grouped_work_lists_longer_than_the_tile_table(gemm_kernel):
         return o
 
     both(k_grouped)
+
+
+@pytest.mark.parametrize("groups,half,W", [(40, 640, 1800), (256, 896, 2200)])
+def test_k_grouped_schedule_with_two_outputs_and_a_second_table(gemm_kernel, groups, half, W):
+    """The rows of a gate and of an up projection go to two gradients, whose border lies inside a row of tiles, under the
+    schedule of skewed groups; with 256 groups the workgroups that get small tiles alone take more than the 48 that
+    the tile table holds.  The bits of one small tile per workgroup into one output."""
+    from pith_train_amd import _lib
+
+    if gemm_kernel != "auto":
+        pytest.skip("the test selects the kernels itself; run once")
+    g = torch.Generator(device="cuda").manual_seed(groups)
+    N = 2 * half
+    tiles = -(-N // 256) * -(-W // 256)
+    blocks = torch.randint(0, 2, (groups,), generator=torch.Generator().manual_seed(groups))
+    blocks[groups // 3] = 60 if groups == 256 else int(1.3 * 96 * 256 / tiles)
+    cost = blocks + 3
+    share = cost.sum().item() * tiles / 256
+    assert share >= 96 and cost.max() * 4 >= share  # what the rule asks for
+    assert groups != 256 or share / 4 > 52  # small tiles cost 3 or 4: a workgroup without a big one
+    offs, M = torch.cumsum(blocks * 128, 0).int().cuda(), int(blocks.sum()) * 128
+
+    def fp8(*shape):
+        return torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # finite values below 2
+
+    def scale(*shape):
+        return torch.exp2(torch.randint(-6, 3, shape, device="cuda", generator=g).float())
+
+    d, sd, x, sx = fp8(N, M), scale(M // 128, N), fp8(W, M), scale(M // 128, W)
+    start = torch.randn((groups, N, W), device="cuda", generator=g).bfloat16()
+    operands = _lib.ptr(d), _lib.ptr(sd), _lib.ptr(x), _lib.ptr(sx)
+    for add in (0, 1):
+        _lib.call("pt_gemm_select_kernel", b"s128")
+        want = start.clone()
+        rest = _lib.dtype_code(want.dtype), add, _lib.ptr(offs), groups, M, N, W, _lib.stream_ptr()
+        _lib.call("pt_gemm_k_grouped_wgrad", *operands, _lib.ptr(want), *rest)
+        _lib.call("pt_gemm_select_kernel", b"r0")
+        one, gate, up = start.clone(), start[:, :half].contiguous(), start[:, half:].contiguous()
+        _lib.call("pt_gemm_k_grouped_wgrad", *operands, _lib.ptr(one), *rest)
+        _lib.call("pt_gemm_k_grouped_wgrad_pair", *operands, _lib.ptr(gate), _lib.ptr(up), half, *rest)
+        assert torch.equal(one, want)
+        assert torch.equal(gate, want[:, :half]) and torch.equal(up, want[:, half:])
