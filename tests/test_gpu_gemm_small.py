@@ -131,3 +131,42 @@ def test_groups_of_a_few_rows(rows, n, k, scatter, bias):
                 want[row : row + r] = y
         row += r
     assert row == M and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("G,n,k", [(66, 1000, 2048), (70, 15000, 128), (64, 1024, 2048), (9, 7304, 2048)])
+@pytest.mark.parametrize("scatter,bias", [(False, False), (True, True)])
+def test_groups_of_a_few_rows_whose_weights_are_streamed(G, n, k, scatter, bias):
+    """Weights of 128 MiB and a little more, the least that is read past the memory-side cache: a last column tile that is
+    not full (8 wide the last time), a reduction of one block, exactly 128 MiB."""
+    from pith_train_amd import _lib
+
+    assert 2**27 <= G * n * k < 2**27 * 1.01 and k % 128 == 0
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+
+    def fp8(*shape):
+        return torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # finite values below 2
+
+    def scale(*shape):
+        return torch.exp2(torch.randint(-8, 2, shape, device="cuda", generator=g).float())
+
+    rows = torch.tensor([64, 0, 192, 128, 64, 64, 0], dtype=torch.int32).repeat(G)[:G]
+    offs, M, cap = rows.cumsum(0).int().cuda(), int(rows.sum()), int(rows.sum()) + 128
+    a, sa, b, sb = fp8(cap, k), scale(cap, k // 128), fp8(G, n, k), scale(G, _cdiv(n, 128), k // 128)
+    bias_rows = torch.randn((G, n), device="cuda", generator=g).bfloat16() if bias else None
+    index = torch.randperm(cap, device="cuda", generator=g).int() if scatter else None
+    out = torch.zeros((cap, n), device="cuda", dtype=torch.bfloat16)
+    args = [_lib.PT_BF16, offs.data_ptr(), G, cap, n, k, _lib.ptr(index), cap, _lib.ptr(bias_rows), _lib.stream_ptr()]
+    _lib.call("pt_gemm_m_grouped_nt_few_rows", a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), out.data_ptr(), *args)
+    want, row = torch.zeros_like(out), 0
+    for q, r in enumerate(rows.tolist()):
+        if r:
+            y = torch.empty((r, n), device="cuda", dtype=torch.bfloat16)
+            _lib.call("pt_gemm_nt_dense", a[row:].data_ptr(), sa[row:].data_ptr(), b[q].data_ptr(), sb[q].data_ptr(), y.data_ptr(),
+                      _lib.PT_BF16, r, n, k, _lib.stream_ptr())
+            y = y + bias_rows[q] if bias else y
+            if scatter:
+                want[index[row : row + r].long()] = y
+            else:
+                want[row : row + r] = y
+        row += r
+    assert row == M and torch.equal(out, want)
