@@ -579,3 +579,76 @@ def test_stage3_with_and_without_the_transposed_weight_twin_agree_bit_for_bit(ki
 
     a, b = run(True), run(False)
     assert len(a) == len(b) and all(torch.equal(u, v) for u, v in zip(a, b))
+
+
+@pytest.mark.parametrize("form", ["rows", "expanded", "clamped", "few_rows"])
+def test_steps_with_row_scales_by_row_and_by_block_agree_bit_for_bit(form):
+    """``pt_experts_forward`` / ``_backward`` keep the scales of their row-scaled operands as [M, K/128], the ``_by_block`` forms
+    that the blocks call as [K/128, M]: the same scales in the other order, and the bits of everything else.  Grouped rows in
+    place; deduplicated and scattered ones; the clamped activation with biases; groups of 64 rows without a backward."""
+    import struct
+
+    from pith_train_amd import _lib
+    from pith_train_amd.operators.token_scatter import group_rows_with_sizes
+
+    G_, K, half, H, routed = 4, 272, 144, 272, 500
+    g = torch.Generator(device="cuda").manual_seed(1)
+    clamped, few, mapped = form == "clamped", form == "few_rows", form != "rows"
+    idx = torch.tensor([0, 2, 2, 3, 2], device="cuda").repeat(routed // 5)[torch.randperm(routed, device="cuda", generator=g)]
+    _, offs, _, _, row_map = group_rows_with_sizes(idx, G_, 64 if few else 128, device=idx.device, host_sizes=False, need_reverse=False)
+    M = row_map.shape[0] if mapped else 1024
+    if not mapped:
+        offs = torch.tensor([128, 128, 896, 1024], dtype=torch.int32, device="cuda")
+    repeat, expand = 5 if few else 1, None
+    if form == "expanded":
+        expand = torch.randint(0, 300, (routed,), device="cuda", generator=g)
+
+    def normal(*shape, std=1.0):
+        return (torch.randn(shape, device="cuda", generator=g) * std).bfloat16()
+
+    def fp8(*shape):
+        return torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # finite values below 2
+
+    def scale(*shape):
+        return torch.exp2(torch.randint(-6, -3, shape, device="cuda", generator=g).float())
+
+    out_rows = routed if mapped else M
+    x, grad = normal(M if not mapped else 300 if form == "expanded" else routed // repeat, K), normal(out_rows, H)
+    gu, gu_s, dn, dn_s = fp8(G_, 2 * half, K), scale(G_, 3, 3), fp8(G_, H, half), scale(G_, 3, 2)
+    gu_b, dn_b = (normal(G_, 2 * half), normal(G_, H)) if clamped else (None, None)
+    at = lambda t: t.data_ptr() if t is not None else 0  # noqa: E731
+
+    def step(by_block):
+        """Every buffer of a step by name (all start as zeros: rows behind the last group are not written)."""
+        byte = lambda *s: torch.zeros(s, dtype=torch.uint8, device="cuda")  # noqa: E731
+        real = lambda *s, dtype=torch.float32: torch.zeros(s, dtype=dtype, device="cuda")  # noqa: E731
+        scales = (lambda w: real(-(-w // 128), M)) if by_block else (lambda w: real(M, -(-w // 128)))
+        b = dict(gate_up=real(M, 2 * half, dtype=torch.bfloat16), out=real(out_rows, H, dtype=torch.bfloat16), x_fp8=byte(M, K), h_fp8=byte(M, half),
+                 x_scale=scales(K), h_scale=scales(half), map=torch.zeros(M, dtype=torch.int32, device="cuda"))
+        kept = dict(x_t=byte(K, M), x_ts=real(M // 128, K), h_t=byte(half, M), h_ts=real(M // 128, half))
+        if not few:
+            b.update(kept)
+        saved = [at(b.get(n)) for n in ("x_t", "x_ts", "h_t", "h_ts")]
+        limits = 1.702, 7.0
+        name = "_by_block" if by_block else ""
+        stream = _lib.stream_ptr()
+        _lib.call("pt_experts_forward" + name, struct.pack(
+            "=25q2d10q", at(x), x.shape[0], K, M, K, half, H, G_, at(offs), at(row_map) if mapped else 0, at(expand), routed if expand is not None else 0,
+            repeat, few, at(gu), at(gu_s), at(gu_b), at(dn), at(dn_s), at(dn_b), at(b["gate_up"]), at(b["out"]), out_rows, mapped, clamped, *limits, *saved,
+            *(at(b[n]) for n in ("map", "x_fp8", "x_scale", "h_fp8", "h_scale")), stream))
+        if few:
+            return b
+        b.update(dgu_fp8=byte(M, 2 * half), dgu_scale=scales(2 * half), dy_fp8=byte(M, H), dy_scale=scales(H), dy_t=byte(H, M), dy_ts=real(M // 128, H),
+                 dgu_t=byte(2 * half, M), dgu_ts=real(M // 128, 2 * half), grad_h=real(M, half, dtype=torch.bfloat16), sums=real(M // 128, 2 * half),
+                 dw=real(G_, H, half, dtype=torch.bfloat16), d_gu=real(G_, 2 * half), d_dn=real(G_, H))
+        _lib.call("pt_experts_backward" + name, struct.pack(
+            "=35q2d5q", at(grad), out_rows, M, K, half, H, G_, at(offs), at(row_map) if mapped else 0, mapped, at(dn), at(dn_s), 1, at(b["gate_up"]), *saved,
+            *(at(b[n]) for n in ("dgu_fp8", "dgu_scale", "dy_t", "dy_ts", "dgu_t", "dgu_ts", "dy_fp8", "dy_scale", "grad_h", "sums")), at(b["dw"]), 0, 0, 0, 0, 0,
+            clamped, *limits, at(b["d_gu"]) if clamped else 0, _lib.PT_F32, at(b["d_dn"]) if clamped else 0, _lib.PT_F32, stream))
+        return b
+
+    rows, blocks = step(False), step(True)
+    for name, want in rows.items():
+        got = blocks[name].t() if name.endswith("_scale") else blocks[name]
+        assert want.float().abs().sum() > 0 or name == "map" or (not clamped and name in ("sums", "d_gu", "d_dn")), name
+        assert torch.equal(want, got), name
