@@ -24,8 +24,7 @@ namespace pt {
 template <int BM> static constexpr int kSmallStages = BM == 64 ? 3 : 2;
 template <int BM> static constexpr size_t kSmallLds = (size_t)kSmallStages<BM> * (BM + 128) * (128 + 4) + 256;
 
-// STREAM: b is read once and is more than the memory-side cache holds, so its loads pass it by (evaluation, 21 rows
-// an expert, 128 experts of 1536 x 2048: 82 us -> 75.5; 2048 x 768: 48.4 -> 45.0).
+// STREAM: the loads of b pass the memory-side cache by (launch_small_mode has the rule and both sides).
 template <int MODE, int BM, bool ACC, bool BT, bool STREAM = false>
 __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
   constexpr int BN = 128, BK = 128, NS = kSmallStages<BM>;
@@ -298,9 +297,15 @@ static int launch_small_mode(const GemmArgs& a, hipStream_t stream) {
   switch (a.mode) {
     case GEMM_DENSE: return launch_small<GEMM_DENSE, BM, false, false>(a, stream);
     case GEMM_M_GROUPED:
-      // Groups of up to 64 rows read their weights once; whether the next reader finds them in the 256 MiB
-      // memory-side cache is decided by their size, and a row that is no whole 128-byte lines shares one with the
-      // next (32 experts of 5760 x 2880: 127 us, 132 past the cache).
+      // Groups of up to 64 rows read their weights once.  Past the memory-side cache (256 MiB) they arrive faster, whatever
+      // their size, when the weights of other layers are read before they are wanted again, as in a model (1536 x 2048 an
+      // expert, us through the cache / past it: 96 MiB 25.7 / 23.8, 129 MiB 36.9 / 33.8, 192 40.9 / 37.9, 384 80.1 / 74.8).
+      // A block that runs alone finds what is left of its own last pass, while its two operands fit together (gate_up and
+      // a down of half its size in turn, us a product: 129 MiB of gate_up 22.6 / 25.2, 162 26.0 / 28.4, 192 31.8 / 29.9, 258
+      // 48.5 / 45.0), and a single product repeated (162 MiB 29.8 / 33.8, 225 39.5 / 46.2, 321 71.6 / 65.8).  A launch
+      // sees one operand and not what comes between: from half of the cache on it is taken for the first case, below for
+      // the others, so a block alone loses a tenth between 128 and 170 MiB and a model 5 to 8 % below 128.  A row that is
+      // no whole 128-byte lines shares one with the next (32 experts of 5760 x 2880: 127 us, 132 past the cache).
       if (BM == 64 && a.few_rows && a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0)
         return launch_small<GEMM_M_GROUPED, 64, false, false, true>(a, stream);
       return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true>(a, stream)
