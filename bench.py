@@ -34,7 +34,7 @@ HBM_PEAK_GBS = 8000.0
 # of known size).  FETCH_SIZE counts what the L2 asks of the fabric, whether the memory-side cache
 # or HBM answers: where successive waves of tiles re-read operand panels that the 4 MiB L2 of an
 # XCD cannot keep (GPT-OSS: 2.5x the algorithmic bytes) most of the excess is served by that cache.
-GEMM_TRAFFIC_BYTES_PER_LAUNCH = {"qwen3-30b-a3b-moe": 754e6, "dsv2-lite-moe": 637e6, "gpt-oss-20b-moe": 2889e6,
+GEMM_TRAFFIC_BYTES_PER_LAUNCH = {"qwen3-30b-a3b-moe": 754e6, "dsv2-lite-moe": 584e6, "gpt-oss-20b-moe": 2889e6,
                                  "qwen3-decoder-linears-32k": 912e6}
 
 WORKLOADS = {

@@ -187,3 +187,12 @@ def test_bench_times_every_gemm_entry_point_of_the_library():
     header = open(os.path.join(os.path.dirname(__file__), "..", "include", "pithtrain_hip.h")).read()
     declared = set(re.findall(r"\bint (pt_gemm_(?!select_kernel)\w+)\(", header))
     assert declared == set(bench.GemmTimer.NAMES), declared ^ set(bench.GemmTimer.NAMES)
+
+
+def test_bench_states_the_traffic_that_the_profiles_show():
+    import bench
+
+    for workload, stated in bench.GEMM_TRAFFIC_BYTES_PER_LAUNCH.items():
+        with open(os.path.join(ROOT, "profiles", f"hbm_traffic_gemm_{workload}.txt")) as f:
+            (measured,) = re.findall(r"launches of a step: (\d+) MB per launch", f.read())
+        assert stated == float(measured) * 1e6, workload
