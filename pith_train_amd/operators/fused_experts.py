@@ -105,9 +105,8 @@ def clamped_swiglu_bwd_quant(grad_h: torch.Tensor, gate_up: torch.Tensor, alpha:
 
 def supported(x: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor) -> bool:
     """bf16 activations, half width and hidden size multiples of 8 (16-byte accesses)."""
-    half = w_gate_up.shape[1] // 2
-    return (x.dtype == torch.bfloat16 and w_gate_up.shape[1] % 2 == 0 and half % 8 == 0
-            and w_down.shape[1] % 8 == 0 and w_down.shape[2] == half)
+    gate_up, down = w_gate_up.shape, w_down.shape
+    return x.dtype == torch.bfloat16 and gate_up[1] == 2 * down[2] and down[2] % 8 == 0 and down[1] % 8 == 0
 
 
 def compose_row_maps(row_map: torch.Tensor, expand_idx: torch.Tensor, n_src: int) -> torch.Tensor:
@@ -235,9 +234,8 @@ class FP8SwiGLUSplitExpertsFunc:
 
 def supported_split(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor) -> bool:
     """As :func:`supported`, and the halves must be whole 128-row blocks of the fused operand."""
-    half = w_gate.shape[1]
-    return (x.dtype == torch.bfloat16 and w_gate.shape == w_up.shape and half % 128 == 0
-            and w_down.shape[1] % 8 == 0 and w_down.shape[2] == half)
+    gate, down = w_gate.shape, w_down.shape
+    return x.dtype == torch.bfloat16 and gate[1] == down[2] and gate[1] % 128 == 0 and down[1] % 8 == 0 and gate == w_up.shape
 
 
 class FP8ClampedSwiGLUExpertsFunc:
