@@ -52,15 +52,16 @@ def _cached(cache, version: int, now: int, twin: bool) -> bool:
 
 
 def _whole_blocks(row_map, grouped_mm_offs):
-    """The row map and the group ends of groups that are multiples of 64 rows, spread to multiples of 128.  A block is
+    """Row map, group ends and group sizes of groups that are multiples of 64 rows, spread to multiples of 128.  A block is
     handed the former where nothing should be kept for a backward; if its forward finds otherwise (a pre-hook made the rows
     require a gradient, or changed their type), what runs then reads groups of whole 128-row tiles."""
-    ends = ((torch.diff(grouped_mm_offs, prepend=grouped_mm_offs.new_zeros(1)) + 127) // 128 * 128).cumsum(0, dtype=torch.int32)
+    sizes = (torch.diff(grouped_mm_offs, prepend=grouped_mm_offs.new_zeros(1)) + 127) // 128 * 128
+    ends = sizes.cumsum(0, dtype=torch.int32)
     rows = torch.arange(row_map.shape[0], device=row_map.device, dtype=torch.int32)
     moved = torch.cat([ends.new_zeros(1), ends - grouped_mm_offs])  # rows of padding before a group, and behind the last one
     at = rows + moved[torch.searchsorted(grouped_mm_offs, rows, right=True)]
     whole = row_map.new_full(((row_map.shape[0] + 64 * ends.shape[0] + 127) // 128 * 128,), -1)
-    return whole.index_copy_(0, at.long(), row_map), ends
+    return whole.index_copy_(0, at.long(), row_map), ends, sizes
 
 
 class Qwen3MoeExperts(nn.Module):
@@ -130,13 +131,13 @@ class Qwen3MoeExperts(nn.Module):
                 return fused_experts.forward_only(x, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
                                                   few_rows=few_rows)  # fmt: skip
             if few_rows:
-                row_map, grouped_mm_offs = _whole_blocks(row_map, grouped_mm_offs)
+                row_map, grouped_mm_offs, ks_tensor = _whole_blocks(row_map, grouped_mm_offs)
             return fused_experts.FP8SwiGLUSplitExpertsFunc.apply(
                 x, gate, up, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
             )  # fmt: skip
         assert expand_idx is None, "expand_idx needs the one-node FP8 path"
         if few_rows:
-            row_map, grouped_mm_offs = _whole_blocks(row_map, grouped_mm_offs)
+            row_map, grouped_mm_offs, ks_tensor = _whole_blocks(row_map, grouped_mm_offs)
         gi = precompute_group_indices(grouped_mm_offs, x.shape[0])
         kwargs = dict(grouped_mm_offs=grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, group_indices=gi)
         if row_map is not None:
@@ -230,14 +231,14 @@ class Qwen35MoeExperts(nn.Module):
                 return fused_experts.forward_only(x, down, grouped_mm_offs, *self._quantized_weights(), row_map, expand_idx,
                                                   few_rows=few_rows)  # fmt: skip
             if few_rows:
-                row_map, grouped_mm_offs = _whole_blocks(row_map, grouped_mm_offs)
+                row_map, grouped_mm_offs, ks_tensor = _whole_blocks(row_map, grouped_mm_offs)
             return fused_experts.FP8SwiGLUExpertsFunc.apply(
                 x, gate_up, down, grouped_mm_offs, ks, ks_tensor,
                 *self._quantized_weights(), row_map, expand_idx,
             )  # fmt: skip
         assert expand_idx is None, "expand_idx needs the one-node FP8 path"
         if few_rows:
-            row_map, grouped_mm_offs = _whole_blocks(row_map, grouped_mm_offs)
+            row_map, grouped_mm_offs, ks_tensor = _whole_blocks(row_map, grouped_mm_offs)
         gi = precompute_group_indices(grouped_mm_offs, x.shape[0])
         kwargs = dict(grouped_mm_offs=grouped_mm_offs, ks=ks, ks_tensor=ks_tensor, group_indices=gi)
         if row_map is not None:
@@ -331,7 +332,7 @@ class GptOssExperts(nn.Module):
                     (1.702, self.swiglu_limit), (gate_up_bias, down_bias), few_rows,
                 )
             if few_rows:
-                row_map, grouped_mm_offs = _whole_blocks(row_map, grouped_mm_offs)
+                row_map, grouped_mm_offs, ks_tensor = _whole_blocks(row_map, grouped_mm_offs)
             return fused_experts.FP8ClampedSwiGLUExpertsFunc.apply(
                 x, gate_up, gate_up_bias, down, down_bias, grouped_mm_offs,
                 *self._quantized_weights(), 1.702, self.swiglu_limit, row_map, scatter_output,

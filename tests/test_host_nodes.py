@@ -166,7 +166,7 @@ def test_groups_of_64_rows_spread_to_whole_blocks():
     expert_idxs = torch.cat([torch.full((n,), e) for e, n in enumerate((1, 0, 64, 65, 128, 0, 200, 3))])
     expert_idxs = expert_idxs[torch.randperm(len(expert_idxs), generator=torch.Generator().manual_seed(0))]
     _, ends, _, _, few = _grouped(expert_idxs, 8, 64)
-    _, want_ends, _, _, want = _grouped(expert_idxs, 8)
-    got, got_ends = _whole_blocks(torch.cat([few, few.new_full((256,), -1)]), ends)  # longer than the grouped rows
-    assert got_ends.dtype == torch.int32 and torch.equal(got_ends, want_ends) and len(got) % 128 == 0
+    _, want_ends, _, want_sizes, want = _grouped(expert_idxs, 8)
+    got, got_ends, got_sizes = _whole_blocks(torch.cat([few, few.new_full((256,), -1)]), ends)  # longer than the grouped rows
+    assert got_ends.dtype == torch.int32 and torch.equal(got_ends, want_ends) and torch.equal(got_sizes, want_sizes) and len(got) % 128 == 0
     assert torch.equal(got[: len(want)], want) and (got[len(want) :] == -1).all()
