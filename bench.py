@@ -151,7 +151,7 @@ class GemmTimer:
     """HIP events (on the stream the kernels are launched on) around every GEMM entry point."""
 
     NAMES = ("pt_gemm_m_grouped_nt", "pt_gemm_m_grouped_nt_scatter", "pt_gemm_m_grouped_nt_bias",
-             "pt_gemm_m_grouped_nn", "pt_gemm_m_grouped_nn_scatter", "pt_gemm_m_grouped_by_block",
+             "pt_gemm_m_grouped_nn", "pt_gemm_m_grouped_nn_scatter", "pt_gemm_m_grouped_by_block", "pt_gemm_m_grouped_by_block_two",
              "pt_gemm_m_grouped_nt_scatter_bias", "pt_gemm_k_grouped_wgrad",
              "pt_gemm_k_grouped_wgrad_ld", "pt_gemm_k_grouped_wgrad_pair",
              "pt_gemm_nt_dense", "pt_gemm_nt_dense_splitk", "pt_gemm_nt_dense_ld", "pt_gemm_nt_dense_splitk_ld", "pt_gemm_nt_dense_heads", "pt_gemm_nt_dense_pair", "pt_gemm_m_grouped_nt_few_rows")
@@ -182,6 +182,7 @@ class GemmTimer:
                 sizes = {"pt_gemm_nt_dense": args[6:9], "pt_gemm_nt_dense_splitk": args[7:10],
                          "pt_gemm_nt_dense_ld": args[8:11], "pt_gemm_nt_dense_splitk_ld": args[9:12],
                          "pt_gemm_k_grouped_wgrad": args[9:12], "pt_gemm_m_grouped_by_block": args[9:12],
+                         "pt_gemm_m_grouped_by_block_two": args[10:13],
                          "pt_gemm_k_grouped_wgrad_ld": args[11:14],
                          "pt_gemm_k_grouped_wgrad_pair": args[11:14]}.get(name, args[8:11])
                 timer.records.append((name, a, b, "x".join(str(int(v)) for v in sizes)))

@@ -318,6 +318,12 @@ int pt_gemm_m_grouped_by_block(const void* a_fp8, const float* a_scale, const vo
                                int b_reduction_major, void* out, int out_dtype, const int32_t* offs, int32_t num_groups,
                                int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows,
                                pt_stream_t stream);
+/* The same stored to two outputs: result row r to row out_row_index[r] of out (out_rows rows), an index of -2 - i to row i
+ * of out2 (out2_rows rows), -1 nowhere.  The index is not checked against out_rows and out2_rows on the device. */
+int pt_gemm_m_grouped_by_block_two(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale,
+                                   int b_reduction_major, void* out, void* out2, int out_dtype, const int32_t* offs,
+                                   int32_t num_groups, int64_t M, int64_t N, int64_t K, const int32_t* out_row_index,
+                                   int64_t out_rows, int64_t out2_rows, pt_stream_t stream);
 
 /* pt_gemm_m_grouped_nt followed by `out + bias[group of the row]` in the output type (the result
  * is rounded to bf16, then the bias row of its group is added and the sum rounded again): the
@@ -437,6 +443,17 @@ int64_t pt_gather_rows_backward_workspace_bytes(int64_t n, int64_t rows);
 int pt_gather_rows_backward(const void* grad_out, int64_t ld_go, void* grad_in, int64_t ld_gi,
                             const int64_t* index, int64_t n, int64_t rows, int64_t H, int dtype,
                             void* workspace, int64_t workspace_bytes, pt_stream_t stream);
+/* The same in two parts around the kernel that writes grad_out from grouped rows (a GEMM that un-permutes on the way):
+ * _begin fills the workspace from the index and says in dest[q], q < M, where the row of grouped row q belongs, whose
+ * index entry is j = row_map[q] (negative: padding): index[j] where no other entry names that row, -2 - j where
+ * others do, -1 for padding and for an entry outside [0, rows).  Rows with one source then need no sum: the kernel writes
+ * them to grad_in, the others to row j of grad_out (pt_gemm_m_grouped_by_block_two), and _shared adds those up from
+ * the same workspace and zeroes the rows that no entry names. */
+int pt_gather_rows_backward_begin(const int64_t* index, int64_t n, int64_t rows, void* workspace, int64_t workspace_bytes,
+                                  const int32_t* row_map, int32_t* dest, int64_t M, pt_stream_t stream);
+int pt_gather_rows_backward_shared(const void* grad_out, int64_t ld_go, void* grad_in, int64_t ld_gi, int64_t n,
+                                   int64_t rows, int64_t H, int dtype, void* workspace, int64_t workspace_bytes,
+                                   pt_stream_t stream);
 
 /* group_ids[r] = min(#{g : offs[g] <= r}, G-1), r < M; out_dtype_bytes 4 (int32) or 8 (int64).
  * precompute_group_indices, token_scatter.py:370-384; GptOssExperts.forward,

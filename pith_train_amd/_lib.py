@@ -61,6 +61,7 @@ SIGNATURES = {
     "pt_gemm_m_grouped_nn": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P]),
     "pt_gemm_m_grouped_nn_scatter": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P]),
     "pt_gemm_m_grouped_by_block": (c_int, [P, P, P, P, c_int, P, c_int, P, I32, I64, I64, I64, P, I64, P]),
+    "pt_gemm_m_grouped_by_block_two": (c_int, [P, P, P, P, c_int, P, P, c_int, P, I32, I64, I64, I64, P, I64, I64, P]),
     "pt_gemm_m_grouped_nt_bias": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, P]),
     "pt_gemm_m_grouped_nt_scatter_bias": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P, P]),
     "pt_gemm_m_grouped_nt_scatter": (c_int, [P, P, P, P, P, c_int, P, I32, I64, I64, I64, P, I64, P]),
@@ -88,6 +89,8 @@ SIGNATURES = {
     "pt_gather_rows": (c_int, [P, I64, P, I64, P, I64, I64, I32, P]),
     "pt_gather_rows_backward_workspace_bytes": (I64, [I64, I64]),
     "pt_gather_rows_backward": (c_int, [P, I64, P, I64, P, I64, I64, I64, c_int, P, I64, P]),
+    "pt_gather_rows_backward_begin": (c_int, [P, I64, I64, P, I64, P, P, I64, P]),
+    "pt_gather_rows_backward_shared": (c_int, [P, I64, P, I64, I64, I64, I64, c_int, P, I64, P]),
     "pt_group_indices": (c_int, [P, I32, I64, P, I32, P]),
     "pt_dedup_workspace_bytes": (I64, [I64, I32, I32, I32]),
     "pt_dedup_prepare_dispatch": (c_int, [P, I64, I64, I32, I32, I32, I32, P, P, P, P, P, P, P, I64, P]),

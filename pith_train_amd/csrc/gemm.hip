@@ -527,7 +527,7 @@ extern "C" int pt_sum_partials(const float* partial, int32_t splits, int64_t n, 
 
 int pt::gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order, const void* b_fp8, const float* b_scale, void* out, int out_dtype,
                        const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows,
-                       const void* bias, pt_stream_t stream, bool b_kmajor, bool few_rows) {
+                       const void* bias, pt_stream_t stream, bool b_kmajor, bool few_rows, void* out2, int64_t out2_rows) {
   PT_REQUIRE(M >= 0 && N >= 0 && K >= 0 && G > 0, "gemm_m_grouped_nt: bad sizes");
   if (M == 0 || N == 0) return PT_OK;
   PT_REQUIRE(M % (few_rows ? 64 : 128) == 0, "gemm_m_grouped_nt: M=%lld must be a multiple of %d", (long long)M, few_rows ? 64 : 128);
@@ -558,6 +558,11 @@ int pt::gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order,
     PT_REQUIRE(out_rows >= 0 && N % 8 == 0 && al16(out) && out_rows * N * 2 < (1ll << 32),
                "gemm_m_grouped_nt_scatter: needs N %% 8 == 0, a 16-byte aligned output smaller than 4 GiB");
     g.out_row_index = out_row_index; g.out_rows = out_rows;
+    if (out2) {
+      PT_REQUIRE(!bias && al16(out2) && out2_rows >= 0 && out2_rows * N * 2 < (1ll << 32),
+                 "gemm_m_grouped: the second output has no bias, is 16-byte aligned and smaller than 4 GiB");
+      g.out2 = out2;
+    }
   }
   if (bias) {
     PT_REQUIRE(N % 8 == 0 && al16(out) && al16(bias),
@@ -623,6 +628,14 @@ extern "C" int pt_gemm_m_grouped_by_block(const void* a_fp8, const float* a_scal
                                           const int32_t* out_row_index, int64_t out_rows, pt_stream_t stream) {
   return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_BLOCK, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, nullptr,
                         stream, b_reduction_major != 0);
+}
+
+extern "C" int pt_gemm_m_grouped_by_block_two(const void* a_fp8, const float* a_scale, const void* b_fp8, const float* b_scale, int b_reduction_major,
+                                              void* out, void* out2, int out_dtype, const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K,
+                                              const int32_t* out_row_index, int64_t out_rows, int64_t out2_rows, pt_stream_t stream) {
+  PT_REQUIRE(out2 && out_row_index, "gemm_m_grouped_by_block_two: null output or index");
+  return gemm_m_grouped(a_fp8, a_scale, RowScales::BY_BLOCK, b_fp8, b_scale, out, out_dtype, offs, G, M, N, K, out_row_index, out_rows, nullptr,
+                        stream, b_reduction_major != 0, false, out2, out2_rows);
 }
 
 static int gemm_k_grouped_wgrad_impl(const void* dy_t_fp8, const float* dy_scale, int64_t ld_dy_scale, const void* x_t_fp8,

@@ -24,7 +24,8 @@ struct GemmArgs {
   int64_t out_rows;                       // rows of the output when out_row_index is given
   const void* bias;                       // m-grouped only: [G, rows_b] in the output's type, row g added to the rows of group g
   int64_t split_len;                      // k-grouped with offs == null: group g reduces over [g, g + 1) * split_len (split-K)
-  void* out2; int64_t split_row;          // k-grouped: result rows from split_row on (a multiple of 128; 0 = none) go to out2, a second
+  void* out2; int64_t split_row;          // m-grouped with out_row_index: row -2 - i of the index goes to row i of out2.
+                                          // k-grouped: result rows from split_row on (a multiple of 128; 0 = none) go to out2, a second
                                           // parameter's gradient (group stride out2_stride_g) whose row 0 is row split_row
   int64_t out2_stride_g;
   int head_a, head_b;                     // dense only: result column h * (head_a + head_b) + c is out[h * head_a + c] for c < head_a, else

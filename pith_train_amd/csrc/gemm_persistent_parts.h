@@ -672,6 +672,21 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[TM][TN], const Gemm
       else dst[i] = p.out_row_index[r < T.a_lim ? r : T.a_row0];
       if (r >= T.a_lim) dst[i] = -1;
     }
+    if (p.out2) {
+      // Two outputs, -2 - r for row r of the second: 64-bit addresses, since no descriptor spans both.  (Rows of an
+      // input gradient that nobody else adds to go to their place at once, see pt_gather_rows_backward_begin.)
+      if (kAblateStores) return;
+#pragma unroll
+      for (int j = 0; j < TN; j += 2) {
+        const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;
+        stage_column<false>(acc, j, stg, lane, [&](int i, int q, v4i w) {
+          const int row = __shfl(dst[i], q * 8 + (lane >> 3));
+          char* to = (char*)(row >= 0 ? p.out : p.out2) + (uint64_t)(uint32_t)(row >= 0 ? row : -2 - row) * pitch + (uint32_t)colc * 2;
+          if (row != -1 && colc < T.b_lim) __builtin_nontemporal_store(w, (v4i*)to);
+        });
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < TN; j += 2) {
       const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;

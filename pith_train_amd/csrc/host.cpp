@@ -89,6 +89,8 @@ struct Library {
   PT_FN(pt_gather_rows);
   PT_FN(pt_gather_rows_backward_workspace_bytes);
   PT_FN(pt_gather_rows_backward);
+  PT_FN(pt_gather_rows_backward_begin);
+  PT_FN(pt_gather_rows_backward_shared);
   PT_FN(pt_permute_rows);
   PT_FN(pt_silu_mul_fwd);
   PT_FN(pt_silu_mul_bwd);
@@ -107,6 +109,7 @@ struct Library {
   PT_FN(pt_adjust_expand_idx);
   PT_FN(pt_quant_rowwise_colwise_by_block);
   PT_FN(pt_gemm_m_grouped_by_block);
+  PT_FN(pt_gemm_m_grouped_by_block_two);
   PT_FN(pt_gemm_k_grouped_wgrad);
   PT_FN(pt_sum_branches);
 #undef PT_FN
@@ -142,6 +145,8 @@ void init(const std::string& path) {
   PT_FN(pt_gather_rows);
   PT_FN(pt_gather_rows_backward_workspace_bytes);
   PT_FN(pt_gather_rows_backward);
+  PT_FN(pt_gather_rows_backward_begin);
+  PT_FN(pt_gather_rows_backward_shared);
   PT_FN(pt_permute_rows);
   PT_FN(pt_silu_mul_fwd);
   PT_FN(pt_silu_mul_bwd);
@@ -160,6 +165,7 @@ void init(const std::string& path) {
   PT_FN(pt_adjust_expand_idx);
   PT_FN(pt_quant_rowwise_colwise_by_block);
   PT_FN(pt_gemm_m_grouped_by_block);
+  PT_FN(pt_gemm_m_grouped_by_block_two);
   PT_FN(pt_gemm_k_grouped_wgrad);
   PT_FN(pt_sum_branches);
 #undef PT_FN
@@ -1063,6 +1069,30 @@ Tensor grouped_linear(const Tensor& x, const Tensor& weight, const Tensor& offs,
       x, weight);
 }
 
+// Input gradient of an expert block whose routed rows expand `src_rows` rows: what the scattering GEMM and the backward of
+// the expanding gather after it give, but a row with one routed row goes to its place from the GEMM's store and is not
+// read, added to nothing and written again (262 144 rows of 2048, a quarter of them repeats: sum 299 -> 132 us, and 6 for the destinations;
+// 32 768 rows that five of eight ranks' tokens share: 39 -> 28 and 5).
+Tensor expanded_input_gradient(const Tensor& dgu, const Tensor& dgu_s, const Tensor& w, const Tensor& w_s, bool forward_layout, const Tensor& offs,
+                               const Tensor& row_map, const Tensor& expand_idx, int64_t src_rows, int64_t K, int64_t stream) {
+  const auto st = (pt_stream_t)stream;
+  const auto dev = dgu.device();
+  const int64_t n = expand_idx.size(0), M = row_map.size(0), N = dgu.size(1), G = offs.size(0);
+  Tensor out = empty({cdiv(src_rows, kRowAlignment) * kRowAlignment, K}, at::kBFloat16, dev), shared = empty({n, K}, at::kBFloat16, dev);
+  const int64_t bytes = up256(lib.pt_gather_rows_backward_workspace_bytes(n, src_rows));
+  Tensor ws = empty({bytes + 4 * M}, at::kByte, dev);
+  int32_t* const dest = (int32_t*)((char*)ptr(ws) + bytes);
+  check(lib.pt_gather_rows_backward_begin((const int64_t*)ptr(expand_idx), n, src_rows, ptr(ws), bytes, (const int32_t*)ptr(row_map), dest, M, st),
+        "pt_gather_rows_backward_begin");
+  const char* what = forward_layout ? "pt_gemm_m_grouped_nn_scatter" : "pt_gemm_m_grouped_nt_scatter";
+  lib.pt_observe(what, 1, M, K, N);
+  check(lib.pt_gemm_m_grouped_by_block_two(ptr(dgu), (const float*)ptr(dgu_s), ptr(w), (const float*)ptr(w_s), forward_layout, ptr(out), ptr(shared), PT_BF16,
+                                           (const int32_t*)ptr(offs), (int32_t)G, M, K, N, dest, src_rows, n, st), what);
+  lib.pt_observe(what, 0, M, K, N);
+  check(lib.pt_gather_rows_backward_shared(ptr(shared), K, ptr(out), K, n, src_rows, K, PT_BF16, ptr(ws), bytes, st), "pt_gather_rows_backward_shared");
+  return out.narrow(0, 0, src_rows);
+}
+
 // ---- expert block -----------------------------------------------------------------------------------------
 struct ExpertsNode : HipNode {
   Dims d;
@@ -1098,11 +1128,19 @@ struct ExpertsNode : HipNode {
     }
     ExpertsBackward step(g[0], d, offs, row_map, scatter, saved[DN_DG].get(), saved[DN_DG_S].get(), dn_forward, saved[GATE_UP].get(), std::move(kept),
                          clamped, alpha, limit, gu_bias, dn_bias, std::move(weights), (int64_t)stream);
-    Tensor gx = empty({row_map ? routed : d.M, d.K}, g[0].scalar_type(), g[0].device());
-    {
+    // Rows that expand the same source row are summed (the backward of the expanding gather), right behind the GEMM
+    // that wrote them: after the weight gradient they come from HBM.  Only a sum of bf16 rows below 4 GiB takes two outputs.
+    const bool two = expand_idx && row_map && g[0].scalar_type() == at::kBFloat16 && d.K % 8 == 0 && src_rows * d.K < (1ll << 31) &&
+                     routed * d.K < (1ll << 31);
+    Tensor gx;
+    if (two) gx = expanded_input_gradient(step.dgu, step.dgu_s, gu_dg, gu_dg_s, gu_forward, offs, *row_map, *expand_idx, src_rows, d.K, (int64_t)stream);
+    else gx = empty({row_map ? routed : d.M, d.K}, g[0].scalar_type(), g[0].device());
+    if (!two || deferred) {
       py::gil_scoped_acquire gil;
-      const py::handle dgrad(g_dgrad);
-      dgrad(py::make_tuple(step.dgu, step.dgu_s), gu_dg, gu_dg_s, gu_forward, gx, offs, row_map);
+      if (!two) {
+        const py::handle dgrad(g_dgrad);
+        dgrad(py::make_tuple(step.dgu, step.dgu_s), gu_dg, gu_dg_s, gu_forward, gx, offs, row_map);
+      }
       if (deferred) {
         const auto op = step.operands();
         auto pair = [](const std::pair<Tensor, Tensor>& p) { return py::make_tuple(p.first, p.second); };
@@ -1119,9 +1157,7 @@ struct ExpertsNode : HipNode {
     }
     step.dgu.reset();
     step.dgu_s.reset();
-    // rows that expand the same source row are summed (the backward of the expanding gather), right behind the GEMM
-    // that wrote them: after the weight gradient they come from HBM
-    if (expand_idx) gx = scatter_sum(gx, *expand_idx, src_rows, kRowAlignment, (int64_t)stream);
+    if (expand_idx && !two) gx = scatter_sum(gx, *expand_idx, src_rows, kRowAlignment, (int64_t)stream);
     if (!deferred) step.weight_gradient();
     if (repeat > 1) gx = gx.view({src_rows, repeat, d.K});
     return {gx, Tensor(), Tensor(), Tensor(), step.d_gu_bias.value_or(Tensor()), step.d_dn_bias.value_or(Tensor())};

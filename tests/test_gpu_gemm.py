@@ -524,6 +524,51 @@ def test_row_scales_by_block(gemm_kernel, N, K):
         assert torch.equal(want, got)
 
 
+@pytest.mark.parametrize("users", ["one", "some", "many", "outside"])
+@pytest.mark.parametrize("N,K", [(256, 128), (272, 272), (2880, 1408)])
+def test_rows_of_two_outputs(gemm_kernel, N, K, users):
+    """An input gradient whose rows are summed by the row they expand: stored to the sum's place where there is nothing
+    to add, and summed from a second output elsewhere, against scattering all of it and summing all of it.  Every
+    source row used once, some not at all and some by two, one by more than a wave's lanes, indices outside the rows."""
+    from pith_train_amd import _lib
+
+    if gemm_kernel in ("p0", "q0", "q1", "t"):
+        pytest.skip("names of r0, and a kernel that stores no scattered rows")
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    rows = torch.tensor([128, 0, 384, 640], dtype=torch.int32)
+    G_, M, KB = len(rows), int(rows.sum()), (K + 127) // 128
+    offs = torch.cumsum(rows, 0).int().cuda()
+    n = M - 200  # rows of padding among the grouped ones
+    row_map = torch.full((M,), -1, dtype=torch.int32, device="cuda")
+    row_map[torch.randperm(M, device="cuda", generator=g)[:n]] = torch.randperm(n, device="cuda", generator=g).int()
+    src = {"one": n, "some": n, "many": 40, "outside": n // 2}[users]
+    index = torch.randperm(n, device="cuda", generator=g) if users == "one" else torch.randint(0, src, (n,), device="cuda", generator=g)
+    if users == "many":
+        index[: n // 2] = 7
+    if users == "outside":
+        index[::5] = src
+        index[1::7] = -1
+    q = torch.randint(0, 256, (M, K), dtype=torch.uint8, device="cuda", generator=g) & 0xBF
+    q_s = torch.exp2(torch.randint(-6, 3, (KB, M), device="cuda", generator=g).float())
+    b = torch.randint(0, 256, (G_, N, K), dtype=torch.uint8, device="cuda", generator=g) & 0xBF
+    b_s = torch.exp2(torch.randint(-6, 3, (G_, (N + 127) // 128, KB), device="cuda", generator=g).float())
+    bf16, stream = _lib.dtype_code(torch.bfloat16), _lib.stream_ptr()
+    size = _lib.query("pt_gather_rows_backward_workspace_bytes", n, src)
+    ws, dest = torch.empty(size, dtype=torch.uint8, device="cuda"), torch.empty(M, dtype=torch.int32, device="cuda")
+    for reduction_major in (0, 1):
+        w, w_s = (b.transpose(1, 2).contiguous(), b_s.transpose(1, 2).contiguous()) if reduction_major else (b, b_s)
+        all_rows, shared = (torch.full((n, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        want, got = (torch.full((src, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        operands = (_lib.ptr(q), _lib.ptr(q_s), _lib.ptr(w), _lib.ptr(w_s), reduction_major)
+        _lib.call("pt_gemm_m_grouped_by_block", *operands, _lib.ptr(all_rows), bf16, _lib.ptr(offs), G_, M, N, K, _lib.ptr(row_map), n, stream)
+        _lib.call("pt_gather_rows_backward", _lib.ptr(all_rows), N, _lib.ptr(want), N, _lib.ptr(index), n, src, N, bf16, _lib.ptr(ws), size, stream)
+        _lib.call("pt_gather_rows_backward_begin", _lib.ptr(index), n, src, _lib.ptr(ws), size, _lib.ptr(row_map), _lib.ptr(dest), M, stream)
+        _lib.call("pt_gemm_m_grouped_by_block_two", *operands, _lib.ptr(got), _lib.ptr(shared), bf16, _lib.ptr(offs), G_, M, N, K, _lib.ptr(dest), src, n,
+                  stream)
+        _lib.call("pt_gather_rows_backward_shared", _lib.ptr(shared), N, _lib.ptr(got), N, n, src, N, bf16, _lib.ptr(ws), size, stream)
+        assert torch.isfinite(want.float()).all() and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("tiles", [1, 3, 4, 10])
 def test_grouped_tile_order_at_the_edges_of_its_strips(gemm_kernel, tiles):
     """Groups with more row tiles than column tiles and the other way round, one strip and several of unequal
