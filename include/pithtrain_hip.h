@@ -374,7 +374,7 @@ int pt_gemm_k_grouped_wgrad_pair(const void* dy_t_fp8, const float* dy_scale, co
  * shape; the default unless the environment variable PT_GEMM_IMPL names one of the others),
  * "r0" persistent kernel, one 256x256 tile after the other per compute unit ("p0", "q0" and "q1", names of
  * main loops that it has replaced, mean the same), "s64" / "s128" one 64x128 / 128x128 tile per workgroup
- * (small problems), "t" one 128x128 tile per workgroup through 64-bit addresses.
+ * (small problems), "s128d" the latter with one workgroup per compute unit (dense products, else "s128"), "t" one 128x128 tile per workgroup through 64-bit addresses.
  * Every choice computes the same function; this exists for measurements and for tests that
  * cover each kernel.  Process-wide, not synchronised with concurrent GEMM calls.
  * No counterpart in the reference (DeepGEMM selects its kernels internally). */

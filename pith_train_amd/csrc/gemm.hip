@@ -264,7 +264,7 @@ static int launch_gemm(const GemmArgs& a, hipStream_t stream) {
 // PT_GEMM_IMPL overrides the choice of kernel for measurements: "t" = one 128x128 tile per
 // workgroup, "r0" = persistent kernel with the row-split loop ("p0", "q0", "q1", names of main loops that it
 // has replaced, mean the same), "s64" / "s128" = one 64 / 128 x 128 tile per workgroup with a deep load
-// ring.  Unset: chosen per call from the shape (below).
+// ring, "s128d" = the form of "s128" with one workgroup per compute unit (dense products; the others take "s128").  Unset: chosen per call from the shape (below).
 enum { IMPL_UNSET = -3, IMPL_AUTO = -2, IMPL_TILE = -1, IMPL_ROWSPLIT = 0, IMPL_SMALL = 1000 };
 static int g_impl = IMPL_UNSET;
 static bool parse_impl(const char* e, int& impl) {
@@ -273,6 +273,7 @@ static bool parse_impl(const char* e, int& impl) {
   else if (!strcmp(e, "r0") || !strcmp(e, "p0") || !strcmp(e, "q0") || !strcmp(e, "q1")) impl = IMPL_ROWSPLIT;
   else if (!strcmp(e, "s64")) impl = IMPL_SMALL + 64;
   else if (!strcmp(e, "s128")) impl = IMPL_SMALL + 128;
+  else if (!strcmp(e, "s128d")) impl = IMPL_SMALL + kDeepTile;
   else return false;
   return true;
 }
@@ -287,7 +288,10 @@ static int gemm_impl() {
 // Problems too small for 256 x 256 tiles to fill 256 compute units evenly go to the kernel with one 64 x 128
 // or 128 x 128 tile per workgroup and two workgroups per compute unit (gemm_small.hip): tile rows, or 0
 // when the persistent kernel is the better choice.  While all 64-row tiles run at once the smaller tile
-// wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 21.5 for the large one).  Then both
+// wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 21.5 for the large one).  While the 128-row tiles do,
+// dense ones with a long reduction take the form with one workgroup per unit (us, two per unit / one: 1001 x 4096 x 1536 14.7 / 13.1,
+// 1792 17.3 / 14.0, 2880 27.7 / 20.8; 2048 x 2048 x 1536 11.5 / 11.5, 1792 13.3 / 12.8, 2048 16.4 / 14.0; 4096 x 1024 x 1792 12.1 /
+// 12.5, 2048 13.3 / 13.4, 2880 24.1 / 19.0).  Then both
 // kinds are priced in rounds of the GPU: a round of 256 large tiles is the unit, a round of 512 small ones
 // (a quarter of the area each, half of it in all) costs 0.72 of it in the m-grouped mode, 0.68 in
 // the dense one (0.45 up to a reduction of 512, most of it filling and draining), 0.36 for a weight gradient
@@ -306,6 +310,7 @@ static int small_tile_rows(const GemmArgs& g) {
   const int64_t cols = cdiv(g.rows_b, 128) * groups, cols_large = cdiv(g.rows_b, 256) * groups;
   if (cdiv(g.rows_a, 64) * cols <= 256) return 64;
   int64_t small = cdiv(g.rows_a, 128) * cols;
+  if (small <= 256 && g.mode == GEMM_DENSE && g.red >= 1792) return kDeepTile;
   if (small <= 512) return 128;
   int64_t rows_large = cdiv(g.rows_a, 256);
   if (g.mode == GEMM_M_GROUPED) {
@@ -370,7 +375,7 @@ using namespace pt;
 
 extern "C" int pt_gemm_select_kernel(const char* name) {
   int impl;
-  PT_REQUIRE(parse_impl(name, impl), "gemm_select_kernel: unknown kernel '%s' (auto, r0, s64, s128, t; p0, q0 and q1 mean r0)", name);
+  PT_REQUIRE(parse_impl(name, impl), "gemm_select_kernel: unknown kernel '%s' (auto, r0, s64, s128, s128d, t; p0, q0 and q1 mean r0)", name);
   g_impl = impl;
   return PT_OK;
 }
@@ -417,11 +422,20 @@ extern "C" int pt_gemm_nt_dense_pair(const pt_dense_gemm* two, int out_dtype, pt
   }
   // One launch where each would take the small-tile kernel and their tiles together still make one round
   // of two workgroups per compute unit, 64-row tiles if those do (4096 x 512 x 4096 twice, 256 tiles
-  // each: 39.7 us in two launches, 11 less in one).
+  // each: 39.7 us in two launches, 11 less in one).  Where 64-row tiles nearly fill or overfill that round, one workgroup per unit
+  // with its deep ring is ahead, if the first product's reduction is long and the second one's tiles all run, one after
+  // the other, on the units that the first leaves while it lasts.  Us, 64- or 128-row tiles / deep: 4096 x 512 x 4096 twice 30.2 /
+  // 27.5, 3300 rows (464 tiles) 25.0 / 24.4, 2900 (440) 23.0 / 23.9; 700 x 2048 x 2048 with 2048 x 2048 x 700 18.1 / 14.6,
+  // 900 rows 18.6 / 16.8, 1200 (the second one's tiles do not fit) 18.9 / 22.8; 800 x 2048 x 4096 with 4096 x 2048 x 800
+  // 33.6 / 31.0, 900 rows (do not fit) 31.0 / 33.8.
   if (gemm_impl() == IMPL_AUTO && fits_persistent(g[0]) && fits_persistent(g[1]) && small_tile_rows(g[0]) && small_tile_rows(g[1])) {
+    const auto tiles = [&](int i, int rows) { return cdiv(g[i].rows_a, rows) * cdiv(g[i].rows_b, 128); };
+    // tiles of the second that take as long as one of the first (a block of 128 more each for the change of tiles)
+    const int64_t in_turn = (cdiv(g[0].red, 128) + 2) / (cdiv(g[1].red, 128) + 1);
+    if (g[0].red >= 2048 && in_turn >= 1 && tiles(0, 64) + tiles(1, 64) > 456 && tiles(0, 128) + cdiv(tiles(1, 128), in_turn) <= 256)
+      return launch_gemm_small_pair(g[0], g[1], kDeepTile, (hipStream_t)stream);
     for (int rows : {64, 128})
-      if (cdiv(g[0].rows_a, rows) * cdiv(g[0].rows_b, 128) + cdiv(g[1].rows_a, rows) * cdiv(g[1].rows_b, 128) <= 512)
-        return launch_gemm_small_pair(g[0], g[1], rows, (hipStream_t)stream);
+      if (tiles(0, rows) + tiles(1, rows) <= 512) return launch_gemm_small_pair(g[0], g[1], rows, (hipStream_t)stream);
   }
   if (int rc = dispatch_gemm(g[0], (hipStream_t)stream)) return rc;
   return dispatch_gemm(g[1], (hipStream_t)stream);

@@ -45,7 +45,9 @@ __device__ __forceinline__ int k_group_end(const GemmArgs& p, int g) {
 
 // persistent kernel whose two steps per 128-block split the tile by rows (gemm_rowsplit.hip)
 int launch_gemm_rowsplit(const GemmArgs& a, hipStream_t stream);
-// one tile of 64 or 128 rows x 128 columns per workgroup, for small problems (gemm_small.hip)
+// one tile of 64 or 128 rows x 128 columns per workgroup, for small problems (gemm_small.hip); kDeepTile: 128 rows, one
+// workgroup per compute unit (dense products)
+static constexpr int kDeepTile = 129;
 int launch_gemm_small(const GemmArgs& a, int rows, hipStream_t stream);
 // the tiles of two independent dense products in one launch of that kernel
 int launch_gemm_small_pair(const GemmArgs& a, const GemmArgs& b, int rows, hipStream_t stream);

@@ -4,9 +4,12 @@
 // that work spend their time waiting for one operand stage after the other.  Here a workgroup of
 // four waves owns one BM x 128 tile (BM = 64 or 128) with a ring of two or three 128-deep stages, small
 // enough that a compute unit holds two workgroups: while one waits for its first stage, drains its
-// pipeline or stores its result, the other multiplies.  (One workgroup per unit with four to five stages
-// in flight is level while there is only one tile per unit, and slower with more: 512 tiles of
-// 4096 x 2048 x 2048 28.7 us against 19.3, 128 groups of 128 rows with 1536 x 2048 weights 105 against 95.)
+// pipeline or stores its result, the other multiplies.
+// DEEP: where there is one 128-row tile per unit and a long reduction, nobody else fills a workgroup's waits.  There
+// eight waves own the tile, two a SIMD, with a ring of four stages (three in flight instead of one): us with two
+// stages and four waves / four and four / four and eight, 1001 x 4096 x 2048 20.1 / 16.3 / 15.5, 2048 x 2048 x 4096
+// 28.9 / 26.1 / 23.9, 2048 x 2048 x 2816 21.1 / 18.1 / 17.2; 2048 x 1536 x 1024 9.0 / 9.6 / 9.4.  With two tiles per unit
+// the two workgroups are the better way (2048 x 4096 x 2048 21.0, deep 29.1).
 // There is no persistent loop, no tile table and no scan over the groups (a tile finds its group with
 // one ballot over the group ends), which keeps the time before the first load and the code that has to
 // be fetched short.  Operand traffic bounds it from the L2 on (tiles x reduction x (BM + 128) bytes): 4096 x 2048 x
@@ -22,16 +25,18 @@ namespace pt {
 // LDS of a workgroup: the ring of stages, their scales, a sink for scale loads that nobody needs
 // (65.3 or 74.5 KiB: two workgroups share a compute unit)
 template <int BM> static constexpr int kSmallStages = BM == 64 ? 3 : 2;
+static constexpr int kDeepStages = 4;
+static constexpr size_t kDeepLds = (size_t)kDeepStages * (128 + 128) * (128 + 4) + 256;
 template <int BM> static constexpr size_t kSmallLds = (size_t)kSmallStages<BM> * (BM + 128) * (128 + 4) + 256;
 
 // STREAM: the loads of b pass the memory-side cache by (launch_small_mode has the rule and both sides).
-template <int MODE, int BM, bool ACC, bool BT, bool STREAM = false>
+template <int MODE, int BM, bool ACC, bool BT, bool STREAM = false, bool DEEP = false>
 __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
-  constexpr int BN = 128, BK = 128, NS = kSmallStages<BM>;
-  static_assert(2 * kSmallLds<BM> <= 160 * 1024, "two workgroups per compute unit");
-  constexpr int TM = BM / 64, TN = 2;   // waves 2 x 2, each TM x 2 blocks of 32 x 32
+  constexpr int BN = 128, BK = 128, NS = DEEP ? kDeepStages : kSmallStages<BM>, NW = DEEP ? 8 : 4;
+  static_assert(DEEP ? BM == 128 && kDeepLds <= 160 * 1024 : 2 * kSmallLds<BM> <= 160 * 1024, "one deep workgroup or two others per compute unit");
+  constexpr int TM = BM / (16 * NW), TN = 2;   // waves NW / 2 x 2, each TM x 2 blocks of 32 x 32
   constexpr int STAGE = (BM + BN) * BK;
-  constexpr int LA = BM / 32, LB = BN / 32;  // 1 KiB loads of a and of b per wave and stage
+  constexpr int LA = BM / (8 * NW), LB = BN / (8 * NW);  // 1 KiB loads of a and of b per wave and stage
   constexpr int NP = LA + LB + 1;            // and one of scales
   constexpr int kWait = (NS - 2) * NP;       // loads of the stages after the one a step needs
   static_assert(kWait < 64, "vmcnt is a 6-bit counter");
@@ -39,7 +44,7 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm0 = (wave >> 1) * (BM / 2), wn0 = (wave & 1) * 64;
+  const int wm0 = (wave >> 1) * (32 * TM), wn0 = (wave & 1) * 64;
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const uint32_t sc_base = lds_base + NS * STAGE;
 
@@ -115,12 +120,12 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
     const bool in = ok && (int)(koff + chunk * 16) < T.k_len;
 #pragma unroll
     for (int k = 0; k < LA; ++k) {
-      const int q = 4 * k + wave;
+      const int q = NW * k + wave;
       dma16(rs_a, in && 8 * q < a_rows ? va : kOob, soA0 + koff + (uint32_t)(8 * q) * (uint32_t)p.lda, sA + q * 1024);
     }
 #pragma unroll
     for (int k = 0; k < LB; ++k) {
-      const int q = 4 * k + wave;
+      const int q = NW * k + wave;
       if constexpr (BT) dma16(rs_b, ok && bt_in ? vb : kOob, soB0 + (koff + 8 * q) * (uint32_t)p.ldb, sB + q * 1024);
       else              dma16<STREAM>(rs_b, in ? vb : kOob, soB0 + koff + (uint32_t)(8 * q) * (uint32_t)p.ldb, sB + q * 1024);
     }
@@ -236,14 +241,18 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_small_kernel(GemmArgs p) {
   small_tile_body<MODE, BM, ACC, BT, STREAM>(p, blockIdx.x);
 }
 
+__global__ __launch_bounds__(512, 2) void fp8_gemm_deep_kernel(GemmArgs p) {
+  small_tile_body<GEMM_DENSE, 128, false, false, false, true>(p, blockIdx.x);
+}
+
 // Two products that do not depend on each other (the input and the weight gradient of a dense linear): the
 // workgroups past `second` (a multiple of 8) take the second one's tiles, so that compute units which
 // either would leave with one workgroup or none hold two.
 struct GemmPair { GemmArgs g[2]; int second; };
-template <int BM>
-__global__ __launch_bounds__(256, 2) void fp8_gemm_small_pair_kernel(GemmPair q) {
+template <int BM, bool DEEP>
+__global__ __launch_bounds__(DEEP ? 512 : 256, 2) void fp8_gemm_small_pair_kernel(GemmPair q) {
   const bool late = (int)blockIdx.x >= q.second;
-  small_tile_body<GEMM_DENSE, BM, false, false>(late ? q.g[1] : q.g[0], (int)blockIdx.x - (late ? q.second : 0));
+  small_tile_body<GEMM_DENSE, BM, false, false, false, DEEP>(late ? q.g[1] : q.g[0], (int)blockIdx.x - (late ? q.second : 0));
 }
 
 template <int MODE, int BM>
@@ -262,21 +271,32 @@ static int reserve_lds(Kernel kernel, size_t lds, bool& done) {
   return PT_OK;
 }
 
-template <int BM>
+template <int BM, bool DEEP = false>
 static int launch_pair(const GemmArgs& a, const GemmArgs& b, hipStream_t stream) {
+  constexpr size_t lds = DEEP ? kDeepLds : kSmallLds<BM>;
   static bool reserved = false;
-  if (int rc = reserve_lds(fp8_gemm_small_pair_kernel<BM>, kSmallLds<BM>, reserved)) return rc;
+  auto kernel = fp8_gemm_small_pair_kernel<BM, DEEP>;
+  if (int rc = reserve_lds(kernel, lds, reserved)) return rc;
   GemmPair q = {{a, b}, 0};
   count_small_tiles<GEMM_DENSE, BM>(q.g[0]);
   count_small_tiles<GEMM_DENSE, BM>(q.g[1]);
   q.second = (int)(cdiv(q.g[0].total_tiles, 8) * 8);
-  hipLaunchKernelGGL(fp8_gemm_small_pair_kernel<BM>, dim3((unsigned)(q.second + cdiv(q.g[1].total_tiles, 8) * 8)), dim3(256), kSmallLds<BM>, stream, q);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(q.second + cdiv(q.g[1].total_tiles, 8) * 8)), dim3(DEEP ? 512 : 256), lds, stream, q);
   return check_launch("fp8_gemm_small_pair_kernel");
 }
 
 int launch_gemm_small_pair(const GemmArgs& a, const GemmArgs& b, int rows, hipStream_t stream) {
-  PT_REQUIRE(rows == 64 || rows == 128, "gemm: the small-problem kernel has tiles of 64 or 128 rows");
-  return rows == 64 ? launch_pair<64>(a, b, stream) : launch_pair<128>(a, b, stream);
+  PT_REQUIRE(rows == 64 || rows == 128 || rows == kDeepTile, "gemm: the small-problem kernel has tiles of 64 or 128 rows");
+  return rows == 64 ? launch_pair<64>(a, b, stream) : rows == 128 ? launch_pair<128>(a, b, stream) : launch_pair<128, true>(a, b, stream);
+}
+
+static int launch_deep(GemmArgs a, hipStream_t stream) {
+  static bool reserved = false;
+  if (int rc = reserve_lds(fp8_gemm_deep_kernel, kDeepLds, reserved)) return rc;
+  count_small_tiles<GEMM_DENSE, 128>(a);
+  if (a.total_tiles == 0) return PT_OK;
+  hipLaunchKernelGGL(fp8_gemm_deep_kernel, dim3((unsigned)(cdiv(a.total_tiles, 8) * 8)), dim3(512), kDeepLds, stream, a);
+  return check_launch("fp8_gemm_deep_kernel");
 }
 
 template <int MODE, int BM, bool ACC, bool BT, bool STREAM = false>
@@ -317,6 +337,10 @@ static int launch_small_mode(const GemmArgs& a, hipStream_t stream) {
 }
 
 int launch_gemm_small(const GemmArgs& a, int rows, hipStream_t stream) {
+  if (rows == kDeepTile) {
+    if (a.mode == GEMM_DENSE) return launch_deep(a, stream);
+    rows = 128;
+  }
   PT_REQUIRE(rows == 64 || rows == 128, "gemm: the small-problem kernel has tiles of 64 or 128 rows");
   return rows == 64 ? launch_small_mode<64>(a, stream) : launch_small_mode<128>(a, stream);
 }

@@ -79,6 +79,34 @@ def test_grouped(rows, n, k, form):
     _same_bits(lambda: m_grouped_fp8_gemm_nn((a, sa), (b, sb), out, offs, index), out, "r0")
 
 
+@pytest.mark.parametrize("m,n,k", [(1001, 4096, 1792), (4090, 1000, 2064), (129, 8, 4096), (1, 16, 1808)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_one_deep_workgroup_per_unit(m, n, k, dtype):
+    """The form of the 128-row tiles with eight waves and four stages, forced and where the library picks it: the bits of the
+    large tiles', with ragged rows, columns and reductions, more stages than blocks left over at the end, one row."""
+    from pith_train_amd import _lib
+
+    g = torch.Generator().manual_seed(m)
+    a, sa, b, sb = _fp8(g, m, k), _scale(g, m, _cdiv(k, 128)), _fp8(g, n, k), _scale(g, _cdiv(n, 128), _cdiv(k, 128))
+    results = []
+    try:
+        for kernel in (b"r0", b"s128d", b"auto"):
+            _lib.call("pt_gemm_select_kernel", kernel)
+            results.append(torch.full((m, n), 0.5, device="cuda", dtype=dtype))
+            _lib.call("pt_gemm_nt_dense", a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), results[-1].data_ptr(), _lib.dtype_code(dtype),
+                      m, n, k, _lib.stream_ptr())
+    finally:
+        _lib.call("pt_gemm_select_kernel", None)
+    assert all(torch.equal(r, results[0]) for r in results)
+
+
+@pytest.mark.parametrize("first,second", [((4000, 512, 4096), (4096, 512, 4000)), ((700, 2048, 2048), (2048, 2048, 704)), ((901, 2048, 4096), (4096, 2048, 912)),
+                                          ((300, 4096, 2064), (2056, 4096, 304))])
+def test_two_products_of_deep_tiles(first, second):
+    """Pairs of long and short reductions at the rule's two sides: the bits of two launches."""
+    test_two_products_in_one_launch(first, second, torch.bfloat16)
+
+
 @pytest.mark.parametrize("first,second", [((1, 16, 16), (70, 24, 144)), ((1001, 2048, 512), (512, 2048, 1008)), ((640, 264, 400), (129, 1000, 272)),
                                           ((2048, 2048, 256), (2048, 2048, 128)), ((4096, 2048, 128), (128, 128, 128))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
