@@ -152,6 +152,13 @@ int pt_quant_heads_rowwise_transpose_ld(const void* x, const void* x2, int64_t M
                                         int64_t head_a, int64_t head_b, void* tok_fp8, float* tok_scale,
                                         void* t_fp8, int64_t ld_t, float* t_scale, pt_stream_t stream);
 
+/* The same and pt_quant_rowwise_blockwise_transpose_ld's transposed results alone of a bf16 input [M, K] (row stride
+ * ld_input, the same ld_t), in one launch: what the backward of a latent projection quantises. */
+int pt_quant_heads_and_input(const void* x, const void* x2, int64_t M, int64_t heads, int64_t head_a, int64_t head_b,
+                             void* tok_fp8, float* tok_scale, void* t_fp8, int64_t ld_t, float* t_scale,
+                             const void* input, int64_t K, int64_t ld_input, void* blk_t_fp8, float* blk_t_scale,
+                             pt_stream_t stream);
+
 /* rowwise(x) + 128x128 blockwise(x^T): blk_t_fp8[K,M], blk_t_scale[ceil(K/128),ceil(M/128)].
  * fp8cast_rowwise_blockwise_transpose, deepgemm_quantize.py:575-629 */
 int pt_quant_rowwise_blockwise_transpose(const void* x, int dtype, int64_t M, int64_t K,

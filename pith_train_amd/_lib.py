@@ -43,6 +43,7 @@ SIGNATURES = {
     "pt_quant_rowwise_transpose_ld": (c_int, [P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_rowwise_blockwise_transpose_ld": (c_int, [P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_heads_rowwise_transpose_ld": (c_int, [P, P, I64, I64, I64, I64, P, P, P, I64, P, P]),
+    "pt_quant_heads_and_input": (c_int, [P, P, I64, I64, I64, I64, P, P, P, I64, P, P, I64, I64, P, P, P]),
     "pt_quant_dense_operands": (c_int, [c_char_p, I32, P, c_int, I64, I64, I64, P, P, P, I64, P, P]),
     "pt_quant_linear_operands": (c_int, [P, P, c_int, I64, I64, I64, I64, I64, P, P, P, I64, P, P, P, P, P, P]),
     "pt_quant_blockwise_transpose_batched": (c_int, [P, c_int, I64, I64, I64, I64, I64, P, P, P, P, P]),

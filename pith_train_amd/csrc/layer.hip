@@ -275,19 +275,25 @@ extern "C" int pt_linear_backward(const pt_linear_backward_args* args) {
   const void* x_t = a.x_t;
   const float* x_ts = a.x_t_scale;
   int64_t ld_xt = a.ld_xt;
+  bool quantised = false;
   if (!x_t) {
     void* t = ws.bytes(a.K * (a.M + 384));
     float* ts = ws.floats(cdiv(a.K, 128) * cdiv(a.M, 128));
     ld_xt = ld_t;
-    PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, nullptr, nullptr, t, ld_xt, ts, a.stream);
+    quantised = a.grad2 && a.dtype == PT_BF16;  // the gradients with it
+    if (quantised)
+      PT_STEP(pt_quant_heads_and_input, a.M, a.N, a.M, a.grad, a.grad2, a.M, a.N / (a.head_a + a.head_b), a.head_a, a.head_b, g_fp8, g_s, g_t, ld_t, g_ts,
+              a.x, a.K, a.ldx, t, ts, a.stream);
+    else
+      PT_STEP(pt_quant_rowwise_blockwise_transpose_ld, a.M, a.K, a.M, a.x, (int)a.dtype, a.M, a.K, a.ldx, nullptr, nullptr, t, ld_xt, ts, a.stream);
     x_t = t;
     x_ts = ts;
   }
   float* slabs = (float*)(void*)ws.p;
-  if (a.grad2)
+  if (!quantised && a.grad2)
     PT_STEP(pt_quant_heads_rowwise_transpose_ld, a.M, a.N, a.M, a.grad, a.grad2, a.M, a.N / (a.head_a + a.head_b), a.head_a, a.head_b, g_fp8,
             g_s, g_t, ld_t, g_ts, a.stream);
-  else
+  else if (!quantised)
     PT_STEP(pt_quant_rowwise_transpose_ld, a.M, a.N, a.M, a.grad, (int)a.dtype, a.M, a.N, a.ldg, g_fp8, g_s, g_t, ld_t, g_ts, a.stream);
   const pt_dense_gemm two[2] = {{g_fp8, a.N, g_s, a.w_t_fp8, a.N, a.w_t_scale, a.grad_x, a.M, a.K, a.N},
                                 {g_t, ld_t, g_ts, x_t, ld_xt, x_ts, a.grad_w, a.N, a.K, red}};

@@ -699,6 +699,42 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
   }
 }
 
+// Row and column tile (and group) of workgroup `bid`.
+// Row-scaled launches (one group): which XCD runs which tile decides whether the 4-byte scale
+// writes merge into whole lines.  Row scales are [M, tiles_n] floats (or [tiles_n, M], whole lines of a tile), so the
+// column tiles of one row block write neighbouring floats; column scales in the [N, tiles_m] layout put the same
+// column of neighbouring row blocks next to each other.  Workgroup b runs on XCD b % 8: with the
+// column tile as the fastest index all of those writes would meet in eight different L2s and
+// leave as one 32-byte sector per float (8x their bytes; 12 % of the kernel's write traffic).
+// So XCD x takes octets of row blocks (octet o with o % 8 == x) and runs an octet's tiles back
+// to back, the eight row blocks of a column tile first: both kinds of neighbours are written by
+// one XCD within a few microseconds and merge in its L2.  Row blocks that do not fill eight
+// octets are dealt singly (row block r to XCD r % 8, its column tiles back to back: the row
+// scales still merge), the last tiles_m % 8 in plain order.
+template <int AM>
+__device__ __forceinline__ void place_tile(int64_t bid, int tiles_m, int tiles_n, int& tr, int& tc, int64_t& g) {
+  const int64_t per_oct = 8 * (int64_t)tiles_n;
+  const int oct_rows = ((tiles_m >> 3) & ~7) * 8;  // row blocks in whole rounds of eight octets
+  const int64_t oct_region = (int64_t)oct_rows * tiles_n;
+  const int64_t remapped = (int64_t)(tiles_m & ~7) * tiles_n;
+  g = 0;
+  if (AM == A_ROW && bid < oct_region) {
+    const int64_t s = bid >> 3;
+    const int64_t o = (s / per_oct) * 8 + (bid & 7);
+    const int r = (int)(s % per_oct);
+    tc = r >> 3;
+    tr = (int)o * 8 + (r & 7);
+  } else if (AM == A_ROW && bid < remapped) {
+    const int64_t b2 = bid - oct_region, s = b2 >> 3;
+    tc = (int)(s % tiles_n);
+    tr = oct_rows + (int)(s / tiles_n) * 8 + (int)(b2 & 7);
+  } else {
+    tc = (int)(bid % tiles_n); bid /= tiles_n;
+    tr = (int)(bid % tiles_m);
+    g = bid / tiles_m;
+  }
+}
+
 // Register budget: the kernel is bound by memory latency, so resident waves matter more than
 // keeping every load of a tile in flight at once (which is what the compiler does when it is given
 // the whole register file: 256 registers and one wave per SIMD for the paired SwiGLU backward).
@@ -710,42 +746,12 @@ void quant_tile_kernel(QuantArgs p) {
   __shared__ __attribute__((aligned(16))) uint8_t s_t[128 * 128];
   __shared__ float s_colsum[writes_sums(PRO) ? 4 : 1][128];
 
-  int64_t bid = blockIdx.x;
   // PRO_SILU_BWD_PAIR: one workgroup produces the dgate tile and its dup twin (half / 128 column
   // tiles further right) from one read of grad_h, gate and up
   const int tiles_n_grid = PRO == PRO_SILU_BWD_PAIR ? p.tiles_n / 2 : p.tiles_n;
-  // Row-scaled launches (one group): which XCD runs which tile decides whether the 4-byte scale
-  // writes merge into whole lines.  Row scales are [M, tiles_n] floats (or [tiles_n, M], whole lines of a tile), so the
-  // column tiles of one row block write neighbouring floats; column scales in the [N, tiles_m] layout put the same
-  // column of neighbouring row blocks next to each other.  Workgroup b runs on XCD b % 8: with the
-  // column tile as the fastest index all of those writes would meet in eight different L2s and
-  // leave as one 32-byte sector per float (8x their bytes; 12 % of the kernel's write traffic).
-  // So XCD x takes octets of row blocks (octet o with o % 8 == x) and runs an octet's tiles back
-  // to back, the eight row blocks of a column tile first: both kinds of neighbours are written by
-  // one XCD within a few microseconds and merge in its L2.  Row blocks that do not fill eight
-  // octets are dealt singly (row block r to XCD r % 8, its column tiles back to back: the row
-  // scales still merge), the last tiles_m % 8 in plain order.
   int tc, tr;
-  int64_t g = 0;
-  const int64_t per_oct = 8 * (int64_t)tiles_n_grid;
-  const int oct_rows = ((p.tiles_m >> 3) & ~7) * 8;  // row blocks in whole rounds of eight octets
-  const int64_t oct_region = (int64_t)oct_rows * tiles_n_grid;
-  const int64_t remapped = (int64_t)(p.tiles_m & ~7) * tiles_n_grid;
-  if (AM == A_ROW && bid < oct_region) {
-    const int64_t s = bid >> 3;
-    const int64_t o = (s / per_oct) * 8 + (bid & 7);
-    const int r = (int)(s % per_oct);
-    tc = r >> 3;
-    tr = (int)o * 8 + (r & 7);
-  } else if (AM == A_ROW && bid < remapped) {
-    const int64_t b2 = bid - oct_region, s = b2 >> 3;
-    tc = (int)(s % tiles_n_grid);
-    tr = oct_rows + (int)(s / tiles_n_grid) * 8 + (int)(b2 & 7);
-  } else {
-    tc = (int)(bid % tiles_n_grid); bid /= tiles_n_grid;
-    tr = (int)(bid % p.tiles_m);
-    g = bid / p.tiles_m;
-  }
+  int64_t g;
+  place_tile<AM>(blockIdx.x, p.tiles_m, tiles_n_grid, tr, tc, g);
   // The caller may size the tensors for the largest row count a routing can produce and tell the
   // real one through device memory (no host round trip): tiles past it have nothing to do.
   if (p.row_limit && (int64_t)tr * 128 >= *p.row_limit) return;
@@ -809,6 +815,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void q
   } else {
     if (full) quant_tile_body<T, A_ROW, B_BLOCK, BL_TRANSPOSED, BS_MB_N, PRO_NONE, true>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
     else      quant_tile_body<T, A_ROW, B_BLOCK, BL_TRANSPOSED, BS_MB_N, PRO_NONE, false>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
+  }
+}
+
+// The gradients of a latent projection, given per head in two tensors (row scales and the transposed form), and the transposed
+// form of its input in one launch, both bf16: the input's tiles, an eighth of the others, come last (4096 rows, 512 and 4096 wide:
+// 15.3 + 4.4 us).
+struct QuantHeadsArgs { QuantArgs grad, x; };
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void quant_heads_kernel(QuantHeadsArgs q) {
+  __shared__ float s_colmax[4][128];
+  __shared__ float s_blk[4];
+  __shared__ __attribute__((aligned(16))) uint8_t s_t[128 * 128];
+  const int64_t first = (int64_t)q.grad.tiles_m * q.grad.tiles_n;
+  const bool input = (int64_t)blockIdx.x >= first;
+  const QuantArgs& p = input ? q.x : q.grad;
+  int tc, tr;
+  int64_t g;
+  place_tile<A_ROW>(input ? blockIdx.x - first : blockIdx.x, p.tiles_m, p.tiles_n, tr, tc, g);
+  const bool full = (int64_t)tr * 128 + 128 <= p.M && (int64_t)tc * 128 + 128 <= p.N && p.vec_in && p.vec_out && p.vec_out_t;
+  if (input) {
+    if (full) quant_tile_body<bf16_tag, A_ROW, B_BLOCK, BL_TRANSPOSED, BS_MB_N, PRO_NONE, true>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
+    else      quant_tile_body<bf16_tag, A_ROW, B_BLOCK, BL_TRANSPOSED, BS_MB_N, PRO_NONE, false>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
+  } else {
+    if (full) quant_tile_body<bf16_tag, A_ROW, B_COL, BL_TRANSPOSED, BS_N_MB, PRO_HEADS, true>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
+    else      quant_tile_body<bf16_tag, A_ROW, B_COL, BL_TRANSPOSED, BS_N_MB, PRO_HEADS, false>(p, s_colmax, s_blk, s_t, nullptr, tc, tr, 0);
   }
 }
 
@@ -968,41 +998,65 @@ extern "C" int pt_quant_rowwise_transpose_ld(const void* x, int dtype, int64_t M
   return quant_rowwise_transpose_impl(x, dtype, M, N, ldx, tok_fp8, tok_scale, t_fp8, ld_t, t_scale, stream);
 }
 
-extern "C" int pt_quant_heads_rowwise_transpose_ld(const void* x, const void* x2, int64_t M, int64_t heads, int64_t head_a, int64_t head_b,
-                                                   void* tok_fp8, float* tok_scale, void* t_fp8, int64_t ld_t, float* t_scale,
-                                                   pt_stream_t stream) {
+static int fill_heads(QuantArgs& a, const void* x, const void* x2, int64_t M, int64_t heads, int64_t head_a, int64_t head_b, void* tok_fp8,
+                      float* tok_scale, void* t_fp8, int64_t ld_t, float* t_scale) {
   const int64_t N = heads * (head_a + head_b);
   PT_REQUIRE(M >= 0 && heads >= 0 && head_a > 0 && head_b > 0 && N < (1ll << 31) && ld_t >= M, "quant_heads_rowwise_transpose: bad shape");
-  if (M == 0 || N == 0) return PT_OK;
-  PT_REQUIRE(x && x2 && tok_fp8 && tok_scale && t_fp8 && t_scale, "quant_heads_rowwise_transpose: null pointer");
-  PT_REQUIRE(head_a % 8 == 0 && head_b % 8 == 0 && (((uintptr_t)x | (uintptr_t)x2) & 15) == 0,
+  PT_REQUIRE(M == 0 || N == 0 || (x && x2 && tok_fp8 && tok_scale && t_fp8 && t_scale), "quant_heads_rowwise_transpose: null pointer");
+  PT_REQUIRE(M == 0 || N == 0 || (head_a % 8 == 0 && head_b % 8 == 0 && (((uintptr_t)x | (uintptr_t)x2) & 15) == 0),
              "quant_heads_rowwise_transpose: head widths must be multiples of 8 elements, pointers 16-byte aligned");
-  QuantArgs a;
   fill_common(a, x, PT_BF16, M, N, N);
   a.x2 = x2; a.head_a = (int32_t)head_a; a.head_b = (int32_t)head_b;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)t_fp8; a.b_scale = t_scale;
   a.ld_t = ld_t;
   a.vec_out_t = whole_chunks(M, ld_t, t_fp8);
-  const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
-  PT_REQUIRE(blocks < (1ll << 31), "quant: grid too large (%lld tiles)", (long long)blocks);
-  hipLaunchKernelGGL((quant_tile_kernel<bf16_tag, A_ROW, B_COL, BL_TRANSPOSED, BS_N_MB, PRO_HEADS>), dim3((unsigned)blocks), dim3(256), 0,
+  PT_REQUIRE((int64_t)a.tiles_m * a.tiles_n < (1ll << 30), "quant: grid too large (%lld tiles)", (long long)a.tiles_m * a.tiles_n);
+  return PT_OK;
+}
+
+extern "C" int pt_quant_heads_rowwise_transpose_ld(const void* x, const void* x2, int64_t M, int64_t heads, int64_t head_a, int64_t head_b,
+                                                   void* tok_fp8, float* tok_scale, void* t_fp8, int64_t ld_t, float* t_scale,
+                                                   pt_stream_t stream) {
+  QuantArgs a;
+  if (int rc = fill_heads(a, x, x2, M, heads, head_a, head_b, tok_fp8, tok_scale, t_fp8, ld_t, t_scale)) return rc;
+  if (M == 0 || heads == 0) return PT_OK;
+  hipLaunchKernelGGL((quant_tile_kernel<bf16_tag, A_ROW, B_COL, BL_TRANSPOSED, BS_N_MB, PRO_HEADS>), dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(256), 0,
                      (hipStream_t)stream, a);
   return check_launch("quant_tile_kernel(heads)");
+}
+
+static int fill_rowwise_blockwise_transpose(QuantArgs& a, const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, void* tok_fp8, float* tok_scale,
+                                            void* blk_t_fp8, int64_t ld_t, float* blk_t_scale) {
+  PT_REQUIRE(M >= 0 && K >= 0 && ldx >= K && ld_t >= M, "quant_rowwise_blockwise_transpose: bad shape");
+  PT_REQUIRE(M == 0 || K == 0 || (x && (tok_fp8 == nullptr) == (tok_scale == nullptr) && (blk_t_fp8 == nullptr) == (blk_t_scale == nullptr) &&
+                                  (tok_fp8 || blk_t_fp8)), "quant_rowwise_blockwise_transpose: null pointer");
+  fill_common(a, x, dtype, M, K, ldx);
+  a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)blk_t_fp8; a.b_scale = blk_t_scale;
+  a.ld_t = ld_t;
+  a.vec_out_t = whole_chunks(M, ld_t, blk_t_fp8);
+  return PT_OK;
 }
 
 static int quant_rowwise_blockwise_transpose_impl(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, void* tok_fp8,
                                                   float* tok_scale, void* blk_t_fp8, int64_t ld_t, float* blk_t_scale,
                                                   pt_stream_t stream) {
-  PT_REQUIRE(M >= 0 && K >= 0 && ldx >= K && ld_t >= M, "quant_rowwise_blockwise_transpose: bad shape");
-  if (M == 0 || K == 0) return PT_OK;
-  PT_REQUIRE(x && (tok_fp8 == nullptr) == (tok_scale == nullptr) && (blk_t_fp8 == nullptr) == (blk_t_scale == nullptr) && (tok_fp8 || blk_t_fp8),
-             "quant_rowwise_blockwise_transpose: null pointer");
   QuantArgs a;
-  fill_common(a, x, dtype, M, K, ldx);
-  a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)blk_t_fp8; a.b_scale = blk_t_scale;
-  a.ld_t = ld_t;
-  a.vec_out_t = whole_chunks(M, ld_t, blk_t_fp8);
+  if (int rc = fill_rowwise_blockwise_transpose(a, x, dtype, M, K, ldx, tok_fp8, tok_scale, blk_t_fp8, ld_t, blk_t_scale)) return rc;
+  if (M == 0 || K == 0) return PT_OK;
   return launch_quant<A_ROW, B_BLOCK, BL_TRANSPOSED, BS_MB_N>(a, dtype, 1, (hipStream_t)stream);
+}
+
+extern "C" int pt_quant_heads_and_input(const void* x, const void* x2, int64_t M, int64_t heads, int64_t head_a, int64_t head_b, void* tok_fp8,
+                                        float* tok_scale, void* t_fp8, int64_t ld_t, float* t_scale, const void* input, int64_t K, int64_t ld_input,
+                                        void* blk_t_fp8, float* blk_t_scale, pt_stream_t stream) {
+  QuantHeadsArgs q;
+  if (int rc = fill_heads(q.grad, x, x2, M, heads, head_a, head_b, tok_fp8, tok_scale, t_fp8, ld_t, t_scale)) return rc;
+  if (int rc = fill_rowwise_blockwise_transpose(q.x, input, PT_BF16, M, K, ld_input, nullptr, nullptr, blk_t_fp8, ld_t, blk_t_scale)) return rc;
+  const int64_t blocks = (int64_t)q.grad.tiles_m * q.grad.tiles_n + (int64_t)q.x.tiles_m * q.x.tiles_n;
+  if (M == 0 || blocks == 0) return PT_OK;
+  PT_REQUIRE(blocks < (1ll << 31), "quant: grid too large (%lld tiles)", (long long)blocks);
+  hipLaunchKernelGGL(quant_heads_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, q);
+  return check_launch("quant_heads_kernel");
 }
 
 extern "C" int pt_quant_rowwise_blockwise_transpose(const void* x, int dtype, int64_t M, int64_t K,

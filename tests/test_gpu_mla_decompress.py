@@ -77,3 +77,32 @@ def test_per_head_halves_have_the_bits_of_the_concatenated_tensors(rows, heads, 
     want = L.fp8_dgrad_wgrad(torch.cat([dk, dv], -1).view(rows, n), w_t, w_t_s, x_t, x_t_s, rank, _zero_padded=True)
     # the concatenated way rounds to bf16 before it widens
     assert torch.equal(d_x[0].bfloat16(), want[0]) and torch.equal(d_w.bfloat16(), want[1])
+
+
+@pytest.mark.parametrize("rows,heads,nope,vdim,rank", [(1, 1, 8, 8, 16), (257, 3, 24, 40, 144), (8321, 2, 64, 72, 136)])
+def test_gradients_and_latent_quantised_in_one_launch(rows, heads, nope, vdim, rank):
+    """Against the two launches that it stands for: ragged tiles on every side, one tile, and row blocks in whole octets
+    with some left over; the latent's rows lie in a wider buffer."""
+    from pith_train_amd import _lib
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    n, pitch, row_blocks = heads * (nope + vdim), (rows + 15) // 16 * 16 + 128, -(-rows // 128)
+
+    def normal(*shape):
+        return torch.randn(shape, device="cuda", generator=g).bfloat16()
+
+    dk, dv, x = normal(rows, heads * nope), normal(rows, heads * vdim), normal(rows, rank + 8)
+    results = []
+    for together in (False, True):
+        byte = lambda *s: torch.zeros(s, dtype=torch.uint8, device="cuda")  # noqa: E731
+        q, q_t, x_t = byte(rows, n), byte(n, pitch), byte(rank, pitch)
+        s, s_t, xs = (torch.zeros(z, device="cuda") for z in ((rows, -(-n // 128)), (n, row_blocks), (-(-rank // 128), row_blocks)))
+        results.append((q, q_t, x_t, s, s_t, xs))
+        grads = [_lib.ptr(dk), _lib.ptr(dv), rows, heads, nope, vdim, _lib.ptr(q), _lib.ptr(s), _lib.ptr(q_t), pitch, _lib.ptr(s_t)]
+        if together:
+            _lib.call("pt_quant_heads_and_input", *grads, _lib.ptr(x), rank, rank + 8, _lib.ptr(x_t), _lib.ptr(xs), _lib.stream_ptr())
+        else:
+            _lib.call("pt_quant_heads_rowwise_transpose_ld", *grads, _lib.stream_ptr())
+            _lib.call("pt_quant_rowwise_blockwise_transpose_ld", _lib.ptr(x), _lib.PT_BF16, rows, rank, rank + 8, None, None, _lib.ptr(x_t), pitch, _lib.ptr(xs),
+                      _lib.stream_ptr())
+    assert all(torch.equal(a, b) for a, b in zip(*results)) and all(t.float().abs().sum() > 0 for t in results[0])
