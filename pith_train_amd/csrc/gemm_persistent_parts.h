@@ -607,6 +607,7 @@ __device__ __forceinline__ void decode_tile(const GemmArgs& p, const int* s_pref
 
 // Writes one wave's TM x TN blocks of 32 x 32 results of tile T (rows wm0.., columns wn0.. of the
 // tile).  `piece`: the LDS addresses of the wave's four 1 KiB pieces of staging.
+// PAIR: the result has two outputs (k-grouped: where the arguments say so).
 // EXTRAS: the output rows (out_row_index) and the bias of the tile lie in LDS, row wm0 and column wn0 of
 // the tile's at LDS bytes rows_lds + 4 wm0 and bias_lds + 2 wn0: a load here would wait for every store before it.
 template <int MODE, int TM, int TN, bool ACC, bool PAIR = false, bool EXTRAS = false>
@@ -659,7 +660,7 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[TM][TN], const Gemm
         store16<AUX>(w, rs_heads, colc < T.b_lim && r < row_lim ? (uint32_t)r * pitch_h + at : kOob, 0);
       });
     }
-  } else if (MODE == GEMM_M_GROUPED && p.out_row_index) {
+  } else if (MODE == GEMM_M_GROUPED && (PAIR || p.out_row_index)) {
     // Result row r goes to output row out_row_index[r] (the un-permute folded into the store);
     // rows of the group's padding map to a negative index and are dropped.
     const __amdgpu_buffer_rsrc_t rs_sc = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, kAblateStores ? 0 : (int)((uint32_t)p.out_rows * pitch), kRsrcFlags);
@@ -672,7 +673,7 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[TM][TN], const Gemm
       else dst[i] = p.out_row_index[r < T.a_lim ? r : T.a_row0];
       if (r >= T.a_lim) dst[i] = -1;
     }
-    if (p.out2) {
+    if constexpr (PAIR) {
       // Two outputs, -2 - r for row r of the second: 64-bit addresses, since no descriptor spans both.  (Rows of an
       // input gradient that nobody else adds to go to their place at once, see pt_gather_rows_backward_begin.)
       if (kAblateStores) return;
@@ -685,17 +686,17 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[TM][TN], const Gemm
           if (row != -1 && colc < T.b_lim) __builtin_nontemporal_store(w, (v4i*)to);
         });
       }
-      return;
-    }
+    } else {
 #pragma unroll
-    for (int j = 0; j < TN; j += 2) {
-      const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;
-      const v4i bias = bias_of(j, colc);
-      stage_column<false>(acc, j, stg, lane, [&](int i, int q, v4i w) {
-        const int row = __shfl(dst[i], q * 8 + (lane >> 3));
-        store16<AUX>(p.bias ? add_bf16(w, bias) : w, rs_sc, row >= 0 && colc < T.b_lim ? (uint32_t)row * pitch + (uint32_t)(lane & 7) * 16 : kOob,
-                     (uint32_t)(T.b_row0 + wn0 + j * 32) * 2);
-      });
+      for (int j = 0; j < TN; j += 2) {
+        const int colc = T.b_row0 + wn0 + j * 32 + (lane & 7) * 8;
+        const v4i bias = bias_of(j, colc);
+        stage_column<false>(acc, j, stg, lane, [&](int i, int q, v4i w) {
+          const int row = __shfl(dst[i], q * 8 + (lane >> 3));
+          store16<AUX>(p.bias ? add_bf16(w, bias) : w, rs_sc, row >= 0 && colc < T.b_lim ? (uint32_t)row * pitch + (uint32_t)(lane & 7) * 16 : kOob,
+                       (uint32_t)(T.b_row0 + wn0 + j * 32) * 2);
+        });
+      }
     }
   } else if (p.out_dtype != PT_F32 && wide_ok) {
     const bool has_bias = MODE == GEMM_M_GROUPED && p.bias != nullptr;

@@ -63,7 +63,8 @@ static_assert(kRsLds <= 160 * 1024 && kRsPref % 16 == 0, "LDS map");
 
 // BT: the b operand is given reduction-major, [red][rows_b] with row pitch ldb (the forward layout of
 // a weight, read by its input-gradient GEMM), instead of [rows_b][red].
-// PAIR (k-grouped): the result rows from split_row on go to a second output.
+// PAIR: two outputs (k-grouped: the result rows from split_row on go to the second; m-grouped: out_row_index says which).
+// A kernel of its own, so that every other launch keeps its code without a further form of the store.
 template <int MODE, int BM, int BN, int WGM, int WGN, bool ACC, bool BT = false, bool PAIR = false>
 __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel(GemmArgs) {
   constexpr int NW = WGM * WGN;
@@ -460,6 +461,9 @@ static int launch_mode(const GemmArgs& a, hipStream_t stream) {
   switch (a.mode) {
     case GEMM_DENSE: return launch_one<GEMM_DENSE, BM, BN, WGM, WGN, false>(a, stream);
     case GEMM_M_GROUPED:
+      if (a.out2)
+        return a.b_kmajor ? launch_one<GEMM_M_GROUPED, BM, BN, WGM, WGN, false, true, true>(a, stream)
+                          : launch_one<GEMM_M_GROUPED, BM, BN, WGM, WGN, false, false, true>(a, stream);
       return a.b_kmajor ? launch_one<GEMM_M_GROUPED, BM, BN, WGM, WGN, false, true>(a, stream)
                         : launch_one<GEMM_M_GROUPED, BM, BN, WGM, WGN, false>(a, stream);
     default:

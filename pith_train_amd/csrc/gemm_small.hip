@@ -29,8 +29,8 @@ static constexpr int kDeepStages = 4;
 static constexpr size_t kDeepLds = (size_t)kDeepStages * (128 + 128) * (128 + 4) + 256;
 template <int BM> static constexpr size_t kSmallLds = (size_t)kSmallStages<BM> * (BM + 128) * (128 + 4) + 256;
 
-// STREAM: the loads of b pass the memory-side cache by (launch_small_mode has the rule and both sides).
-template <int MODE, int BM, bool ACC, bool BT, bool STREAM = false, bool DEEP = false>
+// STREAM: the loads of b pass the memory-side cache by (launch_small_mode has the rule and both sides).  TWO (m-grouped): two outputs.
+template <int MODE, int BM, bool ACC, bool BT, bool STREAM = false, bool DEEP = false, bool TWO = false>
 __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
   constexpr int BN = 128, BK = 128, NS = DEEP ? kDeepStages : kSmallStages<BM>, NW = DEEP ? 8 : 4;
   static_assert(DEEP ? BM == 128 && kDeepLds <= 160 * 1024 : 2 * kSmallLds<BM> <= 160 * 1024, "one deep workgroup or two others per compute unit");
@@ -233,12 +233,12 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
   if (MODE == GEMM_K_GROUPED && nk == 0 && ACC) return;
   __syncthreads();  // every wave has read its last stage and has nothing in flight: the ring's memory is free
   const uint32_t stg = lds_base + wave * 4096, piece[4] = {stg, stg + 1024, stg + 2048, stg + 3072};
-  store_tile<MODE, TM, TN, ACC, MODE == GEMM_K_GROUPED>(acc, p, T, wm0, wn0, lane, piece);
+  store_tile<MODE, TM, TN, ACC, MODE == GEMM_K_GROUPED || TWO>(acc, p, T, wm0, wn0, lane, piece);
 }
 
-template <int MODE, int BM, bool ACC, bool BT, bool STREAM>
+template <int MODE, int BM, bool ACC, bool BT, bool STREAM, bool TWO>
 __global__ __launch_bounds__(256, 2) void fp8_gemm_small_kernel(GemmArgs p) {
-  small_tile_body<MODE, BM, ACC, BT, STREAM>(p, blockIdx.x);
+  small_tile_body<MODE, BM, ACC, BT, STREAM, false, TWO>(p, blockIdx.x);
 }
 
 __global__ __launch_bounds__(512, 2) void fp8_gemm_deep_kernel(GemmArgs p) {
@@ -299,11 +299,11 @@ static int launch_deep(GemmArgs a, hipStream_t stream) {
   return check_launch("fp8_gemm_deep_kernel");
 }
 
-template <int MODE, int BM, bool ACC, bool BT, bool STREAM = false>
+template <int MODE, int BM, bool ACC, bool BT, bool STREAM = false, bool TWO = false>
 static int launch_small(GemmArgs a, hipStream_t stream) {
   constexpr size_t lds = kSmallLds<BM>;
   static bool reserved = false;
-  auto kernel = fp8_gemm_small_kernel<MODE, BM, ACC, BT, STREAM>;
+  auto kernel = fp8_gemm_small_kernel<MODE, BM, ACC, BT, STREAM, TWO>;
   if (int rc = reserve_lds(kernel, lds, reserved)) return rc;
   count_small_tiles<MODE, BM>(a);
   if (a.total_tiles == 0) return PT_OK;
@@ -328,6 +328,9 @@ static int launch_small_mode(const GemmArgs& a, hipStream_t stream) {
       // no whole 128-byte lines shares one with the next (32 experts of 5760 x 2880: 127 us, 132 past the cache).
       if (BM == 64 && a.few_rows && a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0)
         return launch_small<GEMM_M_GROUPED, 64, false, false, true>(a, stream);
+      if (a.out2)
+        return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true, false, true>(a, stream)
+                          : launch_small<GEMM_M_GROUPED, BM, false, false, false, true>(a, stream);
       return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true>(a, stream)
                         : launch_small<GEMM_M_GROUPED, BM, false, false>(a, stream);
     default:
