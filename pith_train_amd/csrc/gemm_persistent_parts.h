@@ -374,21 +374,23 @@ __device__ __forceinline__ int xcd_first_tile(const GemmArgs& p, const int* s_pr
 // ---- k-grouped tiles of skewed groups -------------------------------------------------------------
 // Tiles of groups of 64 blocks and of one stand in the same list, so a cut of the list by cost that rounds to whole
 // rounds of workgroups, and dealing it out by count, leave workgroups idle where the largest tile is a good part of
-// a workgroup's share.  There every XCD takes an eighth of every group of big tiles (more than an eighth of a share each;
-// neighbours in the group's order, the remainders of the eighths in turn), and deals them out one by one, largest
-// first, to the workgroup that has the least.  The other groups stay together: their list is cut by cost, and the
-// workgroups of an XCD take its part in turns, one that has less so far the earlier, as if each took the next
-// tile when it is done.  All of it is the same arithmetic in every workgroup (one wave).  Weight gradients with
-// Zipf-distributed popularity, us: 8192 tokens of 6 in 64 groups 2816 x 2048 372 -> 317, 2048 x 1408 229 -> 172, of 8 in
-// 128 groups 1536 x 2048 325 -> 291; 16384 of 8 in 64 groups 518 -> 425.
+// a workgroup's share.  There an XCD deals out its big tiles one by one, largest first, to the workgroup that has
+// the least, and its workgroups take the small ones in turns, one that has less so far the earlier, as if each took
+// the next tile when it is done.  What an XCD's tiles are has two forms:
+//   eighths  every XCD takes an eighth of every group of big tiles (neighbours in the group's order, the remainders of
+//            the eighths in turn), and a part of the list of the other groups by cost
+//   parts    the whole list is cut by cost, as without a schedule but anywhere.  XCDs whose part is idle groups, which only
+//            store, then run beside XCDs that mostly multiply, where eighths have all of them multiply first and store last;
+//            but an XCD whose 32 workgroups get 33 big tiles of nearly a share each takes two rounds for them
+// All of it is the same arithmetic in every workgroup (one wave).
+enum Schedule { kInOrder, kEighths, kParts };
 static constexpr int kSchedGroups = 256;  // groups it is made for: four a lane
-static constexpr int kSchedPart = 8;
 static constexpr int kNoLoad = 0x3fffffff;
 struct KSchedule {  // in LDS
   int tiles[kSchedGroups + 1], cost[kSchedGroups + 1];  // of the small groups before g: tiles, and their cost
   int ahead[64];                                        // the XCD's workgroups: cost of their big tiles in small ones
   int big[128];                                         // this workgroup's big tiles: group * 2^22 + place in the group
-  int n_big, first, last, n;                            // how many; the XCD's small tiles; how many tiles in all
+  int n_big, first, n;                                  // how many; the XCD's first small tile; how many tiles in all
 };
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_min(int v) {
@@ -406,20 +408,32 @@ __device__ __forceinline__ int wave_scan(int v, int lane) {  // sum up to this l
   for (int d = 1; d < 64; d <<= 1) { const int y = __shfl_up(v, d); if (lane >= d) v += y; }
   return v;
 }
-// an XCD's tiles of a big group: from .. from + number
+// eighths: an XCD's tiles of a big group, from .. from + number
 __device__ __forceinline__ void xcd_share(int per_g, int xcd, int g, int& from, int& number) {
   const int y = (xcd + g) & 7;
   from = per_g * y >> 3;
   number = (per_g * (y + 1) >> 3) - from;
 }
-// Whether a launch is scheduled so: its largest tile makes a quarter of a workgroup's share, and that share 96 blocks (the
-// schedule takes 6 us and its rounds some more: shares of 60 and 87 blocks 87 -> 104 and 145 -> 163 us, of 15 40 -> 63;
-// largest tiles of 0.17 of a share 607 -> 719).  What the lists above can hold (a workgroup's share in big tiles
-// and one more); sums that stay below 2^29, a workgroup's below 2^22.
-__device__ __forceinline__ bool scheduled_groups(const GemmArgs& p, const int* s_pref, int workers) {
-  const int64_t per_g = (int64_t)p.tiles_a * p.tiles_b, total = s_pref[p.G] * per_g;
-  return p.offs && p.G <= kSchedGroups && workers <= 64 && per_g < (1 << 22) && total < (8ll << 22) * workers && total < (1ll << 29) && !level_groups(p, s_pref) &&
-         (int64_t)s_pref[p.G + 1] * 4 * 8 * workers >= total && total >= 96ll * 8 * workers;
+// Which form a launch takes, by the cost of its largest tile and a workgroup's share, in blocks.  Weight gradients with
+// Zipf-distributed popularity, us in order / eighths / parts, means of four orders of the same groups:
+//   results weigh as much as their products (a mean group costs up to 7.5 blocks): parts from shares of 96 on.  4293 tokens
+//     of 8 in 128 groups 1536 x 2048 - / 212 / 195, 6000 - / 246 / 224
+//   the largest tile is a whole share or more, so that no XCD has more big tiles than workgroups: parts from shares of 24
+//     on.  8942 of 8 in 128, 512 x 2048 133 / 136 / 106; 15000 264 / - / 204; 9000 of 8 in 16, 768 x 2048 143 / - / 122;
+//     30000 of 4 in 32, 1024 x 2048 344 / 343 / 312; 16384 of 8 in 64, 2048 x 768 251 / 258 / 226.  Shorter ones lose (share
+//     15: 40 -> 63), and so do shares of 28 and 29 whose largest tile is half or a third of one: 50 -> 57, 55 -> 74
+//   it is a quarter of a share of 96 or more: eighths.  8192 of 6 in 64, 2816 x 2048 419 / 354 / 376; 11686 of 8 in 128, 1024 x
+//     2048 - / 260 / 295; with smaller ones 607 -> 719, shares of 60 and 87 87 -> 104 and 145 -> 163
+// Limits: what the lists above can hold (a workgroup's big tiles are at most its share and one tile); sums that stay
+// below 2^29, a workgroup's below 2^22.
+__device__ __forceinline__ Schedule schedule_of(const GemmArgs& p, const int* s_pref, int workers) {
+  const int64_t per_g = (int64_t)p.tiles_a * p.tiles_b, total = s_pref[p.G] * per_g, all_workers = 8 * workers;
+  if (!p.offs || p.G > kSchedGroups || workers > 64 || per_g >= (1 << 22) || total >= (8ll << 22) * workers || total >= (1ll << 29)) return kInOrder;
+  if (level_groups(p, s_pref)) return kInOrder;
+  const int64_t largest = s_pref[p.G + 1] * all_workers;  // against total, as the tile against a share
+  if (total < 96 * all_workers) return total >= 24 * all_workers && largest >= total ? kParts : kInOrder;
+  if (largest * 4 < total) return kInOrder;
+  return largest >= total || 2 * s_pref[p.G] <= 15 * p.G ? kParts : kEighths;
 }
 // Place of workgroup `me`'s small tile j in the XCD's part of their list.  ahead: on lane w the big tiles of workgroup w
 // in small ones; tiles are taken in the order of (ahead + count so far, workgroup).
@@ -432,10 +446,15 @@ __device__ __forceinline__ int small_place(int ahead, int me, int workers, int j
   }
   return place;
 }
-// By the first wave; the caller waits for the workgroup.  `workers` workgroups an XCD, this one is `me`.
-__device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* s_pref, KSchedule& s, int xcd, int me, int workers, int lane) {
+// By the first wave; the caller waits for the workgroup.  `workers` workgroups an XCD, this one is `me`; parts: the XCD's
+// part of the list is t_first .. t_last.
+__device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* s_pref, KSchedule& s, bool parts, int xcd, int t_first, int t_last,
+                                                  int me, int workers, int lane) {
   const int per_g = p.tiles_a * p.tiles_b;
-  const int least = (int)((int64_t)s_pref[p.G] * per_g / (kSchedPart * 8 * workers)) + 1;  // cost of a big tile
+  // cost of a big tile: an eighth of a share; of shares from 140 on, which pay for a longer schedule, a sixteenth (16384
+  // tokens of 8 in 128 groups 1536 x 2048 532 -> 462 us; shares of 113 and 130 172 -> 178 and 208 -> 221)
+  const int64_t total = (int64_t)s_pref[p.G] * per_g, all_workers = 8 * workers;
+  const int least = (int)(total / ((total >= 140 * all_workers ? 16 : 8) * all_workers)) + 1;
   int cost[4];
   unsigned left = 0;  // the lane's groups of big tiles that have not been dealt out
 #pragma unroll
@@ -461,8 +480,17 @@ __device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* 
   }
   if (lane == 0) { s.tiles[kSchedGroups] = all_tiles; s.cost[kSchedGroups] = all; }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's own writes
-  int part;
-  {
+  int part, n_near = all_tiles, cost_near = all;  // small tiles whose mean cost the XCD's own have, and their cost
+  if (parts) {
+    // small tiles before a place of the list, and their cost, on lanes 0 and 1 for the two ends of the part
+    const int end = (lane & 1) ? t_last : t_first, g = end / per_g < kSchedGroups ? end / per_g : kSchedGroups - 1;
+    const int n = s.tiles[g + 1] - s.tiles[g], in_g = n ? end - g * per_g : 0;
+    const int below = s.tiles[g] + in_g, spent = s.cost[g] + (n ? in_g * ((s.cost[g + 1] - s.cost[g]) / n) : 0);
+    const int first = __builtin_amdgcn_readlane(below, 0);
+    n_near = part = __builtin_amdgcn_readlane(below, 1) - first;
+    cost_near = __builtin_amdgcn_readlane(spent, 1) - __builtin_amdgcn_readlane(spent, 0);
+    if (lane == 0) s.first = first;
+  } else {
     // number of tiles whose middle lies below y, on lanes 0 and 1 for the two ends of the part
     const int y = (int)((int64_t)all * (xcd + (lane & 1)) / 8);
     int lo = 0, hi = kSchedGroups - 1;  // last g with cost[g] <= y
@@ -474,7 +502,7 @@ __device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* 
     const int b = (2 * (y - s.cost[lo]) + c - 1) / (2 * c), below = s.tiles[lo] + (b < n ? b : n);
     const int first = __builtin_amdgcn_readlane(below, 0), last = xcd == 7 ? all_tiles : __builtin_amdgcn_readlane(below, 1);
     part = last - first;
-    if (lane == 0) { s.first = first; s.last = last; }
+    if (lane == 0) s.first = first;
   }
   // ---- the big ones ----
   int load = lane < workers ? 0 : kNoLoad, n_big = 0;
@@ -492,7 +520,12 @@ __device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* 
     if (lane == owner) left &= ~(1u << mine);
     const int g = 4 * owner + __builtin_amdgcn_readlane(mine, owner);
     int at, n;
-    xcd_share(per_g, xcd, g, at, n);
+    if (parts) {
+      at = t_first - g * per_g > 0 ? t_first - g * per_g : 0;
+      n = (t_last - g * per_g < per_g ? t_last - g * per_g : per_g) - at;
+    } else {
+      xcd_share(per_g, xcd, g, at, n);
+    }
     while (n > 0) {
       // every workgroup that would still be ahead of another with one more takes one; if there are too few, those with the least
       const int low = wave_min(load);
@@ -509,7 +542,7 @@ __device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* 
       n -= deal;
     }
   }
-  const int ahead = all_tiles ? (int)((float)load * ((float)all_tiles / (float)all) + 0.5f) : 0;
+  const int ahead = n_near ? (int)((float)load * ((float)n_near / (float)cost_near) + 0.5f) : 0;
   s.ahead[lane] = ahead;
   n_big = __builtin_amdgcn_readlane(n_big, me);
   if (lane == 0) s.n_big = n_big;

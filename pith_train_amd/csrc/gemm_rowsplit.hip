@@ -95,13 +95,13 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
   const int xcd = blockIdx.x & 7;
   // lanes 0 and 1 find the two ends of this XCD's share of the list side by side
   int t_step = gridDim.x >> 3;
-  const int t_cut = xcd_first_tile<MODE>(p, s_pref, total_tiles, xcd + (lane & 1), t_step);
+  const Schedule scheduled = MODE == GEMM_K_GROUPED ? schedule_of(p, s_pref, t_step) : kInOrder;
+  const int t_cut = xcd_first_tile<MODE>(p, s_pref, total_tiles, xcd + (lane & 1), scheduled ? 1 : t_step);
   int t_end = __builtin_amdgcn_readlane(t_cut, 1);
   int t_next = __builtin_amdgcn_readlane(t_cut, 0) + (blockIdx.x >> 3);
   KSchedule& sched = *(KSchedule*)(lds + kRsSched);
-  const bool scheduled = MODE == GEMM_K_GROUPED && scheduled_groups(p, s_pref, t_step);
   if (scheduled) {
-    if (tid < 64) schedule_k_groups(p, s_pref, sched, xcd, blockIdx.x >> 3, t_step, lane);
+    if (tid < 64) schedule_k_groups(p, s_pref, sched, scheduled == kParts, xcd, __builtin_amdgcn_readlane(t_cut, 0), t_end, blockIdx.x >> 3, t_step, lane);
     __syncthreads();
     t_next = 0;
     t_end = __builtin_amdgcn_readfirstlane(sched.n);

@@ -665,6 +665,47 @@ def test_grouped_work_lists_longer_than_the_tile_table(gemm_kernel):
     both(k_grouped)
 
 
+@pytest.mark.parametrize("groups,big,rest,N,W", [
+    (2, (300, 40), 0, 1024, 1280),      # fewer tiles than workgroups; XCD parts that end inside a group
+    (19, (90, 61, 33), 3, 1100, 1800),  # ragged tile grid, counts of groups and tiles that no eighth divides
+    (256, (130, 128, 90), 1, 512, 1024),  # as many groups as the schedule holds, the last ones idle
+    (64, (37, 36, 30), 5, 2816, 2048),  # results that weigh as much as their products, several big tiles a workgroup
+])
+def test_k_grouped_schedule_of_xcds_with_parts_of_the_list(gemm_kernel, groups, big, rest, N, W):
+    """Groups whose largest tile is a workgroup's share or more, and launches of many results over few rows: every XCD
+    deals out its own part of the list.  Every tile once (accumulating), with the bits of one small tile per workgroup."""
+    from pith_train_amd import _lib
+
+    if gemm_kernel != "auto":
+        pytest.skip("the test selects the kernels itself; run once")
+    g = torch.Generator(device="cuda").manual_seed(groups)
+    tiles = -(-N // 256) * -(-W // 256)
+    blocks = torch.randint(0, rest + 1, (groups,), generator=torch.Generator().manual_seed(groups))
+    for i, b in enumerate(big):
+        blocks[i * (groups // len(big))] = b
+    cost = blocks + 3
+    share = cost.sum().item() * tiles / 256
+    assert (share >= 24 and cost.max() >= share) or (share >= 96 and cost.max() * 4 >= share and cost.sum() <= 7.5 * groups), share  # the rule
+    offs, M = torch.cumsum(blocks * 128, 0).int().cuda(), int(blocks.sum()) * 128
+
+    def fp8(*shape):
+        return torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # finite values below 2
+
+    def scale(*shape):
+        return torch.exp2(torch.randint(-6, 3, shape, device="cuda", generator=g).float())
+
+    d, sd, x, sx = fp8(N, M), scale(M // 128, N), fp8(W, M), scale(M // 128, W)
+    start = torch.randn((groups, N, W), device="cuda", generator=g).bfloat16()
+    for add in (0, 1):
+        out = []
+        for kernel in ("s128", "r0"):
+            _lib.call("pt_gemm_select_kernel", kernel.encode())
+            out.append(start.clone())
+            _lib.call("pt_gemm_k_grouped_wgrad", _lib.ptr(d), _lib.ptr(sd), _lib.ptr(x), _lib.ptr(sx), _lib.ptr(out[-1]), _lib.dtype_code(torch.bfloat16),
+                      add, _lib.ptr(offs), groups, M, N, W, _lib.stream_ptr())
+        assert torch.equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("groups,half,W", [(40, 640, 1800), (256, 896, 2200)])
 def test_k_grouped_schedule_with_two_outputs_and_a_second_table(gemm_kernel, groups, half, W):
     """The rows of a gate and of an up projection go to two gradients, whose border lies inside a row of tiles, under the
