@@ -377,11 +377,10 @@ __device__ __forceinline__ int xcd_first_tile(const GemmArgs& p, const int* s_pr
 // a workgroup's share.  There an XCD deals out its big tiles one by one, largest first, to the workgroup that has
 // the least, and its workgroups take the small ones in turns, one that has less so far the earlier, as if each took
 // the next tile when it is done.  What an XCD's tiles are has two forms:
-//   eighths  every XCD takes an eighth of every group of big tiles (neighbours in the group's order, the remainders of
-//            the eighths in turn), and a part of the list of the other groups by cost
-//   parts    the whole list is cut by cost, as without a schedule but anywhere.  XCDs whose part is idle groups, which only
-//            store, then run beside XCDs that mostly multiply, where eighths have all of them multiply first and store last;
-//            but an XCD whose 32 workgroups get 33 big tiles of nearly a share each takes two rounds for them
+//   eighths  every XCD takes an eighth of every group (neighbours in the group's order, the remainders of the eighths in
+//            turn), so that all have the same to multiply, to store and to fetch from HBM
+//   parts    the whole list is cut by cost, as without a schedule but anywhere: an operand is read by one XCD or two,
+//            but one whose 32 workgroups get 33 big tiles of nearly a share each takes two rounds for them
 // All of it is the same arithmetic in every workgroup (one wave).
 enum Schedule { kInOrder, kEighths, kParts };
 static constexpr int kSchedGroups = 256;  // groups it is made for: four a lane
@@ -390,7 +389,7 @@ struct KSchedule {  // in LDS
   int tiles[kSchedGroups + 1], cost[kSchedGroups + 1];  // of the small groups before g: tiles, and their cost
   int ahead[64];                                        // the XCD's workgroups: cost of their big tiles in small ones
   int big[128];                                         // this workgroup's big tiles: group * 2^22 + place in the group
-  int n_big, first, n;                                  // how many; the XCD's first small tile; how many tiles in all
+  int n_big, first, n;                                  // how many; parts: the XCD's first small tile; how many tiles in all
 };
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_min(int v) {
@@ -408,22 +407,35 @@ __device__ __forceinline__ int wave_scan(int v, int lane) {  // sum up to this l
   for (int d = 1; d < 64; d <<= 1) { const int y = __shfl_up(v, d); if (lane >= d) v += y; }
   return v;
 }
-// eighths: an XCD's tiles of a big group, from .. from + number
+// eighths: an XCD's tiles of a group, from .. from + number
 __device__ __forceinline__ void xcd_share(int per_g, int xcd, int g, int& from, int& number) {
   const int y = (xcd + g) & 7;
   from = per_g * y >> 3;
   number = (per_g * (y + 1) >> 3) - from;
 }
+// eighths of groups of per_g tiles, in the order of the groups: how many tiles an XCD has, and its tile j (of group h, its
+// place there).  Eight groups' eighths are one of each, which together are per_g tiles from the XCD's own eighth on, around.
+__device__ __forceinline__ int eighths_tiles(int per_g, int xcd, int groups) {
+  const int from = per_g * xcd >> 3, last = xcd + (groups & 7);
+  return (groups >> 3) * per_g + (last < 8 ? per_g * last >> 3 : per_g + (per_g * (last - 8) >> 3)) - from;
+}
+__device__ __forceinline__ void eighths_tile(int per_g, int xcd, int j, int& h, int& place) {
+  const int round = j / per_g;
+  place = j - round * per_g + (per_g * xcd >> 3);
+  if (place >= per_g) place -= per_g;
+  const int y = (8 * place + 7 + per_g) / per_g - 1;  // the first eighth that ends behind it
+  h = 8 * round + ((y - xcd) & 7);
+}
 // Which form a launch takes, by the cost of its largest tile and a workgroup's share, in blocks.  Weight gradients with
-// Zipf-distributed popularity, us in order / eighths / parts, means of four orders of the same groups:
-//   results weigh as much as their products (a mean group costs up to 7.5 blocks): parts from shares of 96 on.  4293 tokens
-//     of 8 in 128 groups 1536 x 2048 - / 212 / 195, 6000 - / 246 / 224
+// Zipf-distributed popularity whose operands come from HBM, as in a step, us in order / eighths / parts, means of four
+// orders of the same groups:
 //   the largest tile is a whole share or more, so that no XCD has more big tiles than workgroups: parts from shares of 24
-//     on.  8942 of 8 in 128, 512 x 2048 133 / 136 / 106; 15000 264 / - / 204; 9000 of 8 in 16, 768 x 2048 143 / - / 122;
-//     30000 of 4 in 32, 1024 x 2048 344 / 343 / 312; 16384 of 8 in 64, 2048 x 768 251 / 258 / 226.  Shorter ones lose (share
-//     15: 40 -> 63), and so do shares of 28 and 29 whose largest tile is half or a third of one: 50 -> 57, 55 -> 74
-//   it is a quarter of a share of 96 or more: eighths.  8192 of 6 in 64, 2816 x 2048 419 / 354 / 376; 11686 of 8 in 128, 1024 x
-//     2048 - / 260 / 295; with smaller ones 607 -> 719, shares of 60 and 87 87 -> 104 and 145 -> 163
+//     on.  8942 tokens of 8 in 128 groups 512 x 2048 177 / 156 / 145; 15000 268 / 218 / 201; 9000 of 8 in 16, 768 x 2048 162 /
+//     130 / 126; 30000 of 4 in 32, 1024 x 2048 311 / 321 / 307; 16384 of 8 in 64, 2048 x 768 280 / 235 / 219.
+//     Shorter ones lose (share 15: 40 -> 63)
+//   the others: eighths from shares of 56 on.  8192 of 6 in 64, 2816 x 2048 393 / 336 / 381; 16384 of 8 in 128, 1536 x 2048 566 / 452 /
+//     498, less skewed 467 / 477 / -; 3500 of 4 in 32, 5760 x 2880 453 / 363 / 461, of 10000 less skewed 686 / 627 / -; 4293 of 8 in
+//     128, 768 x 2048 157 / 150 / 150.  Shares of 28 and 29 lose: 64 -> 66, 67 -> 88
 // Limits: what the lists above can hold (a workgroup's big tiles are at most its share and one tile); sums that stay
 // below 2^29, a workgroup's below 2^22.
 __device__ __forceinline__ Schedule schedule_of(const GemmArgs& p, const int* s_pref, int workers) {
@@ -431,9 +443,8 @@ __device__ __forceinline__ Schedule schedule_of(const GemmArgs& p, const int* s_
   if (!p.offs || p.G > kSchedGroups || workers > 64 || per_g >= (1 << 22) || total >= (8ll << 22) * workers || total >= (1ll << 29)) return kInOrder;
   if (level_groups(p, s_pref)) return kInOrder;
   const int64_t largest = s_pref[p.G + 1] * all_workers;  // against total, as the tile against a share
-  if (total < 96 * all_workers) return total >= 24 * all_workers && largest >= total ? kParts : kInOrder;
-  if (largest * 4 < total) return kInOrder;
-  return largest >= total || 2 * s_pref[p.G] <= 15 * p.G ? kParts : kEighths;
+  if (largest >= total) return total >= 24 * all_workers ? kParts : kInOrder;
+  return total >= 56 * all_workers ? kEighths : kInOrder;
 }
 // Place of workgroup `me`'s small tile j in the XCD's part of their list.  ahead: on lane w the big tiles of workgroup w
 // in small ones; tiles are taken in the order of (ahead + count so far, workgroup).
@@ -480,7 +491,7 @@ __device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* 
   }
   if (lane == 0) { s.tiles[kSchedGroups] = all_tiles; s.cost[kSchedGroups] = all; }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's own writes
-  int part, n_near = all_tiles, cost_near = all;  // small tiles whose mean cost the XCD's own have, and their cost
+  int part, n_near = all_tiles, cost_near = all;  // the XCD's small tiles; those whose mean cost they have, and their cost
   if (parts) {
     // small tiles before a place of the list, and their cost, on lanes 0 and 1 for the two ends of the part
     const int end = (lane & 1) ? t_last : t_first, g = end / per_g < kSchedGroups ? end / per_g : kSchedGroups - 1;
@@ -491,18 +502,7 @@ __device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* 
     cost_near = __builtin_amdgcn_readlane(spent, 1) - __builtin_amdgcn_readlane(spent, 0);
     if (lane == 0) s.first = first;
   } else {
-    // number of tiles whose middle lies below y, on lanes 0 and 1 for the two ends of the part
-    const int y = (int)((int64_t)all * (xcd + (lane & 1)) / 8);
-    int lo = 0, hi = kSchedGroups - 1;  // last g with cost[g] <= y
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (s.cost[mid] <= y) lo = mid; else hi = mid - 1;
-    }
-    const int n = s.tiles[lo + 1] - s.tiles[lo], c = n ? (s.cost[lo + 1] - s.cost[lo]) / n : 1;
-    const int b = (2 * (y - s.cost[lo]) + c - 1) / (2 * c), below = s.tiles[lo] + (b < n ? b : n);
-    const int first = __builtin_amdgcn_readlane(below, 0), last = xcd == 7 ? all_tiles : __builtin_amdgcn_readlane(below, 1);
-    part = last - first;
-    if (lane == 0) s.first = first;
+    part = eighths_tiles(per_g, xcd, all_tiles / per_g);
   }
   // ---- the big ones ----
   int load = lane < workers ? 0 : kNoLoad, n_big = 0;
@@ -556,12 +556,19 @@ __device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* 
 }
 
 // the workgroup's tile i, one on every lane of the first wave: its group and its place in it
-__device__ __forceinline__ void scheduled_tile(const KSchedule& s, int me, int workers, int lane, int i, int& g, int& idx) {
-  const int t = s.first + small_place(s.ahead[lane], me, workers, i - s.n_big);
+__device__ __forceinline__ void scheduled_tile(const KSchedule& s, bool parts, int per_g, int xcd, int me, int workers, int lane, int i, int& g, int& idx) {
+  const int j = small_place(s.ahead[lane], me, workers, i - s.n_big);
   if (i < s.n_big) {
     g = s.big[i] >> 22;
     idx = s.big[i] & ((1 << 22) - 1);
     return;
+  }
+  int t, place = 0;  // a tile of the small groups' list
+  if (parts) {
+    t = s.first + j;
+  } else {
+    eighths_tile(per_g, xcd, j, t, place);
+    t *= per_g;
   }
   int lo = 0, hi = kSchedGroups - 1;  // last g with tiles[g] <= t
   while (lo < hi) {
@@ -569,7 +576,7 @@ __device__ __forceinline__ void scheduled_tile(const KSchedule& s, int me, int w
     if (s.tiles[mid] <= t) lo = mid; else hi = mid - 1;
   }
   g = lo;
-  idx = t - s.tiles[lo];
+  idx = t - s.tiles[lo] + place;
 }
 
 // Geometry of logical tile t (k-grouped, with group >= 0: of that group's tile t); plain per-lane arithmetic (every lane

@@ -291,7 +291,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void fp8_gemm_nt_rowsplit_kernel
     n_tiles = (t_end - t_next + t_step - 1) / t_step;
     if (n_tiles > kRsTiles) n_tiles = kRsTiles;
     int t = t_next + tid * t_step, group = -1;
-    if (scheduled && tid < 64) scheduled_tile(sched, blockIdx.x >> 3, gridDim.x >> 3, lane, t, group, t);
+    if (scheduled && tid < 64) scheduled_tile(sched, scheduled == kParts, p.tiles_a * p.tiles_b, xcd, blockIdx.x >> 3, gridDim.x >> 3, lane, t, group, t);
     if (tid < n_tiles) {
       Tile T;
       decode_tile<MODE, BM, BN>(p, s_pref, t, T, group);
