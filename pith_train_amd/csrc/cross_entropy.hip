@@ -46,8 +46,28 @@ struct CeArgs {
   float* loss;
   int64_t* n_non_ignore;
   const float* grad_output;
+  int vec;  // rows start at multiples of their element size
+};
+
+// A row in 16-byte chunks.  Rows whose length is no multiple of 16 bytes start anywhere in one, so the chunks begin at
+// the first boundary; the elements before it and behind the last whole chunk (at most 7 of either, "edges") belong to
+// threads 0 .. 7 and 8 .. 15 of the workgroup, one each.
+template <typename S>
+struct CeRow {
+  static constexpr int kPer = 16 / S::kBytes;  // elements of a chunk
+  char* x;
+  int head, tail;
   uint32_t chunks;
-  int vec;
+  __device__ __forceinline__ CeRow(char* row, int64_t V) : x(row) {
+    const int64_t to_boundary = (int64_t)(-(uintptr_t)row & 15) / S::kBytes;
+    head = (int)(to_boundary < V ? to_boundary : V);
+    chunks = (uint32_t)((V - head) / kPer);
+    tail = (int)((V - head) % kPer);
+  }
+  __device__ __forceinline__ char* body() const { return x + head * S::kBytes; }
+  // whether thread tid has an edge element, and its byte offset in the row
+  __device__ __forceinline__ bool edge(int tid) const { return tid < 8 ? tid < head : tid < 8 + tail; }
+  __device__ __forceinline__ int64_t edge_at(int tid) const { return (tid < 8 ? tid : head + (int64_t)chunks * kPer + tid - 8) * S::kBytes; }
 };
 
 __device__ __forceinline__ float fast_exp(float v) { return __builtin_amdgcn_exp2f(v * kLog2e); }
@@ -78,6 +98,59 @@ __device__ __forceinline__ void merge_md(float& m, float& d, float m2, float d2)
   d = a + b;
 }
 
+typedef int ce_v4i __attribute__((ext_vector_type(4)));
+
+template <typename S>
+__device__ __forceinline__ void unpack(const ce_v4i& w, float (&v)[CeRow<S>::kPer]) {
+  if constexpr (S::kBytes == 2) {
+    S::load8(&w, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __int_as_float(w[i]);
+  }
+}
+template <typename S>
+__device__ __forceinline__ ce_v4i pack(const float (&v)[CeRow<S>::kPer]) {
+  ce_v4i w;
+  if constexpr (S::kBytes == 2) {
+    S::store8(&w, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = __float_as_int(v[i]);
+  }
+  return w;
+}
+// one chunk (or one edge element) into a thread's running (m, d), rescaled where the maximum grows
+template <int N>
+__device__ __forceinline__ void absorb(const float (&v)[N], float& m, float& d) {
+  float cm = v[0];
+#pragma unroll
+  for (int i = 1; i < N; ++i) cm = fmaxf(cm, v[i]);
+  if (cm > m) {
+    d = d * fast_exp(m - cm);  // m = -inf on the first chunk: d is 0 and exp2(-inf) is 0
+    m = cm;
+  }
+  if (m != -INFINITY) {  // a chunk of -inf logits (masked vocabulary) adds nothing
+    const float mb = m * kLog2e;
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) s += __builtin_amdgcn_exp2f(v[i] * kLog2e - mb);
+    d += s;
+  }
+}
+// logits into gradients of the mean loss; off: the target's place among them (anything else: not there)
+template <typename S, int N, class I>
+__device__ __forceinline__ void gradient(float (&v)[N], float mb, float inv_d, float inv_n, I off) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = (__builtin_amdgcn_exp2f(v[i] * kLog2e - mb) * inv_d) * inv_n;
+  if (off >= 0 && off < N) {
+    // the reference stores the softmax term first and corrects the stored value afterwards
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (i == (int)off) v[i] = S::round(v[i]) - inv_n;
+  }
+}
+
 template <typename S>
 __global__ __launch_bounds__(1024) void ce_fwd_kernel(CeArgs p) {
   __shared__ float s_m[16], s_d[16];
@@ -85,43 +158,31 @@ __global__ __launch_bounds__(1024) void ce_fwd_kernel(CeArgs p) {
   char* x = p.x + row * p.ld;
   const int64_t y = p.target[row];
   const int tid = threadIdx.x;
+  const CeRow<S> r(x, p.V);
+  ce_v4i* body = (ce_v4i*)r.body();
+  const bool edge = p.vec && r.edge(tid);
   if (y == p.ignore_index) {
     if (p.vec) {
-      const uint4 z = {0, 0, 0, 0};
-      for (uint32_t c = tid; c < p.chunks; c += kCeThreads) {
-        if (S::kBytes == 4) {
-          ((uint4*)x)[2 * c] = z;
-          ((uint4*)x)[2 * c + 1] = z;
-        } else {
-          ((uint4*)x)[c] = z;
-        }
-      }
+      const ce_v4i z = {0, 0, 0, 0};
+      for (uint32_t c = tid; c < r.chunks; c += kCeThreads) body[c] = z;
+      if (edge) S::store1(x + r.edge_at(tid), 0.f);
     } else {
       for (int64_t i = tid; i < p.V; i += kCeThreads) S::store1(x + i * S::kBytes, 0.f);
     }
     if (tid == 0) p.loss_rows[row] = 0.f;
     return;
   }
-  // pass 1: per-thread running (m, d), rescaled once per 8-element chunk
+  // pass 1: per-thread running (m, d), rescaled once per chunk
   float m = -INFINITY, d = 0.f;
   if (p.vec) {
-    for (uint32_t c = tid; c < p.chunks; c += kCeThreads) {
-      float v[8];
-      S::load8(x + (int64_t)c * 8 * S::kBytes, v);
-      float cm = v[0];
-#pragma unroll
-      for (int i = 1; i < 8; ++i) cm = fmaxf(cm, v[i]);
-      if (cm > m) {
-        d = d * fast_exp(m - cm);  // m = -inf on the first chunk: d is 0 and exp2(-inf) is 0
-        m = cm;
-      }
-      if (m != -INFINITY) {  // a chunk of -inf logits (masked vocabulary) adds nothing
-        const float mb = m * kLog2e;
-        float s = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s += __builtin_amdgcn_exp2f(v[i] * kLog2e - mb);
-        d += s;
-      }
+    for (uint32_t c = tid; c < r.chunks; c += kCeThreads) {
+      float v[CeRow<S>::kPer];
+      unpack<S>(body[c], v);
+      absorb(v, m, d);
+    }
+    if (edge) {
+      const float v[1] = {S::load1(x + r.edge_at(tid))};
+      absorb(v, m, d);
     }
   } else {
     for (int64_t i = tid; i < p.V; i += kCeThreads) {
@@ -162,20 +223,17 @@ __global__ __launch_bounds__(1024) void ce_fwd_kernel(CeArgs p) {
   const float inv_d = 1.0f / d, inv_n = 1.0f / n;
   const float neg_inv_n = -1.0f / n;
   if (p.vec) {
-    for (uint32_t c = tid; c < p.chunks; c += kCeThreads) {
-      float v[8];
-      char* q = x + (int64_t)c * 8 * S::kBytes;
-      S::load8(q, v);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = (__builtin_amdgcn_exp2f(v[i] * kLog2e - mb) * inv_d) * inv_n;
-      const int64_t off = y - (int64_t)c * 8;
-      if (off >= 0 && off < 8) {
-        // the reference stores the softmax term first and corrects the stored value afterwards
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (i == (int)off) v[i] = S::round(v[i]) + neg_inv_n;
-      }
-      S::store8(q, v);
+    for (uint32_t c = tid; c < r.chunks; c += kCeThreads) {
+      float v[CeRow<S>::kPer];
+      unpack<S>(body[c], v);
+      gradient<S>(v, mb, inv_d, inv_n, y - r.head - (int64_t)c * CeRow<S>::kPer);
+      body[c] = pack<S>(v);
+    }
+    if (edge) {
+      char* q = x + r.edge_at(tid);
+      float v[1] = {S::load1(q)};
+      gradient<S>(v, mb, inv_d, inv_n, y - (q - x) / S::kBytes);
+      S::store1(q, v[0]);
     }
   } else {
     for (int64_t i = tid; i < p.V; i += kCeThreads) {
@@ -186,22 +244,14 @@ __global__ __launch_bounds__(1024) void ce_fwd_kernel(CeArgs p) {
   }
 }
 
-// The same computation with the row held on chip between the passes: 16-bit logits, up to
-// kCeRegChunks 16-byte chunks per thread in registers and the chunks past those in LDS, so the
+// The same computation with the row held on chip between the passes: up to kCeRegChunks 16-byte
+// chunks per thread in registers and the chunks past those in LDS, so the
 // logits cross the memory bus once each way (the generic kernel's second read of a 300 KB row
 // mostly misses the caches when 256 rows are in flight).
-static constexpr int kCeRegChunks = 15;                                  // 15 x 1024 x 8 = 122 880 elements
+static constexpr int kCeRegChunks = 15;                                  // 15 x 1024 x 16 bytes: 122 880 elements of 16 bits
 static constexpr int kCeLdsChunks = (160 * 1024 - 256) / 16;             // + 81 792 elements in the rest of the 160 KiB of LDS
 
 static constexpr int64_t kCeWorkgroups = 256;  // one per compute unit
-
-typedef int ce_v4i __attribute__((ext_vector_type(4)));
-
-template <typename S>
-__device__ __forceinline__ void unpack8(const ce_v4i& w, float* v) {
-  static_assert(S::kBytes == 2, "16-bit storage only");
-  S::load8(&w, v);
-}
 
 // 16 bytes per lane from base + voff (per lane) + soff (uniform) into LDS at lds_off + 16 * lane.
 __device__ __forceinline__ void ce_load_to_lds(ce_v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds_off) {
@@ -224,41 +274,42 @@ __global__ __launch_bounds__(1024) void ce_fwd_onchip_kernel(CeArgs p) {
   __shared__ float s_m[16], s_d[16];
   const int tid = threadIdx.x;
   const uint32_t voff = (uint32_t)tid * 16u;
-  const int row_bytes = (int)(p.V * S::kBytes);
   ce_v4i cache[kCeRegChunks];
   // The chunks past the registers go straight from memory into LDS (direct-to-LDS loads: a wave's
   // 64 lanes fill 1 KiB, lane l the 16 bytes of the chunk thread l of that wave owns).
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) ce_v4i*)s_over;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Raw buffer descriptor over a row: a lane's byte offset is tid * 16 for every chunk, the
-  // chunk's i * 16 KiB goes into the uniform offset, and accesses past the row's end are dropped by
+  // Raw buffer descriptor over a row's chunks: a lane's byte offset is tid * 16 for every chunk, the
+  // chunk's i * 16 KiB goes into the uniform offset, and accesses past the last chunk are dropped by
   // the hardware (loads return 0) instead of needing an address and a predicate per chunk.
-  auto row_words = [&](const char* x) {
-    const uint64_t a = (uint64_t)(uintptr_t)x;
-    ce_v4i r;
-    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
-    r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)((a >> 32) & 0xFFFF));
-    r[2] = __builtin_amdgcn_readfirstlane(row_bytes);
-    r[3] = 0x00020000;
-    return r;
+  auto row_words = [&](const CeRow<S>& r) {
+    const uint64_t a = (uint64_t)(uintptr_t)r.body();
+    ce_v4i w;
+    w[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+    w[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)((a >> 32) & 0xFFFF));
+    w[2] = __builtin_amdgcn_readfirstlane((int)(r.chunks * 16));
+    w[3] = 0x00020000;
+    return w;
   };
+  auto edge_logit = [&](const CeRow<S>& r) { return r.edge(tid) ? S::load1(r.x + r.edge_at(tid)) : 0.f; };
   auto target_logit = [&](const char* x, int64_t y) { return y >= 0 && y < p.V ? S::load1(x + y * S::kBytes) : NAN; };
 
   int64_t row = blockIdx.x;  // the grid has at most as many workgroups as there are rows
-  char* x = p.x + row * p.ld;
+  CeRow<S> r(p.x + row * p.ld, p.V);
   int64_t y = p.target[row];
-  float xy = target_logit(x, y);
+  float xy = target_logit(r.x, y);
+  float xe = edge_logit(r);
   {
-    const ce_v4i words = row_words(x);
+    const ce_v4i words = row_words(r);
 #pragma unroll 1
-    for (uint32_t c0 = kCeRegChunks * kCeThreads + wave * 64; c0 < p.chunks; c0 += kCeThreads)
+    for (uint32_t c0 = kCeRegChunks * kCeThreads + wave * 64; c0 < r.chunks; c0 += kCeThreads)
       ce_load_to_lds(words, (uint32_t)(tid & 63) * 16u, c0 * 16u, lds_base + (c0 - kCeRegChunks * kCeThreads) * 16u);
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(x, 0, row_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(r.body(), 0, (int)(r.chunks * 16), 0x00020000);
 #pragma unroll
     for (int i = 0; i < kCeRegChunks; ++i) cache[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, i * kCeThreads * 16, (PT_CE_NT & 1) ? 2 : 0);
   }
   const float n = (float)*p.n_non_ignore;
-  const float inv_n = 1.0f / n, neg_inv_n = -1.0f / n;
+  const float inv_n = 1.0f / n;
 
 #pragma unroll 1
   for (;;) {
@@ -266,31 +317,22 @@ __global__ __launch_bounds__(1024) void ce_fwd_onchip_kernel(CeArgs p) {
     const bool more = next < p.N;
     const bool ignored = y == p.ignore_index;
     float m = -INFINITY, d = 0.f;
-    auto absorb = [&](const ce_v4i& w) {
-      float v[8];
-      unpack8<S>(w, v);
-      float cm = v[0];
-#pragma unroll
-      for (int i = 1; i < 8; ++i) cm = fmaxf(cm, v[i]);
-      if (cm > m) {
-        d = d * fast_exp(m - cm);
-        m = cm;
-      }
-      if (m != -INFINITY) {
-        const float mb = m * kLog2e;
-        float s = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s += __builtin_amdgcn_exp2f(v[i] * kLog2e - mb);
-        d += s;
-      }
+    auto absorb_chunk = [&](const ce_v4i& w) {
+      float v[CeRow<S>::kPer];
+      unpack<S>(w, v);
+      absorb(v, m, d);
       __builtin_amdgcn_sched_barrier(0);  // one chunk's temporaries at a time: the cache owns the registers
     };
 #pragma unroll
     for (int i = 0; i < kCeRegChunks; ++i)
-      if ((uint32_t)i * kCeThreads + tid < p.chunks) absorb(cache[i]);
+      if ((uint32_t)i * kCeThreads + tid < r.chunks) absorb_chunk(cache[i]);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the LDS part has landed (each thread reads only its own chunks)
 #pragma unroll 1
-    for (uint32_t c = kCeRegChunks * kCeThreads + tid; c < p.chunks; c += kCeThreads) absorb(s_over[c - kCeRegChunks * kCeThreads]);
+    for (uint32_t c = kCeRegChunks * kCeThreads + tid; c < r.chunks; c += kCeThreads) absorb_chunk(s_over[c - kCeRegChunks * kCeThreads]);
+    if (r.edge(tid)) {
+      const float v[1] = {xe};
+      absorb(v, m, d);
+    }
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) {
       const float m2 = __shfl_xor(m, s), d2 = __shfl_xor(d, s);
@@ -308,42 +350,45 @@ __global__ __launch_bounds__(1024) void ce_fwd_onchip_kernel(CeArgs p) {
     if (tid == 0) p.loss_rows[row] = ignored ? 0.f : -(xy - m - logf(d));
     // the next row's target and logit are requested before its chunks
     const int64_t row2 = more ? next : row;
-    const char* x2 = p.x + row2 * p.ld;
+    const CeRow<S> r2(p.x + row2 * p.ld, p.V);
     const int64_t y2 = p.target[row2];
-    const float xy2 = target_logit(x2, y2);
+    const float xy2 = target_logit(r2.x, y2);
+    const float xe2 = edge_logit(r2);
     const float mb = m * kLog2e;
     // The two divisions of the reference become multiplications by reciprocals computed once per
     // row: an fp32 division per element costs more issue cycles than everything else in the pass.
     const float inv_d = 1.0f / d;
+    // the target's place in the body (before it, where there is none: rows of this kernel are far shorter)
+    const int y_body = y >= 0 && y < p.V ? (int)y - r.head : -16;
     // gradient of one chunk, packed for a 16-byte store
     auto grad_of = [&](const ce_v4i& w, uint32_t c) {
-      float v[8];
-      unpack8<S>(w, v);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = (__builtin_amdgcn_exp2f(v[i] * kLog2e - mb) * inv_d) * inv_n;
-      const int64_t off = y - (int64_t)c * 8;
-      if (off >= 0 && off < 8) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (i == (int)off) v[i] = S::round(v[i]) + neg_inv_n;
-      }
-      ce_v4i out;
-      S::store8(&out, v);
+      float v[CeRow<S>::kPer];
+      unpack<S>(w, v);
+      gradient<S>(v, mb, inv_d, inv_n, y_body - (int)c * CeRow<S>::kPer);
+      ce_v4i out = pack<S>(v);
       if (ignored) out = ce_v4i{0, 0, 0, 0};
       return out;
     };
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(x, 0, row_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsrc2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(x2), 0, more ? row_bytes : 0, 0x00020000);
+    if (r.edge(tid)) {
+      float v[1] = {xe};
+      gradient<S>(v, mb, inv_d, inv_n, y - r.edge_at(tid) / S::kBytes);
+      S::store1(r.x + r.edge_at(tid), ignored ? 0.f : v[0]);
+    }
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(r.body(), 0, (int)(r.chunks * 16), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc2 = __builtin_amdgcn_make_buffer_rsrc(r2.body(), 0, more ? (int)(r2.chunks * 16) : 0, 0x00020000);
     // LDS part first: its loads are the slower kind to drain at the end of the next statistics pass
     {
-      const ce_v4i words2 = row_words(x2);
+      const ce_v4i words2 = row_words(r2);
+      // (the next row may have a chunk more or less than this one)
+      const uint32_t most = more && r2.chunks > r.chunks ? r2.chunks : r.chunks;
 #pragma unroll 1
-      for (uint32_t c0 = kCeRegChunks * kCeThreads + wave * 64; c0 < p.chunks; c0 += kCeThreads) {
+      for (uint32_t c0 = kCeRegChunks * kCeThreads + wave * 64; c0 < most; c0 += kCeThreads) {
         const uint32_t c = c0 + (tid & 63);
-        if (c < p.chunks) {
+        if (c < r.chunks) {
           const ce_v4i g = grad_of(s_over[c - kCeRegChunks * kCeThreads], c);
-          if (PT_CE_NT & 2) __builtin_nontemporal_store(g, (ce_v4i*)(x + (int64_t)c * 16));
-          else *(ce_v4i*)(x + (int64_t)c * 16) = g;
+          ce_v4i* q = (ce_v4i*)r.body() + c;
+          if (PT_CE_NT & 2) __builtin_nontemporal_store(g, q);
+          else *q = g;
         }
         // (the wave's reads of these 1 KiB have returned: their values are in the stores above)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -361,9 +406,10 @@ __global__ __launch_bounds__(1024) void ce_fwd_onchip_kernel(CeArgs p) {
     }
     if (!more) break;
     row = next;
-    x = const_cast<char*>(x2);
+    r = r2;
     y = y2;
     xy = xy2;
+    xe = xe2;
   }
 }
 
@@ -395,30 +441,27 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(CeArgs p, uint32_t blocks
   const uint32_t row = blockIdx.x / blocks_per_row, rb = blockIdx.x % blocks_per_row;
   char* x = p.x + (int64_t)row * p.ld;
   if (p.vec) {
+    const CeRow<S> r(x, p.V);
+    ce_v4i* body = (ce_v4i*)r.body();
     const uint32_t c0 = rb * 1024 + threadIdx.x;
-    float v[4][8];
+    if (rb == 0 && r.edge(threadIdx.x)) {
+      char* q = x + r.edge_at(threadIdx.x);
+      S::store1(q, S::load1(q) * s);
+    }
+    ce_v4i w[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      if (c0 + q * 256 < p.chunks) {
-        if (S::kBytes == 2 && (PT_CE_NT & 1)) {
-          const ce_v4i w = __builtin_nontemporal_load((const ce_v4i*)(x + (int64_t)(c0 + q * 256) * 16));
-          S::load8(&w, v[q]);
-        } else {
-          S::load8(x + (int64_t)(c0 + q * 256) * 8 * S::kBytes, v[q]);
-        }
-      }
+      if (c0 + q * 256 < r.chunks) w[q] = (PT_CE_NT & 1) ? __builtin_nontemporal_load(body + c0 + q * 256) : body[c0 + q * 256];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      if (c0 + q * 256 < p.chunks) {
+      if (c0 + q * 256 < r.chunks) {
+        float v[CeRow<S>::kPer];
+        unpack<S>(w[q], v);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[q][i] = v[q][i] * s;
-        if (S::kBytes == 2 && (PT_CE_NT & 2)) {
-          ce_v4i w;
-          S::store8(&w, v[q]);
-          __builtin_nontemporal_store(w, (ce_v4i*)(x + (int64_t)(c0 + q * 256) * 16));
-        } else {
-          S::store8(x + (int64_t)(c0 + q * 256) * 8 * S::kBytes, v[q]);
-        }
+        for (int i = 0; i < CeRow<S>::kPer; ++i) v[i] = v[i] * s;
+        const ce_v4i g = pack<S>(v);
+        if (PT_CE_NT & 2) __builtin_nontemporal_store(g, body + c0 + q * 256);
+        else body[c0 + q * 256] = g;
       }
     }
   } else {
@@ -433,8 +476,7 @@ static int ce_args(CeArgs& a, const char* who, void* logits, int64_t ld, int dty
   PT_REQUIRE(dtype == PT_BF16 || dtype == PT_F16 || dtype == PT_F32, "%s: unsupported dtype %d", who, dtype);
   const int eb = dtype == PT_F32 ? 4 : 2;
   a.x = (char*)logits; a.ld = ld * eb; a.N = N; a.V = V;
-  a.chunks = (uint32_t)cdiv(V, 8);
-  a.vec = V % 8 == 0 && ((uintptr_t)logits & 15) == 0 && a.ld % 16 == 0;
+  a.vec = (uintptr_t)logits % eb == 0;
   return PT_OK;
 }
 
@@ -451,26 +493,30 @@ extern "C" int pt_cross_entropy_fwd(void* logits, int64_t ld, int dtype, const i
   a.target = target; a.ignore_index = ignore_index; a.loss_rows = loss_rows; a.loss = loss; a.n_non_ignore = n_non_ignore;
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(ce_count_kernel, dim3(1), dim3(1024), 0, s, target, N, ignore_index, n_non_ignore);
-  const int64_t over = (int64_t)a.chunks - (int64_t)kCeRegChunks * kCeThreads;
+  const int64_t chunks = V * (dtype == PT_F32 ? 4 : 2) / 16, over = chunks - (int64_t)kCeRegChunks * kCeThreads;  // at most, of a row
   // PITHTRAIN_CE_KERNEL=twopass keeps the generic kernel for every shape (for measurements)
   static const bool onchip_allowed = [] {
     const char* e = getenv("PITHTRAIN_CE_KERNEL");
     return !(e && strcmp(e, "twopass") == 0);
   }();
-  if (N && a.vec && dtype != PT_F32 && over <= kCeLdsChunks && onchip_allowed) {
+  if (N && a.vec && over <= kCeLdsChunks && onchip_allowed) {
     const size_t lds = over > 0 ? (size_t)over * 16 : 0;
     // more than 64 KiB of dynamic LDS has to be allowed per kernel, once per process
     static const hipError_t allow = [] {
       hipError_t e = hipFuncSetAttribute((const void*)ce_fwd_onchip_kernel<st_bf16>,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, kCeLdsChunks * 16);
       if (e != hipSuccess) return e;
-      return hipFuncSetAttribute((const void*)ce_fwd_onchip_kernel<st_f16>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      e = hipFuncSetAttribute((const void*)ce_fwd_onchip_kernel<st_f16>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kCeLdsChunks * 16);
+      if (e != hipSuccess) return e;
+      return hipFuncSetAttribute((const void*)ce_fwd_onchip_kernel<st_f32>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  kCeLdsChunks * 16);
     }();
     PT_REQUIRE(allow == hipSuccess, "cross_entropy_fwd: hipFuncSetAttribute failed: %s", hipGetErrorString(allow));
     const unsigned blocks = (unsigned)(N < kCeWorkgroups ? N : kCeWorkgroups);
     if (dtype == PT_BF16) hipLaunchKernelGGL(ce_fwd_onchip_kernel<st_bf16>, dim3(blocks), dim3(kCeThreads), lds, s, a);
-    else hipLaunchKernelGGL(ce_fwd_onchip_kernel<st_f16>, dim3(blocks), dim3(kCeThreads), lds, s, a);
+    else if (dtype == PT_F16) hipLaunchKernelGGL(ce_fwd_onchip_kernel<st_f16>, dim3(blocks), dim3(kCeThreads), lds, s, a);
+    else hipLaunchKernelGGL(ce_fwd_onchip_kernel<st_f32>, dim3(blocks), dim3(kCeThreads), lds, s, a);
   } else if (N) {
     switch (dtype) {
       case PT_BF16: hipLaunchKernelGGL(ce_fwd_kernel<st_bf16>, dim3((unsigned)N), dim3(kCeThreads), 0, s, a); break;
@@ -489,7 +535,7 @@ extern "C" int pt_cross_entropy_bwd(void* grad, int64_t ld, int dtype, int64_t N
   if (N == 0) return PT_OK;
   PT_REQUIRE(grad && grad_output, "cross_entropy_bwd: null pointer");
   a.grad_output = grad_output;
-  const int64_t bx = a.vec ? cdiv(a.chunks, 1024) : (cdiv(V, 256) < 1024 ? cdiv(V, 256) : 1024);
+  const int64_t bx = a.vec ? cdiv(cdiv(V * (dtype == PT_F32 ? 4 : 2), 16), 1024) : (cdiv(V, 256) < 1024 ? cdiv(V, 256) : 1024);
   PT_REQUIRE(N * bx < (1ll << 31), "cross_entropy_bwd: too many rows for one launch");
   const dim3 grid((unsigned)(N * bx));
   switch (dtype) {

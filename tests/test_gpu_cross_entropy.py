@@ -31,7 +31,8 @@ def _check_grad(got, ref, dtype):
         torch.testing.assert_close(got, ref, rtol=2e-5, atol=1e-10)
         return
     step = 2.0**-7 if dtype == torch.bfloat16 else 2.0**-10
-    assert ((got - ref).abs() <= ref.abs() * step + 1e-30).all(), "more than one rounding step apart"
+    least = 1e-30 if dtype == torch.bfloat16 else 2.0**-24  # below 2^-14 the float16 values are 2^-24 apart
+    assert ((got - ref).abs() <= ref.abs() * step + least).all(), "more than one rounding step apart"
     assert (got == ref).float().mean() > 0.98
 
 
@@ -154,3 +155,35 @@ def test_more_rows_than_workgroups(N, V, dtype):
         at_target[torch.arange(len(yp), device="cuda"), yp.clamp(min=0)] = step
         assert ((a - b).abs() <= step * b.abs() + at_target + (2.0 ** -20 if dtype == torch.float16 else 1e-20) * n).all()
     torch.testing.assert_close(loss.double(), total / n, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("N,V,start", [
+    (19, 1, 0), (19, 3, 1), (19, 9, 5),  # rows that are edges alone, or hold one chunk or none
+    (600, 1003, 0),      # more rows than compute units: a row's neighbour starts elsewhere in a chunk
+    (260, 50257, 3),
+    (3, 61441, 1), (2, 122888, 7),  # as long as the registers hold, and a chunk more or less by where a row starts
+    (2, 204665, 0), (2, 102337, 2),  # as long as registers and LDS hold, of 16 and of 32 bits; past it the row is read twice
+    (2, 300007, 6),
+])
+def test_rows_that_start_anywhere(N, V, start, dtype):
+    """Rows of a length that is no multiple of a chunk, in a buffer that starts inside one: targets among the first and the
+    last elements of a row, and nothing written outside of the rows."""
+    from pith_train_amd.operators.cross_entropy import cross_entropy
+
+    x, y = _case(N, V, N + V, dtype)
+    y[::3] = torch.arange(len(y[::3])) % min(V, 9)
+    y[1::3] = V - 1 - torch.arange(len(y[1::3])) % min(V, 9)
+    y[-1] = -100
+    o_loss, o_grad, _, _ = CE.cross_entropy_fwd(x, y)
+    flat = torch.full((start + N * V + 16,), 7.0, dtype=dtype, device="cuda")
+    buf = flat[start : start + N * V].view(N, V)
+    buf.copy_(x)
+    buf.requires_grad_(True)
+    loss = cross_entropy(buf.view(N, V), y.cuda())
+    torch.testing.assert_close(loss.detach().cpu(), o_loss, rtol=1e-5, atol=1e-6)
+    stored = buf.detach().clone()
+    _check_grad(stored, o_grad, dtype)
+    (grad,) = torch.autograd.grad(loss * 0.3, buf)
+    assert torch.equal(grad, stored * torch.tensor(0.3).to(dtype))
+    assert (flat[:start] == 7).all() and (flat[start + N * V :] == 7).all()
