@@ -249,9 +249,13 @@ __global__ __launch_bounds__(1024) void ce_fwd_kernel(CeArgs p) {
 // logits cross the memory bus once each way (the generic kernel's second read of a 300 KB row
 // mostly misses the caches when 256 rows are in flight).
 static constexpr int kCeRegChunks = 15;                                  // 15 x 1024 x 16 bytes: 122 880 elements of 16 bits
+// Rows of up to 64 KiB leave room for two workgroups a compute unit, one of which reads while the other is between its
+// last load and its first store: 4096 x 32 000 bf16 with its copy 380 -> 307 us.  With 8 chunks the kernel spills (358;
+// 32 000 float32 593 -> 607).
+static constexpr int kCeShortChunks = 4;
 static constexpr int kCeLdsChunks = (160 * 1024 - 256) / 16;             // + 81 792 elements in the rest of the 160 KiB of LDS
 
-static constexpr int64_t kCeWorkgroups = 256;  // one per compute unit
+static constexpr int64_t kCeUnits = 256;  // compute units
 
 // 16 bytes per lane from base + voff (per lane) + soff (uniform) into LDS at lds_off + 16 * lane.
 __device__ __forceinline__ void ce_load_to_lds(ce_v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds_off) {
@@ -268,13 +272,13 @@ __device__ __forceinline__ void ce_load_to_lds(ce_v4i rsrc, uint32_t voff, uint3
 // per row a compute unit first only read and then only wrote (4096 x 151 936 bf16: 546 us against
 // 523 here, where a plain copy of the logits takes 471; what is left is the pause of every row between
 // its last load and its first store).
-template <typename S>
-__global__ __launch_bounds__(1024) void ce_fwd_onchip_kernel(CeArgs p) {
+template <typename S, int CHUNKS>
+__global__ __launch_bounds__(1024, CHUNKS == kCeRegChunks ? 4 : 8) void ce_fwd_onchip_kernel(CeArgs p) {
   extern __shared__ ce_v4i s_over[];
   __shared__ float s_m[16], s_d[16];
   const int tid = threadIdx.x;
   const uint32_t voff = (uint32_t)tid * 16u;
-  ce_v4i cache[kCeRegChunks];
+  ce_v4i cache[CHUNKS];
   // The chunks past the registers go straight from memory into LDS (direct-to-LDS loads: a wave's
   // 64 lanes fill 1 KiB, lane l the 16 bytes of the chunk thread l of that wave owns).
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) ce_v4i*)s_over;
@@ -302,11 +306,11 @@ __global__ __launch_bounds__(1024) void ce_fwd_onchip_kernel(CeArgs p) {
   {
     const ce_v4i words = row_words(r);
 #pragma unroll 1
-    for (uint32_t c0 = kCeRegChunks * kCeThreads + wave * 64; c0 < r.chunks; c0 += kCeThreads)
-      ce_load_to_lds(words, (uint32_t)(tid & 63) * 16u, c0 * 16u, lds_base + (c0 - kCeRegChunks * kCeThreads) * 16u);
+    for (uint32_t c0 = CHUNKS * kCeThreads + wave * 64; c0 < r.chunks; c0 += kCeThreads)
+      ce_load_to_lds(words, (uint32_t)(tid & 63) * 16u, c0 * 16u, lds_base + (c0 - CHUNKS * kCeThreads) * 16u);
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(r.body(), 0, (int)(r.chunks * 16), 0x00020000);
 #pragma unroll
-    for (int i = 0; i < kCeRegChunks; ++i) cache[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, i * kCeThreads * 16, (PT_CE_NT & 1) ? 2 : 0);
+    for (int i = 0; i < CHUNKS; ++i) cache[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, i * kCeThreads * 16, (PT_CE_NT & 1) ? 2 : 0);
   }
   const float n = (float)*p.n_non_ignore;
   const float inv_n = 1.0f / n;
@@ -324,11 +328,11 @@ __global__ __launch_bounds__(1024) void ce_fwd_onchip_kernel(CeArgs p) {
       __builtin_amdgcn_sched_barrier(0);  // one chunk's temporaries at a time: the cache owns the registers
     };
 #pragma unroll
-    for (int i = 0; i < kCeRegChunks; ++i)
+    for (int i = 0; i < CHUNKS; ++i)
       if ((uint32_t)i * kCeThreads + tid < r.chunks) absorb_chunk(cache[i]);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the LDS part has landed (each thread reads only its own chunks)
 #pragma unroll 1
-    for (uint32_t c = kCeRegChunks * kCeThreads + tid; c < r.chunks; c += kCeThreads) absorb_chunk(s_over[c - kCeRegChunks * kCeThreads]);
+    for (uint32_t c = CHUNKS * kCeThreads + tid; c < r.chunks; c += kCeThreads) absorb_chunk(s_over[c - CHUNKS * kCeThreads]);
     if (r.edge(tid)) {
       const float v[1] = {xe};
       absorb(v, m, d);
@@ -382,21 +386,21 @@ __global__ __launch_bounds__(1024) void ce_fwd_onchip_kernel(CeArgs p) {
       // (the next row may have a chunk more or less than this one)
       const uint32_t most = more && r2.chunks > r.chunks ? r2.chunks : r.chunks;
 #pragma unroll 1
-      for (uint32_t c0 = kCeRegChunks * kCeThreads + wave * 64; c0 < most; c0 += kCeThreads) {
+      for (uint32_t c0 = CHUNKS * kCeThreads + wave * 64; c0 < most; c0 += kCeThreads) {
         const uint32_t c = c0 + (tid & 63);
         if (c < r.chunks) {
-          const ce_v4i g = grad_of(s_over[c - kCeRegChunks * kCeThreads], c);
+          const ce_v4i g = grad_of(s_over[c - CHUNKS * kCeThreads], c);
           ce_v4i* q = (ce_v4i*)r.body() + c;
           if (PT_CE_NT & 2) __builtin_nontemporal_store(g, q);
           else *q = g;
         }
         // (the wave's reads of these 1 KiB have returned: their values are in the stores above)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (more) ce_load_to_lds(words2, (uint32_t)(tid & 63) * 16u, c0 * 16u, lds_base + (c0 - kCeRegChunks * kCeThreads) * 16u);
+        if (more) ce_load_to_lds(words2, (uint32_t)(tid & 63) * 16u, c0 * 16u, lds_base + (c0 - CHUNKS * kCeThreads) * 16u);
       }
     }
 #pragma unroll
-    for (int i = 0; i < kCeRegChunks; ++i) {
+    for (int i = 0; i < CHUNKS; ++i) {
       const uint32_t c = (uint32_t)i * kCeThreads + tid;
       asm volatile("" : "+v"(cache[i]));  // unpack again rather than keep 120 values from the statistics pass
       // a chunk past the row's end computes on zeros and its store is dropped by the descriptor
@@ -500,23 +504,30 @@ extern "C" int pt_cross_entropy_fwd(void* logits, int64_t ld, int dtype, const i
     return !(e && strcmp(e, "twopass") == 0);
   }();
   if (N && a.vec && over <= kCeLdsChunks && onchip_allowed) {
+    const bool short_rows = chunks <= kCeShortChunks * kCeThreads;
     const size_t lds = over > 0 ? (size_t)over * 16 : 0;
     // more than 64 KiB of dynamic LDS has to be allowed per kernel, once per process
     static const hipError_t allow = [] {
-      hipError_t e = hipFuncSetAttribute((const void*)ce_fwd_onchip_kernel<st_bf16>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, kCeLdsChunks * 16);
-      if (e != hipSuccess) return e;
-      e = hipFuncSetAttribute((const void*)ce_fwd_onchip_kernel<st_f16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              kCeLdsChunks * 16);
-      if (e != hipSuccess) return e;
-      return hipFuncSetAttribute((const void*)ce_fwd_onchip_kernel<st_f32>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 kCeLdsChunks * 16);
+      for (const void* k : {(const void*)ce_fwd_onchip_kernel<st_bf16, kCeRegChunks>, (const void*)ce_fwd_onchip_kernel<st_f16, kCeRegChunks>,
+                            (const void*)ce_fwd_onchip_kernel<st_f32, kCeRegChunks>}) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kCeLdsChunks * 16);
+        if (e != hipSuccess) return e;
+      }
+      return hipSuccess;
     }();
     PT_REQUIRE(allow == hipSuccess, "cross_entropy_fwd: hipFuncSetAttribute failed: %s", hipGetErrorString(allow));
-    const unsigned blocks = (unsigned)(N < kCeWorkgroups ? N : kCeWorkgroups);
-    if (dtype == PT_BF16) hipLaunchKernelGGL(ce_fwd_onchip_kernel<st_bf16>, dim3(blocks), dim3(kCeThreads), lds, s, a);
-    else if (dtype == PT_F16) hipLaunchKernelGGL(ce_fwd_onchip_kernel<st_f16>, dim3(blocks), dim3(kCeThreads), lds, s, a);
-    else hipLaunchKernelGGL(ce_fwd_onchip_kernel<st_f32>, dim3(blocks), dim3(kCeThreads), lds, s, a);
+    const int64_t most = short_rows ? 2 * kCeUnits : kCeUnits;
+    const dim3 blocks((unsigned)(N < most ? N : most)), threads(kCeThreads);
+    switch (dtype) {
+#define PT_CE_LAUNCH(S)                                                                                        \
+  if (short_rows) hipLaunchKernelGGL((ce_fwd_onchip_kernel<S, kCeShortChunks>), blocks, threads, 0, s, a);         \
+  else hipLaunchKernelGGL((ce_fwd_onchip_kernel<S, kCeRegChunks>), blocks, threads, lds, s, a);               \
+  break;
+      case PT_BF16: PT_CE_LAUNCH(st_bf16)
+      case PT_F16: PT_CE_LAUNCH(st_f16)
+      default: PT_CE_LAUNCH(st_f32)
+#undef PT_CE_LAUNCH
+    }
   } else if (N) {
     switch (dtype) {
       case PT_BF16: hipLaunchKernelGGL(ce_fwd_kernel<st_bf16>, dim3((unsigned)N), dim3(kCeThreads), 0, s, a); break;

@@ -162,6 +162,7 @@ def test_more_rows_than_workgroups(N, V, dtype):
     (19, 1, 0), (19, 3, 1), (19, 9, 5),  # rows that are edges alone, or hold one chunk or none
     (600, 1003, 0),      # more rows than compute units: a row's neighbour starts elsewhere in a chunk
     (260, 50257, 3),
+    (3, 32767, 1), (3, 32776, 0), (3, 16384, 3),  # the longest of the short rows and the next, of 16 and of 32 bits
     (3, 61441, 1), (2, 122888, 7),  # as long as the registers hold, and a chunk more or less by where a row starts
     (2, 204665, 0), (2, 102337, 2),  # as long as registers and LDS hold, of 16 and of 32 bits; past it the row is read twice
     (2, 300007, 6),
