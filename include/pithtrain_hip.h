@@ -652,7 +652,8 @@ int pt_gate_linear_bwd(const void* d_logits, int dtype, const void* x, const voi
  * GEMMs' stores; otherwise silu(gate) * up on concatenated halves.  x_t [K, M] and h_t [half, M] bytes with
  * scales [M/128, K] and [M/128, half]: the transposed activations that the weight gradients read (all four
  * NULL: no backward follows).  repeat > 1 (with row_map, without expand_idx): grouped row r is
- * x[row_map[r] / repeat].  few_rows != 0 (no backward): the groups are multiples of 64 rows.  Not
+ * x[row_map[r] / repeat].  few_rows != 0 (no backward): the groups are multiples of 64 rows,
+ * and with scatter what stands for their padding in gate_up is not defined.  Not
  * needed afterwards: composed_map int32 [M] (with expand_idx), x_fp8 [M, K] and h_fp8 [M, half] with
  * their 1x128 scales. */
 typedef struct {

@@ -541,7 +541,7 @@ extern "C" int pt_sum_partials(const float* partial, int32_t splits, int64_t n, 
 
 int pt::gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order, const void* b_fp8, const float* b_scale, void* out, int out_dtype,
                        const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows,
-                       const void* bias, pt_stream_t stream, bool b_kmajor, bool few_rows, void* out2, int64_t out2_rows) {
+                       const void* bias, pt_stream_t stream, bool b_kmajor, bool few_rows, void* out2, int64_t out2_rows, const int32_t* row_used) {
   PT_REQUIRE(M >= 0 && N >= 0 && K >= 0 && G > 0, "gemm_m_grouped_nt: bad sizes");
   if (M == 0 || N == 0) return PT_OK;
   PT_REQUIRE(M % (few_rows ? 64 : 128) == 0, "gemm_m_grouped_nt: M=%lld must be a multiple of %d", (long long)M, few_rows ? 64 : 128);
@@ -557,7 +557,7 @@ int pt::gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order,
   g.sb = b_scale; g.sb_rs = KB; g.sb_ks = 1; g.sb_shift = 7;
   g.out = out; g.ldo = N; g.out_dtype = out_dtype; g.accumulate = 0;
   g.rows_a = M; g.rows_b = N; g.red = K; g.mode = GEMM_M_GROUPED; g.offs = offs; g.G = G;
-  g.b_stride_g = N * K; g.sb_stride_g = NB * KB; g.few_rows = few_rows;
+  g.b_stride_g = N * K; g.sb_stride_g = NB * KB; g.few_rows = few_rows; g.row_used = few_rows ? row_used : nullptr;
   g.a_bytes = M * K; g.b_bytes = N * K; g.sa_bytes = M * KB * 4; g.sb_bytes = NB * KB * 4;
   g.tiles_a = (int)(M / 128); g.tiles_b = (int)NB;
   g.total_tiles = (int64_t)g.tiles_a * g.tiles_b;

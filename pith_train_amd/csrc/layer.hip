@@ -61,13 +61,15 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order)
   const int32_t G = (int32_t)a.G;
   const int32_t* limit = a.row_map ? a.offs + G - 1 : nullptr;  // rows past it hold nothing
   const int32_t* in_map = a.row_map;
+  // where the rows go back to their places, nobody sees what stands for the padding of groups of 64
+  const int32_t* used = a.few_rows && a.scatter ? a.row_map : nullptr;
   if (a.expand_idx) {
     PT_STEP(pt_compose_row_map, a.M, 0, 0, a.row_map, a.M, a.expand_idx, a.n_expand, a.x_rows, a.composed_map, a.stream);
     in_map = a.composed_map;
   }
   const auto quant_x = [&](int64_t repeat, const int32_t* rows_of, const int32_t* ends) {
     return quant_rowwise_colwise(a.x, a.x_rows, repeat, PT_BF16, a.M, a.K, a.ldx, rows_of, a.x_fp8, a.x_scale, order, a.x_t, a.x_t_scale,
-                                 PT_CH_TRANSPOSED, ends, ends ? G : 0, a.stream);
+                                 PT_CH_TRANSPOSED, ends, ends ? G : 0, a.stream, nullptr, used);
   };
   if (a.repeat > 1)
     PT_STEP_AS(pt_quant_rowwise_colwise_rows_repeat, a.M, a.K, a.x_rows, quant_x(a.repeat, in_map, a.offs));
@@ -78,7 +80,7 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order)
   const int64_t N = 2 * a.half;
   const auto gate_up = [&](const void* bias) {
     return gemm_m_grouped(a.x_fp8, a.x_scale, order, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M, N, a.K, nullptr, 0, bias, a.stream,
-                          false, a.few_rows != 0);
+                          false, a.few_rows != 0, nullptr, 0, used);
   };
   if (a.few_rows)
     PT_STEP_AS(pt_gemm_m_grouped_nt_few_rows, a.M, N, a.K, gate_up(a.gu_bias));
@@ -89,13 +91,13 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order)
   if (a.clamped)
     PT_STEP_AS(pt_clamped_swiglu_quant_rowwise_colwise, a.M, a.half, 0,
                clamped_swiglu_quant(a.gate_up, a.M, a.half, N, (float)a.alpha, (float)a.limit, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit, order,
-                                    a.stream));
+                                    a.stream, used));
   else
     PT_STEP_AS(pt_silu_mul_quant_rowwise_colwise, a.M, a.half, 0,
-               silu_mul_quant(a.gate_up, a.M, a.half, N, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit, order, a.stream));
+               silu_mul_quant(a.gate_up, a.M, a.half, N, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit, order, a.stream, used));
   const auto down = [&](const void* bias) {
     return gemm_m_grouped(a.h_fp8, a.h_scale, order, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H, a.half, a.scatter ? a.row_map : nullptr,
-                          a.scatter ? a.out_rows : 0, bias, a.stream, false, a.few_rows != 0);
+                          a.scatter ? a.out_rows : 0, bias, a.stream, false, a.few_rows != 0, nullptr, 0, used);
   };
   if (a.few_rows)
     PT_STEP_AS(pt_gemm_m_grouped_nt_few_rows, a.M, a.H, a.half, down(a.dn_bias));

@@ -82,6 +82,7 @@ struct QuantArgs {
   int64_t ld_t;                  // row pitch of the transposed twin (bytes = elements); M unless it is a column slice
   int64_t bs_ld;                 // row length of the twin's block-scale grid; tiles_m unless it is a column slice
   float alpha, limit;            // fused clamped SwiGLU: its two constants
+  const int32_t* row_used = nullptr;  // row-scaled launches without a twin: negative where nobody reads row r of the results (null: all are)
   float* col_sum;                // PRO_SUMS and fused clamped SwiGLU backward: [tiles_m, N] column sums of each 128-row tile
   int32_t head_a, head_b;        // per-head halves in two tensors: column h * (head_a + head_b) + c is x[h * head_a + c] or x2[h * head_b + c - head_a]
 };
@@ -237,6 +238,14 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
   const int64_t row0 = (int64_t)tr * 128 + rg * 8;
   const int64_t col0 = (int64_t)tc * 128 + cc * 8;
   const char* xb = reinterpret_cast<const char*>(p.x) + g * p.x_stride_g * Loader<T>::kBytes;
+  if constexpr (AM == A_ROW && (PRO == PRO_NONE || PRO == PRO_SILU_FWD || PRO == PRO_CSWIGLU_FWD)) {
+    // A thread whose eight rows are padding that nobody reads (a thread's sixteen neighbours have the same rows, and
+    // nothing behind this waits for the workgroup).
+    if (p.row_used) {
+      const int4 lo = *reinterpret_cast<const int4*>(p.row_used + row0), hi = *reinterpret_cast<const int4*>(p.row_used + row0 + 4);
+      if ((lo.x & lo.y & lo.z & lo.w & hi.x & hi.y & hi.z & hi.w) < 0) return;
+    }
+  }
 
   Frag<T> f;
   [[maybe_unused]] Frag<T> f_up;  // PRO_SILU_BWD_PAIR only
@@ -876,7 +885,7 @@ static void fill_common(QuantArgs& a, const void* x, int dtype, int64_t M, int64
   a.tiles_m = (int32_t)cdiv(M, 128); a.tiles_n = (int32_t)cdiv(N, 128);
   a.as_rs = a.tiles_n; a.as_ks = 1;
   a.offs = nullptr; a.num_groups = 0; a.row_index = nullptr; a.row_mul = 0; a.x2 = nullptr; a.ldx2 = 0; a.half = 0;
-  a.row_limit = nullptr; a.ld_t = M; a.bs_ld = a.tiles_m; a.alpha = 0.f; a.limit = 0.f; a.col_sum = nullptr;
+  a.row_limit = nullptr; a.ld_t = M; a.bs_ld = a.tiles_m; a.alpha = 0.f; a.limit = 0.f; a.col_sum = nullptr; a.row_used = nullptr;
   a.head_a = a.head_b = 0;
   const int eb = dtype == PT_F32 ? 4 : 2;
   a.vec_in = (N % 8 == 0) && ((ldx * eb) % 16 == 0) && (((uintptr_t)x) % 16 == 0);
@@ -895,7 +904,7 @@ static bool repeat_fits(int64_t rows, int64_t repeat) {
 
 int quant_rowwise_colwise(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
                           void* tok_fp8, float* tok_scale, RowScales order, void* ch_fp8, float* ch_scale, int ch_layout, const int32_t* offs,
-                          int32_t num_groups, pt_stream_t stream, float* col_sum) {
+                          int32_t num_groups, pt_stream_t stream, float* col_sum, const int32_t* row_used) {
   PT_REQUIRE(M >= 0 && N >= 0 && M % 128 == 0, "quant_rowwise_colwise: M=%lld must be a multiple of 128", (long long)M);
   PT_REQUIRE(ldx >= N, "quant_rowwise_colwise: ldx < N");
   PT_REQUIRE(repeat == 1 || (repeat_fits(rows, repeat) && (row_index || M == 0)), "quant_rowwise_colwise: %lld rows, each %lld times, are too many",
@@ -909,6 +918,7 @@ int quant_rowwise_colwise(const void* x, int64_t rows, int64_t repeat, int dtype
   a.row_index = row_index;
   if (repeat > 1) a.row_mul = (uint32_t)(((1ull << 32) + repeat - 1) / repeat);
   if (offs && num_groups > 0) a.row_limit = offs + (num_groups - 1);
+  if (!ch_fp8) a.row_used = row_used;
   hipStream_t s = (hipStream_t)stream;
   if (col_sum) {
     PT_REQUIRE(dtype == PT_BF16 && ch_layout == PT_CH_TRANSPOSED && ch_fp8, "quant_rowwise_colwise: column sums go with bf16 rows and the transposed twin");
@@ -1211,7 +1221,7 @@ static int launch_silu_quant(const QuantArgs& a, hipStream_t stream) {
 
 namespace pt {
 int silu_mul_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up, void* tok_fp8, float* tok_scale, void* ch_t_fp8, float* ch_scale,
-                   const int32_t* valid_rows, RowScales order, pt_stream_t stream) {
+                   const int32_t* valid_rows, RowScales order, pt_stream_t stream, const int32_t* row_used) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half, "silu_mul_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
   PT_REQUIRE(gate_up && tok_fp8 && tok_scale && (ch_t_fp8 == nullptr) == (ch_scale == nullptr), "silu_mul_quant: null pointer");
@@ -1220,6 +1230,7 @@ int silu_mul_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate
   QuantArgs a;
   fill_common(a, gate_up, PT_BF16, M, half, ld_gate_up);
   a.half = half; a.row_limit = valid_rows;
+  if (!ch_t_fp8) a.row_used = row_used;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_t_fp8; a.b_scale = ch_scale;
   order_scales(a, order);
   return launch_silu_quant<PRO_SILU_FWD>(a, (hipStream_t)stream);
@@ -1297,7 +1308,8 @@ extern "C" int pt_silu_mul_bwd_quant_rowwise_transpose_ld(const void* grad_h, in
 // ---- clamped SwiGLU (interleaved gate/up) fused into the activation quantisation -----------------
 namespace pt {
 int clamped_swiglu_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up, float alpha, float limit, void* tok_fp8, float* tok_scale,
-                         void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream) {
+                         void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream,
+                         const int32_t* row_used) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half, "clamped_swiglu_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
   PT_REQUIRE(gate_up && tok_fp8 && tok_scale && (ch_t_fp8 == nullptr) == (ch_scale == nullptr), "clamped_swiglu_quant: null pointer");
@@ -1306,6 +1318,7 @@ int clamped_swiglu_quant(const void* gate_up, int64_t M, int64_t half, int64_t l
   QuantArgs a;
   fill_common(a, gate_up, PT_BF16, M, half, ld_gate_up);
   a.half = half; a.row_limit = valid_rows; a.alpha = alpha; a.limit = limit;
+  if (!ch_t_fp8) a.row_used = row_used;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_t_fp8; a.b_scale = ch_scale;
   order_scales(a, order);
   return launch_silu_quant<PRO_CSWIGLU_FWD>(a, (hipStream_t)stream);

@@ -198,3 +198,41 @@ def test_groups_of_a_few_rows_whose_weights_are_streamed(G, n, k, scatter, bias)
                 want[row : row + r] = y
         row += r
     assert row == M and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("clamp", [None, (1.702, 7.0)])
+def test_padding_of_groups_of_a_few_rows_is_left_out(clamp):
+    """Groups of 64 whose rows go back to their places: nothing is read or written for padding, eight rows at a time.  The
+    bits of the form that writes every grouped row, for counts around the eights, rows left out inside a group and a whole
+    tile of them; what the buffers held before does not matter."""
+    from pith_train_amd.operators.fused_experts import forward_only
+
+    counts = [1, 0, 7, 8, 9, 31, 33, 63, 64, 65, 130]
+    G, K, half, H = len(counts), 400, 272, 264
+    g = torch.Generator().manual_seed(3)
+    ends = torch.tensor([_cdiv(c, 64) * 64 for c in counts]).cumsum(0)
+    M = _cdiv(int(ends[-1]), 128) * 128 + 128  # rows behind the last group
+    row_map, n = torch.full((M,), -1, dtype=torch.int32), 0
+    for q, c in enumerate(counts):
+        first = int(ends[q - 1]) if q else 0
+        row_map[first : first + c] = torch.arange(n, n + c)
+        n += c
+    row_map[int(ends[5]) + 3] = -1                              # a hole
+    row_map[int(ends[9]) : int(ends[9]) + 64] = -1              # a tile of the last group
+    src = torch.randperm(n, generator=g).int()
+    row_map = torch.where(row_map >= 0, src[row_map.clamp_min(0).long()], row_map).cuda()
+    x = torch.randn((n, K), generator=g).bfloat16().cuda()
+    q_gu = _fp8(g, G, 2 * half, K), _scale(g, G, _cdiv(2 * half, 128), _cdiv(K, 128))
+    q_dn = _fp8(g, G, H, half), _scale(g, G, _cdiv(H, 128), _cdiv(half, 128))
+    down = torch.empty((G, H, half), dtype=torch.bfloat16, device="cuda")
+    biases = tuple(torch.randn((G, w), generator=g).bfloat16().cuda() for w in (2 * half, H)) if clamp else (None, None)
+
+    def run(scatter):
+        dirt = [torch.full((8 << 20,), 0xFF, dtype=torch.uint8, device="cuda") for _ in range(4)]  # buffers of not-a-numbers
+        del dirt
+        return forward_only(x, down, ends.int().cuda(), q_gu, q_dn, row_map, scatter=scatter, clamp=clamp, biases=biases, few_rows=True)
+
+    grouped, placed = run(False), run(True)
+    rows = (row_map >= 0).nonzero().squeeze(1)
+    assert placed.shape == (n, H) and torch.equal(placed[row_map[rows].long()], grouped[rows])
+    assert placed[row_map[rows].long()].float().abs().sum() > 0
