@@ -216,15 +216,16 @@ __device__ __forceinline__ float row16_allmax(float v) {
 enum class RowScales { BY_ROW, BY_BLOCK };
 
 // The entry points of the same names (with pt_ in front) with the scales in either form
-// (col_sum: fp32 [M/128, N], the column sums of every 128 rows of x, for bf16 rows and the transposed twin; row_used, without a
-// twin or groups of whole 128-row tiles: negative where nobody reads row r of the results, which may then be left unwritten)
+// (col_sum: fp32 [M/128, N], the column sums of every 128 rows of x, for bf16 rows and the transposed twin; row_used:
+// negative where nobody reads row r of the row-scaled output or of the result, which may then be left unwritten, and whose source may hold anything; the twin is zero there)
 int quant_rowwise_colwise(const void* x, int64_t rows, int64_t repeat, int dtype, int64_t M, int64_t N, int64_t ldx, const int32_t* row_index,
                           void* tok_fp8, float* tok_scale, RowScales order, void* ch_fp8, float* ch_scale, int ch_layout, const int32_t* offs,
                           int32_t num_groups, pt_stream_t stream, float* col_sum = nullptr, const int32_t* row_used = nullptr);
 int silu_mul_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up, void* tok_fp8, float* tok_scale, void* ch_t_fp8, float* ch_scale,
                    const int32_t* valid_rows, RowScales order, pt_stream_t stream, const int32_t* row_used = nullptr);
 int silu_mul_bwd_quant(const void* grad_h, int64_t ld_grad_h, const void* gate_up, int64_t ld_gate_up, int64_t M, int64_t half, void* tok_fp8,
-                       float* tok_scale, void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream);
+                       float* tok_scale, void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream,
+                       const int32_t* row_used = nullptr);
 int clamped_swiglu_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate_up, float alpha, float limit, void* tok_fp8, float* tok_scale,
                          void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream,
                          const int32_t* row_used = nullptr);

@@ -32,7 +32,7 @@ struct GemmArgs {
                                           // out2[h * head_b + c - head_a]; out2 lies behind out in one allocation (head_a == 0: one output)
   int64_t out_extent;                     // with head_a: bytes from out to the end of out2, below 2 GiB
   int few_rows;                           // m-grouped: the group ends are multiples of 64, not of 128
-  const int32_t* row_used;                // with few_rows: negative where row r of a holds nothing, and row r of the result is not wanted
+  const int32_t* row_used;                // m-grouped: negative (with out2: -1) where row r of the result is not wanted; row r of a may hold anything there
   int b_kmajor;                           // m-grouped, row-split kernel: b is [red, rows_b] per group (row pitch ldb) instead of [rows_b, red]
 };
 

@@ -88,14 +88,22 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
     }
   }
   const int nk = (T.k_len + 127) >> 7;
-  if constexpr (MODE == GEMM_M_GROUPED && BM == 64) {
+  if constexpr (MODE == GEMM_M_GROUPED) {
     // Groups of a few rows end in tiles that are padding for the most part (333 tokens of 8 in 128 experts: 21 of 64 rows):
-    // eights of rows behind the last used one are neither loaded nor stored (a block of them, gate_up
-    // and down 178 -> 158 us a pass; 100 tokens of 4 in 32 experts 2880 x 2880 247 -> 217).
+    // eights of rows behind the last used one are neither loaded nor stored.  Stores between the weights' reads cost 0.7 us a
+    // MB: a block of them, gate_up and down 178 -> 158 us a pass; 100 tokens of 4 in 32 experts 2880 x 2880 247 -> 217.
     if (p.row_used) {
-      const uint64_t used = __ballot(p.row_used[T.a_row0 + lane] >= 0);
+      int row[BM / 64];
+#pragma unroll
+      for (int h = 0; h < BM / 64; ++h) row[h] = p.row_used[T.a_row0 + 64 * h + lane];
+      int used = 0;
+#pragma unroll
+      for (int h = 0; h < BM / 64; ++h) {
+        const uint64_t m = __ballot(TWO ? row[h] != -1 : row[h] >= 0);
+        if (m) used = 64 * h + (71 - __builtin_clzll(m)) / 8 * 8;
+      }
       if (!used) return;
-      T.a_lim = T.a_row0 + (71 - __builtin_clzll(used)) / 8 * 8;
+      T.a_lim = T.a_row0 + used;
     }
   }
 
@@ -336,7 +344,7 @@ static int launch_small_mode(const GemmArgs& a, hipStream_t stream) {
       // sees one operand and not what comes between: from half of the cache on it is taken for the first case, below for
       // the others, so a block alone loses a tenth between 128 and 170 MiB and a model 5 to 8 % below 128.  A row that is
       // no whole 128-byte lines shares one with the next (32 experts of 5760 x 2880: 127 us, 132 past the cache).
-      if (BM == 64 && a.few_rows && a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0)
+      if (BM == 64 && !a.out2 && !a.b_kmajor && (a.few_rows || a.row_used) && a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0)
         return launch_small<GEMM_M_GROUPED, 64, false, false, true>(a, stream);
       if (a.out2)
         return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true, false, true>(a, stream)

@@ -434,6 +434,15 @@ struct Dims {
   Pieces backward_temp(bool sums) const { return Pieces({2 * M * half, sums ? M / 128 * half * 8 : 0}); }  // grad_h, column sums
 };
 
+// Whether a block leaves out what stands for padding (PT_PADDING_UNDEFINED): the rows go back to their places, and groups of whole
+// 128-row blocks are padding for a good part: up to 96 rows per expert (d.M holds 127 a group for it), us a pass with padding
+// written / left out: 128 experts of 2048 x 768, 16 rows each 966 / 903, 48 981 / 942, 96 1013 / 1008, 128 1158 / 1167; 64 of
+// 2048 x 1408, 16 839 / 795, 64 860 / 836.  Biases and the clamped activation make other values than zero of padding, which the
+// column scales of the transposed activations see: such blocks write it.
+bool leaves_padding(const Dims& d, bool placed, bool biased) {
+  return placed && !biased && d.M <= (127 + 96) * d.G;
+}
+
 // Forward of an expert block (see fused_experts._forward): (out, gate_up, kept buffers).
 std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x, int64_t repeat, const Maybe& row_map, const Maybe& expand_idx,
                                                                 const Tensor& offs, const Tensor& gu, const Tensor& gu_s, const Tensor& dn,
@@ -465,7 +474,7 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x,
   a.M = d.M; a.K = K; a.half = half; a.H = d.H; a.G = d.G;
   a.offs = (const int32_t*)ptr(offs); a.row_map = (const int32_t*)ptr(row_map);
   a.expand_idx = (const int64_t*)ptr(expand_idx); a.n_expand = expand_idx ? routed : 0;
-  a.repeat = repeat; a.few_rows = few_rows;
+  a.repeat = repeat; a.few_rows = few_rows ? 1 : keep && leaves_padding(d, (bool)row_map && scatter, clamped || gu_bias) ? PT_PADDING_UNDEFINED : 0;
   a.gu_fp8 = ptr(gu); a.gu_scale = (const float*)ptr(gu_s); a.gu_bias = ptr(gu_bias);
   a.dn_fp8 = ptr(dn); a.dn_scale = (const float*)ptr(dn_s); a.dn_bias = ptr(dn_bias);
   a.gate_up = ptr(gate_up); a.out = ptr(out); a.out_rows = out.size(0); a.scatter = scatter;
@@ -541,7 +550,7 @@ struct ExpertsBackward {
     if (weights.size() > 0) down.aim(weights[0]);
     a.grad_out = ptr(grad_out); a.grad_rows = grad_out.size(0);
     a.M = d.M; a.K = d.K; a.half = d.half; a.H = d.H; a.G = d.G;
-    a.offs = (const int32_t*)ptr(offs); a.out_map = scatter ? (const int32_t*)ptr(row_map) : nullptr; a.limit_rows = (bool)row_map;
+    a.offs = (const int32_t*)ptr(offs); a.out_map = scatter ? (const int32_t*)ptr(row_map) : nullptr; a.limit_rows = leaves_padding(d, row_map && scatter, clamped || gu_bias_like) ? PT_PADDING_UNDEFINED : (bool)row_map;
     a.dn_dg = ptr(dn_dg); a.dn_dg_scale = (const float*)ptr(dn_dg_s); a.dn_forward_layout = dn_forward;
     a.gate_up = ptr(gate_up_saved);
     a.x_t = kept.at(0); a.x_t_scale = (const float*)kept.at(1); a.h_t = kept.at(2); a.h_t_scale = (const float*)kept.at(3);

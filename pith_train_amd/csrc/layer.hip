@@ -54,14 +54,16 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order)
   PT_REQUIRE(a.offs && a.gate_up && a.out && a.x_fp8 && a.x_scale && a.h_fp8 && a.h_scale && keep == (a.h_t != nullptr) &&
                  keep == (a.x_t_scale != nullptr) && keep == (a.h_t_scale != nullptr), "experts_forward: null pointer");
   PT_REQUIRE(a.repeat >= 1 && (a.repeat == 1 || (a.row_map && !a.expand_idx)), "experts_forward: repeat needs row_map and no expand_idx");
-  PT_REQUIRE(!a.few_rows || !keep, "experts_forward: a backward needs groups of whole 128-row blocks");
+  PT_REQUIRE(a.few_rows == PT_PADDING_UNDEFINED || !a.few_rows || !keep, "experts_forward: a backward needs groups of whole 128-row blocks");
   PT_REQUIRE(!a.expand_idx || a.composed_map, "experts_forward: expand_idx needs composed_map");
   PT_REQUIRE(a.row_map || (!a.expand_idx && !a.scatter), "experts_forward: expand_idx and scatter need row_map");
   if (a.M == 0) return PT_OK;
   const int32_t G = (int32_t)a.G;
   const int32_t* limit = a.row_map ? a.offs + G - 1 : nullptr;  // rows past it hold nothing
   const int32_t* in_map = a.row_map;
-  // where the rows go back to their places, nobody sees what stands for the padding of groups of 64
+  // where the rows go back to their places, nobody sees what stands for padding
+  const bool few = a.few_rows && a.few_rows != PT_PADDING_UNDEFINED;
+  PT_REQUIRE(a.few_rows != PT_PADDING_UNDEFINED || (keep && a.scatter && !a.gu_bias && !a.clamped), "experts_forward: padding is left out of scattered rows of a SwiGLU block only");
   const int32_t* used = a.few_rows && a.scatter ? a.row_map : nullptr;
   if (a.expand_idx) {
     PT_STEP(pt_compose_row_map, a.M, 0, 0, a.row_map, a.M, a.expand_idx, a.n_expand, a.x_rows, a.composed_map, a.stream);
@@ -80,9 +82,9 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order)
   const int64_t N = 2 * a.half;
   const auto gate_up = [&](const void* bias) {
     return gemm_m_grouped(a.x_fp8, a.x_scale, order, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M, N, a.K, nullptr, 0, bias, a.stream,
-                          false, a.few_rows != 0, nullptr, 0, used);
+                          false, few, nullptr, 0, used);
   };
-  if (a.few_rows)
+  if (few)
     PT_STEP_AS(pt_gemm_m_grouped_nt_few_rows, a.M, N, a.K, gate_up(a.gu_bias));
   else if (a.gu_bias)
     PT_STEP_AS(pt_gemm_m_grouped_nt_bias, a.M, N, a.K, gate_up(a.gu_bias));
@@ -97,9 +99,9 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order)
                silu_mul_quant(a.gate_up, a.M, a.half, N, a.h_fp8, a.h_scale, a.h_t, a.h_t_scale, limit, order, a.stream, used));
   const auto down = [&](const void* bias) {
     return gemm_m_grouped(a.h_fp8, a.h_scale, order, a.dn_fp8, a.dn_scale, a.out, PT_BF16, a.offs, G, a.M, a.H, a.half, a.scatter ? a.row_map : nullptr,
-                          a.scatter ? a.out_rows : 0, bias, a.stream, false, a.few_rows != 0, nullptr, 0, used);
+                          a.scatter ? a.out_rows : 0, bias, a.stream, false, few, nullptr, 0, used);
   };
-  if (a.few_rows)
+  if (few)
     PT_STEP_AS(pt_gemm_m_grouped_nt_few_rows, a.M, a.H, a.half, down(a.dn_bias));
   else if (a.scatter && a.dn_bias)
     PT_STEP_AS(pt_gemm_m_grouped_nt_scatter_bias, a.M, a.H, a.half, down(a.dn_bias));
@@ -121,6 +123,8 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
   if (a.M == 0) return PT_OK;
   const int32_t G = (int32_t)a.G;
   const int32_t* limit = a.limit_rows ? a.offs + G - 1 : nullptr;
+  PT_REQUIRE(a.limit_rows != PT_PADDING_UNDEFINED || (a.out_map && !a.clamped && !a.d_gu_bias), "experts_backward: padding is left out of scattered rows of a SwiGLU block only");
+  const int32_t* used = a.limit_rows == PT_PADDING_UNDEFINED ? a.out_map : nullptr;
   // The gradient of the down bias is the sum of the rows that are quantised here: the kernel that reads them adds up
   // every 128 (groups are whole 128-row tiles) where col_sum, which the activation's backward fills afterwards, has
   // room for those sums (16384 tokens x 4 of 2880 columns: a second pass over the rows took 110 us, the sums here cost
@@ -128,7 +132,7 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
   float* const dy_sums = a.d_dn_bias && a.clamped && a.H <= 2 * a.half ? a.col_sum : nullptr;
   const auto quant_dy = [&](const int32_t* ends) {
     return quant_rowwise_colwise(a.grad_out, a.grad_rows, 1, PT_BF16, a.M, a.H, a.H, a.out_map, a.dy_fp8, a.dy_scale, order, a.dy_t, a.dy_t_scale,
-                                 PT_CH_TRANSPOSED, ends, ends ? G : 0, a.stream, dy_sums);
+                                 PT_CH_TRANSPOSED, ends, ends ? G : 0, a.stream, dy_sums, used);
   };
   if (a.out_map)
     PT_STEP_AS(pt_quant_rowwise_colwise_rows, a.M, a.H, a.grad_rows, quant_dy(a.offs));
@@ -145,7 +149,7 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
   }
   const auto grad_h = [&] {
     return gemm_m_grouped(a.dy_fp8, a.dy_scale, order, a.dn_dg, a.dn_dg_scale, a.grad_h, PT_BF16, a.offs, G, a.M, a.half, a.H, nullptr, 0, nullptr,
-                          a.stream, a.dn_forward_layout != 0);
+                          a.stream, a.dn_forward_layout != 0, false, nullptr, 0, used);
   };
   if (a.dn_forward_layout)
     PT_STEP_AS(pt_gemm_m_grouped_nn, a.M, a.half, a.H, grad_h());
@@ -161,7 +165,7 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
   else
     PT_STEP_AS(pt_silu_mul_bwd_quant_rowwise_colwise, a.M, a.half, 0,
                silu_mul_bwd_quant(a.grad_h, a.half, a.gate_up, 2 * a.half, a.M, a.half, a.dgu_fp8, a.dgu_scale, a.dgu_t, a.dgu_t_scale, limit, order,
-                                  a.stream));
+                                  a.stream, used));
   if (a.d_gu_bias)  // groups are whole 128-row tiles: their ends in tiles index the per-tile column sums
     PT_STEP(pt_segment_sum_tiles, a.M / 128, 2 * a.half, 0, a.col_sum, a.offs, 128, G, a.d_gu_bias, a.M / 128, 2 * a.half,
             (int)a.d_gu_bias_dtype, a.stream);

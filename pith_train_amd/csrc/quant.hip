@@ -82,7 +82,7 @@ struct QuantArgs {
   int64_t ld_t;                  // row pitch of the transposed twin (bytes = elements); M unless it is a column slice
   int64_t bs_ld;                 // row length of the twin's block-scale grid; tiles_m unless it is a column slice
   float alpha, limit;            // fused clamped SwiGLU: its two constants
-  const int32_t* row_used = nullptr;  // row-scaled launches without a twin: negative where nobody reads row r of the results (null: all are)
+  const int32_t* row_used = nullptr;  // row-scaled launches: negative where nobody reads row r of the row-scaled output and the twin's is zero (null: all are)
   float* col_sum;                // PRO_SUMS and fused clamped SwiGLU backward: [tiles_m, N] column sums of each 128-row tile
   int32_t head_a, head_b;        // per-head halves in two tensors: column h * (head_a + head_b) + c is x[h * head_a + c] or x2[h * head_b + c - head_a]
 };
@@ -238,18 +238,27 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
   const int64_t row0 = (int64_t)tr * 128 + rg * 8;
   const int64_t col0 = (int64_t)tc * 128 + cc * 8;
   const char* xb = reinterpret_cast<const char*>(p.x) + g * p.x_stride_g * Loader<T>::kBytes;
-  if constexpr (AM == A_ROW && (PRO == PRO_NONE || PRO == PRO_SILU_FWD || PRO == PRO_CSWIGLU_FWD)) {
-    // A thread whose eight rows are padding that nobody reads (a thread's sixteen neighbours have the same rows, and
-    // nothing behind this waits for the workgroup).
+  // Eight rows of padding that nobody reads: they are not read, hold zeros in the twin and are not written to the other output
+  // (a thread's sixteen neighbours have the same rows; without a twin nothing behind this waits for the workgroup).
+  bool idle = false;
+  constexpr bool kCanIdle = AM == A_ROW && (PRO == PRO_NONE || PRO == PRO_SILU_FWD || PRO == PRO_CSWIGLU_FWD || PRO == PRO_SILU_BWD || PRO == PRO_SILU_BWD_PAIR);
+  if constexpr (kCanIdle) {
     if (p.row_used) {
       const int4 lo = *reinterpret_cast<const int4*>(p.row_used + row0), hi = *reinterpret_cast<const int4*>(p.row_used + row0 + 4);
-      if ((lo.x & lo.y & lo.z & lo.w & hi.x & hi.y & hi.z & hi.w) < 0) return;
+      idle = (lo.x & lo.y & lo.z & lo.w & hi.x & hi.y & hi.z & hi.w) < 0;
+      if (idle && !p.b_out) return;
     }
   }
 
   Frag<T> f;
   [[maybe_unused]] Frag<T> f_up;  // PRO_SILU_BWD_PAIR only
-  if constexpr (PRO == PRO_SILU_BWD_PAIR) {
+  if (kCanIdle && idle) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      f.zero_row(i);
+      if constexpr (PRO == PRO_SILU_BWD_PAIR) f_up.zero_row(i);
+    }
+  } else if constexpr (PRO == PRO_SILU_BWD_PAIR) {
     const bool col_ok = FULL || col0 < p.half;
     // Two rows in flight: row i + 2 is addressed through a register that an empty assembly statement
     // ties to the packed results of row i.  Left alone, the compiler starts all eight rows at once
@@ -492,7 +501,7 @@ __device__ __forceinline__ void quant_tile_body(const QuantArgs& p, float (*s_co
   };
   // Row-scaled output needs nothing from the other phases: write it now so that the row maxima
   // are dead before the column phase starts (fewer live registers, more resident waves).
-  if (AM == A_ROW && p.a_out) write_same_orientation(0.f, 0.f);
+  if (AM == A_ROW && p.a_out && !idle) write_same_orientation(0.f, 0.f);
   if (AM == A_ROW && !p.b_out) return;  // nobody reads the twin (no backward follows)
 
   f.fence();
@@ -918,7 +927,7 @@ int quant_rowwise_colwise(const void* x, int64_t rows, int64_t repeat, int dtype
   a.row_index = row_index;
   if (repeat > 1) a.row_mul = (uint32_t)(((1ull << 32) + repeat - 1) / repeat);
   if (offs && num_groups > 0) a.row_limit = offs + (num_groups - 1);
-  if (!ch_fp8) a.row_used = row_used;
+  a.row_used = row_used;
   hipStream_t s = (hipStream_t)stream;
   if (col_sum) {
     PT_REQUIRE(dtype == PT_BF16 && ch_layout == PT_CH_TRANSPOSED && ch_fp8, "quant_rowwise_colwise: column sums go with bf16 rows and the transposed twin");
@@ -1230,7 +1239,7 @@ int silu_mul_quant(const void* gate_up, int64_t M, int64_t half, int64_t ld_gate
   QuantArgs a;
   fill_common(a, gate_up, PT_BF16, M, half, ld_gate_up);
   a.half = half; a.row_limit = valid_rows;
-  if (!ch_t_fp8) a.row_used = row_used;
+  a.row_used = row_used;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_t_fp8; a.b_scale = ch_scale;
   order_scales(a, order);
   return launch_silu_quant<PRO_SILU_FWD>(a, (hipStream_t)stream);
@@ -1244,7 +1253,8 @@ extern "C" int pt_silu_mul_quant_rowwise_colwise(const void* gate_up, int64_t M,
 
 namespace pt {
 int silu_mul_bwd_quant(const void* grad_h, int64_t ld_grad_h, const void* gate_up, int64_t ld_gate_up, int64_t M, int64_t half, void* tok_fp8,
-                       float* tok_scale, void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream) {
+                       float* tok_scale, void* ch_t_fp8, float* ch_scale, const int32_t* valid_rows, RowScales order, pt_stream_t stream,
+                       const int32_t* row_used) {
   PT_REQUIRE(M >= 0 && half >= 0 && M % 128 == 0 && ld_gate_up >= 2 * half && ld_grad_h >= half, "silu_mul_bwd_quant: bad shape");
   if (M == 0 || half == 0) return PT_OK;
   PT_REQUIRE(grad_h && gate_up && tok_fp8 && tok_scale && ch_t_fp8 && ch_scale, "silu_mul_bwd_quant: null pointer");
@@ -1253,7 +1263,7 @@ int silu_mul_bwd_quant(const void* grad_h, int64_t ld_grad_h, const void* gate_u
              "silu_mul_bwd_quant: widths and row strides must be multiples of 8 elements, pointers 16-byte aligned");
   QuantArgs a;
   fill_common(a, grad_h, PT_BF16, M, 2 * half, ld_grad_h);
-  a.half = half; a.x2 = gate_up; a.ldx2 = ld_gate_up; a.row_limit = valid_rows;
+  a.half = half; a.x2 = gate_up; a.ldx2 = ld_gate_up; a.row_limit = valid_rows; a.row_used = row_used;
   a.a_out = (uint8_t*)tok_fp8; a.a_scale = tok_scale; a.b_out = (uint8_t*)ch_t_fp8; a.b_scale = ch_scale;
   order_scales(a, order);
   // with whole 128-column tiles per half, each workgroup makes a dgate tile and its dup twin

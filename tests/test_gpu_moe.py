@@ -652,3 +652,47 @@ def test_steps_with_row_scales_by_row_and_by_block_agree_bit_for_bit(form):
         got = blocks[name].t() if name.endswith("_scale") else blocks[name]
         assert want.float().abs().sum() > 0 or name == "map" or (not clamped and name in ("sums", "d_gu", "d_dn")), name
         assert torch.equal(want, got), name
+
+
+@pytest.mark.parametrize("kind", ["fused", "split"])
+@pytest.mark.parametrize("E,H,I,T,k,dedup,holes", [
+    (8, 272, 256, 40, 2, False, False),      # ten rows an expert, ragged widths
+    (130, 256, 128, 64, 8, False, True),     # four; some experts get none, one all of 64 tokens
+    (6, 1040, 384, 250, 2, True, False),     # 83: eights that end inside a tile; rows of the expanded form
+    (4, 256, 128, 384, 1, False, False),     # 96, the most for which padding is left out
+    (4, 256, 128, 390, 1, False, False),     # and more
+])
+def test_training_step_that_leaves_padding_out(kind, E, H, I, T, k, dedup, holes):
+    """Few rows per expert: padding is neither read nor written but for the zeros of the transposed operands.  The bits of the
+    scatter, the block on its grouped rows, and the gather, whatever the buffers held before."""
+    from pith_train_amd.dualpipe_utils import FP8WeightCacheControl
+    from pith_train_amd.modules.experts import Qwen3MoeExperts, Qwen35MoeExperts, forward_stage3
+
+    g = torch.Generator(device="cuda").manual_seed(E + T)
+    mod = (Qwen35MoeExperts if kind == "fused" else Qwen3MoeExperts)(H, I, E).cuda().bfloat16()
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.normal_(0.0, 0.02, generator=g)
+    scores = torch.rand((T, E), device="cuda", generator=g)
+    if holes:
+        scores[:, ::7] = -1.0
+        scores[:, 3] = 2.0
+    ids = scores.topk(k, dim=1).indices.reshape(-1)
+    rows = T * k
+    expand = torch.randint(0, rows - rows // 4, (rows,), device="cuda", generator=g) if dedup else None
+    x = torch.randn((rows - rows // 4 if dedup else rows, H), device="cuda", generator=g).bfloat16()
+    grad = torch.randn((rows, H), device="cuda", generator=g).bfloat16()
+
+    def run(fuse_permute):
+        FP8WeightCacheControl.step()
+        mod.zero_grad(set_to_none=True)
+        dirt = [torch.full((n << 20,), 0xFF, dtype=torch.uint8, device="cuda") for n in (1, 1, 2, 2, 4, 8, 16, 32)]  # not-a-numbers
+        del dirt
+        t = x.clone().requires_grad_(True)
+        out = forward_stage3(mod, t, ids, E, expand_idx=expand, fuse_permute=fuse_permute)
+        out.backward(grad)
+        return [out.detach(), t.grad] + [p.grad for p in mod.parameters()]
+
+    ours, composed = run(True), run(False)
+    for n, (a, b) in enumerate(zip(ours, composed)):
+        assert b.float().abs().sum() > 0 and torch.equal(a, b), n
