@@ -144,7 +144,7 @@ __device__ __forceinline__ void small_tile_body(const GemmArgs& p, int block) {
 #pragma unroll
     for (int k = 0; k < LB; ++k) {
       const int q = NW * k + wave;
-      if constexpr (BT) dma16(rs_b, ok && bt_in ? vb : kOob, soB0 + (koff + 8 * q) * (uint32_t)p.ldb, sB + q * 1024);
+      if constexpr (BT) dma16<STREAM>(rs_b, ok && bt_in ? vb : kOob, soB0 + (koff + 8 * q) * (uint32_t)p.ldb, sB + q * 1024);
       else              dma16<STREAM>(rs_b, in ? vb : kOob, soB0 + koff + (uint32_t)(8 * q) * (uint32_t)p.ldb, sB + q * 1024);
     }
     const uint32_t dst = sc_real ? sc_base + slot * (BM + BN) * 4 + wave * 256 : sc_base + NS * (BM + BN) * 4;
@@ -335,7 +335,7 @@ static int launch_small_mode(const GemmArgs& a, hipStream_t stream) {
   switch (a.mode) {
     case GEMM_DENSE: return launch_small<GEMM_DENSE, BM, false, false>(a, stream);
     case GEMM_M_GROUPED:
-      // Groups of up to 64 rows read their weights once.  Past the memory-side cache (256 MiB) they arrive faster, whatever
+      // Groups of one or two tiles of rows read their weights once or, from the L2, twice.  Past the memory-side cache (256 MiB) they arrive faster, whatever
       // their size, when the weights of other layers are read before they are wanted again, as in a model (1536 x 2048 an
       // expert, us through the cache / past it: 96 MiB 25.7 / 23.8, 129 MiB 36.9 / 33.8, 192 40.9 / 37.9, 384 80.1 / 74.8).
       // A block that runs alone finds what is left of its own last pass, while its two operands fit together (gate_up and
@@ -344,8 +344,16 @@ static int launch_small_mode(const GemmArgs& a, hipStream_t stream) {
       // sees one operand and not what comes between: from half of the cache on it is taken for the first case, below for
       // the others, so a block alone loses a tenth between 128 and 170 MiB and a model 5 to 8 % below 128.  A row that is
       // no whole 128-byte lines shares one with the next (32 experts of 5760 x 2880: 127 us, 132 past the cache).
-      if (BM == 64 && !a.out2 && !a.b_kmajor && (a.few_rows || a.row_used) && a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0)
-        return launch_small<GEMM_M_GROUPED, 64, false, false, true>(a, stream);
+      // Training steps, whose weights are read again only after the other layers', through / past, us a pass: 128 experts of
+      // 2048 x 768, 16 rows each 903 / 856, 64 964 / 914; 64 of 2048 x 1408, 16 rows 798 / 760; 128 of 2048 x 512, 64 rows 704 /
+      // 649; with single operators 128 of 2048 x 768, 48 rows 1217 / 1195.
+      if (a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0) {
+        if (a.out2)
+          return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true, true, true>(a, stream)
+                            : launch_small<GEMM_M_GROUPED, BM, false, false, true, true>(a, stream);
+        return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true, true>(a, stream)
+                          : launch_small<GEMM_M_GROUPED, BM, false, false, true>(a, stream);
+      }
       if (a.out2)
         return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true, false, true>(a, stream)
                           : launch_small<GEMM_M_GROUPED, BM, false, false, false, true>(a, stream);

@@ -236,3 +236,32 @@ def test_padding_of_groups_of_a_few_rows_is_left_out(clamp):
     rows = (row_map >= 0).nonzero().squeeze(1)
     assert placed.shape == (n, H) and torch.equal(placed[row_map[rows].long()], grouped[rows])
     assert placed[row_map[rows].long()].float().abs().sum() > 0
+
+
+@pytest.mark.parametrize("form", ["nt", "nn", "scatter", "nn scatter"])
+def test_weights_past_the_memory_side_cache_in_tiles_of_128_rows(form):
+    """Weights of 128 MiB and more of whole lines are loaded past that cache: the bits of the large tiles' kernel, for one,
+    several and no tile of rows a group."""
+    from pith_train_amd import _lib
+    from pith_train_amd.operators.grouped_linear import m_grouped_fp8_gemm_nn, m_grouped_fp8_gemm_nt
+
+    g = torch.Generator().manual_seed(5)
+    G, N, K = 68, 1024, 2048
+    rows = torch.tensor([128, 0, 384] + [128] * (G - 4) + [256])
+    offs, M = rows.cumsum(0).int().cuda(), int(rows.sum())
+    a = _fp8(g, M, K), _scale(g, M, K // 128)
+    nn = "nn" in form
+    gemm = m_grouped_fp8_gemm_nn if nn else m_grouped_fp8_gemm_nt
+    one = _fp8(g, 1, K, N) if nn else _fp8(g, 1, N, K)
+    b = one.view(torch.uint8).repeat(G, 1, 1)
+    b[G // 2] = b[G // 2].flip(0)
+    b = b.view(one.dtype), _scale(g, G, K // 128, N // 128) if nn else _scale(g, G, N // 128, K // 128)
+    assert b[0].numel() >= 128 << 20
+    index = (torch.randperm(M, generator=g).int().cuda(),) if "scatter" in form else ()
+    out = []
+    for kernel in (b"s128", b"r0"):
+        _lib.call("pt_gemm_select_kernel", kernel)
+        out.append(torch.zeros((M, N), device="cuda", dtype=torch.bfloat16))
+        gemm(a, b, out[-1], offs, *index)
+    _lib.call("pt_gemm_select_kernel", b"auto")
+    assert out[0].float().abs().sum() > 0 and torch.equal(*out)
