@@ -309,10 +309,13 @@ static int small_tile_rows(const GemmArgs& g) {
   const int64_t groups = g.mode == GEMM_K_GROUPED ? g.G : 1;
   const int64_t cols = cdiv(g.rows_b, 128) * groups, cols_large = cdiv(g.rows_b, 256) * groups;
   if (cdiv(g.rows_a, 64) * cols <= 256) return 64;
-  // Where padding is known and left out, up to 96 rows a group (the row count holds 127 more for each): 128-row tiles, which end
+  // Where padding is known and left out, up to 96 rows a group (the row count holds 127 more for each and some): 128-row tiles, which end
   // at their last used row.  Layers of 128 experts 2048 x 768, us a pass in large tiles / these: 16 rows each 943 / 903, 48 974 /
   // 942, 96 1029 / 1008, 128 1170 / 1167, 200 1249 / 1300; in tiles of 64 rows, of which every second finds nothing, 969 at 16.
-  if (g.row_used && g.rows_a <= (127 + 96) * (int64_t)g.G) return 128;
+  if (g.row_used && g.rows_a <= 224 * (int64_t)g.G + 256) return 128;
+  // Weights that come from HBM and are read once, mostly: single operators on 128 groups of 48 rows 2048 x 768 1191 / 1182, of 96
+  // 1222 / 1209.
+  if (g.mode == GEMM_M_GROUPED && streams_weights(g) && g.rows_a <= 140 * (int64_t)g.G) return 128;
   int64_t small = cdiv(g.rows_a, 128) * cols;
   if (small <= 256 && g.mode == GEMM_DENSE && g.red >= 1792) return kDeepTile;
   if (small <= 512) return 128;

@@ -44,6 +44,9 @@ __device__ __forceinline__ int k_group_end(const GemmArgs& p, int g) {
 }
 
 
+// m-grouped: weights that the small-problem kernel loads past the memory-side cache (launch_small_mode has the rule's reasons)
+inline bool streams_weights(const GemmArgs& a) { return a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0; }
+
 // persistent kernel whose two steps per 128-block split the tile by rows (gemm_rowsplit.hip)
 int launch_gemm_rowsplit(const GemmArgs& a, hipStream_t stream);
 // one tile of 64 or 128 rows x 128 columns per workgroup, for small problems (gemm_small.hip); kDeepTile: 128 rows, one

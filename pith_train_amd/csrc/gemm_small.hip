@@ -347,7 +347,7 @@ static int launch_small_mode(const GemmArgs& a, hipStream_t stream) {
       // Training steps, whose weights are read again only after the other layers', through / past, us a pass: 128 experts of
       // 2048 x 768, 16 rows each 903 / 856, 64 964 / 914; 64 of 2048 x 1408, 16 rows 798 / 760; 128 of 2048 x 512, 64 rows 704 /
       // 649; with single operators 128 of 2048 x 768, 48 rows 1217 / 1195.
-      if (a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0) {
+      if (streams_weights(a)) {
         if (a.out2)
           return a.b_kmajor ? launch_small<GEMM_M_GROUPED, BM, false, true, true, true>(a, stream)
                             : launch_small<GEMM_M_GROUPED, BM, false, false, true, true>(a, stream);
