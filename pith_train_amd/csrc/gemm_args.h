@@ -44,6 +44,9 @@ __device__ __forceinline__ int k_group_end(const GemmArgs& p, int g) {
 }
 
 
+// m-grouped: groups from which on the kernel of large tiles looks for the padding behind each
+static constexpr int kPaddedGroups = 64;
+
 // m-grouped: weights that the small-problem kernel loads past the memory-side cache (launch_small_mode has the rule's reasons)
 inline bool streams_weights(const GemmArgs& a) { return a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0; }
 

@@ -436,11 +436,12 @@ struct Dims {
 
 // Whether a block leaves out what stands for padding (PT_PADDING_UNDEFINED): the rows go back to their places, and groups of whole
 // 128-row blocks are padding for a good part: up to 96 rows per expert (d.M holds 127 a group and up to 255 for it), us a pass with padding
-// written / left out: 128 experts of 2048 x 768, 16 rows each 966 / 903, 48 981 / 942, 96 1013 / 1008, 128 1158 / 1167; 64 of
-// 2048 x 1408, 16 839 / 795, 64 860 / 836.  Biases and the clamped activation make other values than zero of padding, which the
+// written / left out: 128 experts of 2048 x 768, 16 rows each 966 / 903, 48 981 / 942, 96 1013 / 1008; 64 of
+// 2048 x 1408, 16 839 / 795, 64 860 / 836; and from 64 groups on, whatever their rows, where the kernel of large tiles looks for it
+// (gemm_rowsplit.hip has both sides).  Biases and the clamped activation make other values than zero of padding, which the
 // column scales of the transposed activations see: such blocks write it.
 bool leaves_padding(const Dims& d, bool placed, bool biased) {
-  return placed && !biased && d.M <= 224 * d.G + 256;
+  return placed && !biased && (d.M <= 224 * d.G + 256 || d.G >= 64);
 }
 
 // Forward of an expert block (see fused_experts._forward): (out, gate_up, kept buffers).

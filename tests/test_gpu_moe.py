@@ -661,6 +661,7 @@ def test_steps_with_row_scales_by_row_and_by_block_agree_bit_for_bit(form):
     (6, 1040, 384, 250, 2, True, False),     # 83: eights that end inside a tile; rows of the expanded form
     (4, 256, 128, 384, 1, False, False),     # 96, the most for which padding is left out
     (4, 256, 128, 390, 1, False, False),     # and more
+    (66, 528, 384, 2900, 6, True, True),     # many groups of the large tiles' kernel: ends of groups of every length
 ])
 def test_training_step_that_leaves_padding_out(kind, E, H, I, T, k, dedup, holes):
     """Few rows per expert: padding is neither read nor written but for the zeros of the transposed operands.  The bits of the
