@@ -453,9 +453,13 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(CeArgs p, uint32_t blocks
       S::store1(q, S::load1(q) * s);
     }
     ce_v4i w[4];
+    if (r.chunks == 0) return;
+    // (from a clamped place: behind a condition each load would wait for the one before)
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (c0 + q * 256 < r.chunks) w[q] = (PT_CE_NT & 1) ? __builtin_nontemporal_load(body + c0 + q * 256) : body[c0 + q * 256];
+    for (int q = 0; q < 4; ++q) {
+      const ce_v4i* from = body + (c0 + q * 256 < r.chunks ? c0 + q * 256 : r.chunks - 1);
+      w[q] = (PT_CE_NT & 1) ? __builtin_nontemporal_load(from) : *from;
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if (c0 + q * 256 < r.chunks) {

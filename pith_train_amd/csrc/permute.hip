@@ -158,6 +158,111 @@ __global__ __launch_bounds__(256) void gr_rank_kernel(const int64_t* keys, int64
   }
 }
 
+// The sort in two launches: the histograms are those of blocks of 1024 keys, and the workgroups of the second launch add up
+// the others' themselves, up to kBlockCounts numbers (64 KiB from the L2 each), instead of waiting for two scans in launches
+// of their own.  Four launches / two, us: 65 536 keys of 128 groups 15.3 / 12.6, 131 072 18.2 / 17.3, 32 768 of 16 12.8 / 7.7,
+// 262 144 of 64 22.5 / 17.0; past the limit 262 144 of 128 24.1 / 25.9.  (One workgroup and two launches: 4096 keys of 128 groups
+// 8.5 / 8.7, 8192 12.6 / 9.1; but so short a list belongs to a step that waits for the host, whom a launch costs 4.)
+static constexpr int kBlockKeys = 4 * kWaveKeys, kBlockCounts = 16384, kBlockGroups = 256;
+__global__ __launch_bounds__(256) void gr_block_hist_kernel(const int64_t* keys, int64_t m, int G, int32_t* counts /*[blocks][G]*/, int32_t* src_of,
+                                                            int64_t cap) {
+  __shared__ int32_t s_hist[kBlockGroups];
+  const int t = threadIdx.x;
+  for (int g = t; g < G; g += 256) s_hist[g] = 0;
+  int64_t k[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t i = (int64_t)blockIdx.x * kBlockKeys + 256 * u + t;
+    k[u] = i < m ? keys[i] : -1;
+  }
+  for (int64_t i = (int64_t)blockIdx.x * 256 + t; i < cap; i += (int64_t)gridDim.x * 256) src_of[i] = -1;  // (see gr_hist_kernel)
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (k[u] >= 0 && k[u] < G) atomicAdd(&s_hist[k[u]], 1);
+  __syncthreads();
+  for (int g = t; g < G; g += 256) counts[(int64_t)blockIdx.x * G + g] = s_hist[g];
+}
+
+__global__ __launch_bounds__(256) void gr_block_rank_kernel(const int64_t* keys, int64_t m, int G, int nbits, int alignment, const int32_t* counts,
+                                                            int32_t* offs, int32_t* ks, int64_t* reverse, int32_t* src_of, int64_t cap) {
+  __shared__ int32_t s_run[4 * kBlockGroups], s_total[kBlockGroups], s_before[kBlockGroups], s_w[4];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, block = blockIdx.x, blocks = gridDim.x;
+  int32_t* run = s_run + wave * G;
+  const int64_t base = (int64_t)block * kBlockKeys + wave * kWaveKeys;
+  int64_t keys4[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t i = base + 64 * u + lane;
+    keys4[u] = i < m ? keys[i] : -1;
+  }
+  for (int g = t; g < G; g += 256) s_total[g] = s_before[g] = 0;
+  for (int g = lane; g < G; g += 64) run[g] = 0;
+  __syncthreads();
+  // every group's keys in all blocks and in those before this one: as many threads to a group as there are
+  const int parts = 256 / G, g = t % G, part = t / G;
+  if (part < parts) {
+    int32_t total = 0, before = 0;
+#pragma unroll 16
+    for (int b = part; b < blocks; b += parts) {
+      const int32_t c = counts[b * G + g];
+      total += c;
+      before += b < block ? c : 0;
+    }
+    if (total) {
+      atomicAdd(&s_total[g], total);
+      if (before) atomicAdd(&s_before[g], before);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (keys4[u] >= 0 && keys4[u] < G) atomicAdd(&run[keys4[u]], 1);
+  __syncthreads();
+  // thread g: the group's padded size, where it starts, and where each wave's rows do
+  const int32_t size = t < G ? (int32_t)(((int64_t)s_total[t] + alignment - 1) / alignment * alignment) : 0;
+  int32_t incl = size;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t up = __shfl_up(incl, d);
+    if (lane >= d) incl += up;
+  }
+  if (lane == 63) s_w[wave] = incl;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) incl += w < wave ? s_w[w] : 0;
+  if (t < G) {
+    int32_t at = incl - size + s_before[t];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int32_t c = s_run[w * G + t];
+      s_run[w * G + t] = at;
+      at += c;
+    }
+    if (block == 0) {
+      offs[t] = incl;
+      ks[t] = size;
+    }
+  }
+  __syncthreads();
+  const uint64_t lt = lanemask_lt();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t i = base + 64 * u + lane;
+    int64_t k = keys4[u];
+    const bool active = i < m && k >= 0 && k < G;
+    if (!active) k = 0;
+    const uint64_t mask = wave_match((uint32_t)k, active, nbits);
+    const int rank = __popcll(mask & lt);
+    const int32_t b = run[k];
+    __builtin_amdgcn_wave_barrier();
+    if (active && rank == 0) run[k] = b + __popcll(mask);
+    __builtin_amdgcn_wave_barrier();
+    const int64_t pos = active ? (int64_t)b + rank : 0;  // a key outside [0, G): see gr_rank_kernel
+    if (i < m && reverse) reverse[i] = pos;
+    if (active && pos < cap) src_of[pos] = (int32_t)i;
+  }
+}
+
 // The whole sort in one workgroup, for lists short enough that three more launches cost more than one
 // compute unit's memory path: 16 waves own contiguous segments of the keys; histogram, scan and
 // ranks as above, with the [wave][group] counters in LDS and workgroup barriers between the phases.
@@ -714,7 +819,7 @@ extern "C" int64_t pt_group_rows_workspace_bytes(int64_t m, int32_t num_groups) 
   return align_up(W * num_groups * 4, 256) + align_up((int64_t)num_groups * 4, 256);
 }
 
-// The four launches of the stable counting sort (chunk histograms, scan over the chunks, scan over
+// The two launches of the stable counting sort, or four of a long one (chunk histograms, scan over the chunks, scan over
 // the groups, ranks); `workspace` holds the [W][G] chunk counts and the G group starts
 // (pt_group_rows_workspace_bytes), every byte of which is written before it is read.  (One kernel
 // for both scans, with the last workgroup to finish doing the second, measured slower: the
@@ -725,8 +830,13 @@ static int group_rows_launch(const int64_t* keys, int64_t m, int32_t G, int32_t 
     gr_one_kernel<<<1, 1024, 0, s>>>(keys, m, G, bits_for(G), alignment, offs, ks, reverse, src_of, cap);
     return check_launch("group_rows");
   }
-  const int64_t W = cdiv(m, kWaveKeys);
+  const int64_t W = cdiv(m, kWaveKeys), lists = cdiv(m, kBlockKeys);
   int32_t* counts = (int32_t*)workspace;
+  if (lists * G <= kBlockCounts && G <= kBlockGroups) {
+    gr_block_hist_kernel<<<(unsigned)lists, 256, 0, s>>>(keys, m, G, counts, src_of, cap);
+    gr_block_rank_kernel<<<(unsigned)lists, 256, 0, s>>>(keys, m, G, bits_for(G), alignment, counts, offs, ks, reverse, src_of, cap);
+    return check_launch("group_rows");
+  }
   int32_t* group_start = (int32_t*)((char*)workspace + align_up(W * G * 4, 256));
   const unsigned blocks = (unsigned)cdiv(W, 4);
   const size_t lds = (size_t)4 * G * sizeof(int32_t);
