@@ -4,7 +4,8 @@
 // chunk of keys, (1) counts them into a private LDS histogram, (2) one workgroup turns the
 // [chunk][group] counts into exclusive bases, (3) every wavefront replays its chunk 64 keys at a
 // time, ranking equal keys inside the wave with ballot masks (one ballot per key bit) on top of
-// its running LDS counters.  No global atomics decide a position, so the result is the
+// its running LDS counters.  Up to 8192 keys one workgroup does all three; more take one launch for (1) and one in which every
+// workgroup scans the counts itself before (3), or, with many chunks or groups, a launch each.  No global atomics decide a position, so the result is the
 // ascending-source-row order inside every group on every run.
 //
 // Row movement is a separate pass over the *destination* rows (one wavefront per row, 16-byte
@@ -747,6 +748,166 @@ __global__ __launch_bounds__(256) void dd_rank_kernel(const int64_t* ids, int64_
   }
 }
 
+// The same in two launches, up to kBlockCounts numbers in the count table (64 KiB from the L2 for each workgroup of the second
+// launch) and kDedupBlockTopK choices a token.  A workgroup takes 256 tokens and loads their choices flat, four a lane in
+// flight, instead of a lane the choices of its token one after the other.  What bounds it is the chain of loads, scans and
+// ballots.  Four launches / two, us for 128 experts of 8 ranks, 8 choices a token: 256 tokens 22.0 / 14.1, 4096 22.8 / 15.3, 30 000
+// 28.3 / 20.3; 65 536 tokens, 4 of 32 experts of 4 ranks 25.5 / 12.8.  (The limits are those of the sort above: past them
+// every workgroup reads more counts than the two scans take.)
+static constexpr int kDedupBlockTopK = 16;
+static bool dedup_in_two_launches(int64_t m, int k, int E, int ep) {
+  return k <= kDedupBlockTopK && E + ep <= kBlockGroups && cdiv(m, 4 * kWaveTokens) * (E + ep) <= kBlockCounts;
+}
+
+// f(position in the wave's flat list, token of the wave, choice or -1) for the wave's tokens from t0 on
+template <typename F>
+__device__ __forceinline__ void for_choices(const int64_t* ids, int64_t ld, int64_t m, int k, int E, int64_t t0, F f) {
+  const int lane = threadIdx.x & 63;
+  const int n = (int)(m - t0 < kWaveTokens ? (m - t0 > 0 ? m - t0 : 0) : kWaveTokens) * k;
+  for (int q = lane; q < n; q += 4 * 64) {
+    int64_t e[4];
+    int token[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {  // (from a clamped place: behind a condition each load would wait for the one before)
+      const int fl = q + 64 * u < n ? q + 64 * u : q;
+      token[u] = fl / k;
+      e[u] = ids[(t0 + token[u]) * ld + (fl - token[u] * k)];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (q + 64 * u < n) f(q + 64 * u, token[u], e[u] >= 0 && e[u] < E ? (int)e[u] : -1);
+  }
+}
+
+__global__ __launch_bounds__(256) void dd_block_hist_kernel(const int64_t* ids, int64_t ld, int64_t m, int k, int E, int ep, int epr,
+                                                            int32_t* counts /*[blocks][E + ep]*/) {
+  __shared__ int32_t s_count[kBlockGroups];
+  __shared__ uint32_t s_visited[256];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  s_count[t] = 0;
+  s_visited[t] = 0;
+  __syncthreads();
+  for_choices(ids, ld, m, k, E, ((int64_t)blockIdx.x * 4 + wave) * kWaveTokens, [&](int, int token, int e) {
+    if (e < 0) return;
+    atomicAdd(&s_count[e], 1);
+    atomicOr(&s_visited[wave * 64 + token], 1u << (e / epr));
+  });
+  __syncthreads();
+  const uint32_t visited = s_visited[t];
+  for (int g = 0; g < ep; ++g) {
+    const int n = __popcll(__ballot((visited >> g) & 1u));
+    if (lane == 0 && n) atomicAdd(&s_count[E + g], n);
+  }
+  __syncthreads();
+  if (t < E + ep) counts[(int64_t)blockIdx.x * (E + ep) + t] = s_count[t];
+}
+
+__global__ __launch_bounds__(256) void dd_block_rank_kernel(const int64_t* ids, int64_t ld, int64_t m, int k, int E, int ep, int epr, int nbits,
+                                                            const int32_t* counts, int64_t* tokens_per_ep_rank,
+                                                            int64_t* dedup_tokens_per_gpu, int64_t* send_meta, int64_t* dispatch,
+                                                            int64_t* idxs, int64_t* expand_idx) {
+  extern __shared__ int32_t s_b[];  // per wave: run[E + ep], lp[64][ep], the choices [64][k]
+  __shared__ int32_t s_total[kBlockGroups], s_before[kBlockGroups], s_start[kBlockGroups], s_w[4];
+  __shared__ uint32_t s_visited[256];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, block = blockIdx.x, blocks = gridDim.x, C = E + ep;
+  const int per_wave = C + 64 * ep + 64 * k;
+  int32_t* run = s_b + wave * per_wave;
+  int32_t* lp = run + C;
+  int32_t* choice = lp + 64 * ep;
+  const int64_t t0 = ((int64_t)block * 4 + wave) * kWaveTokens;
+  s_total[t] = s_before[t] = 0;
+  s_visited[t] = 0;
+  for (int c = lane; c < C; c += 64) run[c] = 0;
+  __syncthreads();
+  // every column's sum over all blocks and over those before this one: as many threads to a column as there are
+  const int parts = 256 / C, col = t % C, part = t / C;
+  if (part < parts) {
+    int32_t total = 0, before = 0;
+#pragma unroll 16
+    for (int b = part; b < blocks; b += parts) {
+      const int32_t c = counts[b * C + col];
+      total += c;
+      before += b < block ? c : 0;
+    }
+    if (total) {
+      atomicAdd(&s_total[col], total);
+      if (before) atomicAdd(&s_before[col], before);
+    }
+  }
+  for_choices(ids, ld, m, k, E, t0, [&](int fl, int token, int e) {
+    choice[fl] = e;
+    if (e < 0) return;
+    atomicAdd(&run[e], 1);
+    atomicOr(&s_visited[wave * 64 + token], 1u << (e / epr));
+  });
+  __syncthreads();
+  const uint32_t visited = s_visited[t];
+  for (int g = 0; g < ep; ++g) {
+    const int n = __popcll(__ballot((visited >> g) & 1u));
+    if (lane == 0) run[E + g] = n;
+  }
+  const int32_t size = s_total[t];
+  int32_t incl = size;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t up = __shfl_up(incl, d);
+    if (lane >= d) incl += up;
+  }
+  if (lane == 63) s_w[wave] = incl;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) incl += w < wave ? s_w[w] : 0;
+  s_start[t] = incl - size;  // of the ranks behind all experts: their sum is taken off below
+  if (t < C) {
+    // where each wave's rows of an expert go, and its unique tokens in the slice of a rank
+    int32_t at = (t < E ? incl - size : 0) + s_before[t];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      int32_t* r = s_b + w * per_wave + t;
+      const int32_t c = *r;
+      *r = at;
+      at += c;
+    }
+  }
+  __syncthreads();
+  if (block == 0 && t < E) send_meta[(t / epr) * (epr + 1) + t % epr] = size;
+  if (block == 0 && t >= E && t < C) {
+    const int g = t - E;
+    tokens_per_ep_rank[g] = s_start[(g + 1) * epr] - s_start[g * epr];
+    dedup_tokens_per_gpu[g] = size;
+    send_meta[g * (epr + 1) + epr] = size;
+  }
+  const uint64_t lt = lanemask_lt();
+  for (int g = 0; g < ep; ++g) {
+    const bool v = (visited >> g) & 1u;
+    const uint64_t bal = __ballot(v);
+    if (v) {
+      const int32_t pos = run[E + g] + __popcll(bal & lt);
+      lp[lane * ep + g] = pos;
+      dispatch[(int64_t)(s_start[E + g] - s_start[E]) + pos] = t0 + lane;
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  const int n = (int)(m - t0 < kWaveTokens ? (m - t0 > 0 ? m - t0 : 0) : kWaveTokens) * k;
+  for (int q = 0; q < n; q += 64) {
+    const int fl = q + lane;
+    int e = fl < n ? choice[fl] : -1;
+    const bool active = e >= 0;
+    if (!active) e = 0;
+    const uint64_t mask = wave_match((uint32_t)e, active, nbits);
+    const int rank = __popcll(mask & lt);
+    const int32_t b = run[e];
+    __builtin_amdgcn_wave_barrier();
+    if (active && rank == 0) run[e] = b + __popcll(mask);
+    __builtin_amdgcn_wave_barrier();
+    if (active) {
+      const int64_t pos = (int64_t)b + rank;
+      idxs[pos] = t0 * k + fl;
+      expand_idx[pos] = lp[(fl / k) * ep + e / epr];
+    }
+  }
+}
+
 __global__ __launch_bounds__(256) void build_expert_idxs_kernel(const int64_t* counts, int E, int ep, int epr,
                                                                 int64_t max_total, int64_t* expert_idxs,
                                                                 int64_t* output_splits) {
@@ -1074,6 +1235,14 @@ extern "C" int pt_dedup_prepare_dispatch(const int64_t* topk_ids, int64_t ld_ids
   int32_t* gpu_starts = (int32_t*)wsp; wsp += 256;
   int32_t* totals = (int32_t*)wsp;
   const unsigned blocks = (unsigned)cdiv(W, 4);
+  if (dedup_in_two_launches(m, k, E, ep)) {
+    int32_t* counts = (int32_t*)workspace;  // blocks x (E + ep): less than the two tables
+    dd_block_hist_kernel<<<blocks, 256, 0, s>>>(topk_ids, ld_ids, m, k, E, ep, epr, counts);
+    dd_block_rank_kernel<<<blocks, 256, (size_t)4 * (E + ep + 64 * ep + 64 * k) * 4, s>>>(
+        topk_ids, ld_ids, m, k, E, ep, epr, bits_for(E), counts, tokens_per_ep_rank, dedup_tokens_per_gpu, send_meta, dispatch_token_idxs,
+        idxs, expand_idx);
+    return check_launch("dedup_prepare_dispatch");
+  }
   dd_hist_kernel<<<blocks, 256, (size_t)4 * (E + 32) * 4, s>>>(topk_ids, ld_ids, m, k, E, ep, epr, cnt_e, cnt_g);
   dd_scan_cols_kernel<<<(unsigned)cdiv(E + ep, 4), 256, 0, s>>>(cnt_e, cnt_g, W, E, ep, totals);
   dd_scan_totals_kernel<<<1, 64, 0, s>>>(totals, E, ep, epr, tokens_per_ep_rank, dedup_tokens_per_gpu, send_meta, expert_starts,

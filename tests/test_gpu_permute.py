@@ -141,6 +141,34 @@ def test_fused_dedup_prepare_dispatch(m, k, E, ep, seed):
     assert torch.equal(disp[gs[rank] + exp], idxs // k)
 
 
+@pytest.mark.parametrize("m,k,E,ep", [(1, 1, 1, 1), (63, 3, 9, 3), (65, 16, 240, 16), (255, 17, 240, 16), (257, 16, 31, 31), (500, 8, 256, 1), (1025, 5, 224, 32),
+                                      (32768, 8, 120, 8), (32769, 8, 120, 8)])  # fmt: skip
+def test_dedup_at_the_edges_of_its_blocks_and_limits(m, k, E, ep):
+    """Both forms of the dispatch lists (the one in two launches ends at 16 choices, E + ep = 256 and 16 384 counts), with choices
+    that repeat, choices out of range, which are dropped, and rows wider than their choices."""
+    from pith_train_amd.operators.ep_dispatch import fused_dedup_prepare_dispatch
+
+    g = torch.Generator().manual_seed(m + k)
+    epr = E // ep
+    wide = torch.randint(-1, E + 1, (m, k + 3), generator=g)
+    got = [t.cpu() for t in fused_dedup_prepare_dispatch(wide.cuda()[:, :k], E, ep, epr)]
+    ids = wide[:, :k]
+    flat = ids.reshape(-1)
+    valid = (flat >= 0) & (flat < E)
+    counts = torch.bincount(flat[valid], minlength=E)
+    # (token, rank) pairs in the order of ranks, then tokens, each once
+    tokens = torch.arange(m).repeat_interleave(k)
+    pairs = torch.unique((flat[valid] // epr) * m + tokens[valid])
+    per_rank = torch.bincount(pairs // m, minlength=ep)
+    starts = per_rank.cumsum(0) - per_rank
+    order = torch.argsort(torch.where(valid, flat, E), stable=True)[: int(valid.sum())]
+    place = torch.searchsorted(pairs, (flat[order] // epr) * m + tokens[order]) - starts[flat[order] // epr]
+    assert torch.equal(got[0], counts.view(ep, epr).sum(1)) and torch.equal(got[1], per_rank)
+    assert torch.equal(got[2][: pairs.numel()], pairs % m)
+    assert torch.equal(got[3][: order.numel()], order) and torch.equal(got[4][: order.numel()], place)
+    assert torch.equal(got[5].view(ep, epr + 1), torch.cat([counts.view(ep, epr), per_rank[:, None]], 1))
+
+
 def test_dedup_duplicate_experts_in_a_row_and_empty():
     from pith_train_amd.operators.ep_dispatch import fused_dedup_prepare_dispatch
 
