@@ -86,7 +86,7 @@ template <> struct GateOperand<float> {
     }
     set(v);
   }
-  __device__ __forceinline__ void load_column(const float* p, int64_t pitch, int n) {  // n of eight, one per row
+  __device__ __forceinline__ void load_column(const float* p, int64_t pitch, int n, const float*) {  // n of eight, one per row
     float v[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = k < n ? p[k * pitch] : 0.f;
@@ -100,10 +100,16 @@ template <> struct GateOperand<uint16_t> {
     const uint4 u = ok ? *reinterpret_cast<const uint4*>(p) : make_uint4(0, 0, 0, 0);
     v = {{u.x, u.y, u.z, u.w}};
   }
-  __device__ __forceinline__ void load_column(const uint16_t* p, int64_t pitch, int n) {
+  // From row min(k, n - 1), and `inside` where n is 0, with zeros in place of what is none of the n: behind a condition each 16-bit load
+  // waits for the one before it to be merged with zeros (with the sum of the slabs, 8192 tokens x 2048, 128 experts 52.5 -> 46.0 us, 16 384 tokens
+  // 85.3 -> 71.6; 32-bit loads are masked without a wait, and selecting their zeros afterwards costs 1 us of 44).
+  __device__ __forceinline__ void load_column(const uint16_t* p, int64_t pitch, int n, const uint16_t* inside) {
     uint32_t b[8];
+    p = n ? p : inside;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) b[k] = k < n ? p[k * pitch] : 0u;
+    for (int k = 0; k < 8; ++k) b[k] = p[(k < n ? k : n ? n - 1 : 0) * pitch];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) b[k] = k < n ? b[k] : 0u;
 #pragma unroll
     for (int m = 0; m < 4; ++m) v.w[m] = b[2 * m] | (b[2 * m + 1] << 16);
   }
@@ -189,7 +195,7 @@ __global__ __launch_bounds__(256, 2) void gate_linear_bwd_kernel(GateArgs p) {
       const int64_t row = t0 + 8 * q;
       const int n = e >= p.E || row >= end ? 0 : end - row < 8 ? (int)(end - row) : 8;
       GateOperand<D> g;
-      g.load_column(dl + row * p.E + e, p.E, n);
+      g.load_column(dl + row * p.E + e, p.E, n, dl);
 #pragma unroll
       for (int j = 0; j < 8; ++j) dw[i][j] = g.times(fx[j], dw[i][j]);
     }
