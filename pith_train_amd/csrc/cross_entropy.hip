@@ -91,9 +91,9 @@ __global__ __launch_bounds__(1024) void ce_count_kernel(const int64_t* target, i
 // (m, d) of two disjoint parts of a row -> (m, d) of their union
 __device__ __forceinline__ void merge_md(float& m, float& d, float m2, float d2) {
   const float mn = fmaxf(m, m2);
-  // a part that saw nothing has m = -inf and d = 0: its term is 0 * exp(-inf - mn) = 0
-  const float a = m == -INFINITY ? 0.f : d * fast_exp(m - mn);
-  const float b = m2 == -INFINITY ? 0.f : d2 * fast_exp(m2 - mn);
+  // a part that saw no more than -inf has m = -inf and d = 0, or the not-a-number that it saw
+  const float a = m == -INFINITY ? d : d * fast_exp(m - mn);
+  const float b = m2 == -INFINITY ? d2 : d2 * fast_exp(m2 - mn);
   m = mn;
   d = a + b;
 }
@@ -130,13 +130,12 @@ __device__ __forceinline__ void absorb(const float (&v)[N], float& m, float& d) 
     d = d * fast_exp(m - cm);  // m = -inf on the first chunk: d is 0 and exp2(-inf) is 0
     m = cm;
   }
-  if (m != -INFINITY) {  // a chunk of -inf logits (masked vocabulary) adds nothing
-    const float mb = m * kLog2e;
-    float s = 0.f;
+  // (a chunk of -inf logits, a masked vocabulary, adds zeros; one of them and a not-a-number, which no maximum shows, adds that)
+  const float mb = m == -INFINITY ? 0.f : m * kLog2e;
+  float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < N; ++i) s += __builtin_amdgcn_exp2f(v[i] * kLog2e - mb);
-    d += s;
-  }
+  for (int i = 0; i < N; ++i) s += __builtin_amdgcn_exp2f(v[i] * kLog2e - mb);
+  d += s;
 }
 // logits into gradients of the mean loss; off: the target's place among them (anything else: not there)
 template <typename S, int N, class I>
@@ -191,7 +190,7 @@ __global__ __launch_bounds__(1024) void ce_fwd_kernel(CeArgs p) {
         d = d * fast_exp(m - v);
         m = v;
       }
-      if (m != -INFINITY) d += fast_exp(v - m);
+      d += fast_exp(v - (m == -INFINITY ? 0.f : m));
     }
   }
   // fixed-order combination: xor butterfly inside the wave, then the 16 waves in order

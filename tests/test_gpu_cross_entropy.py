@@ -188,3 +188,23 @@ def test_rows_that_start_anywhere(N, V, start, dtype):
     (grad,) = torch.autograd.grad(loss * 0.3, buf)
     assert torch.equal(grad, stored * torch.tensor(0.3).to(dtype))
     assert (flat[:start] == 7).all() and (flat[start + N * V :] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("V", [3, 9, 304, 1003, 4096, 32776, 102337, 204665, 300007])
+def test_a_nan_among_masked_logits_is_seen(V, dtype):
+    """A logit that is not a number makes the loss and its row's gradient so, wherever it stands: at the ends of a row, which
+    single threads read, and between -inf logits, with which it is all that a thread sees."""
+    from pith_train_amd.operators.cross_entropy import cross_entropy
+
+    places = sorted({p for p in (0, 1, 5, V // 2, V // 2 + 3, V - 2, V - 1) if 0 <= p < V})
+    x, _ = _case(len(places) + 1, V, V, dtype)
+    for row, p in enumerate(places):
+        x[row, max(p - 3, 0) : p + 4] = -math.inf
+        x[row, p] = math.nan
+    y = torch.full((len(x),), V // 3)
+    for row in range(len(places)):
+        buf = x[[row, -1]].cuda()
+        loss = cross_entropy(buf, y[:2].cuda())
+        assert math.isnan(float(loss)), places[row]
+        assert buf[0].isnan().all() and buf[1].isfinite().all()
