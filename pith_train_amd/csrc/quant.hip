@@ -61,30 +61,31 @@ enum { B_COL = 0, B_BLOCK = 1 };                       // scaling of the twin
 enum { BL_ROWMAJOR = 0, BL_TRANSPOSED = 1, BL_KMAJOR = 2, BL_NONE = 3 };  // layout of the twin's bytes (BL_NONE: no twin is written)
 enum { BS_MB_N = 0, BS_N_MB = 1 };                     // twin scale layout for B_COL
 
+// (every field has a value: a kernel looks at optional ones that its entry point may not know)
 struct QuantArgs {
-  const void* x;
-  int64_t M, N, ldx, x_stride_g;
-  uint8_t* a_out;  int64_t a_stride_g;   // [M,N] bytes, ld = N; row-scaled launches: null = not written
-  float* a_scale;  int64_t a_scale_stride_g;
-  int64_t as_rs, as_ks;                  // row-scaled launches: the scale of row r, column tile c is a_scale[r * as_rs + c * as_ks]
-  uint8_t* b_out;  int64_t b_stride_g;   // rowmajor [M,N] / transposed [N,M] / kmajor flat; row-scaled launches: null = not written
-  float* b_scale;  int64_t b_scale_stride_g;
-  int32_t tiles_m, tiles_n;
-  const int32_t* offs; int32_t num_groups;  // KMAJOR only
-  int32_t vec_in;     // 16-byte loads legal (alignment + N % 8 == 0)
-  int32_t vec_out;    // 8-byte row-major stores legal (N % 8 == 0)
-  int32_t vec_out_t;  // 16-byte transposed stores legal
-  const int32_t* row_index;  // optional [M]: source row of output row r (negative: a zero row); null = identity
-  uint32_t row_mul;          // with row_index: the source row is floor(row_index * row_mul / 2^32) (every source row stands for several); 0 = row_index itself
-  const void* x2; int64_t ldx2;  // fused SwiGLU backward: the saved gate_up [M, 2*half]
-  int64_t half;                  // fused SwiGLU: width of one half of gate_up
-  const int32_t* row_limit;      // optional device scalar: row tiles at or past *row_limit are skipped (nothing written)
-  int64_t ld_t;                  // row pitch of the transposed twin (bytes = elements); M unless it is a column slice
-  int64_t bs_ld;                 // row length of the twin's block-scale grid; tiles_m unless it is a column slice
-  float alpha, limit;            // fused clamped SwiGLU: its two constants
+  const void* x = nullptr;
+  int64_t M = 0, N = 0, ldx = 0, x_stride_g = 0;
+  uint8_t* a_out = nullptr;  int64_t a_stride_g = 0;   // [M,N] bytes, ld = N; row-scaled launches: null = not written
+  float* a_scale = nullptr;  int64_t a_scale_stride_g = 0;
+  int64_t as_rs = 0, as_ks = 0;                  // row-scaled launches: the scale of row r, column tile c is a_scale[r * as_rs + c * as_ks]
+  uint8_t* b_out = nullptr;  int64_t b_stride_g = 0;   // rowmajor [M,N] / transposed [N,M] / kmajor flat; row-scaled launches: null = not written
+  float* b_scale = nullptr;  int64_t b_scale_stride_g = 0;
+  int32_t tiles_m = 0, tiles_n = 0;
+  const int32_t* offs = nullptr; int32_t num_groups = 0;  // KMAJOR only
+  int32_t vec_in = 0;     // 16-byte loads legal (alignment + N % 8 == 0)
+  int32_t vec_out = 0;    // 8-byte row-major stores legal (N % 8 == 0)
+  int32_t vec_out_t = 0;  // 16-byte transposed stores legal
+  const int32_t* row_index = nullptr;  // optional [M]: source row of output row r (negative: a zero row); null = identity
+  uint32_t row_mul = 0;          // with row_index: the source row is floor(row_index * row_mul / 2^32) (every source row stands for several); 0 = row_index itself
+  const void* x2 = nullptr; int64_t ldx2 = 0;  // fused SwiGLU backward: the saved gate_up [M, 2*half]
+  int64_t half = 0;                  // fused SwiGLU: width of one half of gate_up
+  const int32_t* row_limit = nullptr;      // optional device scalar: row tiles at or past *row_limit are skipped (nothing written)
+  int64_t ld_t = 0;                  // row pitch of the transposed twin (bytes = elements); M unless it is a column slice
+  int64_t bs_ld = 0;                 // row length of the twin's block-scale grid; tiles_m unless it is a column slice
+  float alpha = 0.f, limit = 0.f;            // fused clamped SwiGLU: its two constants
   const int32_t* row_used = nullptr;  // row-scaled launches: negative where nobody reads row r of the row-scaled output and the twin's is zero (null: all are)
-  float* col_sum;                // PRO_SUMS and fused clamped SwiGLU backward: [tiles_m, N] column sums of each 128-row tile
-  int32_t head_a, head_b;        // per-head halves in two tensors: column h * (head_a + head_b) + c is x[h * head_a + c] or x2[h * head_b + c - head_a]
+  float* col_sum = nullptr;                // PRO_SUMS and fused clamped SwiGLU backward: [tiles_m, N] column sums of each 128-row tile
+  int32_t head_a = 0, head_b = 0;        // per-head halves in two tensors: column h * (head_a + head_b) + c is x[h * head_a + c] or x2[h * head_b + c - head_a]
 };
 
 template <typename T> struct Loader;
@@ -786,8 +787,8 @@ void quant_tile_kernel(QuantArgs p) {
 // (128 experts: 316.6 us against 308.9 in two launches); they keep launches of their own.
 struct QuantWeightsArgs {
   QuantArgs part[PT_QUANT_WEIGHTS_MAX];
-  int64_t end[PT_QUANT_WEIGHTS_MAX];  // number of tiles of the parts up to and including this one
-  int n;
+  int64_t end[PT_QUANT_WEIGHTS_MAX] = {};  // number of tiles of the parts up to and including this one
+  int n = 0;
 };
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void quant_weights_kernel(QuantWeightsArgs w) {
@@ -812,8 +813,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void q
 // of latency, and a launch costs the host four.
 struct QuantDenseArgs {
   QuantArgs w[PT_QUANT_DENSE_MAX], x;
-  int end[PT_QUANT_DENSE_MAX];  // number of tiles of the weights up to and including this one
-  int n;
+  int end[PT_QUANT_DENSE_MAX] = {};  // number of tiles of the weights up to and including this one
+  int n = 0;
 };
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void quant_dense_kernel(QuantDenseArgs q) {
@@ -889,13 +890,10 @@ static int launch_quant(const QuantArgs& a, int dtype, int64_t G, hipStream_t st
 }
 
 static void fill_common(QuantArgs& a, const void* x, int dtype, int64_t M, int64_t N, int64_t ldx) {
-  a.x = x; a.M = M; a.N = N; a.ldx = ldx; a.x_stride_g = 0;
-  a.a_stride_g = 0; a.a_scale_stride_g = 0; a.b_stride_g = 0; a.b_scale_stride_g = 0;
+  a.x = x; a.M = M; a.N = N; a.ldx = ldx;
   a.tiles_m = (int32_t)cdiv(M, 128); a.tiles_n = (int32_t)cdiv(N, 128);
   a.as_rs = a.tiles_n; a.as_ks = 1;
-  a.offs = nullptr; a.num_groups = 0; a.row_index = nullptr; a.row_mul = 0; a.x2 = nullptr; a.ldx2 = 0; a.half = 0;
-  a.row_limit = nullptr; a.ld_t = M; a.bs_ld = a.tiles_m; a.alpha = 0.f; a.limit = 0.f; a.col_sum = nullptr; a.row_used = nullptr;
-  a.head_a = a.head_b = 0;
+  a.ld_t = M; a.bs_ld = a.tiles_m;
   const int eb = dtype == PT_F32 ? 4 : 2;
   a.vec_in = (N % 8 == 0) && ((ldx * eb) % 16 == 0) && (((uintptr_t)x) % 16 == 0);
   a.vec_out = (N % 8 == 0);
@@ -1108,7 +1106,6 @@ static int fill_blockwise(QuantArgs& a, const void* x, int dtype, int64_t G, int
 extern "C" int pt_quant_weights(const pt_quant_weight* parts, int32_t n, int dtype, pt_stream_t stream) {
   PT_REQUIRE(parts && n >= 0 && n <= PT_QUANT_WEIGHTS_MAX, "quant_weights: %d parts (at most %d)", n, PT_QUANT_WEIGHTS_MAX);
   QuantWeightsArgs w;
-  w.n = 0;
   int64_t tiles = 0;
   for (int i = 0; i < n; ++i) {
     const pt_quant_weight& q = parts[i];
