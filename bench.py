@@ -156,7 +156,8 @@ class GemmTimer:
              "pt_gemm_k_grouped_wgrad_ld", "pt_gemm_k_grouped_wgrad_pair",
              "pt_gemm_nt_dense", "pt_gemm_nt_dense_splitk", "pt_gemm_nt_dense_ld", "pt_gemm_nt_dense_splitk_ld", "pt_gemm_nt_dense_heads", "pt_gemm_nt_dense_pair", "pt_gemm_m_grouped_nt_few_rows")
 
-    WHOLE_STEPS = ("pt_experts_forward", "pt_experts_forward_by_block", "pt_experts_backward", "pt_experts_backward_by_block", "pt_experts_weight_gradient", "pt_linear_forward", "pt_linear_backward",
+    WHOLE_STEPS = ("pt_experts_forward", "pt_experts_forward_by_block", "pt_experts_forward_without_padding", "pt_experts_backward", "pt_experts_backward_by_block",
+                   "pt_experts_backward_without_padding", "pt_experts_weight_gradient", "pt_linear_forward", "pt_linear_backward",
                    "pt_mlp_forward", "pt_mlp_backward")
 
     def __init__(self):

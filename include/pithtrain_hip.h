@@ -642,8 +642,6 @@ int pt_gate_linear_bwd(const void* d_logits, int dtype, const void* x, const voi
  * every field is 8 bytes wide.
  * ------------------------------------------------------------------------------------------ */
 
-#define PT_PADDING_UNDEFINED 256
-
 /* Forward of an expert block (gate_up projection, SwiGLU, down projection; FP8 operands).
  * x bf16 [x_rows, K] (row stride ldx).  With row_map (int32 [M], the scatter's source map, negative =
  * padding) grouped row r is x[row_map[r]], or x[expand_idx[row_map[r]]] with expand_idx (int64
@@ -654,10 +652,7 @@ int pt_gate_linear_bwd(const void* d_logits, int dtype, const void* x, const voi
  * GEMMs' stores; otherwise silu(gate) * up on concatenated halves.  x_t [K, M] and h_t [half, M] bytes with
  * scales [M/128, K] and [M/128, half]: the transposed activations that the weight gradients read (all four
  * NULL: no backward follows).  repeat > 1 (with row_map, without expand_idx): grouped row r is
- * x[row_map[r] / repeat].  few_rows != 0 (no backward): the groups are multiples of 64 rows,
- * and with scatter what stands for their padding in gate_up is not defined.  few_rows == PT_PADDING_UNDEFINED (with scatter,
- * without biases; groups of 128 as ever, with a backward that says the same): what stands for padding, row_map[r] < 0, in gate_up,
- * x_fp8 and h_fp8 is not defined, and the transposed activations hold zeros for it.  Not
+ * x[row_map[r] / repeat].  few_rows != 0 (no backward): the groups are multiples of 64 rows.  Not
  * needed afterwards: composed_map int32 [M] (with expand_idx), x_fp8 [M, K] and h_fp8 [M, half] with
  * their 1x128 scales. */
 typedef struct {
@@ -680,13 +675,16 @@ int pt_experts_forward(const pt_experts_forward_args* args /* host */);
 /* The same step with the scales of its row-scaled operands (x_scale, h_scale; in the backward dy_scale and dgu_scale) as
  * [K/128, M] instead of [M, K/128]: the GEMMs read them in whole lines. */
 int pt_experts_forward_by_block(const pt_experts_forward_args* args /* host */);
+/* The latter of scattered rows (scatter != 0), which leaves padding out: what stands for it, row_map[r] < 0, in gate_up, x_fp8 and
+ * h_fp8 is not defined, and the transposed activations hold zeros for it.  Where a backward follows, without the clamped
+ * activation and gu_bias, which make other values of padding, and that backward is pt_experts_backward_without_padding. */
+int pt_experts_forward_without_padding(const pt_experts_forward_args* args /* host */);
 
 /* Backward of the same block, up to the quantised gradient of gate_up: dgu_fp8 [M, 2*half] and dgu_scale
  * [M, ceil(2*half/128)], from which the input gradient follows with one pt_gemm_m_grouped_nn(_scatter) on
  * the gate_up weight.  grad_out bf16 [grad_rows, H]; out_map: row_map when the forward scattered its
  * result (the gradient arrives un-permuted), else NULL; limit_rows != 0: the row count is offs[G-1] (the
- * forward had a row_map; PT_PADDING_UNDEFINED: and left its padding undefined, as this leaves that of dy_fp8, dgu_fp8 and grad_h;
- * needs out_map).  dn_dg: the down weight, dn_forward_layout != 0 for the forward-layout tensor, 0
+ * forward had a row_map).  dn_dg: the down weight, dn_forward_layout != 0 for the forward-layout tensor, 0
  * for the transposed twin.  dy_t [H, M] and dgu_t [2*half, M] bytes with scales [M/128, .]: the transposed
  * gradients of the weight-gradient GEMMs (kept by the caller when it runs those later).  Not needed
  * afterwards: dy_fp8 [M, H] with 1x128 scales, grad_h bf16 [M, half], col_sum fp32 [M/128, 2*half].
@@ -716,6 +714,9 @@ typedef struct {
 } pt_experts_backward_args;
 int pt_experts_backward(const pt_experts_backward_args* args /* host */);
 int pt_experts_backward_by_block(const pt_experts_backward_args* args /* host */); /* see pt_experts_forward_by_block; the input gradient is pt_gemm_m_grouped_by_block's */
+/* The latter after pt_experts_forward_without_padding (out_map: its row_map, limit_rows != 0): what stands for padding in dy_fp8,
+ * dgu_fp8 and grad_h is not defined either, and the transposed gradients hold zeros for it. */
+int pt_experts_backward_without_padding(const pt_experts_backward_args* args /* host */);
 /* The gate_up weight gradient of the same block from the same arguments (dw_gate_up, dw_up): the last
  * launch of a backward, after the caller has queued the input gradient. */
 int pt_experts_weight_gradient(const pt_experts_backward_args* args /* host */);

@@ -110,8 +110,10 @@ SIGNATURES = {
     # whole steps: one host block of 8-byte fields (struct.pack) instead of an argument each
     "pt_experts_forward": (c_int, [c_char_p]),
     "pt_experts_forward_by_block": (c_int, [c_char_p]),
+    "pt_experts_forward_without_padding": (c_int, [c_char_p]),
     "pt_experts_backward": (c_int, [c_char_p]),
     "pt_experts_backward_by_block": (c_int, [c_char_p]),
+    "pt_experts_backward_without_padding": (c_int, [c_char_p]),
     "pt_experts_weight_gradient": (c_int, [c_char_p]),
     "pt_transposed_pitch": (I64, [I64]),
     "pt_linear_forward_workspace_bytes": (I64, [I64, I64, I64, I64]),

@@ -75,7 +75,9 @@ struct Library {
   PT_FN(pt_group_rows_workspace_bytes);
   PT_FN(pt_group_rows);
   PT_FN(pt_experts_forward_by_block);
+  PT_FN(pt_experts_forward_without_padding);
   PT_FN(pt_experts_backward_by_block);
+  PT_FN(pt_experts_backward_without_padding);
   PT_FN(pt_experts_weight_gradient);
   PT_FN(pt_transposed_pitch);
   PT_FN(pt_linear_forward_workspace_bytes);
@@ -131,7 +133,9 @@ void init(const std::string& path) {
   PT_FN(pt_group_rows_workspace_bytes);
   PT_FN(pt_group_rows);
   PT_FN(pt_experts_forward_by_block);
+  PT_FN(pt_experts_forward_without_padding);
   PT_FN(pt_experts_backward_by_block);
+  PT_FN(pt_experts_backward_without_padding);
   PT_FN(pt_experts_weight_gradient);
   PT_FN(pt_transposed_pitch);
   PT_FN(pt_linear_forward_workspace_bytes);
@@ -434,7 +438,7 @@ struct Dims {
   Pieces backward_temp(bool sums) const { return Pieces({2 * M * half, sums ? M / 128 * half * 8 : 0}); }  // grad_h, column sums
 };
 
-// Whether a block leaves out what stands for padding (PT_PADDING_UNDEFINED): the rows go back to their places, and groups of whole
+// Whether a training step leaves out what stands for padding (the _without_padding steps): the rows go back to their places, and groups of whole
 // 128-row blocks are padding for a good part: up to 96 rows per expert (d.M holds 127 a group and up to 255 for it), us a pass with padding
 // written / left out: 128 experts of 2048 x 768, 16 rows each 966 / 903, 48 981 / 942, 96 1013 / 1008; 64 of
 // 2048 x 1408, 16 839 / 795, 64 860 / 836; and from 64 groups on, whatever their rows, where the kernel of large tiles looks for it
@@ -475,7 +479,7 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x,
   a.M = d.M; a.K = K; a.half = half; a.H = d.H; a.G = d.G;
   a.offs = (const int32_t*)ptr(offs); a.row_map = (const int32_t*)ptr(row_map);
   a.expand_idx = (const int64_t*)ptr(expand_idx); a.n_expand = expand_idx ? routed : 0;
-  a.repeat = repeat; a.few_rows = few_rows ? 1 : keep && leaves_padding(d, (bool)row_map && scatter, clamped || gu_bias) ? PT_PADDING_UNDEFINED : 0;
+  a.repeat = repeat; a.few_rows = few_rows;
   a.gu_fp8 = ptr(gu); a.gu_scale = (const float*)ptr(gu_s); a.gu_bias = ptr(gu_bias);
   a.dn_fp8 = ptr(dn); a.dn_scale = (const float*)ptr(dn_s); a.dn_bias = ptr(dn_bias);
   a.gate_up = ptr(gate_up); a.out = ptr(out); a.out_rows = out.size(0); a.scatter = scatter;
@@ -483,7 +487,11 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x,
   if (keep) { a.x_t = kept.at(0); a.x_t_scale = (float*)kept.at(1); a.h_t = kept.at(2); a.h_t_scale = (float*)kept.at(3); }
   a.composed_map = (int32_t*)temp.at(0); a.x_fp8 = temp.at(1); a.x_scale = (float*)temp.at(2); a.h_fp8 = temp.at(3); a.h_scale = (float*)temp.at(4);
   a.stream = (pt_stream_t)stream;
-  check(lib.pt_experts_forward_by_block(&a), "pt_experts_forward_by_block");
+  const bool placed = row_map && scatter;
+  if (keep ? leaves_padding(d, placed, clamped || gu_bias) : placed && few_rows)
+    check(lib.pt_experts_forward_without_padding(&a), "pt_experts_forward_without_padding");
+  else
+    check(lib.pt_experts_forward_by_block(&a), "pt_experts_forward_by_block");
   return {out, gate_up, kept.buffers};
 }
 
@@ -551,7 +559,7 @@ struct ExpertsBackward {
     if (weights.size() > 0) down.aim(weights[0]);
     a.grad_out = ptr(grad_out); a.grad_rows = grad_out.size(0);
     a.M = d.M; a.K = d.K; a.half = d.half; a.H = d.H; a.G = d.G;
-    a.offs = (const int32_t*)ptr(offs); a.out_map = scatter ? (const int32_t*)ptr(row_map) : nullptr; a.limit_rows = leaves_padding(d, row_map && scatter, clamped || gu_bias_like) ? PT_PADDING_UNDEFINED : (bool)row_map;
+    a.offs = (const int32_t*)ptr(offs); a.out_map = scatter ? (const int32_t*)ptr(row_map) : nullptr; a.limit_rows = (bool)row_map;
     a.dn_dg = ptr(dn_dg); a.dn_dg_scale = (const float*)ptr(dn_dg_s); a.dn_forward_layout = dn_forward;
     a.gate_up = ptr(gate_up_saved);
     a.x_t = kept.at(0); a.x_t_scale = (const float*)kept.at(1); a.h_t = kept.at(2); a.h_t_scale = (const float*)kept.at(3);
@@ -563,7 +571,10 @@ struct ExpertsBackward {
     a.d_gu_bias = ptr(d_gu_bias); a.d_gu_bias_dtype = d_gu_bias ? dtype_code(d_gu_bias->scalar_type()) : 0;
     a.d_dn_bias = ptr(d_dn_bias); a.d_dn_bias_dtype = d_dn_bias ? dtype_code(d_dn_bias->scalar_type()) : 0;
     a.stream = (pt_stream_t)stream;
-    check(lib.pt_experts_backward_by_block(&a), "pt_experts_backward_by_block");
+    if (leaves_padding(d, row_map && scatter, clamped || gu_bias_like))
+      check(lib.pt_experts_backward_without_padding(&a), "pt_experts_backward_without_padding");
+    else
+      check(lib.pt_experts_backward_by_block(&a), "pt_experts_backward_by_block");
     grad_out.reset();
   }
 

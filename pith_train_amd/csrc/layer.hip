@@ -46,7 +46,7 @@ extern "C" void pt_observe(const char* name, int begin, int64_t a, int64_t b, in
   if (g_observer) g_observer(name, begin, a, b, c);
 }
 
-static int experts_forward(const pt_experts_forward_args* args, RowScales order) {
+static int experts_forward(const pt_experts_forward_args* args, RowScales order, bool without_padding = false) {
   PT_REQUIRE(args, "experts_forward: null arguments");
   const pt_experts_forward_args& a = *args;
   PT_REQUIRE(a.M >= 0 && a.M % 128 == 0 && a.K > 0 && a.half > 0 && a.H > 0 && a.G > 0 && a.G < (1ll << 31), "experts_forward: bad sizes");
@@ -54,17 +54,17 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order)
   PT_REQUIRE(a.offs && a.gate_up && a.out && a.x_fp8 && a.x_scale && a.h_fp8 && a.h_scale && keep == (a.h_t != nullptr) &&
                  keep == (a.x_t_scale != nullptr) && keep == (a.h_t_scale != nullptr), "experts_forward: null pointer");
   PT_REQUIRE(a.repeat >= 1 && (a.repeat == 1 || (a.row_map && !a.expand_idx)), "experts_forward: repeat needs row_map and no expand_idx");
-  PT_REQUIRE(a.few_rows == PT_PADDING_UNDEFINED || !a.few_rows || !keep, "experts_forward: a backward needs groups of whole 128-row blocks");
+  PT_REQUIRE(!a.few_rows || !keep, "experts_forward: a backward needs groups of whole 128-row blocks");
   PT_REQUIRE(!a.expand_idx || a.composed_map, "experts_forward: expand_idx needs composed_map");
   PT_REQUIRE(a.row_map || (!a.expand_idx && !a.scatter), "experts_forward: expand_idx and scatter need row_map");
   if (a.M == 0) return PT_OK;
   const int32_t G = (int32_t)a.G;
   const int32_t* limit = a.row_map ? a.offs + G - 1 : nullptr;  // rows past it hold nothing
   const int32_t* in_map = a.row_map;
-  // where the rows go back to their places, nobody sees what stands for padding
-  const bool few = a.few_rows && a.few_rows != PT_PADDING_UNDEFINED;
-  PT_REQUIRE(a.few_rows != PT_PADDING_UNDEFINED || (keep && a.scatter && !a.gu_bias && !a.clamped), "experts_forward: padding is left out of scattered rows of a SwiGLU block only");
-  const int32_t* used = a.few_rows && a.scatter ? a.row_map : nullptr;
+  const bool few = a.few_rows != 0;
+  PT_REQUIRE(!without_padding || (a.scatter && (!keep || (!a.gu_bias && !a.clamped))),
+             "experts_forward_without_padding: needs scatter, and before a backward a SwiGLU block without a bias");
+  const int32_t* used = without_padding ? a.row_map : nullptr;
   if (a.expand_idx) {
     PT_STEP(pt_compose_row_map, a.M, 0, 0, a.row_map, a.M, a.expand_idx, a.n_expand, a.x_rows, a.composed_map, a.stream);
     in_map = a.composed_map;
@@ -114,7 +114,7 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order)
   return PT_OK;
 }
 
-static int experts_backward(const pt_experts_backward_args* args, RowScales order) {
+static int experts_backward(const pt_experts_backward_args* args, RowScales order, bool without_padding = false) {
   PT_REQUIRE(args, "experts_backward: null arguments");
   const pt_experts_backward_args& a = *args;
   PT_REQUIRE(a.M >= 0 && a.M % 128 == 0 && a.K > 0 && a.half > 0 && a.H > 0 && a.G > 0 && a.G < (1ll << 31), "experts_backward: bad sizes");
@@ -123,8 +123,9 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
   if (a.M == 0) return PT_OK;
   const int32_t G = (int32_t)a.G;
   const int32_t* limit = a.limit_rows ? a.offs + G - 1 : nullptr;
-  PT_REQUIRE(a.limit_rows != PT_PADDING_UNDEFINED || (a.out_map && !a.clamped && !a.d_gu_bias), "experts_backward: padding is left out of scattered rows of a SwiGLU block only");
-  const int32_t* used = a.limit_rows == PT_PADDING_UNDEFINED ? a.out_map : nullptr;
+  PT_REQUIRE(!without_padding || (a.out_map && a.limit_rows && !a.clamped && !a.d_gu_bias),
+             "experts_backward_without_padding: needs out_map and limit_rows of a SwiGLU block without a bias");
+  const int32_t* used = without_padding ? a.out_map : nullptr;
   // The gradient of the down bias is the sum of the rows that are quantised here: the kernel that reads them adds up
   // every 128 (groups are whole 128-row tiles) where col_sum, which the activation's backward fills afterwards, has
   // room for those sums (16384 tokens x 4 of 2880 columns: a second pass over the rows took 110 us, the sums here cost
@@ -174,8 +175,10 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
 
 extern "C" int pt_experts_forward(const pt_experts_forward_args* args) { return experts_forward(args, RowScales::BY_ROW); }
 extern "C" int pt_experts_forward_by_block(const pt_experts_forward_args* args) { return experts_forward(args, RowScales::BY_BLOCK); }
+extern "C" int pt_experts_forward_without_padding(const pt_experts_forward_args* args) { return experts_forward(args, RowScales::BY_BLOCK, true); }
 extern "C" int pt_experts_backward(const pt_experts_backward_args* args) { return experts_backward(args, RowScales::BY_ROW); }
 extern "C" int pt_experts_backward_by_block(const pt_experts_backward_args* args) { return experts_backward(args, RowScales::BY_BLOCK); }
+extern "C" int pt_experts_backward_without_padding(const pt_experts_backward_args* args) { return experts_backward(args, RowScales::BY_BLOCK, true); }
 
 extern "C" int pt_experts_weight_gradient(const pt_experts_backward_args* args) {
   PT_REQUIRE(args, "experts_weight_gradient: null arguments");

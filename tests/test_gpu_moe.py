@@ -697,3 +697,59 @@ def test_training_step_that_leaves_padding_out(kind, E, H, I, T, k, dedup, holes
     ours, composed = run(True), run(False)
     for n, (a, b) in enumerate(zip(ours, composed)):
         assert b.float().abs().sum() > 0 and torch.equal(a, b), n
+
+
+def test_flags_of_the_steps_are_truth_values():
+    """``few_rows`` and ``limit_rows`` of the C structures say yes with any value but zero, and the steps that are not the
+    ``_without_padding`` ones define what stands for padding: gate_up of groups of 64 rows, whatever the buffer held."""
+    import struct
+
+    from pith_train_amd import _lib
+    from pith_train_amd.operators.token_scatter import group_rows_with_sizes
+
+    G_, K, half, H, routed = 3, 256, 128, 256, 210
+    g = torch.Generator(device="cuda").manual_seed(2)
+    idx = torch.randint(0, G_, (routed,), device="cuda", generator=g)
+    x, grad = (torch.randn((routed, K), device="cuda", generator=g).bfloat16() for _ in range(2))
+    fp8 = lambda *s: torch.randint(0, 256, s, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # noqa: E731
+    gu, gu_s, dn, dn_s = fp8(G_, 2 * half, K), torch.ones((G_, 2, 2), device="cuda"), fp8(G_, H, half), torch.ones((G_, 2, 1), device="cuda")
+
+    def buffers(M):
+        sizes = dict(gate_up=4 * M * half, out=2 * max(M, routed) * H, map=4 * M, x_fp8=M * K, x_s=8 * M, h_fp8=M * half, h_s=4 * M, x_t=K * M, x_ts=4 * K * M // 128,
+                     h_t=half * M, h_ts=4 * half * M // 128, dgu=2 * half * M, dgu_s=8 * M, dy_t=H * M, dy_ts=4 * H * M // 128, dgu_t=2 * half * M,
+                     dgu_ts=8 * half * M // 128, grad_h=2 * M * half)
+        return {n: torch.full((z,), 0xFF, dtype=torch.uint8, device="cuda") for n, z in sizes.items()}
+
+    def forward(b, M, offs, row_map, scatter, few, keep):
+        saved = [b[n].data_ptr() if keep else 0 for n in ("x_t", "x_ts", "h_t", "h_ts")]
+        _lib.call("pt_experts_forward_by_block", struct.pack(
+            "=25q2d10q", x.data_ptr(), routed, K, M, K, half, H, G_, offs.data_ptr(), row_map.data_ptr(), 0, 0, 1, few, gu.data_ptr(), gu_s.data_ptr(), 0,
+            dn.data_ptr(), dn_s.data_ptr(), 0, b["gate_up"].data_ptr(), b["out"].data_ptr(), routed if scatter else M, scatter, 0, 0.0, 0.0, *saved,
+            *(b[n].data_ptr() for n in ("map", "x_fp8", "x_s", "h_fp8", "h_s")), _lib.stream_ptr()))
+
+    _, offs, _, _, row_map = group_rows_with_sizes(idx, G_, 64, device=idx.device, host_sizes=False, need_reverse=False)
+    M, evaluated = row_map.shape[0], []
+    for few in (1, 256):
+        evaluated.append(buffers(M))
+        forward(evaluated[-1], M, offs, row_map, 1, few, False)
+    rows = int(offs[-1])
+    assert (row_map[:rows] < 0).any()
+    for b in evaluated:
+        assert torch.isfinite(b["gate_up"].view(torch.bfloat16).view(M, 2 * half)[:rows].float()).all()
+    assert all(torch.equal(evaluated[0][n], evaluated[1][n]) for n in ("gate_up", "out"))
+
+    _, offs, _, _, row_map = group_rows_with_sizes(idx, G_, 128, device=idx.device, host_sizes=False, need_reverse=False)
+    M, trained = row_map.shape[0], []
+    grouped = torch.where((row_map >= 0)[:, None], grad[row_map.clamp_min(0).long()], torch.zeros_like(grad[:1]))
+    for limit in (1, 256):
+        b = buffers(M)
+        trained.append(b)
+        forward(b, M, offs, row_map, 0, 0, True)
+        at = lambda *names: [b[n].data_ptr() for n in names]  # noqa: E731
+        _lib.call("pt_experts_backward_by_block", struct.pack(
+            "=35q2d5q", grouped.data_ptr(), M, M, K, half, H, G_, offs.data_ptr(), 0, limit, dn.data_ptr(), dn_s.data_ptr(), 1, *at("gate_up", "x_t", "x_ts", "h_t",
+            "h_ts", "dgu", "dgu_s", "dy_t", "dy_ts", "dgu_t", "dgu_ts", "dgu", "dgu_s", "grad_h"), 0, 0, 0, 0, 0, 0, 0, 0, 0.0, 0.0, 0, 0, 0, 0, _lib.stream_ptr()))
+    rows = int(offs[-1])
+    for n, width in (("dgu", 2 * half), ("gate_up", 4 * half)):
+        a, b = (t[n].view(M, width)[:rows] for t in trained)
+        assert torch.equal(a, b)
