@@ -677,7 +677,8 @@ int pt_experts_forward(const pt_experts_forward_args* args /* host */);
 int pt_experts_forward_by_block(const pt_experts_forward_args* args /* host */);
 /* The latter of scattered rows (scatter != 0), which leaves padding out: what stands for it, row_map[r] < 0, in gate_up, x_fp8 and
  * h_fp8 is not defined, and the transposed activations hold zeros for it.  Where a backward follows, without the clamped
- * activation and gu_bias, which make other values of padding, and that backward is pt_experts_backward_without_padding. */
+ * activation and gu_bias, which make other values of padding, and that backward is pt_experts_backward_without_padding.  row_map
+ * is 16-byte aligned. */
 int pt_experts_forward_without_padding(const pt_experts_forward_args* args /* host */);
 
 /* Backward of the same block, up to the quantised gradient of gate_up: dgu_fp8 [M, 2*half] and dgu_scale

@@ -444,12 +444,12 @@ struct Dims {
 // 2048 x 1408, 16 839 / 795, 64 860 / 836; and from 64 groups on, whatever their rows, where the kernel of large tiles looks for it
 // (gemm_rowsplit.hip has both sides).  Biases and the clamped activation make other values than zero of padding, which the
 // column scales of the transposed activations see: such blocks write it.
-bool leaves_padding(const Dims& d, bool placed, bool biased) {
-  return placed && !biased && (d.M <= 224 * d.G + 256 || d.G >= 64);
-}
+bool leaves_padding(const Dims& d, bool biased) { return !biased && (d.M <= 224 * d.G + 256 || d.G >= 64); }
 
-// Forward of an expert block (see fused_experts._forward): (out, gate_up, kept buffers).
-std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x, int64_t repeat, const Maybe& row_map, const Maybe& expand_idx,
+bool in_whole_chunks(const Tensor& map) { return ((uintptr_t)ptr(map) & 15) == 0; }
+
+// Forward of an expert block (see fused_experts._forward): (out, gate_up, kept buffers, whether padding was left out).
+std::tuple<Tensor, Tensor, std::vector<Tensor>, bool> experts_forward(const Tensor& x, int64_t repeat, const Maybe& row_map, const Maybe& expand_idx,
                                                                 const Tensor& offs, const Tensor& gu, const Tensor& gu_s, const Tensor& dn,
                                                                 const Tensor& dn_s, int64_t half, const Maybe& gu_bias, const Maybe& dn_bias, bool scatter,
                                                                 bool clamped, double alpha, double limit, bool keep, bool few_rows, int64_t stream) {
@@ -487,12 +487,13 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> experts_forward(const Tensor& x,
   if (keep) { a.x_t = kept.at(0); a.x_t_scale = (float*)kept.at(1); a.h_t = kept.at(2); a.h_t_scale = (float*)kept.at(3); }
   a.composed_map = (int32_t*)temp.at(0); a.x_fp8 = temp.at(1); a.x_scale = (float*)temp.at(2); a.h_fp8 = temp.at(3); a.h_scale = (float*)temp.at(4);
   a.stream = (pt_stream_t)stream;
-  const bool placed = row_map && scatter;
-  if (keep ? leaves_padding(d, placed, clamped || gu_bias) : placed && few_rows)
+  // (those steps read the map in 16-byte chunks; a slice of a longer one may start anywhere)
+  const bool without_padding = row_map && scatter && in_whole_chunks(*row_map) && (keep ? leaves_padding(d, clamped || gu_bias) : few_rows);
+  if (without_padding)
     check(lib.pt_experts_forward_without_padding(&a), "pt_experts_forward_without_padding");
   else
     check(lib.pt_experts_forward_by_block(&a), "pt_experts_forward_by_block");
-  return {out, gate_up, kept.buffers};
+  return {out, gate_up, kept.buffers, without_padding};
 }
 
 // Where a weight gradient goes: an existing bf16 gradient is accumulated into by the GEMM, otherwise a new
@@ -541,7 +542,7 @@ struct ExpertsBackward {
   Maybe d_gu_bias, d_dn_bias;
   Target down, gate_up, up;
 
-  ExpertsBackward(const Tensor& grad, const Dims& dims, const Tensor& offs, const Maybe& row_map, bool scatter, const Tensor& dn_dg, const Tensor& dn_dg_s,
+  ExpertsBackward(const Tensor& grad, const Dims& dims, const Tensor& offs, const Maybe& row_map, bool scatter, bool without_padding, const Tensor& dn_dg, const Tensor& dn_dg_s,
                   bool dn_forward, const Tensor& gate_up_saved, std::vector<Tensor> kept_buffers, bool clamped, double alpha, double limit,
                   const Maybe& gu_bias_like, const Maybe& dn_bias_like, std::vector<Tensor> weights_ /* down, gate_up or gate, up; empty: deferred */,
                   int64_t stream)
@@ -571,7 +572,7 @@ struct ExpertsBackward {
     a.d_gu_bias = ptr(d_gu_bias); a.d_gu_bias_dtype = d_gu_bias ? dtype_code(d_gu_bias->scalar_type()) : 0;
     a.d_dn_bias = ptr(d_dn_bias); a.d_dn_bias_dtype = d_dn_bias ? dtype_code(d_dn_bias->scalar_type()) : 0;
     a.stream = (pt_stream_t)stream;
-    if (leaves_padding(d, row_map && scatter, clamped || gu_bias_like))
+    if (without_padding)
       check(lib.pt_experts_backward_without_padding(&a), "pt_experts_backward_without_padding");
     else
       check(lib.pt_experts_backward_by_block(&a), "pt_experts_backward_by_block");
@@ -1122,7 +1123,7 @@ struct ExpertsNode : HipNode {
   Saved saved[COUNT];
   std::vector<Saved> activations;  // x^T, h^T with scales
   Maybe gu_bias, dn_bias;
-  bool has_map, has_expand, gu_forward, dn_forward, scatter, clamped;
+  bool has_map, has_expand, gu_forward, dn_forward, scatter, without_padding, clamped;
   double alpha, limit;
   int64_t src_rows, routed, repeat;
   void drop() override {
@@ -1134,6 +1135,7 @@ struct ExpertsNode : HipNode {
     const Tensor offs = saved[OFFS].get(), gu_dg = saved[GU_DG].get(), gu_dg_s = saved[GU_DG_S].get();
     Maybe row_map, expand_idx;
     if (has_map) row_map = saved[ROW_MAP].get();
+    if (without_padding && !in_whole_chunks(*row_map)) row_map = row_map->clone();  // a saved-tensor hook's
     if (has_expand) expand_idx = saved[EXPAND_IDX].get();
     std::vector<Tensor> kept;
     for (const Saved& s : activations) kept.push_back(s.get());
@@ -1147,7 +1149,7 @@ struct ExpertsNode : HipNode {
       weights = {w_down, w_gate};
       if (w_up.defined()) weights.push_back(w_up);
     }
-    ExpertsBackward step(g[0], d, offs, row_map, scatter, saved[DN_DG].get(), saved[DN_DG_S].get(), dn_forward, saved[GATE_UP].get(), std::move(kept),
+    ExpertsBackward step(g[0], d, offs, row_map, scatter, without_padding, saved[DN_DG].get(), saved[DN_DG_S].get(), dn_forward, saved[GATE_UP].get(), std::move(kept),
                          clamped, alpha, limit, gu_bias, dn_bias, std::move(weights), (int64_t)stream);
     // Rows that expand the same source row are summed (the backward of the expanding gather), right behind the GEMM
     // that wrote them: after the weight gradient they come from HBM.  Only a sum of bf16 rows below 4 GiB takes two outputs.
@@ -1194,7 +1196,7 @@ Tensor experts(const Tensor& input, const Tensor& w_gate, const Maybe& w_up, con
                const Maybe& expand_idx, bool scatter, std::optional<std::pair<double, double>> clamp, int64_t stream) {
   const Tensor up = w_up.value_or(Tensor()), b0 = gu_bias.value_or(Tensor()), b1 = dn_bias.value_or(Tensor());
   require_same_device(input, {&w_gate, &up, &w_down, &std::get<0>(gu_dg), &std::get<1>(gu_dg), &std::get<0>(dn_dg), &std::get<1>(dn_dg)});
-  std::tuple<Tensor, Tensor, std::vector<Tensor>> done;
+  std::tuple<Tensor, Tensor, std::vector<Tensor>, bool> done;
   Tensor x;
   int64_t repeat = 1;
   const auto [alpha, limit] = clamp.value_or(std::pair<double, double>{0.0, 0.0});
@@ -1241,7 +1243,7 @@ Tensor experts(const Tensor& input, const Tensor& w_gate, const Maybe& w_up, con
           if (keep[i].defined()) n.saved[i] = Saved(keep[i]);
         for (const Tensor& t : std::get<2>(done)) n.activations.emplace_back(t);
         n.gu_bias = gu_bias; n.dn_bias = dn_bias;
-        n.scatter = scatter; n.clamped = (bool)clamp; n.alpha = alpha; n.limit = limit;
+        n.scatter = scatter; n.without_padding = std::get<3>(done); n.clamped = (bool)clamp; n.alpha = alpha; n.limit = limit;
       },
       input, w_gate, up, w_down, b0, b1);
 }

@@ -62,6 +62,7 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order,
   const int32_t* limit = a.row_map ? a.offs + G - 1 : nullptr;  // rows past it hold nothing
   const int32_t* in_map = a.row_map;
   const bool few = a.few_rows != 0;
+  PT_REQUIRE(!without_padding || ((uintptr_t)a.row_map & 15) == 0, "experts_forward_without_padding: row_map must be 16-byte aligned");
   PT_REQUIRE(!without_padding || (a.scatter && (!keep || (!a.gu_bias && !a.clamped))),
              "experts_forward_without_padding: needs scatter, and before a backward a SwiGLU block without a bias");
   const int32_t* used = without_padding ? a.row_map : nullptr;
@@ -125,6 +126,7 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
   const int32_t* limit = a.limit_rows ? a.offs + G - 1 : nullptr;
   PT_REQUIRE(!without_padding || (a.out_map && a.limit_rows && !a.clamped && !a.d_gu_bias),
              "experts_backward_without_padding: needs out_map and limit_rows of a SwiGLU block without a bias");
+  PT_REQUIRE(!without_padding || ((uintptr_t)a.out_map & 15) == 0, "experts_backward_without_padding: out_map must be 16-byte aligned");
   const int32_t* used = without_padding ? a.out_map : nullptr;
   // The gradient of the down bias is the sum of the rows that are quantised here: the kernel that reads them adds up
   // every 128 (groups are whole 128-row tiles) where col_sum, which the activation's backward fills afterwards, has

@@ -753,3 +753,45 @@ def test_flags_of_the_steps_are_truth_values():
     for n, width in (("dgu", 2 * half), ("gate_up", 4 * half)):
         a, b = (t[n].view(M, width)[:rows] for t in trained)
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("where", ["forward", "backward", "evaluation"])
+def test_row_maps_that_start_anywhere(where):
+    """The steps that leave padding out read the row map in chunks of 16 bytes: a map that starts inside one, the caller's or
+    what a saved-tensor hook gives back, gives the bits of one that does not."""
+    from pith_train_amd.dualpipe_utils import FP8WeightCacheControl
+    from pith_train_amd.modules.experts import Qwen35MoeExperts
+    from pith_train_amd.operators.token_scatter import group_rows_with_sizes
+
+    G_, H, I, rows = 8, 256, 128, 300
+    g = torch.Generator(device="cuda").manual_seed(7)
+    mod = Qwen35MoeExperts(H, I, G_).cuda().bfloat16()
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.normal_(0.0, 0.02, generator=g)
+    x, dy = (torch.randn((rows, H), device="cuda", generator=g).bfloat16() for _ in range(2))
+    few = where == "evaluation"
+    _, offs, _, _, row_map = group_rows_with_sizes(torch.randint(0, G_, (rows,), device="cuda", generator=g), G_, 64 if few else 128,
+                                                   device=x.device, host_sizes=False, need_reverse=False)
+    odd = lambda t: torch.cat([t.new_zeros(1), t])[1:]  # noqa: E731
+    assert odd(row_map).data_ptr() % 16 == 4 and row_map.data_ptr() % 16 == 0
+    FP8WeightCacheControl.step()
+    if few:
+        with torch.no_grad():
+            assert torch.equal(mod(x, offs, row_map=row_map, few_rows=True), mod(x, offs, row_map=odd(row_map), few_rows=True))
+        return
+
+    def step(given, unpack):
+        mod.zero_grad(set_to_none=True)
+        t = x.clone().requires_grad_(True)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            out = mod(t, offs, row_map=given)
+        out.backward(dy)
+        return [out.detach(), t.grad] + [p.grad for p in mod.parameters()]
+
+    want = step(row_map, lambda t: t)
+    if where == "forward":
+        got = step(odd(row_map), lambda t: t)
+    else:
+        got = step(row_map, lambda t: odd(t) if t.dtype == torch.int32 and t.dim() == 1 and t.numel() == row_map.numel() else t)
+    assert all(b.float().abs().sum() > 0 and torch.equal(a, b) for a, b in zip(got, want))
