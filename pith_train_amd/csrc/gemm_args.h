@@ -1,6 +1,7 @@
 // Argument block shared by the FP8 GEMM kernels.
 #pragma once
 #include "common.h"
+#include "gemm_rules.h"
 
 namespace pt {
 

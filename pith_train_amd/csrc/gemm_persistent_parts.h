@@ -382,7 +382,6 @@ __device__ __forceinline__ int xcd_first_tile(const GemmArgs& p, const int* s_pr
 //   parts    the whole list is cut by cost, as without a schedule but anywhere: an operand is read by one XCD or two,
 //            but one whose 32 workgroups get 33 big tiles of nearly a share each takes two rounds for them
 // All of it is the same arithmetic in every workgroup (one wave).
-enum Schedule { kInOrder, kEighths, kParts };
 static constexpr int kSchedGroups = 256;  // groups it is made for: four a lane
 static constexpr int kNoLoad = 0x3fffffff;
 struct KSchedule {  // in LDS
@@ -426,25 +425,13 @@ __device__ __forceinline__ void eighths_tile(int per_g, int xcd, int j, int& h, 
   const int y = (8 * place + 7 + per_g) / per_g - 1;  // the first eighth that ends behind it
   h = 8 * round + ((y - xcd) & 7);
 }
-// Which form a launch takes, by the cost of its largest tile and a workgroup's share, in blocks.  Weight gradients with
-// Zipf-distributed popularity whose operands come from HBM, as in a step, us in order / eighths / parts, means of four
-// orders of the same groups:
-//   the largest tile is a whole share or more, so that no XCD has more big tiles than workgroups: parts from shares of 24
-//     on.  8942 tokens of 8 in 128 groups 512 x 2048 177 / 156 / 145; 15000 268 / 218 / 201; 9000 of 8 in 16, 768 x 2048 162 /
-//     130 / 126; 30000 of 4 in 32, 1024 x 2048 311 / 321 / 307; 16384 of 8 in 64, 2048 x 768 280 / 235 / 219.
-//     Shorter ones lose (share 15: 40 -> 63)
-//   the others: eighths from shares of 56 on.  8192 of 6 in 64, 2816 x 2048 393 / 336 / 381; 16384 of 8 in 128, 1536 x 2048 566 / 452 /
-//     498, less skewed 467 / 477 / -; 3500 of 4 in 32, 5760 x 2880 453 / 363 / 461, of 10000 less skewed 686 / 627 / -; 4293 of 8 in
-//     128, 768 x 2048 157 / 150 / 150.  Shares of 28 and 29 lose: 64 -> 66, 67 -> 88
-// Limits: what the lists above can hold (a workgroup's big tiles are at most its share and one tile); sums that stay
-// below 2^29, a workgroup's below 2^22.
+// Which form a launch takes (schedule_of_groups has the lines).  Limits: what the lists above can hold (a workgroup's big tiles are at
+// most its share and one tile); sums that stay below 2^29, a workgroup's below 2^22.
 __device__ __forceinline__ Schedule schedule_of(const GemmArgs& p, const int* s_pref, int workers) {
   const int64_t per_g = (int64_t)p.tiles_a * p.tiles_b, total = s_pref[p.G] * per_g, all_workers = 8 * workers;
   if (!p.offs || p.G > kSchedGroups || workers > 64 || per_g >= (1 << 22) || total >= (8ll << 22) * workers || total >= (1ll << 29)) return kInOrder;
   if (level_groups(p, s_pref)) return kInOrder;
-  const int64_t largest = s_pref[p.G + 1] * all_workers;  // against total, as the tile against a share
-  if (largest >= total) return total >= 24 * all_workers ? kParts : kInOrder;
-  return total >= 56 * all_workers ? kEighths : kInOrder;
+  return schedule_of_groups(s_pref[p.G + 1], s_pref[p.G], per_g, all_workers);
 }
 // Place of workgroup `me`'s small tile j in the XCD's part of their list.  ahead: on lane w the big tiles of workgroup w
 // in small ones; tiles are taken in the order of (ahead + count so far, workgroup).
@@ -462,10 +449,8 @@ __device__ __forceinline__ int small_place(int ahead, int me, int workers, int j
 __device__ __forceinline__ void schedule_k_groups(const GemmArgs& p, const int* s_pref, KSchedule& s, bool parts, int xcd, int t_first, int t_last,
                                                   int me, int workers, int lane) {
   const int per_g = p.tiles_a * p.tiles_b;
-  // cost of a big tile: an eighth of a share; of shares from 140 on, which pay for a longer schedule, a sixteenth (16384
-  // tokens of 8 in 128 groups 1536 x 2048 532 -> 462 us; shares of 113 and 130 172 -> 178 and 208 -> 221)
   const int64_t total = (int64_t)s_pref[p.G] * per_g, all_workers = 8 * workers;
-  const int least = (int)(total / ((total >= 140 * all_workers ? 16 : 8) * all_workers)) + 1;
+  const int least = (int)(total / (big_tile_parts(parts ? kParts : kEighths, total, all_workers) * all_workers)) + 1;  // cost of a big tile
   int cost[4];
   unsigned left = 0;  // the lane's groups of big tiles that have not been dealt out
 #pragma unroll

@@ -1,0 +1,28 @@
+"""Which form a GEMM launch takes, by its sizes: both sides of every line."""
+
+import pytest
+from gemm_rules import call, schedule
+
+
+@pytest.mark.parametrize("groups,largest,rest,per_group,form", [
+    # a tile of a whole share or more
+    (64, 200, 4, 24, "parts"), (64, 50, 1, 24, "in order"),
+    (16, 900, 1, 60, "parts"),
+    # groups of few tiles, of which an eighth is two or three or none: never eighths, whatever the skew
+    (128, 120, 10, 24, "parts"), (128, 36, 10, 24, "in order"), (120, 48, 25, 5, "parts"), (256, 60, 40, 1, "parts"), (64, 100, 60, 8, "parts"),
+    (128, 70, 4, 24, "parts"),
+    (128, 75, 5, 32, "eighths"), (128, 40, 9, 32, "in order"), (64, 40, 5, 36, "in order"),
+    # from 40 tiles on: a group of a 25th of the work
+    (64, 60, 13, 88, "eighths"), (64, 30, 13, 88, "in order"), (64, 20, 3, 40, "eighths"), (128, 60, 10, 48, "in order"), (128, 80, 8, 48, "eighths"),
+    (32, 18, 5, 276, "eighths"), (128, 15, 10, 144, "eighths"), (128, 15, 10, 120, "in order"), (32, 4, 3, 40, "in order"), (8, 14, 4, 276, "eighths"),
+    (6, 12, 2, 276, "in order"),
+])
+def test_schedule_of_skewed_groups(groups, largest, rest, per_group, form):
+    blocks = [rest] * groups
+    blocks[groups // 3] = largest
+    got, share, most = schedule(blocks, per_group)
+    assert got == form, (got, share, most)
+
+
+def test_parts_of_a_share_that_are_dealt_out_one_by_one():
+    assert [call("big_tile_parts", form, blocks * 256, 256) for form in (1, 2) for blocks in (56, 139, 140, 400)] == [8, 8, 16, 16, 8, 8, 8, 8]

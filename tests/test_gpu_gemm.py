@@ -9,6 +9,7 @@ the fp32 accumulation order and the single bf16 rounding (2**-9).
 
 import pytest
 import torch
+from gemm_rules import schedule
 
 from oracle import fp8 as Q
 from oracle import gemm as G
@@ -465,8 +466,7 @@ def test_k_grouped_schedule_of_skewed_groups(gemm_kernel, groups, N, W):
     for i, share in enumerate((2, 4, 4, 8, 8, 16, 32)[:groups]):
         blocks[i * (groups // 7 or 1)] = int(total / share)
     offs, M = torch.cumsum(blocks * 128, 0).int().cuda(), int(blocks.sum()) * 128
-    cost = blocks + 3
-    assert cost.sum() * tiles >= 96 * 256 and cost.max() * 4 * 256 >= cost.sum() * tiles  # what the rule asks for
+    assert schedule(blocks.tolist(), tiles, min(256, groups * tiles))[0] == "parts"
 
     def fp8(*shape):
         return torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xBF  # finite values below 2
@@ -665,16 +665,18 @@ def test_grouped_work_lists_longer_than_the_tile_table(gemm_kernel):
     both(k_grouped)
 
 
-@pytest.mark.parametrize("groups,big,rest,N,W", [
-    (2, (300, 40), 0, 1024, 1280),      # fewer tiles than workgroups; XCD parts that end inside a group
-    (19, (90, 61, 33), 3, 1100, 1800),  # ragged tile grid, counts of groups and tiles that no eighth divides
-    (256, (130, 128, 90), 1, 512, 1024),  # as many groups as the schedule holds, the last ones idle
-    (70, (37, 36, 30), 4, 2816, 1300),  # no tile of a whole share: an eighth of every group, remainders of tiles and of groups
-    (120, (48,), 49, 256, 1280),  # fewer tiles a group than XCDs
+@pytest.mark.parametrize("groups,big,rest,N,W,form", [
+    (2, (300, 40), 0, 1024, 1280, "parts"),      # fewer tiles than workgroups; XCD parts that end inside a group
+    (19, (90, 61, 33), 3, 1100, 1800, "parts"),  # ragged tile grid, counts of groups and tiles that no eighth divides
+    (256, (130, 128, 90), 1, 512, 1024, "parts"),  # as many groups as the schedule holds, the last ones idle
+    (120, (48,), 49, 256, 1280, "parts"),  # no tile of a whole share; fewer tiles a group than XCDs
+    (70, (37, 36, 30), 4, 2816, 1300, "eighths"),  # remainders of tiles and of groups
+    (53, (90, 80, 66), 14, 1024, 2048, "eighths"),  # the fewest tiles a group that eighths take: four each
+    (45, (70, 80, 66), 24, 1500, 1400, "eighths"),  # 36 of them: four or five
 ])
-def test_k_grouped_schedule_of_shorter_and_less_skewed_launches(gemm_kernel, groups, big, rest, N, W):
-    """Groups whose largest tile is a workgroup's share or more: every XCD deals out its own part of the list.  Long launches
-    of others: an eighth of every group.  Every tile once (accumulating), with the bits of one small tile per workgroup."""
+def test_k_grouped_schedule_of_shorter_and_less_skewed_launches(gemm_kernel, groups, big, rest, N, W, form):
+    """Parts, where every XCD deals out its own part of the list, and eighths of every group, at the ends of what the rule gives
+    them.  Every tile once (accumulating), with the bits of one small tile per workgroup."""
     from pith_train_amd import _lib
 
     if gemm_kernel != "auto":
@@ -684,10 +686,7 @@ def test_k_grouped_schedule_of_shorter_and_less_skewed_launches(gemm_kernel, gro
     blocks = torch.randint(0, rest + 1, (groups,), generator=torch.Generator().manual_seed(groups))
     for i, b in enumerate(big):
         blocks[i * (groups // len(big))] = b
-    cost = blocks + 3
-    workgroups = min(256, groups * tiles)
-    share = cost.sum().item() * tiles / workgroups
-    assert share >= (24 if cost.max() >= share else 56), share  # what the rule asks for
+    assert schedule(blocks.tolist(), tiles, min(256, groups * tiles))[0] == form
     offs, M = torch.cumsum(blocks * 128, 0).int().cuda(), int(blocks.sum()) * 128
 
     def fp8(*shape):
@@ -722,9 +721,8 @@ def test_k_grouped_schedule_with_two_outputs_and_a_second_table(gemm_kernel, gro
     tiles = -(-N // 256) * -(-W // 256)
     blocks = torch.randint(0, 2, (groups,), generator=torch.Generator().manual_seed(groups))
     blocks[groups // 3] = 60 if groups == 256 else int(1.3 * 96 * 256 / tiles)
-    cost = blocks + 3
-    share = cost.sum().item() * tiles / 256
-    assert share >= 96 and cost.max() * 4 >= share  # what the rule asks for
+    form, share, _ = schedule(blocks.tolist(), tiles)
+    assert form != "in order"
     assert groups != 256 or share / 4 > 52  # small tiles cost 3 or 4: a workgroup without a big one
     offs, M = torch.cumsum(blocks * 128, 0).int().cuda(), int(blocks.sum()) * 128
 
