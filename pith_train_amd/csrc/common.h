@@ -234,6 +234,7 @@ int clamped_swiglu_bwd_quant(const void* grad_h, int64_t ld_grad_h, const void* 
                              RowScales order, pt_stream_t stream);
 int gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order, const void* b_fp8, const float* b_scale, void* out, int out_dtype,
                    const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows, const void* bias,
-                   pt_stream_t stream, bool b_kmajor = false, bool few_rows = false, void* out2 = nullptr, int64_t out2_rows = 0, const int32_t* row_used = nullptr);
+                   pt_stream_t stream, bool b_kmajor = false, bool few_rows = false, void* out2 = nullptr, int64_t out2_rows = 0, const int32_t* row_used = nullptr,
+                   int64_t used_rows = 0);
 
 }  // namespace pt

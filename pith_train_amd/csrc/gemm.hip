@@ -285,58 +285,6 @@ static int gemm_impl() {
   return g_impl;
 }
 
-// Problems too small for 256 x 256 tiles to fill 256 compute units evenly go to the kernel with one 64 x 128
-// or 128 x 128 tile per workgroup and two workgroups per compute unit (gemm_small.hip): tile rows, or 0
-// when the persistent kernel is the better choice.  While all 64-row tiles run at once the smaller tile
-// wins (1001 x 512 x 2048: 10.7 us against 12.9 with 128 rows and 21.5 for the large one).  While the 128-row tiles do,
-// dense ones with a long reduction take the form with one workgroup per unit (us, two per unit / one: 1001 x 4096 x 1536 14.7 / 13.1,
-// 1792 17.3 / 14.0, 2880 27.7 / 20.8; 2048 x 2048 x 1536 11.5 / 11.5, 1792 13.3 / 12.8, 2048 16.4 / 14.0; 4096 x 1024 x 1792 12.1 /
-// 12.5, 2048 13.3 / 13.4, 2880 24.1 / 19.0).  Then both
-// kinds are priced in rounds of the GPU: a round of 256 large tiles is the unit, a round of 512 small ones
-// (a quarter of the area each, half of it in all) costs 0.72 of it in the m-grouped mode, 0.68 in
-// the dense one (0.45 up to a reduction of 512, most of it filling and draining), 0.36 for a weight gradient
-// over groups of up to 1024 rows (mostly stores, which one workgroup of a unit does while the other loads), 0.65
-// over longer ones (16 Zipf-distributed groups of 7600 rows 768 x 2048 and 1536 x 2048: whole step 2540 us, 2623 at
-// 0.56).  A partly filled round of small tiles costs half of what it leaves idle.  Fitted to 270
-// shapes timed with both kernels, where the choice now loses 0.9 % to the better one in the mean (m-grouped), 0.2 %
-// (weight gradients) and nothing (dense).  Us, large / small: m-grouped, K 2048, N 1536: 16 groups of 256 rows
-// 25.4 / 19.7, of 512 30.5 / 34.9, of 640 50.1 / 37.4, of 1024 53.0 / 62.8; 64 groups of 128 49.6 / 52.7, of 384
-// 89 / 108; reduction-major b, K 1536, N 2048: 16 groups of 256 24.5 / 25.2, of 640 42.2 / 41.2.  Dense
-// 4096 x 2048 x 2048 26 / 20, 4096 x 4096 x 512 15.0 / 13.6.  Weight gradients 1536 x 2048 of 8 groups of 512
-// rows 26.6 / 23.4, of 1024 35.1 / 32.7; of 16 groups of 512 37.8 / 40.9.  Past two rounds large tiles have
-// no round to waste and need half of the operand traffic.
-static int small_tile_rows(const GemmArgs& g) {
-  const int64_t groups = g.mode == GEMM_K_GROUPED ? g.G : 1;
-  const int64_t cols = cdiv(g.rows_b, 128) * groups, cols_large = cdiv(g.rows_b, 256) * groups;
-  if (cdiv(g.rows_a, 64) * cols <= 256) return 64;
-  // Where padding is known and left out, up to 96 rows a group (the row count holds 127 more for each and some): 128-row tiles, which end
-  // at their last used row.  Layers of 128 experts 2048 x 768, us a pass in large tiles / these: 16 rows each 943 / 903, 48 974 /
-  // 942, 96 1029 / 1008, 128 1170 / 1167, 200 1249 / 1300; in tiles of 64 rows, of which every second finds nothing, 969 at 16.
-  if (g.row_used && g.rows_a <= 224 * (int64_t)g.G + 256) return 128;
-  // Weights that come from HBM and are read once, mostly: single operators on 128 groups of 48 rows 2048 x 768 1191 / 1182, of 96
-  // 1222 / 1209.
-  if (g.mode == GEMM_M_GROUPED && streams_weights(g) && g.rows_a <= 140 * (int64_t)g.G) return 128;
-  int64_t small = cdiv(g.rows_a, 128) * cols;
-  if (small <= 256 && g.mode == GEMM_DENSE && g.red >= 1792) return kDeepTile;
-  if (small <= 512) return 128;
-  int64_t rows_large = cdiv(g.rows_a, 256);
-  if (g.mode == GEMM_M_GROUPED) {
-    // Half of the groups end in half a large tile.  The row count may be a capacity, which exceeds the real
-    // one by half a block per group in the mean, or exact: half of that is taken off.
-    const int64_t blocks = g.rows_a / 128, least = blocks < g.G ? blocks : g.G;
-    rows_large = (blocks + g.G / 2) / 2;
-    if (rows_large < least) rows_large = least;
-    const int64_t fewer = blocks - g.G / 4;
-    small = (fewer > least ? fewer : least) * cols;
-  }
-  const int64_t large = rows_large * cols_large;
-  if (large > 512) return 0;
-  const int64_t depth = g.mode == GEMM_K_GROUPED ? g.red / g.G : g.red;
-  const int64_t price = g.mode == GEMM_M_GROUPED ? 72 : g.mode == GEMM_K_GROUPED ? (depth <= 1024 ? 36 : 65) : depth <= 512 ? 45 : 68;
-  // in units of 1 / (100 * 512 * 2) of a round of large tiles, five percent in favour of those
-  return (small + cdiv(small, 512) * 512) * price * 105 < cdiv(large, 256) * (2 * 512 * 100) * 100 ? 128 : 0;
-}
-
 // The persistent kernel addresses operands through 32-bit buffer offsets (signed range for the
 // loads, whose out-of-range marker is bit 31) and the result through an unsigned 32-bit byte
 // offset from the start of the output (of one group's block in the k-grouped mode, of the
@@ -548,7 +496,8 @@ extern "C" int pt_sum_partials(const float* partial, int32_t splits, int64_t n, 
 
 int pt::gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order, const void* b_fp8, const float* b_scale, void* out, int out_dtype,
                        const int32_t* offs, int32_t G, int64_t M, int64_t N, int64_t K, const int32_t* out_row_index, int64_t out_rows,
-                       const void* bias, pt_stream_t stream, bool b_kmajor, bool few_rows, void* out2, int64_t out2_rows, const int32_t* row_used) {
+                       const void* bias, pt_stream_t stream, bool b_kmajor, bool few_rows, void* out2, int64_t out2_rows, const int32_t* row_used,
+                       int64_t used_rows) {
   PT_REQUIRE(M >= 0 && N >= 0 && K >= 0 && G > 0, "gemm_m_grouped_nt: bad sizes");
   if (M == 0 || N == 0) return PT_OK;
   PT_REQUIRE(M % (few_rows ? 64 : 128) == 0, "gemm_m_grouped_nt: M=%lld must be a multiple of %d", (long long)M, few_rows ? 64 : 128);
@@ -564,7 +513,9 @@ int pt::gemm_m_grouped(const void* a_fp8, const float* a_scale, RowScales order,
   g.sb = b_scale; g.sb_rs = KB; g.sb_ks = 1; g.sb_shift = 7;
   g.out = out; g.ldo = N; g.out_dtype = out_dtype; g.accumulate = 0;
   g.rows_a = M; g.rows_b = N; g.red = K; g.mode = GEMM_M_GROUPED; g.offs = offs; g.G = G;
-  g.b_stride_g = N * K; g.sb_stride_g = NB * KB; g.few_rows = few_rows; g.row_used = out_row_index ? out_row_index : row_used;
+  g.b_stride_g = N * K; g.sb_stride_g = NB * KB; g.few_rows = few_rows;
+  g.row_used = out_row_index ? out_row_index : row_used;
+  g.used_rows = !out_row_index ? used_rows : out2 ? out2_rows : out_rows;
   g.a_bytes = M * K; g.b_bytes = N * K; g.sa_bytes = M * KB * 4; g.sb_bytes = NB * KB * 4;
   g.tiles_a = (int)(M / 128); g.tiles_b = (int)NB;
   g.total_tiles = (int64_t)g.tiles_a * g.tiles_b;

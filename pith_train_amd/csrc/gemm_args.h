@@ -5,8 +5,6 @@
 
 namespace pt {
 
-enum { GEMM_DENSE = 0, GEMM_M_GROUPED = 1, GEMM_K_GROUPED = 2 };
-
 struct GemmArgs {
   const uint8_t* a; int64_t lda;          // [rows_a, red] bytes
   const uint8_t* b; int64_t ldb;          // [rows_b, red] bytes
@@ -34,6 +32,7 @@ struct GemmArgs {
   int64_t out_extent;                     // with head_a: bytes from out to the end of out2, below 2 GiB
   int few_rows;                           // m-grouped: the group ends are multiples of 64, not of 128
   const int32_t* row_used;                // m-grouped: negative (with out2: -1) where row r of the result is not wanted; row r of a may hold anything there
+  int64_t used_rows;                      // with row_used: how many are, at most (rows_a may be a capacity)
   int b_kmajor;                           // m-grouped, row-split kernel: b is [red, rows_b] per group (row pitch ldb) instead of [rows_b, red]
 };
 
@@ -48,14 +47,9 @@ __device__ __forceinline__ int k_group_end(const GemmArgs& p, int g) {
 // m-grouped: groups from which on the kernel of large tiles looks for the padding behind each
 static constexpr int kPaddedGroups = 64;
 
-// m-grouped: weights that the small-problem kernel loads past the memory-side cache (launch_small_mode has the rule's reasons)
-inline bool streams_weights(const GemmArgs& a) { return a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0; }
-
 // persistent kernel whose two steps per 128-block split the tile by rows (gemm_rowsplit.hip)
 int launch_gemm_rowsplit(const GemmArgs& a, hipStream_t stream);
-// one tile of 64 or 128 rows x 128 columns per workgroup, for small problems (gemm_small.hip); kDeepTile: 128 rows, one
-// workgroup per compute unit (dense products)
-static constexpr int kDeepTile = 129;
+// one tile of 64 or 128 rows x 128 columns per workgroup, for small problems, or kDeepTile (gemm_small.hip)
 int launch_gemm_small(const GemmArgs& a, int rows, hipStream_t stream);
 // the tiles of two independent dense products in one launch of that kernel
 int launch_gemm_small_pair(const GemmArgs& a, const GemmArgs& b, int rows, hipStream_t stream);

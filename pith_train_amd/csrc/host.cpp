@@ -21,6 +21,7 @@
 #include <sstream>
 
 #include "../../include/pithtrain_hip.h"
+#include "gemm_rules.h"
 
 namespace py = pybind11;
 using at::Tensor;
@@ -438,14 +439,13 @@ struct Dims {
   Pieces backward_temp(bool sums) const { return Pieces({2 * M * half, sums ? M / 128 * half * 8 : 0}); }  // grad_h, column sums
 };
 
-// Whether a training step leaves out what stands for padding (the _without_padding steps): the rows go back to their places, and groups of whole
-// 128-row blocks are padding for a good part: up to 96 rows per expert (d.M holds 127 a group and up to 255 for it), us a pass with padding
+// Whether a training step of `routed` rows leaves out what stands for padding (the _without_padding steps) when the rows go back
+// to their places: up to few_used_rows, where groups of whole 128-row blocks are padding for a good part, us a pass with padding
 // written / left out: 128 experts of 2048 x 768, 16 rows each 966 / 903, 48 981 / 942, 96 1013 / 1008; 64 of
 // 2048 x 1408, 16 839 / 795, 64 860 / 836; and from 64 groups on, whatever their rows, where the kernel of large tiles looks for it
 // (gemm_rowsplit.hip has both sides).  Biases and the clamped activation make other values than zero of padding, which the
 // column scales of the transposed activations see: such blocks write it.
-bool leaves_padding(const Dims& d, bool biased) { return !biased && (d.M <= 224 * d.G + 256 || d.G >= 64); }
-
+bool leaves_padding(const Dims& d, int64_t routed, bool biased) { return !biased && (pt::few_used_rows(routed, d.G) || d.G >= 64); }
 bool in_whole_chunks(const Tensor& map) { return ((uintptr_t)ptr(map) & 15) == 0; }
 
 // Forward of an expert block (see fused_experts._forward): (out, gate_up, kept buffers, whether padding was left out).
@@ -488,7 +488,7 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>, bool> experts_forward(const Tens
   a.composed_map = (int32_t*)temp.at(0); a.x_fp8 = temp.at(1); a.x_scale = (float*)temp.at(2); a.h_fp8 = temp.at(3); a.h_scale = (float*)temp.at(4);
   a.stream = (pt_stream_t)stream;
   // (those steps read the map in 16-byte chunks; a slice of a longer one may start anywhere)
-  const bool without_padding = row_map && scatter && in_whole_chunks(*row_map) && (keep ? leaves_padding(d, clamped || gu_bias) : few_rows);
+  const bool without_padding = row_map && scatter && in_whole_chunks(*row_map) && (keep ? leaves_padding(d, routed, clamped || gu_bias) : few_rows);
   if (without_padding)
     check(lib.pt_experts_forward_without_padding(&a), "pt_experts_forward_without_padding");
   else

@@ -83,7 +83,7 @@ static int experts_forward(const pt_experts_forward_args* args, RowScales order,
   const int64_t N = 2 * a.half;
   const auto gate_up = [&](const void* bias) {
     return gemm_m_grouped(a.x_fp8, a.x_scale, order, a.gu_fp8, a.gu_scale, a.gate_up, PT_BF16, a.offs, G, a.M, N, a.K, nullptr, 0, bias, a.stream,
-                          false, few, nullptr, 0, used);
+                          false, few, nullptr, 0, used, a.out_rows);
   };
   if (few)
     PT_STEP_AS(pt_gemm_m_grouped_nt_few_rows, a.M, N, a.K, gate_up(a.gu_bias));
@@ -152,7 +152,7 @@ static int experts_backward(const pt_experts_backward_args* args, RowScales orde
   }
   const auto grad_h = [&] {
     return gemm_m_grouped(a.dy_fp8, a.dy_scale, order, a.dn_dg, a.dn_dg_scale, a.grad_h, PT_BF16, a.offs, G, a.M, a.half, a.H, nullptr, 0, nullptr,
-                          a.stream, a.dn_forward_layout != 0, false, nullptr, 0, used);
+                          a.stream, a.dn_forward_layout != 0, false, nullptr, 0, used, a.grad_rows);
   };
   if (a.dn_forward_layout)
     PT_STEP_AS(pt_gemm_m_grouped_nn, a.M, a.half, a.H, grad_h());

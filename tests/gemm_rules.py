@@ -10,7 +10,12 @@ HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))
 SOURCE = f"""
 #include "{HEADER}"
 #define EXPORT extern "C" int64_t
+struct Args {{ int64_t mode, rows_a, rows_b, red, G, row_used, used_rows, b_stride_g, ldb; }};
+EXPORT small_tile_rows(int64_t mode, int64_t rows_a, int64_t rows_b, int64_t red, int64_t G, int64_t row_used, int64_t used_rows, int64_t ldb) {{
+  return pt::small_tile_rows(Args{{mode, rows_a, rows_b, red, G, row_used, used_rows, rows_b * red, ldb}});
+}}
 EXPORT schedule(int64_t largest, int64_t sum, int64_t per_group, int64_t workgroups) {{ return pt::schedule_of_groups(largest, sum, per_group, workgroups); }}
+EXPORT few_used_rows(int64_t rows, int64_t groups) {{ return pt::few_used_rows(rows, groups); }}
 EXPORT big_tile_parts(int64_t form, int64_t total, int64_t workgroups) {{ return pt::big_tile_parts((pt::Schedule)form, total, workgroups); }}
 """
 FORMS = "in order", "eighths", "parts"
@@ -28,6 +33,12 @@ def call(name, *args):
     f = getattr(_library(), name)
     f.restype, f.argtypes = ctypes.c_int64, [ctypes.c_int64] * len(args)
     return f(*args)
+
+
+def m_grouped_tile_rows(rows_a, n, k, groups, used_rows=None, reduction_major=False):
+    """Rows of the tiles that an m-grouped product of ``rows_a`` padded rows takes (0: the large ones).  ``used_rows``: how many
+    of them count, where the launch knows which."""
+    return call("small_tile_rows", 1, rows_a, n, k, groups, used_rows is not None, used_rows or 0, n if reduction_major else k)
 
 
 def schedule(blocks, per_group, workgroups=256):

@@ -1,7 +1,7 @@
 """Which form a GEMM launch takes, by its sizes: both sides of every line."""
 
 import pytest
-from gemm_rules import call, schedule
+from gemm_rules import call, m_grouped_tile_rows, schedule
 
 
 @pytest.mark.parametrize("groups,largest,rest,per_group,form", [
@@ -26,3 +26,19 @@ def test_schedule_of_skewed_groups(groups, largest, rest, per_group, form):
 
 def test_parts_of_a_share_that_are_dealt_out_one_by_one():
     assert [call("big_tile_parts", form, blocks * 256, 256) for form in (1, 2) for blocks in (56, 139, 140, 400)] == [8, 8, 16, 16, 8, 8, 8, 8]
+
+
+def test_few_used_rows_are_counted_without_their_padding():
+    assert [call("few_used_rows", rows, 128) for rows in (0, 128 * 16, 128 * 120, 128 * 120 + 1, 128 * 160)] == [1, 1, 1, 0, 0]
+
+
+
+@pytest.mark.parametrize("groups,n,k", [(128, 1536, 2048), (128, 2048, 768), (64, 2816, 2048)])
+def test_a_capacity_and_exact_sizes_take_the_same_tiles(groups, n, k):
+    """The rows that count decide, not the padded rows that hold them: whole blocks of the routing's own sizes, or as many as
+    any routing could need."""
+    for rows in (16, 64, 96, 120, 121, 128, 136, 150):
+        exact = groups * (128 if rows <= 110 else 128 * 3 // 2)  # a half of the groups past one block, of those with 128 rows in the mean
+        capacity = (rows * groups + 127 * groups + 127) // 128 * 128
+        answers = {m_grouped_tile_rows(padded, n, k, groups, rows * groups) for padded in (exact, capacity)}
+        assert answers == {128 if rows <= 120 else 0}, rows

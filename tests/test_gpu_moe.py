@@ -659,8 +659,10 @@ def test_steps_with_row_scales_by_row_and_by_block_agree_bit_for_bit(form):
     (8, 272, 256, 40, 2, False, False),      # ten rows an expert, ragged widths
     (130, 256, 128, 64, 8, False, True),     # four; some experts get none, one all of 64 tokens
     (6, 1040, 384, 250, 2, True, False),     # 83: eights that end inside a tile; rows of the expanded form
-    (4, 256, 128, 384, 1, False, False),     # 96, the most for which padding is left out
-    (4, 256, 128, 390, 1, False, False),     # and more
+    (4, 256, 128, 384, 1, False, False),     # 96
+    (4, 256, 128, 390, 1, False, False),
+    (4, 256, 128, 480, 1, False, False),     # 120, the most for which fewer than 64 experts leave padding out
+    (4, 256, 128, 481, 1, False, False),     # and more
     (66, 528, 384, 2900, 6, True, True),     # many groups of the large tiles' kernel: ends of groups of every length
 ])
 def test_training_step_that_leaves_padding_out(kind, E, H, I, T, k, dedup, holes):
