@@ -14,9 +14,16 @@ constexpr int64_t up_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // 932, 124 957 / 946
 constexpr bool few_used_rows(int64_t rows, int64_t groups) { return rows <= 120 * groups; }
 
-// Weights that the small-problem kernel loads past the memory-side cache (launch_small_mode has the rule's reasons)
+// Weights that the small-problem kernel loads past the memory-side cache (launch_small_mode has the reasons for their size): those of
+// groups of 64 rows, and in tiles of 128 rows up to one and a half of them a group (rows_a, or where that is a capacity half a tile more than the
+// rows that count).  Weights that are read again come from that cache; operands from HBM, us through / past it for 1, 2, 3 and 5 row tiles: 8 x 4096 x
+// 4096 45 / 43, 62 / 60, 85 / 101, 121 / 139; 32 x 2048 x 2048 38 / 34, 60 / 60, 78 / 82, 118 / 128; reduction-major 43 / 37, 63 / 63, 77 / 81,
+// 118 / 130; 128 x 1536 x 2048 97 / 95, 166 / 170, 213 / 240, 320 / 360
 template <class Args>
-constexpr bool streams_weights(const Args& a) { return a.b_stride_g * a.G >= (128ll << 20) && a.ldb % 128 == 0; }
+constexpr bool streams_weights(const Args& a) {
+  const int64_t groups = a.G, counted = a.used_rows + 64 * groups, rows = a.row_used && counted < a.rows_a ? counted : a.rows_a;
+  return a.b_stride_g * groups >= (128ll << 20) && a.ldb % 128 == 0 && (a.few_rows || rows <= 192 * groups);
+}
 
 // ---- large or small tiles (Args: GemmArgs) -------------------------------------------------------------------------------------
 // Small: 64 or 128 rows x 128 columns, two workgroups per compute unit; kDeepTile: 128 rows, one workgroup (dense products)

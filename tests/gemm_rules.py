@@ -10,9 +10,12 @@ HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))
 SOURCE = f"""
 #include "{HEADER}"
 #define EXPORT extern "C" int64_t
-struct Args {{ int64_t mode, rows_a, rows_b, red, G, row_used, used_rows, b_stride_g, ldb; }};
+struct Args {{ int64_t mode, rows_a, rows_b, red, G, row_used, used_rows, b_stride_g, ldb, few_rows; }};
 EXPORT small_tile_rows(int64_t mode, int64_t rows_a, int64_t rows_b, int64_t red, int64_t G, int64_t row_used, int64_t used_rows, int64_t ldb) {{
-  return pt::small_tile_rows(Args{{mode, rows_a, rows_b, red, G, row_used, used_rows, rows_b * red, ldb}});
+  return pt::small_tile_rows(Args{{mode, rows_a, rows_b, red, G, row_used, used_rows, rows_b * red, ldb, 0}});
+}}
+EXPORT streams_weights(int64_t rows_a, int64_t rows_b, int64_t red, int64_t G, int64_t row_used, int64_t used_rows, int64_t ldb, int64_t few_rows) {{
+  return pt::streams_weights(Args{{1, rows_a, rows_b, red, G, row_used, used_rows, rows_b * red, ldb, few_rows}});
 }}
 EXPORT schedule(int64_t largest, int64_t sum, int64_t per_group, int64_t workgroups) {{ return pt::schedule_of_groups(largest, sum, per_group, workgroups); }}
 EXPORT few_used_rows(int64_t rows, int64_t groups) {{ return pt::few_used_rows(rows, groups); }}

@@ -42,3 +42,16 @@ def test_a_capacity_and_exact_sizes_take_the_same_tiles(groups, n, k):
         capacity = (rows * groups + 127 * groups + 127) // 128 * 128
         answers = {m_grouped_tile_rows(padded, n, k, groups, rows * groups) for padded in (exact, capacity)}
         assert answers == {128 if rows <= 120 else 0}, rows
+
+
+def test_weights_that_are_read_again_stay_in_the_memory_side_cache():
+    """128 MiB and more of whole lines, for groups of up to one and a half tiles of 128 rows, counted with half a tile of padding
+    where a capacity holds them; groups of 64 rows always."""
+
+    def streams(rows, groups=16, n=4096, k=2048, used=None, ldb=None, few=0):
+        return call("streams_weights", rows * groups, n, k, groups, used is not None, (used or 0) * groups, ldb or k, few)
+
+    assert [streams(rows) for rows in (128, 192, 193, 256, 384, 640)] == [1, 1, 0, 0, 0, 0]
+    assert [streams(rows + 127, used=rows) for rows in (16, 120, 128, 129, 300)] == [1, 1, 1, 0, 0]
+    assert streams(192, used=192) and not streams(256, used=192)  # whole blocks of rows that all count
+    assert streams(640, few=1) and not streams(128, n=4080) and not streams(128, groups=15) and not streams(128, ldb=2080)
