@@ -569,6 +569,57 @@ def test_rows_of_two_outputs(gemm_kernel, N, K, users):
         assert torch.isfinite(want.float()).all() and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("reduction_major", [0, 1])
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("N,K", [(528, 272), (768, 1408), (272, 2064)])
+def test_ends_of_many_groups(gemm_kernel, N, K, two, reduction_major):
+    """From 64 groups on the kernel of large tiles ends a group at its last used row, as the one of small tiles always does:
+    groups that end 1, 7, 8, 9, 64, 65, 127 and 128 rows into their last block, of one to three blocks, and empty ones, stored
+    to one output and to two.  The bits of a launch whose rows all count, nothing else written, whatever padding holds."""
+    from pith_train_amd import _lib
+
+    if gemm_kernel in ("p0", "q0", "q1", "t"):
+        pytest.skip("names of r0, and a kernel that stores no scattered rows")
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    G_, KB = 66, (K + 127) // 128
+    ends = [(1, 7, 8, 9, 64, 65, 127, 128)[i % 8] for i in range(G_)]
+    blocks = [0 if i % 11 == 5 else 1 + i % 3 for i in range(G_)]
+    rows = torch.tensor(blocks, dtype=torch.int32) * 128
+    M = int(rows.sum())
+    offs = torch.cumsum(rows, 0).int().cuda()
+    used = torch.cat([(torch.arange(128 * b) < 128 * (b - 1) + e) for b, e in zip(blocks, ends)]).cuda()
+    q = torch.randint(0, 256, (M, K), dtype=torch.uint8, device="cuda", generator=g) & 0xBF
+    q_s = torch.exp2(torch.randint(-6, 3, (KB, M), device="cuda", generator=g).float())
+    b = torch.randint(0, 256, (G_, K, N) if reduction_major else (G_, N, K), dtype=torch.uint8, device="cuda", generator=g) & 0xBF
+    b_s = torch.exp2(torch.randint(-6, 3, (G_, KB, (N + 127) // 128) if reduction_major else (G_, (N + 127) // 128, KB), device="cuda", generator=g).float())
+    to = torch.randperm(M, device="cuda", generator=g).int()
+    second = torch.rand(M, device="cuda", generator=g) < 0.5
+
+    def run(counts, a, a_s):
+        index = torch.where(counts, torch.where(second, -2 - to, to) if two else to, -1).int()
+        outs = [torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+        args = [_lib.ptr(a), _lib.ptr(a_s), _lib.ptr(b), _lib.ptr(b_s), reduction_major, _lib.ptr(outs[0])]
+        sizes = [_lib.dtype_code(torch.bfloat16), _lib.ptr(offs), G_, M, N, K, _lib.ptr(index), M]
+        if two:
+            _lib.call("pt_gemm_m_grouped_by_block_two", *args, _lib.ptr(outs[1]), *sizes, M, _lib.stream_ptr())
+        else:
+            _lib.call("pt_gemm_m_grouped_by_block", *args, *sizes, _lib.stream_ptr())
+        return outs
+
+    want = run(torch.ones_like(used), q, q_s)
+    dirty, dirty_s = q.clone(), q_s.clone()
+    dirty[~used] = 0x7F  # not a number
+    dirty_s[:, ~used] = float("nan")
+    got = run(used, dirty, dirty_s)
+    for i in range(2):
+        mine = used & (second == bool(i)) if two else used if i == 0 else torch.zeros_like(used)
+        place = to[mine].long()
+        assert torch.isfinite(want[i][place].float()).all() and torch.equal(got[i][place], want[i][place])
+        rest = torch.ones(M, dtype=torch.bool, device="cuda")
+        rest[place] = False
+        assert got[i][rest].isnan().all()
+
+
 @pytest.mark.parametrize("tiles", [1, 3, 4, 10])
 def test_grouped_tile_order_at_the_edges_of_its_strips(gemm_kernel, tiles):
     """Groups with more row tiles than column tiles and the other way round, one strip and several of unequal

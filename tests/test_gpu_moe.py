@@ -663,7 +663,7 @@ def test_steps_with_row_scales_by_row_and_by_block_agree_bit_for_bit(form):
     (4, 256, 128, 390, 1, False, False),
     (4, 256, 128, 480, 1, False, False),     # 120, the most for which fewer than 64 experts leave padding out
     (4, 256, 128, 481, 1, False, False),     # and more
-    (66, 528, 384, 2900, 6, True, True),     # many groups of the large tiles' kernel: ends of groups of every length
+    (66, 528, 384, 2900, 6, True, True),     # many groups, 264 rows each: tiles of both kernels, ends of groups of every length
 ])
 def test_training_step_that_leaves_padding_out(kind, E, H, I, T, k, dedup, holes):
     """Few rows per expert: padding is neither read nor written but for the zeros of the transposed operands.  The bits of the
@@ -699,6 +699,19 @@ def test_training_step_that_leaves_padding_out(kind, E, H, I, T, k, dedup, holes
     ours, composed = run(True), run(False)
     for n, (a, b) in enumerate(zip(ours, composed)):
         assert b.float().abs().sum() > 0 and torch.equal(a, b), n
+
+
+@pytest.mark.parametrize("kind", ["fused", "split"])
+@pytest.mark.parametrize("T", [400, 2900])
+def test_training_step_that_leaves_padding_out_in_large_tiles(kind, T):
+    """The same with every grouped product in the kernel of large tiles, which looks for padding from 64 groups on."""
+    from pith_train_amd import _lib
+
+    _lib.call("pt_gemm_select_kernel", b"r0")
+    try:
+        test_training_step_that_leaves_padding_out(kind, 66, 528, 384, T, 6, True, True)
+    finally:
+        _lib.call("pt_gemm_select_kernel", None)
 
 
 def test_flags_of_the_steps_are_truth_values():
