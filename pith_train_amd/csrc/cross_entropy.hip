@@ -46,7 +46,7 @@ struct CeArgs {
   float* loss;
   int64_t* n_non_ignore;
   const float* grad_output;
-  int vec;  // rows start at multiples of their element size
+  int vec;  // rows start at multiples of their element size, as those of any tensor do; a C caller's elsewhere go element by element
 };
 
 // A row in 16-byte chunks.  Rows whose length is no multiple of 16 bytes start anywhere in one, so the chunks begin at

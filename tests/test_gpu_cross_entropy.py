@@ -22,7 +22,7 @@ def _case(N, V, seed, dtype, ignore_frac=0.2):
     return x, y
 
 
-def _check_grad(got, ref, dtype):
+def _check_grad(got, ref, dtype, least=1e-30):
     got, ref = got.float().cpu(), ref.float()
     assert got.shape == ref.shape
     if got.numel() == 0:
@@ -31,14 +31,13 @@ def _check_grad(got, ref, dtype):
         torch.testing.assert_close(got, ref, rtol=2e-5, atol=1e-10)
         return
     step = 2.0**-7 if dtype == torch.bfloat16 else 2.0**-10
-    least = 1e-30 if dtype == torch.bfloat16 else 2.0**-24  # below 2^-14 the float16 values are 2^-24 apart
     assert ((got - ref).abs() <= ref.abs() * step + least).all(), "more than one rounding step apart"
     assert (got == ref).float().mean() > 0.98
 
 
 @pytest.mark.parametrize("N,V,dtype", [
     (64, 4096, torch.bfloat16), (33, 151936, torch.bfloat16), (16, 50000, torch.float32), (9, 1000, torch.float16),
-    (7, 1003, torch.bfloat16),   # V not a multiple of 8: element-wise path
+    (7, 1003, torch.bfloat16),   # V not a multiple of 8: rows that start inside a chunk
     (3, 5, torch.float32), (1, 201088, torch.bfloat16), (0, 128, torch.bfloat16),
 ])
 def test_forward_backward(N, V, dtype):
@@ -184,7 +183,8 @@ def test_rows_that_start_anywhere(N, V, start, dtype):
     loss = cross_entropy(buf.view(N, V), y.cuda())
     torch.testing.assert_close(loss.detach().cpu(), o_loss, rtol=1e-5, atol=1e-6)
     stored = buf.detach().clone()
-    _check_grad(stored, o_grad, dtype)
+    # (rows of 300 007: float16 gradients below 2^-14 are 2^-24 apart, one step of which is more than 2^-10 of them)
+    _check_grad(stored, o_grad, dtype, 2.0**-24 if dtype == torch.float16 else 1e-30)
     (grad,) = torch.autograd.grad(loss * 0.3, buf)
     assert torch.equal(grad, stored * torch.tensor(0.3).to(dtype))
     assert (flat[:start] == 7).all() and (flat[start + N * V :] == 7).all()
