@@ -378,7 +378,7 @@ __device__ __forceinline__ int xcd_first_tile(const GemmArgs& p, const int* s_pr
 // the least, and its workgroups take the small ones in turns, one that has less so far the earlier, as if each took
 // the next tile when it is done.  What an XCD's tiles are has two forms:
 //   eighths  every XCD takes an eighth of every group (neighbours in the group's order, the remainders of the eighths in
-//            turn), so that all have the same to multiply, to store and to fetch from HBM
+//            turn), so that all have the same to multiply, to store and to fetch from HBM; of groups with tiles enough for it
 //   parts    the whole list is cut by cost, as without a schedule but anywhere: an operand is read by one XCD or two,
 //            but one whose 32 workgroups get 33 big tiles of nearly a share each takes two rounds for them
 // All of it is the same arithmetic in every workgroup (one wave).
